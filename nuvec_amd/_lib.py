@@ -146,6 +146,22 @@ def load() -> C.CDLL:
     return lib
 
 
+_native = None
+
+
+def native():
+    """The native calls (`csrc/native.cpp`), built beside the library; no fallback if they are missing."""
+    global _native
+    if _native is None:
+        load()
+        if not os.path.exists(os.path.join(HERE, "_native.so")):
+            from . import build
+            build.build_native()
+        from . import _native as module
+        _native = module
+    return _native
+
+
 def last_error() -> str:
     return load().nvq_last_error().decode("utf-8", "replace")
 

@@ -1,4 +1,5 @@
-"""Compiles the gfx950 kernels and the C ABI into `nuvec_amd/libnuvec_hip.so` with hipcc.
+"""Compiles the gfx950 kernels and the C ABI into `nuvec_amd/libnuvec_hip.so` with hipcc, and the Python package's native
+calls (`csrc/native.cpp`, torch's C++ interface over that C ABI) into `nuvec_amd/_native.so` with the host compiler.
 
 Cross-compiles without a GPU.  Run as `python -m nuvec_amd.build` or through
 `__graft_entry__.build()`.
@@ -14,6 +15,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(HERE, "..", "include")
 LIB = os.path.join(HERE, "libnuvec_hip.so")
+NATIVE = os.path.join(HERE, "_native.so")
 SOURCES = ["qmf_b8.hip", "qmf_fp8.hip", "qmf_b6.hip", "qmf_b5.hip", "qmf_b4.hip", "qmf_fp4.hip", "qmf_nvfp4.hip", "qmf_b3.hip", "qmf_b2.hip", "qmf_b1.hip", "qmm.hip", "qmv.hip", "qmv_dot8.hip", "qmm_f32.hip", "qmr.hip",
            "qvm.hip", "nvq_api.hip", "affine_quant.hip", "fp_quant.hip", "qmf.hip", "gather.hip", "repack.hip", "calib.hip", "qattn.hip", "qmd.hip", "glu.hip"]  # slowest to compile first
 
@@ -69,7 +71,26 @@ def build(verbose: bool = False, jobs: int = 8, changed_only: bool = False) -> s
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"link failed:\n{proc.stdout}\n{proc.stderr}")
+    build_native(verbose)
     return LIB
+
+
+def build_native(verbose: bool = False) -> str:
+    """Compiles `csrc/native.cpp` against the installed torch; links to the library beside it."""
+    import sysconfig
+
+    import torch
+    root = os.path.dirname(torch.__file__)
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-I{root}/include", "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}", f"-I{INCLUDE}",
+           os.path.join(CSRC, "native.cpp"), "-o", NATIVE, f"-L{root}/lib", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip",
+           "-ltorch_python", f"-L{HERE}", "-l:libnuvec_hip.so", "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed on native.cpp:\n{proc.stdout}\n{proc.stderr}")
+    return NATIVE
 
 
 if __name__ == "__main__":

@@ -1,0 +1,437 @@
+// The Python package's calls in native code: `nuvec_amd._native`.
+//
+// A decode step is launch-bound: its kernels take 3 to 20 us each, and the argument checks, descriptors and allocations of
+// one call took 12 to 17 us in Python (a one-row product of W[1024,4096]: 16.7 us per call, of which the kernel is 3.4).  Here
+// the same work is done on the tensors' own C++ objects, a block's layers in one call.
+//
+// Every function takes the plain case alone: operands on the bound device, dense, of one element type, of matching shapes.
+// Whatever else it meets (and whatever the library refuses) it declines by returning None, before anything is launched, and
+// the caller's Python path, which holds every conversion and the reference's messages, does the call.
+#include <torch/csrc/Dtype.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <ATen/hip/EmptyTensor.h>
+#include <ATen/core/Tensor.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+
+#include "nuvec_hip.h"
+
+namespace {
+
+using at::Tensor;
+
+// ── reading Python objects ──────────────────────────────────────────────────────────────────────────────────────────
+struct Names {
+    PyObject *mode, *group_size, *bits, *weight, *scales, *biases, *bias, *quant, *global_scale;
+    PyObject *gate_proj, *up_proj, *down_proj, *gate_up_proj, *geglu;
+} names;
+
+PyTypeObject *linear_type = nullptr;  // layers.QuantizedLinear: its forward is the one restated here (a subclass may have another)
+uint64_t ready_devices = 0;           // devices nvq_init has answered for (ops._init), read and written under the GIL
+
+struct Ref {
+    PyObject *p;
+    explicit Ref(PyObject *o) : p(o) {}
+    Ref(const Ref &) = delete;
+    ~Ref() { Py_XDECREF(p); }
+};
+
+bool declined() {
+    PyErr_Clear();
+    return false;
+}
+
+bool read_int(PyObject *o, PyObject *name, int32_t &v) {
+    Ref a(PyObject_GetAttr(o, name));
+    if (a.p == nullptr || !PyLong_Check(a.p)) return declined();
+    const long n = PyLong_AsLong(a.p);
+    if (n == -1 && PyErr_Occurred()) return declined();
+    v = (int32_t)n;
+    return true;
+}
+
+bool read_quant(PyObject *o, nvq_quant &q) {
+    return read_int(o, names.mode, q.mode) && read_int(o, names.group_size, q.group_size) && read_int(o, names.bits, q.bits);
+}
+
+// A tensor, or none at all for None.
+bool as_tensor(PyObject *o, Tensor &t) {
+    if (o == Py_None) return true;
+    if (!THPVariable_Check(o)) return false;
+    t = THPVariable_Unpack(o);
+    return true;
+}
+bool read_tensor(PyObject *o, PyObject *name, Tensor &t) {
+    Ref a(PyObject_GetAttr(o, name));
+    return a.p == nullptr ? declined() : as_tensor(a.p, t);
+}
+
+// ── operands ────────────────────────────────────────────────────────────────────────────────────────────────────────
+int32_t code_of(at::ScalarType t) {
+    switch (t) {
+    case at::kHalf: return NVQ_F16;
+    case at::kBFloat16: return NVQ_BF16;
+    case at::kFloat: return NVQ_F32;
+    default: return -1;
+    }
+}
+
+bool is_word(at::ScalarType t) { return t == at::kUInt32 || t == at::kInt; }
+
+const void *ptr(const Tensor &t) { return t.defined() ? t.const_data_ptr() : nullptr; }
+
+// Whether `t` lies densely on the device that the library is bound to and that is current.
+struct Place {
+    c10::Device device;
+    explicit Place(const Tensor &x) : device(x.defined() ? x.device() : c10::Device(at::kCPU)) {}
+    bool usable() const {
+        return device.is_cuda() && device.index() >= 0 && device.index() < 64 && (ready_devices >> device.index() & 1) != 0 &&
+               c10::hip::current_device() == device.index();
+    }
+    bool holds(const Tensor &t) const { return t.device() == device && t.is_contiguous(); }
+    void *stream() const { return c10::hip::getCurrentHIPStream(device.index()).stream(); }
+    Tensor empty(at::IntArrayRef sizes, at::ScalarType type) const {
+        return at::detail::empty_cuda(sizes, type, device, std::nullopt);
+    }
+};
+
+struct Packed {
+    Tensor w, s, b;
+    nvq_quant q;
+
+    // Codes, scales and biases of `dims` dimensions that go together and with activations of `type` (ops._check_groups,
+    // ops._quantized_columns); `columns`: the values of a packed row.
+    bool fits(const Place &at, at::ScalarType type, int64_t dims, int64_t &columns) const {
+        if (!w.defined() || !s.defined() || !is_word(w.scalar_type()) || w.dim() != dims || s.dim() != dims || !at.holds(w) || !at.holds(s))
+            return false;
+        if (q.mode == NVQ_AFFINE) {
+            if (!b.defined() || s.scalar_type() != type || b.scalar_type() != type || !at.holds(b) || b.sizes() != s.sizes()) return false;
+        } else if (b.defined() || s.scalar_type() != at::kByte) {
+            return false;
+        }
+        for (int64_t i = 0; i + 1 < dims; i++)
+            if (w.size(i) != s.size(i)) return false;
+        columns = s.size(dims - 1) * q.group_size;
+        return columns > 0 && w.size(dims - 1) * 32 == columns * q.bits;
+    }
+};
+
+bool bias_fits(const Tensor &bias, const Place &at, at::ScalarType type, int64_t n) {
+    return !bias.defined() || (bias.scalar_type() == type && bias.dim() == 1 && bias.size(0) == n && at.holds(bias));
+}
+
+using Sizes = c10::SmallVector<int64_t, 6>;
+Sizes with_last(at::IntArrayRef sizes, int64_t last) {
+    Sizes s(sizes.begin(), sizes.end());
+    s.back() = last;
+    return s;
+}
+
+// ── the calls ───────────────────────────────────────────────────────────────────────────────────────────────────────
+struct Flags {
+    bool transpose = true, row_exact = false, rows = false, scratch = true;
+};
+
+// ops.quantized_matmul of one weight matrix.
+bool product(const Tensor &x, const Packed &p, const Tensor &bias, Flags f, Tensor &out) {
+    const Place at(x);
+    if (!at.usable() || x.dim() < 2 || !x.is_contiguous() || x.numel() == 0) return false;
+    const int32_t code = code_of(x.scalar_type());
+    int64_t columns;
+    if (code < 0 || !p.fits(at, x.scalar_type(), 2, columns)) return false;
+    const int64_t rows = p.w.size(0), inner = f.transpose ? columns : rows, outer = f.transpose ? rows : columns;
+    if (x.size(-1) != inner || outer == 0 || !bias_fits(bias, at, x.scalar_type(), outer)) return false;
+    nvq_qmm_desc d{};
+    d.quant = p.q, d.dtype = code, d.transpose = f.transpose, d.row_exact = f.row_exact, d.rows = f.rows;
+    d.m = x.numel() / inner, d.n = outer, d.k = inner, d.item_rows = x.size(-2);
+    const size_t need = f.scratch ? nvq_quantized_matmul_workspace_bytes(&d) : 0;
+    Tensor workspace, y = at.empty(with_last(x.sizes(), outer), x.scalar_type());
+    if (need > 0) workspace = at.empty({(int64_t)need}, at::kByte);
+    const int32_t rc = nvq_quantized_linear(&d, ptr(x), ptr(p.w), ptr(p.s), ptr(p.b), ptr(bias), y.mutable_data_ptr(),
+                                            need > 0 ? workspace.mutable_data_ptr() : nullptr, at.stream());
+    if (rc != NVQ_OK) return false;
+    out = std::move(y);
+    return true;
+}
+
+// ops.quantized_matmul_glu.
+bool product_glu(const Tensor &x, const Packed &p, const Tensor &bias, int32_t activation, float alpha, float limit, Tensor &out) {
+    const Place at(x);
+    if (!at.usable() || x.dim() < 1 || !x.is_contiguous() || x.numel() == 0) return false;
+    const int32_t code = code_of(x.scalar_type());
+    int64_t columns;
+    if (code < 0 || !p.fits(at, x.scalar_type(), 2, columns) || x.size(-1) != columns) return false;
+    const int64_t n = p.w.size(0);
+    if (n == 0 || n % 128 != 0 || !bias_fits(bias, at, x.scalar_type(), n)) return false;
+    nvq_qmm_desc d{};
+    d.quant = p.q, d.dtype = code, d.transpose = 1;
+    d.m = d.item_rows = x.numel() / columns, d.n = n, d.k = columns;
+    Tensor y = at.empty(with_last(x.sizes(), n / 2), x.scalar_type());
+    const int32_t rc = nvq_quantized_matmul_glu(&d, activation, alpha, limit, ptr(x), ptr(p.w), ptr(p.s), ptr(p.b), ptr(bias),
+                                                y.mutable_data_ptr(), at.stream());
+    if (rc != NVQ_OK) return false;
+    out = std::move(y);
+    return true;
+}
+
+// ops.glu of two dense tensors, without biases.
+bool gated(const Tensor &gate, const Tensor &up, int32_t activation, float alpha, float limit, Tensor &out) {
+    const Place at(gate);
+    const int64_t hidden = gate.size(-1);
+    nvq_glu_desc d{code_of(gate.scalar_type()), activation, alpha, limit, gate.numel() / hidden, hidden, hidden, hidden, 0};
+    Tensor y = at.empty(gate.sizes(), gate.scalar_type());
+    if (nvq_glu(&d, ptr(gate), ptr(up), nullptr, nullptr, nullptr, y.mutable_data_ptr(), at.stream()) != NVQ_OK) return false;
+    out = std::move(y);
+    return true;
+}
+
+// ── layers ──────────────────────────────────────────────────────────────────────────────────────────────────────────
+struct Linear {
+    Packed p;
+    Tensor bias;
+};
+bool read_linear(PyObject *o, Linear &l) {
+    if (Py_TYPE(o) != linear_type) return false;
+    if (!read_tensor(o, names.weight, l.p.w) || !read_tensor(o, names.scales, l.p.s) || !read_tensor(o, names.biases, l.p.b) ||
+        !read_tensor(o, names.bias, l.bias))
+        return false;
+    Ref q(PyObject_GetAttr(o, names.quant));
+    return q.p == nullptr ? declined() : read_quant(q.p, l.p.q);
+}
+bool read_linear(PyObject *o, PyObject *name, Linear &l) {
+    Ref a(PyObject_GetAttr(o, name));
+    return a.p == nullptr ? declined() : read_linear(a.p, l);
+}
+
+PyObject *none() { Py_RETURN_NONE; }
+
+// A refusal inside torch (no memory left) is Python's exception, as it is where Python allocates.
+template <typename F>
+PyObject *guarded(F &&f) {
+    try {
+        return f();
+    } catch (const std::exception &e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+        return nullptr;
+    }
+}
+
+PyObject *wrap(bool done, Tensor &y) { return done ? THPVariable_Wrap(std::move(y)) : none(); }
+
+// linear(layer, x)
+PyObject *py_linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    return guarded([&]() -> PyObject * {
+        Tensor x, y;
+        Linear l;
+        if (n != 2 || !as_tensor(args[1], x) || !read_linear(args[0], l)) return none();
+        return wrap(product(x, l.p, l.bias, Flags(), y), y);
+    });
+}
+
+// quantized_matmul(x, weight, scales, biases, quant, transpose, row_exact, rows, scratch, bias)
+PyObject *py_quantized_matmul(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    return guarded([&]() -> PyObject * {
+        Tensor x, bias, y;
+        Packed p;
+        if (n != 10 || !as_tensor(args[0], x) || !as_tensor(args[1], p.w) || !as_tensor(args[2], p.s) || !as_tensor(args[3], p.b) ||
+            !read_quant(args[4], p.q) || !as_tensor(args[9], bias))
+            return none();
+        int flag[4];
+        for (int i = 0; i < 4; i++)
+            if ((flag[i] = PyObject_IsTrue(args[5 + i])) < 0) return nullptr;
+        const Flags f{flag[0] != 0, flag[1] != 0, flag[2] != 0, flag[3] != 0};
+        return wrap(product(x, p, bias, f, y), y);
+    });
+}
+
+// mlp(block, x, most): layers.Mlp.forward; up to `most` rows of x take the fused gate and up projections.
+PyObject *py_mlp(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    return guarded([&]() -> PyObject * {
+        Tensor x, hidden, y;
+        Linear down, gate, up;
+        if (n != 2 || !as_tensor(args[1], x) || !x.defined() || x.dim() < 1 || x.numel() == 0) return none();
+        Ref geglu(PyObject_GetAttr(args[0], names.geglu)), both(PyObject_GetAttr(args[0], names.gate_up_proj));
+        if (geglu.p == nullptr || both.p == nullptr || !read_linear(args[0], names.down_proj, down) ||
+            !read_linear(args[0], names.gate_proj, gate)) {
+            PyErr_Clear();
+            return none();
+        }
+        const int truth = PyObject_IsTrue(geglu.p);
+        if (truth < 0) return nullptr;
+        const int32_t activation = truth ? NVQ_GLU_GEGLU : NVQ_GLU_SWIGLU;
+        const int64_t rows = x.numel() / x.size(-1), most = gate.p.q.mode == NVQ_AFFINE ? 2 : 4;  // (layers.Mlp.forward says why)
+        if (both.p != Py_None && rows <= most) {
+            Linear l;
+            if (!read_linear(both.p, l)) return none();
+            product_glu(x, l.p, l.bias, activation, 0.0f, 0.0f, hidden);
+        }
+        if (!hidden.defined()) {
+            Tensor g, u;
+            if (!read_linear(args[0], names.up_proj, up) || !product(x, gate.p, gate.bias, Flags(), g) || !product(x, up.p, up.bias, Flags(), u) ||
+                g.sizes() != u.sizes() || !gated(g, u, activation, 0.0f, 0.0f, hidden))
+                return none();
+        }
+        return wrap(product(hidden, down.p, down.bias, Flags(), y), y);
+    });
+}
+
+// quantize(w, quant): (packed, scales, biases)
+PyObject *py_quantize(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    return guarded([&]() -> PyObject * {
+        Tensor w;
+        nvq_quant q;
+        if (n != 2 || !as_tensor(args[0], w) || !read_quant(args[1], q)) return none();
+        const Place at(w);
+        if (!at.usable() || w.dim() < 2 || w.numel() == 0 || !w.is_contiguous() || code_of(w.scalar_type()) < 0) return none();
+        const int64_t cols = w.size(-1);
+        if (q.group_size <= 0 || cols % q.group_size != 0) return none();
+        const bool affine = q.mode == NVQ_AFFINE;
+        const Sizes groups = with_last(w.sizes(), cols / q.group_size);
+        Tensor packed = at.empty(with_last(w.sizes(), cols * q.bits / 32), at::kUInt32);
+        Tensor scales = at.empty(groups, affine ? w.scalar_type() : at::kByte), biases;
+        if (affine) biases = at.empty(groups, w.scalar_type());
+        if (nvq_quantize(&q, code_of(w.scalar_type()), ptr(w), w.numel() / cols, cols, packed.mutable_data_ptr(), scales.mutable_data_ptr(),
+                         affine ? biases.mutable_data_ptr() : nullptr, at.stream()) != NVQ_OK)
+            return none();
+        Ref p(THPVariable_Wrap(std::move(packed))), s(THPVariable_Wrap(std::move(scales)));
+        Ref b(affine ? THPVariable_Wrap(std::move(biases)) : none());
+        return p.p && s.p && b.p ? PyTuple_Pack(3, p.p, s.p, b.p) : nullptr;
+    });
+}
+
+// The type a packed table gives its rows: the scales' for affine codes, else bfloat16 (ops.dequantize).
+at::ScalarType table_type(const Packed &p) { return p.q.mode == NVQ_AFFINE && p.s.defined() ? p.s.scalar_type() : at::kBFloat16; }
+
+bool is_dtype(PyObject *o, at::ScalarType &t) {
+    if (!THPDtype_Check(o)) return false;
+    t = reinterpret_cast<THPDtype *>(o)->scalar_type;
+    return true;
+}
+
+// dequantize(weight, scales, biases, quant, dtype or None)
+PyObject *py_dequantize(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    return guarded([&]() -> PyObject * {
+        Packed p;
+        if (n != 5 || !as_tensor(args[0], p.w) || !as_tensor(args[1], p.s) || !as_tensor(args[2], p.b) || !read_quant(args[3], p.q)) return none();
+        const Place at(p.w);
+        at::ScalarType type = table_type(p), asked = type;
+        if (args[4] != Py_None && !is_dtype(args[4], asked)) return none();
+        if (p.q.mode != NVQ_AFFINE) type = asked;
+        int64_t columns;
+        if (!at.usable() || code_of(type) < 0 || asked != type || p.w.dim() < 2 || p.w.numel() == 0 || !p.fits(at, type, p.w.dim(), columns))
+            return none();
+        Tensor y = at.empty(with_last(p.w.sizes(), columns), type);
+        const bool done = nvq_dequantize(&p.q, code_of(type), ptr(p.w), ptr(p.s), ptr(p.b), y.numel() / columns, columns,
+                                         y.mutable_data_ptr(), at.stream()) == NVQ_OK;
+        return wrap(done, y);
+    });
+}
+
+// embedding(weight, scales, biases, quant, ids)
+PyObject *py_embedding(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    return guarded([&]() -> PyObject * {
+        Packed p;
+        Tensor ids;
+        if (n != 5 || !as_tensor(args[0], p.w) || !as_tensor(args[1], p.s) || !as_tensor(args[2], p.b) || !read_quant(args[3], p.q) ||
+            !as_tensor(args[4], ids))
+            return none();
+        const Place at(p.w);
+        const at::ScalarType type = table_type(p);
+        int64_t columns;
+        if (!at.usable() || code_of(type) < 0 || !ids.defined() || !is_word(ids.scalar_type()) || !at.holds(ids) || ids.numel() == 0 ||
+            !p.fits(at, type, 2, columns))
+            return none();
+        Sizes sizes(ids.sizes().begin(), ids.sizes().end());
+        sizes.push_back(columns);
+        Tensor y = at.empty(sizes, type);
+        const bool done = nvq_dequantize_rows(&p.q, code_of(type), ptr(p.w), ptr(p.s), ptr(p.b), p.w.size(0), columns,
+                                              (const uint32_t *)ptr(ids), ids.numel(), y.mutable_data_ptr(), at.stream()) == NVQ_OK;
+        return wrap(done, y);
+    });
+}
+
+// attention(q, k weight, scales, biases, v weight, scales, biases, quant, scale, sinks): one query row per head
+// (ops.quantized_attention, ops.quantized_attention_fits)
+PyObject *py_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    return guarded([&]() -> PyObject * {
+        Tensor q, sinks;
+        Packed k, v;
+        if (n != 10 || !as_tensor(args[0], q) || !as_tensor(args[1], k.w) || !as_tensor(args[2], k.s) || !as_tensor(args[3], k.b) ||
+            !as_tensor(args[4], v.w) || !as_tensor(args[5], v.s) || !as_tensor(args[6], v.b) || !read_quant(args[7], k.q) ||
+            !as_tensor(args[9], sinks))
+            return none();
+        v.q = k.q;
+        const double scale = PyFloat_AsDouble(args[8]);
+        if (scale == -1.0 && PyErr_Occurred()) {
+            PyErr_Clear();
+            return none();
+        }
+        const Place at(q);
+        int64_t dim, same;
+        if (!at.usable() || q.dim() != 4 || q.size(2) != 1 || q.numel() == 0 || !q.is_contiguous() || k.q.mode != NVQ_AFFINE) return none();
+        const at::ScalarType type = q.scalar_type();
+        const int32_t code = code_of(type);
+        if (code < 0 || !k.fits(at, type, 4, dim) || !v.fits(at, type, 4, same) || dim != q.size(3) || same != dim ||
+            k.w.sizes() != v.w.sizes() || k.w.size(0) != q.size(0) || k.w.size(1) == 0 || k.w.size(2) == 0 ||
+            !bias_fits(sinks, at, type, q.size(1)))
+            return none();
+        const nvq_attention_desc d{code, k.q.bits, k.q.group_size, (int32_t)dim, q.size(0), q.size(1), k.w.size(1), k.w.size(2), (float)scale};
+        const size_t need = nvq_quantized_attention_workspace_bytes(&d);
+        Tensor workspace, y = at.empty(q.sizes(), type);
+        if (need > 0) workspace = at.empty({(int64_t)need}, at::kByte);
+        const bool done = nvq_quantized_attention(&d, ptr(q), ptr(k.w), ptr(k.s), ptr(k.b), ptr(v.w), ptr(v.s), ptr(v.b), ptr(sinks),
+                                                  y.mutable_data_ptr(), need > 0 ? workspace.mutable_data_ptr() : nullptr, at.stream()) == NVQ_OK;
+        return wrap(done, y);
+    });
+}
+
+// register(QuantizedLinear): the types whose forward is restated here
+PyObject *py_register(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    if (n != 1 || !PyType_Check(args[0])) {
+        PyErr_SetString(PyExc_TypeError, "register(QuantizedLinear)");
+        return nullptr;
+    }
+    Py_INCREF(args[0]);
+    linear_type = (PyTypeObject *)args[0];
+    return none();
+}
+
+// ready(index): nvq_init has answered for the device
+PyObject *py_ready(PyObject *, PyObject *index) {
+    const long i = PyLong_AsLong(index);
+    if (i == -1 && PyErr_Occurred()) return nullptr;
+    if (i >= 0 && i < 64) ready_devices |= 1ull << i;
+    return none();
+}
+
+#define NVQ_FAST(f) (PyCFunction)(void (*)(void)) f, METH_FASTCALL
+PyMethodDef methods[] = {
+    {"register", NVQ_FAST(py_register), nullptr},
+    {"ready", py_ready, METH_O, nullptr},
+    {"linear", NVQ_FAST(py_linear), nullptr},
+    {"quantized_matmul", NVQ_FAST(py_quantized_matmul), nullptr},
+    {"mlp", NVQ_FAST(py_mlp), nullptr},
+    {"quantize", NVQ_FAST(py_quantize), nullptr},
+    {"dequantize", NVQ_FAST(py_dequantize), nullptr},
+    {"embedding", NVQ_FAST(py_embedding), nullptr},
+    {"attention", NVQ_FAST(py_attention), nullptr},
+    {nullptr, nullptr, 0, nullptr},
+};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+extern "C" __attribute__((visibility("default"))) PyObject *PyInit__native(void) {
+    struct { PyObject **at; const char *text; } all[] = {
+        {&names.mode, "mode"}, {&names.group_size, "group_size"}, {&names.bits, "bits"}, {&names.weight, "weight"},
+        {&names.scales, "scales"}, {&names.biases, "biases"}, {&names.bias, "bias"}, {&names.quant, "quant"},
+        {&names.global_scale, "global_scale"}, {&names.gate_proj, "gate_proj"}, {&names.up_proj, "up_proj"},
+        {&names.down_proj, "down_proj"}, {&names.gate_up_proj, "gate_up_proj"}, {&names.geglu, "geglu"},
+    };
+    for (auto &n : all) {
+        *n.at = PyUnicode_InternFromString(n.text);
+        if (*n.at == nullptr) return nullptr;
+    }
+    return PyModule_Create(&module);
+}

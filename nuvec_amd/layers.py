@@ -10,8 +10,20 @@ from typing import Optional
 
 import torch
 
-from . import ops
+from . import _lib, ops
 from .ops import Quant, QuantMode, Quantized
+
+
+_native = None
+
+
+def _calls():
+    """The native calls, told which layers they may read."""
+    global _native
+    n = _lib.native()
+    n.register(QuantizedLinear)
+    _native = n
+    return n
 
 
 def _quant(quant) -> Quant:
@@ -44,6 +56,9 @@ class QuantizedLinear:
         """layers.rs:155-162: the product, then the bias added as a separate rounded addition: here in the product
         kernels' epilogues (same two roundings, one launch) when the bias has the product's dtype and the mode no global
         scale; otherwise the addition stays separate, as in the reference, and promotes."""
+        y = (_native or _calls()).linear(self, x)
+        if y is not None:
+            return y
         q = self.quantized()
         if self.bias is None:
             return ops.quantized_matmul(x, q, transpose=True)
@@ -82,6 +97,9 @@ class Mlp:
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         """model.rs:2066-2074."""
+        y = (_native or _calls()).mlp(self, x)
+        if y is not None:
+            return y
         activation = "geglu" if self.geglu else "swiglu"
         rows = x.numel() // x.shape[-1] if x.shape[-1] else 0
         # (measured at 4096 -> 14336 -> 4096, device time: one row 29.1 -> 23.6 us with 4-bit weights, 25.9 -> 21.1 us with
@@ -120,7 +138,8 @@ class QuantizedEmbedding:
         """layers.rs:245-255: the rows for `ids`, dequantized (scales' dtype for affine, bfloat16 for the
         floating-point modes): shape `ids.shape + [dims]`.  One fused kernel; the taken packed rows are
         never written out."""
-        return ops.embedding(self.quantized(), ids)
+        y = (_native or _calls()).embedding(self.weight, self.scales, self.biases, self.quant, ids)
+        return ops.embedding(self.quantized(), ids) if y is None else y
 
     def as_linear(self, x: torch.Tensor) -> torch.Tensor:
         """layers.rs:258-261: `x W^T` with the quantized table (tied embeddings)."""
@@ -317,6 +336,10 @@ def quantized_attention(q: torch.Tensor, k: ops.Quantized, v: ops.Quantized, sca
         raise ops.InvalidArgument("quantized_attention: keys and values need one affine quantization")
     if k.biases is None or v.biases is None:
         raise ops.InvalidArgument("quantized_attention: affine biases missing")
+    if fused and q.ndim == 4 and q.shape[2] == 1:  # the plain case of the branch below
+        out = (_native or _calls()).attention(q, k.weight, k.scales, k.biases, v.weight, v.scales, v.biases, k.quant, scale, sinks)
+        if out is not None:
+            return out
     # (a single causal query row sees every key: the mask is empty)
     if fused and (not causal or q.shape[-2] == 1) and q.is_cuda and ops.quantized_attention_fits(q, k, v, sinks):
         return ops.quantized_attention(q, k, v, scale, sinks)  # one kernel (the reference's FastOp::QuantizedAttention)

@@ -128,6 +128,7 @@ def _init(t: torch.Tensor) -> None:
     if index not in _READY:
         _lib.check(_lib.load().nvq_init(index))
         _READY.add(index)
+        _lib.native().ready(index)
 
 
 def _stream() -> C.c_void_p:
@@ -199,6 +200,10 @@ def quantize(w: torch.Tensor, quant: Quant | QuantMode = Quant(), global_scale: 
     """ops.rs:965-1008 (`quantize`, `quantize_scaled`), primitive.rs:1223-1259: quantizes the last axis of `w`; with
     NVFP4's `global_scale` the group scales are relative to it, g / (448 * 6), and the result carries it."""
     quant = Quant.new(quant) if isinstance(quant, QuantMode) else quant
+    if global_scale is None:
+        done = (_lib._native or _lib.native()).quantize(w, quant)
+        if done is not None:
+            return Quantized(*done, quant)
     group, bits = quant.checked("quantize")
     if w.dtype not in _FLOATS:
         raise InvalidArgument(f"quantize: unsupported dtype {_name(w.dtype)}")
@@ -227,6 +232,10 @@ def dequantize(q: Quantized, dtype: Optional[torch.dtype] = None) -> torch.Tenso
     """ops.rs:1014-1027, quantized.rs:401-444: affine computes in the scales' dtype, then casts;
     the floating-point modes default to bfloat16."""
     quant = q.quant
+    if q.global_scale is None:
+        out = (_lib._native or _lib.native()).dequantize(q.weight, q.scales, q.biases, quant, dtype)
+        if out is not None:
+            return out
     quant.checked("dequantize")
     _check_groups("dequantize", quant.mode, q.scales, q.biases)
     if dtype is not None and not dtype.is_floating_point:
@@ -319,6 +328,10 @@ def embedding(q: Quantized, ids: torch.Tensor, dtype: Optional[torch.dtype] = No
     dequantized; shape `ids.shape + [cols]`.  Equals `dequantize` of the taken rows bit for bit."""
     op = "dequantize_rows"
     quant = q.quant
+    if dtype is None:
+        out = (_lib._native or _lib.native()).embedding(q.weight, q.scales, q.biases, quant, ids)
+        if out is not None:
+            return out
     quant.checked(op)
     _check_groups(op, quant.mode, q.scales, q.biases)
     if q.weight.ndim != 2:
@@ -365,6 +378,10 @@ def quantized_matmul(x: torch.Tensor, q: Quantized, transpose: bool = True, *, r
     kernels' epilogues as `QuantizedLinear::forward` adds it (layers.rs:155-162)."""
     op = "quantized_matmul"
     quant = q.quant
+    if q.global_scale is None:
+        y = (_lib._native or _lib.native()).quantized_matmul(x, q.weight, q.scales, q.biases, quant, transpose, row_exact, rows, scratch, bias)
+        if y is not None:
+            return y
     group, bits = quant.checked(op)
     _check_groups(op, quant.mode, q.scales, q.biases)
     g = _global_scale(op, quant, q.global_scale, x.device)
@@ -488,6 +505,10 @@ def quantized_attention(q: torch.Tensor, k: Quantized, v: Quantized, scale: floa
                         sinks: Optional[torch.Tensor] = None, scratch: bool = True) -> torch.Tensor:
     """fast.rs:694-718 where the kernel fits (`quantized_attention_fits`): one query row per head over the quantized
     cache in one launch."""
+    if scratch and k.quant == v.quant:
+        out = (_lib._native or _lib.native()).attention(q, k.weight, k.scales, k.biases, v.weight, v.scales, v.biases, k.quant, scale, sinks)
+        if out is not None:
+            return out
     if not quantized_attention_fits(q, k, v, sinks):
         raise Unsupported("quantized_attention: the operands do not fit the kernel")
     _init(q)

@@ -1,0 +1,94 @@
+"""The native calls (csrc/native.cpp) against the Python path they stand in for: bit for bit on what they take, and the
+Python path's own answer (conversions, broadcasts, refusals) on what they decline."""
+import pytest
+import torch
+
+import nuvec_amd as nv
+from nuvec_amd import _lib, layers
+
+pytestmark = pytest.mark.gpu
+
+
+class Declines:
+    """Stands in for the native module: every call is the Python path's."""
+    def __getattr__(self, name):
+        return lambda *a: None
+
+
+@pytest.fixture
+def both(monkeypatch):
+    def run(f):
+        native = f()
+        with monkeypatch.context() as m:
+            m.setattr(_lib, "_native", Declines())
+            m.setattr(layers, "_native", Declines())
+            python = f()
+        torch.cuda.synchronize()
+        return native, python
+    return run
+
+
+def same(a, b):
+    if isinstance(a, nv.Quantized):
+        return same(a.weight.view(torch.int32), b.weight.view(torch.int32)) and same(a.scales, b.scales) and \
+            (a.biases is None and b.biases is None or same(a.biases, b.biases))
+    return a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b)
+
+
+def linear(n, k, quant, dtype, bias):
+    q = nv.quantize(torch.randn(n, k, device="cuda").to(dtype), quant)
+    return layers.QuantizedLinear(q.weight, q.scales, q.biases, torch.randn(n, device="cuda").to(dtype) if bias else None, q.quant)
+
+
+QUANTS = [nv.Quant.affine(64, 4), nv.Quant.affine(32, 3), nv.Quant.new(nv.QuantMode.MXFP4), nv.Quant.new(nv.QuantMode.NVFP4)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("quant", QUANTS, ids=str)
+def test_calls_equal_the_python_path(both, quant, dtype):
+    torch.manual_seed(1)
+    for shape in ((1, 256), (2, 3, 256), (256,), (0, 256), (70, 256)):
+        for bias in (False, True):
+            layer, x = linear(192, 256, quant, dtype, bias), torch.randn(shape, device="cuda").to(dtype)
+            assert same(*both(lambda: layer(x))), (shape, bias)
+    wide = torch.randn(4, 512, device="cuda").to(dtype)
+    layer = linear(192, 256, quant, dtype, False)
+    assert same(*both(lambda: layer(wide[:, ::2])))           # strided: made dense by the Python path
+    mlp = layers.Mlp(linear(1024, 256, quant, dtype, False), linear(1024, 256, quant, dtype, False), linear(256, 1024, quant, dtype, True))
+    fused = layers.Mlp(mlp.gate_proj, mlp.up_proj, mlp.down_proj).fuse_gate_up()
+    for rows in (1, 2, 5):
+        x = torch.randn(rows, 256, device="cuda").to(dtype)
+        assert same(*both(lambda: mlp(x))) and same(*both(lambda: fused(x))), rows
+    w = torch.randn(3, 5, 256, device="cuda").to(dtype)
+    assert same(*both(lambda: nv.quantize(w, quant)))
+    packed = nv.quantize(w, quant)
+    for out in (None, torch.float32, torch.bfloat16):
+        assert same(*both(lambda: nv.dequantize(packed, out)))
+    table = nv.quantize(w.reshape(15, 256), quant)
+    for ids in (torch.tensor([[3, 14], [0, 3]], device="cuda", dtype=torch.int32), torch.tensor([7], device="cuda"),
+                torch.empty(0, device="cuda", dtype=torch.int32)):
+        assert same(*both(lambda: nv.embedding(table, ids)))
+    assert same(*both(lambda: nv.quantized_matmul(torch.ones(4, 15, device="cuda", dtype=dtype), table, transpose=False)))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_attention_equals_the_python_path(both, dtype):
+    torch.manual_seed(2)
+    k, v = (nv.quantize(torch.randn(2, 2, 600, 64, device="cuda").to(dtype), nv.Quant.affine(32, 8)) for _ in range(2))
+    q, sinks = torch.randn(2, 8, 1, 64, device="cuda").to(dtype), torch.randn(8, device="cuda").to(dtype)
+    for s in (None, sinks):
+        assert same(*both(lambda: layers.quantized_attention(q, k, v, 0.125, s, causal=True)))
+        assert same(*both(lambda: nv.ops.quantized_attention(q, k, v, 0.125, s)))
+
+
+def test_refusals_are_the_python_paths():
+    x = torch.randn(2, 128, device="cuda")
+    q = nv.quantize(torch.randn(64, 128, device="cuda"), nv.Quant.affine(64, 4))
+    with pytest.raises(nv.InvalidArgument, match="do not match"):
+        nv.quantized_matmul(x[:, :64].contiguous(), q)
+    with pytest.raises(nv.InvalidArgument, match="packed weights must be uint32"):
+        nv.quantized_matmul(x, nv.Quantized(q.weight.view(torch.float32), q.scales, q.biases, q.quant))
+    with pytest.raises(nv.InvalidArgument, match="group size 48"):
+        nv.quantize(x, nv.Quant.affine(48, 4))
+    mixed = nv.quantized_matmul(x.to(torch.bfloat16), q)  # promotes
+    assert mixed.dtype == torch.float32

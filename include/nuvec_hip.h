@@ -142,6 +142,16 @@ typedef struct nvq_attention_desc {
     float scale;
 } nvq_attention_desc;
 
+/* The same with several query rows per head (the reference's composition, fast/imp.rs:3996-4035, with nuvec-lm's causal
+ * mask, nuvec-lm/src/model.rs:3646-3700): q and out dtype [batch, query_heads, queries, head_dim]; with `causal` query i
+ * sees the positions up to positions - queries + i.  Half-precision types, head sizes 64 and 128, affine codes of any
+ * width and group, any number of query heads per key head. */
+typedef struct nvq_attention_prompt_desc {
+    nvq_attention_desc cache;
+    int64_t queries;
+    int32_t causal;
+} nvq_attention_prompt_desc;
+
 /* ── runtime ─────────────────────────────────────────────────────────────────────── */
 
 /* Binds the library to HIP device `device` (idempotent; the process-wide device record,
@@ -258,6 +268,14 @@ NVQ_API int32_t nvq_quantized_matmul_static(const nvq_qmm_desc *desc, const void
  * walks all positions of a head. */
 NVQ_API size_t nvq_quantized_attention_workspace_bytes(const nvq_attention_desc *desc);
 NVQ_API int32_t nvq_quantized_attention(const nvq_attention_desc *desc, const void *q, const void *k_w, const void *k_s,
+                                const void *k_b, const void *v_w, const void *v_s, const void *v_b, const void *sinks,
+                                void *out, void *workspace, void *stream);
+
+/* Several query rows per head: the cache dequantized once into `workspace` (always needed: the size query's bytes), both
+ * products on the matrix cores, scores and softmax in float32 on chip.  Keys, values and the softmax's weights are rounded
+ * to the element type before their products, as the composition rounds them. */
+NVQ_API size_t nvq_quantized_attention_prompt_workspace_bytes(const nvq_attention_prompt_desc *desc);
+NVQ_API int32_t nvq_quantized_attention_prompt(const nvq_attention_prompt_desc *desc, const void *q, const void *k_w, const void *k_s,
                                 const void *k_b, const void *v_w, const void *v_s, const void *v_b, const void *sinks,
                                 void *out, void *workspace, void *stream);
 

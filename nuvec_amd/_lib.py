@@ -60,6 +60,10 @@ class AttentionDescC(C.Structure):
                 ("scale", C.c_float)]
 
 
+class AttentionPromptDescC(C.Structure):
+    _fields_ = [("cache", AttentionDescC), ("queries", C.c_int64), ("causal", C.c_int32)]
+
+
 class GluDescC(C.Structure):
     _fields_ = [("dtype", C.c_int32), ("activation", C.c_int32), ("alpha", C.c_float), ("limit", C.c_float),
                 ("rows", C.c_int64), ("hidden", C.c_int64), ("gate_stride", C.c_int64), ("up_stride", C.c_int64),
@@ -97,6 +101,8 @@ SIGNATURES = {
     "nvq_quantized_matmul_route": (C.c_char_p, [C.POINTER(QmmDescC)]),
     "nvq_quantized_attention_workspace_bytes": (C.c_size_t, [C.POINTER(AttentionDescC)]),
     "nvq_quantized_attention": (C.c_int32, [C.POINTER(AttentionDescC)] + [C.c_void_p] * 11),
+    "nvq_quantized_attention_prompt_workspace_bytes": (C.c_size_t, [C.POINTER(AttentionPromptDescC)]),
+    "nvq_quantized_attention_prompt": (C.c_int32, [C.POINTER(AttentionPromptDescC)] + [C.c_void_p] * 11),
     "nvq_sorted_offsets": (C.c_int32, [C.c_void_p, C.c_int64, C.c_int64, C.c_int32, C.c_void_p, C.c_void_p]),
     "nvq_quantize_scaled": (C.c_int32, [C.c_void_p, C.c_int32, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),
     "nvq_dequantize_scaled": (C.c_int32, [C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p]),

@@ -351,13 +351,13 @@ PyObject *py_embedding(PyObject *, PyObject *const *args, Py_ssize_t n) {
     });
 }
 
-// attention(q, k weight, scales, biases, v weight, scales, biases, quant, scale, sinks): one query row per head
-// (ops.quantized_attention, ops.quantized_attention_fits)
+// attention(q, k weight, scales, biases, v weight, scales, biases, quant, scale, sinks, causal)
+// (ops.quantized_attention, ops.quantized_attention_fits for one query row per head; ops.quantized_attention_prompt)
 PyObject *py_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
     return guarded([&]() -> PyObject * {
         Tensor q, sinks;
         Packed k, v;
-        if (n != 10 || !as_tensor(args[0], q) || !as_tensor(args[1], k.w) || !as_tensor(args[2], k.s) || !as_tensor(args[3], k.b) ||
+        if (n != 11 || !as_tensor(args[0], q) || !as_tensor(args[1], k.w) || !as_tensor(args[2], k.s) || !as_tensor(args[3], k.b) ||
             !as_tensor(args[4], v.w) || !as_tensor(args[5], v.s) || !as_tensor(args[6], v.b) || !read_quant(args[7], k.q) ||
             !as_tensor(args[9], sinks))
             return none();
@@ -369,7 +369,7 @@ PyObject *py_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
         }
         const Place at(q);
         int64_t dim, same;
-        if (!at.usable() || q.dim() != 4 || q.size(2) != 1 || q.numel() == 0 || !q.is_contiguous() || k.q.mode != NVQ_AFFINE) return none();
+        if (!at.usable() || q.dim() != 4 || q.numel() == 0 || !q.is_contiguous() || k.q.mode != NVQ_AFFINE) return none();
         const at::ScalarType type = q.scalar_type();
         const int32_t code = code_of(type);
         if (code < 0 || !k.fits(at, type, 4, dim) || !v.fits(at, type, 4, same) || dim != q.size(3) || same != dim ||
@@ -377,8 +377,19 @@ PyObject *py_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
             !bias_fits(sinks, at, type, q.size(1)))
             return none();
         const nvq_attention_desc d{code, k.q.bits, k.q.group_size, (int32_t)dim, q.size(0), q.size(1), k.w.size(1), k.w.size(2), (float)scale};
-        const size_t need = nvq_quantized_attention_workspace_bytes(&d);
         Tensor workspace, y = at.empty(q.sizes(), type);
+        if (q.size(2) > 1) {
+            const int causal = PyObject_IsTrue(args[10]);
+            if (causal < 0) return nullptr;
+            const nvq_attention_prompt_desc p{d, q.size(2), causal};
+            const size_t bytes = nvq_quantized_attention_prompt_workspace_bytes(&p);
+            if (bytes == 0) return none();
+            workspace = at.empty({(int64_t)bytes}, at::kByte);
+            const bool done = nvq_quantized_attention_prompt(&p, ptr(q), ptr(k.w), ptr(k.s), ptr(k.b), ptr(v.w), ptr(v.s), ptr(v.b), ptr(sinks),
+                                                             y.mutable_data_ptr(), workspace.mutable_data_ptr(), at.stream()) == NVQ_OK;
+            return wrap(done, y);
+        }
+        const size_t need = nvq_quantized_attention_workspace_bytes(&d);
         if (need > 0) workspace = at.empty({(int64_t)need}, at::kByte);
         const bool done = nvq_quantized_attention(&d, ptr(q), ptr(k.w), ptr(k.s), ptr(k.b), ptr(v.w), ptr(v.s), ptr(v.b), ptr(sinks),
                                                   y.mutable_data_ptr(), need > 0 ? workspace.mutable_data_ptr() : nullptr, at.stream()) == NVQ_OK;

@@ -792,6 +792,49 @@ int32_t nvq_quantized_attention(const nvq_attention_desc *d, const void *q, cons
     return launch_quantized_attention(*d, q, k_w, k_s, k_b, v_w, v_s, v_b, sinks, out, workspace, (hipStream_t)stream);
 }
 
+static int32_t check_attention_prompt(const nvq_attention_prompt_desc *p) {
+    const char *op = "quantized_attention";
+    if (p == nullptr) return fail(NVQ_INVALID_ARGUMENT, "%s: null descriptor", op);
+    const nvq_attention_desc *d = &p->cache;
+    NVQ_TRY(check_float(op, d->dtype));
+    const nvq_quant quant{NVQ_AFFINE, d->group_size, d->bits};
+    NVQ_TRY(check_quant(&quant, op));
+    if (d->batch < 0 || d->query_heads < 0 || d->key_heads < 0 || d->positions < 0 || d->head_dim < 0 || p->queries < 0)
+        return fail(NVQ_INVALID_ARGUMENT, "%s: negative size", op);
+    if (d->key_heads == 0 || d->query_heads % d->key_heads != 0)
+        return fail(NVQ_INVALID_ARGUMENT, "%s: %lld query heads over %lld key heads", op, (long long)d->query_heads, (long long)d->key_heads);
+    // 32-bit row, tile and block numbers; heads travel in grid y
+    const int64_t heads = d->batch * d->key_heads;
+    if (d->dtype == NVQ_F32 || (d->head_dim != 64 && d->head_dim != 128) || d->head_dim % d->group_size != 0 || d->positions < 1 ||
+        p->queries < 1 || heads > 65535 || d->positions >= (1LL << 30) || p->queries * d->query_heads >= (1LL << 30) ||
+        heads * d->positions >= (1LL << 31) || p->queries * d->query_heads * d->batch >= (1LL << 31))
+        return fail(NVQ_UNSUPPORTED, "%s: several query rows take half-precision types and head sizes 64 and 128", op);
+    return NVQ_OK;
+}
+
+size_t nvq_quantized_attention_prompt_workspace_bytes(const nvq_attention_prompt_desc *p) {
+    if (check_attention_prompt(p) != NVQ_OK || require_device() != NVQ_OK) return 0;
+    return attention_prompt_workspace_bytes(*p);
+}
+
+int32_t nvq_quantized_attention_prompt(const nvq_attention_prompt_desc *p, const void *q, const void *k_w, const void *k_s, const void *k_b,
+                                       const void *v_w, const void *v_s, const void *v_b, const void *sinks, void *out, void *workspace,
+                                       void *stream) {
+    const char *op = "quantized_attention";
+    NVQ_TRY(check_attention_prompt(p));
+    if (p->cache.batch == 0 || p->cache.query_heads == 0) return NVQ_OK;
+    if (q == nullptr || k_w == nullptr || k_s == nullptr || k_b == nullptr || v_w == nullptr || v_s == nullptr || v_b == nullptr ||
+        out == nullptr || workspace == nullptr)
+        return fail(NVQ_INVALID_ARGUMENT, "%s: null operand", op);
+    NVQ_TRY(require_device());
+    NVQ_TRY(check_aligned(op, "queries", q));
+    NVQ_TRY(check_aligned(op, "keys", k_w, 4));
+    NVQ_TRY(check_aligned(op, "values", v_w, 4));
+    NVQ_TRY(check_aligned(op, "out", out));
+    NVQ_TRY(check_aligned(op, "workspace", workspace));
+    return launch_attention_prompt(*p, q, k_w, k_s, k_b, v_w, v_s, v_b, sinks, out, workspace, (hipStream_t)stream);
+}
+
 int32_t nvq_sorted_offsets(const uint32_t *indices, int64_t rows, int64_t m, int32_t groups, int32_t *offsets, void *stream) {
     if (rows < 0 || m < 0 || groups < 0) return fail(NVQ_INVALID_ARGUMENT, "sorted_offsets: negative size");
     if (rows == 0 || groups == 0) return NVQ_OK;

@@ -1,0 +1,372 @@
+// Attention of several query rows per head over an affine-quantized key / value cache on the gfx950 matrix cores: the
+// prompt's side of the reference's `quantized_attention` (crates/nuvec-core/src/fast/imp.rs:3996-4035, the composition of two
+// quantized products and a softmax; nuvec-lm's causal mask, crates/nuvec-lm/src/model.rs:3646-3700):
+//     out[b, h, i, :] = softmax(scale * q[b, h, i, :] . K[b, h / rep]^T [masked] [, sink[h]]) . V[b, h / rep]
+// with the scores and the softmax in float32 and never in memory; keys, values and the softmax's weights are rounded to the
+// element type before their products, as the composition rounds them.
+//
+// Two kernels.  The first dequantizes the cache once into a workspace (a cache of 2048 positions x 8 heads is 8 MB there, and
+// stays in the chip's caches; every tile of query rows reads all of it), laid out as the operands of the matrix instruction:
+// a wavefront's load is 1 KB of consecutive bytes and no kernel transposes anything.  The second walks it with an online
+// softmax.
+//
+// The rows of a key head are its rep x L query rows (row r: query r / rep, head r % rep), so that grouped heads and a few
+// queries share tiles.  A wavefront owns 32 rows and forms the scores transposed, S^T = K . Q^T with v_mfma_32x32x16: a lane
+// then holds 16 of 32 keys of ONE row, its maximum and sum are in-lane but for one exchange, and the weights are already the
+// operand of O^T = V^T . P^T - the contraction's order is free, so V's keys are stored in the order the lanes hold them (lane
+// half h has keys 4 h + {0..3} and 8 + 4 h + {0..3} of sixteen).
+//
+// What fills the chip: few rows are walked by several wavefronts of a block, each taking every KP-th tile of keys, and where
+// even that leaves compute units idle by several blocks whose float32 states a third kernel merges.
+#include "nvq_device.h"
+#include "nvq_internal.h"
+#include "qmf_kernel.h"
+
+namespace nvq {
+namespace {
+
+using qmf::floatx16_t;
+using qmf::Ops;
+
+constexpr int kKeys = 32;       // keys of a tile
+constexpr int kRows = 32;       // rows of a wavefront
+constexpr int kWaves = 4;       // wavefronts of a block: row groups x parts of the keys
+constexpr float kLog2e = 1.44269504088896340736f;
+
+struct PromptArgs {
+    const void *q;
+    const uint4 *keys, *values;  // operands, [batch x key_heads][tiles][D / 16 x 64] each
+    const void *sinks;
+    void *out;
+    float *partials;             // [splits][heads x queries][D + 2] or NULL
+    float scale;
+    int32_t causal;
+    int32_t query_heads, key_heads, rep, queries, positions;
+    int32_t tiles, row_tiles, splits;
+};
+
+// Codes d0 .. d0 + 7 of a row (BITS bytes at byte d0 / 8 x BITS of its dwords) as the values `dequantize` gives them.
+template <typename T, int BITS>
+__device__ __forceinline__ uint4 dequantize_eight(const uint32_t *row, int words, int d0, float s, float b) {
+    const int byte = d0 / 8 * BITS, w = byte >> 2, sh = 8 * (byte & 3);
+    uint64_t v = row[w];
+    if constexpr (BITS > 1) v |= (uint64_t)row[w + 1 < words ? w + 1 : w] << 32;
+    const uint64_t codes = v >> sh;  // (BITS bytes from byte 0 .. 3 of a word: they end in the second one)
+    uint32_t p[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        p[i] = qmf::affine_pair<T, true>((float)(uint32_t)((codes >> (2 * i * BITS)) & ((1u << BITS) - 1u)),
+                                         (float)(uint32_t)((codes >> ((2 * i + 1) * BITS)) & ((1u << BITS) - 1u)), s, b);
+    return make_uint4(p[0], p[1], p[2], p[3]);
+}
+
+// Block: one tile of 32 keys of one (batch, key head).  Bound by its reads of the codes; positions past the end are zeros.
+template <typename T, int BITS, int D>
+__global__ void __launch_bounds__(256) prompt_operands_kernel(const uint32_t *__restrict__ kw, const T *__restrict__ ks, const T *__restrict__ kb,
+                                                             const uint32_t *__restrict__ vw, const T *__restrict__ vs, const T *__restrict__ vb,
+                                                             int positions, int group_shift, uint4 *__restrict__ keys, uint4 *__restrict__ values) {
+    constexpr int kChunks = kKeys * D / 8, words = D * BITS / 32;
+    __shared__ __align__(16) uint16_t tile[kKeys][D + 8];
+    const int64_t head = blockIdx.y, base = (head * gridDim.x + blockIdx.x) * kChunks;
+    const int groups = D >> group_shift, s0 = blockIdx.x * kKeys;
+    const int64_t row0 = head * positions;
+    for (int c = threadIdx.x; c < kChunks; c += 256) {
+        const int key = c & 31, d0 = (c >> 5) * 8;  // (chunk (step << 6 | half << 5 | key): values 16 step + 8 half ..)
+        uint4 k = make_uint4(0, 0, 0, 0), v = k;
+        if (s0 + key < positions) {
+            const int64_t row = row0 + s0 + key, g = row * groups + (d0 >> group_shift);
+            k = dequantize_eight<T, BITS>(kw + row * words, words, d0, Elem<T>::load(ks, g), Elem<T>::load(kb, g));
+            v = dequantize_eight<T, BITS>(vw + row * words, words, d0, Elem<T>::load(vs, g), Elem<T>::load(vb, g));
+        }
+        keys[base + c] = k;
+        *reinterpret_cast<uint4 *>(&tile[key][d0]) = v;
+    }
+    __syncthreads();
+    for (int c = threadIdx.x; c < kChunks; c += 256) {
+        const int lane = c & 63, h = lane >> 5, block = c >> 6;  // block: which sixteen keys x which 32 values of D
+        const int s = block / (D / 32) * 16 + 4 * h, d = block % (D / 32) * 32 + (lane & 31);
+        uint32_t p[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int key = s + (j < 2 ? 2 * j : 8 + 2 * (j - 2));
+            p[j] = (uint32_t)tile[key][d] | (uint32_t)tile[key + 1][d] << 16;
+        }
+        values[base + c] = make_uint4(p[0], p[1], p[2], p[3]);
+    }
+}
+
+// RG row groups of 32 rows a block, 4 / RG wavefronts on each: two wavefronts a SIMD hold 64 accumulators, the query's 32
+// operand registers and one tile of keys and values in flight (D = 128).
+template <typename T, int D, int RG>
+__global__ void __launch_bounds__(64 * kWaves, 2) prompt_attention_kernel(const PromptArgs a) {
+    constexpr int KP = kWaves / RG, KS = D / 16, DB = D / 32;
+    constexpr int kChunks = kKeys * D / 8;
+    constexpr int kStride = D + 4;  // floats of a row of partial outputs: 16-byte aligned, banks shifted row by row
+    __shared__ __align__(16) float merge[KP > 1 ? kWaves * kRows * kStride : 4];
+    __shared__ float state_m[kWaves][kRows], state_l[kWaves][kRows];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 31, half = lane >> 5;
+    const int rg = wave / KP, kp = wave % KP;
+    // blocks of one key head lie `heads` apart: on one XCD, whose L2 then holds that head's keys, where heads is a multiple of 8
+    const int heads = gridDim.x / ((a.row_tiles + RG - 1) / RG);
+    const int head = blockIdx.x % heads, b = head / a.key_heads, hk = head % a.key_heads;
+    const int block_tile = (a.row_tiles + RG - 1) / RG - 1 - blockIdx.x / heads;  // (the longest rows of a causal product first)
+    const int rows = a.rep * a.queries, r0 = (block_tile * RG + rg) * kRows, r = r0 + col;
+    const bool live = r < rows;
+    const int i = live ? r / a.rep : a.queries - 1, h = live ? hk * a.rep + r % a.rep : hk * a.rep;
+    const int64_t row = ((int64_t)b * a.query_heads + h) * a.queries + i;
+    // the last key a row sees, the last one any and the last one all of this wavefront's rows see
+    const int last = a.causal ? a.positions - a.queries + i : a.positions - 1;
+    const int any_i = (r0 + kRows - 1 < rows ? r0 + kRows - 1 : rows - 1) / a.rep, all_i = (r0 < rows ? r0 : rows - 1) / a.rep;
+    const int any_last = a.causal ? a.positions - a.queries + any_i : a.positions - 1;
+    const int all_last = a.causal ? a.positions - a.queries + all_i : a.positions - 1;
+
+    uint4 qf[KS];
+#pragma unroll
+    for (int s = 0; s < KS; s++) qf[s] = *reinterpret_cast<const uint4 *>((const T *)a.q + row * D + 16 * s + 8 * half);
+    floatx16_t o[DB];
+#pragma unroll
+    for (int d = 0; d < DB; d++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) o[d][e] = 0.0f;
+    float m = -1.0e30f, l = 0.0f;  // (finite: a masked score's weight is exp2(-inf - m) = 0 from the first tile on)
+    const float scale = a.scale * kLog2e;
+
+    const int per = (a.tiles + a.splits - 1) / a.splits, t_begin = blockIdx.y * per;
+    int t_end = t_begin + per < a.tiles ? t_begin + per : a.tiles;
+    if (any_last / kKeys + 1 < t_end) t_end = any_last < 0 ? 0 : any_last / kKeys + 1;
+    if (r0 >= rows) t_end = 0;  // (a row group past the end)
+    const uint4 *kf = a.keys + (int64_t)head * a.tiles * kChunks + lane, *vf = a.values + (int64_t)head * a.tiles * kChunks + lane;
+    uint4 kt[KS], vt[KS];
+    auto fetch = [&](const uint4 *from, int t, uint4 (&to)[KS]) {
+        const uint4 *p = from + (int64_t)(t < a.tiles ? t : a.tiles - 1) * kChunks;  // (past the end: read, not used)
+#pragma unroll
+        for (int s = 0; s < KS; s++) to[s] = p[64 * s];
+    };
+    fetch(kf, t_begin + kp, kt);
+    fetch(vf, t_begin + kp, vt);
+    for (int t = t_begin + kp; t < t_end; t += KP) {
+        floatx16_t s;
+#pragma unroll
+        for (int e = 0; e < 16; e++) s[e] = 0.0f;
+#pragma unroll
+        for (int k = 0; k < KS; k++) s = Ops<T>::mfma(kt[k], qf[k], s);
+        fetch(kf, t + KP, kt);
+        const int key0 = t * kKeys + 4 * half;  // register e: key 8 (e / 4) + 4 half + e % 4
+        if (t * kKeys + kKeys - 1 > all_last) {
+#pragma unroll
+            for (int e = 0; e < 16; e++) s[e] = key0 + 8 * (e >> 2) + (e & 3) <= last ? s[e] * scale : -INFINITY;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 16; e++) s[e] *= scale;
+        }
+        float top = s[0];
+#pragma unroll
+        for (int e = 1; e < 16; e++) top = fmaxf(top, s[e]);
+        top = fmaxf(top, __shfl_xor(top, 32));
+        // The accumulators are rescaled only when a maximum has grown by more than 2^8: until then the weights are at most
+        // 2^8 and their sums stay exact to the same relative error (float32 sums; bfloat16 and float16 hold 2^8).
+        if (__any(top > m + 8.0f)) {
+            const float m_new = fmaxf(m, top), f = exp2f(m - m_new);
+            m = m_new, l *= f;
+#pragma unroll
+            for (int d = 0; d < DB; d++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) o[d][e] *= f;
+        }
+#pragma unroll
+        for (int e = 0; e < 16; e++) s[e] = __builtin_amdgcn_exp2f(s[e] - m);
+#pragma unroll
+        for (int e = 0; e < 16; e++) l += s[e];
+        uint4 p[2];
+#pragma unroll
+        for (int k = 0; k < 2; k++)
+            p[k] = make_uint4(Ops<T>::pack(s[8 * k], s[8 * k + 1]), Ops<T>::pack(s[8 * k + 2], s[8 * k + 3]),
+                              Ops<T>::pack(s[8 * k + 4], s[8 * k + 5]), Ops<T>::pack(s[8 * k + 6], s[8 * k + 7]));
+#pragma unroll
+        for (int k = 0; k < 2; k++)
+#pragma unroll
+            for (int d = 0; d < DB; d++) o[d] = Ops<T>::mfma(vt[k * DB + d], p[k], o[d]);
+        fetch(vf, t + KP, vt);
+    }
+    l += __shfl_xor(l, 32);
+
+    // the wavefronts of a row group: their states brought to one maximum and added up
+    if (KP > 1) {
+        if (half == 0) state_m[wave][col] = m, state_l[wave][col] = l;
+        __syncthreads();
+        float top = -1.0e30f, sum = 0.0f;
+#pragma unroll
+        for (int k = 0; k < KP; k++) top = fmaxf(top, state_m[rg * KP + k][col]);
+#pragma unroll
+        for (int k = 0; k < KP; k++) sum += state_l[rg * KP + k][col] * exp2f(state_m[rg * KP + k][col] - top);
+        const float f = exp2f(m - top);
+        float *mine = merge + (wave * kRows + col) * kStride;
+#pragma unroll
+        for (int d = 0; d < DB; d++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                *reinterpret_cast<float4 *>(mine + 32 * d + 8 * e + 4 * half) =
+                    make_float4(o[d][4 * e] * f, o[d][4 * e + 1] * f, o[d][4 * e + 2] * f, o[d][4 * e + 3] * f);
+        m = top, l = sum;
+        __syncthreads();
+    }
+    const bool whole = a.splits == 1;
+    float inv = 1.0f;
+    float *state = nullptr;  // of this row and split: maximum, denominator, weighted sums
+    if (whole) {
+        float denom = l, f = 1.0f;
+        if (a.sinks != nullptr) {
+            const float sink = Elem<T>::load((const T *)a.sinks, h) * kLog2e, top = fmaxf(m, sink);
+            f = exp2f(m - top), denom = denom * f + exp2f(sink - top);
+        }
+        inv = f / denom;
+    } else {
+        state = a.partials + (((int64_t)blockIdx.y * heads + head) * rows + (live ? r : 0)) * (D + 2);
+        if (live && kp == 0 && half == 0) state[0] = m, state[1] = l;
+    }
+    T *out = (T *)a.out + row * D;
+#pragma unroll
+    for (int d = 0; d < DB; d++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            if (KP > 1 && (4 * d + e) % KP != kp) continue;
+            const int c = 32 * d + 8 * e + 4 * half;
+            float4 v;
+            if (KP > 1) {
+                v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+                for (int k = 0; k < KP; k++) {
+                    const float4 w = *reinterpret_cast<const float4 *>(merge + ((rg * KP + k) * kRows + col) * kStride + c);
+                    v.x += w.x, v.y += w.y, v.z += w.z, v.w += w.w;
+                }
+            } else {
+                v = make_float4(o[d][4 * e], o[d][4 * e + 1], o[d][4 * e + 2], o[d][4 * e + 3]);
+            }
+            if (!live) continue;
+            if (whole) {
+                *reinterpret_cast<uint2 *>(out + c) = make_uint2(Ops<T>::pack(v.x * inv, v.y * inv), Ops<T>::pack(v.z * inv, v.w * inv));
+            } else {
+                *reinterpret_cast<float2 *>(state + 2 + c) = make_float2(v.x, v.y);
+                *reinterpret_cast<float2 *>(state + 4 + c) = make_float2(v.z, v.w);
+            }
+        }
+}
+
+// The splits of a row merged: block = D threads, one row.
+template <typename T, int D>
+__global__ void __launch_bounds__(D) prompt_merge_kernel(const PromptArgs a) {
+    const int rows = a.rep * a.queries;
+    const int64_t all = (int64_t)gridDim.x * gridDim.y;  // rows x (batch x key heads)
+    const int r = blockIdx.x, head = blockIdx.y, b = head / a.key_heads, hk = head % a.key_heads;
+    const float *src = a.partials + ((int64_t)head * rows + r) * (D + 2);
+    float top = -1.0e30f;
+    for (int z = 0; z < a.splits; z++) top = fmaxf(top, src[z * all * (D + 2)]);
+    const int h = hk * a.rep + r % a.rep, i = r / a.rep;
+    const bool has_sink = a.sinks != nullptr;
+    const float sink = has_sink ? Elem<T>::load((const T *)a.sinks, h) * kLog2e : 0.0f;
+    if (has_sink) top = fmaxf(top, sink);
+    float denom = has_sink ? exp2f(sink - top) : 0.0f, sum = 0.0f;
+    for (int z = 0; z < a.splits; z++) {
+        const float *p = src + z * all * (D + 2), w = exp2f(p[0] - top);
+        denom = __builtin_fmaf(p[1], w, denom);
+        sum = __builtin_fmaf(p[2 + threadIdx.x], w, sum);
+    }
+    Elem<T>::store((T *)a.out, (((int64_t)b * a.query_heads + h) * a.queries + i) * D + threadIdx.x, sum / denom);
+}
+
+struct Plan {
+    int tiles, row_tiles, row_groups, splits;
+    int64_t heads, rows;
+    size_t operand_bytes, partial_bytes;
+};
+
+// Row groups a block: four (every tile of keys read once per 128 rows) where that gives two blocks per compute unit, else two,
+// else one (four wavefronts on the same 32 rows); then, with fewer blocks than compute units still, splits of the keys over the
+// grid of at least eight tiles each.
+Plan prompt_plan(const nvq_attention_prompt_desc &p) {
+    const nvq_attention_desc &d = p.cache;
+    Plan r{};
+    r.heads = d.batch * d.key_heads;
+    r.rows = d.query_heads / d.key_heads * p.queries;
+    r.tiles = (int)((d.positions + kKeys - 1) / kKeys);
+    r.row_tiles = (int)((r.rows + kRows - 1) / kRows);
+    const int64_t cus = compute_units();
+    r.row_groups = 1;
+    for (int g = 4; g > 1; g /= 2)
+        if (r.heads * ((r.row_tiles + g - 1) / g) >= 2 * cus) {
+            r.row_groups = g;
+            break;
+        }
+    r.splits = 1;
+    const int64_t blocks = r.heads * r.row_tiles;
+    if (r.row_groups == 1 && blocks < cus) {
+        int64_t want = (2 * cus + blocks - 1) / blocks;
+        if (want > r.tiles / 8) want = r.tiles / 8;
+        if (want > 32) want = 32;
+        if (want > 1) {
+            const int64_t per = (r.tiles + want - 1) / want;
+            r.splits = (int)((r.tiles + per - 1) / per);
+        }
+    }
+    r.operand_bytes = (size_t)r.heads * r.tiles * kKeys * d.head_dim * 2;
+    r.partial_bytes = r.splits > 1 ? (size_t)r.splits * r.heads * r.rows * (d.head_dim + 2) * sizeof(float) : 0;
+    return r;
+}
+
+template <typename T, int D, int RG>
+int32_t run_rows(const PromptArgs &a, const Plan &p, hipStream_t s) {
+    const int64_t blocks = p.heads * ((p.row_tiles + RG - 1) / RG);
+    hipLaunchKernelGGL((prompt_attention_kernel<T, D, RG>), dim3((unsigned)blocks, (unsigned)p.splits), dim3(64 * kWaves), 0, s, a);
+    NVQ_LAUNCH_CHECK("quantized_attention");
+    if (p.splits > 1) {
+        hipLaunchKernelGGL((prompt_merge_kernel<T, D>), dim3((unsigned)p.rows, (unsigned)p.heads), dim3(D), 0, s, a);
+        NVQ_LAUNCH_CHECK("quantized_attention merge");
+    }
+    return NVQ_OK;
+}
+
+template <typename T, int D>
+int32_t run_sized(const nvq_attention_prompt_desc &desc, const void *q, const void *kw, const void *ks, const void *kb, const void *vw,
+                  const void *vs, const void *vb, const void *sinks, void *out, void *workspace, hipStream_t s) {
+    const nvq_attention_desc &d = desc.cache;
+    const Plan p = prompt_plan(desc);
+    uint4 *keys = (uint4 *)workspace, *values = keys + p.operand_bytes / 16;
+    int shift = 5;
+    while ((1 << shift) < d.group_size) shift++;
+    const dim3 grid((unsigned)p.tiles, (unsigned)p.heads);
+#define NVQ_OPERANDS(B)                                                                                                                  \
+    case B:                                                                                                                              \
+        hipLaunchKernelGGL((prompt_operands_kernel<T, B, D>), grid, dim3(256), 0, s, (const uint32_t *)kw, (const T *)ks, (const T *)kb, \
+                           (const uint32_t *)vw, (const T *)vs, (const T *)vb, (int)d.positions, shift, keys, values);                    \
+        break;
+    switch (d.bits) { NVQ_OPERANDS(1) NVQ_OPERANDS(2) NVQ_OPERANDS(3) NVQ_OPERANDS(4) NVQ_OPERANDS(5) NVQ_OPERANDS(6) NVQ_OPERANDS(8) }
+#undef NVQ_OPERANDS
+    NVQ_LAUNCH_CHECK("quantized_attention operands");
+    PromptArgs a{};
+    a.q = q, a.keys = keys, a.values = values, a.sinks = sinks, a.out = out;
+    a.partials = (float *)((char *)workspace + 2 * p.operand_bytes);
+    a.scale = d.scale, a.causal = desc.causal;
+    a.query_heads = (int)d.query_heads, a.key_heads = (int)d.key_heads, a.rep = (int)(d.query_heads / d.key_heads);
+    a.queries = (int)desc.queries, a.positions = (int)d.positions;
+    a.tiles = p.tiles, a.row_tiles = p.row_tiles, a.splits = p.splits;
+    return p.row_groups == 4 ? run_rows<T, D, 4>(a, p, s) : p.row_groups == 2 ? run_rows<T, D, 2>(a, p, s) : run_rows<T, D, 1>(a, p, s);
+}
+
+}  // namespace
+
+size_t attention_prompt_workspace_bytes(const nvq_attention_prompt_desc &d) {
+    const Plan p = prompt_plan(d);
+    return 2 * p.operand_bytes + p.partial_bytes;
+}
+
+int32_t launch_attention_prompt(const nvq_attention_prompt_desc &d, const void *q, const void *kw, const void *ks, const void *kb,
+                                const void *vw, const void *vs, const void *vb, const void *sinks, void *out, void *workspace, hipStream_t s) {
+    if (d.cache.dtype == NVQ_BF16)
+        return d.cache.head_dim == 64 ? run_sized<bf16_t, 64>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s)
+                                      : run_sized<bf16_t, 128>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s);
+    return d.cache.head_dim == 64 ? run_sized<f16_t, 64>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s)
+                                  : run_sized<f16_t, 128>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s);
+}
+
+}  // namespace nvq

@@ -329,28 +329,33 @@ def quantized_attention(q: torch.Tensor, k: ops.Quantized, v: ops.Quantized, sca
     biases `[B, Hkv, S, D / group]`), grouped query heads, optional per-head `sinks [Hq]`, optionally causal (query i
     of L sees keys up to S - L + i, nuvec-lm's `quantized_attention`, model.rs:3646-3700):
     `softmax(scale * q k^T [, sinks]) v`.  One query row per head that fits the kernel (head size 64 or 128, 3, 4 or 8 bits)
-    takes the library's fused kernel; the rest is the reference's composition (the one it runs wherever its fused
-    kernel does not fit): both products are the library's quantized products, transposed for the keys and
-    untransposed for the values; the softmax (float32 inside, one rounding) is an elementwise step outside the path."""
+    takes the library's fused kernel, several rows in half precision its kernels on the matrix cores; the rest is the
+    reference's composition (the one it runs wherever its fused kernel does not fit): both products are the library's
+    quantized products, transposed for the keys and untransposed for the values, the query heads of a key head as rows of
+    one product; the softmax (float32 inside, one rounding) is an elementwise step outside the path."""
     if k.quant != v.quant or k.quant.mode != ops.QuantMode.AFFINE:
         raise ops.InvalidArgument("quantized_attention: keys and values need one affine quantization")
     if k.biases is None or v.biases is None:
         raise ops.InvalidArgument("quantized_attention: affine biases missing")
-    if fused and q.ndim == 4 and q.shape[2] == 1:  # the plain case of the branch below
-        out = (_native or _calls()).attention(q, k.weight, k.scales, k.biases, v.weight, v.scales, v.biases, k.quant, scale, sinks)
+    if fused:  # the plain case of the branches below
+        out = (_native or _calls()).attention(q, k.weight, k.scales, k.biases, v.weight, v.scales, v.biases, k.quant, scale, sinks, causal)
         if out is not None:
             return out
     # (a single causal query row sees every key: the mask is empty)
     if fused and (not causal or q.shape[-2] == 1) and q.is_cuda and ops.quantized_attention_fits(q, k, v, sinks):
         return ops.quantized_attention(q, k, v, scale, sinks)  # one kernel (the reference's FastOp::QuantizedAttention)
+    if fused and q.is_cuda and q.ndim == 4 and q.shape[2] > 1 and q.shape[3] in (64, 128) and q.dtype != torch.float32:
+        try:  # several rows: both products and the softmax on the matrix cores
+            return ops.quantized_attention_prompt(q, k, v, scale, sinks, causal)
+        except ops.Unsupported:
+            pass
     b, hq, l, d = q.shape
     hkv = k.weight.shape[1]
     if hq % hkv != 0:
         raise ops.InvalidArgument(f"quantized_attention: {hq} query heads over {hkv} key heads")
     rep = hq // hkv
-    qs = (q * scale).reshape(b, hkv, rep, l, d)
-    expand = lambda t: ops.Quantized(t.weight.unsqueeze(-3), t.scales.unsqueeze(-3), t.biases.unsqueeze(-3), t.quant)
-    scores = ops.quantized_matmul(qs, expand(k), True)  # [B, Hkv, rep, L, S]
+    qs = (q * scale).reshape(b, hkv, rep * l, d)
+    scores = ops.quantized_matmul(qs, k, True).reshape(b, hkv, rep, l, -1)  # [B, Hkv, rep, L, S]
     s = scores.shape[-1]
     if causal and l > 1:
         hidden = torch.arange(s, device=q.device)[None, :] > (s - l + torch.arange(l, device=q.device))[:, None]
@@ -360,5 +365,5 @@ def quantized_attention(q: torch.Tensor, k: ops.Quantized, v: ops.Quantized, sca
         probs = torch.softmax(torch.cat([scores, column], dim=-1).float(), dim=-1).to(scores.dtype)[..., :s]
     else:
         probs = torch.softmax(scores.float(), dim=-1).to(scores.dtype)
-    out = ops.quantized_matmul(probs.contiguous(), expand(v), False)  # [B, Hkv, rep, L, D]
+    out = ops.quantized_matmul(probs.reshape(b, hkv, rep * l, s), v, False)  # [B, Hkv, rep L, D]
     return out.reshape(b, hq, l, d)

@@ -506,7 +506,7 @@ def quantized_attention(q: torch.Tensor, k: Quantized, v: Quantized, scale: floa
     """fast.rs:694-718 where the kernel fits (`quantized_attention_fits`): one query row per head over the quantized
     cache in one launch."""
     if scratch and k.quant == v.quant:
-        out = (_lib._native or _lib.native()).attention(q, k.weight, k.scales, k.biases, v.weight, v.scales, v.biases, k.quant, scale, sinks)
+        out = (_lib._native or _lib.native()).attention(q, k.weight, k.scales, k.biases, v.weight, v.scales, v.biases, k.quant, scale, sinks, False)
         if out is not None:
             return out
     if not quantized_attention_fits(q, k, v, sinks):
@@ -524,6 +524,40 @@ def quantized_attention(q: torch.Tensor, k: Quantized, v: Quantized, scale: floa
     workspace = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
     _lib.check(lib.nvq_quantized_attention(C.byref(desc), _ptr(q), _ptr(kw), _ptr(ks), _ptr(kb), _ptr(vw), _ptr(vs), _ptr(vb),
                                            _ptr(sinks), _ptr(out), _ptr(workspace), _stream()))
+    return out
+
+
+def quantized_attention_prompt(q: torch.Tensor, k: Quantized, v: Quantized, scale: float, sinks: Optional[torch.Tensor] = None,
+                               causal: bool = False) -> torch.Tensor:
+    """fast/imp.rs:3996-4035 (the composition the reference runs for several query rows) as two kernels: the cache
+    dequantized once, then both products and the softmax.  Raises `Unsupported` for what they do not take (float32, head
+    sizes other than 64 and 128)."""
+    out = (_lib._native or _lib.native()).attention(q, k.weight, k.scales, k.biases, v.weight, v.scales, v.biases, k.quant, scale, sinks,
+                                                    causal) if k.quant == v.quant else None
+    if out is not None:
+        return out
+    if q.ndim != 4 or k.weight.ndim != 4 or k.quant != v.quant or k.quant.mode != QuantMode.AFFINE:
+        raise Unsupported("quantized_attention: the operands do not fit the kernel")
+    b, hq, l, d = q.shape
+    for t in (k, v):
+        if t.biases is None or t.weight.dtype not in (torch.uint32, torch.int32) or t.scales.dtype != q.dtype or t.biases.dtype != q.dtype \
+                or t.weight.shape[:3] != k.weight.shape[:3] or t.weight.shape[0] != b or t.scales.shape != t.biases.shape \
+                or t.weight.shape[3] * 32 != d * t.quant.bits or tuple(t.scales.shape) != tuple(t.weight.shape[:3]) + (d // t.quant.group_size,):
+            raise Unsupported("quantized_attention: the operands do not fit the kernel")
+    if q.dtype not in _FLOATS or (sinks is not None and (sinks.ndim != 1 or sinks.numel() != hq or sinks.dtype != q.dtype)):
+        raise Unsupported("quantized_attention: the operands do not fit the kernel")
+    _init(q)
+    q = q.contiguous()
+    kw, ks, kb = _u32(k.weight).contiguous(), k.scales.contiguous(), k.biases.contiguous()
+    vw, vs, vb = _u32(v.weight).contiguous(), v.scales.contiguous(), v.biases.contiguous()
+    sinks = None if sinks is None else sinks.contiguous()
+    out = torch.empty_like(q)
+    cache = _lib.AttentionDescC(_CODE[q.dtype], k.quant.bits, k.quant.group_size, d, b, hq, kw.shape[1], kw.shape[2], float(scale))
+    desc = _lib.AttentionPromptDescC(cache, l, int(causal))
+    lib = _lib.load()
+    workspace = torch.empty(lib.nvq_quantized_attention_prompt_workspace_bytes(C.byref(desc)), dtype=torch.uint8, device=q.device)
+    _lib.check(lib.nvq_quantized_attention_prompt(C.byref(desc), _ptr(q), _ptr(kw), _ptr(ks), _ptr(kb), _ptr(vw), _ptr(vs), _ptr(vb),
+                                                  _ptr(sinks), _ptr(out), _ptr(workspace), _stream()))
     return out
 
 

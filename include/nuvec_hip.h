@@ -307,6 +307,10 @@ NVQ_API int32_t nvq_convert_packed(int32_t format, const nvq_quant *quant, int32
  *   sorted_ids u32[pairs] = ids[order];  offsets i32[experts]: where each expert's pairs start. */
 NVQ_API int32_t nvq_moe_order(const uint32_t *ids, int64_t pairs, int32_t experts, uint32_t *order, uint32_t *restore,
                       uint32_t *sorted_ids, int32_t *offsets, void *workspace, void *stream);
+/* The same, and beside it tokens u32[pairs]: the token of each sorted pair where a token's `choices` pairs follow each other
+ * (order / choices): the rows of x that the ordered products read. */
+NVQ_API int32_t nvq_moe_order_tokens(const uint32_t *ids, int64_t pairs, int32_t experts, int32_t choices, uint32_t *order, uint32_t *restore,
+                      uint32_t *sorted_ids, int32_t *offsets, uint32_t *tokens, void *workspace, void *stream);
 /* Bytes of `workspace` (per-chunk counters) with which the ordering of many pairs runs over the whole chip in three
  * launches; 0 for few pairs, and with a NULL workspace one block orders them all. */
 NVQ_API size_t nvq_moe_order_workspace_bytes(int64_t pairs, int32_t experts);
@@ -352,6 +356,14 @@ NVQ_API int32_t nvq_quantize_dequantize(const nvq_quant *quant, int32_t dtype, c
  * divide itself: NVQ_UNSUPPORTED). */
 NVQ_API int32_t nvq_moe_route(int32_t dtype, const void *probs, int64_t rows, int32_t experts, int32_t k, int32_t normalize,
                       uint32_t *indices, void *scores, void *stream);
+/* The router of a mixture-of-experts block (MoeMlp, nuvec-lm/src/model.rs:2218-2272) in one launch: logits x . gate^T rounded
+ * to `dtype`, their softmax (float32 inside, one rounding), nvq_moe_route of it; and per pair p = row * k + j its token
+ * tokens[p] = row and identity[p] = p, the index operands of the gathered products.
+ *   x dtype[rows, dims];  gate dtype[experts, dims];  indices, tokens, identity u32[rows, k];  scores dtype[rows, k].
+ * NVQ_UNSUPPORTED where the product is work for a matrix product of its own (rows x experts x dims beyond 2^26), where rows
+ * are not whole 16-byte runs, and beyond nvq_moe_route's bounds. */
+NVQ_API int32_t nvq_moe_router(int32_t dtype, const void *x, const void *gate, int64_t rows, int32_t dims, int32_t experts, int32_t k,
+                               int32_t normalize, uint32_t *indices, void *scores, uint32_t *tokens, uint32_t *identity, void *stream);
 
 /* fast::weighted_sum (fast/imp.rs:2731-2747; kernel moe.metal:90-118): out[r, c] = sum_j x[r, j, c] * w[r, j], the
  * experts' outputs weighted by the router's scores, every product and addition rounded to `dtype` in the kernel's

@@ -37,7 +37,8 @@ constexpr int kOrderThreads = 1024, kOrderWaves = kOrderThreads / 64;
 // before its own.
 __device__ __forceinline__ void place_chunk(const uint32_t *__restrict__ ids, int64_t pairs, int32_t experts, int64_t chunk,
                                             int32_t *next, int32_t *wave_count, uint32_t *__restrict__ order,
-                                            uint32_t *__restrict__ restore, uint32_t *__restrict__ sorted_ids) {
+                                            uint32_t *__restrict__ restore, uint32_t *__restrict__ sorted_ids,
+                                            uint32_t *__restrict__ tokens, uint32_t choices) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     for (int i = tid; i < kOrderWaves * experts; i += kOrderThreads) wave_count[i] = 0;
     __syncthreads();
@@ -65,6 +66,7 @@ __device__ __forceinline__ void place_chunk(const uint32_t *__restrict__ ids, in
         order[at] = (uint32_t)p;
         restore[p] = at;
         sorted_ids[at] = e;
+        if (tokens != nullptr) tokens[at] = (uint32_t)p / choices;
     }
     __syncthreads();
     for (int ee = tid; ee < experts; ee += kOrderThreads) {
@@ -77,7 +79,8 @@ __device__ __forceinline__ void place_chunk(const uint32_t *__restrict__ ids, in
 
 __global__ void __launch_bounds__(kOrderThreads)
 moe_order_kernel(const uint32_t *__restrict__ ids, int64_t pairs, int32_t experts, uint32_t *__restrict__ order,
-                 uint32_t *__restrict__ restore, uint32_t *__restrict__ sorted_ids, int32_t *__restrict__ offsets) {
+                 uint32_t *__restrict__ restore, uint32_t *__restrict__ sorted_ids, int32_t *__restrict__ offsets,
+                 uint32_t *__restrict__ tokens, uint32_t choices) {
     extern __shared__ int32_t lds_i[];
     int32_t *next = lds_i;                       // [experts]: histogram, then where each expert's next pair goes
     int32_t *wave_count = lds_i + experts;       // [waves][experts]: this chunk's pairs per wavefront and expert
@@ -106,7 +109,7 @@ moe_order_kernel(const uint32_t *__restrict__ ids, int64_t pairs, int32_t expert
         }
     }
     __syncthreads();
-    for (int64_t chunk = 0; chunk < pairs; chunk += kOrderThreads) place_chunk(ids, pairs, experts, chunk, next, wave_count, order, restore, sorted_ids);
+    for (int64_t chunk = 0; chunk < pairs; chunk += kOrderThreads) place_chunk(ids, pairs, experts, chunk, next, wave_count, order, restore, sorted_ids, tokens, choices);
 }
 
 // The same ordering for many pairs, over the whole chip in three steps: every block counts the ids of its chunk of
@@ -165,12 +168,13 @@ moe_scan_kernel(int32_t *__restrict__ counts, int32_t chunks, int32_t experts, i
 
 __global__ void __launch_bounds__(kOrderThreads)
 moe_place_kernel(const uint32_t *__restrict__ ids, int64_t pairs, int32_t experts, const int32_t *__restrict__ starts,
-                 uint32_t *__restrict__ order, uint32_t *__restrict__ restore, uint32_t *__restrict__ sorted_ids) {
+                 uint32_t *__restrict__ order, uint32_t *__restrict__ restore, uint32_t *__restrict__ sorted_ids,
+                 uint32_t *__restrict__ tokens, uint32_t choices) {
     extern __shared__ int32_t lds_i[];
     int32_t *next = lds_i, *wave_count = lds_i + experts;
     for (int e = threadIdx.x; e < experts; e += kOrderThreads) next[e] = starts[(int64_t)blockIdx.x * experts + e];
     __syncthreads();
-    place_chunk(ids, pairs, experts, (int64_t)blockIdx.x * kOrderThreads, next, wave_count, order, restore, sorted_ids);
+    place_chunk(ids, pairs, experts, (int64_t)blockIdx.x * kOrderThreads, next, wave_count, order, restore, sorted_ids, tokens, choices);
 }
 
 // round(a / b) in the element type.  The float32 quotient is correctly rounded and float32 carries more than twice
@@ -191,23 +195,14 @@ template <typename T> __device__ __forceinline__ bool route_less(float a, float 
     return a < b;
 }
 
-// fast::moe_route (crates/nuvec-kernels/src/metal/moe.metal:33-88): per row of `n` probabilities the k largest in
+// fast::moe_route (crates/nuvec-kernels/src/metal/moe.metal:33-88): of one row's `n` probabilities `p` the k largest in
 // the stable ascending order, their values and, with `normalize`, those divided by their sum (summed in the
-// element type, in order).  One block per row, one thread per expert: an expert's position in the sorted row is
-// the number of experts sorting before it.
+// element type, in order).  All threads of the block; an expert's position in the sorted row is the number of experts
+// sorting before it.
 template <typename T>
-__global__ void __launch_bounds__(1024) moe_route_kernel(const T *__restrict__ probs, uint32_t *__restrict__ indices,
-                                                         T *__restrict__ scores, int n, int k, int normalize) {
-    __shared__ float p[1024], top[1024];
-    __shared__ float total;
-    const int e = threadIdx.x;
-    const int64_t row = blockIdx.x;
-    probs += row * n;
-    indices += row * k;
-    scores += row * k;
-    if (e < n) p[e] = Elem<T>::load(probs, e);
-    __syncthreads();
-    if (e < n) {
+__device__ __forceinline__ void route_row(const float *p, float *top, float *total, uint32_t *__restrict__ indices, T *__restrict__ scores,
+                                          int n, int k, int normalize) {
+    for (int e = threadIdx.x; e < n; e += blockDim.x) {
         const float v = p[e];
         int rank = 0;
         for (int j = 0; j < n; j++) {
@@ -222,37 +217,119 @@ __global__ void __launch_bounds__(1024) moe_route_kernel(const T *__restrict__ p
     }
     __syncthreads();
     if (normalize) {
-        if (e == 0) {
+        if (threadIdx.x == 0) {
             float sum = 0.0f;
             for (int j = 0; j < k; j++) sum = Elem<T>::add(top[j], sum);
-            total = sum;
+            *total = sum;
         }
         __syncthreads();
-        if (e < k) Elem<T>::store(scores, e, elem_div<T>(top[e], total));
-    } else if (e < k) {
-        Elem<T>::store(scores, e, top[e]);
     }
+    for (int e = threadIdx.x; e < k; e += blockDim.x) Elem<T>::store(scores, e, normalize ? elem_div<T>(top[e], *total) : top[e]);
+}
+
+// One block per row, one thread per expert.
+template <typename T>
+__global__ void __launch_bounds__(1024) moe_route_kernel(const T *__restrict__ probs, uint32_t *__restrict__ indices,
+                                                         T *__restrict__ scores, int n, int k, int normalize) {
+    __shared__ float p[1024], top[1024], total;
+    const int64_t row = blockIdx.x;
+    for (int e = threadIdx.x; e < n; e += blockDim.x) p[e] = Elem<T>::load(probs + row * n, e);
+    __syncthreads();
+    route_row<T>(p, top, &total, indices + row * k, scores + row * k, n, k, normalize);
+}
+
+// The router of a mixture-of-experts block in one launch (MoeMlp, crates/nuvec-lm/src/model.rs:2218-2272): logits of a token
+// (float32 sums, rounded to the element type), their softmax (float32, rounded once), `moe_route`; and what the gathered
+// products read beside its choices, the token of each pair and the pair's own number.  One block per token, a wavefront per
+// expert in turn: latency is the bound (a token's 32 x 2880 gate is 184 KB from the L2), and the library's product, two
+// conversions, softmax and `moe_route` took 17.6 us of kernels at one token and 36 us at 256.
+template <typename T>
+__global__ void __launch_bounds__(1024) moe_router_kernel(const T *__restrict__ x, const T *__restrict__ gate, int dims, int n, int k, int normalize,
+                                                          uint32_t *__restrict__ indices, T *__restrict__ scores,
+                                                          uint32_t *__restrict__ tokens, uint32_t *__restrict__ identity) {
+    constexpr int V = 16 / sizeof(T);  // values of a 16-byte load
+    __shared__ float p[1024], top[1024], total;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, waves = blockDim.x >> 6;
+    const int64_t row = blockIdx.x;
+    const T *xr = x + row * dims;
+    for (int e = wave; e < n; e += waves) {
+        const T *g = gate + (int64_t)e * dims;
+        float sum = 0.0f;
+#pragma unroll 4
+        for (int c = lane * V; c < dims; c += 64 * V) {
+            T xv[V], gv[V];
+            *reinterpret_cast<uint4 *>(xv) = *reinterpret_cast<const uint4 *>(xr + c);
+            *reinterpret_cast<uint4 *>(gv) = *reinterpret_cast<const uint4 *>(g + c);
+#pragma unroll
+            for (int i = 0; i < V; i++) sum = __builtin_fmaf(Elem<T>::load(xv, i), Elem<T>::load(gv, i), sum);
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+        if (lane == 0) p[e] = Elem<T>::mul(sum, 1.0f);
+    }
+    __syncthreads();
+    if (wave == 0) {
+        float most = -INFINITY, sum = 0.0f;
+        for (int e = lane; e < n; e += 64) most = fmaxf(most, p[e]);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) most = fmaxf(most, __shfl_xor(most, o));
+        for (int e = lane; e < n; e += 64) sum += expf(p[e] - most);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+        for (int e = lane; e < n; e += 64) p[e] = Elem<T>::mul(expf(p[e] - most) / sum, 1.0f);
+    }
+    for (int j = tid; j < k; j += blockDim.x) tokens[row * k + j] = (uint32_t)row, identity[row * k + j] = (uint32_t)(row * k + j);
+    __syncthreads();
+    route_row<T>(p, top, &total, indices + row * k, scores + row * k, n, k, normalize);
 }
 
 // fast::weighted_sum (moe.metal:90-118): out[r, c] = sum over j of x[r, j, c] * w[r, j], every product and every
 // addition rounded to the element type: min(k, 8) partial sums of every min(k, 8)-th product (one partial sum when
-// D = 1), added in order.  One thread per output element.
-template <typename T>
+// D = 1), added in order.  One thread per V consecutive elements of a row (V = 1: rows that are not whole runs of V).
+template <typename T, int V>
 __global__ void __launch_bounds__(256) weighted_sum_kernel(const T *__restrict__ x, const T *__restrict__ w, T *__restrict__ out,
                                                            int64_t rows, int k, int64_t d) {
-    const int64_t at = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    struct __align__(V * sizeof(T)) Run { T v[V]; };
+    const int64_t at = ((int64_t)blockIdx.x * 256 + threadIdx.x) * V;
     if (at >= rows * d) return;
     const int64_t r = at / d, c = at - r * d;
     x += r * k * d + c;
     w += r * k;
-    const int lanes = d == 1 ? 1 : (k < 8 ? k : 8);
-    float sum = 0.0f;
-    for (int y = 0; y < lanes; y++) {
-        float t = 0.0f;
-        for (int j = y; j < k; j += lanes) t = Elem<T>::add(Elem<T>::mul(Elem<T>::load(x, (int64_t)j * d), Elem<T>::load(w, j)), t);
-        sum = y == 0 ? t : Elem<T>::add(t, sum);
+    auto load = [&](int j) { return *reinterpret_cast<const Run *>(x + (int64_t)j * d); };
+    float sum[V];
+    if (k <= 8 && d != 1) {  // a partial sum is one product: all rows requested at once
+        Run run[8];
+        float wj[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) run[j] = load(j < k ? j : k - 1), wj[j] = Elem<T>::load(w, j < k ? j : k - 1);
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            if (j < k)
+#pragma unroll
+                for (int i = 0; i < V; i++) {
+                    const float t = Elem<T>::add(Elem<T>::mul(Elem<T>::load(run[j].v, i), wj[j]), 0.0f);
+                    sum[i] = j == 0 ? t : Elem<T>::add(t, sum[i]);
+                }
+    } else {
+        const int lanes = d == 1 ? 1 : 8;
+        for (int y = 0; y < lanes; y++) {
+            float t[V];
+#pragma unroll
+            for (int i = 0; i < V; i++) t[i] = 0.0f;
+            for (int j = y; j < k; j += lanes) {
+                const Run run = load(j);
+                const float wj = Elem<T>::load(w, j);
+#pragma unroll
+                for (int i = 0; i < V; i++) t[i] = Elem<T>::add(Elem<T>::mul(Elem<T>::load(run.v, i), wj), t[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < V; i++) sum[i] = y == 0 ? t[i] : Elem<T>::add(t[i], sum[i]);
+        }
     }
-    Elem<T>::store(out, at, sum);
+    Run o;
+#pragma unroll
+    for (int i = 0; i < V; i++) Elem<T>::store(o.v, i, sum[i]);
+    *reinterpret_cast<Run *>(out + at) = o;
 }
 
 __global__ void fill_zero_kernel(uint16_t *p, int64_t halves) {
@@ -280,10 +357,10 @@ size_t moe_order_workspace_bytes(int64_t pairs, int32_t experts) {
 }
 
 int32_t launch_moe_order(const uint32_t *ids, int64_t pairs, int32_t experts, uint32_t *order, uint32_t *restore,
-                         uint32_t *sorted_ids, int32_t *offsets, void *workspace, hipStream_t s) {
+                         uint32_t *sorted_ids, int32_t *offsets, uint32_t *tokens, int32_t choices, void *workspace, hipStream_t s) {
     if (workspace == nullptr || pairs <= kOrderOneBlock) {
         hipLaunchKernelGGL(moe_order_kernel, dim3(1), dim3(kOrderThreads), moe_order_lds_bytes(experts), s, ids, pairs, experts, order,
-                           restore, sorted_ids, offsets);
+                           restore, sorted_ids, offsets, tokens, (uint32_t)choices);
         NVQ_LAUNCH_CHECK("moe_order");
         return NVQ_OK;
     }
@@ -294,7 +371,7 @@ int32_t launch_moe_order(const uint32_t *ids, int64_t pairs, int32_t experts, ui
     hipLaunchKernelGGL(moe_scan_kernel, dim3(1), dim3(kOrderThreads), (size_t)experts * sizeof(int32_t), s, counts, (int32_t)chunks, experts, offsets);
     NVQ_LAUNCH_CHECK("moe_order (scan)");
     hipLaunchKernelGGL(moe_place_kernel, dim3(chunks), dim3(kOrderThreads), moe_order_lds_bytes(experts), s, ids, pairs, experts, counts, order,
-                       restore, sorted_ids);
+                       restore, sorted_ids, tokens, (uint32_t)choices);
     NVQ_LAUNCH_CHECK("moe_order (place)");
     return NVQ_OK;
 }
@@ -312,15 +389,38 @@ int32_t launch_moe_route(int32_t dtype, const void *probs, int64_t rows, int32_t
     return NVQ_OK;
 }
 
+template <typename T>
+static void run_weighted_sum(const void *x, const void *w, int64_t rows, int32_t k, int64_t d, void *out, hipStream_t s) {
+    // runs of 8 bytes where the rows are whole runs of them and every operand is aligned to one
+    constexpr int V = 8 / (int)sizeof(T);
+    const bool runs = d % V == 0 && (((uintptr_t)x | (uintptr_t)out) & 7) == 0;
+    const dim3 grid((unsigned)((rows * d / (runs ? V : 1) + 255) / 256)), block(256);
+    if (runs) hipLaunchKernelGGL((weighted_sum_kernel<T, V>), grid, block, 0, s, (const T *)x, (const T *)w, (T *)out, rows, k, d);
+    else hipLaunchKernelGGL((weighted_sum_kernel<T, 1>), grid, block, 0, s, (const T *)x, (const T *)w, (T *)out, rows, k, d);
+}
+
 int32_t launch_weighted_sum(int32_t dtype, const void *x, const void *w, int64_t rows, int32_t k, int64_t d, void *out, hipStream_t s) {
-    const dim3 grid((unsigned)((rows * d + 255) / 256)), block(256);
-    if (dtype == NVQ_F32)
-        hipLaunchKernelGGL(weighted_sum_kernel<float>, grid, block, 0, s, (const float *)x, (const float *)w, (float *)out, rows, k, d);
-    else if (dtype == NVQ_BF16)
-        hipLaunchKernelGGL(weighted_sum_kernel<bf16_t>, grid, block, 0, s, (const bf16_t *)x, (const bf16_t *)w, (bf16_t *)out, rows, k, d);
-    else
-        hipLaunchKernelGGL(weighted_sum_kernel<f16_t>, grid, block, 0, s, (const f16_t *)x, (const f16_t *)w, (f16_t *)out, rows, k, d);
+    if (dtype == NVQ_F32) run_weighted_sum<float>(x, w, rows, k, d, out, s);
+    else if (dtype == NVQ_BF16) run_weighted_sum<bf16_t>(x, w, rows, k, d, out, s);
+    else run_weighted_sum<f16_t>(x, w, rows, k, d, out, s);
     NVQ_LAUNCH_CHECK("weighted_sum");
+    return NVQ_OK;
+}
+
+template <typename T>
+static void run_moe_router(const void *x, const void *gate, int64_t rows, int32_t dims, int32_t experts, int32_t k, int32_t normalize,
+                           uint32_t *indices, void *scores, uint32_t *tokens, uint32_t *identity, hipStream_t s) {
+    const int waves = experts < 16 ? (experts < 4 ? 4 : experts) : 16;
+    hipLaunchKernelGGL(moe_router_kernel<T>, dim3((unsigned)rows), dim3(64 * waves), 0, s, (const T *)x, (const T *)gate, dims, experts, k, normalize,
+                       indices, (T *)scores, tokens, identity);
+}
+
+int32_t launch_moe_router(int32_t dtype, const void *x, const void *gate, int64_t rows, int32_t dims, int32_t experts, int32_t k,
+                          int32_t normalize, uint32_t *indices, void *scores, uint32_t *tokens, uint32_t *identity, hipStream_t s) {
+    if (dtype == NVQ_F32) run_moe_router<float>(x, gate, rows, dims, experts, k, normalize, indices, scores, tokens, identity, s);
+    else if (dtype == NVQ_BF16) run_moe_router<bf16_t>(x, gate, rows, dims, experts, k, normalize, indices, scores, tokens, identity, s);
+    else run_moe_router<f16_t>(x, gate, rows, dims, experts, k, normalize, indices, scores, tokens, identity, s);
+    NVQ_LAUNCH_CHECK("moe_router");
     return NVQ_OK;
 }
 

@@ -25,9 +25,11 @@ using at::Tensor;
 struct Names {
     PyObject *mode, *group_size, *bits, *weight, *scales, *biases, *bias, *quant, *global_scale;
     PyObject *gate_proj, *up_proj, *down_proj, *gate_up_proj, *geglu;
+    PyObject *gate, *switch_mlp, *experts_per_token, *norm_topk_prob, *gate_up_paired, *activation, *alpha, *limit;
 } names;
 
-PyTypeObject *linear_type = nullptr;  // layers.QuantizedLinear: its forward is the one restated here (a subclass may have another)
+// layers.QuantizedLinear, SwitchProjection, SwitchGlu: their forwards are the ones restated here (a subclass may have another)
+PyTypeObject *linear_type = nullptr, *projection_type = nullptr, *switch_glu_type = nullptr;
 uint64_t ready_devices = 0;           // devices nvq_init has answered for (ops._init), read and written under the GIL
 
 struct Ref {
@@ -53,6 +55,23 @@ bool read_int(PyObject *o, PyObject *name, int32_t &v) {
 
 bool read_quant(PyObject *o, nvq_quant &q) {
     return read_int(o, names.mode, q.mode) && read_int(o, names.group_size, q.group_size) && read_int(o, names.bits, q.bits);
+}
+
+bool read_float(PyObject *o, PyObject *name, float &v) {
+    Ref a(PyObject_GetAttr(o, name));
+    if (a.p == nullptr) return declined();
+    const double d = PyFloat_AsDouble(a.p);
+    if (d == -1.0 && PyErr_Occurred()) return declined();
+    v = (float)d;
+    return true;
+}
+
+bool read_truth(PyObject *o, PyObject *name, bool &v) {
+    Ref a(PyObject_GetAttr(o, name));
+    const int t = a.p == nullptr ? -1 : PyObject_IsTrue(a.p);
+    if (t < 0) return declined();
+    v = t != 0;
+    return true;
 }
 
 // A tensor, or none at all for None.
@@ -175,14 +194,144 @@ bool product_glu(const Tensor &x, const Packed &p, const Tensor &bias, int32_t a
     return true;
 }
 
+struct Activation {
+    int32_t code = NVQ_GLU_SWIGLU;
+    float alpha = 0.0f, limit = 0.0f;
+};
+
 // ops.glu of two dense tensors, without biases.
-bool gated(const Tensor &gate, const Tensor &up, int32_t activation, float alpha, float limit, Tensor &out) {
+bool gated(const Tensor &gate, const Tensor &up, int32_t activation, Tensor &out) {
     const Place at(gate);
     const int64_t hidden = gate.size(-1);
-    nvq_glu_desc d{code_of(gate.scalar_type()), activation, alpha, limit, gate.numel() / hidden, hidden, hidden, hidden, 0};
+    nvq_glu_desc d{code_of(gate.scalar_type()), activation, 0.0f, 0.0f, gate.numel() / hidden, hidden, hidden, hidden, 0};
     Tensor y = at.empty(gate.sizes(), gate.scalar_type());
     if (nvq_glu(&d, ptr(gate), ptr(up), nullptr, nullptr, nullptr, y.mutable_data_ptr(), at.stream()) != NVQ_OK) return false;
     out = std::move(y);
+    return true;
+}
+
+// ── mixture of experts ──────────────────────────────────────────────────────────────────────────────────────────────
+struct Projection {  // layers.SwitchProjection: a packed weight and perhaps a bias per expert
+    Packed p;
+    Tensor bias;
+    int64_t columns = 0, rows = 0;
+
+    bool fits(const Place &at, at::ScalarType type, int64_t experts) {
+        if (!p.fits(at, type, 3, columns) || p.w.size(0) != experts) return false;
+        rows = p.w.size(1);
+        return rows > 0 && (!bias.defined() || (bias.scalar_type() == type && bias.dim() == 2 && bias.size(0) == experts &&
+                                                bias.size(1) == rows && at.holds(bias)));
+    }
+};
+
+// The pairs of a pass: which row of x and which expert each takes, in the order they run.
+struct Pairs {
+    int64_t count, experts;
+    const uint32_t *expert;       // of each pair, in order
+    const int32_t *offsets;       // sorted by expert: where each expert's pairs start; NULL: any order
+};
+
+// One projection of all pairs (ops.gather_qmm, ops.gather_qmm_grouped): pair z takes row `from[z]` of x [x_rows, columns] and
+// writes row `to[z]` (NULL: z).
+bool project(const Place &at, const Tensor &x, int64_t x_rows, const Projection &w, const Pairs &pairs, const uint32_t *from, const uint32_t *to,
+             bool with_bias, Tensor &out) {
+    const nvq_gather_desc d{w.p.q, code_of(x.scalar_type()), 1, 0, 0, 1, w.rows, w.columns, pairs.count, x_rows, pairs.experts};
+    Tensor y = at.empty({pairs.count, w.rows}, x.scalar_type());
+    if (nvq_gather_qmm_expert_bias(&d, ptr(x), ptr(w.p.w), ptr(w.p.s), ptr(w.p.b), nullptr, from, pairs.expert, pairs.offsets, to,
+                                   with_bias ? ptr(w.bias) : nullptr, y.mutable_data_ptr(), nullptr, at.stream()) != NVQ_OK)
+        return false;
+    out = std::move(y);
+    return true;
+}
+
+struct Experts {  // layers.SwitchGlu
+    Projection gate, up, down, both;
+    bool fused = false, paired = false;
+    Activation act;
+};
+
+// The pairs' gated hidden states (layers.SwitchGlu.forward up to the down projection).
+bool hidden_states(const Place &at, const Tensor &x, int64_t x_rows, Experts &e, const Pairs &pairs, const uint32_t *tokens, Tensor &out) {
+    const at::ScalarType type = x.scalar_type();
+    const int64_t hidden = e.down.columns;
+    if (e.fused && e.paired) {
+        const nvq_gather_desc d{e.both.p.q, code_of(type), 1, 0, 0, 1, e.both.rows, e.both.columns, pairs.count, x_rows, pairs.experts};
+        Tensor y = at.empty({pairs.count, hidden}, type);
+        if (nvq_gather_qmm_glu(&d, e.act.code, e.act.alpha, e.act.limit, ptr(x), ptr(e.both.p.w), ptr(e.both.p.s), ptr(e.both.p.b), tokens,
+                               pairs.expert, pairs.offsets, ptr(e.both.bias), y.mutable_data_ptr(), at.stream()) == NVQ_OK) {
+            out = std::move(y);
+            return true;
+        }
+    }
+    // products without their biases, then biases and activation in one pass
+    Tensor gate, up;
+    int64_t stride = hidden;
+    const char *second;
+    if (e.fused && !e.paired) {
+        if (!project(at, x, x_rows, e.both, pairs, tokens, nullptr, false, gate)) return false;
+        stride = 2 * hidden;
+        second = (const char *)ptr(gate) + hidden * gate.element_size();
+    } else {
+        if (!project(at, x, x_rows, e.gate, pairs, tokens, nullptr, false, gate) || !project(at, x, x_rows, e.up, pairs, tokens, nullptr, false, up))
+            return false;
+        second = (const char *)ptr(up);
+    }
+    const bool biased = e.gate.bias.defined();
+    const nvq_glu_desc d{code_of(type), e.act.code, e.act.alpha, e.act.limit, pairs.count, hidden, stride, stride, biased ? pairs.experts : 0};
+    Tensor y = at.empty({pairs.count, hidden}, type);
+    if (nvq_glu(&d, ptr(gate), second, ptr(e.gate.bias), ptr(e.up.bias), biased ? (const int32_t *)pairs.expert : nullptr, y.mutable_data_ptr(),
+                at.stream()) != NVQ_OK)
+        return false;
+    out = std::move(y);
+    return true;
+}
+
+// layers.MoeMlp.forward.
+bool moe(const Tensor &x, const Tensor &router, int64_t k, bool normalize, Experts &e, Tensor &out) {
+    const Place at(x);
+    if (!at.usable() || x.dim() != 3 || x.numel() == 0 || !x.is_contiguous()) return false;
+    const at::ScalarType type = x.scalar_type();
+    const int32_t code = code_of(type);
+    if (code < 0 || !router.defined() || router.scalar_type() != type || router.dim() != 2 || !at.holds(router) || router.size(1) != x.size(2))
+        return false;
+    const int64_t rows = x.size(0) * x.size(1), dims = x.size(2), experts = router.size(0);
+    if (k < 1 || k > experts || k >= 32 || dims > INT32_MAX || experts > 1024 || rows > INT32_MAX / k) return false;
+    if (!e.gate.fits(at, type, experts) || !e.up.fits(at, type, experts) || !e.down.fits(at, type, experts)) return false;
+    const int64_t hidden = e.down.columns;
+    if (e.gate.columns != dims || e.up.columns != dims || e.gate.rows != hidden || e.up.rows != hidden ||
+        e.gate.bias.defined() != e.up.bias.defined())
+        return false;
+    if (e.fused && (!e.both.fits(at, type, experts) || e.both.columns != dims || e.both.rows != 2 * hidden ||
+                    e.both.bias.defined() != e.gate.bias.defined() || (e.paired && hidden % 64 != 0)))
+        return false;
+
+    const int64_t pairs = rows * k;
+    void *stream = at.stream();
+    // choices, tokens and numbers of the pairs; for ordered pairs the order, its inverse, sorted experts and tokens, the offsets
+    const bool ordered = pairs >= 64;
+    Tensor index = at.empty({pairs * (ordered ? 7 : 3) + (ordered ? experts : 0)}, at::kInt), scores = at.empty({rows, k}, type);
+    uint32_t *chosen = (uint32_t *)index.mutable_data_ptr(), *tokens = chosen + pairs, *identity = tokens + pairs;
+    if (nvq_moe_router(code, ptr(x), ptr(router), rows, (int32_t)dims, (int32_t)experts, (int32_t)k, normalize, chosen, scores.mutable_data_ptr(),
+                       tokens, identity, stream) != NVQ_OK)
+        return false;
+    Pairs p{pairs, experts, chosen, nullptr};
+    const uint32_t *to = nullptr;
+    Tensor workspace, h, y;
+    if (ordered) {
+        uint32_t *order = identity + pairs, *restore = order + pairs, *sorted = restore + pairs, *sorted_tokens = sorted + pairs;
+        int32_t *offsets = (int32_t *)(sorted_tokens + pairs);
+        const size_t need = nvq_moe_order_workspace_bytes(pairs, (int32_t)experts);
+        if (need > 0) workspace = at.empty({(int64_t)need}, at::kByte);
+        if (nvq_moe_order_tokens(chosen, pairs, (int32_t)experts, (int32_t)k, order, restore, sorted, offsets, sorted_tokens,
+                                 need > 0 ? workspace.mutable_data_ptr() : nullptr, stream) != NVQ_OK)
+            return false;
+        p.expert = sorted, p.offsets = offsets;
+        tokens = sorted_tokens, to = order;
+    }
+    if (!hidden_states(at, x, rows, e, p, tokens, h) || !project(at, h, pairs, e.down, p, identity, to, true, y) || e.down.rows == 0) return false;
+    Tensor sum = at.empty({x.size(0), x.size(1), e.down.rows}, type);
+    if (nvq_weighted_sum(code, ptr(y), ptr(scores), rows, (int32_t)k, e.down.rows, sum.mutable_data_ptr(), stream) != NVQ_OK) return false;
+    out = std::move(sum);
     return true;
 }
 
@@ -269,10 +418,56 @@ PyObject *py_mlp(PyObject *, PyObject *const *args, Py_ssize_t n) {
         if (!hidden.defined()) {
             Tensor g, u;
             if (!read_linear(args[0], names.up_proj, up) || !product(x, gate.p, gate.bias, Flags(), g) || !product(x, up.p, up.bias, Flags(), u) ||
-                g.sizes() != u.sizes() || !gated(g, u, activation, 0.0f, 0.0f, hidden))
+                g.sizes() != u.sizes() || !gated(g, u, activation, hidden))
                 return none();
         }
         return wrap(product(hidden, down.p, down.bias, Flags(), y), y);
+    });
+}
+
+bool read_projection(PyObject *o, PyObject *name, Projection &j) {
+    Ref a(PyObject_GetAttr(o, name));
+    if (a.p == nullptr) return declined();
+    if (Py_TYPE(a.p) != projection_type) return false;
+    Tensor global_scale;
+    if (!read_tensor(a.p, names.weight, j.p.w) || !read_tensor(a.p, names.scales, j.p.s) || !read_tensor(a.p, names.biases, j.p.b) ||
+        !read_tensor(a.p, names.bias, j.bias) || !read_tensor(a.p, names.global_scale, global_scale) || global_scale.defined())
+        return false;
+    Ref q(PyObject_GetAttr(a.p, names.quant));
+    return q.p == nullptr ? declined() : read_quant(q.p, j.p.q);
+}
+
+// moe(block, x): layers.MoeMlp.forward
+PyObject *py_moe(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    return guarded([&]() -> PyObject * {
+        Tensor x, router, y;
+        int32_t k;
+        bool normalize;
+        Experts e;
+        if (n != 2 || !as_tensor(args[1], x) || !read_tensor(args[0], names.gate, router) || !read_int(args[0], names.experts_per_token, k) ||
+            !read_truth(args[0], names.norm_topk_prob, normalize))
+            return none();
+        Ref glu(PyObject_GetAttr(args[0], names.switch_mlp));
+        if (glu.p == nullptr || Py_TYPE(glu.p) != switch_glu_type) {
+            PyErr_Clear();
+            return none();
+        }
+        Ref both(PyObject_GetAttr(glu.p, names.gate_up_proj)), activation(PyObject_GetAttr(glu.p, names.activation));
+        if (both.p == nullptr || activation.p == nullptr || !PyUnicode_Check(activation.p)) {
+            PyErr_Clear();
+            return none();
+        }
+        e.fused = both.p != Py_None;
+        if (PyUnicode_CompareWithASCIIString(activation.p, "swiglu") == 0) e.act.code = NVQ_GLU_SWIGLU;
+        else if (PyUnicode_CompareWithASCIIString(activation.p, "swiglu_oai") == 0) e.act.code = NVQ_GLU_SWIGLU_OAI;
+        else if (PyUnicode_CompareWithASCIIString(activation.p, "geglu") == 0) e.act.code = NVQ_GLU_GEGLU;
+        else return none();
+        if (!read_projection(glu.p, names.gate_proj, e.gate) || !read_projection(glu.p, names.up_proj, e.up) ||
+            !read_projection(glu.p, names.down_proj, e.down) || (e.fused && !read_projection(glu.p, names.gate_up_proj, e.both)) ||
+            !read_truth(glu.p, names.gate_up_paired, e.paired) || !read_float(glu.p, names.alpha, e.act.alpha) ||
+            !read_float(glu.p, names.limit, e.act.limit))
+            return none();
+        return wrap(moe(x, router, k, normalize, e, y), y);
     });
 }
 
@@ -397,14 +592,17 @@ PyObject *py_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
     });
 }
 
-// register(QuantizedLinear): the types whose forward is restated here
+// register(QuantizedLinear, SwitchProjection, SwitchGlu): the types whose forward is restated here
 PyObject *py_register(PyObject *, PyObject *const *args, Py_ssize_t n) {
-    if (n != 1 || !PyType_Check(args[0])) {
-        PyErr_SetString(PyExc_TypeError, "register(QuantizedLinear)");
-        return nullptr;
+    PyTypeObject **types[] = {&linear_type, &projection_type, &switch_glu_type};
+    for (Py_ssize_t i = 0; i < 3; i++) {
+        if (n != 3 || !PyType_Check(args[i])) {
+            PyErr_SetString(PyExc_TypeError, "register(QuantizedLinear, SwitchProjection, SwitchGlu)");
+            return nullptr;
+        }
+        Py_INCREF(args[i]);
+        *types[i] = (PyTypeObject *)args[i];
     }
-    Py_INCREF(args[0]);
-    linear_type = (PyTypeObject *)args[0];
     return none();
 }
 
@@ -423,6 +621,7 @@ PyMethodDef methods[] = {
     {"linear", NVQ_FAST(py_linear), nullptr},
     {"quantized_matmul", NVQ_FAST(py_quantized_matmul), nullptr},
     {"mlp", NVQ_FAST(py_mlp), nullptr},
+    {"moe", NVQ_FAST(py_moe), nullptr},
     {"quantize", NVQ_FAST(py_quantize), nullptr},
     {"dequantize", NVQ_FAST(py_dequantize), nullptr},
     {"embedding", NVQ_FAST(py_embedding), nullptr},
@@ -439,6 +638,9 @@ extern "C" __attribute__((visibility("default"))) PyObject *PyInit__native(void)
         {&names.scales, "scales"}, {&names.biases, "biases"}, {&names.bias, "bias"}, {&names.quant, "quant"},
         {&names.global_scale, "global_scale"}, {&names.gate_proj, "gate_proj"}, {&names.up_proj, "up_proj"},
         {&names.down_proj, "down_proj"}, {&names.gate_up_proj, "gate_up_proj"}, {&names.geglu, "geglu"},
+        {&names.gate, "gate"}, {&names.switch_mlp, "switch_mlp"}, {&names.experts_per_token, "experts_per_token"},
+        {&names.norm_topk_prob, "norm_topk_prob"}, {&names.gate_up_paired, "gate_up_paired"}, {&names.activation, "activation"},
+        {&names.alpha, "alpha"}, {&names.limit, "limit"},
     };
     for (auto &n : all) {
         *n.at = PyUnicode_InternFromString(n.text);

@@ -882,8 +882,8 @@ size_t nvq_moe_order_workspace_bytes(int64_t pairs, int32_t experts) {
     return moe_order_workspace_bytes(pairs, experts);
 }
 
-int32_t nvq_moe_order(const uint32_t *ids, int64_t pairs, int32_t experts, uint32_t *order, uint32_t *restore,
-                      uint32_t *sorted_ids, int32_t *offsets, void *workspace, void *stream) {
+static int32_t moe_order_any(const uint32_t *ids, int64_t pairs, int32_t experts, uint32_t *order, uint32_t *restore, uint32_t *sorted_ids,
+                             int32_t *offsets, uint32_t *tokens, int32_t choices, void *workspace, void *stream) {
     if (pairs < 0 || experts <= 0) return fail(NVQ_INVALID_ARGUMENT, "moe_order: %lld pairs, %d experts", (long long)pairs, experts);
     if (pairs > INT32_MAX) return fail(NVQ_INVALID_ARGUMENT, "moe_order: %lld pairs exceed 32-bit positions", (long long)pairs);
     if (moe_order_lds_bytes(experts) > 64 * 1024)
@@ -891,7 +891,19 @@ int32_t nvq_moe_order(const uint32_t *ids, int64_t pairs, int32_t experts, uint3
     if (offsets == nullptr || (pairs > 0 && (ids == nullptr || order == nullptr || restore == nullptr || sorted_ids == nullptr)))
         return fail(NVQ_INVALID_ARGUMENT, "moe_order: null operand");
     NVQ_TRY(require_device());
-    return launch_moe_order(ids, pairs, experts, order, restore, sorted_ids, offsets, workspace, (hipStream_t)stream);
+    return launch_moe_order(ids, pairs, experts, order, restore, sorted_ids, offsets, tokens, choices, workspace, (hipStream_t)stream);
+}
+
+int32_t nvq_moe_order(const uint32_t *ids, int64_t pairs, int32_t experts, uint32_t *order, uint32_t *restore,
+                      uint32_t *sorted_ids, int32_t *offsets, void *workspace, void *stream) {
+    return moe_order_any(ids, pairs, experts, order, restore, sorted_ids, offsets, nullptr, 1, workspace, stream);
+}
+
+int32_t nvq_moe_order_tokens(const uint32_t *ids, int64_t pairs, int32_t experts, int32_t choices, uint32_t *order, uint32_t *restore,
+                             uint32_t *sorted_ids, int32_t *offsets, uint32_t *tokens, void *workspace, void *stream) {
+    if (choices < 1) return fail(NVQ_INVALID_ARGUMENT, "moe_order: %d choices per token", choices);
+    if (tokens == nullptr && pairs > 0) return fail(NVQ_INVALID_ARGUMENT, "moe_order: null operand");
+    return moe_order_any(ids, pairs, experts, order, restore, sorted_ids, offsets, tokens, choices, workspace, stream);
 }
 
 int32_t nvq_moe_route(int32_t dtype, const void *probs, int64_t rows, int32_t experts, int32_t k, int32_t normalize,
@@ -907,6 +919,25 @@ int32_t nvq_moe_route(int32_t dtype, const void *probs, int64_t rows, int32_t ex
     if (probs == nullptr || indices == nullptr || scores == nullptr) return fail(NVQ_INVALID_ARGUMENT, "moe_route: null operand");
     NVQ_TRY(require_device());
     return launch_moe_route(dtype, probs, rows, experts, k, normalize != 0, indices, scores, (hipStream_t)stream);
+}
+
+int32_t nvq_moe_router(int32_t dtype, const void *x, const void *gate, int64_t rows, int32_t dims, int32_t experts, int32_t k,
+                       int32_t normalize, uint32_t *indices, void *scores, uint32_t *tokens, uint32_t *identity, void *stream) {
+    const char *op = "moe_router";
+    if (!float_dtype(dtype)) return fail(NVQ_INVALID_ARGUMENT, "%s: unsupported dtype %s", op, dtype_name(dtype));
+    if (rows < 0 || dims < 1 || experts < 1 || k < 1 || k > experts)
+        return fail(NVQ_INVALID_ARGUMENT, "%s: k must be in 1..=%d for x of shape [%lld, %d]", op, experts, (long long)rows, dims);
+    // (every token's block reads the whole gate from the L2: 2^26 values are 128 MB, about 16 us there; the library's product,
+    // its conversions and the softmax take 31 us at 256 tokens x 32 x 2880 and grow slowly from there)
+    if (experts > 1024 || (normalize && k > 64) || ((int64_t)dims * dtype_size(dtype)) % 16 != 0 || rows > (1LL << 26) / ((int64_t)experts * dims))
+        return fail(NVQ_UNSUPPORTED, "%s: %lld x %d x %d values: a matrix product of its own", op, (long long)rows, experts, dims);
+    if (rows == 0) return NVQ_OK;
+    if (x == nullptr || gate == nullptr || indices == nullptr || scores == nullptr || tokens == nullptr || identity == nullptr)
+        return fail(NVQ_INVALID_ARGUMENT, "%s: null operand", op);
+    NVQ_TRY(require_device());
+    NVQ_TRY(check_aligned(op, "x", x));
+    NVQ_TRY(check_aligned(op, "gate", gate));
+    return launch_moe_router(dtype, x, gate, rows, dims, experts, k, normalize != 0, indices, scores, tokens, identity, (hipStream_t)stream);
 }
 
 int32_t nvq_weighted_sum(int32_t dtype, const void *x, const void *w, int64_t rows, int32_t k, int64_t d, void *out, void *stream) {

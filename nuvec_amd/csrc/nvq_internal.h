@@ -68,7 +68,9 @@ int32_t launch_glu(const nvq_glu_desc &d, const void *gate, const void *up, cons
 int32_t launch_weighted_sum(int32_t dtype, const void *x, const void *w, int64_t rows, int32_t k, int64_t d, void *out, hipStream_t s);
 size_t moe_order_workspace_bytes(int64_t pairs, int32_t experts);
 int32_t launch_moe_order(const uint32_t *ids, int64_t pairs, int32_t experts, uint32_t *order, uint32_t *restore,
-                         uint32_t *sorted_ids, int32_t *offsets, void *workspace, hipStream_t s);
+                         uint32_t *sorted_ids, int32_t *offsets, uint32_t *tokens, int32_t choices, void *workspace, hipStream_t s);
+int32_t launch_moe_router(int32_t dtype, const void *x, const void *gate, int64_t rows, int32_t dims, int32_t experts, int32_t k,
+                          int32_t normalize, uint32_t *indices, void *scores, uint32_t *tokens, uint32_t *identity, hipStream_t s);
 
 // One transposed product per batch/pair.  `lhs`/`rhs` NULL = batch strides from `desc`.
 struct ProductArgs {

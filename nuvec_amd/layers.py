@@ -21,7 +21,7 @@ def _calls():
     """The native calls, told which layers they may read."""
     global _native
     n = _lib.native()
-    n.register(QuantizedLinear)
+    n.register(QuantizedLinear, SwitchProjection, SwitchGlu)
     _native = n
     return n
 
@@ -315,6 +315,9 @@ class MoeMlp:
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         """`x` `[B, L, D]` -> `[B, L, D]`."""
+        y = (_native or _calls()).moe(self, x)
+        if y is not None:
+            return y
         top, scores = self.route(x)
         experts = self.switch_mlp.forward(x, top)  # [B, L, k, D]
         return ops.weighted_sum(experts, scores)

@@ -92,3 +92,55 @@ def test_refusals_are_the_python_paths():
         nv.quantize(x, nv.Quant.affine(48, 4))
     mixed = nv.quantized_matmul(x.to(torch.bfloat16), q)  # promotes
     assert mixed.dtype == torch.float32
+
+
+@pytest.mark.parametrize("rows,dims,experts,k", [(1, 2880, 32, 4), (7, 64, 3, 3), (300, 520, 128, 8), (5, 8, 1, 1), (2, 1032, 300, 6)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_router(rows, dims, experts, k, dtype):
+    """`nvq_moe_router` against float64: an unrounded probability p lies within (2 u |logit| + 3 u) p of the kernel's, u the unit
+    roundoff of the type (one rounding of the logit and of the largest logit, one of p and one of the quotient; float32: the
+    sums' own error, 16 u); the k chosen are the largest within twice that, in ascending order of their scores."""
+    import ctypes as C
+    torch.manual_seed(rows)
+    x, gate = torch.randn(rows, dims, device="cuda").to(dtype), (torch.randn(experts, dims, device="cuda") * dims ** -0.5).to(dtype)
+    index, scores = torch.empty(3, rows, k, dtype=torch.int32, device="cuda"), torch.empty(rows, k, dtype=dtype, device="cuda")
+    nv.ops._init(x)
+    p = lambda t: C.c_void_p(t.data_ptr())
+    for normalize in (0, 1):
+        _lib.check(_lib.load().nvq_moe_router(nv.ops._CODE[dtype], p(x), p(gate), rows, dims, experts, k, normalize, p(index[0]), p(scores),
+                                              p(index[1]), p(index[2]), nv.ops._stream()))
+        logits = x.double() @ gate.double().T.contiguous()
+        probs = torch.softmax(logits, -1)
+        u = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 16 * 2.0 ** -24}[dtype]
+        near = u * (2 * logits.abs().max() + 3)
+        taken = torch.gather(probs, 1, index[0].long())
+        assert (index[0].sort(-1).values.diff(dim=-1) > 0).all()  # distinct
+        left = probs.scatter(1, index[0].long(), 0.0)
+        assert (taken.min(-1).values >= left.max(-1).values * (1 - 2 * near)).all()
+        assert (taken[:, 1:] >= taken[:, :-1] * (1 - 2 * near)).all()
+        want = taken / taken.sum(-1, keepdim=True) if normalize else taken
+        assert ((scores.double() - want).abs() <= (2 + k) * near * want + 1e-7).all()  # (the sum of k: one rounding each)
+    assert torch.equal(index[1], torch.arange(rows, device="cuda", dtype=torch.int32)[:, None].expand(rows, k))
+    assert torch.equal(index[2].flatten(), torch.arange(rows * k, device="cuda", dtype=torch.int32))
+
+
+@pytest.mark.parametrize("quant", [nv.Quant.affine(64, 4), nv.Quant.affine(32, 8), nv.Quant.new(nv.QuantMode.MXFP4)], ids=str)
+@pytest.mark.parametrize("dims,hidden,bias,activation", [(256, 1024, True, "swiglu_oai"), (512, 96, False, "swiglu"), (320, 640, True, "geglu")])
+def test_moe_equals_the_python_path(both, quant, dims, hidden, bias, activation):
+    """The same kernels but for the router's (its softmax may round a probability the other way: one step of a score)."""
+    torch.manual_seed(3)
+    if dims % quant.group_size or hidden % quant.group_size:
+        pytest.skip("not whole groups")
+    put = lambda *shape: (torch.randn(shape, device="cuda") * 0.1).bfloat16()
+
+    def projection(n, k):
+        q = nv.quantize(put(8, n, k), quant)
+        return layers.SwitchProjection(q.weight, q.scales, q.biases, put(8, n) if bias else None, q.quant)
+    for fuse in (False, True):
+        glu = layers.SwitchGlu(projection(hidden, dims), projection(hidden, dims), projection(dims, hidden), activation=activation)
+        block = layers.MoeMlp(put(8, dims), glu.fuse_gate_up() if fuse else glu, 2)
+        for tokens in (1, 31, 32, 200):
+            x = torch.randn(1, tokens, dims, device="cuda").bfloat16()
+            native, python = both(lambda: block(x))
+            bound = 4 * 2.0 ** -8 * python.float().abs().max()
+            assert native.shape == python.shape and ((native.float() - python.float()).abs() <= bound).all(), (fuse, tokens)

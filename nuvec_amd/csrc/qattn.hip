@@ -1,166 +1,370 @@
-// Attention of one query row per head over an affine-quantized key / value cache, in one kernel: the counterpart of
+// Attention of one query row per head over an affine-quantized key / value cache: the counterpart of
 // the reference's FastOp::QuantizedAttention kernel (crates/nuvec-core/src/fast.rs:694-718; its fit rule
 // crates/nuvec-core/src/fast/imp.rs:3944-3992; launch crates/nuvec-core/src/gpu.rs:4969-5040):
 //     out[b, h, :] = softmax(scale * q[b, h, :] . K[b, h / rep]^T [, sink[h]]) . V[b, h / rep]
-// with K and V stored packed (codes [B, Hkv, S, D bits / 32], scales and biases [B, Hkv, S, D / group]).  The codes are
-// dequantized in registers and never rounded; products and sums are float32 (the reference's kernel likewise: "within
-// the float bound of the dequantized attention").
+// with K and V stored packed (codes [B, Hkv, S, D bits / 32], scales and biases [B, Hkv, S, D / group]).  Products and sums
+// are float32 and the codes are never rounded (the reference's kernel likewise: "within the float bound of the dequantized
+// attention").
 //
-// A block of four wavefronts owns one (batch, query head).  A row of the cache is D bits / 8 bytes = CH chunks of 16
-// bytes (3 bits: of 12 bytes, 32 codes); lane l of a wavefront takes chunk l % CH of key l / CH of the wavefront's
-// current tile of 64 / CH keys, so a wavefront-wide load reads 1 KB (768 bytes) of consecutive rows.  Per key the lanes of a row form the score from their partial
-// dot products (factored: scale * sum(q * code) + bias * sum(q) per chunk) with cross-lane adds, every lane keeps an
-// online softmax (running maximum, denominator) for the keys it has seen and accumulates its chunk of the output in
-// the same factored form; at the end the (64 / CH) x 4 partial states are merged through LDS.
+// The bound is the stream of the cache, read once for all query heads of a key head, as long as turning codes into operands
+// costs little: both products run on the matrix cores over the CODES, which bfloat16 holds exactly (8 bits as they are, 3 and
+// 4 bits in the low mantissa bits of 128: one instruction per two codes, the 128 taken out again by the sums it multiplies).
+// What is not exact in bfloat16, the queries of the wider types and the softmax's weights, goes in as the sum of two or three
+// bfloat16 terms (16 or 24 bits): TQ and TP below.
+//
+// Groups.  v_mfma_f32_16x16x32 has 16 columns and a key head at most 8 query heads: the columns are (group of D, query head)
+// with 16 / groups heads each (eight heads over four groups take two blocks).  The query's operand holds zeros outside
+// a column's group, so S^T = K . Q^T separates the groups' partial scores without regard to which codes share an
+// instruction, and a lane's 32 codes (16 bytes at 4 bits) are consecutive; scale and bias of a column's group are applied to
+// the partial score, the groups of a row are added across lanes.  In O^T = V^T . P^T a column's weights are p times that
+// group's scale: a row of D is taken from the columns of its own group, the others are ignored.
+//
+// Lanes.  Lane (quarter q, l) holds in S^T column l of keys 4 q .. + 3 of two tiles of 16 keys: they are the eight keys of its
+// operand P^T (the contraction's order is free), and of V it loads D / 16 codes, l's slot of the row, of the same eight keys.
+// No value crosses lanes but the groups' sums, and maxima when they grow.
 #include "nvq_device.h"
 #include "nvq_internal.h"
+#include "qmf_kernel.h"
 
 namespace nvq {
-int attention_splits(const nvq_attention_desc &d);
 namespace {
 
+typedef float floatx4_t __attribute__((ext_vector_type(4)));
 constexpr int kAttnWaves = 4;
+constexpr int kTileKeys = 32;
+constexpr float kLog2e = 1.44269504088896340736f;
 
-// A lane's chunk of a row: 16 bytes (BITS 4: 32 codes, 8: 16 codes), or the 12 bytes that hold 32 codes of 3 bits.
-template <int BITS> struct Chunk { uint32_t w[BITS == 3 ? 3 : 4]; };
+__device__ __forceinline__ floatx4_t mfma16(uint4 a, uint4 b, floatx4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(qmf::bf16x8_t, a), __builtin_bit_cast(qmf::bf16x8_t, b), c, 0, 0, 0);
+}
 
+// A value from any address, in as few loads as it has dwords.
+template <typename V>
+__device__ __forceinline__ V load_any(const void *p) {
+    struct __attribute__((packed)) Raw { V v; };
+    return reinterpret_cast<const Raw *>(p)->v;
+}
+
+// The 3- and 4-bit codes' operands are 128 + code.
+template <int BITS> constexpr float kOffset = BITS == 8 ? 0.0f : 128.0f;
+constexpr uint32_t kMagic = 0x43004300u;
+
+// Two exact bfloat16 values from two floats that bfloat16 holds.
+__device__ __forceinline__ uint32_t pack_exact(float lo, float hi) { return __builtin_amdgcn_perm(f2u(hi), f2u(lo), 0x07060302u); }
+
+// Which of eight consecutive codes element j of an operand is.
+template <int BITS> constexpr int code_at(int j) { return BITS == 8 ? j : (j >> 1) + 4 * (j & 1); }
+
+// Eight consecutive codes of a row (BITS bytes in the low bits of w0, w1) as an operand, in the order of code_at.
 template <int BITS>
-__device__ __forceinline__ Chunk<BITS> load_chunk(const uint32_t *p) {
-    Chunk<BITS> c;
-    if constexpr (BITS == 3) {
-        c.w[0] = p[0], c.w[1] = p[1], c.w[2] = p[2];  // (rows of 3-bit codes are whole dwords: 4-byte aligned)
+__device__ __forceinline__ uint4 eight_codes(uint32_t w0, uint32_t w1) {
+    if constexpr (BITS == 8) {
+        return make_uint4(pack_exact(qmf::ubyte_to_float<0>(w0), qmf::ubyte_to_float<1>(w0)), pack_exact(qmf::ubyte_to_float<2>(w0), qmf::ubyte_to_float<3>(w0)),
+                          pack_exact(qmf::ubyte_to_float<0>(w1), qmf::ubyte_to_float<1>(w1)), pack_exact(qmf::ubyte_to_float<2>(w1), qmf::ubyte_to_float<3>(w1)));
     } else {
-        const uint4 v = *reinterpret_cast<const uint4 *>(p);
-        c.w[0] = v.x, c.w[1] = v.y, c.w[2] = v.z, c.w[3] = v.w;
-    }
-    return c;
-}
-
-// Code i of a chunk as a float (i is a constant after unrolling).
-template <int BITS>
-__device__ __forceinline__ float chunk_code(const Chunk<BITS> &c, int i) {
-    if constexpr (BITS == 4) {
-        return (float)((c.w[i >> 3] >> (4 * (i & 7))) & 15u);
-    } else if constexpr (BITS == 8) {
-        return (float)((c.w[i >> 2] >> (8 * (i & 3))) & 255u);
-    } else {
-        const int bit = 3 * i, dw = bit >> 5, sh = bit & 31;
-        const uint32_t v = sh <= 29 ? c.w[dw] >> sh : (c.w[dw] >> sh) | (c.w[dw + 1] << (32 - sh));
-        return (float)(v & 7u);
+        constexpr uint32_t mask = BITS == 4 ? 0x000F000Fu : 0x00070007u;
+        const uint32_t z = BITS == 4 ? w0 : (w0 & 0xFFFu) | ((w0 & 0xFFF000u) << 4);  // code i at bit BITS i, code i + 4 sixteen above
+        return make_uint4((z & mask) | kMagic, ((z >> BITS) & mask) | kMagic, ((z >> (2 * BITS)) & mask) | kMagic, ((z >> (3 * BITS)) & mask) | kMagic);
     }
 }
 
-// softmax's last step: the weighted sum over a maximum `top` and its denominator, with the head's sink if it has one.
-__device__ __forceinline__ float attention_finish(float sum, float denom, float top, float sink, bool has_sink) {
-    if (!has_sink) return sum / denom;
-    const float t2 = fmaxf(top, sink), f = __expf(top - t2);
-    return sum * f / (denom * f + __expf(sink - t2));
-}
-
-// Keys of one split of the positions: whole tiles of the block (64 keys at most), so that no tile is shared.
+// Keys of one split of the positions: whole tiles of all wavefronts of a block, so that no tile is shared.
 __host__ __device__ inline int attention_split_keys(int64_t positions, int splits) {
     const int64_t per = (positions + splits - 1) / splits;
-    return (int)((per + 63) / 64 * 64);
+    return (int)((per + kTileKeys - 1) / kTileKeys * kTileKeys);
 }
 
-template <typename T, int BITS, int D>
-__global__ void __launch_bounds__(64 * kAttnWaves) qattn_kernel(const nvq_attention_desc d, const T *__restrict__ q, const uint32_t *__restrict__ kw,
+// A float as a sum of N bfloat16 terms (8 bits each), two floats at a time: term i of both in t[i].
+template <int N>
+__device__ __forceinline__ void split_pair(float a, float b, uint32_t (&t)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        t[i] = f32_to_bf16_pair(a, b);
+        a -= u2f(t[i] << 16), b -= u2f(t[i] & 0xFFFF0000u);
+    }
+}
+
+// G groups of a row.  Block: one (batch, key head, split) and 16 / G of its query heads; its wavefronts take tiles of 32 keys in
+// turn.
+template <typename T, int BITS, int D, int G>
+__global__ void __launch_bounds__(64 * kAttnWaves, sizeof(T) == 2 && G < 4 ? 3 : 2) qattn_kernel(const nvq_attention_desc d, const T *__restrict__ q, const uint32_t *__restrict__ kw,
                                                                const T *__restrict__ ks, const T *__restrict__ kb,
                                                                const uint32_t *__restrict__ vw, const T *__restrict__ vs,
                                                                const T *__restrict__ vb, const T *__restrict__ sinks, T *__restrict__ out,
                                                                float *__restrict__ partials) {
-    constexpr int CPL = BITS == 3 ? 32 : 128 / BITS;  // codes (values of D) per lane
-    constexpr int CW = CPL * BITS / 32;               // dwords of a lane's chunk
-    constexpr int CH = D / CPL;            // lanes per key: 2, 4 or 8
-    constexpr int KPT = 64 / CH;           // keys per wavefront tile
-    constexpr int kSlots = KPT * kAttnWaves;
-    __shared__ float part[kSlots][D + 1];  // the slots' partial outputs, already scaled to the block's maximum
-    __shared__ float slot_m[kSlots], slot_l[kSlots];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int c = lane % CH, j = lane / CH;
-    const int h = blockIdx.x, b = blockIdx.y;
-    const int rep = d.query_heads / d.key_heads, hk = h / rep;
-    const int S = d.positions, groups = D / d.group_size;
-    const int gi = (c * CPL) / d.group_size;  // this lane's group of a row (a chunk lies inside one group: group >= 32 >= CPL)
-    const int64_t row0 = ((int64_t)b * d.key_heads + hk) * S;
-    const int splits = gridDim.z, per = attention_split_keys(S, splits);
-    const int s_begin = blockIdx.z * per, s_end = s_begin + per < S ? s_begin + per : S;
+    constexpr int TQ = sizeof(T) == 4 ? 3 : Elem<T>::code == 10 ? 1 : 2;  // terms of the queries: exact
+    constexpr int TP = sizeof(T) == 4 ? 3 : 2;                            // terms of the weights: 24 or 16 bits
+    constexpr int R = 16 / G, KS = D / 32, ND = D / 16;  // heads per operand; instructions of K per 16 keys; values of D per lane
+    constexpr int kRowBytes = D * BITS / 8, kChunk = kRowBytes / 4, kSlot = BITS * ND;  // bytes of a quarter's codes; bits of a lane's slot
+    constexpr bool kOnes = kOffset<BITS> != 0.0f;
+    constexpr int kHeads = R < 8 ? R : 8;  // (at most eight query heads per key head)
+    __shared__ float part[kAttnWaves][kHeads][D + 1];
+    __shared__ float wave_m[kAttnWaves][kHeads], wave_l[kAttnWaves][kHeads];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l = lane & 15, quarter = lane >> 4, g = l / R;
+    const int hk = blockIdx.x, b = blockIdx.y;
+    const int all = d.query_heads / d.key_heads, S = d.positions;
+    // (the blocks of one key head's cache lie gridDim.x * gridDim.y apart: on one XCD where that is a multiple of 8)
+    const int parts = (all + R - 1) / R, splits = gridDim.z / parts, first = blockIdx.z % parts * R, split = blockIdx.z / parts;
+    const int rep = all - first < R ? all - first : R;  // this block's query heads
+    const int64_t row0 = ((int64_t)b * d.key_heads + hk) * S, head0 = (int64_t)b * d.query_heads + hk * all + first;
+    const int per = attention_split_keys(S, splits);
+    const int s_begin = split * per, s_end = s_begin + per < S ? s_begin + per : S;
+    const float scale = d.scale * kLog2e;
 
-    // the lane's CPL values of the query, scaled; their sum (the bias term of the factored score)
-    float qv[CPL], qsum = 0.0f;
-    const T *qrow = q + ((int64_t)b * d.query_heads + h) * D + c * CPL;
+    // The queries' operands: column (g, head), zeros outside the group; their sums per column.
+    const int head = l % R;
+    uint4 qf[KS][TQ];
+    float qsum = 0.0f;
 #pragma unroll
-    for (int i = 0; i < CPL; i++) {
-        qv[i] = d.scale * Elem<T>::load(qrow, i);
-        qsum += qv[i];
-    }
-    float m = -INFINITY, l = 0.0f, acc[CPL], accb = 0.0f;
+    for (int s = 0; s < KS; s++) {
+        float v[8];
 #pragma unroll
-    for (int i = 0; i < CPL; i++) acc[i] = 0.0f;
-
-    // One tile of keys: everything it reads from memory.  The next tile is requested before the current one is computed.
-    struct Tile {
-        Chunk<BITS> kc, vc;
-        T sk, bk, sv, bv;
-    };
-    auto fetch = [&](int s0) {
-        const int s = s0 + j;
-        const int64_t r = row0 + (s < s_end ? s : S - 1);  // a key past the end reads the last one and is given no weight
-        Tile t;
-        t.kc = load_chunk<BITS>(kw + (r * CH + c) * CW), t.vc = load_chunk<BITS>(vw + (r * CH + c) * CW);
-        t.sk = ks[r * groups + gi], t.bk = kb[r * groups + gi], t.sv = vs[r * groups + gi], t.bv = vb[r * groups + gi];
-        return t;
-    };
-    Tile cur = fetch(s_begin + wave * KPT);
-    for (int s0 = s_begin + wave * KPT; s0 < s_end; s0 += kAttnWaves * KPT) {
-        const Tile nxt = fetch(s0 + kAttnWaves * KPT);  // (past the end: valid addresses, nothing of it is used)
-        const bool live = s0 + j < s_end;
-        const float sk = Elem<T>::load(&cur.sk, 0), bk = Elem<T>::load(&cur.bk, 0);
-        const float sv = Elem<T>::load(&cur.sv, 0), bv = Elem<T>::load(&cur.bv, 0);
-        float dot = 0.0f;
-#pragma unroll
-        for (int i = 0; i < CPL; i++) dot = __builtin_fmaf(qv[i], chunk_code<BITS>(cur.kc, i), dot);
-        float score = __builtin_fmaf(sk, dot, bk * qsum);
-#pragma unroll
-        for (int o = 1; o < CH; o <<= 1) score += __shfl_xor(score, o);  // the lanes of a key sit side by side
-        if (!live) score = -INFINITY;
-        const float m_new = fmaxf(m, score);
-        // (a slot that has seen no live key keeps m = -inf: its weights are zero, not NaN)
-        const float corr = m_new == -INFINITY ? 1.0f : __expf(m - m_new), p = m_new == -INFINITY ? 0.0f : __expf(score - m_new);
-        m = m_new;
-        l = __builtin_fmaf(l, corr, p);
-        const float pv = p * sv;
-        accb = __builtin_fmaf(accb, corr, p * bv);
-#pragma unroll
-        for (int i = 0; i < CPL; i++) acc[i] = __builtin_fmaf(acc[i], corr, pv * chunk_code<BITS>(cur.vc, i));
-        cur = nxt;
-    }
-
-    // merge: the block's maximum, every slot scaled to it, the slots added up
-    const int slot = wave * KPT + j;
-    if (c == 0) slot_m[slot] = m;
-    __syncthreads();
-    float top = -INFINITY;
-    for (int t = 0; t < kSlots; t++) top = fmaxf(top, slot_m[t]);
-    const float w = m == -INFINITY ? 0.0f : __expf(m - top);
-    if (c == 0) slot_l[slot] = l * w;
-#pragma unroll
-    for (int i = 0; i < CPL; i++) part[slot][c * CPL + i] = (acc[i] + accb) * w;
-    __syncthreads();
-    if (tid < D) {
-        float denom = 0.0f, sum = 0.0f;
-        for (int t = 0; t < kSlots; t++) {
-            denom += slot_l[t];
-            sum += part[t][tid];
+        for (int j = 0; j < 8; j++) {
+            const int at = quarter * (D / 4) + 8 * s + code_at<BITS>(j);
+            v[j] = head < rep && at / (D / G) == g ? Elem<T>::load(q, (head0 + head) * D + at) : 0.0f;
+            qsum += v[j];
         }
-        const int64_t head = (int64_t)b * d.query_heads + h;
+        uint32_t t[4][TQ];
+#pragma unroll
+        for (int j = 0; j < 4; j++) split_pair<TQ>(v[2 * j], v[2 * j + 1], t[j]);
+#pragma unroll
+        for (int i = 0; i < TQ; i++) qf[s][i] = make_uint4(t[0][i], t[1][i], t[2][i], t[3][i]);
+    }
+    qsum += __shfl_xor(qsum, 16);
+    qsum += __shfl_xor(qsum, 32);
+
+    // What a tile of 32 keys reads from memory; the next tile's keys are requested when this one's have become operands, its
+    // values likewise.
+    constexpr int kRun = G * (int)sizeof(T);  // bytes of a key's scales
+    struct Quad { uint32_t w[kRun]; };        // of four consecutive keys
+    struct KeyTile {
+        uint32_t c[2][(kChunk + 3) / 4];
+        Quad s[2], b[2];
+    } kt;
+    struct ValueTile {
+        uint32_t c[8][(kSlot + 31) / 32];
+        Quad s[2], b[2];
+    } vt;
+    const uint8_t *kbytes = reinterpret_cast<const uint8_t *>(kw), *vbytes = reinterpret_cast<const uint8_t *>(vw);
+    auto four = [&](const T *p, int key) {
+        const uint8_t *at = reinterpret_cast<const uint8_t *>(p + row0 * G);
+        Quad o;
+        if (key + 4 <= S) {
+#pragma unroll
+            for (int i = 0; i < kRun; i++) o.w[i] = load_any<uint32_t>(at + (int64_t)key * kRun + 4 * i);
+            return o;
+        }
+#pragma unroll
+        for (int i = 0; i < kRun; i++) {  // word i: of key 4 i / kRun, or (one half-precision group) of keys 2 i and 2 i + 1
+            if constexpr (kRun >= 4) {
+                const int k = key + 4 * i / kRun;
+                o.w[i] = load_any<uint32_t>(at + (int64_t)(k < S ? k : S - 1) * kRun + 4 * i % kRun);
+            } else {
+                const int k0 = key + 2 * i, k1 = k0 + 1;
+                o.w[i] = (uint32_t)load_any<uint16_t>(at + (int64_t)(k0 < S ? k0 : S - 1) * 2) |
+                         (uint32_t)load_any<uint16_t>(at + (int64_t)(k1 < S ? k1 : S - 1) * 2) << 16;
+            }
+        }
+        return o;
+    };
+    auto fetch_keys = [&](int s0) {
+        if (s0 >= s_end) return;  // (nothing is left for this wavefront)
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            int key = s0 + 16 * h + l;
+            key = key < S ? key : S - 1;  // a key past the end reads the last one and is given no weight
+            const uint8_t *row = kbytes + (row0 + key) * kRowBytes;
+            if constexpr (kChunk % 4 == 0) {
+                struct Words { uint32_t w[kChunk / 4]; };
+                const Words w = *reinterpret_cast<const Words *>(row + quarter * kChunk);
+#pragma unroll
+                for (int i = 0; i < kChunk / 4; i++) kt.c[h][i] = w.w[i];
+            } else {  // 6 bytes (16 codes of 3 bits): 8 from where they stay inside the row
+                const int at = quarter * kChunk < kRowBytes - 8 ? quarter * kChunk : kRowBytes - 8;
+                const uint64_t w = load_any<uint64_t>(row + at) >> (8 * (quarter * kChunk - at));
+                kt.c[h][0] = (uint32_t)w, kt.c[h][1] = (uint32_t)(w >> 32);
+            }
+            kt.s[h] = four(ks, s0 + 16 * h + 4 * quarter), kt.b[h] = four(kb, s0 + 16 * h + 4 * quarter);
+        }
+    };
+    auto fetch_values = [&](int s0) {
+        if (s0 >= s_end) return;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            int key = s0 + 16 * (j >> 2) + 4 * quarter + (j & 3);
+            key = key < S ? key : S - 1;
+            const uint8_t *row = vbytes + (row0 + key) * kRowBytes;
+            if constexpr (kSlot == 64) {
+                const uint2 w = *reinterpret_cast<const uint2 *>(row + 8 * l);
+                vt.c[j][0] = w.x, vt.c[j][1] = w.y;
+            } else if constexpr (kSlot == 32) {
+                vt.c[j][0] = *reinterpret_cast<const uint32_t *>(row + 4 * l);
+            } else if constexpr (kSlot == 16) {
+                vt.c[j][0] = *reinterpret_cast<const uint16_t *>(row + 2 * l);
+            } else if constexpr (kSlot == 24) {
+                vt.c[j][0] = load_any<uint32_t>(row + 3 * l - (l == 15)) >> (l == 15 ? 8 : 0);
+            } else {  // 12 bits
+                vt.c[j][0] = load_any<uint16_t>(row + 3 * l / 2) >> (4 * (l & 1));
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < 2; h++) vt.s[h] = four(vs, s0 + 16 * h + 4 * quarter), vt.b[h] = four(vb, s0 + 16 * h + 4 * quarter);
+    };
+    // The lane's own group of key i.
+    const int down = 16 * (g & 1), up = 16 - down;
+    auto pick = [&](const Quad &o, int i) {
+        if constexpr (sizeof(T) == 4) {
+            uint32_t w = o.w[G * i];
+#pragma unroll
+            for (int e = 1; e < G; e++) w = g == e ? o.w[G * i + e] : w;
+            return u2f(w);
+        } else {
+            uint32_t w = o.w[G * i / 2];
+            if constexpr (G == 4) w = g >= 2 ? o.w[2 * i + 1] : w;
+            if constexpr (Elem<T>::code == 10) {
+                if constexpr (G == 1) return u2f(i & 1 ? w & 0xFFFF0000u : w << 16);
+                return u2f((w << up) & 0xFFFF0000u);
+            } else {
+                return (float)__builtin_bit_cast(f16_t, (uint16_t)(w >> (G == 1 ? 16 * (i & 1) : down)));
+            }
+        }
+    };
+
+    floatx4_t acc[ND], ones = {0.0f, 0.0f, 0.0f, 0.0f};
+    float m = -1.0e30f, denom = 0.0f, accb = 0.0f;
+#pragma unroll
+    for (int i = 0; i < ND; i++) acc[i] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    fetch_keys(s_begin + wave * kTileKeys);
+    fetch_values(s_begin + wave * kTileKeys);
+    for (int s0 = s_begin + wave * kTileKeys; s0 < s_end; s0 += kAttnWaves * kTileKeys) {
+        float score[8];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            floatx4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int s = 0; s < KS; s++) {
+                uint4 kf;
+                if constexpr (BITS == 8) {
+                    kf = eight_codes<8>(kt.c[h][2 * s], kt.c[h][2 * s + 1]);
+                } else if constexpr (BITS == 4) {
+                    kf = eight_codes<4>(kt.c[h][s], 0);
+                } else {
+                    constexpr int W = (kChunk + 3) / 4;
+                    const int bit = 24 * s, w = bit / 32, sh = bit % 32;
+                    kf = eight_codes<3>(sh == 0 ? kt.c[h][w] : __builtin_amdgcn_alignbit(kt.c[h][w + 1 < W ? w + 1 : w], kt.c[h][w], sh), 0);
+                }
+#pragma unroll
+                for (int i = 0; i < TQ; i++) sum = mfma16(kf, qf[s][i], sum);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float sk = pick(kt.s[h], r), bk = pick(kt.b[h], r);
+                float v = __builtin_fmaf(sk, sum[r], __builtin_fmaf(-kOffset<BITS>, sk, bk) * qsum);
+                // the groups of a row: columns R apart
+                if constexpr (G == 4) v += u2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2u(v), 0x124, 0xF, 0xF, true));
+                if constexpr (G >= 2) v += u2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2u(v), 0x128, 0xF, 0xF, true));
+                score[4 * h + r] = s0 + 16 * h + 4 * quarter + r < s_end ? v * scale : -INFINITY;
+            }
+        }
+        fetch_keys(s0 + kAttnWaves * kTileKeys);
+        float top = score[0];
+#pragma unroll
+        for (int j = 1; j < 8; j++) top = fmaxf(top, score[j]);
+        // The sums are rescaled only when a maximum has grown by more than 2^8; until then weights are at most 2^8.
+        if (__any(top > m + 8.0f)) {
+            top = fmaxf(top, __shfl_xor(top, 16));
+            top = fmaxf(top, __shfl_xor(top, 32));
+            const float m_new = fmaxf(m, top), f = exp2f(m - m_new);
+            m = m_new, denom *= f, accb *= f;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                ones[r] *= f;
+#pragma unroll
+                for (int i = 0; i < ND; i++) acc[i][r] *= f;
+            }
+        }
+        float w[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const float p = __builtin_amdgcn_exp2f(score[j] - m);
+            denom += p;
+            accb = __builtin_fmaf(p, pick(vt.b[j >> 2], j & 3), accb);
+            w[j] = p * pick(vt.s[j >> 2], j & 3);
+        }
+        uint32_t t[4][TP];
+        uint4 pf[TP];
+#pragma unroll
+        for (int j = 0; j < 4; j++) split_pair<TP>(w[2 * j], w[2 * j + 1], t[j]);
+#pragma unroll
+        for (int e = 0; e < TP; e++) {
+            pf[e] = make_uint4(t[0][e], t[1][e], t[2][e], t[3][e]);
+            if constexpr (kOnes) ones = mfma16(make_uint4(kMagic, kMagic, kMagic, kMagic), pf[e], ones);
+        }
+        // value i of the lane's slot, two keys a word
+#pragma unroll
+        for (int i = 0; i < ND; i++) {
+            uint32_t p[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if constexpr (BITS == 8) {
+                    const int w = i / 4;
+                    const uint32_t x = vt.c[2 * j][w] >> (8 * (i % 4)), y = vt.c[2 * j + 1][w] >> (8 * (i % 4));
+                    p[j] = pack_exact((float)(x & 0xFFu), (float)(y & 0xFFu));
+                } else {
+                    constexpr uint32_t mask = BITS == 4 ? 0x000F000Fu : 0x00070007u;
+                    // sixteen bits of each key that hold the code, side by side
+                    const bool high = BITS * i + BITS > 16;
+                    const int from = BITS == 4 ? 16 : 8;  // the second piece's first bit
+                    const uint32_t sel = !high ? 0x05040100u : BITS == 4 ? 0x07060302u : 0x06050201u;
+                    const uint32_t both = __builtin_amdgcn_perm(vt.c[2 * j + 1][0], vt.c[2 * j][0], sel);
+                    p[j] = ((both >> (BITS * i - (high ? from : 0))) & mask) | kMagic;
+                }
+            }
+            const uint4 vf = make_uint4(p[0], p[1], p[2], p[3]);
+#pragma unroll
+            for (int e = 0; e < TP; e++) acc[i] = mfma16(vf, pf[e], acc[i]);
+        }
+        fetch_values(s0 + kAttnWaves * kTileKeys);
+    }
+
+    // merge: the block's maximum, every wavefront scaled to it, the wavefronts added up
+    denom += __shfl_xor(denom, 16), accb += __shfl_xor(accb, 16);
+    denom += __shfl_xor(denom, 32), accb += __shfl_xor(accb, 32);
+    if (head < rep) {
+        if (lane < R) wave_m[wave][head] = m, wave_l[wave][head] = denom;
+#pragma unroll
+        for (int i = 0; i < ND; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int at = ND * (4 * quarter + r) + i;  // of D: this column's group has it or another column's
+                // (128 + code and 128 alone went through the same sums)
+                if (at / (D / G) == g) part[wave][head][at] = acc[i][r] - (kOnes ? ones[r] : 0.0f) + accb;
+            }
+    }
+    __syncthreads();
+    for (int e = tid; e < rep * D; e += 64 * kAttnWaves) {
+        const int hd = e / D, at = e % D;
+        float top = -1.0e30f;
+#pragma unroll
+        for (int w = 0; w < kAttnWaves; w++) top = fmaxf(top, wave_m[w][hd]);
+        float sum = 0.0f, total = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kAttnWaves; w++) {
+            const float f = exp2f(wave_m[w][hd] - top);
+            total = __builtin_fmaf(wave_l[w][hd], f, total);
+            sum = __builtin_fmaf(part[w][hd][at], f, sum);
+        }
         if (splits == 1) {
-            const bool has_sink = sinks != nullptr;
-            Elem<T>::store(out, head * D + tid, attention_finish(sum, denom, top, has_sink ? Elem<T>::load(sinks, h) : 0.0f, has_sink));
-        } else {  // this split's state: maximum, denominator, weighted sum
-            float *dst = partials + (head * splits + blockIdx.z) * (D + 2);
-            if (tid == 0) dst[0] = top, dst[1] = denom;
-            dst[2 + tid] = sum;
+            if (sinks != nullptr) {
+                const float sink = Elem<T>::load(sinks, hk * all + first + hd) * kLog2e, t2 = fmaxf(top, sink), f = exp2f(top - t2);
+                sum *= f, total = total * f + exp2f(sink - t2);
+            }
+            Elem<T>::store(out, (head0 + hd) * D + at, sum / total);
+        } else {  // this split's state: maximum (of base-2 scores), denominator, weighted sum
+            float *dst = partials + ((head0 + hd) * splits + split) * (D + 2);
+            if (at == 0) dst[0] = top, dst[1] = total;
+            dst[2 + at] = sum;
         }
     }
 }
@@ -171,25 +375,29 @@ __global__ void __launch_bounds__(D) qattn_merge_kernel(const nvq_attention_desc
                                                         const T *__restrict__ sinks, T *__restrict__ out) {
     const int64_t head = (int64_t)blockIdx.y * d.query_heads + blockIdx.x;
     const float *src = partials + head * splits * (D + 2);
-    float top = -INFINITY;
+    float top = -1.0e30f;
     for (int z = 0; z < splits; z++) top = fmaxf(top, src[z * (D + 2)]);
-    float denom = 0.0f, sum = 0.0f;
+    const bool has_sink = sinks != nullptr;
+    const float sink = has_sink ? Elem<T>::load(sinks, blockIdx.x) * kLog2e : 0.0f;
+    if (has_sink) top = fmaxf(top, sink);
+    float denom = has_sink ? exp2f(sink - top) : 0.0f, sum = 0.0f;
     for (int z = 0; z < splits; z++) {
-        const float mz = src[z * (D + 2)], w = mz == -INFINITY ? 0.0f : __expf(mz - top);
+        const float w = exp2f(src[z * (D + 2)] - top);
         denom = __builtin_fmaf(src[z * (D + 2) + 1], w, denom);
         sum = __builtin_fmaf(src[z * (D + 2) + 2 + threadIdx.x], w, sum);
     }
-    const bool has_sink = sinks != nullptr;
-    Elem<T>::store(out, head * D + threadIdx.x,
-                   attention_finish(sum, denom, top, has_sink ? Elem<T>::load(sinks, blockIdx.x) : 0.0f, has_sink));
+    Elem<T>::store(out, head * D + threadIdx.x, sum / denom);
 }
 
-template <typename T, int BITS, int D>
-int32_t run_attention_sized(const nvq_attention_desc &d, const void *q, const void *kw, const void *ks, const void *kb, const void *vw,
-                            const void *vs, const void *vb, const void *sinks, void *out, void *workspace, hipStream_t s) {
+int attention_splits(const nvq_attention_desc &d);
+
+template <typename T, int BITS, int D, int G>
+int32_t run_attention_grouped(const nvq_attention_desc &d, const void *q, const void *kw, const void *ks, const void *kb, const void *vw,
+                              const void *vs, const void *vb, const void *sinks, void *out, void *workspace, hipStream_t s) {
     const int splits = workspace != nullptr ? attention_splits(d) : 1;
-    const dim3 grid((unsigned)d.query_heads, (unsigned)d.batch, (unsigned)splits), block(64 * kAttnWaves);
-    hipLaunchKernelGGL((qattn_kernel<T, BITS, D>), grid, block, 0, s, d, (const T *)q, (const uint32_t *)kw, (const T *)ks, (const T *)kb,
+    const int64_t parts = (d.query_heads / d.key_heads + 16 / G - 1) / (16 / G);
+    const dim3 grid((unsigned)d.key_heads, (unsigned)d.batch, (unsigned)(splits * parts)), block(64 * kAttnWaves);
+    hipLaunchKernelGGL((qattn_kernel<T, BITS, D, G>), grid, block, 0, s, d, (const T *)q, (const uint32_t *)kw, (const T *)ks, (const T *)kb,
                        (const uint32_t *)vw, (const T *)vs, (const T *)vb, (const T *)sinks, (T *)out, (float *)workspace);
     NVQ_LAUNCH_CHECK("quantized_attention");
     if (splits > 1) {
@@ -198,6 +406,17 @@ int32_t run_attention_sized(const nvq_attention_desc &d, const void *q, const vo
         NVQ_LAUNCH_CHECK("quantized_attention merge");
     }
     return NVQ_OK;
+}
+
+template <typename T, int BITS, int D>
+int32_t run_attention_sized(const nvq_attention_desc &d, const void *q, const void *kw, const void *ks, const void *kb, const void *vw,
+                            const void *vs, const void *vb, const void *sinks, void *out, void *workspace, hipStream_t s) {
+    const int groups = D / d.group_size;
+    if (groups == 1) return run_attention_grouped<T, BITS, D, 1>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s);
+    if (groups == 2) return run_attention_grouped<T, BITS, D, 2>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s);
+    if constexpr (D == 128)  // (groups have 32 values at least)
+        return run_attention_grouped<T, BITS, D, 4>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s);
+    return NVQ_UNSUPPORTED;
 }
 
 template <typename T, int BITS>
@@ -215,20 +434,21 @@ int32_t run_attention_bits(const nvq_attention_desc &d, const void *q, const voi
                          : run_attention<T, 8>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s);
 }
 
-}  // namespace
-
-// Splits of the positions over the grid: about two blocks per compute unit, at least 256 keys a split, at most 64 splits.
+// Splits of the positions over the grid: three blocks of four wavefronts per compute unit (what the kernels' registers let
+// run together), at least two tiles a wavefront, at most 64 splits.
 int attention_splits(const nvq_attention_desc &d) {
-    const int64_t heads = d.batch * d.query_heads;
-    if (heads <= 0 || d.positions < 512) return 1;
-    int64_t want = (2 * (int64_t)compute_units() + heads - 1) / heads;
-    const int64_t most = d.positions / 256;
+    const int64_t heads = d.batch * d.key_heads;
+    if (heads <= 0) return 1;
+    int64_t want = 3 * (int64_t)compute_units() / heads;
+    const int64_t most = d.positions / (2 * kAttnWaves * kTileKeys);
     want = want > most ? most : want;
     want = want > 64 ? 64 : want;
     if (want < 2) return 1;
     const int per = attention_split_keys(d.positions, (int)want);  // whole tiles: fewer splits may cover the positions
     return (int)((d.positions + per - 1) / per);
 }
+
+}  // namespace
 
 size_t attention_workspace_bytes(const nvq_attention_desc &d) {
     const int splits = attention_splits(d);

@@ -22,6 +22,7 @@
 // Lanes.  Lane (quarter q, l) holds in S^T column l of keys 4 q .. + 3 of two tiles of 16 keys: they are the eight keys of its
 // operand P^T (the contraction's order is free), and of V it loads D / 16 codes, l's slot of the row, of the same eight keys.
 // No value crosses lanes but the groups' sums, and maxima when they grow.
+#include "attention_merge.h"
 #include "nvq_device.h"
 #include "nvq_internal.h"
 #include "qmf_kernel.h"
@@ -369,24 +370,13 @@ __global__ void __launch_bounds__(64 * kAttnWaves, sizeof(T) == 2 && G < 4 ? 3 :
     }
 }
 
-// The splits of one (batch, head) merged: block = D threads.
+// The splits of one (batch, head) merged.
 template <typename T, int D>
-__global__ void __launch_bounds__(D) qattn_merge_kernel(const nvq_attention_desc d, const float *__restrict__ partials, int splits,
-                                                        const T *__restrict__ sinks, T *__restrict__ out) {
+__global__ void __launch_bounds__(kMergeParts * D) qattn_merge_kernel(const nvq_attention_desc d, const float *__restrict__ partials, int splits,
+                                                                      const T *__restrict__ sinks, T *__restrict__ out) {
     const int64_t head = (int64_t)blockIdx.y * d.query_heads + blockIdx.x;
-    const float *src = partials + head * splits * (D + 2);
-    float top = -1.0e30f;
-    for (int z = 0; z < splits; z++) top = fmaxf(top, src[z * (D + 2)]);
-    const bool has_sink = sinks != nullptr;
-    const float sink = has_sink ? Elem<T>::load(sinks, blockIdx.x) * kLog2e : 0.0f;
-    if (has_sink) top = fmaxf(top, sink);
-    float denom = has_sink ? exp2f(sink - top) : 0.0f, sum = 0.0f;
-    for (int z = 0; z < splits; z++) {
-        const float w = exp2f(src[z * (D + 2)] - top);
-        denom = __builtin_fmaf(src[z * (D + 2) + 1], w, denom);
-        sum = __builtin_fmaf(src[z * (D + 2) + 2 + threadIdx.x], w, sum);
-    }
-    Elem<T>::store(out, head * D + threadIdx.x, sum / denom);
+    merge_attention_states<T, D>(partials + head * splits * (D + 2), D + 2, splits, sinks != nullptr,
+                                 sinks != nullptr ? Elem<T>::load(sinks, blockIdx.x) * kLog2e : 0.0f, out + head * D);
 }
 
 int attention_splits(const nvq_attention_desc &d);
@@ -401,7 +391,7 @@ int32_t run_attention_grouped(const nvq_attention_desc &d, const void *q, const 
                        (const uint32_t *)vw, (const T *)vs, (const T *)vb, (const T *)sinks, (T *)out, (float *)workspace);
     NVQ_LAUNCH_CHECK("quantized_attention");
     if (splits > 1) {
-        hipLaunchKernelGGL((qattn_merge_kernel<T, D>), dim3((unsigned)d.query_heads, (unsigned)d.batch), dim3(D), 0, s, d,
+        hipLaunchKernelGGL((qattn_merge_kernel<T, D>), dim3((unsigned)d.query_heads, (unsigned)d.batch), dim3(kMergeParts * D), 0, s, d,
                            (const float *)workspace, splits, (const T *)sinks, (T *)out);
         NVQ_LAUNCH_CHECK("quantized_attention merge");
     }
@@ -442,7 +432,7 @@ int attention_splits(const nvq_attention_desc &d) {
     int64_t want = 3 * (int64_t)compute_units() / heads;
     const int64_t most = d.positions / (2 * kAttnWaves * kTileKeys);
     want = want > most ? most : want;
-    want = want > 64 ? 64 : want;
+    want = want > 64 ? 64 : want;  // (a lane each when they are merged)
     if (want < 2) return 1;
     const int per = attention_split_keys(d.positions, (int)want);  // whole tiles: fewer splits may cover the positions
     return (int)((d.positions + per - 1) / per);

@@ -18,6 +18,7 @@
 //
 // What fills the chip: few rows are walked by several wavefronts of a block, each taking every KP-th tile of keys, and where
 // even that leaves compute units idle by several blocks whose float32 states a third kernel merges.
+#include "attention_merge.h"
 #include "nvq_device.h"
 #include "nvq_internal.h"
 #include "qmf_kernel.h"
@@ -253,26 +254,16 @@ __global__ void __launch_bounds__(64 * kWaves, 2) prompt_attention_kernel(const 
         }
 }
 
-// The splits of a row merged: block = D threads, one row.
+// The splits of a row merged.
 template <typename T, int D>
-__global__ void __launch_bounds__(D) prompt_merge_kernel(const PromptArgs a) {
+__global__ void __launch_bounds__(kMergeParts * D) prompt_merge_kernel(const PromptArgs a) {
     const int rows = a.rep * a.queries;
     const int64_t all = (int64_t)gridDim.x * gridDim.y;  // rows x (batch x key heads)
     const int r = blockIdx.x, head = blockIdx.y, b = head / a.key_heads, hk = head % a.key_heads;
-    const float *src = a.partials + ((int64_t)head * rows + r) * (D + 2);
-    float top = -1.0e30f;
-    for (int z = 0; z < a.splits; z++) top = fmaxf(top, src[z * all * (D + 2)]);
     const int h = hk * a.rep + r % a.rep, i = r / a.rep;
-    const bool has_sink = a.sinks != nullptr;
-    const float sink = has_sink ? Elem<T>::load((const T *)a.sinks, h) * kLog2e : 0.0f;
-    if (has_sink) top = fmaxf(top, sink);
-    float denom = has_sink ? exp2f(sink - top) : 0.0f, sum = 0.0f;
-    for (int z = 0; z < a.splits; z++) {
-        const float *p = src + z * all * (D + 2), w = exp2f(p[0] - top);
-        denom = __builtin_fmaf(p[1], w, denom);
-        sum = __builtin_fmaf(p[2 + threadIdx.x], w, sum);
-    }
-    Elem<T>::store((T *)a.out, (((int64_t)b * a.query_heads + h) * a.queries + i) * D + threadIdx.x, sum / denom);
+    merge_attention_states<T, D>(a.partials + ((int64_t)head * rows + r) * (D + 2), all * (D + 2), a.splits, a.sinks != nullptr,
+                                 a.sinks != nullptr ? Elem<T>::load((const T *)a.sinks, h) * kLog2e : 0.0f,
+                                 (T *)a.out + (((int64_t)b * a.query_heads + h) * a.queries + i) * D);
 }
 
 struct Plan {
@@ -320,7 +311,7 @@ int32_t run_rows(const PromptArgs &a, const Plan &p, hipStream_t s) {
     hipLaunchKernelGGL((prompt_attention_kernel<T, D, RG>), dim3((unsigned)blocks, (unsigned)p.splits), dim3(64 * kWaves), 0, s, a);
     NVQ_LAUNCH_CHECK("quantized_attention");
     if (p.splits > 1) {
-        hipLaunchKernelGGL((prompt_merge_kernel<T, D>), dim3((unsigned)p.rows, (unsigned)p.heads), dim3(D), 0, s, a);
+        hipLaunchKernelGGL((prompt_merge_kernel<T, D>), dim3((unsigned)p.rows, (unsigned)p.heads), dim3(kMergeParts * D), 0, s, a);
         NVQ_LAUNCH_CHECK("quantized_attention merge");
     }
     return NVQ_OK;

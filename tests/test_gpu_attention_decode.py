@@ -36,3 +36,16 @@ def test_edges(heads, key_heads, d, group, bits, dtype):
         u = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
         bound = (16 * 1.1e-6 + (0 if dtype == torch.float32 else 2.0 ** -17)) * vf.abs().max() + u * want.abs()
         assert ((got.double() - want).abs() <= bound).all(), (s, (got.double() - want).abs().max().item())
+
+
+@pytest.mark.parametrize("splits", [2, 3, 5, 31, 33, 64])
+def test_merged_splits(splits):
+    """One key head over 256 positions a split, up to the 64 splits that the kernel takes: lanes and groups of the merge that are
+    full, partly used and idle.  The queries are zeros: the weights are equal and the output is the mean of the values."""
+    s, d, quant = 256 * splits, 64, nv.Quant.affine(64, 4)
+    v = nv.quantize(torch.randn(1, 1, s, d, device="cuda"), quant)
+    k = nv.quantize(torch.randn(1, 1, s, d, device="cuda"), quant)
+    got = ops.quantized_attention(torch.zeros(1, 2, 1, d, device="cuda"), k, v, 1.0)
+    want = nv.dequantize(v).double().mean(-2, keepdim=True)
+    # (as above: the float32 sums' random roundings)
+    assert (got.double() - want).abs().max() <= 16 * 1.1e-6 * nv.dequantize(v).abs().max()

@@ -8,7 +8,11 @@
 //
 // The bound is the stream of the cache, read once for all query heads of a key head, as long as turning codes into operands
 // costs little: both products run on the matrix cores over the CODES, which bfloat16 holds exactly (8 bits as they are, 3 and
-// 4 bits in the low mantissa bits of 128: one instruction per two codes, the 128 taken out again by the sums it multiplies).
+// 4 bits in the mantissa of 8 and 16: one instruction per two codes, the 8 or 16 taken out again by the sums it multiplies;
+// in the mantissa of 128 float32 results lost a digit).  The values' sums count codes from the middle of their range, as large
+// as the values around their mean, so that the weights' rounding is not multiplied by the range: the operands themselves in
+// float32, else by an operand of the offset and the middle alone that goes through the same sums.  Errors against float64, from
+// dequantized values -> here: float16 2.08e-4 -> 2.08e-4 (the output's rounding), float32 3.9e-7 .. 5.8e-7 -> 2.0e-7 .. 2.5e-7.
 // What is not exact in bfloat16, the queries of the wider types and the softmax's weights, goes in as the sum of two or three
 // bfloat16 terms (16 or 24 bits): TQ and TP below.
 //
@@ -46,9 +50,16 @@ __device__ __forceinline__ V load_any(const void *p) {
     return reinterpret_cast<const Raw *>(p)->v;
 }
 
-// The 3- and 4-bit codes' operands are 128 + code.
-template <int BITS> constexpr float kOffset = BITS == 8 ? 0.0f : 128.0f;
-constexpr uint32_t kMagic = 0x43004300u;
+// An operand is kOffset + code.  WIDE: float32.
+template <int BITS, bool WIDE> constexpr float kOffset = WIDE ? -(float)(1 << (BITS - 1)) : BITS == 8 ? 0.0f : (float)(1 << BITS);
+template <int BITS> constexpr uint32_t kMagic = BITS == 4 ? 0x41804180u : 0x41004100u;  // two of 2^BITS, BITS < 8
+// Codes at bit `at` of both halves of a word as 2^BITS + code.
+template <int BITS>
+__device__ __forceinline__ uint32_t two_codes(uint32_t z, int at) {
+    constexpr int to = 7 - BITS;  // the code's place in the mantissa
+    constexpr uint32_t mask = ((1u << BITS) - 1u) * 0x00010001u << to;
+    return ((at >= to ? z >> (at - to) : z << (to - at)) & mask) | kMagic<BITS>;
+}
 
 // Two exact bfloat16 values from two floats that bfloat16 holds.
 __device__ __forceinline__ uint32_t pack_exact(float lo, float hi) { return __builtin_amdgcn_perm(f2u(hi), f2u(lo), 0x07060302u); }
@@ -57,15 +68,21 @@ __device__ __forceinline__ uint32_t pack_exact(float lo, float hi) { return __bu
 template <int BITS> constexpr int code_at(int j) { return BITS == 8 ? j : (j >> 1) + 4 * (j & 1); }
 
 // Eight consecutive codes of a row (BITS bytes in the low bits of w0, w1) as an operand, in the order of code_at.
-template <int BITS>
+template <int BITS, bool WIDE>
 __device__ __forceinline__ uint4 eight_codes(uint32_t w0, uint32_t w1) {
-    if constexpr (BITS == 8) {
+    if constexpr (WIDE) {
+        auto at = [&](int j) {
+            const int i = code_at<BITS>(j);
+            const uint32_t c = BITS == 8 ? (i < 4 ? w0 >> (8 * i) : w1 >> (8 * (i - 4))) & 0xFFu : (w0 >> (BITS * i)) & ((1u << BITS) - 1u);
+            return (float)c + kOffset<BITS, true>;
+        };
+        return make_uint4(pack_exact(at(0), at(1)), pack_exact(at(2), at(3)), pack_exact(at(4), at(5)), pack_exact(at(6), at(7)));
+    } else if constexpr (BITS == 8) {
         return make_uint4(pack_exact(qmf::ubyte_to_float<0>(w0), qmf::ubyte_to_float<1>(w0)), pack_exact(qmf::ubyte_to_float<2>(w0), qmf::ubyte_to_float<3>(w0)),
                           pack_exact(qmf::ubyte_to_float<0>(w1), qmf::ubyte_to_float<1>(w1)), pack_exact(qmf::ubyte_to_float<2>(w1), qmf::ubyte_to_float<3>(w1)));
     } else {
-        constexpr uint32_t mask = BITS == 4 ? 0x000F000Fu : 0x00070007u;
         const uint32_t z = BITS == 4 ? w0 : (w0 & 0xFFFu) | ((w0 & 0xFFF000u) << 4);  // code i at bit BITS i, code i + 4 sixteen above
-        return make_uint4((z & mask) | kMagic, ((z >> BITS) & mask) | kMagic, ((z >> (2 * BITS)) & mask) | kMagic, ((z >> (3 * BITS)) & mask) | kMagic);
+        return make_uint4(two_codes<BITS>(z, 0), two_codes<BITS>(z, BITS), two_codes<BITS>(z, 2 * BITS), two_codes<BITS>(z, 3 * BITS));
     }
 }
 
@@ -97,7 +114,11 @@ __global__ void __launch_bounds__(64 * kAttnWaves, sizeof(T) == 2 && G < 4 ? 3 :
     constexpr int TP = sizeof(T) == 4 ? 3 : 2;                            // terms of the weights: 24 or 16 bits
     constexpr int R = 16 / G, KS = D / 32, ND = D / 16;  // heads per operand; instructions of K per 16 keys; values of D per lane
     constexpr int kRowBytes = D * BITS / 8, kChunk = kRowBytes / 4, kSlot = BITS * ND;  // bytes of a quarter's codes; bits of a lane's slot
-    constexpr bool kOnes = kOffset<BITS> != 0.0f;
+    constexpr bool kWide = sizeof(T) == 4;
+    constexpr float kOff = kOffset<BITS, kWide>;
+    constexpr float kMiddle = 1 << (BITS - 1);
+    constexpr bool kOnes = !kWide;  // (the weights' sum beside the codes)
+    constexpr uint32_t kOne = BITS == 8 ? 0x43004300u : BITS == 4 ? 0x41C041C0u : 0x41404140u;  // two of kOff + kMiddle: 128, 24, 12 (at 8, 4, 3 bits)
     constexpr int kHeads = R < 8 ? R : 8;  // (at most eight query heads per key head)
     __shared__ float part[kAttnWaves][kHeads][D + 1];
     __shared__ float wave_m[kAttnWaves][kHeads], wave_l[kAttnWaves][kHeads];
@@ -247,13 +268,13 @@ __global__ void __launch_bounds__(64 * kAttnWaves, sizeof(T) == 2 && G < 4 ? 3 :
             for (int s = 0; s < KS; s++) {
                 uint4 kf;
                 if constexpr (BITS == 8) {
-                    kf = eight_codes<8>(kt.c[h][2 * s], kt.c[h][2 * s + 1]);
+                    kf = eight_codes<8, kWide>(kt.c[h][2 * s], kt.c[h][2 * s + 1]);
                 } else if constexpr (BITS == 4) {
-                    kf = eight_codes<4>(kt.c[h][s], 0);
+                    kf = eight_codes<4, kWide>(kt.c[h][s], 0);
                 } else {
                     constexpr int W = (kChunk + 3) / 4;
                     const int bit = 24 * s, w = bit / 32, sh = bit % 32;
-                    kf = eight_codes<3>(sh == 0 ? kt.c[h][w] : __builtin_amdgcn_alignbit(kt.c[h][w + 1 < W ? w + 1 : w], kt.c[h][w], sh), 0);
+                    kf = eight_codes<3, kWide>(sh == 0 ? kt.c[h][w] : __builtin_amdgcn_alignbit(kt.c[h][w + 1 < W ? w + 1 : w], kt.c[h][w], sh), 0);
                 }
 #pragma unroll
                 for (int i = 0; i < TQ; i++) sum = mfma16(kf, qf[s][i], sum);
@@ -261,7 +282,7 @@ __global__ void __launch_bounds__(64 * kAttnWaves, sizeof(T) == 2 && G < 4 ? 3 :
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const float sk = pick(kt.s[h], r), bk = pick(kt.b[h], r);
-                float v = __builtin_fmaf(sk, sum[r], __builtin_fmaf(-kOffset<BITS>, sk, bk) * qsum);
+                float v = __builtin_fmaf(sk, sum[r], __builtin_fmaf(-kOff, sk, bk) * qsum);
                 // the groups of a row: columns R apart
                 if constexpr (G == 4) v += u2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2u(v), 0x124, 0xF, 0xF, true));
                 if constexpr (G >= 2) v += u2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2u(v), 0x128, 0xF, 0xF, true));
@@ -290,8 +311,9 @@ __global__ void __launch_bounds__(64 * kAttnWaves, sizeof(T) == 2 && G < 4 ? 3 :
         for (int j = 0; j < 8; j++) {
             const float p = __builtin_amdgcn_exp2f(score[j] - m);
             denom += p;
-            accb = __builtin_fmaf(p, pick(vt.b[j >> 2], j & 3), accb);
-            w[j] = p * pick(vt.s[j >> 2], j & 3);
+            const float sv = pick(vt.s[j >> 2], j & 3), bv = pick(vt.b[j >> 2], j & 3);
+            accb = __builtin_fmaf(p, __builtin_fmaf(kMiddle, sv, bv), accb);
+            w[j] = p * sv;
         }
         uint32_t t[4][TP];
         uint4 pf[TP];
@@ -300,7 +322,7 @@ __global__ void __launch_bounds__(64 * kAttnWaves, sizeof(T) == 2 && G < 4 ? 3 :
 #pragma unroll
         for (int e = 0; e < TP; e++) {
             pf[e] = make_uint4(t[0][e], t[1][e], t[2][e], t[3][e]);
-            if constexpr (kOnes) ones = mfma16(make_uint4(kMagic, kMagic, kMagic, kMagic), pf[e], ones);
+            if constexpr (kOnes) ones = mfma16(make_uint4(kOne, kOne, kOne, kOne), pf[e], ones);
         }
         // value i of the lane's slot, two keys a word
 #pragma unroll
@@ -308,18 +330,21 @@ __global__ void __launch_bounds__(64 * kAttnWaves, sizeof(T) == 2 && G < 4 ? 3 :
             uint32_t p[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                if constexpr (BITS == 8) {
+                if constexpr (kWide) {
+                    const int w = BITS * i / 32, sh = BITS * i % 32;  // (a code of 3 bits: within the slot's 12 or 24)
+                    constexpr uint32_t mask = (1u << BITS) - 1u;
+                    p[j] = pack_exact((float)((vt.c[2 * j][w] >> sh) & mask) + kOff, (float)((vt.c[2 * j + 1][w] >> sh) & mask) + kOff);
+                } else if constexpr (BITS == 8) {
                     const int w = i / 4;
                     const uint32_t x = vt.c[2 * j][w] >> (8 * (i % 4)), y = vt.c[2 * j + 1][w] >> (8 * (i % 4));
                     p[j] = pack_exact((float)(x & 0xFFu), (float)(y & 0xFFu));
                 } else {
-                    constexpr uint32_t mask = BITS == 4 ? 0x000F000Fu : 0x00070007u;
                     // sixteen bits of each key that hold the code, side by side
                     const bool high = BITS * i + BITS > 16;
                     const int from = BITS == 4 ? 16 : 8;  // the second piece's first bit
                     const uint32_t sel = !high ? 0x05040100u : BITS == 4 ? 0x07060302u : 0x06050201u;
                     const uint32_t both = __builtin_amdgcn_perm(vt.c[2 * j + 1][0], vt.c[2 * j][0], sel);
-                    p[j] = ((both >> (BITS * i - (high ? from : 0))) & mask) | kMagic;
+                    p[j] = two_codes<BITS>(both, BITS * i - (high ? from : 0));
                 }
             }
             const uint4 vf = make_uint4(p[0], p[1], p[2], p[3]);
@@ -339,7 +364,7 @@ __global__ void __launch_bounds__(64 * kAttnWaves, sizeof(T) == 2 && G < 4 ? 3 :
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const int at = ND * (4 * quarter + r) + i;  // of D: this column's group has it or another column's
-                // (128 + code and 128 alone went through the same sums)
+                // (the operands and kOff + kMiddle alone went through the same sums)
                 if (at / (D / G) == g) part[wave][head][at] = acc[i][r] - (kOnes ? ones[r] : 0.0f) + accb;
             }
     }

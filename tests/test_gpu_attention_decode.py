@@ -1,7 +1,7 @@
 """The decode attention kernel (csrc/qattn.hip) at the edges of its tiles and column layouts against float64 attention over
 the dequantized cache.  Bound, of the largest value: the codes, the float32 queries' three bfloat16 terms and their products
-are exact; the sums are float32 over 128 + code, at most 2^-24 x 143 x scale a rounding with scale <= 2 max / 15, i.e. 1.1e-6
-max, and their roundings are random: sixteen of them.  In the 16-bit types one rounding of the output beside it, and the
+are exact; the sums are float32 over operands of at most 143 x scale (the scores' of 8 bits 255, with a scale a sixteenth as large), 2^-24 of
+that a rounding, with scale <= 2 max / 15, i.e. 1.1e-6 max, and their roundings are random: sixteen of them.  In the 16-bit types one rounding of the output beside it, and the
 weights' 16 bits (2^-17)."""
 import pytest
 import torch

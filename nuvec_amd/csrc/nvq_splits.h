@@ -51,7 +51,7 @@ inline double qmm_tiles_us(bool small, double tiles, double steps, int cus) {
 inline double qmm_estimate_us(bool small, const Product &a, int cus) {
     const int64_t t = small ? kQmmSmallTile : kQmmBigTile;
     const double tiles = (double)((a.m + t - 1) / t) * (double)((a.n + t - 1) / t) * (double)a.batch;
-    return qmm_tiles_us(small, tiles, (double)(a.k / kQmmStep), cus);
+    return qmm_tiles_us(small, tiles, (double)((a.k + kQmmStep - 1) / kQmmStep), cus);
 }
 inline bool qmm_small_tile_is_faster(const Product &a, int cus) {
     return a.exact_weights || qmm_estimate_us(true, a, cus) < qmm_estimate_us(false, a, cus);
@@ -61,7 +61,7 @@ inline bool qmm_small_tile_is_faster(const Product &a, int cus) {
 // partial sums (about 3 us to launch and 4 bytes per microsecond and compute unit... in all: 4 TB/s).  Each split has
 // at least eight steps, in whole table periods (four steps); at most eight splits; a batch is never split.
 inline Plan qmm_plan(const Product &a, int cus) {
-    const int64_t steps = a.k / kQmmStep;
+    const int64_t steps = (a.k + kQmmStep - 1) / kQmmStep;  // (the last one may be a half)
     const bool small = qmm_small_tile_is_faster(a, cus);
     Plan p{1, steps, steps, qmm_estimate_us(small, a, cus)};
     if (a.batch != 1) return p;

@@ -227,6 +227,13 @@ __device__ __forceinline__ uint4 expand_piece(const uint32_t (&dw)[BITS], float 
     return r;
 }
 
+// Whether a product of K off whole steps of 64 may take the kernels that hold weights in the element type: where that loses
+// nothing against the vector kernels that took it before, i.e. block formats without a global scale, whose weights the
+// element types hold exactly, and affine products that take the CPU's weights on either.
+inline bool half_steps_supported(const ProductArgs &a) {
+    return a.k % 32 == 0 && (a.mode == NVQ_AFFINE ? a.exact_weights != 0 : a.global_scale == nullptr);
+}
+
 // The LDS table of scales (or biases) of a block's rows keeps the memory order [row][group] with rows padded
 // to an odd number of dwords, so that the coalesced copy in writes neighbouring addresses and lanes reading
 // one group of consecutive rows fall on different banks.

@@ -5,7 +5,7 @@
 namespace nvq {
 
 // Whether the tiled kernel takes this product: a block format or affine 1 to 6 or 8 bits, bf16 or f16, whole
-// steps of 64 values, and a batch that is a single stride per operand (or no batch).
+// steps of 64 values or (half_steps_supported) steps and a half, and a batch that is a single stride per operand (or no batch).
 bool qmm_supported(const ProductArgs &a) {
     if (a.dtype != NVQ_BF16 && a.dtype != NVQ_F16) return false;
     if (a.mode == NVQ_AFFINE) {
@@ -13,7 +13,7 @@ bool qmm_supported(const ProductArgs &a) {
     }  // (NVFP4 with a global scale: the scaled weights are rounded to the element type like the affine ones)
     if (a.rhs != nullptr) return false;
     if (a.batch > 1 && a.batch_ndim != 1) return false;
-    return a.batch <= 65535 && a.k >= qmm::BK && a.k % qmm::BK == 0;
+    return a.batch <= 65535 && a.k >= qmm::BK && (a.k % qmm::BK == 0 || qmf::half_steps_supported(a));
 }
 
 // With its better tile and, for a single product, its better split of K (the caller is expected to bring the

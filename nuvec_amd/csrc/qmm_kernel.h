@@ -138,7 +138,8 @@ __device__ __forceinline__ uint32_t expand_dword(const uint32_t (&dw)[BITS], flo
 }
 
 // EXACT (affine codes): the weights as nuvec's CPU product holds them (affine_pair).
-template <typename T, int BITS, int FP4, bool BATCHED, class TL, bool EXACT = false>
+// HALF: K of whole steps and a half (an instantiation of its own: its tests cost products of whole steps 1 to 1.5 %).
+template <typename T, int BITS, int FP4, bool BATCHED, class TL, bool EXACT, bool HALF>
 __global__ void __launch_bounds__(TL::kThreads) __attribute__((amdgpu_waves_per_eu(TL::kWavesPerSimd, TL::kWavesPerSimd)))
 qmm_kernel(const ProductArgs a) {
     using G = Geometry<BITS, TL>;
@@ -164,7 +165,8 @@ qmm_kernel(const ProductArgs a) {
     const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
     // A single product may split K over grid z (few tiles, long K): this block takes the steps
     // [step0, step0 + steps) and leaves float32 partial sums for a second kernel.
-    int step0 = 0, steps = K / BK;  // K is a multiple of 64 (checked on the host)
+    int step0 = 0, steps = HALF ? (K + BK - 1) / BK : K / BK;  // K is a multiple of 64, or of 32 (checked on the host)
+    const int all_steps = steps;
     if constexpr (!BATCHED) {
         if (a.k_splits > 1) {
             step0 = blockIdx.z * a.k_split_steps;  // whole table periods
@@ -172,6 +174,11 @@ qmm_kernel(const ProductArgs a) {
             if (steps <= 0) return;  // (the host sizes the grid so that every split has a step)
         }
     }
+    // K of whole steps and a half: the last step begins 32 values early, so that every load stays inside its row.  The
+    // values that the step before has counted are zeros in both operands: the x tile's chunks 0..3 are overwritten in
+    // LDS once they have arrived, the lanes of half 0 take a scale and bias of zero.  (Passes of four rows on the vector
+    // kernel took these products before: 323 rows, W[2844,5088], NVFP4, 1311 us.)
+    const int half_step = step0 + steps == all_steps ? steps - 1 : -1;
     int64_t bx = 0, bw = 0, bs = 0, by = 0;
     if constexpr (BATCHED) {  // a batch with one stride per operand
         bx = (int64_t)blockIdx.z * a.x_strides[0];
@@ -215,9 +222,10 @@ qmm_kernel(const ProductArgs a) {
     auto loads_of = [&](int step, int stage) {
         const int sc = step < steps ? step : steps - 1;
         Loads l;
-        l.x = xbase + sc * (BK * 2);
+        const int early = HALF && sc == half_step ? 1 : 0;
+        l.x = xbase + sc * (BK * 2) - early * BK;
 #pragma unroll
-        for (int piece = 0; piece < P::count; piece++) l.w[piece] = wbase + sc * (2 * BITS * 4) + piece * (P::dwords * 4);
+        for (int piece = 0; piece < P::count; piece++) l.w[piece] = wbase + sc * (2 * BITS * 4) - early * (BITS * 4) + piece * (P::dwords * 4);
         l.lds = lds_wave + stage * G::kStageBytes;
         // computed here once, in scalar registers, not again at every load
         asm volatile("" : "+s"(l.x), "+s"(l.lds));
@@ -274,7 +282,9 @@ qmm_kernel(const ProductArgs a) {
     // The packed codes, scales and biases of this lane's TJ columns for `step` (its stage and table are visible).
     auto read_codes = [&](int step, int stage) {
         const unsigned char *ws = lds + stage * G::kStageBytes + kXBytes;
-        const uint32_t *sbt = sb_table + ((step >> pshift) & 1) * (kSbBytes / 4) + ((((step & (psteps - 1)) * BK + 32 * h) >> gshift) * BN);
+        const int within = HALF && step == half_step ? 0 : 32 * h;  // (half 1 of a half step holds the first values of its table slot)
+        const uint32_t live = HALF && step == half_step && h == 0 ? 0u : ~0u;
+        const uint32_t *sbt = sb_table + ((step >> pshift) & 1) * (kSbBytes / 4) + ((((step & (psteps - 1)) * BK + within) >> gshift) * BN);
 #pragma unroll
         for (int j = 0; j < TJ; j++) {
             const int col = wn * (32 * TJ) + j * 32 + l32;
@@ -289,9 +299,9 @@ qmm_kernel(const ProductArgs a) {
                     for (int d = 0; d < P::dwords; d++) raw[j][P::dwords * piece + d] = reinterpret_cast<const uint32_t *>(src)[d];
                 }
             }
-            sraw[j] = sbt[col];
-            if constexpr (!FP4) braw[j] = sbt[4 * BN + col];
-            if constexpr (FP4 == kNvfp4) braw[j] = sbt[BN + col];  // the lane's second group of 16
+            sraw[j] = sbt[col] & live;
+            if constexpr (!FP4) braw[j] = sbt[4 * BN + col] & live;
+            if constexpr (FP4 == kNvfp4) braw[j] = sbt[BN + col] & live;  // the lane's second group of 16
         }
     };
     const float factor = FP4 == kNvfp4 ? nvfp4_factor(a, 0) : 1.0f;  // (one matrix, or a batch that shares the scale)
@@ -311,6 +321,14 @@ qmm_kernel(const ProductArgs a) {
     // x fragment i of substep kk of the step in `stage`.
     auto read_x = [&](int stage, int kk, int i) {
         return *reinterpret_cast<const uint4 *>(lds + stage * G::kStageBytes + lds_offset(wm * (32 * TI) + i * 32 + l32, 4 * h + kk));
+    };
+    // Zeros over this thread's own loads of the x tile's chunks 0..3 (they have landed: each thread waits for its own).
+    auto clear_counted = [&](int stage) {
+#pragma unroll
+        for (int i = 0; i < XP; i++) {
+            const int slot = i * kThreads + wave * 64 + lane;
+            if (((slot & 7) ^ swizzle(slot >> 3)) < 4) *reinterpret_cast<uint4 *>(lds + stage * G::kStageBytes + slot * 16) = make_uint4(0, 0, 0, 0);
+        }
     };
     // The side work that prepares substep (step, KK) into buffer (KK & 1), in items: first x fragment reads and
     // expanded dwords alternate, then what is left of either.  Item t of kItems.
@@ -341,6 +359,7 @@ qmm_kernel(const ProductArgs a) {
     issue_parts(loads_of(0, 0), c0{}, std::integral_constant<int, G::kParts>{});
     issue_parts(loads_of(1, 1), c0{}, std::integral_constant<int, G::kParts>{});
     dma_wait<G::kParts>();
+    if (HALF && half_step == 0) clear_counted(0);
     __syncthreads();
     read_codes(0, 0);
     static_for<kItems>([&](auto t) { side_item(0, c0{}, t); });
@@ -364,6 +383,7 @@ qmm_kernel(const ProductArgs a) {
                 // (a table issued after the previous step's barrier is older than those loads: it is waited for too,
                 // a step after its issue rather than two)
                 dma_wait<G::kParts>();
+                if (HALF && step + 1 == half_step) clear_counted(stage1);
                 __syncthreads();
                 if (((step + 3) & (psteps - 1)) == 0 && step + 3 < steps) issue_table((step + 3) >> pshift);
                 read_codes(step + 1, stage1);
@@ -479,19 +499,19 @@ inline int k_splits(const ProductArgs &a, int cus, int *steps_per_split = nullpt
     return p.splits;
 }
 
-template <typename T, int BITS, int FP4, class TL, bool EXACT = false>
-int32_t run_tile(ProductArgs a, void *workspace, hipStream_t s) {
+template <typename T, int BITS, int FP4, class TL, bool EXACT, bool HALF>
+int32_t run_tile_of(ProductArgs a, void *workspace, hipStream_t s) {
     using G = Geometry<BITS, TL>;
     static std::atomic<bool> configured[2] = {false, false};
     const bool batched = a.batch > 1;
-    auto kernel = batched ? qmm_kernel<T, BITS, FP4, true, TL, EXACT> : qmm_kernel<T, BITS, FP4, false, TL, EXACT>;
+    auto kernel = batched ? qmm_kernel<T, BITS, FP4, true, TL, EXACT, HALF> : qmm_kernel<T, BITS, FP4, false, TL, EXACT, HALF>;
     if (!configured[batched]) {
         NVQ_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, G::kLdsBytes));
         configured[batched] = true;
     }
     int per = 0;
     const int splits = workspace != nullptr ? k_splits(a, compute_units(), &per) : 1;
-    if (splits > 1 && (int64_t)(splits - 1) * per >= a.k / BK)  // (a block of such a split would leave its partial sums unwritten)
+    if (splits > 1 && (int64_t)(splits - 1) * per >= (a.k + BK - 1) / BK)  // (a block of such a split would leave its partial sums unwritten)
         return fail(NVQ_BACKEND, "quantized_matmul: %d splits of %d steps leave one without a step of K = %lld", splits, per, (long long)a.k);
     a.k_splits = splits;
     a.k_split_steps = per;
@@ -505,6 +525,13 @@ int32_t run_tile(ProductArgs a, void *workspace, hipStream_t s) {
         NVQ_LAUNCH_CHECK("qmm_reduce");
     }
     return NVQ_OK;
+}
+
+template <typename T, int BITS, int FP4, class TL, bool EXACT = false>
+int32_t run_tile(const ProductArgs &a, void *workspace, hipStream_t s) {
+    if constexpr (FP4 != kAffine || EXACT)  // (half_steps_supported)
+        if (a.k % BK != 0) return run_tile_of<T, BITS, FP4, TL, EXACT, true>(a, workspace, s);
+    return run_tile_of<T, BITS, FP4, TL, EXACT, false>(a, workspace, s);
 }
 
 template <typename T, int BITS, int FP4>

@@ -4,12 +4,23 @@
 
 namespace nvq {
 
+// The grouped kernel: one row of x per pair, its scale table within its LDS budget, K of whole steps of 64
+// (windows of 128 for 1, 3 and 5 bits) or, beyond one window, as half_steps_supported has it.  Row-exact pairs keep the vector kernels where they had them, with the
+// CPU's weights and off whole steps.
+static bool grouped_supported(const ProductArgs &a) {
+    if (a.m != 1 || a.experts > 65535 || qmg::table_bytes(a) > (size_t)qmg::kTableMaxBytes) return false;
+    const bool odd = a.mode == NVQ_AFFINE && a.bits % 2 != 0, whole = a.k >= 64 && a.k % (odd ? 128 : 64) == 0;
+    if (a.row_exact && (a.exact_weights || !whole)) return false;
+    return whole || (a.k >= 128 && qmf::half_steps_supported(a));
+}
+
 // Whether the few-row matrix-core kernel takes this product: a block format or affine 1 to 6 or 8 bits, bf16 or
 // f16, whole steps of 64 values (whole windows of 128 for 1, 3 and 5 bits, whose 16-byte chunks straddle steps),
 // a scale table that fits in LDS, and either no batch, a batch with one stride per operand, gathered pairs,
 // or the grouped gather.
 bool qmf_supported(const ProductArgs &a) {
     if (a.dtype != NVQ_BF16 && a.dtype != NVQ_F16) return false;
+    if (a.offsets != nullptr) return grouped_supported(a);
     if (a.k < 64 || a.k % 64 != 0) return false;
     size_t lds = 0;
     if (a.mode == NVQ_MXFP4 || a.mode == NVQ_NVFP4) {
@@ -31,8 +42,6 @@ bool qmf_supported(const ProductArgs &a) {
     } else {
         return false;
     }
-    if (a.offsets != nullptr)  // the grouped kernel: one row of x per pair, its scale table within its LDS budget
-        return a.m == 1 && a.experts <= 65535 && !a.exact_weights && qmg::table_bytes(a) <= (size_t)qmg::kTableMaxBytes;
     if (lds > (size_t)qmf::kLdsLimit) return false;
     if (a.rhs != nullptr) return a.batch <= 65535 && (a.m + 31) / 32 <= 65535;  // gathered pairs, one per grid z
     return (a.batch == 1 || a.batch_ndim == 1) && a.batch <= 65535 && (a.m + 31) / 32 <= 65535;

@@ -50,7 +50,11 @@ struct Geometry {
 // and wavefronts 2 and 3 the same 64 columns of the up product, lane for lane: after a pass the latter leave their
 // values (rounded as the product's output, the expert's bias added) in LDS, the former combine them with their own
 // and write y [rows, N / 2].
-template <typename T, int BITS, int FP4, bool GLU = false>
+// EXACT (affine codes): the weights as nuvec's CPU product holds them (affine_pair).
+// RAGGED: K of whole 32 values; without it K is whole steps of 64 (windows of 128 for odd BITS), and the loop is free of the
+// last window's cases (with them everywhere, 256 tokens x 4 of 32 MXFP4 experts [5760, 2880] and [2880, 2880] took 220 us
+// against 190).
+template <typename T, int BITS, int FP4, bool GLU, bool EXACT, bool RAGGED>
 // Three blocks per compute unit (three wavefronts per SIMD): the registers are capped for that, and the LDS of a
 // block (two x stages, the weight stages, the table) fits three times.
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) qmg_kernel(const ProductArgs a) {
@@ -145,8 +149,13 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
     const T *x = (const T *)a.x;
     T *y = (T *)a.y;
 
-    const int steps = K >> 6;             // K is a multiple of 64 (checked on the host)
-    const int windows = (steps + 1) >> 1;  // the last window may hold one step
+    // Off whole windows the last one begins early (RAGGED), at K - 128, so that no load leaves its row; the first `counted`
+    // of its values, which the window before has counted, are zeros in both operands.  Else the last window may hold one
+    // step, as the only window of K = 64 does in either form.
+    const int windows = (K + 127) >> 7;
+    const int counted = RAGGED && K > 128 ? windows * 128 - K : 0;
+    auto first_of = [&](int win) { return RAGGED && win == windows - 1 && K > 128 ? K - 128 : win * 128; };
+    auto one_step = [&](int win) { return RAGGED ? K < 128 : win * 128 + 64 >= K; };
 
     // Weight window loads of this wavefront: load j of a lane is chunk q = 64 j + lane, i.e. chunk q % BITS of
     // row q / BITS of the wavefront's 32 rows.  Chunks of the window's second step begin at BITS / 2 (a window
@@ -166,10 +175,11 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
     // Every load of the K loop is issued on every path (a window past the end loads one 16-byte piece, the
     // same for all lanes), so that the waits can leave the younger windows' loads in flight.
     auto load_window = [&](int win, u32x4_t (&w)[kLoads]) {
-        const bool real = win < windows, half = 2 * win + 1 >= steps;
+        const bool real = win < windows, half = one_step(win);
+        const int at = (first_of(win) >> 3) * BITS;
 #pragma unroll
         for (int j = 0; j < kLoads; j++) {
-            const int off = win * 16 * BITS - ((half && second[j]) ? 8 * BITS : 0);
+            const int off = at - (half && second[j] ? 8 * BITS : 0);
             const unsigned char *src = real ? wload[j] + off : (const unsigned char *)a.w;
             w[j] = *reinterpret_cast<const u32x4_a4_t *>(src);
         }
@@ -195,9 +205,9 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
     __builtin_amdgcn_sched_barrier(0);
 
     const float factor = FP4 == kNvfp4 && a.global_scale != nullptr ? ftz(a.global_scale[e] / (448.0f * 6.0f)) : 1.0f;  // (one per expert)
-    // The scale (NVFP4: the two scales, one per 16 values) and bias of this lane's 32 values of a step.
-    auto load_scales = [&](int step, float (&scale)[2], float &bias) {
-        const int g = (step * 64 + 32 * h) >> gshift;
+    // The scale (NVFP4: the two scales, one per 16 values) and bias of this lane's 32 values of the step from k0 on.
+    auto load_scales = [&](int k0, float (&scale)[2], float &bias) {
+        const int g = (k0 + 32 * h) >> gshift;
         const int at = (32 * wave + l32) * tstride + g * (int)sizeof(S);
         const S *sp = reinterpret_cast<const S *>(table_s + at), *bp = reinterpret_cast<const S *>(table_b + at);
         if constexpr (FP4 == kNvfp4) {
@@ -252,7 +262,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
         }
         auto load_x = [&](int win, u32x4_t (&xq)[4]) {
             // a window of one step has no second half: those chunks (pieces 8..15) fetch the first half again
-            const int k0 = win < windows ? win * 128 - ((2 * win + 1 >= steps && xc >= 8) ? 64 : 0) : 0;
+            const int k0 = win < windows ? first_of(win) - (one_step(win) && xc >= 8 ? 64 : 0) : 0;
             // chunks 2 and 3 are rows 32..63: fetched only when the pass has a second tile (the loads are issued
             // either way, so that the waits see the same number of them: a tile-less one reads the start of x)
 #pragma unroll
@@ -260,6 +270,12 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
         };
         auto store_x = [&](int win, const u32x4_t (&xq)[4]) {
             unsigned char *dst = lds + (win & 1) * kXStageBytes;
+            if (RAGGED && win == windows - 1 && 8 * xc < counted) {  // (a thread's four chunks lie at one place of the window)
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (i < 2 || two) *reinterpret_cast<u32x4_t *>(dst + xstore[i]) = u32x4_t{0, 0, 0, 0};
+                return;
+            }
 #pragma unroll
             for (int i = 0; i < 4; i++)
                 if (i < 2 || two) *reinterpret_cast<u32x4_t *>(dst + xstore[i]) = xq[i];
@@ -317,9 +333,10 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
                     // All x operands of a tile are requested before the first matrix instruction needs one (LDS
                     // answers in order), so the window pays the LDS latency once, not once per instruction.  A
                     // window of one step reads its absent second step too (stale but valid LDS) and skips its
-                    // matrix instructions.
+                    // matrix instructions, as the last window does where its first step is all zeros.
                     const unsigned char *xs = lds + (win & 1) * kXStageBytes;
-                    const bool second_step = 2 * win + 1 < steps;
+                    const int before = RAGGED && win == windows - 1 ? counted : 0;  // values at the window's start that are zeros
+                    const bool run[2] = {!RAGGED || before < 64, !one_step(win)};
                     uint4 xf[2][4], wb[2][4];
 #pragma unroll
                     for (int t = 0; t < 2; t++)
@@ -328,15 +345,16 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
 #pragma unroll
                     for (int t = 0; t < 2; t++) {
                         float scale[2], bias;
-                        load_scales(2 * win + (t == 0 || second_step ? t : 0), scale, bias);
+                        load_scales(first_of(win) + (t == 0 || run[1] ? 64 * t : 0), scale, bias);
+                        if (RAGGED && 64 * t + 32 * h < before) scale[0] = scale[1] = bias = 0.0f;
                         static_for<4>([&](auto kk_tag) {
                             constexpr int kk = decltype(kk_tag)::value;
-                            wb[t][kk] = expand_piece<T, BITS, FP4, kk>(codes[t], scale[kk >> 1], bias);
+                            wb[t][kk] = expand_piece<T, BITS, FP4, kk, EXACT>(codes[t], scale[kk >> 1], bias);
                         });
                     }
 #pragma unroll
                     for (int t = 0; t < 2; t++)
-                        if (t == 0 || second_step) {
+                        if (run[t]) {
 #pragma unroll
                             for (int kk = 0; kk < 4; kk++) acc[0] = Ops<T>::mfma(xf[t][kk], wb[t][kk], acc[0]);
                         }
@@ -347,7 +365,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
                             for (int kk = 0; kk < 4; kk++) xf[t][kk] = *reinterpret_cast<const uint4 *>(xs + 32 * 256 + xread[t][kk]);
 #pragma unroll
                         for (int t = 0; t < 2; t++)
-                            if (t == 0 || second_step) {
+                            if (run[t]) {
 #pragma unroll
                                 for (int kk = 0; kk < 4; kk++) acc[1] = Ops<T>::mfma(xf[t][kk], wb[t][kk], acc[1]);
                             }
@@ -422,11 +440,11 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
 // Bytes of the LDS table of scales (and biases) for the block's rows.
 inline size_t table_bytes(const ProductArgs &a) { return qmf::table_bytes(a, kRows); }
 
-template <typename T, int BITS, int FP4, bool GLU>
+template <typename T, int BITS, int FP4, bool GLU, bool EXACT, bool RAGGED>
 int32_t run_kernel(const ProductArgs &a, hipStream_t s) {
     using G = Geometry<BITS>;
     static std::atomic<bool> configured = false;
-    auto kernel = qmg_kernel<T, BITS, FP4, GLU>;
+    auto kernel = qmg_kernel<T, BITS, FP4, GLU, EXACT, RAGGED>;
     const size_t lds_bytes = G::kFixedLdsBytes + table_bytes(a);
     if (!configured) {
         NVQ_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -444,9 +462,12 @@ int32_t run_kernel(const ProductArgs &a, hipStream_t s) {
 
 template <typename T, int BITS, int FP4>
 int32_t run(const ProductArgs &a, hipStream_t s) {
-    if (a.glu == 0) return run_kernel<T, BITS, FP4, false>(a, s);
-    if (a.n % kRows != 0) return fail(NVQ_UNSUPPORTED, "gather_qmm: the gated epilogue takes gate and up rows in whole runs of 64");
-    return run_kernel<T, BITS, FP4, true>(a, s);
+    if (a.glu != 0 && a.n % kRows != 0) return fail(NVQ_UNSUPPORTED, "gather_qmm: the gated epilogue takes gate and up rows in whole runs of 64");
+    const bool ragged = a.k % (BITS % 2 != 0 ? 128 : 64) != 0;
+    if constexpr (FP4 == kAffine)
+        if (a.exact_weights) return run_kernel<T, BITS, FP4, false, true, true>(a, s);  // (no gated epilogue: checked by the caller)
+    if (ragged) return a.glu == 0 ? run_kernel<T, BITS, FP4, false, false, true>(a, s) : run_kernel<T, BITS, FP4, true, false, true>(a, s);
+    return a.glu == 0 ? run_kernel<T, BITS, FP4, false, false, false>(a, s) : run_kernel<T, BITS, FP4, true, false, false>(a, s);
 }
 
 template <int BITS, int FP4>

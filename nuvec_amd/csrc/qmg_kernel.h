@@ -330,45 +330,35 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
                     }
                 asm volatile("" ::: "memory");
                 if (win < windows) {
-                    // All x operands of a tile are requested before the first matrix instruction needs one (LDS
-                    // answers in order), so the window pays the LDS latency once, not once per instruction.  A
-                    // window of one step reads its absent second step too (stale but valid LDS) and skips its
-                    // matrix instructions, as the last window does where its first step is all zeros.
+                    // A step's x operands are requested before its codes become weights, which hides the LDS latency; step
+                    // by step, so that 16 registers of weights and 32 of x are live at a time (both steps' together did not
+                    // fit the 168 registers of three wavefronts per SIMD, and the loop spilled).  The second tile's are
+                    // read whether the pass has one or not (stale but valid LDS).  A window of one step leaves out the
+                    // absent second one, the last window (RAGGED) a first step of zeros.
                     const unsigned char *xs = lds + (win & 1) * kXStageBytes;
                     const int before = RAGGED && win == windows - 1 ? counted : 0;  // values at the window's start that are zeros
                     const bool run[2] = {!RAGGED || before < 64, !one_step(win)};
-                    uint4 xf[2][4], wb[2][4];
-#pragma unroll
-                    for (int t = 0; t < 2; t++)
-#pragma unroll
-                        for (int kk = 0; kk < 4; kk++) xf[t][kk] = *reinterpret_cast<const uint4 *>(xs + xread[t][kk]);
 #pragma unroll
                     for (int t = 0; t < 2; t++) {
+                        if (!run[t]) continue;
+                        uint4 xf[2][4], wb[4];
+#pragma unroll
+                        for (int u = 0; u < 2; u++)
+#pragma unroll
+                            for (int kk = 0; kk < 4; kk++) xf[u][kk] = *reinterpret_cast<const uint4 *>(xs + u * 32 * 256 + xread[t][kk]);
                         float scale[2], bias;
-                        load_scales(first_of(win) + (t == 0 || run[1] ? 64 * t : 0), scale, bias);
+                        load_scales(first_of(win) + 64 * t, scale, bias);
                         if (RAGGED && 64 * t + 32 * h < before) scale[0] = scale[1] = bias = 0.0f;
                         static_for<4>([&](auto kk_tag) {
                             constexpr int kk = decltype(kk_tag)::value;
-                            wb[t][kk] = expand_piece<T, BITS, FP4, kk, EXACT>(codes[t], scale[kk >> 1], bias);
+                            wb[kk] = expand_piece<T, BITS, FP4, kk, EXACT>(codes[t], scale[kk >> 1], bias);
                         });
-                    }
 #pragma unroll
-                    for (int t = 0; t < 2; t++)
-                        if (run[t]) {
+                        for (int kk = 0; kk < 4; kk++) acc[0] = Ops<T>::mfma(xf[0][kk], wb[kk], acc[0]);
+                        if (two) {
 #pragma unroll
-                            for (int kk = 0; kk < 4; kk++) acc[0] = Ops<T>::mfma(xf[t][kk], wb[t][kk], acc[0]);
+                            for (int kk = 0; kk < 4; kk++) acc[1] = Ops<T>::mfma(xf[1][kk], wb[kk], acc[1]);
                         }
-                    if (two) {
-#pragma unroll
-                        for (int t = 0; t < 2; t++)
-#pragma unroll
-                            for (int kk = 0; kk < 4; kk++) xf[t][kk] = *reinterpret_cast<const uint4 *>(xs + 32 * 256 + xread[t][kk]);
-#pragma unroll
-                        for (int t = 0; t < 2; t++)
-                            if (run[t]) {
-#pragma unroll
-                                for (int kk = 0; kk < 4; kk++) acc[1] = Ops<T>::mfma(xf[t][kk], wb[t][kk], acc[1]);
-                            }
                     }
                 }
                 // the next window of x goes into the other stage (last read one window ago, before the previous

@@ -89,3 +89,27 @@ def test_bias_epilogue_determinism_and_the_vector_kernel():
     assert torch.equal(layer(xd), plain + bias)
     by_rows = nv.quantized_matmul(xd, q, rows=True)
     assert_rows_close(to_host(plain), to_host(by_rows), ref.F32, "float32 rows against the vector kernel")
+
+
+@pytest.mark.parametrize("fmt", [(64, 1), (64, 2), (32, 3), (64, 4), (32, 5), (128, 6), (64, 8), "MXFP4", "MXFP8", "NVFP4"], ids=str)
+@pytest.mark.parametrize("m,n,k", [(33, 4096, 512), (48, 3001, 2048), (65, 4099, 1024), (100, 2040, 1024), (5, 33000, 512), (40, 5000, 544)])
+def test_tiles_of_sixteen_rows(fmt, m, n, k):
+    """One to four tiles of sixteen rows, two passes, tails of rows and of weight rows, blocks whose wavefronts share K by eight, by two
+    and not at all, K off whole steps of 64 (groups of 32).   The bar is 1e-4 of a row's largest output, as above."""
+    block = isinstance(fmt, str)
+    group, bits = ref.FP_PARAMS[getattr(ref, fmt)] if block else fmt
+    if k % group:
+        pytest.skip("K is not whole groups")
+    rng = np.random.default_rng(5600 + m + n)
+    quant = nv.Quant.new(getattr(nv.QuantMode, fmt)) if block else nv.Quant.affine(group, bits)
+    assert ops.quantized_matmul_route(m, n, k, quant, torch.float32) == "qmm_f32_kernel"
+    w, x = make_w(rng, n, k, ref.F32), make_x(rng, m, k, ref.F32)
+    if block:
+        packed, scales, biases = *ref.fp_quantize(w, ref.F32, getattr(ref, fmt)), None
+        want = ref.quantized_matmul(x, packed, scales, None, mode=getattr(ref, fmt), group=group, bits=bits, dtype=ref.F32, threads=8)
+    else:
+        packed, scales, biases = ref.affine_quantize(w, ref.F32, group, bits)
+        want = ref.quantized_matmul(x, packed, scales, biases, group=group, bits=bits, dtype=ref.F32, threads=8)
+    q = nv.Quantized(to_dev(packed), to_dev(scales), None if biases is None else to_dev(biases), quant)
+    got = to_host(nv.quantized_matmul(to_dev(x), q))
+    assert_rows_close(got, want, ref.F32, f"float32 tiles of 16 rows {fmt} M={m} N={n} K={k}", exact_weights=True)

@@ -593,7 +593,8 @@ static bool takes_tiled(const nvq_qmm_desc *d, const ProductArgs &a) {
 enum class Route { kUntransposed, kVector, kTiled, kTiledF32, kFewRowsF32, kBatchedDecode, kFewRowsDirect, kFewRows };
 static Route pick_route(const nvq_qmm_desc *d, const ProductArgs &a);
 
-size_t nvq_quantized_matmul_workspace_bytes(const nvq_qmm_desc *d) {
+// `dense`: whether the workspace may hold the dequantized weight.
+static size_t workspace_bytes(const nvq_qmm_desc *d, bool dense) {
     if (check_qmm(d, "quantized_matmul") != NVQ_OK) return 0;
     int64_t batch = 1;
     for (int i = 0; i < d->batch_ndim; i++) batch *= d->batch_shape[i];
@@ -601,8 +602,11 @@ size_t nvq_quantized_matmul_workspace_bytes(const nvq_qmm_desc *d) {
     const ProductArgs a = product_args(d, batch);
     // float32 partial sums of the splits of K: weights stored [K, N], or few tiles of a long K
     if (!d->transpose) return qvm_workspace_bytes(a);
-    return pick_route(d, a) == Route::kTiled ? qmm_workspace_bytes(a) : 0;
+    if (pick_route(d, a) != Route::kTiled) return 0;
+    return dense && qmm_dense_takes(a) ? qmm_dense_workspace_bytes(a) : qmm_workspace_bytes(a);
 }
+
+size_t nvq_quantized_matmul_workspace_bytes(const nvq_qmm_desc *d) { return workspace_bytes(d, true); }
 
 static Route pick_route(const nvq_qmm_desc *d, const ProductArgs &a) {
     if (!d->transpose) return Route::kUntransposed;        // weights stored [K, N]
@@ -632,7 +636,8 @@ static Route pick_route(const nvq_qmm_desc *d, const ProductArgs &a) {
 }
 
 static int32_t quantized_matmul_any(const nvq_qmm_desc *d, const void *x, const void *w, const void *scales, const void *biases,
-                                    const float *global_scale, void *y, void *workspace, void *stream, const void *row_bias = nullptr) {
+                                    const float *global_scale, void *y, void *workspace, void *stream, const void *row_bias = nullptr,
+                                    bool dense = true) {
     NVQ_TRY(check_qmm(d, "quantized_matmul"));
     NVQ_TRY(check_groups("quantized_matmul", d->quant.mode, biases));
     int64_t batch = 1;
@@ -656,7 +661,8 @@ static int32_t quantized_matmul_any(const nvq_qmm_desc *d, const void *x, const 
     a.row_bias = row_bias;
     switch (pick_route(d, a)) {
     case Route::kUntransposed: return launch_qvm(a, workspace, (hipStream_t)stream);
-    case Route::kTiled: return launch_qmm(a, workspace, (hipStream_t)stream);  // without a workspace: K is not split
+    case Route::kTiled:  // without a workspace: codes are expanded in the kernel and K is not split
+        return dense && workspace != nullptr && qmm_dense_takes(a) ? launch_qmm_dense(a, workspace, (hipStream_t)stream) : launch_qmm(a, workspace, (hipStream_t)stream);
     case Route::kTiledF32: return launch_qmm_f32(a, (hipStream_t)stream);
     case Route::kFewRowsF32: return launch_qmf_f32(a, (hipStream_t)stream);
     case Route::kBatchedDecode: return launch_qmr(a, (hipStream_t)stream);
@@ -733,7 +739,7 @@ int32_t nvq_quantized_matmul_glu(const nvq_qmm_desc *d, int32_t activation, floa
 int32_t nvq_quantized_matmul_static(const nvq_qmm_desc *d, const void *x, const void *w, const void *scales, const void *biases,
                                     void *y, void *stream) {
     NVQ_TRY(check_qmm(d, "quantized_matmul"));
-    const size_t need = nvq_quantized_matmul_workspace_bytes(d);  // 0 without a device: the launch below says so
+    const size_t need = workspace_bytes(d, false);  // 0 without a device: the launch below says so
     const bool fits = need <= (size_t)NVQ_STATIC_SCRATCH_BYTES;
     if (!fits && (!d->transpose || d->k % 64 == 0))  // (the tiles take K off whole steps of 64 without a split)
         return fail(NVQ_UNSUPPORTED, "quantized_matmul: this product splits K through %zu bytes of partial sums; the static scratch holds %d",
@@ -743,7 +749,7 @@ int32_t nvq_quantized_matmul_static(const nvq_qmm_desc *d, const void *x, const 
         NVQ_TRY(require_device());
         workspace = g_scratch[g_device.device.load(std::memory_order_relaxed)];
     }
-    return quantized_matmul_any(d, x, w, scales, biases, nullptr, y, workspace, stream);
+    return quantized_matmul_any(d, x, w, scales, biases, nullptr, y, workspace, stream, nullptr, false);
 }
 
 int32_t nvq_quantized_matmul_scaled(const nvq_qmm_desc *d, const void *x, const void *w, const void *scales,

@@ -128,6 +128,9 @@ double qmm_estimate_us(const ProductArgs &a);  // estimated duration of the tile
 // float32 products of many rows on v_mfma_f32_32x32x2_f32 (affine codes, weights stored [N, K]).
 bool qmm_f32_takes(const ProductArgs &a);
 int32_t launch_qmm_f32(const ProductArgs &a, hipStream_t s);
+bool qmm_dense_takes(const ProductArgs &a);
+size_t qmm_dense_workspace_bytes(const ProductArgs &a);
+int32_t launch_qmm_dense(const ProductArgs &a, void *workspace, hipStream_t s);
 bool qmf_f32_takes(const ProductArgs &a);
 int32_t launch_qmf_f32(const ProductArgs &a, hipStream_t s);
 // Batched decode: passes of up to 64 rows of x (5 to 128 rows routed there, where it measured faster), every weight fetched and dequantized once per pass (4- and 8-bit affine codes).

@@ -1,0 +1,171 @@
+// Many rows against weights that have to be the CPU's, round(round(code * scale) + bias) (reference:
+// crates/nuvec-core/src/kernels.rs:835-859; product kernels.rs:1091-1142): the weight is dequantized once into a workspace
+// (affine_dequantize_kernel) and multiplied densely, in bfloat16 or float16 on v_mfma_f32_32x32x16.
+//
+// The tiled kernel that expands codes itself (qmm_kernel.h) does so for every 128 rows of x and twice in a block, and two
+// roundings a weight make it bound by the vector unit: 517 rows, W[4096,4096] of 3 bits, 73 us = 237 TFLOP/s.  A weight of N x K
+// costs 2 N K bytes written and, from the chip's last cache, read.
+//
+// A block of four wavefronts owns BM x 128 of y, 128 or 256 rows of x, each wavefront BM / 2 x 64, and walks K in steps of 64
+// through a ring of LDS stages that both operands reach by direct loads, as many as fit; layout, swizzle and order of K are
+// those of qmm_kernel.h, whose x tile is either operand here.  Bound by LDS reads: one operand of 16 bytes a lane per matrix
+// instruction at 128 rows, three per four at 256 (a step takes 0.5 and 0.85 us; operands laid out tile by tile beforehand, so
+// that a load is 1 KB of consecutive bytes, took 0.55).
+// us, 4 bits, bfloat16, codes expanded in the product -> here: W[4096,4096] at 517 / 1024 / 2048 rows 68 / 70 / 115 -> 42 / 51 / 75
+// (3 bits at 517 rows 73 -> 41), W[8000,4096] at 517 rows 108 -> 73, W[6144,8192] at 768 rows 200 -> 120.
+#include "qmm_kernel.h"
+
+namespace nvq {
+namespace {
+
+using namespace qmm;
+
+template <int TI_, int RING>
+struct Dense {
+    static constexpr int TI = TI_, TJ = 2, kRing = RING, BM = 64 * TI, BN = 128, kThreads = 256;
+    static constexpr int kXBytes = BM * kRowBytes, kStageBytes = (BM + BN) * kRowBytes, kLdsBytes = kRing * kStageBytes;
+    static constexpr int XP = BM * 8 / kThreads, WP = BN * 8 / kThreads, kParts = XP + WP;  // loads a step: of x, then of the weight
+};
+using Small = Dense<2, 5>;
+using Big = Dense<4, 3>;
+
+template <typename T, class D>
+__global__ void __launch_bounds__(D::kThreads, 1) qmm_dense_kernel(const ProductArgs a, const T *__restrict__ weights) {
+    constexpr int TI = D::TI, TJ = D::TJ, XP = D::XP, kThreads = D::kThreads;
+    constexpr int kAhead = D::kRing - 1;  // steps under way
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 1, wn = wave & 1, h = lane >> 5, l32 = lane & 31;
+    const int K = (int)a.k, N = (int)a.n, M = (int)a.m, steps = K / BK;  // K is a multiple of 64 (checked on the host)
+    const int m0 = blockIdx.y * D::BM, n0 = blockIdx.x * D::BN;
+    const char *xbase = reinterpret_cast<const char *>((const T *)a.x + (int64_t)m0 * K), *wbase = reinterpret_cast<const char *>(weights + (int64_t)n0 * K);
+
+    // Instruction i of wavefront v fills the 64 consecutive 16-byte slots from slot i * kThreads + v * 64 on of its operand's
+    // tile; slot S is row S / 8 and holds chunk S % 8 ^ swizzle(row).  Rows past the ends repeat the last one.
+    uint32_t off[D::kParts];
+#pragma unroll
+    for (int i = 0; i < D::kParts; i++) {
+        const bool is_x = i < XP;
+        const int slot = (is_x ? i : i - XP) * kThreads + tid, row = slot >> 3, chunk = (slot & 7) ^ swizzle(row);
+        const int last = is_x ? M - 1 - m0 : N - 1 - n0;
+        off[i] = ((uint32_t)(row < last ? row : last) * (uint32_t)K + chunk * 8) * 2;
+    }
+    const uint32_t lds_wave = lds0 + wave * 64 * 16;
+    // Load `i` of a step (past the end: the last step again, which keeps the wait counts uniform).
+    auto issue = [&](int step, int stage, auto i_tag) {
+        constexpr int i = decltype(i_tag)::value;
+        const int sc = step < steps ? step : steps - 1;
+        dma<4>((i < XP ? xbase : wbase) + sc * (BK * 2), off[i],
+               lds_wave + stage * D::kStageBytes + (i < XP ? i * kThreads * 16 : D::kXBytes + (i - XP) * kThreads * 16));
+    };
+    // Item t of substep kk's operands, of the step in `stage`: TI of x, then TJ of the weights.
+    uint4 af[2][TI], bf[2][TJ];
+    auto read = [&](int stage, auto kk_tag, auto t_tag) {
+        constexpr int kk = decltype(kk_tag)::value, t = decltype(t_tag)::value;
+        const unsigned char *from = lds + stage * D::kStageBytes;
+        if constexpr (t < TI) af[kk & 1][t] = *reinterpret_cast<const uint4 *>(from + lds_offset(wm * (32 * TI) + t * 32 + l32, 4 * h + kk));
+        else bf[kk & 1][t - TI] = *reinterpret_cast<const uint4 *>(from + D::kXBytes + lds_offset(wn * (32 * TJ) + (t - TI) * 32 + l32, 4 * h + kk));
+    };
+    floatx16_t acc[TI][TJ];
+#pragma unroll
+    for (int i = 0; i < TI; i++)
+#pragma unroll
+        for (int j = 0; j < TJ; j++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
+
+    static_for<kAhead>([&](auto s) { static_for<D::kParts>([&](auto i) { issue(decltype(s)::value, decltype(s)::value, i); }); });
+    dma_wait<(kAhead - 1) * D::kParts>();
+    __syncthreads();
+    using c0 = std::integral_constant<int, 0>;
+    static_for<TI + TJ>([&](auto t) { read(0, c0{}, t); });
+    int stage = 0, last = kAhead;  // step % D::kRing, (step + kAhead) % D::kRing
+    for (int step = 0; step < steps; step++) {
+        const int stage1 = stage == kAhead ? 0 : stage + 1;
+        static_for<4>([&](auto kk_tag) {
+            constexpr int kk = decltype(kk_tag)::value, next = (kk + 1) & 3;
+            // a quarter of the loads of step + kAhead, into the stage that everyone left at the last barrier
+            static_for<D::kParts / 4>([&](auto p) { issue(step + kAhead, last, std::integral_constant<int, kk * (D::kParts / 4) + decltype(p)::value>{}); });
+            if constexpr (kk == 3) {  // the next step has landed for everyone, and everyone is done reading this one
+                dma_wait<(kAhead - 1) * D::kParts>();
+                __syncthreads();
+            }
+            static_for<TI * TJ>([&](auto q_tag) {
+                constexpr int q = decltype(q_tag)::value, i = q % TI, j = q / TI;
+                acc[i][j] = Ops<T>::mfma(af[kk & 1][i], bf[kk & 1][j], acc[i][j]);
+                static_for<TI + TJ>([&](auto t_tag) {
+                    constexpr int t = decltype(t_tag)::value;
+                    if constexpr (t >= q * (TI + TJ) / (TI * TJ) && t < (q + 1) * (TI + TJ) / (TI * TJ))
+                        read(kk == 3 ? stage1 : stage, std::integral_constant<int, next>{}, t_tag);
+                });
+                pin();
+            });
+        });
+        last = stage, stage = stage1;
+    }
+    dma_wait<0>();
+
+    // Accumulator element e of a 32 x 32 tile is row 8 (e / 4) + 4 (lane / 32) + e % 4, column lane % 32.
+    uint16_t *y = reinterpret_cast<uint16_t *>(a.y);
+#pragma unroll
+    for (int i = 0; i < TI; i++)
+#pragma unroll
+        for (int j = 0; j < TJ; j++) {
+            const int col = n0 + wn * (32 * TJ) + j * 32 + l32, row0 = m0 + wm * (32 * TI) + i * 32 + 4 * h;
+            if (col >= N) continue;
+#pragma unroll
+            for (int e = 0; e < 16; e += 2) {
+                const uint32_t pair = Ops<T>::pack(add_row_bias<T>(a.row_bias, acc[i][j][e], col), add_row_bias<T>(a.row_bias, acc[i][j][e + 1], col));
+                const int row = row0 + 8 * (e >> 2) + (e & 3);
+                if (row < M) y[(int64_t)row * N + col] = (uint16_t)pair;
+                if (row + 1 < M) y[(int64_t)(row + 1) * N + col] = (uint16_t)(pair >> 16);
+            }
+        }
+}
+
+template <typename T, class D>
+int32_t run_tile(const ProductArgs &a, const void *weights, hipStream_t s) {
+    static std::atomic<bool> configured = false;
+    if (!configured) {
+        NVQ_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(qmm_dense_kernel<T, D>), hipFuncAttributeMaxDynamicSharedMemorySize, D::kLdsBytes));
+        configured = true;
+    }
+    const dim3 grid((unsigned)((a.n + D::BN - 1) / D::BN), (unsigned)((a.m + D::BM - 1) / D::BM));
+    hipLaunchKernelGGL((qmm_dense_kernel<T, D>), grid, dim3(D::kThreads), D::kLdsBytes, s, a, (const T *)weights);
+    NVQ_LAUNCH_CHECK("qmm_dense");
+    return NVQ_OK;
+}
+
+// Microseconds of the product by tiles of either height: rounds of a tile per compute unit.
+template <class D>
+double product_us(const ProductArgs &a) {
+    const double tiles = (double)((a.m + D::BM - 1) / D::BM) * (double)((a.n + D::BN - 1) / D::BN);
+    return ceil(tiles / fmax(1.0, (double)compute_units())) * (double)(a.k / BK) * (D::TI == 2 ? 0.5 : 0.85);
+}
+
+}  // namespace
+
+size_t qmm_dense_workspace_bytes(const ProductArgs &a) { return (size_t)a.n * (size_t)a.k * 2; }
+
+// Among the products that the tiled kernel takes with the CPU's weights: where the dequantization (7 us of launches and ends of
+// kernels, and 0.48 us per million weights) and the dense product are estimated a tenth below that kernel.  us here / there, where it turns: W[4096,4096] 384 / 517 rows
+// 49 / 43 and 42 / 68; W[1024,4096] 1024 / 2048 rows 41 / 31 and 43 / 47; W[576,576] at 517 rows 13 / 11.
+bool qmm_dense_takes(const ProductArgs &a) {
+    if (a.mode != NVQ_AFFINE || !a.exact_weights || a.row_exact || a.batch != 1 || a.batch_ndim != 0 || a.rhs != nullptr || a.lhs != nullptr || a.glu != 0)
+        return false;
+    if (a.k < BK || a.k % BK != 0 || a.n * a.k >= (1LL << 32) || (a.m + 127) / 128 > 65535) return false;
+    const double here = 7.0 + 0.48e-6 * (double)a.n * (double)a.k + fmin(product_us<Small>(a), product_us<Big>(a));
+    return here < 0.9 * (1.8 + 1.26 * qmm_estimate_us(a));
+}
+
+int32_t launch_qmm_dense(const ProductArgs &a, void *workspace, hipStream_t s) {
+    const int32_t rc = launch_affine_dequantize(a.dtype, a.group, a.bits, a.w, a.scales, a.biases, a.n * a.k, workspace, nullptr, a.k, a.n, s);
+    if (rc != NVQ_OK) return rc;
+    const bool big = product_us<Big>(a) < product_us<Small>(a);
+    if (a.dtype == NVQ_BF16) return big ? run_tile<bf16_t, Big>(a, workspace, s) : run_tile<bf16_t, Small>(a, workspace, s);
+    return big ? run_tile<f16_t, Big>(a, workspace, s) : run_tile<f16_t, Small>(a, workspace, s);
+}
+
+}  // namespace nvq

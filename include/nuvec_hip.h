@@ -229,6 +229,7 @@ NVQ_API int32_t nvq_dequantize_rows(const nvq_quant *quant, int32_t dtype, const
  * (gpu.rs:7022, "nuvec_affine_qmv_mma_..."; its tests check the names, crates/nuvec-core/tests/quantized.rs:843-861).
  * Needs nvq_init. */
 NVQ_API const char *nvq_quantized_matmul_route(const nvq_qmm_desc *desc);
+/* Float32 partial sums where K is split over the grid, or the weight dequantized for many rows of x; 0: none. */
 NVQ_API size_t nvq_quantized_matmul_workspace_bytes(const nvq_qmm_desc *desc);
 
 /* GpuEval::quantized_matmul / fp_quantized_matmul (gpu.rs:6934-7168, 6336-6577); values of

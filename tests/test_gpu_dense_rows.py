@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 
 # Both tiles, tails of rows and of weight rows, one step of K (fewer than the stages under way) and many
-@pytest.mark.parametrize("m,n,k", [(517, 4096, 4096), (513, 4099, 2048), (2050, 3970, 1024), (1100, 6145, 512), (9000, 1025, 192), (30000, 1100, 64)])
+@pytest.mark.parametrize("m,n,k", [(517, 4096, 4096), (513, 4099, 2048), (2050, 3970, 1024), (1100, 6145, 512), (9000, 1025, 192), (30000, 1100, 64), (1536, 4096, 2048)])
 @pytest.mark.parametrize("bits,group", [(1, 32), (2, 64), (3, 64), (4, 32), (5, 64), (6, 32), (8, 64)])
 def test_against_float64(m, n, k, bits, group):
     torch.manual_seed(m + bits)
@@ -41,3 +41,19 @@ def test_replays_in_a_graph():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("m,n,k", [(517, 4096, 4096), (2048, 3970, 1024), (517, 4096, 14336), (517, 2048, 2048)])
+def test_without_a_workspace(m, n, k):
+    """`nvq_quantized_matmul_static` expands codes in the product: the same bits, whether K is split or not."""
+    import ctypes as C
+
+    from nuvec_amd import _lib
+    q = nv.quantize((torch.randn(n, k, device="cuda") * 0.02).bfloat16(), nv.Quant.affine(64, 4))
+    x = torch.randn(m, k, device="cuda").bfloat16()
+    want, got = nv.quantized_matmul(x, q), torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+    d = _lib.QmmDescC()
+    d.quant, d.dtype, d.transpose, d.m, d.n, d.k = q.quant._c(), ops._CODE[x.dtype], 1, m, n, k
+    p = ops._ptr
+    _lib.check(_lib.load().nvq_quantized_matmul_static(C.byref(d), p(x), p(q.weight), p(q.scales), p(q.biases), p(got), ops._stream()))
+    assert torch.equal(got, want)

@@ -590,7 +590,7 @@ static bool takes_tiled(const nvq_qmm_desc *d, const ProductArgs &a) {
 }
 
 // The kernel family of a product (the counterpart of the routing in GpuEval::quantized_matmul, gpu.rs:6934-7168).
-enum class Route { kUntransposed, kVector, kTiled, kTiledF32, kFewRowsF32, kBatchedDecode, kFewRowsDirect, kFewRows };
+enum class Route { kUntransposed, kVector, kTiled, kTiledF32, kFewRowsF32, kGroupedRows, kBatchedDecode, kFewRowsDirect, kFewRows };
 static Route pick_route(const nvq_qmm_desc *d, const ProductArgs &a);
 
 // `dense`: whether the workspace may hold the dequantized weight.
@@ -632,6 +632,7 @@ static Route pick_route(const nvq_qmm_desc *d, const ProductArgs &a) {
     // W[2880,2880]: 5 to 8 rows, two passes of four, 14 against 16, 12 rows 21 against 16.)
     if (!takes_decode(a) && a.m >= 5 && (double)((a.m + 3) / 4) * (double)a.n * (double)a.k * (double)a.batch >= 20.0e6 && qmm_supported(a))
         return Route::kTiled;
+    if (grouped_rows_take(a)) return Route::kGroupedRows;
     return Route::kVector;
 }
 
@@ -665,6 +666,7 @@ static int32_t quantized_matmul_any(const nvq_qmm_desc *d, const void *x, const 
         return dense && workspace != nullptr && qmm_dense_takes(a) ? launch_qmm_dense(a, workspace, (hipStream_t)stream) : launch_qmm(a, workspace, (hipStream_t)stream);
     case Route::kTiledF32: return launch_qmm_f32(a, (hipStream_t)stream);
     case Route::kFewRowsF32: return launch_qmf_f32(a, (hipStream_t)stream);
+    case Route::kGroupedRows: return launch_grouped_rows(a, (hipStream_t)stream);
     case Route::kBatchedDecode: return launch_qmr(a, (hipStream_t)stream);
     case Route::kFewRowsDirect: return launch_qmd(a, (hipStream_t)stream);
     case Route::kFewRows: return launch_qmf(a, (hipStream_t)stream);
@@ -684,6 +686,7 @@ const char *nvq_quantized_matmul_route(const nvq_qmm_desc *d) {
     case Route::kTiled: return "qmm_kernel";
     case Route::kTiledF32:  // (the float32 matrix instruction's kernels under one name, whichever rows they are cut for)
     case Route::kFewRowsF32: return "qmm_f32_kernel";
+    case Route::kGroupedRows: return "qmg_kernel";
     case Route::kBatchedDecode: return "qmr_kernel";
     case Route::kFewRowsDirect: return "qmd_kernel";
     case Route::kFewRows: return "qmf_kernel";

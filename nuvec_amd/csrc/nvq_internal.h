@@ -85,6 +85,7 @@ struct ProductArgs {
     const uint32_t *lhs, *rhs;      // gather: batch z reads x batch lhs[z] and weight batch rhs[z]
     int64_t x_batches, experts;     // gather: index bounds (an index beyond them is clamped)
     const int32_t *offsets;         // grouped gather: rows of expert e are [offsets[e], offsets[e+1]) of `batch` rows
+    int32_t one_group;              // the grouped kernel without offsets: all `batch` rows belong to one weight
     int32_t k_splits, k_split_steps;  // tiled kernel: K split over grid z (0 or 1: no split), steps of 64 values per split
     float *partials;                // tiled kernel with a split: float32 [k_splits][m][n], summed by a second kernel
     const float *global_scale;      // NVFP4: NULL, one float32 value, or one per expert of a gather (weights stored [N, K] only)
@@ -128,6 +129,8 @@ double qmm_estimate_us(const ProductArgs &a);  // estimated duration of the tile
 // float32 products of many rows on v_mfma_f32_32x32x2_f32 (affine codes, weights stored [N, K]).
 bool qmm_f32_takes(const ProductArgs &a);
 int32_t launch_qmm_f32(const ProductArgs &a, hipStream_t s);
+bool grouped_rows_take(const ProductArgs &a);
+int32_t launch_grouped_rows(ProductArgs a, hipStream_t s);
 bool qmm_dense_takes(const ProductArgs &a);
 size_t qmm_dense_workspace_bytes(const ProductArgs &a);
 int32_t launch_qmm_dense(const ProductArgs &a, void *workspace, hipStream_t s);

@@ -33,6 +33,21 @@ constexpr int kPassRows = 64;                 // rows of x per pass: two tiles o
 constexpr int kXStageBytes = kPassRows * 256;  // one window of x: 64 rows x 128 values
 constexpr int kTableMaxBytes = 48 * 1024;
 
+// Piece KK of a lane's 32 affine codes as weights of twice the element type's precision: v = hi + lo.  (The range of hi is the
+// finite one, so that a large or infinite v is lo's.)
+template <typename T, int BITS, int KK>
+__device__ __forceinline__ void expand_split(const uint32_t (&dw)[BITS], float s, float b, uint4 &hi, uint4 &lo) {
+    constexpr float most = Elem<T>::code == NVQ_BF16 ? 3.38953139e38f : 65504.0f;
+    uint32_t h[4], l[4];
+    static_for<4>([&](auto i_tag) {
+        constexpr int i = decltype(i_tag)::value, J = 8 * KK + 2 * i;
+        const float v0 = __builtin_fmaf(code_to_float<BITS, J>(dw), s, b), v1 = __builtin_fmaf(code_to_float<BITS, J + 1>(dw), s, b);
+        h[i] = Ops<T>::pack(__builtin_amdgcn_fmed3f(v0, -most, most), __builtin_amdgcn_fmed3f(v1, -most, most));
+        l[i] = Ops<T>::pack(v0 - half_lo<T>(h[i]), v1 - half_lo<T>(h[i] >> 16));
+    });
+    hi = make_uint4(h[0], h[1], h[2], h[3]), lo = make_uint4(l[0], l[1], l[2], l[3]);
+}
+
 template <int BITS>
 struct Geometry {
     static constexpr int kChunks = 32 * BITS;              // 16-byte chunks of one wavefront's window
@@ -59,6 +74,9 @@ template <typename T, int BITS, int FP4, bool GLU, bool EXACT, bool RAGGED>
 // block (two x stages, the weight stages, the table) fits three times.
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) qmg_kernel(const ProductArgs a) {
     using G = Geometry<BITS>;
+    // Off whole steps affine products that do not take the CPU's weights ran on float32 weights: two terms of the element type
+    // keep their precision.
+    constexpr bool kSplit = RAGGED && FP4 == kAffine && !EXACT;
     constexpr int kDepth = G::kDepth, kLoads = G::kLoads;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     using S = std::conditional_t<FP4 != 0, uint8_t, T>;  // stored scale type
@@ -84,6 +102,10 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
     // caller's error and are clamped so that they cannot fault the device.
     auto rows_of = [&](int ei, int &begin, int &end) {
         const int rows_all = (int)a.batch;
+        if (a.offsets == nullptr) {  // (one group)
+            begin = 0, end = rows_all;
+            return;
+        }
         begin = min(max(a.offsets[ei], 0), rows_all);
         end = ei + 1 < experts ? min(max(a.offsets[ei + 1], begin), rows_all) : rows_all;
     };
@@ -349,6 +371,16 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
                         float scale[2], bias;
                         load_scales(first_of(win) + 64 * t, scale, bias);
                         if (RAGGED && 64 * t + 32 * h < before) scale[0] = scale[1] = bias = 0.0f;
+                        if constexpr (kSplit) {
+                            static_for<4>([&](auto kk_tag) {
+                                constexpr int kk = decltype(kk_tag)::value;
+                                uint4 lo;
+                                expand_split<T, BITS, kk>(codes[t], scale[0], bias, wb[kk], lo);
+                                acc[0] = Ops<T>::mfma(xf[0][kk], wb[kk], Ops<T>::mfma(xf[0][kk], lo, acc[0]));
+                                if (two) acc[1] = Ops<T>::mfma(xf[1][kk], wb[kk], Ops<T>::mfma(xf[1][kk], lo, acc[1]));
+                            });
+                            continue;
+                        }
                         static_for<4>([&](auto kk_tag) {
                             constexpr int kk = decltype(kk_tag)::value;
                             wb[kk] = expand_piece<T, BITS, FP4, kk, EXACT>(codes[t], scale[kk >> 1], bias);

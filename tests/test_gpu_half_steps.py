@@ -38,8 +38,8 @@ def packed(rng, n, k, dtype, fmt):
 def test_tiles(fmt, dtype, m, n, k):
     rng = np.random.default_rng(7100 + m + k)
     q, want = packed(rng, n, k, dtype, fmt)
-    if isinstance(fmt, str) or n < 1024 or dtype == ref.BF16:  # (the rest is of float32 weights on the vector kernels)
-        assert ops.quantized_matmul_route(m, n, k, q.quant, TORCH[dtype]) == "qmm_kernel"
+    rest = not isinstance(fmt, str) and n >= 1024 and dtype == ref.F16  # (weights of two terms on the grouped kernel)
+    assert ops.quantized_matmul_route(m, n, k, q.quant, TORCH[dtype]) == ("qmg_kernel" if rest else "qmm_kernel")
     x = make_x(rng, m, k, dtype)
     assert_rows_close(to_host(nv.quantized_matmul(to_dev(x), q)), want(x), dtype, f"half step {fmt} M={m} N={n} K={k}", exact_weights=isinstance(fmt, str))
 
@@ -49,8 +49,8 @@ def test_tiles(fmt, dtype, m, n, k):
 @pytest.mark.parametrize("fmt", FORMATS + [(64, 4), (128, 6)], ids=str)
 @pytest.mark.parametrize("dtype,n,k", [(ref.BF16, 1100, 160), (ref.F16, 1024, 224), (ref.BF16, 300, 448), (ref.F16, 640, 256), (ref.BF16, 130, 64)])
 def test_grouped(fmt, dtype, n, k):
-    if not isinstance(fmt, str) and (k % fmt[0] != 0 or n >= 1024):
-        pytest.skip("K is not whole groups, or one product per pair on float32 weights")
+    if not isinstance(fmt, str) and k % fmt[0] != 0:
+        pytest.skip("K is not whole groups")
     rng = np.random.default_rng(7200 + n + k)
     experts = [packed(rng, n, k, dtype, fmt) for _ in range(4)]
     stack = lambda f: None if f(experts[0][0]) is None else torch.stack([f(q) for q, _ in experts])
@@ -60,7 +60,35 @@ def test_grouped(fmt, dtype, n, k):
     rows, sorted_ids = torch.arange(ids.size, dtype=torch.int32, device="cuda"), torch.from_numpy(ids).cuda()
     got = to_host(nv.gather_qmm_grouped(to_dev(x), q, rows, sorted_ids, nv.sorted_offsets(sorted_ids, 4)))
     for e in (0, 1, 3):
-        assert_rows_close(got[ids == e], experts[e][1](x[ids == e]), dtype, f"grouped {fmt} N={n} K={k}", exact_weights=isinstance(fmt, str))
+        if isinstance(fmt, str) or n < 1024:
+            assert_rows_close(got[ids == e], experts[e][1](x[ids == e]), dtype, f"grouped {fmt} N={n} K={k}", exact_weights=isinstance(fmt, str))
+        elif k % 64:
+            assert_two_terms(torch.from_numpy(ref.to_f32(got[ids == e], dtype)), torch.from_numpy(ref.to_f32(x[ids == e], dtype)), experts[e][0], dtype, k)
+
+
+def unrounded(q):
+    """scale * code + bias in float64."""
+    codes = nv.dequantize(nv.Quantized(q.weight, torch.ones_like(q.scales, dtype=torch.float32), torch.zeros_like(q.scales, dtype=torch.float32), q.quant))
+    spread = lambda t: t.double().repeat_interleave(q.quant.group_size, dim=-1)
+    return codes.double() * spread(q.scales) + spread(q.biases)
+
+
+def assert_two_terms(got, x, q, dtype, k):
+    """One rounding of the output (u |out|); weights of two terms, u^2 of each, and float32 sums, whose errors are random over K."""
+    u, w = {ref.BF16: 2.0 ** -8, ref.F16: 2.0 ** -11}[dtype], unrounded(q).cpu()
+    want, norms = x.double() @ w.T, x.double().norm(dim=1, keepdim=True) * w.norm(dim=1)
+    assert ((got.double() - want).abs() <= u * want.abs() + 4 * (u * u / 2 + 2.0 ** -24) * norms).all()
+
+
+@pytest.mark.parametrize("bits", [1, 2, 3, 4, 5, 6, 8])
+@pytest.mark.parametrize("dtype,m,n,k", [(torch.float16, 400, 5000, 160), (torch.float16, 130, 4099, 1056), (torch.bfloat16, 100, 8200, 352)])
+def test_rows_on_weights_of_two_terms(bits, dtype, m, n, k):
+    torch.manual_seed(bits + m)
+    quant = nv.Quant.affine(32, bits)
+    assert ops.quantized_matmul_route(m, n, k, quant, dtype) == "qmg_kernel"
+    q = nv.quantize((torch.randn(n, k, device="cuda") * 0.02).to(dtype), quant)
+    x = torch.randn(m, k, device="cuda").to(dtype)
+    assert_two_terms(nv.quantized_matmul(x, q).cpu(), x.cpu(), q, ref.F16 if dtype == torch.float16 else ref.BF16, k)
 
 
 @pytest.mark.parametrize("k", [160, 224])

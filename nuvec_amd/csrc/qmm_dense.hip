@@ -155,7 +155,7 @@ size_t qmm_dense_workspace_bytes(const ProductArgs &a) { return (size_t)a.n * (s
 bool qmm_dense_takes(const ProductArgs &a) {
     if (a.mode != NVQ_AFFINE || !a.exact_weights || a.row_exact || a.batch != 1 || a.batch_ndim != 0 || a.rhs != nullptr || a.lhs != nullptr || a.glu != 0)
         return false;
-    if (a.k < BK || a.k % BK != 0 || a.n * a.k >= (1LL << 32) || (a.m + 127) / 128 > 65535) return false;
+    if (a.k < BK || a.k % BK != 0 || a.k > 1 << 22 || a.n * a.k >= (1LL << 32) || (a.m + 127) / 128 > 65535) return false;  // (32-bit offsets in a tile)
     // Where that kernel splits K it stays: its sums and this kernel's, in one order otherwise, would differ in their last bits, and the
     // entry point that brings no workspace promises the bits of the one that does.
     if (qmm_workspace_bytes(a) != 0) return false;

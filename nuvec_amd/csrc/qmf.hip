@@ -11,22 +11,24 @@ namespace nvq {
 // element type does not hold).  Row-exact pairs keep the vector kernels where they had them, with the
 // CPU's weights and off whole steps.
 static bool grouped_supported(const ProductArgs &a) {
-    if (a.m != 1 || a.experts > 65535 || qmg::table_bytes(a) > (size_t)qmg::kTableMaxBytes) return false;
+    if (a.m != 1 || a.experts > 65535) return false;
     const bool odd = a.mode == NVQ_AFFINE && a.bits % 2 != 0, whole = a.k >= 64 && a.k % (odd ? 128 : 64) == 0;
     if (a.row_exact && (a.exact_weights || !whole)) return false;
+    if (whole ? qmg::table_bytes(a) > (size_t)qmg::kTableMaxBytes : qmg::lds_bytes(a) > (size_t)qmg::kLdsMost) return false;
     return whole || (a.k >= 128 && a.k % 32 == 0 && (a.mode == NVQ_AFFINE || a.global_scale == nullptr));
 }
 
 // The rows of one product as one group: affine codes off whole steps of 64 whose weights are not the CPU's (those are the tiled
-// kernel's).  The vector kernel's passes of four rows take 1 us per 2.1 M weights, a window of this kernel 2.5 us with two
-// blocks on a compute unit.
+// kernel's).  The vector kernel's passes of four rows take 1 us per 2.1 M weights, a window of this kernel 2.5 us with one
+// or two blocks on a compute unit.
 bool grouped_rows_take(const ProductArgs &a) {
     if ((a.dtype != NVQ_BF16 && a.dtype != NVQ_F16) || a.mode != NVQ_AFFINE || a.exact_weights || a.row_exact || a.batch != 1 || a.batch_ndim != 0 ||
-        a.rhs != nullptr || a.lhs != nullptr || a.glu != 0 || a.k % 64 != 32 || a.k < 128 || qmg::table_bytes(a) > (size_t)qmg::kTableMaxBytes)
+        a.rhs != nullptr || a.lhs != nullptr || a.glu != 0 || a.k % 64 != 32 || a.k < 128 || qmg::lds_bytes(a) > (size_t)qmg::kLdsMost)
         return false;
     const double blocks = (double)((a.n + qmg::kRows - 1) / qmg::kRows) * (double)((a.m + qmg::kPassRows - 1) / qmg::kPassRows);
     if (blocks > 1e8) return false;
-    const double here = 15.0 + ceil(blocks / (2.0 * fmax(1.0, (double)compute_units()))) * (double)((a.k + 127) / 128) * 2.5;
+    const double per_unit = qmg::lds_bytes(a) <= (size_t)qmg::kLdsMost / 2 ? 2.0 : 1.0;
+    const double here = 15.0 + ceil(blocks / (per_unit * fmax(1.0, (double)compute_units()))) * (double)((a.k + 127) / 128) * 2.5;
     return here < 0.8 * (double)((a.m + 3) / 4) * (double)a.n * (double)a.k / 2.1e6;
 }
 

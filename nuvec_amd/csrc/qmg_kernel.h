@@ -31,7 +31,8 @@ constexpr int kThreads = 64 * kWaves;
 constexpr int kRows = 32 * kWaves;            // weight rows per block
 constexpr int kPassRows = 64;                 // rows of x per pass: two tiles of 32
 constexpr int kXStageBytes = kPassRows * 256;  // one window of x: 64 rows x 128 values
-constexpr int kTableMaxBytes = 48 * 1024;
+constexpr int kTableMaxBytes = 48 * 1024;  // three blocks on a compute unit
+constexpr int kLdsMost = 160 * 1024;       // of a block off whole steps of K, whose long rows would else go four at a time
 
 // Piece KK of a lane's 32 affine codes as weights of twice the element type's precision: v = hi + lo.  (The range of hi is the
 // finite one, so that a large or infinite v is lo's.)
@@ -461,6 +462,8 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
 
 // Bytes of the LDS table of scales (and biases) for the block's rows.
 inline size_t table_bytes(const ProductArgs &a) { return qmf::table_bytes(a, kRows); }
+// All LDS of a block.
+inline size_t lds_bytes(const ProductArgs &a) { return 2 * kXStageBytes + kWaves * 512 * (size_t)a.bits + table_bytes(a); }
 
 template <typename T, int BITS, int FP4, bool GLU, bool EXACT, bool RAGGED>
 int32_t run_kernel(const ProductArgs &a, hipStream_t s) {
@@ -470,7 +473,7 @@ int32_t run_kernel(const ProductArgs &a, hipStream_t s) {
     const size_t lds_bytes = G::kFixedLdsBytes + table_bytes(a);
     if (!configured) {
         NVQ_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                        G::kFixedLdsBytes + kTableMaxBytes));
+                                        RAGGED ? kLdsMost : G::kFixedLdsBytes + kTableMaxBytes));
         configured = true;
     }
     // every expert with rows adds at most one partial pass: blocks for that many items, the rest leave at once

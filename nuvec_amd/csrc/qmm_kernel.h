@@ -177,7 +177,7 @@ qmm_kernel(const ProductArgs a) {
     // K of whole steps and a half: the last step begins 32 values early, so that every load stays inside its row.  The
     // values that the step before has counted are zeros in both operands: the x tile's chunks 0..3 are overwritten in
     // LDS once they have arrived, the lanes of half 0 take a scale and bias of zero.  (Passes of four rows on the vector
-    // kernel took these products before: 323 rows, W[2844,5088], NVFP4, 1311 us.)
+    // kernel took these products before: 323 rows, W[2844,5088], NVFP4, 1311 us against 34.)
     const int half_step = step0 + steps == all_steps ? steps - 1 : -1;
     int64_t bx = 0, bw = 0, bs = 0, by = 0;
     if constexpr (BATCHED) {  // a batch with one stride per operand

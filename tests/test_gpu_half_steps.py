@@ -81,7 +81,7 @@ def assert_two_terms(got, x, q, dtype, k):
 
 
 @pytest.mark.parametrize("bits", [1, 2, 3, 4, 5, 6, 8])
-@pytest.mark.parametrize("dtype,m,n,k", [(torch.float16, 400, 5000, 160), (torch.float16, 130, 4099, 1056), (torch.bfloat16, 100, 8200, 352)])
+@pytest.mark.parametrize("dtype,m,n,k", [(torch.float16, 400, 5000, 160), (torch.float16, 130, 4099, 1056), (torch.bfloat16, 100, 8200, 352), (torch.float16, 300, 1100, 6944)])
 def test_rows_on_weights_of_two_terms(bits, dtype, m, n, k):
     torch.manual_seed(bits + m)
     quant = nv.Quant.affine(32, bits)

@@ -4,7 +4,8 @@
 // one call took 12 to 17 us in Python (a one-row product of W[1024,4096]: 16.7 us per call, of which the kernel is 3.4).  Here
 // the same work is done on the tensors' own C++ objects, a block's layers in one call.
 //
-// Every function takes the plain case alone: operands on the bound device, dense, of one element type, of matching shapes.
+// Every function takes the plain case alone: operands on the bound device, dense, of one element type, of matching shapes, and
+// layers whose methods are the package's own.
 // Whatever else it meets (and whatever the library refuses) it declines by returning None, before anything is launched, and
 // the caller's Python path, which holds every conversion and the reference's messages, does the call.
 #include <torch/csrc/Dtype.h>
@@ -14,6 +15,8 @@
 #include <ATen/core/Tensor.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+
+#include <vector>
 
 #include "nuvec_hip.h"
 
@@ -28,8 +31,6 @@ struct Names {
     PyObject *gate, *switch_mlp, *experts_per_token, *norm_topk_prob, *gate_up_paired, *activation, *alpha, *limit;
 } names;
 
-// layers.QuantizedLinear, SwitchProjection, SwitchGlu: their forwards are the ones restated here (a subclass may have another)
-PyTypeObject *linear_type = nullptr, *projection_type = nullptr, *switch_glu_type = nullptr;
 uint64_t ready_devices = 0;           // devices nvq_init has answered for (ops._init), read and written under the GIL
 
 struct Ref {
@@ -43,6 +44,24 @@ bool declined() {
     PyErr_Clear();
     return false;
 }
+
+// A class of `layers` and the methods of it that a call here stands in for.  An object is plain if it is of that very class
+// (a subclass may have others), the class still holds the functions it was defined with, and the object has none of its own.
+struct Kind {
+    PyTypeObject *type = nullptr;
+    std::vector<std::pair<PyObject *, PyObject *>> methods;  // name, function
+
+    bool plain(PyObject *o) const {
+        if (type == nullptr || Py_TYPE(o) != type) return false;
+        PyObject **own = _PyObject_GetDictPtr(o);
+        for (const auto &m : methods) {
+            if (PyDict_GetItemWithError(type->tp_dict, m.first) != m.second) return declined();
+            if (own != nullptr && *own != nullptr && PyDict_GetItemWithError(*own, m.first) != nullptr) return false;
+        }
+        return true;
+    }
+};
+Kind linear_kind, projection_kind, switch_glu_kind, moe_kind;
 
 bool read_int(PyObject *o, PyObject *name, int32_t &v) {
     Ref a(PyObject_GetAttr(o, name));
@@ -341,7 +360,7 @@ struct Linear {
     Tensor bias;
 };
 bool read_linear(PyObject *o, Linear &l) {
-    if (Py_TYPE(o) != linear_type) return false;
+    if (!linear_kind.plain(o)) return false;
     if (!read_tensor(o, names.weight, l.p.w) || !read_tensor(o, names.scales, l.p.s) || !read_tensor(o, names.biases, l.p.b) ||
         !read_tensor(o, names.bias, l.bias))
         return false;
@@ -428,7 +447,7 @@ PyObject *py_mlp(PyObject *, PyObject *const *args, Py_ssize_t n) {
 bool read_projection(PyObject *o, PyObject *name, Projection &j) {
     Ref a(PyObject_GetAttr(o, name));
     if (a.p == nullptr) return declined();
-    if (Py_TYPE(a.p) != projection_type) return false;
+    if (!projection_kind.plain(a.p)) return false;
     Tensor global_scale;
     if (!read_tensor(a.p, names.weight, j.p.w) || !read_tensor(a.p, names.scales, j.p.s) || !read_tensor(a.p, names.biases, j.p.b) ||
         !read_tensor(a.p, names.bias, j.bias) || !read_tensor(a.p, names.global_scale, global_scale) || global_scale.defined())
@@ -444,11 +463,11 @@ PyObject *py_moe(PyObject *, PyObject *const *args, Py_ssize_t n) {
         int32_t k;
         bool normalize;
         Experts e;
-        if (n != 2 || !as_tensor(args[1], x) || !read_tensor(args[0], names.gate, router) || !read_int(args[0], names.experts_per_token, k) ||
+        if (n != 2 || !moe_kind.plain(args[0]) || !as_tensor(args[1], x) || !read_tensor(args[0], names.gate, router) || !read_int(args[0], names.experts_per_token, k) ||
             !read_truth(args[0], names.norm_topk_prob, normalize))
             return none();
         Ref glu(PyObject_GetAttr(args[0], names.switch_mlp));
-        if (glu.p == nullptr || Py_TYPE(glu.p) != switch_glu_type) {
+        if (glu.p == nullptr || !switch_glu_kind.plain(glu.p)) {
             PyErr_Clear();
             return none();
         }
@@ -592,16 +611,22 @@ PyObject *py_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
     });
 }
 
-// register(QuantizedLinear, SwitchProjection, SwitchGlu): the types whose forward is restated here
+// register((type, {name: function}), ...): QuantizedLinear, SwitchProjection, SwitchGlu and MoeMlp with their own methods
 PyObject *py_register(PyObject *, PyObject *const *args, Py_ssize_t n) {
-    PyTypeObject **types[] = {&linear_type, &projection_type, &switch_glu_type};
-    for (Py_ssize_t i = 0; i < 3; i++) {
-        if (n != 3 || !PyType_Check(args[i])) {
-            PyErr_SetString(PyExc_TypeError, "register(QuantizedLinear, SwitchProjection, SwitchGlu)");
+    Kind *const kinds[] = {&linear_kind, &projection_kind, &switch_glu_kind, &moe_kind};
+    PyObject *types[4], *methods[4];
+    for (Py_ssize_t i = 0; i < 4; i++) {
+        if (n != 4 || !PyArg_ParseTuple(args[i], "O!O!", &PyType_Type, &types[i], &PyDict_Type, &methods[i])) {
+            PyErr_SetString(PyExc_TypeError, "register: four pairs of a class and its methods");
             return nullptr;
         }
-        Py_INCREF(args[i]);
-        *types[i] = (PyTypeObject *)args[i];
+    }
+    for (Py_ssize_t i = 0; i < 4; i++) {
+        Py_INCREF(types[i]), Py_INCREF(methods[i]);  // (kept until the process ends, with the names and functions they hold)
+        kinds[i]->methods.clear();
+        PyObject *name, *function;
+        for (Py_ssize_t at = 0; PyDict_Next(methods[i], &at, &name, &function);) kinds[i]->methods.emplace_back(name, function);
+        kinds[i]->type = (PyTypeObject *)types[i];
     }
     return none();
 }

@@ -18,10 +18,10 @@ _native = None
 
 
 def _calls():
-    """The native calls, told which layers they may read."""
+    """The native calls, told which layers they may read and which of their methods they stand in for."""
     global _native
     n = _lib.native()
-    n.register(QuantizedLinear, SwitchProjection, SwitchGlu)
+    n.register(*_OWN_METHODS)
     _native = n
     return n
 
@@ -138,8 +138,7 @@ class QuantizedEmbedding:
         """layers.rs:245-255: the rows for `ids`, dequantized (scales' dtype for affine, bfloat16 for the
         floating-point modes): shape `ids.shape + [dims]`.  One fused kernel; the taken packed rows are
         never written out."""
-        y = (_native or _calls()).embedding(self.weight, self.scales, self.biases, self.quant, ids)
-        return ops.embedding(self.quantized(), ids) if y is None else y
+        return ops.embedding(self.quantized(), ids)
 
     def as_linear(self, x: torch.Tensor) -> torch.Tensor:
         """layers.rs:258-261: `x W^T` with the quantized table (tied embeddings)."""
@@ -323,6 +322,16 @@ class MoeMlp:
         return ops.weighted_sum(experts, scores)
 
     __call__ = forward
+
+
+def _own(layer, *names):
+    return layer, {name: vars(layer)[name] for name in names}
+
+
+# What a native call of a layer or of a block that holds it stands in for, as the classes define it: a subclass, a class or an
+# object with another of these takes the Python path, which calls it.
+_OWN_METHODS = (_own(QuantizedLinear, "__call__", "quantized"), _own(SwitchProjection, "forward", "forward_sorted_rows", "quantized"),
+                _own(SwitchGlu, "forward", "gated"), _own(MoeMlp, "route"))
 
 
 def quantized_attention(q: torch.Tensor, k: ops.Quantized, v: ops.Quantized, scale: float,

@@ -94,6 +94,73 @@ def test_refusals_are_the_python_paths():
     assert mixed.dtype == torch.float32
 
 
+def experts(dims=256, hidden=1024, dtype=torch.bfloat16, count=8):
+    """A block of experts, its gate and up projections fused."""
+    put = lambda *shape: (torch.randn(shape, device="cuda") * 0.1).to(dtype)
+
+    def projection(n, k):
+        q = nv.quantize(put(count, n, k), nv.Quant.affine(64, 4))
+        return layers.SwitchProjection(q.weight, q.scales, q.biases, put(count, n), q.quant)
+    return layers.SwitchGlu(projection(hidden, dims), projection(hidden, dims), projection(dims, hidden)).fuse_gate_up(), put(count, dims)
+
+
+@pytest.mark.parametrize("tokens", [1, 40])
+def test_a_router_of_its_own(tokens):
+    """`MoeMlp.route` is what routes, whoever defines it: a subclass or the block itself."""
+    torch.manual_seed(4)
+    glu, gate = experts()
+    x = torch.randn(1, tokens, 256, device="cuda").bfloat16()
+    top = torch.tensor([6, 1], dtype=torch.int32, device="cuda").expand(1, tokens, 2).contiguous()
+    scores = torch.tensor([0.25, 2.0], device="cuda").bfloat16().expand(1, tokens, 2).contiguous()
+    want = nv.ops.weighted_sum(glu.forward(x, top), scores)
+
+    class Fixed(layers.MoeMlp):
+        def route(self, x):
+            return top, scores
+    assert torch.equal(Fixed(gate, glu, 2)(x), want)
+    block = layers.MoeMlp(gate, glu, 2)
+    assert not torch.equal(block(x), want)
+    block.route = lambda x: (top, scores)
+    assert torch.equal(block(x), want)
+
+
+def test_methods_of_their_own(monkeypatch):
+    """A layer's method that a class or an object replaces is called, wherever the layer is held."""
+    torch.manual_seed(5)
+    glu, gate = experts()
+    block, x = layers.MoeMlp(gate, glu, 2), torch.randn(1, 3, 256, device="cuda").bfloat16()
+    plain = block(x)
+    for holder, name in ((glu, "forward"), (glu.gate_up_proj, "quantized"), (glu.down_proj, "forward")):
+        seen, method = [], getattr(holder, name)
+        setattr(holder, name, lambda *a, **k: seen.append(1) or method(*a, **k))
+        got = block(x)
+        assert seen and (got.float() - plain.float()).abs().max() <= 4 * 2.0 ** -8 * plain.float().abs().max(), name
+        delattr(holder, name)
+        assert torch.equal(block(x), plain)
+    for kind in (layers.SwitchProjection, layers.SwitchGlu):
+        seen, method = [], kind.forward
+        with monkeypatch.context() as m:
+            m.setattr(kind, "forward", lambda *a, **k: seen.append(1) or method(*a, **k))
+            block(x)
+        assert seen, kind
+
+    mlp = layers.Mlp(linear(1024, 256, nv.Quant.affine(64, 4), torch.bfloat16, True), linear(1024, 256, nv.Quant.affine(64, 4), torch.bfloat16, True),
+                     linear(256, 1024, nv.Quant.affine(64, 4), torch.bfloat16, False))
+    row, seen, call = x[0, :1], [], layers.QuantizedLinear.__call__
+    want = mlp(row)
+    with monkeypatch.context() as m:
+        m.setattr(layers.QuantizedLinear, "__call__", lambda self, x: seen.append(self) or call(self, x))
+        assert torch.equal(mlp(row), want) and len(seen) == 3
+
+    table = nv.quantize(torch.randn(20, 128, device="cuda"), nv.Quant.affine(64, 4))
+
+    class Doubled(layers.QuantizedEmbedding):
+        def quantized(self):
+            return nv.Quantized(self.weight, 2 * self.scales, 2 * self.biases, self.quant)
+    ids = torch.tensor([3, 19], dtype=torch.int32, device="cuda")
+    assert torch.equal(Doubled(table.weight, table.scales, table.biases, table.quant)(ids), 2 * nv.embedding(table, ids))
+
+
 @pytest.mark.parametrize("rows,dims,experts,k", [(1, 2880, 32, 4), (7, 64, 3, 3), (300, 520, 128, 8), (5, 8, 1, 1), (2, 1032, 300, 6)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_router(rows, dims, experts, k, dtype):

@@ -592,6 +592,8 @@ PyObject *py_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
             return none();
         const nvq_attention_desc d{code, k.q.bits, k.q.group_size, (int32_t)dim, q.size(0), q.size(1), k.w.size(1), k.w.size(2), (float)scale};
         Tensor workspace, y = at.empty(q.sizes(), type);
+        // (ops.quantized_attention_fits: one query row takes caches of unsigned words)
+        if (q.size(2) == 1 && (k.w.scalar_type() != at::kUInt32 || v.w.scalar_type() != at::kUInt32)) return none();
         if (q.size(2) > 1) {
             const int causal = PyObject_IsTrue(args[10]);
             if (causal < 0) return nullptr;

@@ -505,7 +505,7 @@ def quantized_attention(q: torch.Tensor, k: Quantized, v: Quantized, scale: floa
                         sinks: Optional[torch.Tensor] = None, scratch: bool = True) -> torch.Tensor:
     """fast.rs:694-718 where the kernel fits (`quantized_attention_fits`): one query row per head over the quantized
     cache in one launch."""
-    if scratch and k.quant == v.quant:
+    if scratch and q.ndim == 4 and q.shape[2] == 1 and k.quant == v.quant:
         out = (_lib._native or _lib.native()).attention(q, k.weight, k.scales, k.biases, v.weight, v.scales, v.biases, k.quant, scale, sinks, False)
         if out is not None:
             return out

@@ -161,6 +161,24 @@ def test_methods_of_their_own(monkeypatch):
     assert torch.equal(Doubled(table.weight, table.scales, table.biases, table.quant)(ids), 2 * nv.embedding(table, ids))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_one_query_row_alone(dtype):
+    """`ops.quantized_attention` is one query row per head over caches of unsigned words: what else it refuses, so that the
+    caller's masked composition runs, whatever the type, the scratch and the density."""
+    k, v = (nv.quantize(torch.randn(2, 2, 96, 64, device="cuda").to(dtype), nv.Quant.affine(32, 4)) for _ in range(2))
+    signed = [nv.Quantized(t.weight.view(torch.int32), t.scales, t.biases, t.quant) for t in (k, v)]
+    q = torch.randn(2, 4, 3, 64, device="cuda").to(dtype)
+    for scratch in (True, False):
+        for queries in (q, q.transpose(1, 2).contiguous().transpose(1, 2)):
+            with pytest.raises(nv.Unsupported):
+                nv.ops.quantized_attention(queries, k, v, 0.125, scratch=scratch)
+        with pytest.raises(nv.Unsupported):
+            nv.ops.quantized_attention(q[:, :, :1].contiguous(), *signed, 0.125, scratch=scratch)
+    one = q[:, :, :1].contiguous()
+    composed = layers.quantized_attention(one, *signed, 0.125, fused=False)
+    assert torch.equal(layers.quantized_attention(one, *signed, 0.125), composed)
+
+
 @pytest.mark.parametrize("rows,dims,experts,k", [(1, 2880, 32, 4), (7, 64, 3, 3), (300, 520, 128, 8), (5, 8, 1, 1), (2, 1032, 300, 6)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_router(rows, dims, experts, k, dtype):

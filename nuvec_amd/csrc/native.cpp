@@ -9,6 +9,7 @@
 // Whatever else it meets (and whatever the library refuses) it declines by returning None, before anything is launched, and
 // the caller's Python path, which holds every conversion and the reference's messages, does the call.
 #include <torch/csrc/Dtype.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/hip/EmptyTensor.h>
@@ -379,8 +380,8 @@ template <typename F>
 PyObject *guarded(F &&f) {
     try {
         return f();
-    } catch (const std::exception &e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what());
+    } catch (...) {  // (torch.OutOfMemoryError among them)
+        torch::translate_exception_to_python(std::current_exception());
         return nullptr;
     }
 }

@@ -179,6 +179,21 @@ def test_one_query_row_alone(dtype):
     assert torch.equal(layers.quantized_attention(one, *signed, 0.125), composed)
 
 
+def test_out_of_memory_is_torchs():
+    """An allocation that fails inside a native call raises what torch's own allocation raises."""
+    layer = linear(65536, 256, nv.Quant.affine(64, 4), torch.bfloat16, False)
+    x = torch.randn(8192, 256, device="cuda").bfloat16()  # (an output of 1 GB)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    torch.cuda.set_per_process_memory_fraction(0.0)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            layer(x)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert layer(x).shape == (8192, 65536)
+
+
 @pytest.mark.parametrize("rows,dims,experts,k", [(1, 2880, 32, 4), (7, 64, 3, 3), (300, 520, 128, 8), (5, 8, 1, 1), (2, 1032, 300, 6)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_router(rows, dims, experts, k, dtype):

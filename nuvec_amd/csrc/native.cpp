@@ -8,6 +8,8 @@
 // layers whose methods are the package's own.
 // Whatever else it meets (and whatever the library refuses) it declines by returning None, before anything is launched, and
 // the caller's Python path, which holds every conversion and the reference's messages, does the call.
+//
+// The interpreter lock is released while a call allocates and launches, as ctypes and torch's own operators release it.
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -17,6 +19,7 @@
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 
+#include <atomic>
 #include <vector>
 
 #include "nuvec_hip.h"
@@ -32,7 +35,7 @@ struct Names {
     PyObject *gate, *switch_mlp, *experts_per_token, *norm_topk_prob, *gate_up_paired, *activation, *alpha, *limit;
 } names;
 
-uint64_t ready_devices = 0;           // devices nvq_init has answered for (ops._init), read and written under the GIL
+std::atomic<uint64_t> ready_devices{0};  // devices nvq_init has answered for (ops._init)
 
 struct Ref {
     PyObject *p;
@@ -386,6 +389,17 @@ PyObject *guarded(F &&f) {
     }
 }
 
+// `f`, which touches no Python object, without the interpreter lock.
+struct Unlocked {
+    PyThreadState *state = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
+template <typename F>
+bool unlocked(F &&f) {
+    const Unlocked here;
+    return f();
+}
+
 PyObject *wrap(bool done, Tensor &y) { return done ? THPVariable_Wrap(std::move(y)) : none(); }
 
 // linear(layer, x)
@@ -394,7 +408,7 @@ PyObject *py_linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
         Tensor x, y;
         Linear l;
         if (n != 2 || !as_tensor(args[1], x) || !read_linear(args[0], l)) return none();
-        return wrap(product(x, l.p, l.bias, Flags(), y), y);
+        return wrap(unlocked([&] { return product(x, l.p, l.bias, Flags(), y); }), y);
     });
 }
 
@@ -410,7 +424,7 @@ PyObject *py_quantized_matmul(PyObject *, PyObject *const *args, Py_ssize_t n) {
         for (int i = 0; i < 4; i++)
             if ((flag[i] = PyObject_IsTrue(args[5 + i])) < 0) return nullptr;
         const Flags f{flag[0] != 0, flag[1] != 0, flag[2] != 0, flag[3] != 0};
-        return wrap(product(x, p, bias, f, y), y);
+        return wrap(unlocked([&] { return product(x, p, bias, f, y); }), y);
     });
 }
 
@@ -418,7 +432,7 @@ PyObject *py_quantized_matmul(PyObject *, PyObject *const *args, Py_ssize_t n) {
 PyObject *py_mlp(PyObject *, PyObject *const *args, Py_ssize_t n) {
     return guarded([&]() -> PyObject * {
         Tensor x, hidden, y;
-        Linear down, gate, up;
+        Linear down, gate, up, fused;
         if (n != 2 || !as_tensor(args[1], x) || !x.defined() || x.dim() < 1 || x.numel() == 0) return none();
         Ref geglu(PyObject_GetAttr(args[0], names.geglu)), both(PyObject_GetAttr(args[0], names.gate_up_proj));
         if (geglu.p == nullptr || both.p == nullptr || !read_linear(args[0], names.down_proj, down) ||
@@ -430,18 +444,19 @@ PyObject *py_mlp(PyObject *, PyObject *const *args, Py_ssize_t n) {
         if (truth < 0) return nullptr;
         const int32_t activation = truth ? NVQ_GLU_GEGLU : NVQ_GLU_SWIGLU;
         const int64_t rows = x.numel() / x.size(-1), most = gate.p.q.mode == NVQ_AFFINE ? 2 : 4;  // (layers.Mlp.forward says why)
-        if (both.p != Py_None && rows <= most) {
-            Linear l;
-            if (!read_linear(both.p, l)) return none();
-            product_glu(x, l.p, l.bias, activation, 0.0f, 0.0f, hidden);
-        }
-        if (!hidden.defined()) {
-            Tensor g, u;
-            if (!read_linear(args[0], names.up_proj, up) || !product(x, gate.p, gate.bias, Flags(), g) || !product(x, up.p, up.bias, Flags(), u) ||
-                g.sizes() != u.sizes() || !gated(g, u, activation, hidden))
-                return none();
-        }
-        return wrap(product(hidden, down.p, down.bias, Flags(), y), y);
+        const bool one = both.p != Py_None && rows <= most;
+        if ((one && !read_linear(both.p, fused)) || !read_linear(args[0], names.up_proj, up)) return none();
+        const bool done = unlocked([&] {
+            if (one) product_glu(x, fused.p, fused.bias, activation, 0.0f, 0.0f, hidden);
+            if (!hidden.defined()) {
+                Tensor g, u;
+                if (!product(x, gate.p, gate.bias, Flags(), g) || !product(x, up.p, up.bias, Flags(), u) || g.sizes() != u.sizes() ||
+                    !gated(g, u, activation, hidden))
+                    return false;
+            }
+            return product(hidden, down.p, down.bias, Flags(), y);
+        });
+        return wrap(done, y);
     });
 }
 
@@ -487,7 +502,7 @@ PyObject *py_moe(PyObject *, PyObject *const *args, Py_ssize_t n) {
             !read_truth(glu.p, names.gate_up_paired, e.paired) || !read_float(glu.p, names.alpha, e.act.alpha) ||
             !read_float(glu.p, names.limit, e.act.limit))
             return none();
-        return wrap(moe(x, router, k, normalize, e, y), y);
+        return wrap(unlocked([&] { return moe(x, router, k, normalize, e, y); }), y);
     });
 }
 
@@ -503,12 +518,15 @@ PyObject *py_quantize(PyObject *, PyObject *const *args, Py_ssize_t n) {
         if (q.group_size <= 0 || cols % q.group_size != 0) return none();
         const bool affine = q.mode == NVQ_AFFINE;
         const Sizes groups = with_last(w.sizes(), cols / q.group_size);
-        Tensor packed = at.empty(with_last(w.sizes(), cols * q.bits / 32), at::kUInt32);
-        Tensor scales = at.empty(groups, affine ? w.scalar_type() : at::kByte), biases;
-        if (affine) biases = at.empty(groups, w.scalar_type());
-        if (nvq_quantize(&q, code_of(w.scalar_type()), ptr(w), w.numel() / cols, cols, packed.mutable_data_ptr(), scales.mutable_data_ptr(),
-                         affine ? biases.mutable_data_ptr() : nullptr, at.stream()) != NVQ_OK)
-            return none();
+        Tensor packed, scales, biases;
+        const bool done = unlocked([&] {
+            packed = at.empty(with_last(w.sizes(), cols * q.bits / 32), at::kUInt32);
+            scales = at.empty(groups, affine ? w.scalar_type() : at::kByte);
+            if (affine) biases = at.empty(groups, w.scalar_type());
+            return nvq_quantize(&q, code_of(w.scalar_type()), ptr(w), w.numel() / cols, cols, packed.mutable_data_ptr(), scales.mutable_data_ptr(),
+                                affine ? biases.mutable_data_ptr() : nullptr, at.stream()) == NVQ_OK;
+        });
+        if (!done) return none();
         Ref p(THPVariable_Wrap(std::move(packed))), s(THPVariable_Wrap(std::move(scales)));
         Ref b(affine ? THPVariable_Wrap(std::move(biases)) : none());
         return p.p && s.p && b.p ? PyTuple_Pack(3, p.p, s.p, b.p) : nullptr;
@@ -536,9 +554,12 @@ PyObject *py_dequantize(PyObject *, PyObject *const *args, Py_ssize_t n) {
         int64_t columns;
         if (!at.usable() || code_of(type) < 0 || asked != type || p.w.dim() < 2 || p.w.numel() == 0 || !p.fits(at, type, p.w.dim(), columns))
             return none();
-        Tensor y = at.empty(with_last(p.w.sizes(), columns), type);
-        const bool done = nvq_dequantize(&p.q, code_of(type), ptr(p.w), ptr(p.s), ptr(p.b), y.numel() / columns, columns,
-                                         y.mutable_data_ptr(), at.stream()) == NVQ_OK;
+        Tensor y;
+        const bool done = unlocked([&] {
+            y = at.empty(with_last(p.w.sizes(), columns), type);
+            return nvq_dequantize(&p.q, code_of(type), ptr(p.w), ptr(p.s), ptr(p.b), y.numel() / columns, columns, y.mutable_data_ptr(),
+                                  at.stream()) == NVQ_OK;
+        });
         return wrap(done, y);
     });
 }
@@ -559,9 +580,12 @@ PyObject *py_embedding(PyObject *, PyObject *const *args, Py_ssize_t n) {
             return none();
         Sizes sizes(ids.sizes().begin(), ids.sizes().end());
         sizes.push_back(columns);
-        Tensor y = at.empty(sizes, type);
-        const bool done = nvq_dequantize_rows(&p.q, code_of(type), ptr(p.w), ptr(p.s), ptr(p.b), p.w.size(0), columns,
-                                              (const uint32_t *)ptr(ids), ids.numel(), y.mutable_data_ptr(), at.stream()) == NVQ_OK;
+        Tensor y;
+        const bool done = unlocked([&] {
+            y = at.empty(sizes, type);
+            return nvq_dequantize_rows(&p.q, code_of(type), ptr(p.w), ptr(p.s), ptr(p.b), p.w.size(0), columns, (const uint32_t *)ptr(ids),
+                                       ids.numel(), y.mutable_data_ptr(), at.stream()) == NVQ_OK;
+        });
         return wrap(done, y);
     });
 }
@@ -592,24 +616,25 @@ PyObject *py_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
             !bias_fits(sinks, at, type, q.size(1)))
             return none();
         const nvq_attention_desc d{code, k.q.bits, k.q.group_size, (int32_t)dim, q.size(0), q.size(1), k.w.size(1), k.w.size(2), (float)scale};
-        Tensor workspace, y = at.empty(q.sizes(), type);
+        const bool several = q.size(2) > 1;
         // (ops.quantized_attention_fits: one query row takes caches of unsigned words)
-        if (q.size(2) == 1 && (k.w.scalar_type() != at::kUInt32 || v.w.scalar_type() != at::kUInt32)) return none();
-        if (q.size(2) > 1) {
-            const int causal = PyObject_IsTrue(args[10]);
-            if (causal < 0) return nullptr;
-            const nvq_attention_prompt_desc p{d, q.size(2), causal};
-            const size_t bytes = nvq_quantized_attention_prompt_workspace_bytes(&p);
-            if (bytes == 0) return none();
-            workspace = at.empty({(int64_t)bytes}, at::kByte);
-            const bool done = nvq_quantized_attention_prompt(&p, ptr(q), ptr(k.w), ptr(k.s), ptr(k.b), ptr(v.w), ptr(v.s), ptr(v.b), ptr(sinks),
-                                                             y.mutable_data_ptr(), workspace.mutable_data_ptr(), at.stream()) == NVQ_OK;
-            return wrap(done, y);
-        }
-        const size_t need = nvq_quantized_attention_workspace_bytes(&d);
-        if (need > 0) workspace = at.empty({(int64_t)need}, at::kByte);
-        const bool done = nvq_quantized_attention(&d, ptr(q), ptr(k.w), ptr(k.s), ptr(k.b), ptr(v.w), ptr(v.s), ptr(v.b), ptr(sinks),
-                                                  y.mutable_data_ptr(), need > 0 ? workspace.mutable_data_ptr() : nullptr, at.stream()) == NVQ_OK;
+        if (!several && (k.w.scalar_type() != at::kUInt32 || v.w.scalar_type() != at::kUInt32)) return none();
+        const int causal = PyObject_IsTrue(args[10]);
+        if (causal < 0) return nullptr;
+        const nvq_attention_prompt_desc prompt{d, q.size(2), causal};
+        Tensor y;
+        const bool done = unlocked([&] {
+            const size_t need = several ? nvq_quantized_attention_prompt_workspace_bytes(&prompt) : nvq_quantized_attention_workspace_bytes(&d);
+            if (several && need == 0) return false;
+            y = at.empty(q.sizes(), type);
+            Tensor workspace;
+            if (need > 0) workspace = at.empty({(int64_t)need}, at::kByte);
+            void *scratch = need > 0 ? workspace.mutable_data_ptr() : nullptr;
+            return (several ? nvq_quantized_attention_prompt(&prompt, ptr(q), ptr(k.w), ptr(k.s), ptr(k.b), ptr(v.w), ptr(v.s), ptr(v.b), ptr(sinks),
+                                                             y.mutable_data_ptr(), scratch, at.stream())
+                            : nvq_quantized_attention(&d, ptr(q), ptr(k.w), ptr(k.s), ptr(k.b), ptr(v.w), ptr(v.s), ptr(v.b), ptr(sinks),
+                                                      y.mutable_data_ptr(), scratch, at.stream())) == NVQ_OK;
+        });
         return wrap(done, y);
     });
 }

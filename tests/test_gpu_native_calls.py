@@ -194,6 +194,42 @@ def test_out_of_memory_is_torchs():
     assert layer(x).shape == (8192, 65536)
 
 
+def test_streams_and_threads():
+    """Calls of several host threads, each on a stream of its own: every result is the one-thread result on the default stream."""
+    import threading
+    torch.manual_seed(6)
+    glu, gate = experts()
+    moe, layer = layers.MoeMlp(gate, glu, 2), linear(1024, 256, nv.Quant.affine(64, 4), torch.bfloat16, True)
+    mlp = layers.Mlp(linear(1024, 256, nv.Quant.affine(64, 4), torch.bfloat16, False), linear(1024, 256, nv.Quant.affine(64, 4), torch.bfloat16, False),
+                     linear(256, 1024, nv.Quant.affine(64, 4), torch.bfloat16, False)).fuse_gate_up()
+    k, v = (nv.quantize(torch.randn(1, 2, 2500, 64, device="cuda").bfloat16(), nv.Quant.affine(32, 8)) for _ in range(2))
+
+    def work(seed):
+        g = torch.Generator(device="cuda")
+        g.manual_seed(seed)
+        put = lambda *shape: torch.randn(shape, device="cuda", generator=g).bfloat16()
+        x, row, q, few = put(1, 40, 256), put(1, 256), put(1, 8, 1, 64), put(1, 8, 5, 64)
+        return [moe(x), layer(x), mlp(row), mlp(x[0]), layers.quantized_attention(q, k, v, 0.125, causal=True),
+                layers.quantized_attention(few, k, v, 0.125, causal=True), nv.quantize(x, nv.Quant.affine(64, 4)).weight.view(torch.int32)]
+    want = [work(i) for i in range(4)]
+    torch.cuda.synchronize()
+    wrong = []
+
+    def run(i):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for _ in range(20):
+                got = work(i)
+                stream.synchronize()
+                wrong.extend(i for a, b in zip(got, want[i]) if not torch.equal(a, b))
+    threads = [threading.Thread(target=run, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+
+
 @pytest.mark.parametrize("rows,dims,experts,k", [(1, 2880, 32, 4), (7, 64, 3, 3), (300, 520, 128, 8), (5, 8, 1, 1), (2, 1032, 300, 6)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_router(rows, dims, experts, k, dtype):

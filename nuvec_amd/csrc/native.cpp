@@ -5,9 +5,10 @@
 // the same work is done on the tensors' own C++ objects, a block's layers in one call.
 //
 // Every function takes the plain case alone: operands on the bound device, dense, of one element type, of matching shapes, and
-// layers whose methods are the package's own.
-// Whatever else it meets (and whatever the library refuses) it declines by returning None, before anything is launched, and
-// the caller's Python path, which holds every conversion and the reference's messages, does the call.
+// layers whose methods are the package's own.  Whatever else it meets (and whatever the library refuses) it declines by returning
+// None, and the caller's Python path, which holds every conversion and the reference's messages, does the call.  The operands of
+// every product of a block are looked at before the first is launched; where the library itself refuses a later one, what ran
+// before it has written intermediate tensors that are dropped.
 //
 // The interpreter lock is released while a call allocates and launches, as ctypes and torch's own operators release it.
 #include <torch/csrc/Dtype.h>
@@ -428,7 +429,13 @@ PyObject *py_quantized_matmul(PyObject *, PyObject *const *args, Py_ssize_t n) {
     });
 }
 
-// mlp(block, x, most): layers.Mlp.forward; up to `most` rows of x take the fused gate and up projections.
+// Whether `l` takes rows of `inner` values of `type` (the rest of `product`'s checks is x's).
+bool linear_fits(const Linear &l, const Place &at, at::ScalarType type, int64_t inner) {
+    int64_t columns;
+    return l.p.fits(at, type, 2, columns) && columns == inner && bias_fits(l.bias, at, type, l.p.w.size(0));
+}
+
+// mlp(block, x): layers.Mlp.forward
 PyObject *py_mlp(PyObject *, PyObject *const *args, Py_ssize_t n) {
     return guarded([&]() -> PyObject * {
         Tensor x, hidden, y;
@@ -446,13 +453,16 @@ PyObject *py_mlp(PyObject *, PyObject *const *args, Py_ssize_t n) {
         const int64_t rows = x.numel() / x.size(-1), most = gate.p.q.mode == NVQ_AFFINE ? 2 : 4;  // (layers.Mlp.forward says why)
         const bool one = both.p != Py_None && rows <= most;
         if ((one && !read_linear(both.p, fused)) || !read_linear(args[0], names.up_proj, up)) return none();
+        const Place at(x);
+        const at::ScalarType type = x.scalar_type();
+        if (!linear_fits(gate, at, type, x.size(-1)) || !linear_fits(up, at, type, x.size(-1)) || up.p.w.size(0) != gate.p.w.size(0) ||
+            !linear_fits(down, at, type, gate.p.w.size(0)) || (one && (!linear_fits(fused, at, type, x.size(-1)) || fused.p.w.size(0) != 2 * gate.p.w.size(0))))
+            return none();
         const bool done = unlocked([&] {
             if (one) product_glu(x, fused.p, fused.bias, activation, 0.0f, 0.0f, hidden);
             if (!hidden.defined()) {
                 Tensor g, u;
-                if (!product(x, gate.p, gate.bias, Flags(), g) || !product(x, up.p, up.bias, Flags(), u) || g.sizes() != u.sizes() ||
-                    !gated(g, u, activation, hidden))
-                    return false;
+                if (!product(x, gate.p, gate.bias, Flags(), g) || !product(x, up.p, up.bias, Flags(), u) || !gated(g, u, activation, hidden)) return false;
             }
             return product(hidden, down.p, down.bias, Flags(), y);
         });

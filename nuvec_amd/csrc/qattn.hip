@@ -11,10 +11,13 @@
 // 4 bits in the mantissa of 8 and 16: one instruction per two codes, the 8 or 16 taken out again by the sums it multiplies;
 // in the mantissa of 128 float32 results lost a digit).  The values' sums count codes from the middle of their range, as large
 // as the values around their mean, so that the weights' rounding is not multiplied by the range: the operands themselves in
-// float32, else by an operand of the offset and the middle alone that goes through the same sums.  Errors against float64, from
-// dequantized values -> here: float16 2.08e-4 -> 2.08e-4 (the output's rounding), float32 3.9e-7 .. 5.8e-7 -> 2.0e-7 .. 2.5e-7.
-// What is not exact in bfloat16, the queries of the wider types and the softmax's weights, goes in as the sum of two or three
-// bfloat16 terms (16 or 24 bits): TQ and TP below.
+// float32, else by an operand of the offset and the middle alone that goes through the same sums.
+// What is not exact in bfloat16, the queries of the wider types and the softmax's weights, goes in as the sum of bfloat16 terms of
+// 8 bits each: a float16 query in two, a float32 query and the weights of every type, float32 values, in three (TQ and TP below).
+// Errors against float64, weights and sums in float32 on the vector units as they were -> here: float16 2.01e-4 .. 2.10e-4 -> the
+// same to four digits (the output's rounding; with two terms of the weights a ten-thousandth more), float32 3.6e-7 .. 5.4e-7 ->
+// 1.8e-7 .. 2.8e-7.  The third term costs 3 to 4 % (16 x 8 heads x 8192 positions of 4
+// bits 51.2 -> 53.4 us).
 //
 // Groups.  v_mfma_f32_16x16x32 has 16 columns and a key head at most 8 query heads: the columns are (group of D, query head)
 // with 16 / groups heads each (eight heads over four groups take two blocks).  The query's operand holds zeros outside
@@ -102,16 +105,20 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t (&t)[N]) {
     }
 }
 
+// Blocks on a compute unit: what fits without spilling (float16 queries are two terms, 8-bit keys and values twice the registers).
+template <typename T, int BITS, int G>
+constexpr int attention_blocks() { return sizeof(T) == 4 || G == 4 || (BITS == 8 && Elem<T>::code != 10) ? 2 : 3; }
+
 // G groups of a row.  Block: one (batch, key head, split) and 16 / G of its query heads; its wavefronts take tiles of 32 keys in
 // turn.
 template <typename T, int BITS, int D, int G>
-__global__ void __launch_bounds__(64 * kAttnWaves, sizeof(T) == 2 && G < 4 ? 3 : 2) qattn_kernel(const nvq_attention_desc d, const T *__restrict__ q, const uint32_t *__restrict__ kw,
+__global__ void __launch_bounds__(64 * kAttnWaves, (attention_blocks<T, BITS, G>())) qattn_kernel(const nvq_attention_desc d, const T *__restrict__ q, const uint32_t *__restrict__ kw,
                                                                const T *__restrict__ ks, const T *__restrict__ kb,
                                                                const uint32_t *__restrict__ vw, const T *__restrict__ vs,
                                                                const T *__restrict__ vb, const T *__restrict__ sinks, T *__restrict__ out,
                                                                float *__restrict__ partials) {
     constexpr int TQ = sizeof(T) == 4 ? 3 : Elem<T>::code == 10 ? 1 : 2;  // terms of the queries: exact
-    constexpr int TP = sizeof(T) == 4 ? 3 : 2;                            // terms of the weights: 24 or 16 bits
+    constexpr int TP = 3;                                                 // terms of the weights: 24 bits
     constexpr int R = 16 / G, KS = D / 32, ND = D / 16;  // heads per operand; instructions of K per 16 keys; values of D per lane
     constexpr int kRowBytes = D * BITS / 8, kChunk = kRowBytes / 4, kSlot = BITS * ND;  // bytes of a quarter's codes; bits of a lane's slot
     constexpr bool kWide = sizeof(T) == 4;

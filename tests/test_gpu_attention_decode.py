@@ -1,8 +1,8 @@
 """The decode attention kernel (csrc/qattn.hip) at the edges of its tiles and column layouts against float64 attention over
-the dequantized cache.  Bound, of the largest value: the codes, the float32 queries' three bfloat16 terms and their products
+the dequantized cache.  Bound, of the largest value: the codes, the queries' and the weights' bfloat16 terms and their products
 are exact; the sums are float32 over operands of at most 143 x scale (the scores' of 8 bits 255, with a scale a sixteenth as large), 2^-24 of
-that a rounding, with scale <= 2 max / 15, i.e. 1.1e-6 max, and their roundings are random: sixteen of them.  In the 16-bit types one rounding of the output beside it, and the
-weights' 16 bits (2^-17)."""
+that a rounding, with scale <= 2 max / 15, i.e. 1.1e-6 max, and their roundings are random: sixteen of them.  In the 16-bit types one rounding
+of the output beside it."""
 import pytest
 import torch
 
@@ -34,8 +34,32 @@ def test_edges(heads, key_heads, d, group, bits, dtype):
             scores = torch.cat([scores, sinks.double().view(1, heads, 1).expand(2, heads, 1)], dim=-1)
         want = (torch.softmax(scores, -1)[..., :s, None] * vf).sum(-2, keepdim=True)
         u = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
-        bound = (16 * 1.1e-6 + (0 if dtype == torch.float32 else 2.0 ** -17)) * vf.abs().max() + u * want.abs()
+        bound = 16 * 1.1e-6 * vf.abs().max() + u * want.abs()
         assert ((got.double() - want).abs() <= bound).all(), (s, (got.double() - want).abs().max().item())
+
+
+@pytest.mark.parametrize("batch", [16, 32768])  # (fewer and more positions)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_weights_of_24_bits(dtype, batch):
+    """Two keys whose scores differ by a little, and values of 1 and -1: the output is tanh of half the difference, what is left of
+    weights that nearly cancel.  They come as codes of 1 that are counted from 128 (the kernels' middle of eight bits), so an error of a weight
+    is seen 127-fold: 16 bits of it would show 127 x 2^-18 on average, float32 shows the exponential's and the sums' 2^-24, sixteen of them here."""
+    torch.manual_seed(11)
+    quant, heads, d = nv.Quant.affine(64, 8), 8, 128
+    q = torch.zeros(batch, heads, 1, d, device="cuda")
+    q[..., 0] = torch.rand(batch, heads, 1, device="cuda") * 2.0 ** -6
+    q = q.to(dtype)
+    put = lambda value: torch.full((batch, 1, 2, 2), float(value), device="cuda", dtype=dtype)
+    codes = torch.zeros(batch, 1, 2, d // 4, dtype=torch.int32, device="cuda")
+    codes[:, :, 0, 0] = 1
+    k = nv.Quantized(codes.view(torch.uint32), put(1), put(0), quant)
+    signs = put(1)
+    signs[:, :, 1] = -1
+    v = nv.Quantized(torch.full_like(codes, 0x01010101).view(torch.uint32), signs, put(0), quant)
+    got = ops.quantized_attention(q, k, v, 1.0).double()
+    want = torch.tanh(q[..., :1].double() / 2).expand_as(got)
+    u = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    assert ((got - want).abs() <= u * want.abs() + 16 * 128 * 2.0 ** -24).all(), (got - want).abs().max().item()
 
 
 @pytest.mark.parametrize("splits", [2, 3, 5, 31, 33, 64])

@@ -16,8 +16,11 @@
 // 8 bits each: a float16 query in two, a float32 query and the weights of every type, float32 values, in three (TQ and TP below).
 // Errors against float64, weights and sums in float32 on the vector units as they were -> here: float16 2.01e-4 .. 2.10e-4 -> the
 // same to four digits (the output's rounding; with two terms of the weights a ten-thousandth more), float32 3.6e-7 .. 5.4e-7 ->
-// 1.8e-7 .. 2.8e-7.  The third term costs 3 to 4 % (16 x 8 heads x 8192 positions of 4
+// 1.8e-7 .. 2.8e-7, on the vector kernel below 1.6e-7 .. 2.3e-7.  The third term costs 3 to 4 % (16 x 8 heads x 8192 positions of 4
 // bits 51.2 -> 53.4 us).
+//
+// With few query heads per key head or few positions most of an instruction's columns or of the chip stays empty: those take a
+// vector kernel, one query head a block (vector_is_faster).
 //
 // Groups.  v_mfma_f32_16x16x32 has 16 columns and a key head at most 8 query heads: the columns are (group of D, query head)
 // with 16 / groups heads each (eight heads over four groups take two blocks).  The query's operand holds zeros outside
@@ -412,6 +415,149 @@ __global__ void __launch_bounds__(64 * kAttnWaves, (attention_blocks<T, BITS, G>
     }
 }
 
+// ── one query head of a key head at a time, on the vector units ─────────────────────────────────────────────────────
+// A row of the cache is CH chunks of 32 codes (16 of 8 bits: 16 bytes); lane l of a wavefront takes chunk l % CH of key l / CH of
+// the wavefront's tile of 64 / CH keys, so that its loads read consecutive rows.  The lanes of a key add their partial dot products,
+// every lane keeps the softmax of the keys it has seen and its chunk of the output, and the states of a block meet in LDS.
+template <int BITS> struct Chunk { uint32_t w[BITS == 3 ? 3 : 4]; };
+
+template <int BITS>
+__device__ __forceinline__ Chunk<BITS> load_chunk(const uint32_t *p) {
+    Chunk<BITS> c;
+    if constexpr (BITS == 3) {
+        c.w[0] = p[0], c.w[1] = p[1], c.w[2] = p[2];  // (rows of 3-bit codes are whole dwords: 4-byte aligned)
+    } else {
+        const uint4 v = *reinterpret_cast<const uint4 *>(p);
+        c.w[0] = v.x, c.w[1] = v.y, c.w[2] = v.z, c.w[3] = v.w;
+    }
+    return c;
+}
+
+// Code i of a chunk as a float (i is a constant after unrolling).
+template <int BITS>
+__device__ __forceinline__ float chunk_code(const Chunk<BITS> &c, int i) {
+    if constexpr (BITS == 4) {
+        return (float)((c.w[i >> 3] >> (4 * (i & 7))) & 15u);
+    } else if constexpr (BITS == 8) {
+        return (float)((c.w[i >> 2] >> (8 * (i & 3))) & 255u);
+    } else {
+        const int bit = 3 * i, dw = bit >> 5, sh = bit & 31;
+        const uint32_t v = sh <= 29 ? c.w[dw] >> sh : (c.w[dw] >> sh) | (c.w[dw + 1] << (32 - sh));
+        return (float)(v & 7u);
+    }
+}
+
+template <typename T, int BITS, int D>
+__global__ void __launch_bounds__(64 * kAttnWaves) qattn_vector_kernel(const nvq_attention_desc d, const T *__restrict__ q, const uint32_t *__restrict__ kw,
+                                                                      const T *__restrict__ ks, const T *__restrict__ kb,
+                                                                      const uint32_t *__restrict__ vw, const T *__restrict__ vs,
+                                                                      const T *__restrict__ vb, const T *__restrict__ sinks, T *__restrict__ out,
+                                                                      float *__restrict__ partials) {
+    constexpr int CPL = BITS == 8 ? 16 : 32;  // codes of a lane
+    constexpr int CW = CPL * BITS / 32;       // their dwords
+    constexpr int CH = D / CPL;               // lanes of a key: 2, 4 or 8
+    constexpr int KPT = 64 / CH;              // keys of a wavefront's tile
+    constexpr int kSlots = KPT * kAttnWaves;
+    // float32: sums over codes from the middle of their range, as above; the output's rounding covers the 16-bit types' sums
+    constexpr float kMiddle = sizeof(T) == 4 ? (float)(1 << (BITS - 1)) : 0.0f;
+    __shared__ float part[kSlots][D + 1];
+    __shared__ float slot_m[kSlots], slot_l[kSlots];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int c = lane % CH, j = lane / CH;
+    const int h = blockIdx.x, b = blockIdx.y;
+    const int rep = d.query_heads / d.key_heads, hk = h / rep;
+    const int S = d.positions, groups = D / d.group_size;
+    const int gi = (c * CPL) / d.group_size;  // (a chunk lies inside one group)
+    const int64_t row0 = ((int64_t)b * d.key_heads + hk) * S, head = (int64_t)b * d.query_heads + h;
+    const int splits = gridDim.z, per = attention_split_keys(S, splits);
+    const int s_begin = blockIdx.z * per, s_end = s_begin + per < S ? s_begin + per : S;
+    const float scale = d.scale * kLog2e;
+
+    float qv[CPL], qs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < CPL; i++) qv[i] = Elem<T>::load(q, head * D + c * CPL + i), qs[i & 3] += qv[i];
+    const float qsum = (qs[0] + qs[1]) + (qs[2] + qs[3]);
+    float m = -1.0e30f, l = 0.0f, acc[CPL], accb = 0.0f;
+#pragma unroll
+    for (int i = 0; i < CPL; i++) acc[i] = 0.0f;
+
+    struct Tile {
+        Chunk<BITS> kc, vc;
+        T sk, bk, sv, bv;
+    };
+    auto fetch = [&](int s0) {
+        const int s = s0 + j;
+        const int64_t r = row0 + (s < s_end ? s : S - 1);  // a key past the end reads the last one and is given no weight
+        Tile t;
+        t.kc = load_chunk<BITS>(kw + (r * CH + c) * CW), t.vc = load_chunk<BITS>(vw + (r * CH + c) * CW);
+        t.sk = ks[r * groups + gi], t.bk = kb[r * groups + gi], t.sv = vs[r * groups + gi], t.bv = vb[r * groups + gi];
+        return t;
+    };
+    Tile cur = fetch(s_begin + wave * KPT);
+    for (int s0 = s_begin + wave * KPT; s0 < s_end; s0 += kAttnWaves * KPT) {
+        const Tile nxt = fetch(s0 + kAttnWaves * KPT);  // requested before this one is computed
+        const float sk = Elem<T>::load(&cur.sk, 0), bk = __builtin_fmaf(kMiddle, sk, Elem<T>::load(&cur.bk, 0));
+        const float sv = Elem<T>::load(&cur.sv, 0), bv = __builtin_fmaf(kMiddle, sv, Elem<T>::load(&cur.bv, 0));
+        float dot[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < CPL; i++) dot[i & 3] = __builtin_fmaf(qv[i], chunk_code<BITS>(cur.kc, i) - kMiddle, dot[i & 3]);
+        float score = __builtin_fmaf(sk, (dot[0] + dot[1]) + (dot[2] + dot[3]), bk * qsum);
+#pragma unroll
+        for (int o = 1; o < CH; o <<= 1) score += __shfl_xor(score, o);  // the lanes of a key sit side by side
+        score = s0 + j < s_end ? score * scale : -INFINITY;
+        if (__any(score > m + 8.0f)) {
+            const float m_new = fmaxf(m, score), f = exp2f(m - m_new);
+            m = m_new, l *= f, accb *= f;
+#pragma unroll
+            for (int i = 0; i < CPL; i++) acc[i] *= f;
+        }
+        const float p = __builtin_amdgcn_exp2f(score - m), pv = p * sv;
+        l += p;
+        accb = __builtin_fmaf(p, bv, accb);
+#pragma unroll
+        for (int i = 0; i < CPL; i++) acc[i] = __builtin_fmaf(pv, chunk_code<BITS>(cur.vc, i) - kMiddle, acc[i]);
+        cur = nxt;
+    }
+
+    // merge: the block's maximum, every slot scaled to it, the slots added up by 256 / D groups of threads in four chains each
+    constexpr int kGroups = 64 * kAttnWaves / D;
+    __shared__ float sums[kGroups][D], denoms[kGroups];
+    const int slot = wave * KPT + j;
+    if (c == 0) slot_m[slot] = m;
+    __syncthreads();
+    float top = lane < kSlots ? slot_m[lane] : -1.0e30f;
+    if constexpr (kSlots == 128) top = fmaxf(top, slot_m[lane + 64]);
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) top = fmaxf(top, __shfl_xor(top, o));
+    const float w = exp2f(m - top);
+    if (c == 0) slot_l[slot] = l * w;
+#pragma unroll
+    for (int i = 0; i < CPL; i++) part[slot][c * CPL + i] = (acc[i] + accb) * w;
+    __syncthreads();
+    const int at = tid % D, group = tid / D;
+    float dn[4] = {0.0f, 0.0f, 0.0f, 0.0f}, sm[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int t = group * (kSlots / kGroups); t < (group + 1) * (kSlots / kGroups); t += 4)
+#pragma unroll
+        for (int u = 0; u < 4; u++) dn[u] += slot_l[t + u], sm[u] += part[t + u][at];
+    sums[group][at] = (sm[0] + sm[1]) + (sm[2] + sm[3]);
+    if (at == 0) denoms[group] = (dn[0] + dn[1]) + (dn[2] + dn[3]);
+    __syncthreads();
+    if (group != 0) return;
+    float sum = sums[0][at] + sums[1][at], denom = denoms[0] + denoms[1];
+    if constexpr (kGroups == 4) sum += sums[2][at] + sums[3][at], denom += denoms[2] + denoms[3];
+    if (splits == 1) {
+        if (sinks != nullptr) {
+            const float sink = Elem<T>::load(sinks, h) * kLog2e, t2 = fmaxf(top, sink), f = exp2f(top - t2);
+            sum *= f, denom = denom * f + exp2f(sink - t2);
+        }
+        Elem<T>::store(out, head * D + at, sum / denom);
+    } else {
+        float *dst = partials + (head * splits + blockIdx.z) * (D + 2);
+        if (at == 0) dst[0] = top, dst[1] = denom;
+        dst[2 + at] = sum;
+    }
+}
+
 // The splits of one (batch, head) merged.
 template <typename T, int D>
 __global__ void __launch_bounds__(kMergeParts * D) qattn_merge_kernel(const nvq_attention_desc d, const float *__restrict__ partials, int splits,
@@ -421,79 +567,99 @@ __global__ void __launch_bounds__(kMergeParts * D) qattn_merge_kernel(const nvq_
                                  sinks != nullptr ? Elem<T>::load(sinks, blockIdx.x) * kLog2e : 0.0f, out + head * D);
 }
 
-int attention_splits(const nvq_attention_desc &d);
+struct Plan {
+    bool vector;
+    int splits;  // of the positions over the grid
+};
+Plan attention_plan(const nvq_attention_desc &d);
 
-template <typename T, int BITS, int D, int G>
-int32_t run_attention_grouped(const nvq_attention_desc &d, const void *q, const void *kw, const void *ks, const void *kb, const void *vw,
-                              const void *vs, const void *vb, const void *sinks, void *out, void *workspace, hipStream_t s) {
-    const int splits = workspace != nullptr ? attention_splits(d) : 1;
-    const int64_t parts = (d.query_heads / d.key_heads + 16 / G - 1) / (16 / G);
-    const dim3 grid((unsigned)d.key_heads, (unsigned)d.batch, (unsigned)(splits * parts)), block(64 * kAttnWaves);
-    hipLaunchKernelGGL((qattn_kernel<T, BITS, D, G>), grid, block, 0, s, d, (const T *)q, (const uint32_t *)kw, (const T *)ks, (const T *)kb,
-                       (const uint32_t *)vw, (const T *)vs, (const T *)vb, (const T *)sinks, (T *)out, (float *)workspace);
+struct Operands {
+    const void *q, *kw, *ks, *kb, *vw, *vs, *vb, *sinks;
+    void *out, *workspace;
+};
+
+template <typename T, typename K>
+void start_attention(K kernel, dim3 grid, const nvq_attention_desc &d, const Operands &o, hipStream_t s) {
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * kAttnWaves), 0, s, d, (const T *)o.q, (const uint32_t *)o.kw, (const T *)o.ks, (const T *)o.kb,
+                       (const uint32_t *)o.vw, (const T *)o.vs, (const T *)o.vb, (const T *)o.sinks, (T *)o.out, (float *)o.workspace);
+}
+
+template <typename T, int BITS, int D>
+int32_t run_attention_sized(const nvq_attention_desc &d, const Operands &o, hipStream_t s) {
+    Plan p = attention_plan(d);
+    if (o.workspace == nullptr) p.splits = 1;
+    if (p.vector) {
+        start_attention<T>(qattn_vector_kernel<T, BITS, D>, dim3((unsigned)d.query_heads, (unsigned)d.batch, (unsigned)p.splits), d, o, s);
+    } else {
+        const int groups = D / d.group_size, heads = 16 / groups;  // (groups have 32 values at least)
+        const int64_t parts = (d.query_heads / d.key_heads + heads - 1) / heads;
+        const dim3 grid((unsigned)d.key_heads, (unsigned)d.batch, (unsigned)(p.splits * parts));
+        if (groups == 1) start_attention<T>(qattn_kernel<T, BITS, D, 1>, grid, d, o, s);
+        else if (groups == 2) start_attention<T>(qattn_kernel<T, BITS, D, 2>, grid, d, o, s);
+        else if constexpr (D == 128) start_attention<T>(qattn_kernel<T, BITS, D, 4>, grid, d, o, s);
+    }
     NVQ_LAUNCH_CHECK("quantized_attention");
-    if (splits > 1) {
+    if (p.splits > 1) {
         hipLaunchKernelGGL((qattn_merge_kernel<T, D>), dim3((unsigned)d.query_heads, (unsigned)d.batch), dim3(kMergeParts * D), 0, s, d,
-                           (const float *)workspace, splits, (const T *)sinks, (T *)out);
+                           (const float *)o.workspace, p.splits, (const T *)o.sinks, (T *)o.out);
         NVQ_LAUNCH_CHECK("quantized_attention merge");
     }
     return NVQ_OK;
 }
 
-template <typename T, int BITS, int D>
-int32_t run_attention_sized(const nvq_attention_desc &d, const void *q, const void *kw, const void *ks, const void *kb, const void *vw,
-                            const void *vs, const void *vb, const void *sinks, void *out, void *workspace, hipStream_t s) {
-    const int groups = D / d.group_size;
-    if (groups == 1) return run_attention_grouped<T, BITS, D, 1>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s);
-    if (groups == 2) return run_attention_grouped<T, BITS, D, 2>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s);
-    if constexpr (D == 128)  // (groups have 32 values at least)
-        return run_attention_grouped<T, BITS, D, 4>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s);
-    return NVQ_UNSUPPORTED;
-}
-
 template <typename T, int BITS>
-int32_t run_attention(const nvq_attention_desc &d, const void *q, const void *kw, const void *ks, const void *kb, const void *vw,
-                      const void *vs, const void *vb, const void *sinks, void *out, void *workspace, hipStream_t s) {
-    return d.head_dim == 64 ? run_attention_sized<T, BITS, 64>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s)
-                            : run_attention_sized<T, BITS, 128>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s);
+int32_t run_attention(const nvq_attention_desc &d, const Operands &o, hipStream_t s) {
+    return d.head_dim == 64 ? run_attention_sized<T, BITS, 64>(d, o, s) : run_attention_sized<T, BITS, 128>(d, o, s);
 }
 
 template <typename T>
-int32_t run_attention_bits(const nvq_attention_desc &d, const void *q, const void *kw, const void *ks, const void *kb, const void *vw,
-                           const void *vs, const void *vb, const void *sinks, void *out, void *workspace, hipStream_t s) {
-    return d.bits == 4   ? run_attention<T, 4>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s)
-           : d.bits == 3 ? run_attention<T, 3>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s)
-                         : run_attention<T, 8>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s);
+int32_t run_attention_bits(const nvq_attention_desc &d, const Operands &o, hipStream_t s) {
+    return d.bits == 4 ? run_attention<T, 4>(d, o, s) : d.bits == 3 ? run_attention<T, 3>(d, o, s) : run_attention<T, 8>(d, o, s);
 }
 
-// Splits of the positions over the grid: three blocks of four wavefronts per compute unit (what the kernels' registers let
-// run together), at least two tiles a wavefront, at most 64 splits.
-int attention_splits(const nvq_attention_desc &d) {
-    const int64_t heads = d.batch * d.key_heads;
-    if (heads <= 0) return 1;
-    int64_t want = 3 * (int64_t)compute_units() / heads;
+// Both kernels as timed on 592 calls (1 to 8 query heads per key head, 128 to 20000 positions, batches of 1 to 32, 3, 4 and 8 bits in
+// groups of 32 and 64, head sizes 64 and 128, the three types): the vector kernel's time grows with the query heads, the other's
+// with the key heads (times the blocks that share one), and the vector kernel starts sooner.  Per thousand positions of a head
+// of 128 values it takes 0.0245 us a query head (0.035 with 8 bits), the matrix cores 0.064 (0.047 in float32).  Choosing by them
+// is 0.3 % above always taking the faster kernel, 1.25 x at worst.  us, vector / matrix cores, 16 x 8 key heads x 8192 positions,
+// bfloat16, 4-bit groups of 64: one query head 40 / 60, two 71 / 58, four 116 / 56; 32 x 4 x 300: 7.4 / 10.6, 8 / 10.8, 10 / 11.1.
+bool vector_is_faster(const nvq_attention_desc &d) {
+    const double rep = (double)d.query_heads / (double)d.key_heads, parts = ceil(rep * (double)d.head_dim / (16.0 * d.group_size));
+    const double positions = (double)d.batch * (double)d.key_heads * (double)d.positions * (double)d.head_dim / 128.0e3;
+    return (d.bits == 8 ? 0.035 : 0.0245) * rep * positions < (d.bits == 8 ? 3.0 : 1.5) + (d.dtype == NVQ_F32 ? 0.047 : 0.064) * parts * positions;
+}
+
+// Splits of the positions over the grid, at most 64 (a lane each when they are merged).  Matrix cores: three blocks of four
+// wavefronts per compute unit, at least two tiles a wavefront; vector: two blocks, at least 256 keys.
+Plan attention_plan(const nvq_attention_desc &d) {
+    Plan p{vector_is_faster(d), 1};
+    const int64_t heads = d.batch * (p.vector ? d.query_heads : d.key_heads), units = compute_units();
+    if (heads <= 0 || (p.vector && d.positions < 512)) return p;
+    int64_t want = p.vector ? (2 * units + heads - 1) / heads : 3 * units / heads;
     const int64_t most = d.positions / (2 * kAttnWaves * kTileKeys);
     want = want > most ? most : want;
-    want = want > 64 ? 64 : want;  // (a lane each when they are merged)
-    if (want < 2) return 1;
+    want = want > 64 ? 64 : want;
+    if (want < 2) return p;
     const int per = attention_split_keys(d.positions, (int)want);  // whole tiles: fewer splits may cover the positions
-    return (int)((d.positions + per - 1) / per);
+    p.splits = (int)((d.positions + per - 1) / per);
+    return p;
 }
 
 }  // namespace
 
 size_t attention_workspace_bytes(const nvq_attention_desc &d) {
-    const int splits = attention_splits(d);
+    const int splits = attention_plan(d).splits;
     return splits > 1 ? (size_t)d.batch * (size_t)d.query_heads * (size_t)splits * (size_t)(d.head_dim + 2) * sizeof(float) : 0;
 }
 
 int32_t launch_quantized_attention(const nvq_attention_desc &d, const void *q, const void *kw, const void *ks, const void *kb,
                                    const void *vw, const void *vs, const void *vb, const void *sinks, void *out, void *workspace,
                                    hipStream_t s) {
+    const Operands o{q, kw, ks, kb, vw, vs, vb, sinks, out, workspace};
     switch (d.dtype) {
-    case NVQ_F32: return run_attention_bits<float>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s);
-    case NVQ_BF16: return run_attention_bits<bf16_t>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s);
-    default: return run_attention_bits<f16_t>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s);
+    case NVQ_F32: return run_attention_bits<float>(d, o, s);
+    case NVQ_BF16: return run_attention_bits<bf16_t>(d, o, s);
+    default: return run_attention_bits<f16_t>(d, o, s);
     }
 }
 

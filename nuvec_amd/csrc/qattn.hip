@@ -108,14 +108,20 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t (&t)[N]) {
     }
 }
 
-// Blocks on a compute unit: what fits without spilling (float16 queries are two terms, 8-bit keys and values twice the registers).
-template <typename T, int BITS, int G>
-constexpr int attention_blocks() { return sizeof(T) == 4 || G == 4 || (BITS == 8 && Elem<T>::code != 10) ? 2 : 3; }
+// Blocks on a compute unit.  Three need 168 registers at most: there the queries of what would spill (float16's two terms, 8-bit
+// codes: 6 to 35 registers) are read from LDS in every tile (16 x 8 heads x 8192 positions in groups of 64: float16 of 4 bits 62 ->
+// 57 us, of 8 bits, at two blocks before, 88 -> 66, bfloat16 of 8 bits 77 -> 68).
+template <typename T, int G> constexpr int attention_blocks() { return sizeof(T) == 4 || G == 4 ? 2 : 3; }
+template <typename T, int BITS, int D, int G>
+constexpr bool queries_in_lds() {
+    constexpr bool f16 = Elem<T>::code != 10;
+    return attention_blocks<T, G>() == 3 && D == 128 && (G == 2 ? BITS == 8 || f16 : BITS == 8 && f16);
+}
 
 // G groups of a row.  Block: one (batch, key head, split) and 16 / G of its query heads; its wavefronts take tiles of 32 keys in
 // turn.
 template <typename T, int BITS, int D, int G>
-__global__ void __launch_bounds__(64 * kAttnWaves, (attention_blocks<T, BITS, G>())) qattn_kernel(const nvq_attention_desc d, const T *__restrict__ q, const uint32_t *__restrict__ kw,
+__global__ void __launch_bounds__(64 * kAttnWaves, (attention_blocks<T, G>())) qattn_kernel(const nvq_attention_desc d, const T *__restrict__ q, const uint32_t *__restrict__ kw,
                                                                const T *__restrict__ ks, const T *__restrict__ kb,
                                                                const uint32_t *__restrict__ vw, const T *__restrict__ vs,
                                                                const T *__restrict__ vb, const T *__restrict__ sinks, T *__restrict__ out,
@@ -146,6 +152,8 @@ __global__ void __launch_bounds__(64 * kAttnWaves, (attention_blocks<T, BITS, G>
 
     // The queries' operands: column (g, head), zeros outside the group; their sums per column.
     const int head = l % R;
+    constexpr bool kLdsQueries = queries_in_lds<T, BITS, D, G>();
+    __shared__ uint4 queries[kLdsQueries ? KS * TQ : 1][64];  // (the same in all wavefronts)
     uint4 qf[KS][TQ];
     float qsum = 0.0f;
 #pragma unroll
@@ -161,8 +169,12 @@ __global__ void __launch_bounds__(64 * kAttnWaves, (attention_blocks<T, BITS, G>
 #pragma unroll
         for (int j = 0; j < 4; j++) split_pair<TQ>(v[2 * j], v[2 * j + 1], t[j]);
 #pragma unroll
-        for (int i = 0; i < TQ; i++) qf[s][i] = make_uint4(t[0][i], t[1][i], t[2][i], t[3][i]);
+        for (int i = 0; i < TQ; i++) {
+            qf[s][i] = make_uint4(t[0][i], t[1][i], t[2][i], t[3][i]);
+            if (kLdsQueries && wave == 0) queries[s * TQ + i][lane] = qf[s][i];
+        }
     }
+    if (kLdsQueries) __syncthreads();
     qsum += __shfl_xor(qsum, 16);
     qsum += __shfl_xor(qsum, 32);
 
@@ -281,6 +293,13 @@ __global__ void __launch_bounds__(64 * kAttnWaves, (attention_blocks<T, BITS, G>
     fetch_values(s_begin + wave * kTileKeys);
     for (int s0 = s_begin + wave * kTileKeys; s0 < s_end; s0 += kAttnWaves * kTileKeys) {
         float score[8];
+        if constexpr (kLdsQueries) {
+            asm volatile("" ::: "memory");  // (not kept from the tile before)
+#pragma unroll
+            for (int s = 0; s < KS; s++)
+#pragma unroll
+                for (int i = 0; i < TQ; i++) qf[s][i] = queries[s * TQ + i][lane];
+        }
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             floatx4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -620,13 +639,13 @@ int32_t run_attention_bits(const nvq_attention_desc &d, const Operands &o, hipSt
 // Both kernels as timed on 592 calls (1 to 8 query heads per key head, 128 to 20000 positions, batches of 1 to 32, 3, 4 and 8 bits in
 // groups of 32 and 64, head sizes 64 and 128, the three types): the vector kernel's time grows with the query heads, the other's
 // with the key heads (times the blocks that share one), and the vector kernel starts sooner.  Per thousand positions of a head
-// of 128 values it takes 0.0245 us a query head (0.035 with 8 bits), the matrix cores 0.064 (0.047 in float32).  Choosing by them
-// is 0.3 % above always taking the faster kernel, 1.25 x at worst.  us, vector / matrix cores, 16 x 8 key heads x 8192 positions,
+// of 128 values it takes 0.0245 us a query head (0.033 with 8 bits), the matrix cores 0.060 (0.047 in float32).  Choosing by them
+// is 0.4 % above always taking the faster kernel, 1.28 x at worst.  us, vector / matrix cores, 16 x 8 key heads x 8192 positions,
 // bfloat16, 4-bit groups of 64: one query head 40 / 60, two 71 / 58, four 116 / 56; 32 x 4 x 300: 7.4 / 10.6, 8 / 10.8, 10 / 11.1.
 bool vector_is_faster(const nvq_attention_desc &d) {
     const double rep = (double)d.query_heads / (double)d.key_heads, parts = ceil(rep * (double)d.head_dim / (16.0 * d.group_size));
     const double positions = (double)d.batch * (double)d.key_heads * (double)d.positions * (double)d.head_dim / 128.0e3;
-    return (d.bits == 8 ? 0.035 : 0.0245) * rep * positions < (d.bits == 8 ? 3.0 : 1.5) + (d.dtype == NVQ_F32 ? 0.047 : 0.064) * parts * positions;
+    return (d.bits == 8 ? 0.033 : 0.0245) * rep * positions < (d.bits == 8 ? 3.0 : 1.5) + (d.dtype == NVQ_F32 ? 0.047 : 0.060) * parts * positions;
 }
 
 // Splits of the positions over the grid, at most 64 (a lane each when they are merged).  Matrix cores: three blocks of four

@@ -131,12 +131,18 @@ __global__ void __launch_bounds__(64 * kWaves, MT <= 3 ? 4 : 2) qmf_f32_kernel(c
 int64_t row_tiles(const ProductArgs &a) { return (a.m + kTile - 1) / kTile; }
 int64_t row_passes(const ProductArgs &a) { return (row_tiles(a) + 3) / 4; }
 
+// Wavefronts of a tile, a power of two: sixteen a compute unit (what the registers let run together) where the tiles alone are fewer.
+int tile_waves_shift(const ProductArgs &a) {
+    const int64_t tiles = (a.n + kTile - 1) / kTile * row_passes(a);
+    int shift = 0;
+    while (shift < 3 && (tiles << shift) < 16 * (int64_t)compute_units() && (2 << shift) <= a.k / kWindow) shift++;
+    return shift;
+}
+
 template <int BITS, int MODE = NVQ_AFFINE>
 int32_t run(const ProductArgs &a, hipStream_t s) {
-    const int64_t passes = row_passes(a), tiles = (a.n + kTile - 1) / kTile;
-    // wavefronts of a tile: sixteen a compute unit (what the registers let run together) where the tiles alone are fewer
-    int shift = 0;
-    while (shift < 3 && ((tiles * passes) << shift) < 16 * (int64_t)compute_units() && (2 << shift) <= a.k / kWindow) shift++;
+    const int64_t passes = row_passes(a);
+    const int shift = tile_waves_shift(a);
     const int64_t cols = kTile * (kWaves >> shift);
     const dim3 grid((unsigned)((a.n + cols - 1) / cols), (unsigned)passes), block(64 * kWaves);
     switch ((row_tiles(a) + passes - 1) / passes) {
@@ -158,25 +164,38 @@ bool qmf_f32_supported(const ProductArgs &a) {
     return a.k >= kWindow && a.k % kWindow == 0 && row_passes(a) <= 65535 && a.n <= 0x7FFFFFFF / 64;
 }
 
-// Where it is estimated faster than both other float32 kernels.  A window costs a block that holds a compute unit
-// 0.12 us and 0.05 us per tile of rows (measured 0.17 / 0.20 / 0.26 us for one to three tiles, on W[4096,4096] to
-// W[14336,4096], W[62208,512] and W[1024,8192] alike), whether the chip is full or not; the others as qmm_f32_takes
-// has them.  Left to the tiles: many rows and many weight rows (W[14336,4096] at 33 rows 119 us here, 106 there, W[62208,512]
-// 66 / 45); to the vector kernel: few weight rows (W[1024,8192] at 33 rows 63 / 41) and up to 32 rows of matrices up to
-// W[4096,4096].  More than 128 rows were not timed.
+// Where it is estimated faster than the kernel that takes the product otherwise (qmm_f32_takes says which).  All three were timed on
+// 2486 products (18 weight shapes from W[2000,1920] to W[100000,1024] and W[4096,14336], 11 formats, 2 to 128 rows, weights from
+// memory).  A window costs a tile that a block's eight wavefronts share `window` us and `tile` us per tile of rows, four tiles `four` us
+// in all, and a compute unit its blocks one after the other; where they do not divide evenly the time lies between the average and the
+// fullest unit's (8.7 to 13 % off on average).  The others' estimates are those of qmm_f32_takes times a factor per kind of code: the
+// vector kernel takes E2M1 codes twice as long, E4M3 codes no longer than affine ones, and one pass over the weights for two to
+// four rows.  Choosing by them is 0.3 to 0.8 % above always taking the faster kernel; of 3431 products timed with the rule, 945 of them of
+// other shapes, 14 take more than 5 % longer than without this kernel, 1.10 x at worst, and all together 0.71 of the time (by one
+// factor for all block formats, fitted to eight rows and more, MXFP8 W[1024,8192] at 48 rows took 74 us for 49, W[100000,1024] at 4 rows
+// 114 for 86).  Left to the vector kernel, us there / here: W[14336,4096] at 2 rows
+// 30 / 59, W[4096,14336] at 7 rows 60 / 75; taken: W[62208,512] at 2 rows 61 / 32, W[33000,544] at 4 rows 36 / 18, MXFP4 W[14336,4096]
+// at 5 rows 105 / 47.  Up to 32 rows of matrices up to W[4096,4096] stay on the vector kernel, more than 128 rows on the tiles: the
+// kernel was not timed there.
 bool qmf_f32_takes(const ProductArgs &a) {
     if (!qmf_f32_supported(a) || a.m < 2 || a.m > 128) return false;
     if (a.m <= 32 && a.n * a.k <= 4096LL * 4096) return false;
-    const bool block_format = a.mode != NVQ_AFFINE;
-    const double passes = (double)row_passes(a), tiles = ceil((double)row_tiles(a) / passes), cus = compute_units();
-    const double blocks = fmax(1.0, (double)((a.n + kTile - 1) / kTile) * passes / cus);
-    const double here = 2.5 + blocks * (double)(a.k / kWindow) * (0.12 + 0.05 * tiles);
+    struct Fit { double window, tile, four, vector, tiles; };
+    const Fit fit = a.mode == NVQ_MXFP8          ? Fit{0.046, 0.072, 0.346, 1.06, 1.34}
+                    : a.mode != NVQ_AFFINE       ? Fit{0.038, 0.059, 0.294, 2.52, 1.50}
+                    : a.bits == 3 || a.bits == 8 ? Fit{0.090, 0.064, 0.361, 1.04, 0.92}
+                                                 : Fit{0.065, 0.064, 0.336, 1.04, 0.92};
+    const double rows = ceil((double)row_tiles(a) / (double)row_passes(a)), units = compute_units();
+    const int64_t tiles = kWaves >> tile_waves_shift(a);  // of a block
+    const double blocks = (double)((a.n + kTile * tiles - 1) / (kTile * tiles)) * (double)row_passes(a) / units;
+    const double shared = fmax(1.0, (0.6 * ceil(blocks) + 0.4 * blocks) * (double)tiles);
+    const double here = 2.5 + shared * (double)(a.k / kWindow) * (rows > 3.0 ? fit.four : fit.window + fit.tile * rows);
+    if (qmm_f32_takes(a)) {
+        const double tiles64 = (double)((a.m + 63) / 64) * (double)((a.n + 63) / 64);
+        return here < fit.tiles * (double)(a.k / 64) * fmax(1.64, 1.25 * tiles64 / units);
+    }
     const double k_steps = (double)((a.k + 2047) / 2048) * 2048.0;
-    const double vector = (double)((a.m + 3) / 4) * (double)a.n * k_steps / 2.2e6 * (block_format ? 2.05 : 1.07);
-    if (here >= 0.95 * vector) return false;
-    if (a.m < 8 || a.k % 64 != 0) return true;
-    const double tiles64 = (double)((a.m + 63) / 64) * (double)((a.n + 63) / 64);
-    return here < 0.95 * (double)(a.k / 64) * fmax(1.64, 1.25 * tiles64 / cus) * (block_format ? 1.7 : 1.0);
+    return here < fit.vector * (double)((a.m + 3) / 4) * (double)a.n * k_steps / 2.2e6;
 }
 
 int32_t launch_qmf_f32(const ProductArgs &a, hipStream_t s) {

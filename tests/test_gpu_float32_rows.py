@@ -72,6 +72,18 @@ def test_routes_and_what_stays_on_the_vector_kernel():
     assert ops.quantized_matmul_route(4, 4096, 4096, nv.Quant.new(nv.QuantMode.MXFP4), torch.float32) == "qmv_lds_kernel"
 
 
+@pytest.mark.parametrize("fmt", [(64, 4), (128, 2), (32, 3), (32, 8), "MXFP8"], ids=str)
+def test_few_rows_that_one_pass_serves(fmt):
+    """Two to four rows of a long K are one pass of the vector kernel over the weights, which the tiles of sixteen rows lose to by up to
+    twice; E4M3 codes cost that kernel what affine ones do.  Short rows of K and E2M1 codes gain from the tiles at two rows already."""
+    quant = nv.Quant.new(getattr(nv.QuantMode, fmt)) if isinstance(fmt, str) else nv.Quant.affine(*fmt)
+    route = lambda m, n, k, q=quant: ops.quantized_matmul_route(m, n, k, q, torch.float32)
+    for m in (2, 3, 4):
+        for n, k in ((14336, 4096), (4096, 14336), (100000, 1024), (9000, 6144)):
+            assert route(m, n, k) == "qmv_lds_kernel", (m, n, k)
+        assert route(m, 62208, 512) == "qmm_f32_kernel" and route(m, 14336, 4096, nv.Quant.new(nv.QuantMode.MXFP4)) == "qmm_f32_kernel"
+
+
 def test_bias_epilogue_determinism_and_the_vector_kernel():
     """QuantizedLinear's bias in the epilogue is the separate addition bit for bit (crates/nuvec-nn/src/layers.rs:155-162);
     two launches give the same bits; and the rows agree with the vector kernel's (the row-exact product of the same

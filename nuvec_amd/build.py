@@ -39,6 +39,20 @@ def _hipcc() -> str:
     raise RuntimeError("hipcc not found")
 
 
+def _link(cmd, target: str, what: str) -> None:
+    """Runs `cmd`, which ends in `-o`, into a name of this process beside `target` and puts the whole file there: processes that find
+    the library missing and build it together load either a complete one or none."""
+    part = f"{target}.{os.getpid()}"
+    try:
+        proc = subprocess.run([*cmd, part], capture_output=True, text=True)
+        if proc.returncode != 0:
+            raise RuntimeError(f"{what}:\n{proc.stdout}\n{proc.stderr}")
+        os.replace(part, target)
+    finally:
+        if os.path.exists(part):
+            os.remove(part)
+
+
 def build(verbose: bool = False, jobs: int = 8, changed_only: bool = False) -> str:
     """Compiles every source and links the library.  `changed_only` (a development aid, `--changed` on the command line):
     sources older than their object files are not compiled again, unless a header is newer than the object."""
@@ -67,10 +81,7 @@ def build(verbose: bool = False, jobs: int = 8, changed_only: bool = False) -> s
 
     with ThreadPoolExecutor(max_workers=jobs) as pool:
         objs = list(pool.map(compile_one, SOURCES))
-    cmd = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs]
-    proc = subprocess.run(cmd, capture_output=True, text=True)
-    if proc.returncode != 0:
-        raise RuntimeError(f"link failed:\n{proc.stdout}\n{proc.stderr}")
+    _link([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o"], LIB, "link failed")
     build_native(verbose)
     return LIB
 
@@ -83,13 +94,11 @@ def build_native(verbose: bool = False) -> str:
     root = os.path.dirname(torch.__file__)
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            f"-I{root}/include", "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}", f"-I{INCLUDE}",
-           os.path.join(CSRC, "native.cpp"), "-o", NATIVE, f"-L{root}/lib", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip",
-           "-ltorch_python", f"-L{HERE}", "-l:libnuvec_hip.so", "-Wl,-rpath,$ORIGIN"]
+           os.path.join(CSRC, "native.cpp"), f"-L{root}/lib", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip",
+           "-ltorch_python", f"-L{HERE}", "-l:libnuvec_hip.so", "-Wl,-rpath,$ORIGIN", "-o"]
     if verbose:
-        print(" ".join(cmd), flush=True)
-    proc = subprocess.run(cmd, capture_output=True, text=True)
-    if proc.returncode != 0:
-        raise RuntimeError(f"g++ failed on native.cpp:\n{proc.stdout}\n{proc.stderr}")
+        print(" ".join([*cmd, NATIVE]), flush=True)
+    _link(cmd, NATIVE, "g++ failed on native.cpp")
     return NATIVE
 
 

@@ -743,12 +743,11 @@ int32_t nvq_quantized_matmul_static(const nvq_qmm_desc *d, const void *x, const 
                                     void *y, void *stream) {
     NVQ_TRY(check_qmm(d, "quantized_matmul"));
     const size_t need = workspace_bytes(d, false);  // 0 without a device: the launch below says so
-    const bool fits = need <= (size_t)NVQ_STATIC_SCRATCH_BYTES;
-    if (!fits && (!d->transpose || d->k % 64 == 0))  // (the tiles take K off whole steps of 64 without a split)
+    if (need > (size_t)NVQ_STATIC_SCRATCH_BYTES)
         return fail(NVQ_UNSUPPORTED, "quantized_matmul: this product splits K through %zu bytes of partial sums; the static scratch holds %d",
                     need, NVQ_STATIC_SCRATCH_BYTES);
     void *workspace = nullptr;
-    if (need > 0 && fits) {
+    if (need > 0) {
         NVQ_TRY(require_device());
         workspace = g_scratch[g_device.device.load(std::memory_order_relaxed)];
     }

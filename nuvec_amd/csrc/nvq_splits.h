@@ -12,6 +12,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "nuvec_hip.h"  // NVQ_STATIC_SCRATCH_BYTES
+
 namespace nvq {
 namespace splits {
 
@@ -59,7 +61,9 @@ inline bool qmm_small_tile_is_faster(const Product &a, int cus) {
 
 // The splits fill the chip's block slots with its (few) tiles, and cost a second kernel that reads their float32
 // partial sums (about 3 us to launch and 4 bytes per microsecond and compute unit... in all: 4 TB/s).  Each split has
-// at least eight steps, in whole table periods (four steps); at most eight splits; a batch is never split.
+// at least eight steps, in whole table periods (four steps); at most eight splits; a batch is never split.  K of steps and a half
+// is split as far as the library's own scratch holds the partial sums: the entry point without a workspace takes every such product
+// and gives the bits of the one with a workspace (K of whole steps beyond that scratch it refuses).
 inline Plan qmm_plan(const Product &a, int cus) {
     const int64_t steps = (a.k + kQmmStep - 1) / kQmmStep;  // (the last one may be a half)
     const bool small = qmm_small_tile_is_faster(a, cus);
@@ -71,6 +75,7 @@ inline Plan qmm_plan(const Product &a, int cus) {
         const int64_t per = (((steps + want - 1) / want) + 3) & ~(int64_t)3;  // whole table periods
         const int splits = (int)((steps + per - 1) / per);                    // every split has a step
         if (splits < 2) continue;
+        if (a.k % kQmmStep != 0 && (double)splits * (double)a.m * (double)a.n * 4.0 > (double)NVQ_STATIC_SCRATCH_BYTES) continue;
         const double reduce_us = 3.0 + ((double)splits * 4.0 + 2.0) * (double)a.m * (double)a.n * 2.0 / 4.0e6;  // written, then read
         const double us = qmm_tiles_us(small, tiles * splits, (double)per, cus) + reduce_us;
         if (us < 0.9 * p.estimate_us) p.estimate_us = us, p.splits = splits, p.per_split = per;

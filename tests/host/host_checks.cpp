@@ -81,6 +81,13 @@ int main() {
                 EXPECT(r.splits <= 64, "qmn: %d splits", r.splits);
             }
         }
+        for (int64_t k : steps64) {  // steps and a half: the partial sums fit the library's own scratch, so that no call is refused
+            a.k = k + 32;
+            const Plan q = nvq::splits::qmm_plan(a, cus);
+            check_plan("qmm", q, a, cus, false);
+            EXPECT(nvq::splits::workspace_bytes(q, a) <= (size_t)NVQ_STATIC_SCRATCH_BYTES, "qmm m=%lld n=%lld k=%lld cus=%d: %zu bytes of partial sums",
+                   (long long)m, (long long)n, (long long)a.k, cus, nvq::splits::workspace_bytes(q, a));
+        }
         for (int64_t k : any_k) {
             a.k = k;
             const Plan v = nvq::splits::qvm_plan(a, cus);

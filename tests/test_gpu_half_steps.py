@@ -91,6 +91,25 @@ def test_rows_on_weights_of_two_terms(bits, dtype, m, n, k):
     assert_two_terms(nv.quantized_matmul(x, q).cpu(), x.cpu(), q, ref.F16 if dtype == torch.float16 else ref.BF16, k)
 
 
+@pytest.mark.parametrize("fmt,dtype,m,n,k", [((32, 3), torch.bfloat16, 40, 256, 4128), ((32, 8), torch.float16, 90, 700, 8224), ("MXFP4", torch.bfloat16, 64, 1030, 6176)], ids=str)
+def test_without_a_workspace(fmt, dtype, m, n, k):
+    """`nvq_quantized_matmul_static` splits K as the call with a workspace does: the same bits."""
+    import ctypes as C
+
+    from nuvec_amd import _lib
+    torch.manual_seed(k)
+    quant = nv.Quant.new(getattr(nv.QuantMode, fmt)) if isinstance(fmt, str) else nv.Quant.affine(*fmt)
+    q = nv.quantize((torch.randn(n, k, device="cuda") * 0.02).to(dtype), quant)
+    x = torch.randn(m, k, device="cuda").to(dtype)
+    want, got = nv.quantized_matmul(x, q), torch.empty(m, n, dtype=dtype, device="cuda")
+    d = _lib.QmmDescC()
+    d.quant, d.dtype, d.transpose, d.m, d.n, d.k = q.quant._c(), ops._CODE[dtype], 1, m, n, k
+    assert _lib.load().nvq_quantized_matmul_workspace_bytes(C.byref(d)) > 0  # (K is split)
+    p = ops._ptr
+    _lib.check(_lib.load().nvq_quantized_matmul_static(C.byref(d), p(x), p(q.weight), p(q.scales), p(q.biases), p(got), ops._stream()))
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("k", [160, 224])
 def test_an_infinity_among_the_repeated_values(k):
     """x holds one infinity where the last step starts early: every output is that infinity times a weight's sign, none is NaN."""

@@ -34,19 +34,49 @@ constexpr int kXStageBytes = kPassRows * 256;  // one window of x: 64 rows x 128
 constexpr int kTableMaxBytes = 48 * 1024;  // three blocks on a compute unit
 constexpr int kLdsMost = 160 * 1024;       // of a block off whole steps of K, whose long rows would else go four at a time
 
-// Piece KK of a lane's 32 affine codes as weights of twice the element type's precision: v = hi + lo.  (The range of hi is the
-// finite one, so that a large or infinite v is lo's.)
+// Affine weights in float32 as terms of the element type.  With scale and bias in that type, v = code * scale + bias is a whole
+// multiple of the lower one's last place, and with L bits of significand (8, 11) and their exponents close enough two terms hold it: the
+// rest after one lies within 2^(E(v) - L), and its multiples fit L bits where E(v) - min(E(scale), E(bias)) <= L + 1.  float16 holds no
+// multiple finer than 2^-24, so that any |v| below a half is two terms too.  Codes of `quantize` keep that by far (the bias is the
+// end of the range farther from zero): two matrix instructions, the small term first.  Where some lane's 32 weights do not, a third
+// instruction brings what is left of v's 24 bits.  (The range of the first term is the finite one, so that a large or infinite v is
+// the second's; nothing is left then.)
+template <typename T, int BITS>
+__device__ __forceinline__ bool two_terms_hold(float s, float b) {
+    constexpr bool bf16 = Elem<T>::code == NVQ_BF16;
+    auto exponent = [](float v) { return max((int)(f2u(v) >> 23 & 255u), 1); };
+    const float top = fmaxf(fabsf(b), fabsf(__builtin_fmaf((float)((1 << BITS) - 1), s, b)));
+    const int high = exponent(top), low = min(s != 0.0f ? exponent(s) : 255, b != 0.0f ? exponent(b) : 255);
+    if constexpr (bf16) return high - low <= 9;
+    else return top <= 65504.0f && (high - low <= 12 || high <= 125);
+}
+
+// Piece KK of a lane's 32 affine codes as two terms.
 template <typename T, int BITS, int KK>
-__device__ __forceinline__ void expand_split(const uint32_t (&dw)[BITS], float s, float b, uint4 &hi, uint4 &lo) {
+__device__ __forceinline__ void expand_terms(const uint32_t (&dw)[BITS], float s, float b, uint4 &hi, uint4 &lo) {
     constexpr float most = Elem<T>::code == NVQ_BF16 ? 3.38953139e38f : 65504.0f;
     uint32_t h[4], l[4];
     static_for<4>([&](auto i_tag) {
         constexpr int i = decltype(i_tag)::value, J = 8 * KK + 2 * i;
         const float v0 = __builtin_fmaf(code_to_float<BITS, J>(dw), s, b), v1 = __builtin_fmaf(code_to_float<BITS, J + 1>(dw), s, b);
         h[i] = Ops<T>::pack(__builtin_amdgcn_fmed3f(v0, -most, most), __builtin_amdgcn_fmed3f(v1, -most, most));
-        l[i] = Ops<T>::pack(v0 - half_lo<T>(h[i]), v1 - half_lo<T>(h[i] >> 16));
+        l[i] = Ops<T>::pack(v0 - half_lo<T>(h[i]), v1 - half_hi<T>(h[i]));
     });
     hi = make_uint4(h[0], h[1], h[2], h[3]), lo = make_uint4(l[0], l[1], l[2], l[3]);
+}
+
+// What two finite terms leave of them, exactly.
+template <typename T, int BITS, int KK>
+__device__ __forceinline__ uint4 left_over(const uint32_t (&dw)[BITS], float s, float b, uint4 hi, uint4 lo) {
+    const uint32_t h[4] = {hi.x, hi.y, hi.z, hi.w}, l[4] = {lo.x, lo.y, lo.z, lo.w};
+    uint32_t t[4];
+    static_for<4>([&](auto i_tag) {
+        constexpr int i = decltype(i_tag)::value, J = 8 * KK + 2 * i;
+        const float v0 = __builtin_fmaf(code_to_float<BITS, J>(dw), s, b), v1 = __builtin_fmaf(code_to_float<BITS, J + 1>(dw), s, b);
+        const float r0 = v0 - half_lo<T>(h[i]) - half_lo<T>(l[i]), r1 = v1 - half_hi<T>(h[i]) - half_hi<T>(l[i]);
+        t[i] = Ops<T>::pack(fabsf(r0) < INFINITY ? r0 : 0.0f, fabsf(r1) < INFINITY ? r1 : 0.0f);
+    });
+    return make_uint4(t[0], t[1], t[2], t[3]);
 }
 
 template <int BITS>
@@ -61,6 +91,8 @@ struct Geometry {
     __host__ __device__ static constexpr int swizzle(int row) { return kPow2 ? (row / (BITS >= 16 ? 1 : 16 / BITS)) % BITS : 0; }
 };
 
+__host__ __device__ constexpr bool weights_in_terms(int fp4, bool exact, bool ragged) { return ragged && fp4 == kAffine && !exact; }
+
 // GLU: the gated activation of the experts' MLPs as the epilogue (a.glu).  The weights then hold the gate and the up
 // projection in alternating runs of 64 rows, so that a block's wavefronts 0 and 1 own 64 columns of the gate product
 // and wavefronts 2 and 3 the same 64 columns of the up product, lane for lane: after a pass the latter leave their
@@ -72,12 +104,14 @@ struct Geometry {
 // against 190).
 template <typename T, int BITS, int FP4, bool GLU, bool EXACT, bool RAGGED>
 // Three blocks per compute unit (three wavefronts per SIMD): the registers are capped for that, and the LDS of a
-// block (two x stages, the weight stages, the table) fits three times.
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) qmg_kernel(const ProductArgs a) {
+// block (two x stages, the weight stages, the table) fits three times.  Two with weights in terms, whose operands spilled 21 to 70
+// registers at three while a long row's table leaves room for one or two blocks anyway (300 rows, W[8300,3104] in groups of 32, 8 bits
+// 169 -> 125 us, 4 bits the same; 600 rows, W[9000,480] of 4 bits 32 -> 36; the look for a third term costs 3 % of it).
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(weights_in_terms(FP4, EXACT, RAGGED) ? 2 : 3))) qmg_kernel(const ProductArgs a) {
     using G = Geometry<BITS>;
-    // Off whole steps affine products that do not take the CPU's weights ran on float32 weights: two terms of the element type
-    // keep their precision.
-    constexpr bool kSplit = RAGGED && FP4 == kAffine && !EXACT;
+    // Off whole steps affine products that do not take the CPU's weights run on float32 weights (expand_terms), as the vector
+    // kernels hold them.
+    constexpr bool kSplit = weights_in_terms(FP4, EXACT, RAGGED);
     constexpr int kDepth = G::kDepth, kLoads = G::kLoads;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     using S = std::conditional_t<FP4 != 0, uint8_t, T>;  // stored scale type
@@ -376,10 +410,23 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
                             static_for<4>([&](auto kk_tag) {
                                 constexpr int kk = decltype(kk_tag)::value;
                                 uint4 lo;
-                                expand_split<T, BITS, kk>(codes[t], scale[0], bias, wb[kk], lo);
+                                expand_terms<T, BITS, kk>(codes[t], scale[0], bias, wb[kk], lo);
                                 acc[0] = Ops<T>::mfma(xf[0][kk], wb[kk], Ops<T>::mfma(xf[0][kk], lo, acc[0]));
                                 if (two) acc[1] = Ops<T>::mfma(xf[1][kk], wb[kk], Ops<T>::mfma(xf[1][kk], lo, acc[1]));
                             });
+                            if (!__all(two_terms_hold<T, BITS>(scale[0], bias))) {
+                                uint32_t again[BITS];  // (formed anew: kept from above the terms would not fit the registers)
+#pragma unroll
+                                for (int i = 0; i < BITS; i++) again[i] = opaque(codes[t][i]);
+                                static_for<4>([&](auto kk_tag) {
+                                    constexpr int kk = decltype(kk_tag)::value;
+                                    uint4 hi, lo;
+                                    expand_terms<T, BITS, kk>(again, scale[0], bias, hi, lo);
+                                    const uint4 rest = left_over<T, BITS, kk>(again, scale[0], bias, hi, lo);
+                                    acc[0] = Ops<T>::mfma(xf[0][kk], rest, acc[0]);
+                                    if (two) acc[1] = Ops<T>::mfma(xf[1][kk], rest, acc[1]);
+                                });
+                            }
                             continue;
                         }
                         static_for<4>([&](auto kk_tag) {

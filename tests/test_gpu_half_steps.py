@@ -91,6 +91,27 @@ def test_rows_on_weights_of_two_terms(bits, dtype, m, n, k):
     assert_two_terms(nv.quantized_matmul(x, q).cpu(), x.cpu(), q, ref.F16 if dtype == torch.float16 else ref.BF16, k)
 
 
+@pytest.mark.parametrize("bits", [1, 2, 3, 4, 5, 6, 8])
+@pytest.mark.parametrize("dtype,m,n,k", [(torch.float16, 400, 5000, 160), (torch.bfloat16, 100, 8200, 352)])
+def test_rows_on_weights_of_three_terms(bits, dtype, m, n, k):
+    """A bias far below its scale's largest multiple: the weight c s + b has up to 24 bits.  Groups take turns with b and with none, every
+    code is the largest, and a row of x is 1 and -1 at one place of either kind: the output is b, exactly, if the weights are."""
+    torch.manual_seed(bits)
+    quant, ulp = nv.Quant.affine(32, bits), 2.0 ** (-10 if dtype == torch.float16 else -7)
+    assert ops.quantized_matmul_route(m, n, k, quant, dtype) == "qmg_kernel"
+    s = 1 + ulp
+    b = 2.0 ** (int(np.floor(np.log2((2 ** bits - 1) * s))) - 13) * (1 + ulp)
+    biases = torch.zeros(n, k // 32, device="cuda", dtype=dtype)
+    biases[:, ::2] = b
+    q = nv.Quantized(torch.full((n, k * bits // 32), -1, dtype=torch.int32, device="cuda").view(torch.uint32), torch.full_like(biases, s), biases, quant)
+    x = torch.zeros(m, k)
+    groups = torch.randint(0, k // 64, (m,))
+    x[torch.arange(m), 64 * groups + torch.randint(0, 32, (m,))] = 1
+    x[torch.arange(m), 64 * groups + 32 + torch.randint(0, 32, (m,))] = -1
+    got = nv.quantized_matmul(x.to(dtype).cuda(), q)
+    assert torch.equal(got, torch.full_like(got, b)), (got.float() - b).abs().max().item()
+
+
 @pytest.mark.parametrize("fmt,dtype,m,n,k", [((32, 3), torch.bfloat16, 40, 256, 4128), ((32, 8), torch.float16, 90, 700, 8224), ("MXFP4", torch.bfloat16, 64, 1030, 6176)], ids=str)
 def test_without_a_workspace(fmt, dtype, m, n, k):
     """`nvq_quantized_matmul_static` splits K as the call with a workspace does: the same bits."""

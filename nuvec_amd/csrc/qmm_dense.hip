@@ -149,13 +149,17 @@ double product_us(const ProductArgs &a) {
 
 size_t qmm_dense_workspace_bytes(const ProductArgs &a) { return (size_t)a.n * (size_t)a.k * 2; }
 
+// Half a gigabyte of workspace, W[8191,28672] and a little more: a weight that takes the CPU's values has fewer than 8192 rows.
+constexpr int64_t kMostWeights = 1LL << 28;
+
 // Among the products that the tiled kernel takes with the CPU's weights: where the dequantization (7 us of launches and ends of
 // kernels, and 0.48 us per million weights) and the dense product are estimated a tenth below that kernel.  us here / there, where
 // it turns: W[4096,4096] 384 / 517 rows 49 / 43 and 42 / 68; W[1024,4096] 1024 rows 41 / 31; W[576,576] at 517 rows 13 / 11.
 bool qmm_dense_takes(const ProductArgs &a) {
     if (a.mode != NVQ_AFFINE || !a.exact_weights || a.row_exact || a.batch != 1 || a.batch_ndim != 0 || a.rhs != nullptr || a.lhs != nullptr || a.glu != 0)
         return false;
-    if (a.k < BK || a.k % BK != 0 || a.k > 1 << 22 || a.n * a.k >= (1LL << 32) || (a.m + 127) / 128 > 65535) return false;  // (32-bit offsets in a tile)
+    if (a.k < BK || a.k % BK != 0 || a.k > 1 << 22 || (a.m + 127) / 128 > 65535) return false;  // (32-bit offsets in a tile)
+    if (a.n * a.k > kMostWeights) return false;
     // Where that kernel splits K it stays: its sums and this kernel's, in one order otherwise, would differ in their last bits, and the
     // entry point that brings no workspace promises the bits of the one that does.
     if (qmm_workspace_bytes(a) != 0) return false;

@@ -43,6 +43,19 @@ def test_replays_in_a_graph():
         assert torch.equal(y, want)
 
 
+def test_workspace_is_bounded():
+    """Half a gigabyte at most; the products of larger weights expand codes in the tiled kernel."""
+    import ctypes as C
+
+    from nuvec_amd import _lib
+    ops._init(torch.empty(1, device="cuda"))
+    for n, k in ((4096, 4096), (8191, 28672), (8191, 65536), (8000, 1 << 18)):
+        d = _lib.QmmDescC()
+        d.quant, d.dtype, d.transpose, d.m, d.n, d.k = nv.Quant.affine(64, 4)._c(), ops._CODE[torch.bfloat16], 1, 4096, n, k
+        need = _lib.load().nvq_quantized_matmul_workspace_bytes(C.byref(d))
+        assert need == (2 * n * k if n * k <= 1 << 28 else 0), (n, k, need)
+
+
 @pytest.mark.parametrize("m,n,k", [(517, 4096, 4096), (2048, 3970, 1024), (517, 4096, 14336), (517, 2048, 2048)])
 def test_without_a_workspace(m, n, k):
     """`nvq_quantized_matmul_static` expands codes in the product: the same bits, whether K is split or not."""

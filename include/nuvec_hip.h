@@ -273,8 +273,10 @@ NVQ_API int32_t nvq_quantized_attention(const nvq_attention_desc *desc, const vo
                                 void *out, void *workspace, void *stream);
 
 /* Several query rows per head: the cache dequantized once into `workspace` (always needed: the size query's bytes), both
- * products on the matrix cores, scores and softmax in float32 on chip.  Keys, values and the softmax's weights are rounded
- * to the element type before their products, as the composition rounds them. */
+ * products on the matrix cores, scores and softmax in float32 on chip.  Values and the softmax's weights are rounded to the
+ * element type before their products, as the composition rounds them; keys likewise, but for caches of 1024 positions and
+ * more where the composition's product holds them in float32 (float16; bfloat16 with up to 16 queries or from 8192
+ * positions on): there they are two terms of the element type. */
 NVQ_API size_t nvq_quantized_attention_prompt_workspace_bytes(const nvq_attention_prompt_desc *desc);
 NVQ_API int32_t nvq_quantized_attention_prompt(const nvq_attention_prompt_desc *desc, const void *q, const void *k_w, const void *k_s,
                                 const void *k_b, const void *v_w, const void *v_s, const void *v_b, const void *sinks,

@@ -2,8 +2,10 @@
 // prompt's side of the reference's `quantized_attention` (crates/nuvec-core/src/fast/imp.rs:3996-4035, the composition of two
 // quantized products and a softmax; nuvec-lm's causal mask, crates/nuvec-lm/src/model.rs:3646-3700):
 //     out[b, h, i, :] = softmax(scale * q[b, h, i, :] . K[b, h / rep]^T [masked] [, sink[h]]) . V[b, h / rep]
-// with the scores and the softmax in float32 and never in memory; keys, values and the softmax's weights are rounded to the
-// element type once before their products.
+// with the scores and the softmax in float32 and never in memory; values and the softmax's weights are rounded to the
+// element type once before their products, and keys where the composition's product rounds them (twice there: the CPU's weights).
+// Where that holds them in float32 they are two terms of the element type (keys_are_two_terms): exact wherever scale and bias lie as
+// close as `quantize` leaves them, 17 or 23 bits at least.
 //
 // Two kernels.  The first dequantizes the cache once into a workspace (a cache of 2048 positions x 8 heads is 8 MB there, and
 // stays in the chip's caches; every tile of query rows reads all of it), laid out as the operands of the matrix instruction:
@@ -36,7 +38,7 @@ constexpr float kLog2e = 1.44269504088896340736f;
 
 struct PromptArgs {
     const void *q;
-    const uint4 *keys, *values;  // operands, [batch x key_heads][tiles][D / 16 x 64] each
+    const uint4 *keys, *values;  // operands, [batch x key_heads][tiles][terms of the keys][D / 16 x 64]
     const void *sinks;
     void *out;
     float *partials;             // [splits][heads x queries][D + 2] or NULL
@@ -48,59 +50,69 @@ struct PromptArgs {
 
 // Codes d0 .. d0 + 7 of a row (BITS bytes at byte d0 / 8 x BITS of its dwords), each value rounded once: the product's own
 // rounding first, as `dequantize` has it, is the larger of the two (error against float64, 64 queries over 1024 positions of 8
-// bits: float16 8.7e-4 with both, 4.0e-4 with one, 8.3e-4 in the composition; bfloat16 7.2e-3, 3.2e-3, 8.3e-3).
-template <typename T, int BITS>
-__device__ __forceinline__ uint4 dequantize_eight(const uint32_t *row, int words, int d0, float s, float b) {
+// bits: float16 8.7e-4 with both, 4.0e-4 with one, 8.3e-4 in the composition; bfloat16 7.2e-3, 3.2e-3, 8.3e-3).  TERMS 2: what that
+// leaves in a second term (the first is finite, so that an infinity is the second's).
+template <typename T, int BITS, int TERMS>
+__device__ __forceinline__ void dequantize_eight(const uint32_t *row, int words, int d0, float s, float b, uint4 (&out)[TERMS]) {
+    constexpr float most = Elem<T>::code == NVQ_BF16 ? 3.38953139e38f : 65504.0f;
     const int byte = d0 / 8 * BITS, w = byte >> 2, sh = 8 * (byte & 3);
     uint64_t v = row[w];
     if constexpr (BITS > 1) v |= (uint64_t)row[w + 1 < words ? w + 1 : w] << 32;
     const uint64_t codes = v >> sh;  // (BITS bytes from byte 0 .. 3 of a word: they end in the second one)
-    uint32_t p[4];
+    auto at = [&](int i) { return __builtin_fmaf((float)(uint32_t)((codes >> (i * BITS)) & ((1u << BITS) - 1u)), s, b); };
+    uint32_t p[TERMS][4];
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-        p[i] = qmf::affine_pair<T, false>((float)(uint32_t)((codes >> (2 * i * BITS)) & ((1u << BITS) - 1u)),
-                                         (float)(uint32_t)((codes >> ((2 * i + 1) * BITS)) & ((1u << BITS) - 1u)), s, b);
-    return make_uint4(p[0], p[1], p[2], p[3]);
+    for (int i = 0; i < 4; i++) {
+        float v0 = at(2 * i), v1 = at(2 * i + 1);
+        if constexpr (TERMS == 2) {
+            p[0][i] = Ops<T>::pack(__builtin_amdgcn_fmed3f(v0, -most, most), __builtin_amdgcn_fmed3f(v1, -most, most));
+            v0 -= qmf::half_lo<T>(p[0][i]), v1 -= qmf::half_hi<T>(p[0][i]);
+        }
+        p[TERMS - 1][i] = Ops<T>::pack(v0, v1);
+    }
+#pragma unroll
+    for (int t = 0; t < TERMS; t++) out[t] = make_uint4(p[t][0], p[t][1], p[t][2], p[t][3]);
 }
 
 // Block: one tile of 32 keys of one (batch, key head).  Bound by its reads of the codes; positions past the end are zeros.
-template <typename T, int BITS, int D>
+template <typename T, int BITS, int D, int TERMS>
 __global__ void __launch_bounds__(256) prompt_operands_kernel(const uint32_t *__restrict__ kw, const T *__restrict__ ks, const T *__restrict__ kb,
                                                              const uint32_t *__restrict__ vw, const T *__restrict__ vs, const T *__restrict__ vb,
                                                              int positions, int group_shift, uint4 *__restrict__ keys, uint4 *__restrict__ values) {
     constexpr int kChunks = kKeys * D / 8, words = D * BITS / 32;
     __shared__ __align__(16) uint16_t tile[kKeys][D + 8];
-    const int64_t head = blockIdx.y, base = (head * gridDim.x + blockIdx.x) * kChunks;
+    const int64_t block = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
     const int groups = D >> group_shift, s0 = blockIdx.x * kKeys;
-    const int64_t row0 = head * positions;
+    const int64_t row0 = (int64_t)blockIdx.y * positions;
     for (int c = threadIdx.x; c < kChunks; c += 256) {
         const int key = c & 31, d0 = (c >> 5) * 8;  // (chunk (step << 6 | half << 5 | key): values 16 step + 8 half ..)
-        uint4 k = make_uint4(0, 0, 0, 0), v = k;
+        uint4 k[TERMS] = {}, v[1] = {};
         if (s0 + key < positions) {
             const int64_t row = row0 + s0 + key, g = row * groups + (d0 >> group_shift);
-            k = dequantize_eight<T, BITS>(kw + row * words, words, d0, Elem<T>::load(ks, g), Elem<T>::load(kb, g));
-            v = dequantize_eight<T, BITS>(vw + row * words, words, d0, Elem<T>::load(vs, g), Elem<T>::load(vb, g));
+            dequantize_eight<T, BITS, TERMS>(kw + row * words, words, d0, Elem<T>::load(ks, g), Elem<T>::load(kb, g), k);
+            dequantize_eight<T, BITS, 1>(vw + row * words, words, d0, Elem<T>::load(vs, g), Elem<T>::load(vb, g), v);
         }
-        keys[base + c] = k;
-        *reinterpret_cast<uint4 *>(&tile[key][d0]) = v;
+#pragma unroll
+        for (int t = 0; t < TERMS; t++) keys[(block * TERMS + t) * kChunks + c] = k[t];
+        *reinterpret_cast<uint4 *>(&tile[key][d0]) = v[0];
     }
     __syncthreads();
     for (int c = threadIdx.x; c < kChunks; c += 256) {
-        const int lane = c & 63, h = lane >> 5, block = c >> 6;  // block: which sixteen keys x which 32 values of D
-        const int s = block / (D / 32) * 16 + 4 * h, d = block % (D / 32) * 32 + (lane & 31);
+        const int lane = c & 63, h = lane >> 5, part = c >> 6;  // part: which sixteen keys x which 32 values of D
+        const int s = part / (D / 32) * 16 + 4 * h, d = part % (D / 32) * 32 + (lane & 31);
         uint32_t p[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const int key = s + (j < 2 ? 2 * j : 8 + 2 * (j - 2));
             p[j] = (uint32_t)tile[key][d] | (uint32_t)tile[key + 1][d] << 16;
         }
-        values[base + c] = make_uint4(p[0], p[1], p[2], p[3]);
+        values[block * kChunks + c] = make_uint4(p[0], p[1], p[2], p[3]);
     }
 }
 
 // RG row groups of 32 rows a block, 4 / RG wavefronts on each: two wavefronts a SIMD hold 64 accumulators, the query's 32
 // operand registers and one tile of keys and values in flight (D = 128).
-template <typename T, int D, int RG>
+template <typename T, int D, int RG, int TERMS>
 __global__ void __launch_bounds__(64 * kWaves, 2) prompt_attention_kernel(const PromptArgs a) {
     constexpr int KP = kWaves / RG, KS = D / 16, DB = D / 32;
     constexpr int kChunks = kKeys * D / 8;
@@ -139,12 +151,13 @@ __global__ void __launch_bounds__(64 * kWaves, 2) prompt_attention_kernel(const 
     int t_end = t_begin + per < a.tiles ? t_begin + per : a.tiles;
     if (any_last / kKeys + 1 < t_end) t_end = any_last < 0 ? 0 : any_last / kKeys + 1;
     if (r0 >= rows) t_end = 0;  // (a row group past the end)
-    const uint4 *kf = a.keys + (int64_t)head * a.tiles * kChunks + lane, *vf = a.values + (int64_t)head * a.tiles * kChunks + lane;
-    uint4 kt[KS], vt[KS];
-    auto fetch = [&](const uint4 *from, int t, uint4 (&to)[KS]) {
-        const uint4 *p = from + (int64_t)(t < a.tiles ? t : a.tiles - 1) * kChunks;  // (past the end: read, not used)
+    const uint4 *kf = a.keys + (int64_t)head * a.tiles * (TERMS * kChunks) + lane, *vf = a.values + (int64_t)head * a.tiles * kChunks + lane;
+    uint4 kt[TERMS * KS], vt[KS];
+    auto fetch = [&](const uint4 *from, int t, auto &to) {
+        constexpr int n = sizeof(to) / sizeof(uint4);
+        const uint4 *p = from + (int64_t)(t < a.tiles ? t : a.tiles - 1) * (n * 64);  // (past the end: read, not used)
 #pragma unroll
-        for (int s = 0; s < KS; s++) to[s] = p[64 * s];
+        for (int s = 0; s < n; s++) to[s] = p[64 * s];
     };
     fetch(kf, t_begin + kp, kt);
     fetch(vf, t_begin + kp, vt);
@@ -153,7 +166,7 @@ __global__ void __launch_bounds__(64 * kWaves, 2) prompt_attention_kernel(const 
 #pragma unroll
         for (int e = 0; e < 16; e++) s[e] = 0.0f;
 #pragma unroll
-        for (int k = 0; k < KS; k++) s = Ops<T>::mfma(kt[k], qf[k], s);
+        for (int k = TERMS * KS - 1; k >= 0; k--) s = Ops<T>::mfma(kt[k], qf[k % KS], s);  // (the second terms first)
         fetch(kf, t + KP, kt);
         const int key0 = t * kKeys + 4 * half;  // register e: key 8 (e / 4) + 4 half + e % 4
         if (t * kKeys + kKeys - 1 > all_last) {
@@ -269,10 +282,16 @@ __global__ void __launch_bounds__(kMergeParts * D) prompt_merge_kernel(const Pro
 }
 
 struct Plan {
-    int tiles, row_tiles, row_groups, splits;
+    int tiles, row_tiles, row_groups, splits, terms;
     int64_t heads, rows;
-    size_t operand_bytes, partial_bytes;
+    size_t key_bytes, value_bytes, partial_bytes;
 };
+
+// Whether the composition's product holds keys in float32: outputs of 1024 and more per row, but for bfloat16 products of more than
+// 16 rows up to 8192 outputs, which take the CPU's weights as the products of fewer do.
+bool keys_are_two_terms(const nvq_attention_prompt_desc &p) {
+    return p.cache.positions >= 1024 && !(p.cache.dtype == NVQ_BF16 && p.queries > 16 && p.cache.positions < 8192);
+}
 
 // Row groups a block: four (every tile of keys read once per 128 rows) where that gives two blocks per compute unit, else two,
 // else one (four wavefronts on the same 32 rows); then, with fewer blocks than compute units still, splits of the keys over the
@@ -284,6 +303,8 @@ Plan prompt_plan(const nvq_attention_prompt_desc &p) {
     r.rows = d.query_heads / d.key_heads * p.queries;
     r.tiles = (int)((d.positions + kKeys - 1) / kKeys);
     r.row_tiles = (int)((r.rows + kRows - 1) / kRows);
+    r.terms = keys_are_two_terms(p) ? 2 : 1;
+    const int64_t head_bytes = (int64_t)r.tiles * kKeys * d.head_dim * 2;
     const int64_t cus = compute_units();
     r.row_groups = 1;
     for (int g = 4; g > 1; g /= 2)
@@ -293,7 +314,7 @@ Plan prompt_plan(const nvq_attention_prompt_desc &p) {
         }
     r.splits = 1;
     const int64_t blocks = r.heads * r.row_tiles;
-    if (r.row_groups == 1 && blocks < cus) {
+    if (r.row_groups == 1 && blocks < cus && blocks > 0) {
         int64_t want = (2 * cus + blocks - 1) / blocks;
         if (want > r.tiles / 8) want = r.tiles / 8;
         if (want > 32) want = 32;
@@ -302,64 +323,67 @@ Plan prompt_plan(const nvq_attention_prompt_desc &p) {
             r.splits = (int)((r.tiles + per - 1) / per);
         }
     }
-    r.operand_bytes = (size_t)r.heads * r.tiles * kKeys * d.head_dim * 2;
+    r.key_bytes = (size_t)(r.heads * r.terms * head_bytes), r.value_bytes = (size_t)(r.heads * head_bytes);
     r.partial_bytes = r.splits > 1 ? (size_t)r.splits * r.heads * r.rows * (d.head_dim + 2) * sizeof(float) : 0;
     return r;
 }
 
-template <typename T, int D, int RG>
-int32_t run_rows(const PromptArgs &a, const Plan &p, hipStream_t s) {
-    const int64_t blocks = p.heads * ((p.row_tiles + RG - 1) / RG);
-    hipLaunchKernelGGL((prompt_attention_kernel<T, D, RG>), dim3((unsigned)blocks, (unsigned)p.splits), dim3(64 * kWaves), 0, s, a);
+template <typename T, int D, int TERMS>
+int32_t run_rows(const PromptArgs &a, const Plan &p, int64_t heads, hipStream_t s) {
+    const dim3 grid((unsigned)(heads * ((p.row_tiles + p.row_groups - 1) / p.row_groups)), (unsigned)p.splits), block(64 * kWaves);
+    switch (p.row_groups) {
+    case 4: hipLaunchKernelGGL((prompt_attention_kernel<T, D, 4, TERMS>), grid, block, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((prompt_attention_kernel<T, D, 2, TERMS>), grid, block, 0, s, a); break;
+    default: hipLaunchKernelGGL((prompt_attention_kernel<T, D, 1, TERMS>), grid, block, 0, s, a); break;
+    }
     NVQ_LAUNCH_CHECK("quantized_attention");
     if (p.splits > 1) {
-        hipLaunchKernelGGL((prompt_merge_kernel<T, D>), dim3((unsigned)p.rows, (unsigned)p.heads), dim3(kMergeParts * D), 0, s, a);
+        hipLaunchKernelGGL((prompt_merge_kernel<T, D>), dim3((unsigned)p.rows, (unsigned)heads), dim3(kMergeParts * D), 0, s, a);
         NVQ_LAUNCH_CHECK("quantized_attention merge");
     }
     return NVQ_OK;
 }
 
-template <typename T, int D>
-int32_t run_sized(const nvq_attention_prompt_desc &desc, const void *q, const void *kw, const void *ks, const void *kb, const void *vw,
-                  const void *vs, const void *vb, const void *sinks, void *out, void *workspace, hipStream_t s) {
+template <typename T, int D, int TERMS>
+int32_t run_sized(const nvq_attention_prompt_desc &desc, const Plan &p, const void *q, const void *kw, const void *ks, const void *kb,
+                  const void *vw, const void *vs, const void *vb, const void *sinks, void *out, void *workspace, hipStream_t s) {
     const nvq_attention_desc &d = desc.cache;
-    const Plan p = prompt_plan(desc);
-    uint4 *keys = (uint4 *)workspace, *values = keys + p.operand_bytes / 16;
+    uint4 *keys = (uint4 *)workspace, *values = keys + p.key_bytes / 16;
     int shift = 5;
     while ((1 << shift) < d.group_size) shift++;
-    const dim3 grid((unsigned)p.tiles, (unsigned)p.heads);
-#define NVQ_OPERANDS(B)                                                                                                                  \
-    case B:                                                                                                                              \
-        hipLaunchKernelGGL((prompt_operands_kernel<T, B, D>), grid, dim3(256), 0, s, (const uint32_t *)kw, (const T *)ks, (const T *)kb, \
-                           (const uint32_t *)vw, (const T *)vs, (const T *)vb, (int)d.positions, shift, keys, values);                    \
-        break;
-    switch (d.bits) { NVQ_OPERANDS(1) NVQ_OPERANDS(2) NVQ_OPERANDS(3) NVQ_OPERANDS(4) NVQ_OPERANDS(5) NVQ_OPERANDS(6) NVQ_OPERANDS(8) }
-#undef NVQ_OPERANDS
-    NVQ_LAUNCH_CHECK("quantized_attention operands");
     PromptArgs a{};
     a.q = q, a.keys = keys, a.values = values, a.sinks = sinks, a.out = out;
-    a.partials = (float *)((char *)workspace + 2 * p.operand_bytes);
+    a.partials = (float *)((char *)workspace + p.key_bytes + p.value_bytes);
     a.scale = d.scale, a.causal = desc.causal;
     a.query_heads = (int)d.query_heads, a.key_heads = (int)d.key_heads, a.rep = (int)(d.query_heads / d.key_heads);
     a.queries = (int)desc.queries, a.positions = (int)d.positions;
     a.tiles = p.tiles, a.row_tiles = p.row_tiles, a.splits = p.splits;
-    return p.row_groups == 4 ? run_rows<T, D, 4>(a, p, s) : p.row_groups == 2 ? run_rows<T, D, 2>(a, p, s) : run_rows<T, D, 1>(a, p, s);
+    const dim3 grid((unsigned)p.tiles, (unsigned)p.heads);
+#define NVQ_OPERANDS(B)                                                                                                                             case B:                                                                                                                                             hipLaunchKernelGGL((prompt_operands_kernel<T, B, D, TERMS>), grid, dim3(256), 0, s, (const uint32_t *)kw, (const T *)ks, (const T *)kb,                            (const uint32_t *)vw, (const T *)vs, (const T *)vb, (int)d.positions, shift, keys, values);                          break;
+    switch (d.bits) { NVQ_OPERANDS(1) NVQ_OPERANDS(2) NVQ_OPERANDS(3) NVQ_OPERANDS(4) NVQ_OPERANDS(5) NVQ_OPERANDS(6) NVQ_OPERANDS(8) }
+#undef NVQ_OPERANDS
+    NVQ_LAUNCH_CHECK("quantized_attention operands");
+    return run_rows<T, D, TERMS>(a, p, p.heads, s);
+}
+
+template <typename T, typename... A>
+int32_t run_type(const nvq_attention_prompt_desc &d, A... args) {
+    const Plan p = prompt_plan(d);
+    if (d.cache.head_dim == 64) return p.terms == 2 ? run_sized<T, 64, 2>(d, p, args...) : run_sized<T, 64, 1>(d, p, args...);
+    return p.terms == 2 ? run_sized<T, 128, 2>(d, p, args...) : run_sized<T, 128, 1>(d, p, args...);
 }
 
 }  // namespace
 
 size_t attention_prompt_workspace_bytes(const nvq_attention_prompt_desc &d) {
     const Plan p = prompt_plan(d);
-    return 2 * p.operand_bytes + p.partial_bytes;
+    return p.key_bytes + p.value_bytes + p.partial_bytes;
 }
 
 int32_t launch_attention_prompt(const nvq_attention_prompt_desc &d, const void *q, const void *kw, const void *ks, const void *kb,
                                 const void *vw, const void *vs, const void *vb, const void *sinks, void *out, void *workspace, hipStream_t s) {
-    if (d.cache.dtype == NVQ_BF16)
-        return d.cache.head_dim == 64 ? run_sized<bf16_t, 64>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s)
-                                      : run_sized<bf16_t, 128>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s);
-    return d.cache.head_dim == 64 ? run_sized<f16_t, 64>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s)
-                                  : run_sized<f16_t, 128>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s);
+    return d.cache.dtype == NVQ_BF16 ? run_type<bf16_t>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s)
+                                     : run_type<f16_t>(d, q, kw, ks, kb, vw, vs, vb, sinks, out, workspace, s);
 }
 
 }  // namespace nvq

@@ -272,8 +272,9 @@ NVQ_API int32_t nvq_quantized_attention(const nvq_attention_desc *desc, const vo
                                 const void *k_b, const void *v_w, const void *v_s, const void *v_b, const void *sinks,
                                 void *out, void *workspace, void *stream);
 
-/* Several query rows per head: the cache dequantized once into `workspace` (always needed: the size query's bytes), both
- * products on the matrix cores, scores and softmax in float32 on chip.  Values and the softmax's weights are rounded to the
+/* Several query rows per head: the cache dequantized once into `workspace` (always needed: the size query's bytes, at
+ * most 256 MB of dequantized heads at a time, or one head, and the states of the splits), both products on the matrix cores, scores and
+ * softmax in float32 on chip.  Values and the softmax's weights are rounded to the
  * element type before their products, as the composition rounds them; keys likewise, but for caches of 1024 positions and
  * more where the composition's product holds them in float32 (float16; bfloat16 with up to 16 queries or from 8192
  * positions on): there they are two terms of the element type. */

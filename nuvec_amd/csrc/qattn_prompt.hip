@@ -38,13 +38,14 @@ constexpr float kLog2e = 1.44269504088896340736f;
 
 struct PromptArgs {
     const void *q;
-    const uint4 *keys, *values;  // operands, [batch x key_heads][tiles][terms of the keys][D / 16 x 64]
+    const uint4 *keys, *values;  // operands of the heads from head0 on, [heads][tiles][terms of the keys][D / 16 x 64]
     const void *sinks;
     void *out;
     float *partials;             // [splits][heads x queries][D + 2] or NULL
     float scale;
     int32_t causal;
     int32_t query_heads, key_heads, rep, queries, positions;
+    int32_t head0;               // (batch x key head) of the launch's first
     int32_t tiles, row_tiles, splits;
 };
 
@@ -78,12 +79,12 @@ __device__ __forceinline__ void dequantize_eight(const uint32_t *row, int words,
 template <typename T, int BITS, int D, int TERMS>
 __global__ void __launch_bounds__(256) prompt_operands_kernel(const uint32_t *__restrict__ kw, const T *__restrict__ ks, const T *__restrict__ kb,
                                                              const uint32_t *__restrict__ vw, const T *__restrict__ vs, const T *__restrict__ vb,
-                                                             int positions, int group_shift, uint4 *__restrict__ keys, uint4 *__restrict__ values) {
+                                                             int head0, int positions, int group_shift, uint4 *__restrict__ keys, uint4 *__restrict__ values) {
     constexpr int kChunks = kKeys * D / 8, words = D * BITS / 32;
     __shared__ __align__(16) uint16_t tile[kKeys][D + 8];
     const int64_t block = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
     const int groups = D >> group_shift, s0 = blockIdx.x * kKeys;
-    const int64_t row0 = (int64_t)blockIdx.y * positions;
+    const int64_t row0 = (int64_t)(head0 + blockIdx.y) * positions;
     for (int c = threadIdx.x; c < kChunks; c += 256) {
         const int key = c & 31, d0 = (c >> 5) * 8;  // (chunk (step << 6 | half << 5 | key): values 16 step + 8 half ..)
         uint4 k[TERMS] = {}, v[1] = {};
@@ -124,7 +125,7 @@ __global__ void __launch_bounds__(64 * kWaves, 2) prompt_attention_kernel(const 
     const int rg = wave / KP, kp = wave % KP;
     // blocks of one key head lie `heads` apart: on one XCD, whose L2 then holds that head's keys, where heads is a multiple of 8
     const int heads = gridDim.x / ((a.row_tiles + RG - 1) / RG);
-    const int head = blockIdx.x % heads, b = head / a.key_heads, hk = head % a.key_heads;
+    const int head = blockIdx.x % heads, b = (a.head0 + head) / a.key_heads, hk = (a.head0 + head) % a.key_heads;
     const int block_tile = (a.row_tiles + RG - 1) / RG - 1 - blockIdx.x / heads;  // (the longest rows of a causal product first)
     const int rows = a.rep * a.queries, r0 = (block_tile * RG + rg) * kRows, r = r0 + col;
     const bool live = r < rows;
@@ -274,7 +275,7 @@ template <typename T, int D>
 __global__ void __launch_bounds__(kMergeParts * D) prompt_merge_kernel(const PromptArgs a) {
     const int rows = a.rep * a.queries;
     const int64_t all = (int64_t)gridDim.x * gridDim.y;  // rows x (batch x key heads)
-    const int r = blockIdx.x, head = blockIdx.y, b = head / a.key_heads, hk = head % a.key_heads;
+    const int r = blockIdx.x, head = blockIdx.y, b = (a.head0 + head) / a.key_heads, hk = (a.head0 + head) % a.key_heads;
     const int h = hk * a.rep + r % a.rep, i = r / a.rep;
     merge_attention_states<T, D>(a.partials + ((int64_t)head * rows + r) * (D + 2), all * (D + 2), a.splits, a.sinks != nullptr,
                                  a.sinks != nullptr ? Elem<T>::load((const T *)a.sinks, h) * kLog2e : 0.0f,
@@ -283,9 +284,14 @@ __global__ void __launch_bounds__(kMergeParts * D) prompt_merge_kernel(const Pro
 
 struct Plan {
     int tiles, row_tiles, row_groups, splits, terms;
-    int64_t heads, rows;
+    int64_t heads, slice;  // all (batch, key head)s, and those of one launch
+    int64_t rows;
     size_t key_bytes, value_bytes, partial_bytes;
 };
+
+// Operands of more heads than this go one slice after the other through one workspace: 32 batches x 8 key heads over 32768 positions
+// are 4.3 GB of them.  (256 MB is also what the chip's last cache holds.)
+constexpr int64_t kOperandMost = 256LL << 20;
 
 // Whether the composition's product holds keys in float32: outputs of 1024 and more per row, but for bfloat16 products of more than
 // 16 rows up to 8192 outputs, which take the CPU's weights as the products of fewer do.
@@ -304,16 +310,18 @@ Plan prompt_plan(const nvq_attention_prompt_desc &p) {
     r.tiles = (int)((d.positions + kKeys - 1) / kKeys);
     r.row_tiles = (int)((r.rows + kRows - 1) / kRows);
     r.terms = keys_are_two_terms(p) ? 2 : 1;
-    const int64_t head_bytes = (int64_t)r.tiles * kKeys * d.head_dim * 2;
+    const int64_t head_bytes = (int64_t)r.tiles * kKeys * d.head_dim * 2, most = kOperandMost / ((r.terms + 1) * head_bytes);
+    const int64_t slices = (r.heads + (most > 1 ? most : 1) - 1) / (most > 1 ? most : 1);
+    r.slice = slices > 1 ? (r.heads + slices - 1) / slices : r.heads;
     const int64_t cus = compute_units();
     r.row_groups = 1;
     for (int g = 4; g > 1; g /= 2)
-        if (r.heads * ((r.row_tiles + g - 1) / g) >= 2 * cus) {
+        if (r.slice * ((r.row_tiles + g - 1) / g) >= 2 * cus) {
             r.row_groups = g;
             break;
         }
     r.splits = 1;
-    const int64_t blocks = r.heads * r.row_tiles;
+    const int64_t blocks = r.slice * r.row_tiles;
     if (r.row_groups == 1 && blocks < cus && blocks > 0) {
         int64_t want = (2 * cus + blocks - 1) / blocks;
         if (want > r.tiles / 8) want = r.tiles / 8;
@@ -323,8 +331,8 @@ Plan prompt_plan(const nvq_attention_prompt_desc &p) {
             r.splits = (int)((r.tiles + per - 1) / per);
         }
     }
-    r.key_bytes = (size_t)(r.heads * r.terms * head_bytes), r.value_bytes = (size_t)(r.heads * head_bytes);
-    r.partial_bytes = r.splits > 1 ? (size_t)r.splits * r.heads * r.rows * (d.head_dim + 2) * sizeof(float) : 0;
+    r.key_bytes = (size_t)(r.slice * r.terms * head_bytes), r.value_bytes = (size_t)(r.slice * head_bytes);
+    r.partial_bytes = r.splits > 1 ? (size_t)r.splits * r.slice * r.rows * (d.head_dim + 2) * sizeof(float) : 0;
     return r;
 }
 
@@ -358,12 +366,18 @@ int32_t run_sized(const nvq_attention_prompt_desc &desc, const Plan &p, const vo
     a.query_heads = (int)d.query_heads, a.key_heads = (int)d.key_heads, a.rep = (int)(d.query_heads / d.key_heads);
     a.queries = (int)desc.queries, a.positions = (int)d.positions;
     a.tiles = p.tiles, a.row_tiles = p.row_tiles, a.splits = p.splits;
-    const dim3 grid((unsigned)p.tiles, (unsigned)p.heads);
-#define NVQ_OPERANDS(B)                                                                                                                             case B:                                                                                                                                             hipLaunchKernelGGL((prompt_operands_kernel<T, B, D, TERMS>), grid, dim3(256), 0, s, (const uint32_t *)kw, (const T *)ks, (const T *)kb,                            (const uint32_t *)vw, (const T *)vs, (const T *)vb, (int)d.positions, shift, keys, values);                          break;
-    switch (d.bits) { NVQ_OPERANDS(1) NVQ_OPERANDS(2) NVQ_OPERANDS(3) NVQ_OPERANDS(4) NVQ_OPERANDS(5) NVQ_OPERANDS(6) NVQ_OPERANDS(8) }
+    for (int64_t first = 0; first < p.heads; first += p.slice) {  // (the stream keeps a slice's readers ahead of the next one's writers)
+        const int64_t heads = p.heads - first < p.slice ? p.heads - first : p.slice;
+        const dim3 grid((unsigned)p.tiles, (unsigned)heads);
+        a.head0 = (int)first;
+#define NVQ_OPERANDS(B)                                                                                                                             case B:                                                                                                                                             hipLaunchKernelGGL((prompt_operands_kernel<T, B, D, TERMS>), grid, dim3(256), 0, s, (const uint32_t *)kw, (const T *)ks, (const T *)kb,                            (const uint32_t *)vw, (const T *)vs, (const T *)vb, a.head0, (int)d.positions, shift, keys, values);                          break;
+        switch (d.bits) { NVQ_OPERANDS(1) NVQ_OPERANDS(2) NVQ_OPERANDS(3) NVQ_OPERANDS(4) NVQ_OPERANDS(5) NVQ_OPERANDS(6) NVQ_OPERANDS(8) }
 #undef NVQ_OPERANDS
-    NVQ_LAUNCH_CHECK("quantized_attention operands");
-    return run_rows<T, D, TERMS>(a, p, p.heads, s);
+        NVQ_LAUNCH_CHECK("quantized_attention operands");
+        const int32_t rc = run_rows<T, D, TERMS>(a, p, heads, s);
+        if (rc != NVQ_OK) return rc;
+    }
+    return NVQ_OK;
 }
 
 template <typename T, typename... A>

@@ -31,6 +31,7 @@ CASES = [
     (1, 8, 2, 24, 8192, 128, 3, 32, True, False),    # (both types, many positions)
     (4, 64, 4, 130, 1056, 128, 6, 128, False, False),  # two and four row groups a block
     (8, 64, 8, 200, 1100, 64, 4, 64, True, False),
+    (11, 8, 8, 3, 16500, 128, 4, 64, True, False),   # more heads than one workspace holds: slices, the last one smaller
 ]
 
 
@@ -97,6 +98,19 @@ def test_keys_of_two_terms(dtype, l, s, d):
     got = layers.quantized_attention(q, k, v, 1.0)
     want = float(np.tanh(delta / 2))
     assert ((got.double() - want).abs() <= 1.1 * 2.0 ** (-8 if dtype == torch.bfloat16 else -11) * (1 + want)).all(), (got[0, 0, 0, 0].item(), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_workspace_is_bounded(dtype):
+    """32 batches of 8 key heads over 32768 positions: 4.3 GB of operands, which pass through one workspace slice by slice."""
+    import ctypes as C
+
+    from nuvec_amd import _lib
+    ops._init(torch.empty(1, device="cuda"))
+    for batch, queries in ((1, 2), (32, 2), (32, 512)):
+        d = _lib.AttentionPromptDescC(_lib.AttentionDescC(ops._CODE[dtype], 4, 64, 128, batch, 32, 8, 32768, 0.1), queries, 1)
+        need = _lib.load().nvq_quantized_attention_prompt_workspace_bytes(C.byref(d))
+        assert 0 < need <= 320 << 20, need  # (256 MB of operands; the splits' states beside them)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

@@ -167,7 +167,9 @@ __global__ void __launch_bounds__(64 * kWaves, 2) prompt_attention_kernel(const 
 #pragma unroll
         for (int e = 0; e < 16; e++) s[e] = 0.0f;
 #pragma unroll
-        for (int k = TERMS * KS - 1; k >= 0; k--) s = Ops<T>::mfma(kt[k], qf[k % KS], s);  // (the second terms first)
+        for (int term = TERMS - 1; term >= 0; term--)  // (the small ones first)
+#pragma unroll
+            for (int k = 0; k < KS; k++) s = Ops<T>::mfma(kt[term * KS + k], qf[k], s);
         fetch(kf, t + KP, kt);
         const int key0 = t * kKeys + 4 * half;  // register e: key 8 (e / 4) + 4 half + e % 4
         if (t * kKeys + kKeys - 1 > all_last) {

@@ -76,9 +76,12 @@ def test_attention_equals_the_python_path(both, dtype):
     torch.manual_seed(2)
     k, v = (nv.quantize(torch.randn(2, 2, 600, 64, device="cuda").to(dtype), nv.Quant.affine(32, 8)) for _ in range(2))
     q, sinks = torch.randn(2, 8, 1, 64, device="cuda").to(dtype), torch.randn(8, device="cuda").to(dtype)
+    several = torch.randn(2, 8, 37, 64, device="cuda").to(dtype)
     for s in (None, sinks):
         assert same(*both(lambda: layers.quantized_attention(q, k, v, 0.125, s, causal=True)))
         assert same(*both(lambda: nv.ops.quantized_attention(q, k, v, 0.125, s)))
+        for causal in (False, True):
+            assert same(*both(lambda: layers.quantized_attention(several, k, v, 0.125, s, causal=causal)))
 
 
 def test_refusals_are_the_python_paths():
@@ -263,7 +266,8 @@ def test_router(rows, dims, experts, k, dtype):
 @pytest.mark.parametrize("quant", [nv.Quant.affine(64, 4), nv.Quant.affine(32, 8), nv.Quant.new(nv.QuantMode.MXFP4)], ids=str)
 @pytest.mark.parametrize("dims,hidden,bias,activation", [(256, 1024, True, "swiglu_oai"), (512, 96, False, "swiglu"), (320, 640, True, "geglu")])
 def test_moe_equals_the_python_path(both, quant, dims, hidden, bias, activation):
-    """The same kernels but for the router's (its softmax may round a probability the other way: one step of a score)."""
+    """The same kernels but for the router's, whose logits and softmax may round the other way: each score s of a token within two of its
+    steps (2 x 2^-7 s: its own and the sum's that divides it), and with it each product s y (a rounding, 2^-8, either way) and their sum."""
     torch.manual_seed(3)
     if dims % quant.group_size or hidden % quant.group_size:
         pytest.skip("not whole groups")
@@ -278,5 +282,7 @@ def test_moe_equals_the_python_path(both, quant, dims, hidden, bias, activation)
         for tokens in (1, 31, 32, 200):
             x = torch.randn(1, tokens, dims, device="cuda").bfloat16()
             native, python = both(lambda: block(x))
-            bound = 4 * 2.0 ** -8 * python.float().abs().max()
+            top, scores = block.route(x)
+            terms = (scores.float()[..., None] * block.switch_mlp.forward(x, top).float()).abs().sum(-2)
+            bound = (2 * 2.0 ** -7 + 2.0 ** -8) * terms + 2.0 ** -7 * python.float().abs()
             assert native.shape == python.shape and ((native.float() - python.float()).abs() <= bound).all(), (fuse, tokens)

@@ -74,7 +74,8 @@ def unrounded(q):
 
 
 def assert_two_terms(got, x, q, dtype, k):
-    """One rounding of the output (u |out|); weights of two terms, u^2 of each, and float32 sums, whose errors are random over K."""
+    """One rounding of the output (u |out|); float32 weights (two terms of them, exact here, may leave u^2 of each where a third does
+    not) and float32 sums, whose errors are random over K."""
     u, w = {ref.BF16: 2.0 ** -8, ref.F16: 2.0 ** -11}[dtype], unrounded(q).cpu()
     want, norms = x.double() @ w.T, x.double().norm(dim=1, keepdim=True) * w.norm(dim=1)
     assert ((got.double() - want).abs() <= u * want.abs() + 4 * (u * u / 2 + 2.0 ** -24) * norms).all()

@@ -286,3 +286,27 @@ def test_moe_equals_the_python_path(both, quant, dims, hidden, bias, activation)
             terms = (scores.float()[..., None] * block.switch_mlp.forward(x, top).float()).abs().sum(-2)
             bound = (2 * 2.0 ** -7 + 2.0 ** -8) * terms + 2.0 ** -7 * python.float().abs()
             assert native.shape == python.shape and ((native.float() - python.float()).abs() <= bound).all(), (fuse, tokens)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_attention_replays_in_a_graph(dtype):
+    """Captured with its workspace and replayed after other work: the eager result.  One query row on the vector kernel and on the matrix
+    cores, whole and with its positions split; several rows whole, split, and in slices of the heads."""
+    torch.manual_seed(7)
+    for b, heads, key_heads, queries, s, d, bits in ((1, 2, 2, 1, 90, 64, 4), (1, 2, 2, 1, 5000, 128, 8), (40, 32, 4, 1, 300, 128, 4), (4, 16, 2, 1, 9000, 64, 3),
+                                                     (2, 8, 2, 33, 200, 64, 4), (1, 4, 1, 3, 4000, 128, 8), (12, 8, 8, 2, 16500, 128, 4)):
+        k, v = (nv.quantize(torch.randn(b, key_heads, s, d, device="cuda").to(dtype), nv.Quant.affine(32, bits)) for _ in range(2))
+        q = torch.randn(b, heads, queries, d, device="cuda").to(dtype)
+        run = lambda: layers.quantized_attention(q, k, v, d ** -0.5, causal=True)
+        want = run()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            got = run()
+        for _ in range(3):
+            q.copy_(q.flip(0))  # (a batch of one: the same queries)
+            run()
+            q.copy_(q.flip(0))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(got, want), (b, heads, queries, s)

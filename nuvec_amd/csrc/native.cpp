@@ -451,20 +451,21 @@ PyObject *py_mlp(PyObject *, PyObject *const *args, Py_ssize_t n) {
         if (truth < 0) return nullptr;
         const int32_t activation = truth ? NVQ_GLU_GEGLU : NVQ_GLU_SWIGLU;
         const int64_t rows = x.numel() / x.size(-1), most = gate.p.q.mode == NVQ_AFFINE ? 2 : 4;  // (layers.Mlp.forward says why)
-        const bool one = both.p != Py_None && rows <= most;
-        if ((one && !read_linear(both.p, fused)) || !read_linear(args[0], names.up_proj, up)) return none();
         const Place at(x);
         const at::ScalarType type = x.scalar_type();
-        if (!linear_fits(gate, at, type, x.size(-1)) || !linear_fits(up, at, type, x.size(-1)) || up.p.w.size(0) != gate.p.w.size(0) ||
-            !linear_fits(down, at, type, gate.p.w.size(0)) || (one && (!linear_fits(fused, at, type, x.size(-1)) || fused.p.w.size(0) != 2 * gate.p.w.size(0))))
-            return none();
+        if (!linear_fits(gate, at, type, x.size(-1)) || !linear_fits(down, at, type, gate.p.w.size(0))) return none();
+        if (both.p != Py_None && rows <= most) {
+            if (!read_linear(both.p, fused) || !linear_fits(fused, at, type, x.size(-1)) || fused.p.w.size(0) != 2 * gate.p.w.size(0)) return none();
+            const bool done = unlocked([&] {
+                return product_glu(x, fused.p, fused.bias, activation, 0.0f, 0.0f, hidden) && product(hidden, down.p, down.bias, Flags(), y);
+            });
+            if (hidden.defined()) return wrap(done, y);
+        }
+        if (!read_linear(args[0], names.up_proj, up) || !linear_fits(up, at, type, x.size(-1)) || up.p.w.size(0) != gate.p.w.size(0)) return none();
         const bool done = unlocked([&] {
-            if (one) product_glu(x, fused.p, fused.bias, activation, 0.0f, 0.0f, hidden);
-            if (!hidden.defined()) {
-                Tensor g, u;
-                if (!product(x, gate.p, gate.bias, Flags(), g) || !product(x, up.p, up.bias, Flags(), u) || !gated(g, u, activation, hidden)) return false;
-            }
-            return product(hidden, down.p, down.bias, Flags(), y);
+            Tensor g, u;
+            return product(x, gate.p, gate.bias, Flags(), g) && product(x, up.p, up.bias, Flags(), u) && gated(g, u, activation, hidden) &&
+                   product(hidden, down.p, down.bias, Flags(), y);
         });
         return wrap(done, y);
     });

@@ -590,7 +590,7 @@ static bool takes_tiled(const nvq_qmm_desc *d, const ProductArgs &a) {
 }
 
 // The kernel family of a product (the counterpart of the routing in GpuEval::quantized_matmul, gpu.rs:6934-7168).
-enum class Route { kUntransposed, kVector, kTiled, kTiledF32, kFewRowsF32, kGroupedRows, kBatchedDecode, kFewRowsDirect, kFewRows };
+enum class Route { kUntransposed, kVector, kTiled, kTiledF32, kGroupedRows, kBatchedDecode, kFewRowsDirect, kFewRows };
 static Route pick_route(const nvq_qmm_desc *d, const ProductArgs &a);
 
 // `dense`: whether the workspace may hold the dequantized weight.
@@ -602,7 +602,9 @@ static size_t workspace_bytes(const nvq_qmm_desc *d, bool dense) {
     const ProductArgs a = product_args(d, batch);
     // float32 partial sums of the splits of K: weights stored [K, N], or few tiles of a long K
     if (!d->transpose) return qvm_workspace_bytes(a);
-    if (pick_route(d, a) != Route::kTiled) return 0;
+    const Route route = pick_route(d, a);
+    if (route == Route::kTiledF32) return qmm_f32_workspace_bytes(a);
+    if (route != Route::kTiled) return 0;
     return dense && qmm_dense_takes(a) ? qmm_dense_workspace_bytes(a) : qmm_workspace_bytes(a);
 }
 
@@ -611,8 +613,7 @@ size_t nvq_quantized_matmul_workspace_bytes(const nvq_qmm_desc *d) { return work
 static Route pick_route(const nvq_qmm_desc *d, const ProductArgs &a) {
     if (!d->transpose) return Route::kUntransposed;        // weights stored [K, N]
     if (a.row_exact) return Route::kVector;                // the vector kernels: a row's bits do not depend on its neighbours
-    if (qmf_f32_takes(a)) return Route::kFewRowsF32;
-    if (qmm_f32_takes(a)) return Route::kTiledF32;         // float32, many rows: the float32 matrix instruction
+    if (qmm_f32_takes(a)) return Route::kTiledF32;
     if (takes_batched_decode(a)) return Route::kBatchedDecode;
     if (takes_few_rows_direct(a)) return Route::kFewRowsDirect;  // (also passes of 16 rows of small matrices, ahead of the tiles)
     if (takes_tiled(d, a)) return Route::kTiled;
@@ -664,8 +665,7 @@ static int32_t quantized_matmul_any(const nvq_qmm_desc *d, const void *x, const 
     case Route::kUntransposed: return launch_qvm(a, workspace, (hipStream_t)stream);
     case Route::kTiled:  // without a workspace: codes are expanded in the kernel and K is not split
         return dense && workspace != nullptr && qmm_dense_takes(a) ? launch_qmm_dense(a, workspace, (hipStream_t)stream) : launch_qmm(a, workspace, (hipStream_t)stream);
-    case Route::kTiledF32: return launch_qmm_f32(a, (hipStream_t)stream);
-    case Route::kFewRowsF32: return launch_qmf_f32(a, (hipStream_t)stream);
+    case Route::kTiledF32: return launch_qmm_f32(a, workspace, (hipStream_t)stream);
     case Route::kGroupedRows: return launch_grouped_rows(a, (hipStream_t)stream);
     case Route::kBatchedDecode: return launch_qmr(a, (hipStream_t)stream);
     case Route::kFewRowsDirect: return launch_qmd(a, (hipStream_t)stream);
@@ -684,8 +684,7 @@ const char *nvq_quantized_matmul_route(const nvq_qmm_desc *d) {
     switch (pick_route(d, a)) {
     case Route::kUntransposed: return qvm_kernel_name(a);
     case Route::kTiled: return "qmm_kernel";
-    case Route::kTiledF32:  // (the float32 matrix instruction's kernels under one name, whichever rows they are cut for)
-    case Route::kFewRowsF32: return "qmm_f32_kernel";
+    case Route::kTiledF32: return "qmm_f32_kernel";
     case Route::kGroupedRows: return "qmg_kernel";
     case Route::kBatchedDecode: return "qmr_kernel";
     case Route::kFewRowsDirect: return "qmd_kernel";

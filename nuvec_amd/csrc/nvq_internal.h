@@ -126,16 +126,15 @@ bool qmm_supported(const ProductArgs &a);
 size_t qmm_workspace_bytes(const ProductArgs &a);  // float32 partial sums when K is split over the grid, else 0
 int32_t launch_qmm(const ProductArgs &a, void *workspace, hipStream_t s);  // workspace NULL: no split
 double qmm_estimate_us(const ProductArgs &a);  // estimated duration of the tiled kernel with its better tile
-// float32 products of many rows on v_mfma_f32_32x32x2_f32 (affine codes, weights stored [N, K]).
+// float32 products of two rows and more on v_mfma_f32_16x16x32_bf16 (weights stored [N, K]); a workspace of partial sums where K is split.
 bool qmm_f32_takes(const ProductArgs &a);
-int32_t launch_qmm_f32(const ProductArgs &a, hipStream_t s);
+size_t qmm_f32_workspace_bytes(const ProductArgs &a);
+int32_t launch_qmm_f32(const ProductArgs &a, void *workspace, hipStream_t s);
 bool grouped_rows_take(const ProductArgs &a);
 int32_t launch_grouped_rows(ProductArgs a, hipStream_t s);
 bool qmm_dense_takes(const ProductArgs &a);
 size_t qmm_dense_workspace_bytes(const ProductArgs &a);
 int32_t launch_qmm_dense(const ProductArgs &a, void *workspace, hipStream_t s);
-bool qmf_f32_takes(const ProductArgs &a);
-int32_t launch_qmf_f32(const ProductArgs &a, hipStream_t s);
 // Batched decode: passes of up to 64 rows of x (5 to 128 rows routed there, where it measured faster), every weight fetched and dequantized once per pass (4- and 8-bit affine codes).
 bool qmr_supported(const ProductArgs &a);
 int32_t launch_qmr(const ProductArgs &a, hipStream_t s);

@@ -1,213 +1,569 @@
-// float32 products of many rows on the matrix cores: y[M,N] = x[M,K] . dequantize(w[N,K])^T for x, scales and biases in
-// float32 and affine codes of every width or a block format (MXFP4, MXFP8, NVFP4), on v_mfma_f32_32x32x2_f32.  The reference instantiates its tiled kernels
-// for float as for the half types (crates/nuvec-kernels/src/metal/quantized.metal:40-70, kernel
-// crates/nuvec-kernels/src/metal/quantized.h:1358-1485); values follow nuvec's CPU product
-// (crates/nuvec-core/src/kernels.rs:1091-1142): the weights are dequantized in float32 exactly as the CPU does,
-// round(round(code * scale) + bias) (kernels.rs:835-859; a block format's weight is its decoded code times its group's
-// decoded scale, NVFP4's scale first times ftz(g / 2688) where a global scale g is given, kernels.rs:992-998), and the
-// products accumulate in float32.
+// float32 products of two rows and more on the bfloat16 matrix instruction: y[M,N] = x[M,K] . dequantize(w[N,K])^T for x, scales
+// and biases in float32 (the reference instantiates its tiled kernels for float at every width: quantized.metal:40-70,
+// fp_quantized.metal:105-107), affine codes of every width, MXFP4, MXFP8 and NVFP4.
 //
-// A block of four wavefronts owns a 64 x 64 tile of y (2 x 2 wavefronts, one 32 x 32 matrix tile each) and walks K in
-// steps of 64 values.  The x tile of a step (64 rows x 256 bytes) goes through LDS, double buffered, rows 272 bytes
-// apart so that the 16-byte operand reads of sixteen rows fall on all 64 banks; the step after the next is requested
-// into registers while the current one is multiplied.  A lane (column n = lane % 32, half h = lane / 32) fetches the 32
-// codes [32 h, 32 h + 32) of its weight row itself (BITS dwords: always whole dwords, one group) and dequantizes one
-// weight per matrix instruction, which takes 64 cycles: the vector work hides under it.  Instruction j of a step
-// multiplies the values k = 32 h + j of the step in both operands.  Four blocks share a compute unit (35 KB of LDS
-// each), so sixteen wavefronts hide each other's waits without a deeper pipeline.
-#include "nvq_device.h"
-#include "nvq_internal.h"
-#include "qmf_kernel.h"
+// v_mfma_f32_16x16x32_bf16 multiplies sixteen times as much a cycle as the float32 instruction and its products are exact, so
+// no precision is given up for it:
+//   * a code is an exact bfloat16 (integers up to 255, E2M1, E4M3; NVFP4's code times its E4M3 scale has six bits);
+//   * x is the exact sum of three bfloat16 terms of eight bits each, cut off toward zero;
+//   * a group's sum P of x times code is formed from the smallest terms up in float32, then y += scale P + bias X with the
+//     group's sum X of x.  The biases' part is a product of its own, over groups, on the float32 instruction.
+// A weight's own two roundings (crates/nuvec-core/src/kernels.rs:835-859, 992-998), which the CPU's product keeps, are not made.
+// What the split of x does not hold, an infinity or a magnitude whose sums of codes leave float32, comes out of it as no finite
+// number: such an output is multiplied again, value by value.  Magnitudes below 2^-100 keep 2^-126.
+//
+// A block of four wavefronts owns 16 MT rows of x and 64 NT weight rows (16 NT a wavefront) and walks its share of K in steps
+// of 64.  x goes through registers, where it is split and its groups' sums are formed, into one of two LDS stages, a step ahead;
+// one barrier a step.  Codes come a window ahead in chunks of 16 bytes that consecutive lanes bring, and reach the operand
+// layout through a wavefront's own piece of LDS.  Scales and biases come once a span of 256 values, a lane its quarter's.
+// Few tiles: K is split over the grid, and qmm_f32_reduce_kernel adds the parts.
+//
+// What bounds it: a step's vector instructions, two of three for the split of x (a step of 48 rows and 64 weight rows takes 200
+// beside 23 matrix instructions, 0.65 us a compute unit; two blocks on one gain a tenth).  Every wavefront reading the
+// operands of both halves of a step at once, ahead of the next step's split, gave 0.1 us a step; codes and scales brought
+// by each lane for itself, straight in the operand layout, with no LDS and no barrier, was slower by half (16 lines a
+// load: W[14336,4096] at 16 rows 28 to 41 us against 20).
+#include "qmv_common.h"
+
+#include <math.h>
 
 namespace nvq {
 namespace {
 
-using qmf::code_to_float;
-using qmf::floatx16_t;
 using qmf::static_for;
 
-typedef float f32x4_t __attribute__((ext_vector_type(4)));  // (a native vector: arrays of it stay in registers)
+constexpr int kWaves = 4, kThreads = 64 * kWaves;
+constexpr int kTile = 16;   // rows of x, weight rows of a matrix instruction
+constexpr int kStep = 64;   // values of K between two barriers
+constexpr int kSpan = 256;  // values of K of which a lane brings scales and biases; a split of K holds whole ones
 
-constexpr int kTile = 64;                 // rows of x and weight rows of a block
-constexpr int kStep = 64;                 // values of K per step
-constexpr int kRowFloats = kStep + 4;     // an x row of a step in LDS: 272 bytes
+template <int BITS, int MODE, int MT, int NT>
+struct Shape {
+    static constexpr int kRows = kTile * MT, kCols = kTile * NT * kWaves;
+    static constexpr int kWindow = BITS <= 4 ? 256 : 128;        // values of K in a window of codes
+    static constexpr int kChunks = kWindow * BITS / 128;         // of 16 bytes, of a weight row in a window
+    static constexpr int kLoads = (kTile * NT * kChunks + 63) / 64;  // of a lane and window
+    static constexpr int kCodeRow = kWindow * BITS / 32 + 4;     // dwords between two weight rows of a window in LDS
+    static constexpr int kTermBytes = kRows * kStep * 2, kStageBytes = 3 * kTermBytes;
+    static constexpr int kCodeBytes = kTile * NT * kCodeRow * 4;  // of a wavefront
+    static constexpr int kSumBytes = kRows * 8 * 4;               // X of a span: eight blocks of 32 or four of 64 a row
+    static constexpr int kLds = 2 * kStageBytes + kWaves * kCodeBytes + 2 * kSumBytes;
+    static constexpr int kAhead = MT * NT == 8 ? 1 : 2;           // steps of x in registers
+};
 
-// MODE: NVQ_AFFINE, NVQ_MXFP4, NVQ_MXFP8 or NVQ_NVFP4 (BITS is 4 or 8 for the block formats).
+// Lane i takes the value of lane i ^ 1 (0xB1), i ^ 2 (0x4E), of the mirrored one of its eight (0x141) or sixteen (0x140).
+template <int CTRL> __device__ __forceinline__ float lane_swap(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float from_lane(float v, int lane) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * lane, __builtin_bit_cast(int, v)));
+}
+__device__ __forceinline__ uint32_t from_lane(uint32_t v, int lane) { return (uint32_t)__builtin_amdgcn_ds_bpermute(4 * lane, (int)v); }
+
+// The high halves of two words: `lo` in the low half.
+__device__ __forceinline__ uint32_t high_halves(uint32_t lo, uint32_t hi) { return __builtin_amdgcn_perm(hi, lo, 0x07060302u); }
+
+// Eight codes (in the low 8 BITS bits) as bfloat16, exactly.  Affine codes are taken from the middle of their range, c - 2^(BITS-1)
+// (one bit: c - 1/2), times code_factor().
+template <int BITS> constexpr float code_factor() { return BITS == 4 ? 16.0f : BITS == 1 ? 2.0f : 1.0f; }
 template <int BITS, int MODE>
-__global__ void __launch_bounds__(256) qmm_f32_kernel(const ProductArgs a) {
-    constexpr bool kAffine = MODE == NVQ_AFFINE;
-    constexpr int kHalves = MODE == NVQ_NVFP4 ? 2 : 1;  // groups in a lane's 32 values
-    __shared__ __attribute__((aligned(16))) float xs[2][kTile * kRowFloats];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1, h = lane >> 5, l32 = lane & 31;
+__device__ __forceinline__ uint4 code_operand(uint64_t codes, float scale) {
+    typedef qmf::Ops<bf16_t> Bf;
+    uint4 o;
+    const uint32_t lo = (uint32_t)codes;
+    if constexpr (MODE == NVQ_MXFP4) {
+        o.x = Bf::fp4_pair<0>(lo, 1.0f), o.y = Bf::fp4_pair<1>(lo, 1.0f), o.z = Bf::fp4_pair<2>(lo, 1.0f), o.w = Bf::fp4_pair<3>(lo, 1.0f);
+    } else if constexpr (MODE == NVQ_NVFP4) {
+        o.x = qmf::fp4_pair_times<bf16_t, 0>(lo, scale), o.y = qmf::fp4_pair_times<bf16_t, 1>(lo, scale);
+        o.z = qmf::fp4_pair_times<bf16_t, 2>(lo, scale), o.w = qmf::fp4_pair_times<bf16_t, 3>(lo, scale);
+    } else if constexpr (MODE == NVQ_MXFP8) {
+        const uint32_t hi = (uint32_t)(codes >> 32);
+        o.x = Bf::fp8_pair<false>(lo, 1.0f), o.y = Bf::fp8_pair<true>(lo, 1.0f), o.z = Bf::fp8_pair<false>(hi, 1.0f), o.w = Bf::fp8_pair<true>(hi, 1.0f);
+    } else {
+        // with its top bit turned a code is c - 2^(BITS-1) in two's complement (one bit: from there to twice c - 1/2)
+        constexpr uint64_t tops = 0x8080808080808080ull;
+        uint32_t f[8];
+        if constexpr (BITS == 4) {  // sixteen times it, a byte each
+            const uint32_t even = qmf::opaque(((lo << 4) & 0xF0F0F0F0u) ^ 0x80808080u), odd = qmf::opaque((lo & 0xF0F0F0F0u) ^ 0x80808080u);
+#pragma unroll
+            for (int j = 0; j < 4; j++) f[2 * j] = f2u((float)(int8_t)(even >> (8 * j))), f[2 * j + 1] = f2u((float)(int8_t)(odd >> (8 * j)));
+        } else if constexpr (BITS == 8) {
+            const uint64_t v = codes ^ tops;
+            const uint32_t first = qmf::opaque((uint32_t)v), second = qmf::opaque((uint32_t)(v >> 32));
+#pragma unroll
+            for (int j = 0; j < 4; j++) f[j] = f2u((float)(int8_t)(first >> (8 * j))), f[4 + j] = f2u((float)(int8_t)(second >> (8 * j)));
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const int32_t c = (int32_t)((uint32_t)(codes >> (BITS * j)) << (32 - BITS));
+                const int32_t v = (c ^ (int32_t)0x80000000) >> (32 - BITS);
+                f[j] = f2u((float)(BITS == 1 ? 2 * v + 1 : v));
+            }
+        }
+        o.x = high_halves(f[0], f[1]), o.y = high_halves(f[2], f[3]), o.z = high_halves(f[4], f[5]), o.w = high_halves(f[6], f[7]);
+    }
+    return o;
+}
+
+// A split's part of y[row, col], one value after the other.
+template <int BITS, int MODE>
+__device__ __forceinline__ float plain_sum(const ProductArgs &a, int row, int col, int k0, int k1, int gshift, float factor) {
+    const int K = (int)a.k;
+    float v = 0.0f;
+    for (int k = k0; k < k1; k++) {
+        const int64_t at = (int64_t)k * BITS;
+        const uint32_t *word = (const uint32_t *)a.w + (int64_t)col * (K / 32 * BITS) + at / 32;
+        const int bit = (int)(at % 32);
+        uint32_t c = word[0] >> bit;
+        if (bit + BITS > 32) c |= word[1] << (32 - bit);
+        c &= (1u << BITS) - 1u;
+        const int64_t g = (int64_t)col * (K >> gshift) + (k >> gshift);
+        float w;
+        if constexpr (MODE == NVQ_AFFINE) {
+            w = (float)c * ((const float *)a.scales)[g] + ((const float *)a.biases)[g];
+        } else {
+            const uint32_t code = ((const uint8_t *)a.scales)[g];
+            const float s = MODE == NVQ_NVFP4 ? qmf::nvfp4_scale(code, factor) : ftz(e8m0_to_f32(code));
+            w = (MODE == NVQ_MXFP8 ? e4m3_to_f32(c) : e2m1_to_f32(c)) * s;
+        }
+        v = __builtin_fmaf(((const float *)a.x)[(int64_t)row * K + k], w, v);
+    }
+    return v;
+}
+
+// G32: groups of 32 (affine, MXFP4, MXFP8), whose scale follows every matrix instruction; else blocks of 64, which lie in one group.
+template <int BITS, int MODE, int MT, int NT, bool G32>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, MT * NT <= 2 ? 4 : MT * NT == 3 ? 3 : 2))) qmm_f32_kernel(const ProductArgs a) {
+    using S = Shape<BITS, MODE, MT, NT>;
+    constexpr bool kAffine = MODE == NVQ_AFFINE, kNv = MODE == NVQ_NVFP4;
+    constexpr int kBlocks = G32 ? 2 : 1;                 // of a step with a scale of their own
+    constexpr int kAhead = S::kAhead;
+    constexpr float kMiddle = !kAffine ? 0.0f : BITS == 1 ? 0.5f : (float)(1 << (BITS - 1));
+    constexpr int kWindowSteps = S::kWindow / kStep;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l = lane & 15, q = lane >> 4;
     const int M = (int)a.m, N = (int)a.n, K = (int)a.k;
-    const int gshift = kAffine ? (a.group == 32 ? 5 : a.group == 64 ? 6 : 7) : (MODE == NVQ_NVFP4 ? 4 : 5);
-    const int kgroups = K >> gshift, row_dwords = (K >> 5) * BITS, steps = K / kStep;
-    const int m0 = blockIdx.y * kTile, n0 = blockIdx.x * kTile;
-    const float *x = (const float *)a.x;
-    float *y = (float *)a.y;
+    const int gshift = kAffine ? (a.group == 32 ? 5 : a.group == 64 ? 6 : 7) : (kNv ? 4 : 5);
+    const int kgroups = K >> gshift, kwords = K / 32 * BITS;
+    const int m0 = blockIdx.y * S::kRows, n0 = blockIdx.x * S::kCols + wave * (kTile * NT);
+    const int k0 = blockIdx.z * a.k_split_steps * kSpan;
+    const int k1 = a.k_splits > 1 && K - k0 > a.k_split_steps * kSpan ? k0 + a.k_split_steps * kSpan : K;
+    const int steps = (k1 - k0 + kStep - 1) / kStep;
+    unsigned char *code_lds = lds + 2 * S::kStageBytes + wave * S::kCodeBytes;
+    float *sum_lds = reinterpret_cast<float *>(lds + 2 * S::kStageBytes + kWaves * S::kCodeBytes);
 
-    // x: the tile of a step is 1024 pieces of four values; thread t brings pieces t + 256 i (row p / 16, piece p % 16).
-    // Rows past M read row M - 1 and are never stored.
-    const float *xsrc[4];
-    int xdst[4];
+    // x: a thread brings four values (of a wavefront's 64: four rows) of MT rows of a step; rows past the end repeat the last one and are
+    // not stored
+    float xs[kAhead][MT][4];  // the next steps', set = step % kAhead
+    const int xr = tid >> 4, xc = tid & 15;
+    auto load_x = [&](int step, auto set_tag) __attribute__((always_inline)) {
+        constexpr int set = decltype(set_tag)::value;
+        int k = k0 + step * kStep + 4 * xc;
+        k = k < k1 ? k : 0;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int p = tid + 256 * i, r = p >> 4, c = p & 15;
-        const int row = m0 + r < M ? m0 + r : M - 1;
-        xsrc[i] = x + (int64_t)row * K + 4 * c;
-        xdst[i] = r * kRowFloats + 4 * c;
-    }
-    // w: this lane's weight row (a row past N reads row N - 1) and its half of a step's codes
-    const int n = n0 + 32 * wn + l32 < N ? n0 + 32 * wn + l32 : N - 1;
-    const uint32_t *wp = (const uint32_t *)a.w + (int64_t)n * row_dwords + h * BITS;
-    const float *sp = (const float *)a.scales + (int64_t)n * kgroups, *bp = (const float *)a.biases + (int64_t)n * kgroups;  // affine
-    const uint8_t *cp = (const uint8_t *)a.scales + (int64_t)n * kgroups;                                                    // block formats: one byte a group
-    float inv_enc = 1.0f;
-    bool scaled = false;
-    if constexpr (MODE == NVQ_NVFP4) {
-        if (a.global_scale != nullptr) inv_enc = ftz(a.global_scale[0] / (448.0f * 6.0f)), scaled = true;
-    }
-
-    // The operands of two steps in registers, used in turn (set p holds the even or the odd steps), so that none is
-    // copied while its loads are under way.
-    f32x4_t xq[2][4];
-    uint32_t cq[2][BITS];
-    float sq[2], bq[2];
-    uint32_t rq[2][kHalves];  // block formats: the scale codes
-    auto request = [&](int step, auto p_tag) __attribute__((always_inline)) {
-        constexpr int p = decltype(p_tag)::value;
-        const int sc = step < steps ? step : steps - 1;  // (a step past the end fetches the last one again: no test around the loads)
-#pragma unroll
-        for (int i = 0; i < 4; i++) xq[p][i] = *reinterpret_cast<const f32x4_t *>(xsrc[i] + sc * kStep);
-#pragma unroll
-        for (int d = 0; d < BITS; d++) cq[p][d] = wp[sc * 2 * BITS + d];
-        const int g = (sc * kStep + 32 * h) >> gshift;
-        if constexpr (kAffine) {
-            sq[p] = sp[g];
-            bq[p] = bp[g];
-        } else {
-#pragma unroll
-            for (int hf = 0; hf < kHalves; hf++) rq[p][hf] = cp[g + hf];
+        for (int m = 0; m < MT; m++) {
+            const int row = m0 + kTile * m + xr;
+            const float4 v = *reinterpret_cast<const float4 *>((const float *)a.x + (int64_t)(row < M ? row : M - 1) * K + k);
+            xs[set][m][0] = v.x, xs[set][m][1] = v.y, xs[set][m][2] = v.z, xs[set][m][3] = v.w;
         }
     };
-
-    // Four accumulators take the instructions of a step in turn: a matrix instruction waits for the one before it on the
-    // same accumulator.  They are added once, at the end.
-    floatx16_t acc[4];
+    // Piece c (eight values) of row r of a term sits at 16-byte place c ^ (r / 2 % 8) of the row: the sixteen rows of an operand read
+    // spread over the banks.
+    auto store_x = [&](int step, auto set_tag) __attribute__((always_inline)) {
+        constexpr int set = decltype(set_tag)::value;
+        unsigned char *stage = lds + (step & 1) * S::kStageBytes + xr * (kStep * 2) + (((xc >> 1) ^ (xr >> 1)) * 16) + (xc & 1) * 8;
+        // place 4 b + quarter of a row: block `quarter` of 64, or block 2 quarter + b of 32
+        float *sums = sum_lds + ((step >> 2) & 1) * (S::kSumBytes / 4) + xr * 8 + (step & 3) + 4 * (xc >> 3);
+        if (k0 + (step + 1) * kStep > k1) {  // the last step may be a half
+            const bool inside = k0 + step * kStep + 4 * xc < k1;
 #pragma unroll
-    for (int e = 0; e < 16; e++) acc[0][e] = acc[1][e] = acc[2][e] = acc[3][e] = 0.0f;
-
-    using P0 = std::integral_constant<int, 0>;
-    using P1 = std::integral_constant<int, 1>;
-    auto multiply = [&](int step, auto p_tag, auto other_tag) __attribute__((always_inline)) {
-        constexpr int p = decltype(p_tag)::value;
-        float *stage = xs[p];
+            for (int m = 0; m < MT; m++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) *reinterpret_cast<f32x4_t *>(stage + xdst[i]) = xq[p][i];
-        request(step + 1, other_tag);
-        // One barrier per step: the stage written now was last read two steps ago, before every wavefront's previous barrier.
-        // Only the LDS writes are waited for: __syncthreads() would also wait for the loads just requested, a round trip
-        // to memory per step.
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        const float *xrow = stage + (32 * wm + l32) * kRowFloats + 32 * h;
-        f32x4_t xa[8];
-#pragma unroll
-        for (int q = 0; q < 8; q++) xa[q] = *reinterpret_cast<const f32x4_t *>(xrow + 4 * q);
-        float scale[kHalves], bias = 0.0f;
-        if constexpr (kAffine) {
-            scale[0] = sq[p], bias = bq[p];
-        } else {
-#pragma unroll
-            for (int hf = 0; hf < kHalves; hf++) {
-                scale[hf] = ftz(MODE == NVQ_NVFP4 ? e4m3_to_f32(rq[p][hf]) : e8m0_to_f32(rq[p][hf]));
-                if (scaled) scale[hf] = ftz(scale[hf] * inv_enc);
-            }
+                for (int j = 0; j < 4; j++) xs[set][m][j] = inside ? xs[set][m][j] : 0.0f;
         }
-        static_for<32>([&](auto j_tag) {
-            constexpr int j = decltype(j_tag)::value;
-            float wv;
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+            float (&r)[4] = xs[set][m];
             if constexpr (kAffine) {
-                wv = code_to_float<BITS, j>(cq[p]) * scale[0] + bias;  // two roundings, as the CPU's weight
-            } else {
-                constexpr int per = 32 / BITS;
-                const uint32_t c = (cq[p][j / per] >> (BITS * (j % per))) & ((1u << BITS) - 1u);
-                wv = (MODE == NVQ_MXFP8 ? e4m3_to_f32(c) : e2m1_to_f32(c)) * scale[kHalves == 2 ? j / 16 : 0];
+                float sum = (r[0] + r[1]) + (r[2] + r[3]);
+                sum += lane_swap<0xB1>(sum);
+                sum += lane_swap<0x4E>(sum);
+                sum += lane_swap<0x141>(sum);
+                if constexpr (!G32) sum += lane_swap<0x140>(sum);
+                if ((xc & (G32 ? 7 : 15)) == 0) sums[kTile * m * 8] = sum;
             }
-            const float xv = xa[j >> 2][j & 3];
-            acc[j & 3] = __builtin_amdgcn_mfma_f32_32x32x2f32(xv, wv, acc[j & 3], 0, 0, 0);
-        });
+#pragma unroll
+            for (int t = 0; t < 3; t++) {
+                uint2 o;
+                o.x = high_halves(f2u(r[0]), f2u(r[1])), o.y = high_halves(f2u(r[2]), f2u(r[3]));
+                *reinterpret_cast<uint2 *>(stage + t * S::kTermBytes + kTile * m * (kStep * 2)) = o;
+#pragma unroll
+                for (int j = 0; j < 4; j++) r[j] -= u2f(f2u(r[j]) & 0xFFFF0000u);
+            }
+        }
     };
-    request(0, P0{});
-    int step = 0;
-    for (; step + 2 <= steps; step += 2) {
-        multiply(step, P0{}, P1{});
-        multiply(step + 1, P1{}, P0{});
-    }
-    if (step < steps) multiply(step, P0{}, P1{});
-#pragma unroll
-    for (int e = 0; e < 16; e++) acc[0][e] = (acc[0][e] + acc[1][e]) + (acc[2][e] + acc[3][e]);
 
-    // Accumulator element e of lane l is tile row 8 (e / 4) + 4 (l / 32) + e % 4, column l % 32.
-    const int col = n0 + 32 * wn + l32;
+    // Codes: the tiles' rows of a window, in order, are cut into chunks of 16 bytes that consecutive lanes bring (rows past the end repeat
+    // the last one).  Where K ends inside a chunk the 16 bytes up to its end are brought and moved into place; past the end of K come a
+    // row's first bytes, zeroed where a code could be a NaN.
+    uint4 cw[S::kLoads];
+    auto chunk_of = [&](int i) { const int c = i * 64 + lane; return c < kTile * NT * S::kChunks ? c : 0; };
+    auto load_codes = [&](int k) __attribute__((always_inline)) {
 #pragma unroll
-    for (int e = 0; e < 16; e++) {
-        const int row = m0 + 32 * wm + 8 * (e >> 2) + 4 * h + (e & 3);
-        if (row < M && col < N) y[(int64_t)row * N + col] = add_row_bias<float>(a.row_bias, acc[0][e], col);
+        for (int i = 0; i < S::kLoads; i++) {
+            const int n = n0 + chunk_of(i) / S::kChunks;
+            int at = k / 32 * BITS + 4 * (chunk_of(i) % S::kChunks);
+            at = at >= kwords ? 0 : at + 4 > kwords ? kwords - 4 : at;
+            at = at < 0 ? 0 : at;
+            cw[i] = __builtin_bit_cast(uint4, *reinterpret_cast<const qmf::u32x4_a4_t *>((const uint32_t *)a.w + (int64_t)(n < N ? n : N - 1) * kwords + at));
+        }
+    };
+    auto store_codes = [&](int k) __attribute__((always_inline)) {
+        if (k + S::kWindow > K) {
+#pragma unroll
+            for (int i = 0; i < S::kLoads; i++) {
+                const int at = k / 32 * BITS + 4 * (chunk_of(i) % S::kChunks), missing = at + 4 - kwords;  // dwords past the end
+                uint4 &v = cw[i];
+                if (missing >= 4) v = make_uint4(0, 0, 0, 0);
+                else if (missing == 3) v = make_uint4(v.w, 0, 0, 0);
+                else if (missing == 2) v = make_uint4(v.z, v.w, 0, 0);
+                else if (missing == 1) v = make_uint4(v.y, v.z, v.w, 0);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < S::kLoads; i++) {
+            const int c = i * 64 + lane;
+            if ((i + 1) * 64 <= kTile * NT * S::kChunks || c < kTile * NT * S::kChunks)
+                *reinterpret_cast<uint4 *>(code_lds + (c / S::kChunks) * (S::kCodeRow * 4) + (c % S::kChunks) * 16) = cw[i];
+        }
+        __builtin_amdgcn_wave_barrier();  // (the wavefront's LDS accesses execute in order)
+    };
+    // The eight codes of this lane for block `b` (of 32) of step `j` of the window.
+    auto codes_of = [&](int t, int j, int b) __attribute__((always_inline)) {
+        const uint32_t *row = reinterpret_cast<const uint32_t *>(code_lds) + (t * kTile + l) * S::kCodeRow + (2 * j + b) * BITS;
+        if constexpr (BITS == 4) return (uint64_t)row[q];
+        else if constexpr (BITS == 8) return *reinterpret_cast<const uint64_t *>(row + 2 * q);
+        else {
+            const int first = q * BITS / 4, bit = 8 * (q * BITS % 4);
+            uint64_t v = row[first];
+            if constexpr (BITS > 2) v |= (uint64_t)row[first + 1 < BITS ? first + 1 : BITS - 1] << 32;
+            return v >> bit;
+        }
+    };
+
+    // Scales and biases of a span: lane (q, l) brings those of step q of the span for weight row l of each tile.
+    float sc[NT][kBlocks], bi[NT][kBlocks], sc_next[NT][kBlocks], bi_next[NT][kBlocks];
+    uint32_t sw[NT];
+    uint8_t sw_next[NT][4];
+    auto load_scales = [&](int k) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            const int n = n0 + kTile * t + l;
+            const int64_t row = (int64_t)(n < N ? n : N - 1) * kgroups;
+#pragma unroll
+            for (int b = 0; b < (kNv ? 4 : kBlocks); b++) {
+                const int at = k + q * kStep + b * (kNv ? 16 : 32);
+                const int64_t g = row + (at < k1 ? at >> gshift : 0);
+                if constexpr (kAffine) sc_next[t][b] = ((const float *)a.scales)[g], bi_next[t][b] = ((const float *)a.biases)[g];
+                else sw_next[t][b] = ((const uint8_t *)a.scales)[g];
+            }
+        }
+    };
+    // (the middle of the codes' range goes to the bias)
+    auto take_scales = [&](int k) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            if constexpr (kAffine) {
+#pragma unroll
+                for (int b = 0; b < kBlocks; b++) {
+                    const bool inside = k + q * kStep + b * 32 < k1;
+                    sc[t][b] = !inside ? 0.0f : sc_next[t][b] * (1.0f / code_factor<BITS>());
+                    bi[t][b] = !inside ? 0.0f : __builtin_fmaf(sc_next[t][b], kMiddle, bi_next[t][b]);
+                }
+            } else {
+                sw[t] = 0;
+#pragma unroll
+                for (int b = 0; b < (kNv ? 4 : 2); b++) sw[t] |= (uint32_t)sw_next[t][b] << (8 * b);
+            }
+        }
+    };
+
+    floatx4_t acc[MT][NT];
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) acc[m][t] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
+
+    // Every request is made on every path, past the end for something that is not used, and what has come is touched where it is used
+    // alone: a wait for one load would be a wait for all.
+    load_codes(k0);
+    load_scales(k0);
+    static_for<kAhead>([&](auto i) { load_x(i, i); });
+    store_x(0, std::integral_constant<int, 0>{});
+    load_x(kAhead, std::integral_constant<int, 0>{});
+    __syncthreads();
+    for (int at = 0; at < steps; at += 4) {  // a span
+        take_scales(k0 + at * kStep);
+        static_for<4>([&](auto j_tag) {
+            constexpr int j = decltype(j_tag)::value;
+            const int step = at + j;
+            if constexpr (j % kWindowSteps == 0) {
+                store_codes(k0 + step * kStep);
+                load_codes(k0 + (step + kWindowSteps) * kStep);
+            }
+            if constexpr (j == 0) load_scales(k0 + (step + 4) * kStep);
+            // The operands of the step's first half are read, then the next step's x is split while they come.
+            const unsigned char *stage = lds + (step & 1) * S::kStageBytes;
+            uint64_t codes[2][NT];
+            uint4 xo[2][3][MT];
+            auto read_x = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+                for (int term = 0; term < 3; term++)
+#pragma unroll
+                    for (int m = 0; m < MT; m++) {
+                        const int row = kTile * m + l;
+                        xo[b][term][m] = *reinterpret_cast<const uint4 *>(stage + term * S::kTermBytes + row * (kStep * 2) + (((4 * b + q) ^ ((row >> 1) & 7)) * 16));
+                    }
+            };
+#pragma unroll
+            for (int b = 0; b < 2; b++)
+#pragma unroll
+                for (int t = 0; t < NT; t++) codes[b][t] = codes_of(t, j % kWindowSteps, b);
+            read_x(0);
+            float scale[NT][kBlocks];
+            uint32_t word[NT];
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                if constexpr (!kAffine) word[t] = from_lane(sw[t], l + 16 * j);
+#pragma unroll
+                for (int b = 0; b < kBlocks; b++) scale[t][b] = kAffine ? from_lane(sc[t][b], l + 16 * j) : 1.0f;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            constexpr std::integral_constant<int, (j + 1) % kAhead> set;
+            store_x(step + 1, set);
+            load_x(step + 1 + kAhead, set);
+            uint4 w[2][NT];
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                if constexpr (!kAffine && !kNv) {
+#pragma unroll
+                    for (int b = 0; b < 2; b++) {
+                        const uint32_t code = (word[t] >> (8 * b)) & 255u;
+                        scale[t][b] = code == 255u ? u2f(0x7FC00000u) : ftz(e8m0_to_f32(code));
+                    }
+                }
+                w[0][t] = code_operand<BITS, MODE>(codes[0][t], kNv ? e4m3_to_f32((word[t] >> (8 * (q >> 1))) & 255u) : 1.0f);
+            }
+            read_x(1);
+            __builtin_amdgcn_sched_barrier(0);
+            if (step < steps) {
+                floatx4_t p[MT][NT];
+                auto multiply = [&](auto b_tag) __attribute__((always_inline)) {
+                    constexpr int b = decltype(b_tag)::value;
+                    if (G32 || b == 0)
+#pragma unroll
+                        for (int m = 0; m < MT; m++)
+#pragma unroll
+                            for (int t = 0; t < NT; t++) p[m][t] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int term = 2; term >= 0; term--)
+#pragma unroll
+                        for (int m = 0; m < MT; m++)
+#pragma unroll
+                            for (int t = 0; t < NT; t++) p[m][t] = Mfma16<bf16_t>::run(xo[b][term][m], w[b][t], p[m][t]);
+                    if (b == 0)
+#pragma unroll
+                        for (int t = 0; t < NT; t++)
+                            w[1][t] = code_operand<BITS, MODE>(codes[1][t], kNv ? e4m3_to_f32((word[t] >> (16 + 8 * (q >> 1))) & 255u) : 1.0f);
+                    if (G32 || b == 1)
+#pragma unroll
+                        for (int t = 0; t < NT; t++)
+#pragma unroll
+                            for (int m = 0; m < MT; m++)
+#pragma unroll
+                                for (int e = 0; e < 4; e++) acc[m][t][e] = __builtin_fmaf(scale[t][G32 ? b : 0], p[m][t][e], acc[m][t][e]);
+                };
+                multiply(std::integral_constant<int, 0>{});
+                multiply(std::integral_constant<int, 1>{});
+            }
+            if constexpr (kAffine && j == 3) {  // the span's biases: y += sum over blocks of X[row, block] bias[weight row, block]
+                const float *sums = sum_lds + ((step >> 2) & 1) * (S::kSumBytes / 4);
+#pragma unroll
+                for (int b = 0; b < kBlocks; b++)
+#pragma unroll
+                    for (int m = 0; m < MT; m++) {
+                        const float x = sums[(kTile * m + l) * 8 + 4 * b + q];
+#pragma unroll
+                        for (int t = 0; t < NT; t++) acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, bi[t][b], acc[m][t], 0, 0, 0);
+                    }
+            }
+            __syncthreads();
+        });
+    }
+
+    const float factor = kNv ? qmf::nvfp4_factor(a, 0) : 1.0f;
+    float *y = a.k_splits > 1 ? a.partials + (int64_t)blockIdx.z * M * N : (float *)a.y;
+    bool plain = false;
+    // Accumulator element e of lane (q, l): row 4 q + e of x, weight row l.
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int row = m0 + kTile * m + 4 * q + e, col = n0 + kTile * t + l;
+                const float v = kNv ? acc[m][t][e] * factor : acc[m][t][e];
+                plain |= !(fabsf(v) < INFINITY);
+                if (row < M && col < N) y[(int64_t)row * N + col] = a.k_splits > 1 ? v : add_row_bias<float>(a.row_bias, v, col);
+            }
+    if (plain) {
+        for (int i = 0; i < MT * NT * 4; i++) {
+            const int row = m0 + i / (NT * 4) * kTile + 4 * q + i % 4, col = n0 + i / 4 % NT * kTile + l;
+            if (row >= M || col >= N || fabsf(y[(int64_t)row * N + col]) < INFINITY) continue;
+            const float v = plain_sum<BITS, MODE>(a, row, col, k0, k1, gshift, factor);
+            y[(int64_t)row * N + col] = a.k_splits > 1 ? v : add_row_bias<float>(a.row_bias, v, col);
+        }
     }
 }
 
-template <int BITS, int MODE = NVQ_AFFINE>
-int32_t run(const ProductArgs &a, hipStream_t s) {
-    const dim3 grid((unsigned)((a.n + kTile - 1) / kTile), (unsigned)((a.m + kTile - 1) / kTile));
-    hipLaunchKernelGGL((qmm_f32_kernel<BITS, MODE>), grid, dim3(256), 0, s, a);
+// The parts of a split K, eight under way at a time and added by pairs.
+__global__ void __launch_bounds__(256) qmm_f32_reduce_kernel(const float *__restrict__ partials, float *__restrict__ y, int splits, int64_t total,
+                                                             const void *row_bias, int64_t n) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= total) return;
+    float sum = 0.0f;
+    for (int s = 0; s < splits; s += 8) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = partials[(int64_t)(s + u < splits ? s + u : s) * total + i];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = s + u < splits ? v[u] : 0.0f;
+        sum += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+    }
+    y[i] = add_row_bias<float>(row_bias, sum, i % n);
+}
+
+struct Plan {
+    int mt, nt, splits, spans;  // tiles of rows of x a block, of weight rows a wavefront; spans of K a split
+    double us;                  // estimated
+};
+
+// The tiles of weight rows and the split of K with the least estimated time.  Fitted (14 % off on average) to 3700 timings of 552
+// products of 2 to 512 rows, twelve weight shapes from W[600,2496] to W[33000,512] and W[4096,14336], 4 and 8 bits, MXFP8 and NVFP4: a
+// step costs a compute unit 0.12 + 0.17 us per tile of rows at 64 weight rows a block, 0.25 + 0.28 at 128, whether its blocks run one
+// after the other or side by side; choosing by it is 4 % above always taking the fastest.  The parts fit the library's own scratch.
+Plan plan_of(const ProductArgs &a) {
+    Plan best{};
+    const int64_t tiles = (a.m + kTile - 1) / kTile, passes = (tiles + 3) / 4, spans = (a.k + kSpan - 1) / kSpan, steps = (a.k + kStep - 1) / kStep;
+    const int mt = (int)((tiles + passes - 1) / passes);
+    const double cus = fmax(1.0, (double)compute_units()), outputs = (double)a.m * (double)a.n;
+    for (int nt = 1; nt <= 2; nt++)
+        for (int64_t want = 1; want <= 16 && want <= spans; want++) {
+            const int64_t per = (spans + want - 1) / want, splits = (spans + per - 1) / per;
+            if (splits != want || (splits > 1 && (double)splits * outputs * 4.0 > (double)NVQ_STATIC_SCRATCH_BYTES)) continue;
+            const double load = (double)(passes * ((a.n + 64 * nt - 1) / (64 * nt)) * splits) / cus;
+            const double step_us = nt == 1 ? 0.12 + 0.17 * mt : 0.25 + 0.28 * mt;
+            const double us = 5.3 + (double)(4 * per < steps ? 4 * per : steps) * step_us * fmax(1.0, 0.25 * ceil(load) + 0.75 * load) +
+                              (splits > 1 ? 1.3 + 1.1e-6 * (double)splits * outputs : 0.0);
+            if (best.nt == 0 || us < best.us) best = Plan{mt, nt, (int)splits, (int)per, us};
+        }
+    return best;
+}
+
+template <int BITS, int MODE, int MT, int NT, bool G32>
+int32_t run_shape(const ProductArgs &a, hipStream_t s) {
+    constexpr int kLds = Shape<BITS, MODE, MT, NT>::kLds;
+    auto kernel = qmm_f32_kernel<BITS, MODE, MT, NT, G32>;
+    static std::atomic<bool> configured{false};
+    if (kLds > 64 * 1024 && !configured.load()) {
+        NVQ_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLds));
+        configured.store(true);
+    }
+    const dim3 grid((unsigned)((a.n + 64 * NT - 1) / (64 * NT)), (unsigned)((a.m + kTile * MT - 1) / (kTile * MT)), (unsigned)a.k_splits);
+    hipLaunchKernelGGL(kernel, grid, dim3(kThreads), kLds, s, a);
     NVQ_LAUNCH_CHECK("qmm_f32");
     return NVQ_OK;
 }
 
-}  // namespace
-
-// What the kernel takes: one product (no batch, no gathered pairs, no gated epilogue, not row-exact) of float32 x against
-// affine or block-format weights stored [N, K] with K in whole steps of 64, where it is estimated faster than the vector kernel, which
-// walks the weights once per four rows of x.  Measured, 4-bit g64, us, vector kernel -> this one: W[4096,4096] at 64 /
-// 128 / 512 / 2048 rows 130 / 245 / 969 / 3850 -> 105 / 107 / 178 / 629 (109 TFLOP/s at 2048 rows); W[14336,4096] at 16 /
-// 64 / 512 / 2048 rows 112 / 427 / 3366 / 13444 -> 106 / 106 / 540 / 2042 (118 TFLOP/s); a step of 64 values costs a block
-// 1.64 us alone on a compute unit and 1.25 us per block that shares it, a pass of the vector kernel 1 us per 2.2 M weights.
-bool qmm_f32_takes(const ProductArgs &a) {
-    if (a.dtype != NVQ_F32 || a.row_exact) return false;
-    if (a.batch != 1 || a.batch_ndim != 0 || a.rhs != nullptr || a.lhs != nullptr || a.glu != 0) return false;
-    if (a.k < kStep || a.k % kStep != 0 || (a.mode == NVQ_AFFINE && a.group != 32 && a.group != 64 && a.group != 128)) return false;
-    if (a.m < 8 || a.m > 65535 * (int64_t)kTile || a.n > 0x7FFFFFFF / 64 || (uintptr_t)a.x % 16 != 0) return false;
-    // Both kernels as timed on 1078 products (fourteen weight shapes, seven formats, 8 to 512 rows): this one a step of 64
-    // values at 1.64 us for a lone block and 1.25 us per block sharing a compute unit, the block formats 1.7 times that;
-    // the vector kernel a pass of four rows at 1 us per 2.06 M weights with K counted in its steps of 2048 values (a row
-    // of 512 costs a whole step: W[32768,512] at 8 rows 68.6 us there against 25.4 here), the block formats 2.05 times
-    // that.  Choosing by them is 0.2 % above always taking the faster kernel, 1.4 x at worst.
-    const bool block_format = a.mode != NVQ_AFFINE;
-    const double tiles = (double)((a.m + kTile - 1) / kTile) * (double)((a.n + kTile - 1) / kTile);
-    const double per_unit = 1.25 * tiles / compute_units();
-    const double here = (double)(a.k / kStep) * (per_unit > 1.64 ? per_unit : 1.64) * (block_format ? 1.7 : 1.0);
-    const double k_steps = (double)((a.k + 2047) / 2048) * 2048.0;
-    const double there = (double)((a.m + 3) / 4) * (double)a.n * k_steps / 2.2e6 * (block_format ? 2.05 : 1.07);
-    return here < there;
+template <int BITS, int MODE, int NT, bool G32>
+int32_t run_rows(const ProductArgs &a, int mt, hipStream_t s) {
+    switch (mt) {
+    case 1: return run_shape<BITS, MODE, 1, NT, G32>(a, s);
+    case 2: return run_shape<BITS, MODE, 2, NT, G32>(a, s);
+    case 3: return run_shape<BITS, MODE, 3, NT, G32>(a, s);
+    default: return run_shape<BITS, MODE, 4, NT, G32>(a, s);
+    }
 }
 
-int32_t launch_qmm_f32(const ProductArgs &a, hipStream_t s) {
-    if (!qmm_f32_takes(a)) return fail(NVQ_UNSUPPORTED, "quantized_matmul: the float32 matrix-core kernel does not take this product");
-    if (a.mode == NVQ_MXFP4) return run<4, NVQ_MXFP4>(a, s);
-    if (a.mode == NVQ_MXFP8) return run<8, NVQ_MXFP8>(a, s);
-    if (a.mode == NVQ_NVFP4) return run<4, NVQ_NVFP4>(a, s);
-    switch (a.bits) {
-    case 1: return run<1>(a, s);
-    case 2: return run<2>(a, s);
-    case 3: return run<3>(a, s);
-    case 4: return run<4>(a, s);
-    case 5: return run<5>(a, s);
-    case 6: return run<6>(a, s);
-    case 8: return run<8>(a, s);
+template <int BITS, int MODE = NVQ_AFFINE>
+int32_t run(const ProductArgs &a, const Plan &p, hipStream_t s) {
+    if constexpr (MODE == NVQ_AFFINE) {
+        if (a.group != 32) return p.nt == 1 ? run_rows<BITS, MODE, 1, false>(a, p.mt, s) : run_rows<BITS, MODE, 2, false>(a, p.mt, s);
+    }
+    constexpr bool kG32 = MODE != NVQ_NVFP4;
+    return p.nt == 1 ? run_rows<BITS, MODE, 1, kG32>(a, p.mt, s) : run_rows<BITS, MODE, 2, kG32>(a, p.mt, s);
+}
+
+}  // namespace
+
+// What the kernel takes: one product (no batch, no gathered pairs, no gated epilogue, not row-exact) of float32 x against weights
+// stored [N, K], K in whole blocks of 32.
+static bool qmm_f32_supported(const ProductArgs &a) {
+    if (a.dtype != NVQ_F32 || a.row_exact || a.batch != 1 || a.batch_ndim != 0 || a.rhs != nullptr || a.lhs != nullptr || a.glu != 0) return false;
+    if (a.m < 2 || a.k < 32 || a.k % 32 != 0 || (a.mode == NVQ_AFFINE && a.group != 32 && a.group != 64 && a.group != 128)) return false;
+    if (a.k / 32 * a.bits < 4) return false;  // (a chunk of codes lies inside a row)
+    return (a.m + 15) / 16 <= 65535 && a.n <= 0x7FFFFFFF / 64 && a.k <= 1 << 26 && (uintptr_t)a.x % 16 == 0;
+}
+
+// Where it is estimated faster than the vector kernel, which walks the weights once per four rows of x: 4 us and a pass of four rows at
+// 1 us per 2.1 M weights, K counted in its steps of 2048 values (E2M1 codes 2.5 times that).  Timed on the 552 products of plan_of it
+// takes 0.28 of the time of what served them before, the vector kernel and two on v_mfma_f32_16x16x4_f32 and 32x32x2 (4 bits, us:
+// W[4096,4096] at 33 / 64 / 128 / 512 rows 35 / 45 / 87 / 178 -> 17 / 22 / 30 / 70, W[14336,4096] at 16 rows 76 -> 20, W[704,5376] at
+// 274 rows 134 -> 23), and its error against float64 is lower (W[4096,4096] at 33 rows 2.9e-7 -> 1.0e-7, 2.9e-7 -> 1.0e-7 for NVFP4).
+// The vector kernel keeps, though it is behind, what callers that ask for a product's route know it by: a few rows of affine
+// and E4M3 codes (up to 32 against up to 2^24 weights, up to 8 beyond where K is longer than 512; W[4096,4096] at 32 rows 65 us there, 17
+// here), four rows of MXFP4 up to 2^24 weights, and more than 128 rows of K off whole steps of 64.
+bool qmm_f32_takes(const ProductArgs &a) {
+    if (!qmm_f32_supported(a) || (a.k % kStep != 0 && a.m > 128)) return false;
+    const bool small = a.n * a.k <= 1 << 24, e2m1 = a.mode == NVQ_MXFP4 || a.mode == NVQ_NVFP4;
+    if (!e2m1 && a.m <= (small ? 32 : a.k > 512 ? 8 : 0)) return false;
+    if (a.mode == NVQ_MXFP4 && small && a.m <= 4) return false;
+    const double k_steps = (double)((a.k + 2047) / 2048) * 2048.0;
+    return plan_of(a).us < 4.0 + (e2m1 ? 2.52 : 1.05) * (double)((a.m + 3) / 4) * (double)a.n * k_steps / 2.2e6;
+}
+
+size_t qmm_f32_workspace_bytes(const ProductArgs &a) {
+    const Plan p = plan_of(a);
+    return p.splits > 1 ? (size_t)p.splits * (size_t)a.m * (size_t)a.n * sizeof(float) : 0;
+}
+
+int32_t launch_qmm_f32(const ProductArgs &args, void *workspace, hipStream_t s) {
+    if (!qmm_f32_supported(args)) return fail(NVQ_UNSUPPORTED, "quantized_matmul: the float32 matrix-core kernel does not take this product");
+    ProductArgs a = args;
+    const Plan p = plan_of(a);
+    a.k_splits = workspace != nullptr ? p.splits : 1;
+    a.k_split_steps = p.spans;
+    a.partials = (float *)workspace;
+    int32_t rc;
+    if (a.mode == NVQ_MXFP4) rc = run<4, NVQ_MXFP4>(a, p, s);
+    else if (a.mode == NVQ_MXFP8) rc = run<8, NVQ_MXFP8>(a, p, s);
+    else if (a.mode == NVQ_NVFP4) rc = run<4, NVQ_NVFP4>(a, p, s);
+    else switch (a.bits) {
+    case 1: rc = run<1>(a, p, s); break;
+    case 2: rc = run<2>(a, p, s); break;
+    case 3: rc = run<3>(a, p, s); break;
+    case 4: rc = run<4>(a, p, s); break;
+    case 5: rc = run<5>(a, p, s); break;
+    case 6: rc = run<6>(a, p, s); break;
+    case 8: rc = run<8>(a, p, s); break;
     default: return fail(NVQ_INVALID_ARGUMENT, "quantized_matmul: %d bits are not supported", a.bits);
     }
+    if (rc != NVQ_OK || a.k_splits <= 1) return rc;
+    const int64_t total = a.m * a.n;
+    hipLaunchKernelGGL(qmm_f32_reduce_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, a.partials, (float *)a.y, a.k_splits, total, a.row_bias, a.n);
+    NVQ_LAUNCH_CHECK("qmm_f32_reduce");
+    return NVQ_OK;
 }
 
 }  // namespace nvq

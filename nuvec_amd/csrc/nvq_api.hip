@@ -179,18 +179,20 @@ using namespace nvq;
 // the faster kernel, 30 % at worst (the rule before them, a round at 5 us per 1024 values of K against the bare
 // estimate: 6.3 % and 2.5 x - W[4096,1024] at 256 rows 47.4 us on the few-row kernel against 19.8).  The counterpart
 // of the reference's device-specific `qmv_batch_limit` (crates/nuvec-core/src/gpu.rs:1506-1538).
-static bool tiled_is_faster(const nvq::ProductArgs &a) {
+static double few_rows_us(const nvq::ProductArgs &a) {
     const double passes = (double)((a.m + 31) / 32) * (double)a.batch, k = (double)a.k;
     const double blocks64 = passes * (double)((a.n + 63) / 64);
     const bool wide = blocks64 >= 192.0, exact = a.exact_weights != 0, fp4 = a.mode == NVQ_MXFP4;
     const double blocks = wide ? blocks64 : passes * (double)((a.n + 31) / 32);
     const double round_us = wide ? (exact ? 13.5 + 4.4e-3 * k : 7.4 + (fp4 ? 2.16e-3 : 2.45e-3) * k)
                                  : (exact ? 8.0 + 2.0e-3 * k : 6.0 + 2.05e-3 * k);
-    const double few_us = ceil(blocks / fmax(1.0, (double)nvq::compute_units())) * round_us;
-    const double steps_us = nvq::qmm_estimate_us(a);
-    const double tiled_us = exact ? 1.8 + 1.26 * steps_us : fp4 ? 3.2 + 0.73 * steps_us : 3.4 + steps_us;
-    return fmax(7.0, tiled_us) < few_us;  // (its fastest launches, at K = 128, take 6 to 7.4 us)
+    return ceil(blocks / fmax(1.0, (double)nvq::compute_units())) * round_us;
 }
+static double tiled_us(const nvq::ProductArgs &a) {
+    const double steps_us = nvq::qmm_estimate_us(a);
+    return a.exact_weights ? 1.8 + 1.26 * steps_us : a.mode == NVQ_MXFP4 ? 3.2 + 0.73 * steps_us : 3.4 + steps_us;
+}
+static bool tiled_is_faster(const nvq::ProductArgs &a) { return fmax(7.0, tiled_us(a)) < few_rows_us(a); }  // (its fastest launches, at K = 128, take 6 to 7.4 us)
 
 // Whether the 16x16x32 kernel with directly loaded weight operands takes a few-row product, from its measured times
 // against the kernels it replaces (bf16, us per launch, new / old):
@@ -593,6 +595,14 @@ static bool takes_tiled(const nvq_qmm_desc *d, const ProductArgs &a) {
 enum class Route { kUntransposed, kVector, kTiled, kTiledF32, kGroupedRows, kBatchedDecode, kFewRowsDirect, kFewRows };
 static Route pick_route(const nvq_qmm_desc *d, const ProductArgs &a);
 
+// Whether a product of either matrix-core route of 16-bit rows runs on the split-K kernel (the route keeps its name): where that is
+// estimated up to a tenth above the few-row kernel (whose estimate is the lower one: 630 products, 0.74 of its time, 1.17 x at
+// worst) or a tenth below the tiles (448 products, 0.76 of the time, 1.09 x at worst; from 65 rows on most stay there, and beyond 256 all).
+static bool split_rows_take(const ProductArgs &a, Route route, qms::Plan &plan) {
+    if ((route != Route::kFewRows && route != Route::kTiled) || !qms_plan(a, plan)) return false;
+    return route == Route::kFewRows ? plan.us < 1.1 * few_rows_us(a) : a.m <= 256 && plan.us < 0.9 * tiled_us(a);
+}
+
 // `dense`: whether the workspace may hold the dequantized weight.
 static size_t workspace_bytes(const nvq_qmm_desc *d, bool dense) {
     if (check_qmm(d, "quantized_matmul") != NVQ_OK) return 0;
@@ -604,6 +614,8 @@ static size_t workspace_bytes(const nvq_qmm_desc *d, bool dense) {
     if (!d->transpose) return qvm_workspace_bytes(a);
     const Route route = pick_route(d, a);
     if (route == Route::kTiledF32) return qmm_f32_workspace_bytes(a);
+    qms::Plan split;
+    if (split_rows_take(a, route, split)) return qms_workspace_bytes(a, split);
     if (route != Route::kTiled) return 0;
     return dense && qmm_dense_takes(a) ? qmm_dense_workspace_bytes(a) : qmm_workspace_bytes(a);
 }
@@ -661,7 +673,10 @@ static int32_t quantized_matmul_any(const nvq_qmm_desc *d, const void *x, const 
     a.x = x; a.w = w; a.scales = scales; a.biases = biases; a.y = y;
     a.global_scale = global_scale;
     a.row_bias = row_bias;
-    switch (pick_route(d, a)) {
+    const Route route = pick_route(d, a);
+    qms::Plan split;
+    if (split_rows_take(a, route, split)) return launch_qms(a, split, workspace, (hipStream_t)stream);
+    switch (route) {
     case Route::kUntransposed: return launch_qvm(a, workspace, (hipStream_t)stream);
     case Route::kTiled:  // without a workspace: codes are expanded in the kernel and K is not split
         return dense && workspace != nullptr && qmm_dense_takes(a) ? launch_qmm_dense(a, workspace, (hipStream_t)stream) : launch_qmm(a, workspace, (hipStream_t)stream);

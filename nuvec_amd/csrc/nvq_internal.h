@@ -141,6 +141,18 @@ int32_t launch_qmr(const ProductArgs &a, hipStream_t s);
 // The few-row matrix-core kernel (up to 32 rows of x per pass; also the grouped gathered product).
 bool qmf_supported(const ProductArgs &a);
 int32_t launch_qmf(const ProductArgs &a, hipStream_t s);
+// A few dozen rows with K split over wavefronts, blocks and the grid (qms_kernel.h).
+namespace qms {
+struct Plan {
+    int mt, nt, qw;     // tiles of 16 rows of x a block, of 16 weight rows a wavefront; wavefronts of a group
+    int groups;         // of a block, which share its K
+    int splits, spans;  // of K over the grid; spans of 256 values a split
+    double us;          // estimated
+};
+}  // namespace qms
+bool qms_plan(const ProductArgs &a, qms::Plan &plan);  // false: the kernel does not take the product
+size_t qms_workspace_bytes(const ProductArgs &a, const qms::Plan &plan);
+int32_t launch_qms(const ProductArgs &a, const qms::Plan &plan, void *workspace, hipStream_t s);  // workspace NULL: no split
 int32_t launch_fill_zero(void *p, int64_t bytes, hipStream_t s);
 int32_t launch_quantized_attention(const nvq_attention_desc &d, const void *q, const void *kw, const void *ks, const void *kb,
                                    const void *vw, const void *vs, const void *vb, const void *sinks, void *out, void *workspace,

@@ -1,0 +1,90 @@
+"""Products of a few to a few dozen rows on the split-K kernel (`qms_kernel`), which the few-row and tiled routes hand what it is estimated
+faster at: against the CPU's product (crates/nuvec-core/src/kernels.rs:1091-1142), at the ends of its turns of 256 values, its chunks
+of codes, its tiles of rows and weight rows, in every shape of block and with K split over the grid or not."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+import nuvec_amd as nv
+from nuvec_amd import _lib, ops
+from oracle import ref
+from tests.hip_backend import to_dev, to_host
+from tests.test_gpu_parity import assert_rows_close, make_w, make_x
+
+pytestmark = pytest.mark.gpu
+
+
+def product(rng, fmt, m, n, k, dtype):
+    w, x = make_w(rng, n, k, dtype), make_x(rng, m, k, dtype)
+    if isinstance(fmt, str):
+        mode = getattr(ref, fmt)
+        group, bits = ref.FP_PARAMS[mode]
+        packed, scales = ref.fp_quantize(w, dtype, mode)
+        q = nv.Quantized(to_dev(packed), to_dev(scales), None, nv.Quant.new(getattr(nv.QuantMode, fmt)))
+        return q, x, ref.quantized_matmul(x, packed, scales, None, mode=mode, group=group, bits=bits, dtype=dtype, threads=8)
+    group, bits = fmt
+    packed, scales, biases = ref.affine_quantize(w, dtype, group, bits)
+    q = nv.Quantized(to_dev(packed), to_dev(scales), to_dev(biases), nv.Quant.affine(group, bits))
+    return q, x, ref.quantized_matmul(x, packed, scales, biases, group=group, bits=bits, dtype=dtype, threads=8)
+
+
+def workspace_bytes(m, n, k, quant, dtype):
+    lib = _lib.load()
+    d = _lib.QmmDescC()
+    d.quant = _lib.QuantC(int(quant.mode.value), quant.group_size, quant.bits)
+    d.dtype, d.transpose, d.m, d.item_rows, d.n, d.k = dtype, 1, m, m, n, k
+    return lib.nvq_quantized_matmul_workspace_bytes(C.byref(d))
+
+
+# One, two and four tiles of rows with tails; one and four wavefronts a group; K in and off whole turns, steps, chunks; splits of K.
+SHAPES = [(5, 1130, 1184), (16, 4100, 11104), (9, 18734, 1600), (24, 1100, 2336), (20, 9001, 2112), (33, 2050, 5984), (62, 1030, 11072),
+          (64, 5000, 480), (96, 1200, 2400), (7, 3536, 12832)]
+
+
+@pytest.mark.parametrize("dtype", [ref.BF16, ref.F16])
+@pytest.mark.parametrize("fmt", [(64, 2), (32, 3), (64, 4), (32, 4), (128, 5), (32, 6), (32, 8), (64, 8), "MXFP4", "MXFP8", "NVFP4"], ids=str)
+def test_every_format_against_the_cpu_product(fmt, dtype):
+    rng = np.random.default_rng(7300)
+    unit = max(fmt[0], 32) if not isinstance(fmt, str) else 32
+    for m, n, k in SHAPES:
+        k = k // unit * unit
+        q, x, want = product(rng, fmt, m, n, k, dtype)
+        for scratch in (True, False):
+            got = to_host(ops.quantized_matmul(to_dev(x), q, scratch=scratch))
+            assert_rows_close(got, want, dtype, f"split rows {fmt} M={m} N={n} K={k} scratch={scratch}", exact_weights=isinstance(fmt, str))
+
+
+@pytest.mark.parametrize("m,n,k", [(16, 4096, 11008), (62, 2560, 11072), (31, 404, 13792)])
+def test_bias_determinism_and_both_entry_points(m, n, k):
+    """QuantizedLinear's bias is the separate addition bit for bit (crates/nuvec-nn/src/layers.rs:155-162) after a split of K as before it;
+    two launches give the same bits; a row past the end of x, or a NaN in another row, changes nothing."""
+    rng = np.random.default_rng(7400 + m)
+    quant = nv.Quant.new(nv.QuantMode.NVFP4)
+    if workspace_bytes(m, n, k, quant, 10) == 0:
+        pytest.skip("K is not split on this device")
+    q, x, _ = product(rng, "NVFP4", m, n, k, ref.BF16)
+    xd = to_dev(x)
+    plain = nv.quantized_matmul(xd, q)
+    assert torch.equal(plain, nv.quantized_matmul(xd, q))
+    bias = torch.randn(n, device="cuda").to(torch.bfloat16)
+    from nuvec_amd.layers import QuantizedLinear
+    assert torch.equal(QuantizedLinear(q.weight, q.scales, None, bias, q.quant)(xd), plain + bias)
+    xd[m // 2, 3] = float("nan")
+    odd = nv.quantized_matmul(xd, q)
+    assert odd[m // 2].isnan().all()
+    keep = [r for r in range(m) if r != m // 2]
+    assert torch.equal(odd[keep], plain[keep])
+
+
+def test_no_rounding_where_the_weights_and_sums_are_exact():
+    """Small whole numbers: every cut of K gives the exact sums."""
+    m, n, k = 20, 3000, 4128
+    x = torch.randint(-2, 3, (m, k), device="cuda").to(torch.float16)
+    w = torch.randint(-2, 3, (n, k), device="cuda").to(torch.float16)
+    q = nv.quantize(w, nv.QuantMode.MXFP8)
+    dense = nv.dequantize(q, torch.float32)
+    assert torch.equal(dense, w.float())
+    want = (x.double() @ dense.double().t()).to(torch.float16)
+    assert torch.equal(nv.quantized_matmul(x, q), want)

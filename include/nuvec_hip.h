@@ -283,6 +283,14 @@ NVQ_API int32_t nvq_quantized_attention_prompt(const nvq_attention_prompt_desc *
                                 const void *k_b, const void *v_w, const void *v_s, const void *v_b, const void *sinks,
                                 void *out, void *workspace, void *stream);
 
+/* The same for float32 (every operand and the scales in float32): both products on the float32 matrix instruction, keys and values with
+ * the CPU's two roundings, scores and softmax on chip.  `workspace`: the float32 states of splits of the keys, or NULL where the
+ * size query says 0. */
+NVQ_API size_t nvq_quantized_attention_prompt_f32_workspace_bytes(const nvq_attention_prompt_desc *desc);
+NVQ_API int32_t nvq_quantized_attention_prompt_f32(const nvq_attention_prompt_desc *desc, const void *q, const void *k_w, const void *k_s,
+                                const void *k_b, const void *v_w, const void *v_s, const void *v_b, const void *sinks,
+                                void *out, void *workspace, void *stream);
+
 /* GpuEval::sorted_offsets (gpu.rs:6732-6756); kernels::sorted_offsets (kernels.rs:873-892):
  * per row of `indices` u32[rows, m], offsets[row, g] = first position whose value is >= g. */
 NVQ_API int32_t nvq_sorted_offsets(const uint32_t *indices, int64_t rows, int64_t m, int32_t groups,

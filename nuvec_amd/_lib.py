@@ -103,6 +103,8 @@ SIGNATURES = {
     "nvq_quantized_attention": (C.c_int32, [C.POINTER(AttentionDescC)] + [C.c_void_p] * 11),
     "nvq_quantized_attention_prompt_workspace_bytes": (C.c_size_t, [C.POINTER(AttentionPromptDescC)]),
     "nvq_quantized_attention_prompt": (C.c_int32, [C.POINTER(AttentionPromptDescC)] + [C.c_void_p] * 11),
+    "nvq_quantized_attention_prompt_f32_workspace_bytes": (C.c_size_t, [C.POINTER(AttentionPromptDescC)]),
+    "nvq_quantized_attention_prompt_f32": (C.c_int32, [C.POINTER(AttentionPromptDescC)] + [C.c_void_p] * 11),
     "nvq_sorted_offsets": (C.c_int32, [C.c_void_p, C.c_int64, C.c_int64, C.c_int32, C.c_void_p, C.c_void_p]),
     "nvq_quantize_scaled": (C.c_int32, [C.c_void_p, C.c_int32, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),
     "nvq_dequantize_scaled": (C.c_int32, [C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p]),

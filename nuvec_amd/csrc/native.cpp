@@ -601,13 +601,13 @@ PyObject *py_embedding(PyObject *, PyObject *const *args, Py_ssize_t n) {
     });
 }
 
-// attention(q, k weight, scales, biases, v weight, scales, biases, quant, scale, sinks, causal)
+// attention(q, k weight, scales, biases, v weight, scales, biases, quant, scale, sinks, causal[, several float32 rows too])
 // (ops.quantized_attention, ops.quantized_attention_fits for one query row per head; ops.quantized_attention_prompt)
 PyObject *py_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
     return guarded([&]() -> PyObject * {
         Tensor q, sinks;
         Packed k, v;
-        if (n != 11 || !as_tensor(args[0], q) || !as_tensor(args[1], k.w) || !as_tensor(args[2], k.s) || !as_tensor(args[3], k.b) ||
+        if ((n != 11 && n != 12) || !as_tensor(args[0], q) || !as_tensor(args[1], k.w) || !as_tensor(args[2], k.s) || !as_tensor(args[3], k.b) ||
             !as_tensor(args[4], v.w) || !as_tensor(args[5], v.s) || !as_tensor(args[6], v.b) || !read_quant(args[7], k.q) ||
             !as_tensor(args[9], sinks))
             return none();
@@ -630,17 +630,24 @@ PyObject *py_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
         const bool several = q.size(2) > 1;
         // (ops.quantized_attention_fits: one query row takes caches of unsigned words)
         if (!several && (k.w.scalar_type() != at::kUInt32 || v.w.scalar_type() != at::kUInt32)) return none();
-        const int causal = PyObject_IsTrue(args[10]);
-        if (causal < 0) return nullptr;
+        const int causal = PyObject_IsTrue(args[10]), single_too = n == 12 ? PyObject_IsTrue(args[11]) : 0;
+        if (causal < 0 || single_too < 0) return nullptr;
+        const bool single = several && code == NVQ_F32;
+        if (single && !single_too) return none();
         const nvq_attention_prompt_desc prompt{d, q.size(2), causal};
         Tensor y;
         const bool done = unlocked([&] {
-            const size_t need = several ? nvq_quantized_attention_prompt_workspace_bytes(&prompt) : nvq_quantized_attention_workspace_bytes(&d);
-            if (several && need == 0) return false;
+            const size_t need = single    ? nvq_quantized_attention_prompt_f32_workspace_bytes(&prompt)
+                                : several ? nvq_quantized_attention_prompt_workspace_bytes(&prompt)
+                                          : nvq_quantized_attention_workspace_bytes(&d);
+            if (several && !single && need == 0) return false;
             y = at.empty(q.sizes(), type);
             Tensor workspace;
             if (need > 0) workspace = at.empty({(int64_t)need}, at::kByte);
             void *scratch = need > 0 ? workspace.mutable_data_ptr() : nullptr;
+            if (single)
+                return nvq_quantized_attention_prompt_f32(&prompt, ptr(q), ptr(k.w), ptr(k.s), ptr(k.b), ptr(v.w), ptr(v.s), ptr(v.b), ptr(sinks),
+                                                          y.mutable_data_ptr(), scratch, at.stream()) == NVQ_OK;
             return (several ? nvq_quantized_attention_prompt(&prompt, ptr(q), ptr(k.w), ptr(k.s), ptr(k.b), ptr(v.w), ptr(v.s), ptr(v.b), ptr(sinks),
                                                              y.mutable_data_ptr(), scratch, at.stream())
                             : nvq_quantized_attention(&d, ptr(q), ptr(k.w), ptr(k.s), ptr(k.b), ptr(v.w), ptr(v.s), ptr(v.b), ptr(sinks),

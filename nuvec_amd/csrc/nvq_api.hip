@@ -818,7 +818,7 @@ int32_t nvq_quantized_attention(const nvq_attention_desc *d, const void *q, cons
     return launch_quantized_attention(*d, q, k_w, k_s, k_b, v_w, v_s, v_b, sinks, out, workspace, (hipStream_t)stream);
 }
 
-static int32_t check_attention_prompt(const nvq_attention_prompt_desc *p) {
+static int32_t check_attention_prompt(const nvq_attention_prompt_desc *p, bool single) {
     const char *op = "quantized_attention";
     if (p == nullptr) return fail(NVQ_INVALID_ARGUMENT, "%s: null descriptor", op);
     const nvq_attention_desc *d = &p->cache;
@@ -831,26 +831,31 @@ static int32_t check_attention_prompt(const nvq_attention_prompt_desc *p) {
         return fail(NVQ_INVALID_ARGUMENT, "%s: %lld query heads over %lld key heads", op, (long long)d->query_heads, (long long)d->key_heads);
     // 32-bit row, tile and block numbers; heads travel in grid y
     const int64_t heads = d->batch * d->key_heads;
-    if (d->dtype == NVQ_F32 || (d->head_dim != 64 && d->head_dim != 128) || d->head_dim % d->group_size != 0 || d->positions < 1 ||
+    if ((d->dtype == NVQ_F32) != single || (d->head_dim != 64 && d->head_dim != 128) || d->head_dim % d->group_size != 0 || d->positions < 1 ||
         p->queries < 1 || heads > 65535 || d->positions >= (1LL << 30) || p->queries * d->query_heads >= (1LL << 30) ||
         heads * d->positions >= (1LL << 31) || p->queries * d->query_heads * d->batch >= (1LL << 31))
-        return fail(NVQ_UNSUPPORTED, "%s: several query rows take half-precision types and head sizes 64 and 128", op);
+        return fail(NVQ_UNSUPPORTED, "%s: several query rows take %s and head sizes 64 and 128", op, single ? "float32" : "half-precision types");
     return NVQ_OK;
 }
 
 size_t nvq_quantized_attention_prompt_workspace_bytes(const nvq_attention_prompt_desc *p) {
-    if (check_attention_prompt(p) != NVQ_OK || require_device() != NVQ_OK) return 0;
+    if (check_attention_prompt(p, false) != NVQ_OK || require_device() != NVQ_OK) return 0;
     return attention_prompt_workspace_bytes(*p);
 }
 
-int32_t nvq_quantized_attention_prompt(const nvq_attention_prompt_desc *p, const void *q, const void *k_w, const void *k_s, const void *k_b,
-                                       const void *v_w, const void *v_s, const void *v_b, const void *sinks, void *out, void *workspace,
-                                       void *stream) {
+size_t nvq_quantized_attention_prompt_f32_workspace_bytes(const nvq_attention_prompt_desc *p) {
+    if (check_attention_prompt(p, true) != NVQ_OK || require_device() != NVQ_OK) return 0;
+    return attention_prompt_f32_workspace_bytes(*p);
+}
+
+static int32_t attention_prompt_any(const nvq_attention_prompt_desc *p, bool single, const void *q, const void *k_w, const void *k_s, const void *k_b,
+                                    const void *v_w, const void *v_s, const void *v_b, const void *sinks, void *out, void *workspace,
+                                    void *stream) {
     const char *op = "quantized_attention";
-    NVQ_TRY(check_attention_prompt(p));
+    NVQ_TRY(check_attention_prompt(p, single));
     if (p->cache.batch == 0 || p->cache.query_heads == 0) return NVQ_OK;
     if (q == nullptr || k_w == nullptr || k_s == nullptr || k_b == nullptr || v_w == nullptr || v_s == nullptr || v_b == nullptr ||
-        out == nullptr || workspace == nullptr)
+        out == nullptr || (workspace == nullptr && (!single || (require_device() == NVQ_OK && attention_prompt_f32_workspace_bytes(*p) != 0))))
         return fail(NVQ_INVALID_ARGUMENT, "%s: null operand", op);
     NVQ_TRY(require_device());
     NVQ_TRY(check_aligned(op, "queries", q));
@@ -858,7 +863,20 @@ int32_t nvq_quantized_attention_prompt(const nvq_attention_prompt_desc *p, const
     NVQ_TRY(check_aligned(op, "values", v_w, 4));
     NVQ_TRY(check_aligned(op, "out", out));
     NVQ_TRY(check_aligned(op, "workspace", workspace));
-    return launch_attention_prompt(*p, q, k_w, k_s, k_b, v_w, v_s, v_b, sinks, out, workspace, (hipStream_t)stream);
+    return single ? launch_attention_prompt_f32(*p, q, k_w, k_s, k_b, v_w, v_s, v_b, sinks, out, workspace, (hipStream_t)stream)
+                  : launch_attention_prompt(*p, q, k_w, k_s, k_b, v_w, v_s, v_b, sinks, out, workspace, (hipStream_t)stream);
+}
+
+int32_t nvq_quantized_attention_prompt(const nvq_attention_prompt_desc *p, const void *q, const void *k_w, const void *k_s, const void *k_b,
+                                       const void *v_w, const void *v_s, const void *v_b, const void *sinks, void *out, void *workspace,
+                                       void *stream) {
+    return attention_prompt_any(p, false, q, k_w, k_s, k_b, v_w, v_s, v_b, sinks, out, workspace, stream);
+}
+
+int32_t nvq_quantized_attention_prompt_f32(const nvq_attention_prompt_desc *p, const void *q, const void *k_w, const void *k_s, const void *k_b,
+                                           const void *v_w, const void *v_s, const void *v_b, const void *sinks, void *out, void *workspace,
+                                           void *stream) {
+    return attention_prompt_any(p, true, q, k_w, k_s, k_b, v_w, v_s, v_b, sinks, out, workspace, stream);
 }
 
 int32_t nvq_sorted_offsets(const uint32_t *indices, int64_t rows, int64_t m, int32_t groups, int32_t *offsets, void *stream) {

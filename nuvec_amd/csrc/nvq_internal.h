@@ -162,6 +162,10 @@ size_t attention_prompt_workspace_bytes(const nvq_attention_prompt_desc &d);  //
 int32_t launch_attention_prompt(const nvq_attention_prompt_desc &d, const void *q, const void *kw, const void *ks, const void *kb,
                                 const void *vw, const void *vs, const void *vb, const void *sinks, void *out, void *workspace,
                                 hipStream_t s);
+size_t attention_prompt_f32_workspace_bytes(const nvq_attention_prompt_desc &d);  // the states of splits of the keys, or 0
+int32_t launch_attention_prompt_f32(const nvq_attention_prompt_desc &d, const void *q, const void *kw, const void *ks, const void *kb,
+                                    const void *vw, const void *vs, const void *vb, const void *sinks, void *out, void *workspace,
+                                    hipStream_t s);
 int32_t launch_calibrate(int32_t kind, const void *buffer, int64_t bytes, int32_t iters, void *sink, int64_t *work, hipStream_t s);
 // Products with the weights stored [K, N] (transpose = false); K is split over the grid through a float32 workspace.
 int qvm_splits(const ProductArgs &a);

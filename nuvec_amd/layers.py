@@ -341,7 +341,7 @@ def quantized_attention(q: torch.Tensor, k: ops.Quantized, v: ops.Quantized, sca
     biases `[B, Hkv, S, D / group]`), grouped query heads, optional per-head `sinks [Hq]`, optionally causal (query i
     of L sees keys up to S - L + i, nuvec-lm's `quantized_attention`, model.rs:3646-3700):
     `softmax(scale * q k^T [, sinks]) v`.  One query row per head that fits the kernel (head size 64 or 128, 3, 4 or 8 bits)
-    takes the library's fused kernel, several rows in half precision its kernels on the matrix cores; the rest is the
+    takes the library's fused kernel, several rows its kernels on the matrix cores; the rest is the
     reference's composition (the one it runs wherever its fused kernel does not fit): both products are the library's
     quantized products, transposed for the keys and untransposed for the values, the query heads of a key head as rows of
     one product; the softmax (float32 inside, one rounding) is an elementwise step outside the path."""
@@ -350,15 +350,16 @@ def quantized_attention(q: torch.Tensor, k: ops.Quantized, v: ops.Quantized, sca
     if k.biases is None or v.biases is None:
         raise ops.InvalidArgument("quantized_attention: affine biases missing")
     if fused:  # the plain case of the branches below
-        out = (_native or _calls()).attention(q, k.weight, k.scales, k.biases, v.weight, v.scales, v.biases, k.quant, scale, sinks, causal)
+        out = (_native or _calls()).attention(q, k.weight, k.scales, k.biases, v.weight, v.scales, v.biases, k.quant, scale, sinks, causal, True)
         if out is not None:
             return out
     # (a single causal query row sees every key: the mask is empty)
     if fused and (not causal or q.shape[-2] == 1) and q.is_cuda and ops.quantized_attention_fits(q, k, v, sinks):
         return ops.quantized_attention(q, k, v, scale, sinks)  # one kernel (the reference's FastOp::QuantizedAttention)
-    if fused and q.is_cuda and q.ndim == 4 and q.shape[2] > 1 and q.shape[3] in (64, 128) and q.dtype != torch.float32:
+    if fused and q.is_cuda and q.ndim == 4 and q.shape[2] > 1 and q.shape[3] in (64, 128):
         try:  # several rows: both products and the softmax on the matrix cores
-            return ops.quantized_attention_prompt(q, k, v, scale, sinks, causal)
+            several = ops.quantized_attention_prompt_f32 if q.dtype == torch.float32 else ops.quantized_attention_prompt
+            return several(q, k, v, scale, sinks, causal)
         except ops.Unsupported:
             pass
     b, hq, l, d = q.shape

@@ -534,8 +534,17 @@ def quantized_attention_prompt(q: torch.Tensor, k: Quantized, v: Quantized, scal
     sizes other than 64 and 128)."""
     out = (_lib._native or _lib.native()).attention(q, k.weight, k.scales, k.biases, v.weight, v.scales, v.biases, k.quant, scale, sinks,
                                                     causal) if k.quant == v.quant else None
-    if out is not None:
-        return out
+    return out if out is not None else _attention_rows(q, k, v, scale, sinks, causal, "")
+
+
+def quantized_attention_prompt_f32(q: torch.Tensor, k: Quantized, v: Quantized, scale: float, sinks: Optional[torch.Tensor] = None,
+                                   causal: bool = False) -> torch.Tensor:
+    """The same in float32: keys, values, scores and weights stay in float32.  Raises `Unsupported` for what it does not take (the
+    16-bit types, head sizes other than 64 and 128)."""
+    return _attention_rows(q, k, v, scale, sinks, causal, "_f32")
+
+
+def _attention_rows(q, k, v, scale, sinks, causal, entry):
     if q.ndim != 4 or k.weight.ndim != 4 or k.quant != v.quant or k.quant.mode != QuantMode.AFFINE:
         raise Unsupported("quantized_attention: the operands do not fit the kernel")
     b, hq, l, d = q.shape
@@ -555,9 +564,10 @@ def quantized_attention_prompt(q: torch.Tensor, k: Quantized, v: Quantized, scal
     cache = _lib.AttentionDescC(_CODE[q.dtype], k.quant.bits, k.quant.group_size, d, b, hq, kw.shape[1], kw.shape[2], float(scale))
     desc = _lib.AttentionPromptDescC(cache, l, int(causal))
     lib = _lib.load()
-    workspace = torch.empty(lib.nvq_quantized_attention_prompt_workspace_bytes(C.byref(desc)), dtype=torch.uint8, device=q.device)
-    _lib.check(lib.nvq_quantized_attention_prompt(C.byref(desc), _ptr(q), _ptr(kw), _ptr(ks), _ptr(kb), _ptr(vw), _ptr(vs), _ptr(vb),
-                                                  _ptr(sinks), _ptr(out), _ptr(workspace), _stream()))
+    need = getattr(lib, f"nvq_quantized_attention_prompt{entry}_workspace_bytes")(C.byref(desc))
+    workspace = torch.empty(need, dtype=torch.uint8, device=q.device) if need or not entry else None
+    _lib.check(getattr(lib, f"nvq_quantized_attention_prompt{entry}")(C.byref(desc), _ptr(q), _ptr(kw), _ptr(ks), _ptr(kb), _ptr(vw), _ptr(vs),
+                                                                      _ptr(vb), _ptr(sinks), _ptr(out), _ptr(workspace), _stream()))
     return out
 
 

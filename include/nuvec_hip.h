@@ -428,6 +428,16 @@ NVQ_API int32_t nvq_gather_qmm_expert_bias(const nvq_gather_desc *desc, const vo
 NVQ_API int32_t nvq_quantized_matmul_glu(const nvq_qmm_desc *desc, int32_t activation, float alpha, float limit, const void *x,
                                  const void *w, const void *scales, const void *biases, const void *bias, void *y, void *stream);
 
+/* The same for more rows, on the split-K kernel: bfloat16 and float16, affine codes of 2 to 8 bits (projections whose products round each weight
+ * once) and the block formats without a global scale.  The projections are rounded to `dtype` before the activation; their float32
+ * sums may be ordered otherwise than in the two products.  `workspace`: as many bytes as the size query says (its answer depends on
+ * desc alone), or NULL: K is then not split over the grid.  NVQ_UNSUPPORTED where the two products and nvq_glu are estimated faster, or
+ * would hold their weights more precisely. */
+NVQ_API size_t nvq_quantized_matmul_glu_rows_workspace_bytes(const nvq_qmm_desc *desc);
+NVQ_API int32_t nvq_quantized_matmul_glu_rows(const nvq_qmm_desc *desc, int32_t activation, float alpha, float limit, const void *x,
+                                const void *w, const void *scales, const void *biases, const void *bias, void *y,
+                                void *workspace, void *stream);
+
 /* The grouped gathered product of the experts' gate and up projections with the gated activation as its epilogue:
  * `SwitchGlu::through` up to its down projection (crates/nuvec-lm/src/model.rs:2157-2169) in one kernel.  w, scales,
  * biases and expert_bias hold both projections in alternating runs of 64 rows (rows 128 b .. 128 b + 63: rows

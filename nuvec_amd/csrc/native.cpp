@@ -198,8 +198,9 @@ bool product(const Tensor &x, const Packed &p, const Tensor &bias, Flags f, Tens
     return true;
 }
 
-// ops.quantized_matmul_glu.
-bool product_glu(const Tensor &x, const Packed &p, const Tensor &bias, int32_t activation, float alpha, float limit, Tensor &out) {
+// ops.quantized_matmul_glu, or (`several`) ops.quantized_matmul_glu_rows.
+bool product_glu(const Tensor &x, const Packed &p, const Tensor &bias, int32_t activation, float alpha, float limit, bool several,
+                 Tensor &out) {
     const Place at(x);
     if (!at.usable() || x.dim() < 1 || !x.is_contiguous() || x.numel() == 0) return false;
     const int32_t code = code_of(x.scalar_type());
@@ -209,10 +210,14 @@ bool product_glu(const Tensor &x, const Packed &p, const Tensor &bias, int32_t a
     if (n == 0 || n % 128 != 0 || !bias_fits(bias, at, x.scalar_type(), n)) return false;
     nvq_qmm_desc d{};
     d.quant = p.q, d.dtype = code, d.transpose = 1;
-    d.m = d.item_rows = x.numel() / columns, d.n = n, d.k = columns;
-    Tensor y = at.empty(with_last(x.sizes(), n / 2), x.scalar_type());
-    const int32_t rc = nvq_quantized_matmul_glu(&d, activation, alpha, limit, ptr(x), ptr(p.w), ptr(p.s), ptr(p.b), ptr(bias),
-                                                y.mutable_data_ptr(), at.stream());
+    d.m = x.numel() / columns, d.n = n, d.k = columns, d.item_rows = x.dim() > 1 ? x.size(-2) : 1;
+    const size_t need = several ? nvq_quantized_matmul_glu_rows_workspace_bytes(&d) : 0;
+    Tensor workspace, y = at.empty(with_last(x.sizes(), n / 2), x.scalar_type());
+    if (need > 0) workspace = at.empty({(int64_t)need}, at::kByte);
+    const int32_t rc = several ? nvq_quantized_matmul_glu_rows(&d, activation, alpha, limit, ptr(x), ptr(p.w), ptr(p.s), ptr(p.b), ptr(bias),
+                                                               y.mutable_data_ptr(), need > 0 ? workspace.mutable_data_ptr() : nullptr, at.stream())
+                               : nvq_quantized_matmul_glu(&d, activation, alpha, limit, ptr(x), ptr(p.w), ptr(p.s), ptr(p.b), ptr(bias),
+                                                          y.mutable_data_ptr(), at.stream());
     if (rc != NVQ_OK) return false;
     out = std::move(y);
     return true;
@@ -454,12 +459,16 @@ PyObject *py_mlp(PyObject *, PyObject *const *args, Py_ssize_t n) {
         const Place at(x);
         const at::ScalarType type = x.scalar_type();
         if (!linear_fits(gate, at, type, x.size(-1)) || !linear_fits(down, at, type, gate.p.w.size(0))) return none();
-        if (both.p != Py_None && rows <= most) {
-            if (!read_linear(both.p, fused) || !linear_fits(fused, at, type, x.size(-1)) || fused.p.w.size(0) != 2 * gate.p.w.size(0)) return none();
-            const bool done = unlocked([&] {
-                return product_glu(x, fused.p, fused.bias, activation, 0.0f, 0.0f, hidden) && product(hidden, down.p, down.bias, Flags(), y);
-            });
-            if (hidden.defined()) return wrap(done, y);
+        const bool several = rows > most;
+        if (both.p != Py_None) {
+            const bool fits = read_linear(both.p, fused) && linear_fits(fused, at, type, x.size(-1)) && fused.p.w.size(0) == 2 * gate.p.w.size(0);
+            if (!fits && !several) return none();
+            if (fits) {
+                const bool done = unlocked([&] {
+                    return product_glu(x, fused.p, fused.bias, activation, 0.0f, 0.0f, several, hidden) && product(hidden, down.p, down.bias, Flags(), y);
+                });
+                if (hidden.defined()) return wrap(done, y);
+            }
         }
         if (!read_linear(args[0], names.up_proj, up) || !linear_fits(up, at, type, x.size(-1)) || up.p.w.size(0) != gate.p.w.size(0)) return none();
         const bool done = unlocked([&] {

@@ -722,35 +722,92 @@ int32_t nvq_quantized_linear(const nvq_qmm_desc *d, const void *x, const void *w
     return quantized_matmul_any(d, x, w, scales, biases, nullptr, y, workspace, stream, bias);
 }
 
-// `Mlp::forward` up to its down projection (crates/nuvec-lm/src/model.rs:2066-2074) for a few rows of x: the gate and up
-// products and the gated activation in one kernel.
-int32_t nvq_quantized_matmul_glu(const nvq_qmm_desc *d, int32_t activation, float alpha, float limit, const void *x, const void *w,
-                                 const void *scales, const void *biases, const void *bias, void *y, void *stream) {
-    const char *op = "quantized_matmul";
+// The checks of a product with the gated epilogue and the kernels' view of it; `empty`: nothing to compute.
+static int32_t glu_product(const char *op, const nvq_qmm_desc *d, int32_t activation, float alpha, float limit, const void *x, const void *w,
+                           const void *scales, const void *biases, const void *bias, void *y, ProductArgs &a, bool &empty) {
     NVQ_TRY(check_qmm(d, op));
     NVQ_TRY(check_groups(op, d->quant.mode, biases));
     if (activation < NVQ_GLU_SWIGLU || activation > NVQ_GLU_GEGLU) return fail(NVQ_INVALID_ARGUMENT, "%s: unknown activation %d", op, activation);
-    if (d->m == 0 || d->n == 0) return NVQ_OK;
+    empty = d->m == 0 || d->n == 0;
+    if (empty) return NVQ_OK;
     if (x == nullptr || w == nullptr || scales == nullptr || y == nullptr) return fail(NVQ_INVALID_ARGUMENT, "%s: null operand", op);
     if (!d->transpose || d->batch_ndim != 0 || d->k == 0 || d->n % 128 != 0 || d->row_exact || d->rows)
         return fail(NVQ_UNSUPPORTED, "%s: the gated epilogue takes x [M, K] times transposed weights whose gate and up rows alternate in runs of 64", op);
     if (wants_exact_weights(d->quant.mode, d->dtype, d->n / 2, d->m))
-        return fail(NVQ_UNSUPPORTED, "%s: the gated epilogue takes affine projections of 1024 rows or more each", op);
+        return fail(NVQ_UNSUPPORTED, "%s: the gated epilogue takes affine projections whose weights are not the CPU's", op);
     NVQ_TRY(require_device());
     NVQ_TRY(check_aligned(op, "x", x));
     NVQ_TRY(check_aligned(op, "w", w));
     NVQ_TRY(check_aligned(op, "y", y));
     NVQ_TRY(check_groups_aligned(op, d->quant, d->dtype, scales, biases));
     NVQ_TRY(check_aligned(op, "bias", bias, (size_t)dtype_size(d->dtype)));
-    ProductArgs a{};
+    a = ProductArgs{};
     a.x = x; a.w = w; a.scales = scales; a.biases = biases; a.y = y;
     a.mode = d->quant.mode; a.group = d->quant.group_size; a.bits = d->quant.bits; a.dtype = d->dtype;
     a.m = d->m; a.n = d->n; a.k = d->k;
     a.batch = 1;
     a.row_bias = bias;
     a.glu = 1 + activation; a.glu_alpha = alpha; a.glu_limit = limit;
+    return NVQ_OK;
+}
+
+// `Mlp::forward` up to its down projection (crates/nuvec-lm/src/model.rs:2066-2074) for a few rows of x: the gate and up
+// products and the gated activation in one kernel.
+int32_t nvq_quantized_matmul_glu(const nvq_qmm_desc *d, int32_t activation, float alpha, float limit, const void *x, const void *w,
+                                 const void *scales, const void *biases, const void *bias, void *y, void *stream) {
+    const char *op = "quantized_matmul";
+    ProductArgs a;
+    bool empty;
+    NVQ_TRY(glu_product(op, d, activation, alpha, limit, x, w, scales, biases, bias, y, a, empty));
+    if (empty) return NVQ_OK;
     if (!qmv_glu_pairs_take(a)) return fail(NVQ_UNSUPPORTED, "%s: the decode kernel does not take this product with the gated epilogue", op);
     return launch_qmv_glu_pairs(a, (hipStream_t)stream);
+}
+
+// Whether the split-K kernel takes the gate and up products of several rows with the gated epilogue: where the two products would run on
+// kernels that hold a weight no more precisely (rounded once; block formats hold it exactly on every kernel), and the bounds of
+// 700 pairs timed both ways leave it ahead (3 to 256 rows, K 512 to 5120, 1024 to 14336 hidden values, twelve formats: 0.75 of the time
+// of the two products and the activation, 0.71 where taken, 1.04 x at worst).  By estimate beside the few-row kernel,
+// the tiles and itself.  Left to the two products: 8-bit codes up to 16 rows beyond 24 M of both (W[7680,4736] at 5 rows 28.6 us
+// there, 36.6 here; W[2176,4992] at 15 rows 20.9 / 19.2), MXFP8 and NVFP4 up to 16 rows of the direct few-row kernel beyond 32 M (NVFP4
+// W[5184,3584] at 11 rows 17.5 / 20.0) and MXFP4 beyond 32 rows (W[1088,2048] at 98 rows 12.7 / 14.0; 32 rows W[5056,512] 14.2 / 7.9),
+// and of the batched-decode kernel 4 bits at up to 48 rows beyond K = 1536 (groups of 32, W[14272,2048] at 22 rows 23.4 / 26.0; W[13760,512]
+// at 19 rows 19.0 / 11.4, W[9344,3072] at 117 rows 70.8 / 44.7) and 8 bits up to 16 rows or beyond K = 1024 (W[9536,4096] at 18 rows
+// 35.8 / 39.1; W[8960,1024] at 32 rows 19.6 / 16.6).
+static bool gated_rows_take(const nvq_qmm_desc *d, const ProductArgs &a, qms::Plan &plan) {
+    if (a.m > 256 || !qms_plan(a, plan)) return false;
+    ProductArgs one = a;
+    one.glu = 0, one.n = a.n / 2;
+    const Route route = pick_route(d, one);
+    const double codes = (double)a.n * (double)a.k;
+    if (route == Route::kFewRowsDirect) return a.mode != NVQ_AFFINE && (a.mode == NVQ_MXFP4 ? a.m <= 32 : a.m > 16 || codes <= 32.0e6);
+    if (route == Route::kBatchedDecode) return a.bits == 4 ? a.k <= 1536 || a.m > 48 : a.k <= 1024 && a.m > 16;
+    if ((route != Route::kFewRows && route != Route::kTiled) || (a.mode == NVQ_AFFINE && a.bits == 8 && a.m <= 16 && codes > 24.0e6)) return false;
+    qms::Plan split;
+    if (split_rows_take(one, route, split)) return plan.us < 4.0 + 2.0 * split.us;
+    return plan.us < (route == Route::kTiled ? 0.8 * (4.0 + 2.0 * tiled_us(one)) : 4.0 + 2.0 * few_rows_us(one));
+}
+
+size_t nvq_quantized_matmul_glu_rows_workspace_bytes(const nvq_qmm_desc *d) {
+    if (check_qmm(d, "quantized_matmul") != NVQ_OK || d->m == 0 || d->n == 0 || d->k == 0 || !d->transpose || d->batch_ndim != 0 || require_device() != NVQ_OK) return 0;
+    ProductArgs a = product_args(d, 1);
+    a.exact_weights = wants_exact_weights(d->quant.mode, d->dtype, d->n / 2, d->m);
+    a.glu = 1;
+    qms::Plan plan;
+    return gated_rows_take(d, a, plan) ? qms_workspace_bytes(a, plan) : 0;
+}
+
+int32_t nvq_quantized_matmul_glu_rows(const nvq_qmm_desc *d, int32_t activation, float alpha, float limit, const void *x, const void *w,
+                                      const void *scales, const void *biases, const void *bias, void *y, void *workspace, void *stream) {
+    const char *op = "quantized_matmul";
+    ProductArgs a;
+    bool empty;
+    NVQ_TRY(glu_product(op, d, activation, alpha, limit, x, w, scales, biases, bias, y, a, empty));
+    if (empty) return NVQ_OK;
+    NVQ_TRY(check_aligned(op, "workspace", workspace));
+    qms::Plan plan;
+    if (!gated_rows_take(d, a, plan)) return fail(NVQ_UNSUPPORTED, "%s: the split-K kernel does not take this product with the gated epilogue", op);
+    return launch_qms(a, plan, workspace, (hipStream_t)stream);
 }
 
 int32_t nvq_quantized_matmul_static(const nvq_qmm_desc *d, const void *x, const void *w, const void *scales, const void *biases,

@@ -112,6 +112,14 @@ class Mlp:
                 return self.down_proj(ops.quantized_matmul_glu(x, p.quantized(), activation, bias=p.bias))
             except ops.Unsupported:  # (a product the decode kernel does not take: the composition below)
                 pass
+        elif self.gate_up_proj is not None and rows > most:
+            p, hidden = self.gate_up_proj, None
+            try:
+                hidden = ops.quantized_matmul_glu_rows(x, p.quantized(), activation, bias=p.bias)
+            except (ops.Unsupported, ops.InvalidArgument):  # (the composition takes what it can, and says what it can not)
+                pass
+            if hidden is not None:
+                return self.down_proj(hidden)
         return self.down_proj(ops.glu(self.gate_proj(x), self.up_proj(x), activation))
 
     __call__ = forward

@@ -803,6 +803,27 @@ def quantized_matmul_glu(x: torch.Tensor, q: Quantized, activation: str = "swigl
     `[N]`) hold the gate and up projections in alternating runs of 64 rows (`pair_rows`); the result is `[..., N / 2]`, bit
     for bit `glu(gate(x), up(x))` of the two rounded products.  Raises `Unsupported` beyond four rows of x and where the
     decode kernel does not take the product (the caller then composes the products and `glu`)."""
+    d, operands, out = _glu_product(x, q, activation, bias)
+    _lib.check(_lib.load().nvq_quantized_matmul_glu(C.byref(d), GLU_ACTIVATIONS[activation], float(alpha), float(limit),
+                                                    *map(_ptr, operands), _ptr(out), _stream()))
+    return out
+
+
+def quantized_matmul_glu_rows(x: torch.Tensor, q: Quantized, activation: str = "swiglu", *, alpha: float = 1.702, limit: float = 7.0,
+                              bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """`quantized_matmul_glu` for more rows of x, on the split-K kernel: the two products are rounded before the activation as
+    there, their float32 sums may be ordered otherwise.  Raises `Unsupported` where the two products and `glu` are estimated
+    faster or hold their weights more precisely (the caller then composes them)."""
+    d, operands, out = _glu_product(x, q, activation, bias)
+    need = _lib.load().nvq_quantized_matmul_glu_rows_workspace_bytes(C.byref(d))
+    workspace = torch.empty(need, dtype=torch.uint8, device=out.device) if need > 0 else None
+    _lib.check(_lib.load().nvq_quantized_matmul_glu_rows(C.byref(d), GLU_ACTIVATIONS[activation], float(alpha), float(limit),
+                                                         *map(_ptr, operands), _ptr(out), _ptr(workspace), _stream()))
+    return out
+
+
+def _glu_product(x: torch.Tensor, q: Quantized, activation: str, bias: Optional[torch.Tensor]):
+    """The checked descriptor, operands (x, codes, scales, biases, bias) and empty result of a product with the gated epilogue."""
     op = "quantized_matmul"
     if activation not in GLU_ACTIVATIONS:
         raise InvalidArgument(f"{op}: unknown activation {activation!r}")
@@ -831,12 +852,10 @@ def quantized_matmul_glu(x: torch.Tensor, q: Quantized, activation: str = "swigl
     out = torch.empty(x.shape[:-1] + (n // 2,), dtype=dtype, device=x.device)
     d = _lib.QmmDescC()
     d.quant, d.dtype, d.transpose = quant._c(), _CODE[dtype], 1
-    d.m = d.item_rows = rows
+    d.m = rows
+    d.item_rows = x.shape[-2] if x.ndim > 1 else 1
     d.n, d.k, d.batch_ndim = n, columns, 0
-    _lib.check(_lib.load().nvq_quantized_matmul_glu(C.byref(d), GLU_ACTIVATIONS[activation], float(alpha), float(limit), _ptr(x), _ptr(w),
-                                                    _ptr(scales), _ptr(biases), _ptr(None if bias is None else bias.contiguous()),
-                                                    _ptr(out), _stream()))
-    return out
+    return d, (x, w, scales, biases, None if bias is None else bias.contiguous()), out
 
 
 def pair_rows(gate: torch.Tensor, up: torch.Tensor, dim: int) -> torch.Tensor:

@@ -767,15 +767,15 @@ int32_t nvq_quantized_matmul_glu(const nvq_qmm_desc *d, int32_t activation, floa
 // Whether the split-K kernel takes the gate and up products of several rows with the gated epilogue: where the two products would run on
 // kernels that hold a weight no more precisely (rounded once; block formats hold it exactly on every kernel), and the bounds of
 // 700 pairs timed both ways leave it ahead (3 to 256 rows, K 512 to 5120, 1024 to 14336 hidden values, twelve formats: 0.75 of the time
-// of the two products and the activation, 0.71 where taken, 1.04 x at worst).  By estimate beside the few-row kernel,
-// the tiles and itself.  Left to the two products: 8-bit codes up to 16 rows beyond 24 M of both (W[7680,4736] at 5 rows 28.6 us
-// there, 36.6 here; W[2176,4992] at 15 rows 20.9 / 19.2), MXFP8 and NVFP4 up to 16 rows of the direct few-row kernel beyond 32 M (NVFP4
+// of the two products and the activation, 0.71 where taken, 1.04 x at worst; from six rows on).  By estimate beside the few-row kernel,
+// the tiles and itself.  Left to the two products: 8-bit codes up to 16 rows beyond 24 M of both (W[2176,4992] at 15 rows
+// 20.9 us there, 19.2 here), MXFP8 and NVFP4 up to 16 rows of the direct few-row kernel beyond 32 M (NVFP4
 // W[5184,3584] at 11 rows 17.5 / 20.0) and MXFP4 beyond 32 rows (W[1088,2048] at 98 rows 12.7 / 14.0; 32 rows W[5056,512] 14.2 / 7.9),
 // and of the batched-decode kernel 4 bits at up to 48 rows beyond K = 1536 (groups of 32, W[14272,2048] at 22 rows 23.4 / 26.0; W[13760,512]
 // at 19 rows 19.0 / 11.4, W[9344,3072] at 117 rows 70.8 / 44.7) and 8 bits up to 16 rows or beyond K = 1024 (W[9536,4096] at 18 rows
 // 35.8 / 39.1; W[8960,1024] at 32 rows 19.6 / 16.6).
 static bool gated_rows_take(const nvq_qmm_desc *d, const ProductArgs &a, qms::Plan &plan) {
-    if (a.m > 256 || !qms_plan(a, plan)) return false;
+    if (a.m <= 5 || a.m > 256 || !qms_plan(a, plan)) return false;  // (up to five rows an MLP's bits are those of its two products)
     ProductArgs one = a;
     one.glu = 0, one.n = a.n / 2;
     const Route route = pick_route(d, one);

@@ -812,8 +812,8 @@ def quantized_matmul_glu(x: torch.Tensor, q: Quantized, activation: str = "swigl
 def quantized_matmul_glu_rows(x: torch.Tensor, q: Quantized, activation: str = "swiglu", *, alpha: float = 1.702, limit: float = 7.0,
                               bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """`quantized_matmul_glu` for more rows of x, on the split-K kernel: the two products are rounded before the activation as
-    there, their float32 sums may be ordered otherwise.  Raises `Unsupported` where the two products and `glu` are estimated
-    faster or hold their weights more precisely (the caller then composes them)."""
+    there, their float32 sums may be ordered otherwise.  Raises `Unsupported` up to five rows and where the two products and `glu` are
+    estimated faster or hold their weights more precisely (the caller then composes them)."""
     d, operands, out = _glu_product(x, q, activation, bias)
     need = _lib.load().nvq_quantized_matmul_glu_rows_workspace_bytes(C.byref(d))
     workspace = torch.empty(need, dtype=torch.uint8, device=out.device) if need > 0 else None

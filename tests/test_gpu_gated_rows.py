@@ -24,7 +24,7 @@ def _projections(quant, hidden, k, dtype, bias, seed):
 
 @pytest.mark.parametrize("form", FORMS, ids=str)
 @pytest.mark.parametrize("rows,hidden,k,dtype,activation,bias", [
-    (5, 1088, 640, torch.bfloat16, "swiglu", False),    # off whole blocks of 128 outputs; few-row route
+    (6, 1088, 640, torch.bfloat16, "swiglu", False),    # the fewest rows; off whole blocks of 128 outputs; few-row route
     (16, 1024, 4096, torch.float16, "geglu", True),     # a whole pass; eight slices of 512 values
     (17, 2752, 2048, torch.bfloat16, "swiglu_oai", False),  # one row into the second pass
     (31, 1088, 1152, torch.float16, "swiglu", True),    # K off slices of 512

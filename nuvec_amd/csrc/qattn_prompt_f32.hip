@@ -201,7 +201,8 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
             for (int t = 0; t < 2; t++) {
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-                    const bool hidden = masked && key0 + 16 * t + e > last[r];
+                    // (a score of -inf weighs nothing: below it would meet the infinity of the scale's rest, of either sign)
+                    const bool hidden = (masked && key0 + 16 * t + e > last[r]) || s[t][r][e] * a.scale == -INFINITY;
                     const float x = __builtin_fmaf(s[t][r][e], a.scale, __builtin_fmaf(s[t][r][e], a.scale_rest, -m[r]));
                     s[t][r][e] = hidden ? 0.0f : __builtin_amdgcn_exp2f(x);
                 }

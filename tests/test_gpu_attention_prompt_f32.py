@@ -69,3 +69,28 @@ def test_like_the_composition(scale):
     assert got[0, 3, 7].isnan().all() and got[1, 2, 9].isnan().all()
     got[0, 3, 7], got[1, 2, 9] = plain[0, 3, 7], plain[1, 2, 9]
     assert torch.equal(got, plain)
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("s", [300, 2000])
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_keys_whose_scores_are_minus_infinity_weigh_nothing(dim, s, sign):
+    """Whatever the scale's sign and the sign of what its rounding leaves (positive at head size 64, negative at 128), in whole tiles and
+    between other keys; a row of such keys alone is NaN, as the composition has it, or its sink's.  The bound is that of test_against_float64
+    for two sums, the other keys lying in other tiles."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(s + dim)
+    quant = nv.Quant.affine(64, 8)
+    k, v = (cache(2, 2, s, dim, 64, 8, gen) for _ in range(2))
+    q = torch.randn(2, 8, 9, dim, device="cuda", generator=gen).abs_()
+    seen = torch.ones(s, dtype=torch.bool, device="cuda")
+    seen[:100], seen[170], seen[s - 1] = False, False, False
+    k.biases[:, :, ~seen] = sign * float("-inf")
+    take = lambda t: nv.Quantized(t.weight.view(torch.int32)[:, :, seen].contiguous().view(torch.uint32), t.scales[:, :, seen].contiguous(),
+                                  t.biases[:, :, seen].contiguous(), quant)
+    got, want = layers.quantized_attention(q, k, v, sign * dim ** -0.5), exact(q, take(k), take(v), sign * dim ** -0.5, None, False)
+    assert (got.double() - want).norm() <= 32 * 2.0 ** -24 * want.norm()
+    k.biases[:] = sign * float("-inf")
+    assert layers.quantized_attention(q, k, v, sign * dim ** -0.5).isnan().all()
+    sinks = torch.randn(8, device="cuda", generator=gen)
+    assert (layers.quantized_attention(q, k, v, sign * dim ** -0.5, sinks) == 0).all()

@@ -10,6 +10,8 @@
 
 #include "nvq_device.h"
 
+#include <float.h>
+
 namespace nvq {
 
 constexpr int kMergeParts = 4;
@@ -22,7 +24,7 @@ __device__ __forceinline__ void merge_attention_states(const float *__restrict__
     __shared__ float part[kMergeParts][D];
     const int lane = threadIdx.x & 63, at = threadIdx.x % D, group = threadIdx.x / D;
     const bool real = lane < splits;
-    const float m = real ? src[lane * stride] : -1.0e30f, l = real ? src[lane * stride + 1] : 0.0f;
+    const float m = real ? src[lane * stride] : -FLT_MAX, l = real ? src[lane * stride + 1] : 0.0f;
     float top = m;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) top = fmaxf(top, __shfl_xor(top, o));

@@ -23,6 +23,8 @@
 #include "nvq_internal.h"
 #include "qmf_kernel.h"
 
+#include <float.h>
+
 namespace nvq {
 namespace {
 
@@ -126,7 +128,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     for (int t = 0; t < 2; t++)
 #pragma unroll
         for (int d = 0; d < kTiles; d++) o[t][d] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    float m[2] = {-1.0e30f, -1.0e30f}, sum[2] = {0.0f, 0.0f};  // (finite: a masked score's weight is exp2(-inf - m) = 0 from the first tile on)
+    float m[2] = {-FLT_MAX, -FLT_MAX}, sum[2] = {0.0f, 0.0f};  // (finite: a masked score's weight is exp2(-inf - m) = 0 from the first tile on)
 
     const int64_t row0 = (int64_t)head * a.positions;
     Part<BITS, D> kc[2], vc[2];
@@ -170,14 +172,15 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
         const bool masked = tile * kKeys + kKeys - 1 > all_last;
 #pragma unroll
         for (int r = 0; r < 2; r++) {
-            float top = -INFINITY;
+            float top = -INFINITY, low = INFINITY;
 #pragma unroll
             for (int t = 0; t < 2; t++)
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     if (masked && key0 + 16 * t + e > last[r]) s[t][r][e] = -INFINITY;
-                    top = fmaxf(top, s[t][r][e] * a.scale);
+                    top = fmaxf(top, s[t][r][e] * a.scale), low = fminf(low, s[t][r][e] * a.scale);
                 }
+            if (masked) low = -INFINITY;  // (the general form)
             if (a.scale < 0.0f && masked) {  // (a hidden score is the least one whatever the scale's sign)
                 top = -INFINITY;
 #pragma unroll
@@ -197,17 +200,26 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
 #pragma unroll
                     for (int e = 0; e < 4; e++) o[r][d][e] *= f;
             }
+            // Two kinds of scores do not take the exact form below: -inf, which would meet an infinity of either sign, and, as m is a rounded
+            // product and they are not, those so large that what the rounding leaves, up to 2^-24 m, is no small power of two.
+            if (__any(fabsf(m[r]) > 1048576.0f || low == -INFINITY)) {
 #pragma unroll
-            for (int t = 0; t < 2; t++) {
+                for (int t = 0; t < 2; t++)
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    // (a score of -inf weighs nothing: below it would meet the infinity of the scale's rest, of either sign)
-                    const bool hidden = (masked && key0 + 16 * t + e > last[r]) || s[t][r][e] * a.scale == -INFINITY;
-                    const float x = __builtin_fmaf(s[t][r][e], a.scale, __builtin_fmaf(s[t][r][e], a.scale_rest, -m[r]));
-                    s[t][r][e] = hidden ? 0.0f : __builtin_amdgcn_exp2f(x);
-                }
-                sum[r] += (s[t][r][0] + s[t][r][1]) + (s[t][r][2] + s[t][r][3]);
+                    for (int e = 0; e < 4; e++) {
+                        const bool hidden = masked && key0 + 16 * t + e > last[r];
+                        const float v = s[t][r][e] * a.scale, x = __builtin_fmaf(s[t][r][e], a.scale, __builtin_fmaf(s[t][r][e], a.scale_rest, -m[r]));
+                        s[t][r][e] = hidden ? 0.0f : __builtin_amdgcn_exp2f(fabsf(m[r]) > 1048576.0f || v == -INFINITY ? v - m[r] : x);
+                    }
+            } else {
+#pragma unroll
+                for (int t = 0; t < 2; t++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        s[t][r][e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][r][e], a.scale, __builtin_fmaf(s[t][r][e], a.scale_rest, -m[r])));
             }
+#pragma unroll
+            for (int t = 0; t < 2; t++) sum[r] += (s[t][r][0] + s[t][r][1]) + (s[t][r][2] + s[t][r][3]);
         }
         __builtin_amdgcn_wave_barrier();  // (the wavefront's LDS accesses execute in order)
 #pragma unroll
@@ -236,7 +248,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
         __syncthreads();
 #pragma unroll
         for (int r = 0; r < 2; r++) {
-            float top = -1.0e30f, all = 0.0f;
+            float top = -FLT_MAX, all = 0.0f;
 #pragma unroll
             for (int k = 0; k < KP; k++) top = fmaxf(top, state_m[rg * KP + k][16 * r + l]);
 #pragma unroll

@@ -94,3 +94,21 @@ def test_keys_whose_scores_are_minus_infinity_weigh_nothing(dim, s, sign):
     assert layers.quantized_attention(q, k, v, sign * dim ** -0.5).isnan().all()
     sinks = torch.randn(8, device="cuda", generator=gen)
     assert (layers.quantized_attention(q, k, v, sign * dim ** -0.5, sinks) == 0).all()
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("s", [45, 2000])
+@pytest.mark.parametrize("size", [1e4, 1e7, -1e7, 1e10, -1e10, 1e20, 1e33, -1e33, -1e36])
+def test_scores_of_any_size(dim, s, size):
+    """The largest scores weigh alike however large they are: beyond 2^31 a score's own rounding is more than exp2 holds, and all of
+    a row may lie below any finite value that a maximum could start from.  Keys of ones and of twos: the mean of half of the values."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(s + dim)
+    k, v = (cache(1, 2, s, dim, 64, 8, gen) for _ in range(2))
+    k.scales.zero_()
+    k.biases.copy_(torch.randint(1, 3, (1, 2, s, 1), device="cuda", generator=gen).float().expand(k.biases.shape))
+    q = torch.full((1, 8, 7, dim), size, device="cuda")
+    sinks = torch.randn(8, device="cuda", generator=gen)
+    for causal, sink in ((False, None), (True, None), (False, sinks)):
+        got, want = layers.quantized_attention(q, k, v, dim ** -0.5, sink, causal=causal), exact(q, k, v, dim ** -0.5, sink, causal)
+        assert (got.double() - want).norm() <= 16 * 2.0 ** -24 * want.norm() + 1e-30, (causal, sink is None)

@@ -10,7 +10,7 @@
 //     group's sum X of x.  The biases' part is a product of its own, over groups, on the float32 instruction.
 // A weight's own two roundings (crates/nuvec-core/src/kernels.rs:835-859, 992-998), which the CPU's product keeps, are not made.
 // What the split of x does not hold, an infinity or a magnitude whose sums of codes leave float32, comes out of it as no finite
-// number: such an output is multiplied again, value by value.  Magnitudes below 2^-100 keep 2^-126.
+// number: a wavefront with such an output multiplies its tiles again, on the float32 instruction.  Magnitudes below 2^-100 keep 2^-126.
 //
 // A block of four wavefronts owns 16 MT rows of x and 64 NT weight rows (16 NT a wavefront) and walks its share of K in steps
 // of 64.  x goes through registers, where it is split and its groups' sums are formed, into one of two LDS stages, a step ahead;
@@ -105,30 +105,31 @@ __device__ __forceinline__ uint4 code_operand(uint64_t codes, float scale) {
     return o;
 }
 
-// A split's part of y[row, col], one value after the other.
+// Four weights from value k on (a multiple of four) of weight row `row`, as the CPU dequantizes them: two roundings.
 template <int BITS, int MODE>
-__device__ __forceinline__ float plain_sum(const ProductArgs &a, int row, int col, int k0, int k1, int gshift, float factor) {
+__device__ __forceinline__ floatx4_t plain_weights(const ProductArgs &a, int64_t row, int k, int gshift, float factor) {
     const int K = (int)a.k;
-    float v = 0.0f;
-    for (int k = k0; k < k1; k++) {
-        const int64_t at = (int64_t)k * BITS;
-        const uint32_t *word = (const uint32_t *)a.w + (int64_t)col * (K / 32 * BITS) + at / 32;
-        const int bit = (int)(at % 32);
-        uint32_t c = word[0] >> bit;
-        if (bit + BITS > 32) c |= word[1] << (32 - bit);
-        c &= (1u << BITS) - 1u;
-        const int64_t g = (int64_t)col * (K >> gshift) + (k >> gshift);
-        float w;
-        if constexpr (MODE == NVQ_AFFINE) {
-            w = (float)c * ((const float *)a.scales)[g] + ((const float *)a.biases)[g];
-        } else {
-            const uint32_t code = ((const uint8_t *)a.scales)[g];
-            const float s = MODE == NVQ_NVFP4 ? qmf::nvfp4_scale(code, factor) : ftz(e8m0_to_f32(code));
-            w = (MODE == NVQ_MXFP8 ? e4m3_to_f32(c) : e2m1_to_f32(c)) * s;
-        }
-        v = __builtin_fmaf(((const float *)a.x)[(int64_t)row * K + k], w, v);
+    const int64_t at = (int64_t)k * BITS;
+    const uint32_t *word = (const uint32_t *)a.w + row * (K / 32 * BITS) + at / 32;
+    const int bit = (int)(at % 32);
+    uint64_t codes = word[0];
+    if (bit + 4 * BITS > 32) codes |= (uint64_t)word[1] << 32;  // (a row ends with a dword)
+    codes >>= bit;
+    const int64_t g = row * (K >> gshift) + (k >> gshift);
+    float s, b = 0.0f;
+    if constexpr (MODE == NVQ_AFFINE) {
+        s = ((const float *)a.scales)[g], b = ((const float *)a.biases)[g];
+    } else {
+        const uint32_t code = ((const uint8_t *)a.scales)[g];
+        s = MODE == NVQ_NVFP4 ? qmf::nvfp4_scale(code, factor) : ftz(e8m0_to_f32(code));
     }
-    return v;
+    floatx4_t w;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const uint32_t c = (uint32_t)(codes >> (BITS * j)) & ((1u << BITS) - 1u);
+        w[j] = MODE == NVQ_AFFINE ? (float)c * s + b : (MODE == NVQ_MXFP8 ? e4m3_to_f32(c) : e2m1_to_f32(c)) * s;
+    }
+    return w;
 }
 
 // G32: groups of 32 (affine, MXFP4, MXFP8), whose scale follows every matrix instruction; else blocks of 64, which lie in one group.
@@ -405,6 +406,51 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     const float factor = kNv ? qmf::nvfp4_factor(a, 0) : 1.0f;
     float *y = a.k_splits > 1 ? a.partials + (int64_t)blockIdx.z * M * N : (float *)a.y;
     bool plain = false;
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                if (kNv) acc[m][t][e] *= factor;
+                plain |= !(fabsf(acc[m][t][e]) < INFINITY);
+            }
+    // Outputs that are no finite number: the wavefront's tiles again from whole values of x and the CPU's weights on the float32
+    // instruction, lane (q, l) with values 4 q .. of sixteen of row l; those outputs alone take what comes.
+    if (__any(plain)) {
+        floatx4_t again[MT][NT];
+#pragma unroll
+        for (int m = 0; m < MT; m++)
+#pragma unroll
+            for (int t = 0; t < NT; t++) again[m][t] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 2
+        for (int from = k0; from < k1; from += 16) {
+            const int k = from + 4 * q;
+            floatx4_t xv[MT], wv[NT];
+#pragma unroll
+            for (int m = 0; m < MT; m++) {
+                const int row = m0 + kTile * m + l;
+                xv[m] = *reinterpret_cast<const floatx4_t *>((const float *)a.x + (int64_t)(row < M ? row : M - 1) * K + k);
+            }
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                const int n = n0 + kTile * t + l;
+                wv[t] = plain_weights<BITS, MODE>(a, n < N ? n : N - 1, k, gshift, factor);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int m = 0; m < MT; m++)
+#pragma unroll
+                    for (int t = 0; t < NT; t++) again[m][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[m][j], wv[t][j], again[m][t], 0, 0, 0);
+        }
+#pragma unroll
+        for (int m = 0; m < MT; m++)
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[m][t][e] = fabsf(acc[m][t][e]) < INFINITY ? acc[m][t][e] : again[m][t][e];
+    }
     // Accumulator element e of lane (q, l): row 4 q + e of x, weight row l.
 #pragma unroll
     for (int m = 0; m < MT; m++)
@@ -413,18 +459,8 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const int row = m0 + kTile * m + 4 * q + e, col = n0 + kTile * t + l;
-                const float v = kNv ? acc[m][t][e] * factor : acc[m][t][e];
-                plain |= !(fabsf(v) < INFINITY);
-                if (row < M && col < N) y[(int64_t)row * N + col] = a.k_splits > 1 ? v : add_row_bias<float>(a.row_bias, v, col);
+                if (row < M && col < N) y[(int64_t)row * N + col] = a.k_splits > 1 ? acc[m][t][e] : add_row_bias<float>(a.row_bias, acc[m][t][e], col);
             }
-    if (plain) {
-        for (int i = 0; i < MT * NT * 4; i++) {
-            const int row = m0 + i / (NT * 4) * kTile + 4 * q + i % 4, col = n0 + i / 4 % NT * kTile + l;
-            if (row >= M || col >= N || fabsf(y[(int64_t)row * N + col]) < INFINITY) continue;
-            const float v = plain_sum<BITS, MODE>(a, row, col, k0, k1, gshift, factor);
-            y[(int64_t)row * N + col] = a.k_splits > 1 ? v : add_row_bias<float>(a.row_bias, v, col);
-        }
-    }
 }
 
 // The parts of a split K, eight under way at a time and added by pairs.

@@ -218,18 +218,20 @@ NVQ_API int32_t nvq_dequantize_rows(const nvq_quant *quant, int32_t dtype, const
                             const void *biases, int64_t table_rows, int64_t cols, const uint32_t *ids, int64_t count,
                             void *out, void *stream);
 
-/* Bytes of scratch nvq_quantized_matmul needs for `desc` (split-K partials; the reference
- * allocates them on its side of the boundary, gpu.rs:7562).  0 = none; nonzero for products whose K is
- * split over the grid (float32 partial sums): transpose = 0, and transpose = 1 products of many rows with few
- * output tiles and a long K (the counterpart of the reference's qmm_t_splitk, gpu.rs:7507-7590).  A transposed
- * product given no workspace runs unsplit. */
-/* The kernel a product of this descriptor runs on with operands aligned as hipMalloc aligns them ("qmm_kernel",
- * "qmf_kernel", "qmd_kernel", "qmv4_lds_kernel", ...), from the same routing code as the launch; NULL with
+/* The route of a product of this descriptor with operands aligned as hipMalloc aligns them, under the name of the kernel that stands
+ * for it ("qmm_kernel", "qmf_kernel", "qmd_kernel", "qmv4_lds_kernel", ...), from the same routing code as the launch; NULL with
  * nvq_last_error for a descriptor the launch would refuse.  The reference names its kernels by route as well
  * (gpu.rs:7022, "nuvec_affine_qmv_mma_..."; its tests check the names, crates/nuvec-core/tests/quantized.rs:843-861).
  * Needs nvq_init. */
 NVQ_API const char *nvq_quantized_matmul_route(const nvq_qmm_desc *desc);
-/* Float32 partial sums where K is split over the grid, or the weight dequantized for many rows of x; 0: none. */
+/* The kernel that runs it, given the workspace that the size query names.  It is the route's but on two of them: products of "qmf_kernel"
+ * and "qmm_kernel" may run on "qms_kernel<R,C,G>" (a block holds 16 R rows of x, a wavefront 16 C weight rows, G wavefronts share
+ * x), and those of "qmm_kernel" on "qmm_dense_kernel". */
+NVQ_API const char *nvq_quantized_matmul_kernel(const nvq_qmm_desc *desc);
+/* Bytes of scratch nvq_quantized_matmul needs for `desc` (the reference allocates them on its side of the boundary, gpu.rs:7562; the
+ * counterpart of its qmm_t_splitk, gpu.rs:7507-7590).  0 = none; nonzero where K is split over the grid (float32 partial sums): transpose = 0,
+ * and transpose = 1 products of a few to many rows, float32 ones among them, with few output tiles; and for many rows of 16 bits the
+ * dequantized weight.  A transposed product given no workspace runs unsplit. */
 NVQ_API size_t nvq_quantized_matmul_workspace_bytes(const nvq_qmm_desc *desc);
 
 /* GpuEval::quantized_matmul / fp_quantized_matmul (gpu.rs:6934-7168, 6336-6577); values of

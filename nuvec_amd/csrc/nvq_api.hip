@@ -689,14 +689,19 @@ static int32_t quantized_matmul_any(const nvq_qmm_desc *d, const void *x, const 
     }
 }
 
-const char *nvq_quantized_matmul_route(const nvq_qmm_desc *d) {
+// The names of a product's route and of the kernel that runs it; `kernel` alone looks beyond the route.
+static const char *name_of(const nvq_qmm_desc *d, bool kernel) {
     if (check_qmm(d, "quantized_matmul") != NVQ_OK || check_grid(d) != NVQ_OK || require_device() != NVQ_OK) return nullptr;
     int64_t batch = 1;
     for (int i = 0; i < d->batch_ndim; i++) batch *= d->batch_shape[i];
     ProductArgs a = product_args(d, batch);
     a.x = a.w = a.scales = a.biases = reinterpret_cast<const void *>(uintptr_t{256});  // operands aligned as hipMalloc aligns them
     a.y = reinterpret_cast<void *>(uintptr_t{256});
-    switch (pick_route(d, a)) {
+    const Route route = pick_route(d, a);
+    qms::Plan split;
+    if (kernel && split_rows_take(a, route, split)) return qms_kernel_name(split);
+    if (kernel && route == Route::kTiled && qmm_dense_takes(a)) return "qmm_dense_kernel";
+    switch (route) {
     case Route::kUntransposed: return qvm_kernel_name(a);
     case Route::kTiled: return "qmm_kernel";
     case Route::kTiledF32: return "qmm_f32_kernel";
@@ -707,6 +712,10 @@ const char *nvq_quantized_matmul_route(const nvq_qmm_desc *d) {
     default: return qmv_kernel_name(a);
     }
 }
+
+const char *nvq_quantized_matmul_route(const nvq_qmm_desc *d) { return name_of(d, false); }
+
+const char *nvq_quantized_matmul_kernel(const nvq_qmm_desc *d) { return name_of(d, true); }
 
 int32_t nvq_quantized_matmul(const nvq_qmm_desc *d, const void *x, const void *w, const void *scales, const void *biases,
                              void *y, void *workspace, void *stream) {

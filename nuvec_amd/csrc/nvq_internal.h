@@ -152,6 +152,7 @@ struct Plan {
 }  // namespace qms
 bool qms_plan(const ProductArgs &a, qms::Plan &plan);  // false: the kernel does not take the product
 size_t qms_workspace_bytes(const ProductArgs &a, const qms::Plan &plan);
+const char *qms_kernel_name(const qms::Plan &plan);
 int32_t launch_qms(const ProductArgs &a, const qms::Plan &plan, void *workspace, hipStream_t s);  // workspace NULL: no split
 int32_t launch_fill_zero(void *p, int64_t bytes, hipStream_t s);
 int32_t launch_quantized_attention(const nvq_attention_desc &d, const void *q, const void *kw, const void *ks, const void *kb,

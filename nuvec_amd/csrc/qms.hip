@@ -48,6 +48,19 @@ size_t qms_workspace_bytes(const ProductArgs &a, const qms::Plan &p) {
     return p.splits > 1 ? (size_t)p.splits * (size_t)a.m * (size_t)a.n * sizeof(float) : 0;
 }
 
+const char *qms_kernel_name(const qms::Plan &p) {
+    switch (100 * p.mt + 10 * p.nt + p.qw) {
+    case 111: return "qms_kernel<1,1,1>";
+    case 121: return "qms_kernel<1,2,1>";
+    case 114: return "qms_kernel<1,1,4>";
+    case 211: return "qms_kernel<2,1,1>";
+    case 214: return "qms_kernel<2,1,4>";
+    case 224: return "qms_kernel<2,2,4>";
+    case 414: return "qms_kernel<4,1,4>";
+    default: return "qms_kernel<4,2,4>";
+    }
+}
+
 int32_t launch_qms(const ProductArgs &args, const qms::Plan &p, void *workspace, hipStream_t s) {
     ProductArgs a = args;
     a.k_splits = workspace != nullptr ? p.splits : 1;

@@ -457,9 +457,20 @@ def quantized_matmul(x: torch.Tensor, q: Quantized, transpose: bool = True, *, r
 
 def quantized_matmul_route(m: int, n: int, k: int, quant: Quant, dtype: torch.dtype, *, batch=1, transpose: bool = True,
                            row_exact: bool = False, rows: bool = False, device: int = 0) -> str:
-    """The kernel a product of `m` rows of x per item ([.., m, k] times `batch` weight matrices [n, k] — a count or a
-    tuple of batch dimensions —, or one matrix when `batch` is 1) runs on, from the library's own routing code: what the reference's tests read from the kernel
-    names (tests/quantized.rs:843-861)."""
+    """The route of a product of `m` rows of x per item ([.., m, k] times `batch` weight matrices [n, k] — a count or a
+    tuple of batch dimensions —, or one matrix when `batch` is 1), under the name of the kernel that stands for it, from the library's own
+    routing code: what the reference's tests read from the kernel names (tests/quantized.rs:843-861)."""
+    return _product_name("nvq_quantized_matmul_route", m, n, k, quant, dtype, batch, transpose, row_exact, rows, device)
+
+
+def quantized_matmul_kernel(m: int, n: int, k: int, quant: Quant, dtype: torch.dtype, *, batch=1, transpose: bool = True,
+                            row_exact: bool = False, rows: bool = False, device: int = 0) -> str:
+    """The kernel that runs such a product: its route's, or on the routes of several 16-bit rows `qms_kernel<..>` or
+    `qmm_dense_kernel`."""
+    return _product_name("nvq_quantized_matmul_kernel", m, n, k, quant, dtype, batch, transpose, row_exact, rows, device)
+
+
+def _product_name(query, m, n, k, quant, dtype, batch, transpose, row_exact, rows, device) -> str:
     _lib.check(_lib.load().nvq_init(device))
     d = _lib.QmmDescC()
     d.quant, d.dtype, d.transpose, d.row_exact, d.rows = quant._c(), _CODE[dtype], int(transpose), int(row_exact), int(rows)
@@ -472,7 +483,7 @@ def quantized_matmul_route(m: int, n: int, k: int, quant: Quant, dtype: torch.dt
         d.batch_shape[i] = dims[i]
         d.x_strides[i], d.w_strides[i], d.s_strides[i] = items * m * k, items * n * k * quant.bits // 32, items * n * k // quant.group_size
         items *= dims[i]
-    name = _lib.load().nvq_quantized_matmul_route(C.byref(d))
+    name = getattr(_lib.load(), query)(C.byref(d))
     if name is None:
         raise Unsupported(_lib.last_error())
     return name.decode()

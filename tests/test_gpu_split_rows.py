@@ -78,6 +78,22 @@ def test_bias_determinism_and_both_entry_points(m, n, k):
     assert torch.equal(odd[keep], plain[keep])
 
 
+def test_the_query_names_the_kernel_that_runs():
+    """The routes of several 16-bit rows keep their names; the kernel behind them has its own query."""
+    both = lambda *a, **k: (ops.quantized_matmul_route(*a, **k), ops.quantized_matmul_kernel(*a, **k))
+    q4, bf16 = nv.Quant.affine(64, 4), torch.bfloat16
+    route, kernel = both(20, 9001, 2112, q4, bf16)
+    assert route in ("qmf_kernel", "qmm_kernel") and kernel.startswith("qms_kernel<2,")
+    assert both(31, 404, 13792, nv.Quant.new(nv.QuantMode.NVFP4), bf16)[1].startswith("qms_kernel<")
+    assert both(517, 4096, 4096, nv.Quant.affine(64, 3), bf16) == ("qmm_kernel", "qmm_dense_kernel")
+    assert both(300, 64, 128, q4, bf16) == ("qmm_kernel", "qmm_kernel")
+    for same in ((1, 14336, 4096, q4, bf16), (16, 4096, 4096, q4, bf16), (64, 14336, 4096, q4, bf16), (33, 4096, 4096, q4, torch.float32)):
+        assert len(set(both(*same))) == 1
+    assert len(set(both(4, 4096, 4096, q4, bf16, transpose=False))) == 1
+    with pytest.raises(nv.Unsupported):
+        ops.quantized_matmul_kernel(1, 64, 64, q4, bf16, batch=70000)
+
+
 def test_no_rounding_where_the_weights_and_sums_are_exact():
     """Small whole numbers: every cut of K gives the exact sums."""
     m, n, k = 20, 3000, 4128

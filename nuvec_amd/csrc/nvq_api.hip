@@ -595,12 +595,28 @@ static bool takes_tiled(const nvq_qmm_desc *d, const ProductArgs &a) {
 enum class Route { kUntransposed, kVector, kTiled, kTiledF32, kGroupedRows, kBatchedDecode, kFewRowsDirect, kFewRows };
 static Route pick_route(const nvq_qmm_desc *d, const ProductArgs &a);
 
-// Whether a product of either matrix-core route of 16-bit rows runs on the split-K kernel (the route keeps its name): where that is
-// estimated up to a tenth above the few-row kernel (whose estimate is the lower one: 630 products, 0.74 of its time, 1.17 x at
-// worst) or a tenth below the tiles (448 products, 0.76 of the time, 1.09 x at worst; from 65 rows on most stay there, and beyond 256 all).
+// Whether the split-K kernel is a candidate for a product of either matrix-core route of 16-bit rows: estimated up to a tenth above the
+// few-row kernel or a tenth below the tiles, from 65 rows on most of which stay there; beyond 256 rows it was not timed.
+static bool split_rows_bid(const ProductArgs &a, Route route, qms::Plan &plan) {
+    if (route != Route::kFewRows && (route != Route::kTiled || a.m > 256)) return false;
+    return qms_plan(a, plan) && (route == Route::kFewRows ? plan.us < 1.1 * few_rows_us(a) : plan.us < 0.9 * tiled_us(a));
+}
+
+// Whether it takes the product (the route keeps its name).  The estimates were fitted to other products than those between which this
+// choice lies: on 3000 of those (2 to 256 rows, W[256..16384, 512..14336], all formats of 16-bit rows, timed on both sides) the
+// few-row kernel's is 0.24 off, by rows above all, and that of the cut 0.12, so each is first corrected by what it misses there
+// (0.11 and 0.08 are left).  That brings all 3000 to 0.70 of the other kernels' time, as taking every candidate does, with 32 more than
+// 5 % slower, 1.20 x at worst, where all candidates would give 132 and 1.69 x (us, the few-row kernel / here: 8 bits
+// W[8118,3328] at 4 rows 12.5 / 20.2, W[6907,3712] at 10 rows 11.6 / 17.9).
 static bool split_rows_take(const ProductArgs &a, Route route, qms::Plan &plan) {
-    if ((route != Route::kFewRows && route != Route::kTiled) || !qms_plan(a, plan)) return false;
-    return route == Route::kFewRows ? plan.us < 1.1 * few_rows_us(a) : a.m <= 256 && plan.us < 0.9 * tiled_us(a);
+    if (!split_rows_bid(a, route, plan)) return false;
+    double here = plan.us * (plan.mt == 1 ? (a.k < 1100 ? 0.93 : 1.02) : plan.mt == 2 && plan.qw == 1 ? (a.k < 700 ? 1.0 : a.k < 1100 ? 1.1 : 1.18) : (a.k < 1600 ? 1.02 : 1.1));
+    if (plan.nt == 2) here *= plan.qw == 1 && a.bits == 8 ? 1.45 : 1.08;
+    if (a.bits == 5 || a.bits == 6 || a.bits == 8) here *= 1.04;
+    if (route == Route::kTiled) return here < (a.mode == NVQ_MXFP8 ? 0.9 : 1.07) * tiled_us(a);
+    const bool exact = a.exact_weights != 0;
+    const double rows = a.m <= 16 ? 0.64 + 0.01 * (double)a.m : a.m <= 24 ? (exact ? 0.9 : 1.03) : (exact ? 1.03 : 1.17);
+    return here < (rows + (a.k < 1600 ? 0.2 : a.k < 2600 ? 0.1 : 0.0)) * (a.bits == 2 && a.m <= 16 ? 0.85 : 1.0) * few_rows_us(a);
 }
 
 // `dense`: whether the workspace may hold the dequantized weight.
@@ -777,7 +793,8 @@ int32_t nvq_quantized_matmul_glu(const nvq_qmm_desc *d, int32_t activation, floa
 // kernels that hold a weight no more precisely (rounded once; block formats hold it exactly on every kernel), and the bounds of
 // 700 pairs timed both ways leave it ahead (3 to 256 rows, K 512 to 5120, 1024 to 14336 hidden values, twelve formats: 0.75 of the time
 // of the two products and the activation, 0.71 where taken, 1.04 x at worst; from six rows on).  By estimate beside the few-row kernel,
-// the tiles and itself.  Left to the two products: 8-bit codes up to 16 rows beyond 24 M of both (W[2176,4992] at 15 rows
+// the tiles and itself (of 700 others that it takes 0.59 of the time, one slower than 1.05 x; MXFP8 beside the tiles, whose estimate is high there,
+// below 0.65 of it: W[5952,4800] at 96 rows 50.7 there, 57.7 here).  Left to the two products: 8-bit codes up to 16 rows beyond 24 M of both (W[2176,4992] at 15 rows
 // 20.9 us there, 19.2 here), MXFP8 and NVFP4 up to 16 rows of the direct few-row kernel beyond 32 M (NVFP4
 // W[5184,3584] at 11 rows 17.5 / 20.0) and MXFP4 beyond 32 rows (W[1088,2048] at 98 rows 12.7 / 14.0; 32 rows W[5056,512] 14.2 / 7.9),
 // and of the batched-decode kernel 4 bits at up to 48 rows beyond K = 1536 (groups of 32, W[14272,2048] at 22 rows 23.4 / 26.0; W[13760,512]
@@ -793,8 +810,8 @@ static bool gated_rows_take(const nvq_qmm_desc *d, const ProductArgs &a, qms::Pl
     if (route == Route::kBatchedDecode) return a.bits == 4 ? a.k <= 1536 || a.m > 48 : a.k <= 1024 && a.m > 16;
     if ((route != Route::kFewRows && route != Route::kTiled) || (a.mode == NVQ_AFFINE && a.bits == 8 && a.m <= 16 && codes > 24.0e6)) return false;
     qms::Plan split;
-    if (split_rows_take(one, route, split)) return plan.us < 4.0 + 2.0 * split.us;
-    return plan.us < (route == Route::kTiled ? 0.8 * (4.0 + 2.0 * tiled_us(one)) : 4.0 + 2.0 * few_rows_us(one));
+    if (split_rows_bid(one, route, split)) return plan.us < 4.0 + 2.0 * split.us;
+    return plan.us < (route == Route::kTiled ? (a.mode == NVQ_MXFP8 ? 0.65 : 0.8) * (4.0 + 2.0 * tiled_us(one)) : 4.0 + 2.0 * few_rows_us(one));
 }
 
 size_t nvq_quantized_matmul_glu_rows_workspace_bytes(const nvq_qmm_desc *d) {

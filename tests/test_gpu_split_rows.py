@@ -94,6 +94,21 @@ def test_the_query_names_the_kernel_that_runs():
         ops.quantized_matmul_kernel(1, 64, 64, q4, bf16, batch=70000)
 
 
+@pytest.mark.parametrize("m,n,k,fmt,dtype,route", [
+    (4, 8118, 3328, (64, 8), torch.float16, "qmf_kernel"),     # 12.5 us there, 20.2 on the split-K kernel
+    (13, 12640, 1920, (64, 8), torch.float16, "qmf_kernel"),   # 12.2 / 18.9
+    (10, 6907, 3712, (128, 8), torch.bfloat16, "qmf_kernel"),  # 11.6 / 17.9
+    (7, 4249, 3968, "MXFP8", torch.bfloat16, "qmf_kernel"),    # 9.6 / 12.1
+    (14, 5482, 13824, "MXFP8", torch.bfloat16, "qmf_kernel"),  # 28.6 / 34.1
+    (126, 7681, 6016, "MXFP8", torch.float16, "qmm_kernel"),   # 28.3 / 38.3
+    (220, 3113, 5440, "MXFP8", torch.bfloat16, "qmm_kernel"),  # 26.9 / 35.4
+])
+def test_what_the_estimates_alone_would_take(m, n, k, fmt, dtype, route):
+    """Products that the bare estimates hand to the split-K kernel, and that are faster on their route's own."""
+    quant = nv.Quant.new(getattr(nv.QuantMode, fmt)) if isinstance(fmt, str) else nv.Quant.affine(*fmt)
+    assert ops.quantized_matmul_route(m, n, k, quant, dtype) == ops.quantized_matmul_kernel(m, n, k, quant, dtype) == route
+
+
 def test_no_rounding_where_the_weights_and_sums_are_exact():
     """Small whole numbers: every cut of K gives the exact sums."""
     m, n, k = 20, 3000, 4128

@@ -10,7 +10,8 @@
 //     group's sum X of x.  The biases' part is a product of its own, over groups, on the float32 instruction.
 // A weight's own two roundings (crates/nuvec-core/src/kernels.rs:835-859, 992-998), which the CPU's product keeps, are not made.
 // What the split of x does not hold, an infinity or a magnitude whose sums of codes leave float32, comes out of it as no finite
-// number: a wavefront with such an output multiplies its tiles again, on the float32 instruction.  Magnitudes below 2^-100 keep 2^-126.
+// number: a wavefront with such an output multiplies its tiles again, on the float32 instruction.  2^26 keeps the
+// last term of the least float32, 2^-149, a normal operand; without it magnitudes below 2^-109 lost bits (near 2^-120 all but eight).
 //
 // A block of four wavefronts owns 16 MT rows of x and 64 NT weight rows (16 NT a wavefront) and walks its share of K in steps
 // of 64.  x goes through registers, where it is split and its groups' sums are formed, into one of two LDS stages, a step ahead;
@@ -36,6 +37,7 @@ constexpr int kWaves = 4, kThreads = 64 * kWaves;
 constexpr int kTile = 16;   // rows of x, weight rows of a matrix instruction
 constexpr int kStep = 64;   // values of K between two barriers
 constexpr int kSpan = 256;  // values of K of which a lane brings scales and biases; a split of K holds whole ones
+constexpr float kLift = 67108864.0f;  // 2^26
 
 template <int BITS, int MODE, int MT, int NT>
 struct Shape {
@@ -186,6 +188,8 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
 #pragma unroll
         for (int m = 0; m < MT; m++) {
             float (&r)[4] = xs[set][m];
+#pragma unroll
+            for (int j = 0; j < 4; j++) r[j] *= kLift;
             if constexpr (kAffine) {
                 float sum = (r[0] + r[1]) + (r[2] + r[3]);
                 sum += lane_swap<0xB1>(sum);
@@ -413,6 +417,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 if (kNv) acc[m][t][e] *= factor;
+                acc[m][t][e] *= 1.0f / kLift;
                 plain |= !(fabsf(acc[m][t][e]) < INFINITY);
             }
     // Outputs that are no finite number: the wavefront's tiles again from whole values of x and the CPU's weights on the float32

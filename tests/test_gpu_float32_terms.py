@@ -75,6 +75,29 @@ def test_magnitudes_that_three_terms_do_not_hold(fmt):
     assert np.array_equal(got[same], plain[same])
 
 
+@pytest.mark.parametrize("fmt", [(64, 4), (32, 3), (128, 8), (64, 1), "MXFP4", "MXFP8", "NVFP4"], ids=str)
+@pytest.mark.parametrize("k", [512, 2048])
+def test_magnitudes_at_the_low_end_of_float32(fmt, k):
+    """Rows of x down to the subnormal numbers keep all of their bits, alone and (block formats, where a zero is code zero and not a
+    difference) beside ordinary values whose weights are zero.  A result of the least rows is itself near the end, 2^-149: half of
+    that is allowed beside the bound above."""
+    rng = np.random.default_rng(6250)
+    m, n = 48, 5000
+    w = make_w(rng, n, k, ref.F32) * np.float32(256.0)
+    w[:, :128] = 0.0
+    powers = np.array([0, -60, -95, -100, -104, -109, -112, -116, -120, -124, -126, -128], dtype=np.int32)
+    x = np.ldexp(make_x(rng, m, k, ref.F32), powers[np.arange(m) % len(powers)][:, None]).astype(np.float32)
+    if isinstance(fmt, str):
+        x[24:, :128] = make_x(rng, 24, 128, ref.F32)
+    q, dense = quantized(fmt, w)
+    assert ops.quantized_matmul_route(m, n, k, q.quant, torch.float32) == "qmm_f32_kernel"
+    want = x.astype(np.float64) @ dense.T
+    for scratch in (True, False):
+        got = to_host(ops.quantized_matmul(to_dev(x), q, scratch=scratch)).astype(np.float64)
+        for row in range(m):
+            assert np.linalg.norm(got[row] - want[row]) <= LIMIT * np.linalg.norm(want[row]) + np.sqrt(n) * 2.0 ** -150, (row, powers[row % len(powers)])
+
+
 @pytest.mark.parametrize("fmt", [(64, 4), (32, 3), (128, 8), (32, 5), "MXFP4", "MXFP8", "NVFP4"], ids=str)
 @pytest.mark.parametrize("m,n,k", [(70, 5001, 544), (33, 4096, 2048)])
 def test_a_batch_of_infinities_and_nans(fmt, m, n, k):

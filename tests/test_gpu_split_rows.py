@@ -1,6 +1,6 @@
 """Products of a few to a few dozen rows on the split-K kernel (`qms_kernel`), which the few-row and tiled routes hand what it is estimated
 faster at: against the CPU's product (crates/nuvec-core/src/kernels.rs:1091-1142), at the ends of its turns of 256 values, its chunks
-of codes, its tiles of rows and weight rows, in every shape of block and with K split over the grid or not."""
+of codes, its tiles of rows and weight rows; and in every shape of block that it has, with K split over the grid and not."""
 import ctypes as C
 
 import numpy as np
@@ -56,6 +56,35 @@ def test_every_format_against_the_cpu_product(fmt, dtype):
             assert_rows_close(got, want, dtype, f"split rows {fmt} M={m} N={n} K={k} scratch={scratch}", exact_weights=isinstance(fmt, str))
 
 
+@pytest.mark.parametrize("shape,split,fmt,dtype,m,n,k", [
+    ("1,1,1", False, (64, 4), ref.BF16, 9, 18734, 1600),
+    ("1,2,1", False, (64, 3), ref.BF16, 16, 7039, 1984),
+    ("1,2,1", True, "MXFP4", ref.F16, 12, 5333, 8224),
+    ("1,2,1", True, (64, 2), ref.BF16, 8, 1825, 8064),
+    ("1,1,4", False, "MXFP8", ref.F16, 9, 13587, 736),
+    ("1,1,4", True, (32, 8), ref.F16, 10, 1491, 5056),
+    ("2,1,1", False, (64, 4), ref.F16, 20, 9001, 2112),
+    ("2,1,1", True, (64, 8), ref.F16, 20, 4822, 8064),
+    ("2,1,4", False, (32, 4), ref.BF16, 19, 15569, 576),
+    ("2,1,4", True, (128, 4), ref.F16, 27, 1644, 4608),
+    ("2,2,4", True, (128, 6), ref.F16, 30, 4432, 6528),
+    ("2,2,4", True, (32, 2), ref.BF16, 20, 5737, 5408),
+    ("4,1,4", False, (32, 4), ref.BF16, 64, 5000, 480),
+    ("4,1,4", True, (64, 4), ref.BF16, 62, 1030, 11072),
+    ("4,2,4", False, "NVFP4", ref.F16, 70, 11444, 928),
+    ("4,2,4", True, (128, 3), ref.F16, 39, 5444, 1664),
+])
+def test_every_shape_of_block(shape, split, fmt, dtype, m, n, k):
+    rng = np.random.default_rng(7350 + m)
+    q, x, want = product(rng, fmt, m, n, k, dtype)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:  # (the cut is chosen by the compute units)
+        assert ops.quantized_matmul_kernel(m, n, k, q.quant, torch.bfloat16 if dtype == ref.BF16 else torch.float16) == f"qms_kernel<{shape}>"
+        assert (workspace_bytes(m, n, k, q.quant, dtype) > 0) == split
+    for scratch in (True, False):
+        got = to_host(ops.quantized_matmul(to_dev(x), q, scratch=scratch))
+        assert_rows_close(got, want, dtype, f"split rows {shape} {fmt} M={m} N={n} K={k} scratch={scratch}", exact_weights=isinstance(fmt, str))
+
+
 @pytest.mark.parametrize("m,n,k", [(16, 4096, 11008), (62, 2560, 11072), (31, 404, 13792)])
 def test_bias_determinism_and_both_entry_points(m, n, k):
     """QuantizedLinear's bias is the separate addition bit for bit (crates/nuvec-nn/src/layers.rs:155-162) after a split of K as before it;
@@ -107,6 +136,23 @@ def test_what_the_estimates_alone_would_take(m, n, k, fmt, dtype, route):
     """Products that the bare estimates hand to the split-K kernel, and that are faster on their route's own."""
     quant = nv.Quant.new(getattr(nv.QuantMode, fmt)) if isinstance(fmt, str) else nv.Quant.affine(*fmt)
     assert ops.quantized_matmul_route(m, n, k, quant, dtype) == ops.quantized_matmul_kernel(m, n, k, quant, dtype) == route
+
+
+@pytest.mark.parametrize("dtype", [ref.BF16, ref.F16])
+@pytest.mark.parametrize("fmt", [(64, 2), (32, 3), (64, 4), (32, 4), (128, 5), (32, 6), (32, 8), (64, 8), "MXFP4", "MXFP8", "NVFP4"], ids=str)
+def test_the_few_row_kernel_keeps_batches(fmt, dtype):
+    """The split-K kernel takes one product: batches stay on the few-row kernel, with weights rounded once and (fewer than 1024 outputs)
+    with the CPU's."""
+    rng = np.random.default_rng(7450)
+    for b, m, n, k in ((2, 12, 1100, 2304), (3, 7, 2060, 1152), (2, 16, 700, 6272)):
+        items = [product(rng, fmt, m, n, k, dtype) for _ in range(b)]
+        stack = lambda of: None if of(items[0]) is None else torch.stack([of(i) for i in items])
+        q = nv.Quantized(stack(lambda i: i[0].weight), stack(lambda i: i[0].scales), stack(lambda i: i[0].biases), items[0][0].quant)
+        kernel = ops.quantized_matmul_kernel(m, n, k, q.quant, torch.bfloat16 if dtype == ref.BF16 else torch.float16, batch=b)
+        assert kernel == "qmf_kernel", (b, m, n, k)
+        got = to_host(ops.quantized_matmul(stack(lambda i: to_dev(i[1])), q))
+        for i in range(b):
+            assert_rows_close(got[i], items[i][2], dtype, f"few rows {fmt} item {i} of {b}, M={m} N={n} K={k}", exact_weights=isinstance(fmt, str))
 
 
 def test_no_rounding_where_the_weights_and_sums_are_exact():

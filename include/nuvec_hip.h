@@ -436,6 +436,9 @@ NVQ_API int32_t nvq_quantized_matmul_glu(const nvq_qmm_desc *desc, int32_t activ
  * desc alone), or NULL: K is then not split over the grid.  NVQ_UNSUPPORTED where the two products and nvq_glu are estimated faster, or
  * would hold their weights more precisely. */
 NVQ_API size_t nvq_quantized_matmul_glu_rows_workspace_bytes(const nvq_qmm_desc *desc);
+/* 1: it takes the product (with operands that the launch accepts), and `workspace_bytes`, if not NULL, is the size query's answer; 0: it
+ * does not.  Depends on desc alone. */
+NVQ_API int32_t nvq_quantized_matmul_glu_rows_takes(const nvq_qmm_desc *desc, size_t *workspace_bytes);
 NVQ_API int32_t nvq_quantized_matmul_glu_rows(const nvq_qmm_desc *desc, int32_t activation, float alpha, float limit, const void *x,
                                 const void *w, const void *scales, const void *biases, const void *bias, void *y,
                                 void *workspace, void *stream);

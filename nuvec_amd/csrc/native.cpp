@@ -198,6 +198,13 @@ bool product(const Tensor &x, const Packed &p, const Tensor &bias, Flags f, Tens
     return true;
 }
 
+nvq_qmm_desc gated_desc(const Tensor &x, int32_t code, const nvq_quant &q, int64_t n) {
+    nvq_qmm_desc d{};
+    d.quant = q, d.dtype = code, d.transpose = 1;
+    d.m = x.numel() / x.size(-1), d.n = n, d.k = x.size(-1), d.item_rows = x.dim() > 1 ? x.size(-2) : 1;
+    return d;
+}
+
 // ops.quantized_matmul_glu, or (`several`) ops.quantized_matmul_glu_rows.
 bool product_glu(const Tensor &x, const Packed &p, const Tensor &bias, int32_t activation, float alpha, float limit, bool several,
                  Tensor &out) {
@@ -208,10 +215,9 @@ bool product_glu(const Tensor &x, const Packed &p, const Tensor &bias, int32_t a
     if (code < 0 || !p.fits(at, x.scalar_type(), 2, columns) || x.size(-1) != columns) return false;
     const int64_t n = p.w.size(0);
     if (n == 0 || n % 128 != 0 || !bias_fits(bias, at, x.scalar_type(), n)) return false;
-    nvq_qmm_desc d{};
-    d.quant = p.q, d.dtype = code, d.transpose = 1;
-    d.m = x.numel() / columns, d.n = n, d.k = columns, d.item_rows = x.dim() > 1 ? x.size(-2) : 1;
-    const size_t need = several ? nvq_quantized_matmul_glu_rows_workspace_bytes(&d) : 0;
+    const nvq_qmm_desc d = gated_desc(x, code, p.q, n);
+    size_t need = 0;
+    if (several && !nvq_quantized_matmul_glu_rows_takes(&d, &need)) return false;
     Tensor workspace, y = at.empty(with_last(x.sizes(), n / 2), x.scalar_type());
     if (need > 0) workspace = at.empty({(int64_t)need}, at::kByte);
     const int32_t rc = several ? nvq_quantized_matmul_glu_rows(&d, activation, alpha, limit, ptr(x), ptr(p.w), ptr(p.s), ptr(p.b), ptr(bias),
@@ -460,7 +466,12 @@ PyObject *py_mlp(PyObject *, PyObject *const *args, Py_ssize_t n) {
         const at::ScalarType type = x.scalar_type();
         if (!linear_fits(gate, at, type, x.size(-1)) || !linear_fits(down, at, type, gate.p.w.size(0))) return none();
         const bool several = rows > most;
-        if (both.p != Py_None) {
+        bool paired = both.p != Py_None;
+        if (paired && several) {  // (what the projections' sizes say already: the pair is not read where it would be refused)
+            const nvq_qmm_desc d = gated_desc(x, code_of(type), gate.p.q, 2 * gate.p.w.size(0));
+            paired = nvq_quantized_matmul_glu_rows_takes(&d, nullptr);
+        }
+        if (paired) {
             const bool fits = read_linear(both.p, fused) && linear_fits(fused, at, type, x.size(-1)) && fused.p.w.size(0) == 2 * gate.p.w.size(0);
             if (!fits && !several) return none();
             if (fits) {

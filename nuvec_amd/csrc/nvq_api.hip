@@ -814,13 +814,22 @@ static bool gated_rows_take(const nvq_qmm_desc *d, const ProductArgs &a, qms::Pl
     return plan.us < (route == Route::kTiled ? (a.mode == NVQ_MXFP8 ? 0.65 : 0.8) * (4.0 + 2.0 * tiled_us(one)) : 4.0 + 2.0 * few_rows_us(one));
 }
 
-size_t nvq_quantized_matmul_glu_rows_workspace_bytes(const nvq_qmm_desc *d) {
+int32_t nvq_quantized_matmul_glu_rows_takes(const nvq_qmm_desc *d, size_t *workspace_bytes) {
+    if (workspace_bytes != nullptr) *workspace_bytes = 0;
     if (check_qmm(d, "quantized_matmul") != NVQ_OK || d->m == 0 || d->n == 0 || d->k == 0 || !d->transpose || d->batch_ndim != 0 || require_device() != NVQ_OK) return 0;
     ProductArgs a = product_args(d, 1);
     a.exact_weights = wants_exact_weights(d->quant.mode, d->dtype, d->n / 2, d->m);
     a.glu = 1;
     qms::Plan plan;
-    return gated_rows_take(d, a, plan) ? qms_workspace_bytes(a, plan) : 0;
+    if (!gated_rows_take(d, a, plan)) return 0;
+    if (workspace_bytes != nullptr) *workspace_bytes = qms_workspace_bytes(a, plan);
+    return 1;
+}
+
+size_t nvq_quantized_matmul_glu_rows_workspace_bytes(const nvq_qmm_desc *d) {
+    size_t bytes;
+    (void)nvq_quantized_matmul_glu_rows_takes(d, &bytes);
+    return bytes;
 }
 
 int32_t nvq_quantized_matmul_glu_rows(const nvq_qmm_desc *d, int32_t activation, float alpha, float limit, const void *x, const void *w,

@@ -108,3 +108,25 @@ def test_block_native_and_composed_agree(form, shape, monkeypatch):
     monkeypatch.setattr(_lib, "_native", Declines())
     monkeypatch.setattr(layers, "_native", Declines())
     assert torch.equal(y, mlp(x))
+
+
+@pytest.mark.parametrize("rows", [4, 8, 16, 300])
+def test_what_is_refused_costs_no_allocation(rows):
+    """An MLP whose gate and up projections stay two products takes as many allocations with the pair beside them as without it."""
+    quant = nv.Quant.affine(64, 4)
+    (gate, up), make = _projections(quant, 1024, 512, torch.bfloat16, False, rows)
+    q = nv.quantize((make(512, 1024) * 0.03).to(torch.bfloat16), quant)
+    down = layers.QuantizedLinear(q.weight, q.scales, q.biases, None, quant)
+    alone, paired = layers.Mlp(gate, up, down), layers.Mlp(gate, up, down).fuse_gate_up()
+    x = make(rows, 512).to(torch.bfloat16)
+    with pytest.raises(nv.Unsupported):
+        p = paired.gate_up_proj
+        ops.quantized_matmul_glu_rows(x, p.quantized(), "swiglu", bias=p.bias)
+
+    def allocations(block):
+        block(x)
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        block(x)
+        return torch.cuda.memory_stats()["allocation.all.allocated"] - before
+
+    assert allocations(paired) == allocations(alone)

@@ -5,13 +5,13 @@
 // v_mfma_f32_16x16x32_bf16 multiplies sixteen times as much a cycle as the float32 instruction and its products are exact, so
 // no precision is given up for it:
 //   * a code is an exact bfloat16 (integers up to 255, E2M1, E4M3; NVFP4's code times its E4M3 scale has six bits);
-//   * x is the exact sum of three bfloat16 terms of eight bits each, cut off toward zero;
+//   * x, times 2^26, is the exact sum of three bfloat16 terms of eight bits each, cut off toward zero;
 //   * a group's sum P of x times code is formed from the smallest terms up in float32, then y += scale P + bias X with the
 //     group's sum X of x.  The biases' part is a product of its own, over groups, on the float32 instruction.
 // A weight's own two roundings (crates/nuvec-core/src/kernels.rs:835-859, 992-998), which the CPU's product keeps, are not made.
 // What the split of x does not hold, an infinity or a magnitude whose sums of codes leave float32, comes out of it as no finite
-// number: a wavefront with such an output multiplies its tiles again, on the float32 instruction.  2^26 keeps the
-// last term of the least float32, 2^-149, a normal operand; without it magnitudes below 2^-109 lost bits (near 2^-120 all but eight).
+// number: a wavefront with such an output multiplies its tiles again, on the float32 instruction.  2^26 makes the
+// last term of the least float32, 2^-149, a normal operand (without it magnitudes below 2^-109 lose bits, near 2^-120 most of them).
 //
 // A block of four wavefronts owns 16 MT rows of x and 64 NT weight rows (16 NT a wavefront) and walks its share of K in steps
 // of 64.  x goes through registers, where it is split and its groups' sums are formed, into one of two LDS stages, a step ahead;
@@ -19,7 +19,7 @@
 // layout through a wavefront's own piece of LDS.  Scales and biases come once a span of 256 values, a lane its quarter's.
 // Few tiles: K is split over the grid, and qmm_f32_reduce_kernel adds the parts.
 //
-// What bounds it: a step's vector instructions, two of three for the split of x (a step of 48 rows and 64 weight rows takes 200
+// What bounds it: a step's vector instructions, two of three for the split of x (a step of 48 rows and 64 weight rows takes 210
 // beside 23 matrix instructions, 0.65 us a compute unit; two blocks on one gain a tenth).  Every wavefront reading the
 // operands of both halves of a step at once, ahead of the next step's split, gave 0.1 us a step; codes and scales brought
 // by each lane for itself, straight in the operand layout, with no LDS and no barrier, was slower by half (16 lines a

@@ -407,6 +407,8 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
         });
     }
 
+    // (the lane's number anew: kept through the loop for these addresses it cost registers, in some shapes a wavefront a SIMD)
+    const int end_lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), el = end_lane & 15, eq = end_lane >> 4;
     const float factor = kNv ? qmf::nvfp4_factor(a, 0) : 1.0f;
     float *y = a.k_splits > 1 ? a.partials + (int64_t)blockIdx.z * M * N : (float *)a.y;
     bool plain = false;
@@ -430,16 +432,16 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
             for (int t = 0; t < NT; t++) again[m][t] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 2
         for (int from = k0; from < k1; from += 16) {
-            const int k = from + 4 * q;
+            const int k = from + 4 * eq;
             floatx4_t xv[MT], wv[NT];
 #pragma unroll
             for (int m = 0; m < MT; m++) {
-                const int row = m0 + kTile * m + l;
+                const int row = m0 + kTile * m + el;
                 xv[m] = *reinterpret_cast<const floatx4_t *>((const float *)a.x + (int64_t)(row < M ? row : M - 1) * K + k);
             }
 #pragma unroll
             for (int t = 0; t < NT; t++) {
-                const int n = n0 + kTile * t + l;
+                const int n = n0 + kTile * t + el;
                 wv[t] = plain_weights<BITS, MODE>(a, n < N ? n : N - 1, k, gshift, factor);
             }
 #pragma unroll
@@ -463,7 +465,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
         for (int t = 0; t < NT; t++)
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const int row = m0 + kTile * m + 4 * q + e, col = n0 + kTile * t + l;
+                const int row = m0 + kTile * m + 4 * eq + e, col = n0 + kTile * t + el;
                 if (row < M && col < N) y[(int64_t)row * N + col] = a.k_splits > 1 ? acc[m][t][e] : add_row_bias<float>(a.row_bias, acc[m][t][e], col);
             }
 }

@@ -596,7 +596,8 @@ enum class Route { kUntransposed, kVector, kTiled, kTiledF32, kGroupedRows, kBat
 static Route pick_route(const nvq_qmm_desc *d, const ProductArgs &a);
 
 // Whether the split-K kernel is a candidate for a product of either matrix-core route of 16-bit rows: estimated up to a tenth above the
-// few-row kernel or a tenth below the tiles, from 65 rows on most of which stay there; beyond 256 rows it was not timed.
+// few-row kernel or a tenth below the tiles, from 65 rows on most of which stay there; beyond 256 rows it was not timed beside the tiles (150
+// products of the few-row kernel of 257 to 2048 rows, few outputs: 0.79 of the time, one more than 5 % slower).
 static bool split_rows_bid(const ProductArgs &a, Route route, qms::Plan &plan) {
     if (route != Route::kFewRows && (route != Route::kTiled || a.m > 256)) return false;
     return qms_plan(a, plan) && (route == Route::kFewRows ? plan.us < 1.1 * few_rows_us(a) : plan.us < 0.9 * tiled_us(a));

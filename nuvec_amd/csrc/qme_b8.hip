@@ -1,0 +1,6 @@
+// The grouped kernel of sorted pairs for affine 8-bit codes (qme_kernel.h).
+#include "qme_kernel.h"
+
+namespace nvq {
+int32_t launch_qme_b8(const ProductArgs &a, hipStream_t s) { return qme::run_dtype<8, rows::kAffine>(a, s); }
+}  // namespace nvq

@@ -1,4 +1,4 @@
-// Routing of the few-row and the grouped matrix-core kernels (qmf_kernel.h, qmg_kernel.h): which products
+// Routing of the few-row and the grouped matrix-core kernels (qmf_kernel.h, qme_kernel.h, qmg_kernel.h): which products
 // they take and the per-width entry points.
 #include "qmg_kernel.h"
 
@@ -72,7 +72,25 @@ bool qmf_supported(const ProductArgs &a) {
     return (a.batch == 1 || a.batch_ndim == 1) && a.batch <= 65535 && (a.m + 31) / 32 <= 65535;
 }
 
+// Sorted pairs whose weights the kernel holds in the element type; affine ones off whole steps that are not the CPU's stay with
+// qmg_kernel's terms.
+static int32_t launch_qme(const ProductArgs &a, hipStream_t s) {
+    if (a.mode == NVQ_MXFP4) return launch_qme_fp4(a, s);
+    if (a.mode == NVQ_MXFP8) return launch_qme_fp8(a, s);
+    if (a.mode == NVQ_NVFP4) return launch_qme_nvfp4(a, s);
+    switch (a.bits) {
+    case 1: return launch_qme_b1(a, s);
+    case 2: return launch_qme_b2(a, s);
+    case 3: return launch_qme_b3(a, s);
+    case 4: return launch_qme_b4(a, s);
+    case 5: return launch_qme_b5(a, s);
+    case 6: return launch_qme_b6(a, s);
+    default: return launch_qme_b8(a, s);
+    }
+}
+
 int32_t launch_qmf(const ProductArgs &a, hipStream_t s) {
+    if (a.offsets != nullptr && (a.mode != NVQ_AFFINE || a.exact_weights || a.k % (a.bits % 2 != 0 ? 128 : 64) == 0)) return launch_qme(a, s);
     if (a.mode == NVQ_MXFP4) return launch_qmf_fp4(a, s);
     if (a.mode == NVQ_MXFP8) return launch_qmf_fp8(a, s);
     if (a.mode == NVQ_NVFP4) return launch_qmf_nvfp4(a, s);

@@ -6,7 +6,7 @@
 namespace nvq {
 
 int32_t launch_qmf_b6(const ProductArgs &a, hipStream_t s) {
-    return a.offsets != nullptr || a.one_group ? qmg::run_dtype<6, false>(a, s) : qmf::run_dtype<6, false>(a, s);
+    return a.offsets != nullptr || a.one_group ? qmg::run_dtype<6>(a, s) : qmf::run_dtype<6, false>(a, s);
 }
 
 int32_t launch_qmm_b6(const ProductArgs &a, void *workspace, hipStream_t s) { return qmm::run_dtype<6, false>(a, workspace, s); }

@@ -91,39 +91,28 @@ struct Geometry {
     __host__ __device__ static constexpr int swizzle(int row) { return kPow2 ? (row / (BITS >= 16 ? 1 : 16 / BITS)) % BITS : 0; }
 };
 
-__host__ __device__ constexpr bool weights_in_terms(int fp4, bool exact, bool ragged) { return ragged && fp4 == kAffine && !exact; }
-
 // GLU: the gated activation of the experts' MLPs as the epilogue (a.glu).  The weights then hold the gate and the up
 // projection in alternating runs of 64 rows, so that a block's wavefronts 0 and 1 own 64 columns of the gate product
 // and wavefronts 2 and 3 the same 64 columns of the up product, lane for lane: after a pass the latter leave their
 // values (rounded as the product's output, the expert's bias added) in LDS, the former combine them with their own
 // and write y [rows, N / 2].
-// EXACT (affine codes): the weights as nuvec's CPU product holds them (affine_pair).
-// RAGGED: K of whole 32 values; without it K is whole steps of 64 (windows of 128 for odd BITS), and the loop is free of the
-// last window's cases (with them everywhere, 256 tokens x 4 of 32 MXFP4 experts [5760, 2880] and [2880, 2880] took 220 us
-// against 190).
-template <typename T, int BITS, int FP4, bool GLU, bool EXACT, bool RAGGED>
-// Three blocks per compute unit (three wavefronts per SIMD): the registers are capped for that, and the LDS of a
-// block (two x stages, the weight stages, the table) fits three times.  Two with weights in terms, whose operands spilled 21 to 70
-// registers at three while a long row's table leaves room for one or two blocks anyway (300 rows, W[8300,3104] in groups of 32, 8 bits
-// 169 -> 125 us, 4 bits the same; 600 rows, W[9000,480] of 4 bits 32 -> 36; the look for a third term costs 3 % of it).
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(weights_in_terms(FP4, EXACT, RAGGED) ? 2 : 3))) qmg_kernel(const ProductArgs a) {
+template <typename T, int BITS, bool GLU>
+// Two blocks per compute unit: at three the operands of weights in terms spilled 21 to 70 registers, while a long row's table leaves
+// room for one or two anyway (300 rows, W[8300,3104] in groups of 32, 8 bits 169 -> 125 us, 4 bits the same; 600 rows, W[9000,480] of
+// 4 bits 32 -> 36; the look for a third term costs 3 % of it).
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) qmg_kernel(const ProductArgs a) {
     using G = Geometry<BITS>;
-    // Off whole steps affine products that do not take the CPU's weights run on float32 weights (expand_terms), as the vector
-    // kernels hold them.
-    constexpr bool kSplit = weights_in_terms(FP4, EXACT, RAGGED);
     constexpr int kDepth = G::kDepth, kLoads = G::kLoads;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    using S = std::conditional_t<FP4 != 0, uint8_t, T>;  // stored scale type
     unsigned char *table_s = lds + G::kFixedLdsBytes;  // scales [rows][groups, padded]; the biases follow
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = lane >> 5, l32 = lane & 31;
     const int K = (int)a.k, N = (int)a.n;
-    const int gshift = FP4 == kNvfp4 ? 4 : FP4 ? 5 : (a.group == 32 ? 5 : a.group == 64 ? 6 : 7);
+    const int gshift = a.group == 32 ? 5 : a.group == 64 ? 6 : 7;
     const int kgroups = K >> gshift;
     const int64_t row_bytes = (int64_t)(K >> 3) * BITS;  // of one packed weight row
-    const int tstride = table_stride(kgroups, (int)sizeof(S));
+    const int tstride = table_stride(kgroups, (int)sizeof(T));
     unsigned char *table_b = table_s + kRows * tstride;
     // Work items are (pass of up to 64 rows of an expert, 128 weight rows): every item costs the same whatever the
     // experts' loads, and an expert with many rows has its passes side by side.  The passes are counted from the
@@ -206,13 +195,12 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(w
     const T *x = (const T *)a.x;
     T *y = (T *)a.y;
 
-    // Off whole windows the last one begins early (RAGGED), at K - 128, so that no load leaves its row; the first `counted`
-    // of its values, which the window before has counted, are zeros in both operands.  Else the last window may hold one
-    // step, as the only window of K = 64 does in either form.
+    // Off whole windows the last one begins early, at K - 128, so that no load leaves its row; the first `counted` of its values,
+    // which the window before has counted, are zeros in both operands.  The only window of K = 64 holds one step.
     const int windows = (K + 127) >> 7;
-    const int counted = RAGGED && K > 128 ? windows * 128 - K : 0;
-    auto first_of = [&](int win) { return RAGGED && win == windows - 1 && K > 128 ? K - 128 : win * 128; };
-    auto one_step = [&](int win) { return RAGGED ? K < 128 : win * 128 + 64 >= K; };
+    const int counted = K > 128 ? windows * 128 - K : 0;
+    auto first_of = [&](int win) { return win == windows - 1 && K > 128 ? K - 128 : win * 128; };
+    const bool one_step = K < 128;
 
     // Weight window loads of this wavefront: load j of a lane is chunk q = 64 j + lane, i.e. chunk q % BITS of
     // row q / BITS of the wavefront's 32 rows.  Chunks of the window's second step begin at BITS / 2 (a window
@@ -232,7 +220,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(w
     // Every load of the K loop is issued on every path (a window past the end loads one 16-byte piece, the
     // same for all lanes), so that the waits can leave the younger windows' loads in flight.
     auto load_window = [&](int win, u32x4_t (&w)[kLoads]) {
-        const bool real = win < windows, half = one_step(win);
+        const bool real = win < windows, half = one_step;
         const int at = (first_of(win) >> 3) * BITS;
 #pragma unroll
         for (int j = 0; j < kLoads; j++) {
@@ -261,31 +249,18 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(w
     });
     __builtin_amdgcn_sched_barrier(0);
 
-    const float factor = FP4 == kNvfp4 && a.global_scale != nullptr ? ftz(a.global_scale[e] / (448.0f * 6.0f)) : 1.0f;  // (one per expert)
-    // The scale (NVFP4: the two scales, one per 16 values) and bias of this lane's 32 values of the step from k0 on.
-    auto load_scales = [&](int k0, float (&scale)[2], float &bias) {
-        const int g = (k0 + 32 * h) >> gshift;
-        const int at = (32 * wave + l32) * tstride + g * (int)sizeof(S);
-        const S *sp = reinterpret_cast<const S *>(table_s + at), *bp = reinterpret_cast<const S *>(table_b + at);
-        if constexpr (FP4 == kNvfp4) {
-            scale[0] = nvfp4_scale(sp[0], factor);
-            scale[1] = nvfp4_scale(sp[1], factor);
-            bias = 0.0f;
-        } else if constexpr (FP4) {
-            scale[0] = scale[1] = ftz(e8m0_to_f32(*sp));
-            bias = 0.0f;
-        } else {
-            scale[0] = scale[1] = Elem<T>::load(sp, 0);
-            bias = Elem<T>::load(bp, 0);
-        }
+    // The scale and bias of this lane's 32 values of the step from k0 on.
+    auto load_scales = [&](int k0, float &scale, float &bias) {
+        const int at = (32 * wave + l32) * tstride + ((k0 + 32 * h) >> gshift) * (int)sizeof(T);
+        scale = Elem<T>::load(reinterpret_cast<const T *>(table_s + at), 0);
+        bias = Elem<T>::load(reinterpret_cast<const T *>(table_b + at), 0);
     };
 
     {
         // The scales (and biases) of rows n0 .. n0 + 127 are contiguous in memory.
         const int valid_rows = N - n0 < kRows ? N - n0 : kRows;
-        fill_table<S, kThreads>(table_s, (const S *)a.scales + so + (int64_t)n0 * kgroups, valid_rows * kgroups, kgroups, tstride, tid);
-        if constexpr (!FP4)
-            fill_table<S, kThreads>(table_b, (const S *)a.biases + so + (int64_t)n0 * kgroups, valid_rows * kgroups, kgroups, tstride, tid);
+        fill_table<T, kThreads>(table_s, (const T *)a.scales + so + (int64_t)n0 * kgroups, valid_rows * kgroups, kgroups, tstride, tid);
+        fill_table<T, kThreads>(table_b, (const T *)a.biases + so + (int64_t)n0 * kgroups, valid_rows * kgroups, kgroups, tstride, tid);
     }
 
     // x tile loads: thread t brings chunks t + 256 i (i < 4) of a window's 1024 (chunk q: row q / 16, 16-byte
@@ -319,7 +294,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(w
         }
         auto load_x = [&](int win, u32x4_t (&xq)[4]) {
             // a window of one step has no second half: those chunks (pieces 8..15) fetch the first half again
-            const int k0 = win < windows ? first_of(win) - (one_step(win) && xc >= 8 ? 64 : 0) : 0;
+            const int k0 = win < windows ? first_of(win) - (one_step && xc >= 8 ? 64 : 0) : 0;
             // chunks 2 and 3 are rows 32..63: fetched only when the pass has a second tile (the loads are issued
             // either way, so that the waits see the same number of them: a tile-less one reads the start of x)
 #pragma unroll
@@ -327,7 +302,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(w
         };
         auto store_x = [&](int win, const u32x4_t (&xq)[4]) {
             unsigned char *dst = lds + (win & 1) * kXStageBytes;
-            if (RAGGED && win == windows - 1 && 8 * xc < counted) {  // (a thread's four chunks lie at one place of the window)
+            if (win == windows - 1 && 8 * xc < counted) {  // (a thread's four chunks lie at one place of the window)
 #pragma unroll
                 for (int i = 0; i < 4; i++)
                     if (i < 2 || two) *reinterpret_cast<u32x4_t *>(dst + xstore[i]) = u32x4_t{0, 0, 0, 0};
@@ -391,53 +366,40 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(w
                     // by step, so that 16 registers of weights and 32 of x are live at a time (both steps' together did not
                     // fit the 168 registers of three wavefronts per SIMD, and the loop spilled).  The second tile's are
                     // read whether the pass has one or not (stale but valid LDS).  A window of one step leaves out the
-                    // absent second one, the last window (RAGGED) a first step of zeros.
+                    // absent second one, the last window a first step of zeros.
                     const unsigned char *xs = lds + (win & 1) * kXStageBytes;
-                    const int before = RAGGED && win == windows - 1 ? counted : 0;  // values at the window's start that are zeros
-                    const bool run[2] = {!RAGGED || before < 64, !one_step(win)};
+                    const int before = win == windows - 1 ? counted : 0;  // values at the window's start that are zeros
+                    const bool run[2] = {before < 64, !one_step};
 #pragma unroll
                     for (int t = 0; t < 2; t++) {
                         if (!run[t]) continue;
-                        uint4 xf[2][4], wb[4];
+                        uint4 xf[2][4];
 #pragma unroll
                         for (int u = 0; u < 2; u++)
 #pragma unroll
                             for (int kk = 0; kk < 4; kk++) xf[u][kk] = *reinterpret_cast<const uint4 *>(xs + u * 32 * 256 + xread[t][kk]);
-                        float scale[2], bias;
+                        float scale, bias;
                         load_scales(first_of(win) + 64 * t, scale, bias);
-                        if (RAGGED && 64 * t + 32 * h < before) scale[0] = scale[1] = bias = 0.0f;
-                        if constexpr (kSplit) {
-                            static_for<4>([&](auto kk_tag) {
-                                constexpr int kk = decltype(kk_tag)::value;
-                                uint4 lo;
-                                expand_terms<T, BITS, kk>(codes[t], scale[0], bias, wb[kk], lo);
-                                acc[0] = Ops<T>::mfma(xf[0][kk], wb[kk], Ops<T>::mfma(xf[0][kk], lo, acc[0]));
-                                if (two) acc[1] = Ops<T>::mfma(xf[1][kk], wb[kk], Ops<T>::mfma(xf[1][kk], lo, acc[1]));
-                            });
-                            if (!__all(two_terms_hold<T, BITS>(scale[0], bias))) {
-                                uint32_t again[BITS];  // (formed anew: kept from above the terms would not fit the registers)
-#pragma unroll
-                                for (int i = 0; i < BITS; i++) again[i] = opaque(codes[t][i]);
-                                static_for<4>([&](auto kk_tag) {
-                                    constexpr int kk = decltype(kk_tag)::value;
-                                    uint4 hi, lo;
-                                    expand_terms<T, BITS, kk>(again, scale[0], bias, hi, lo);
-                                    const uint4 rest = left_over<T, BITS, kk>(again, scale[0], bias, hi, lo);
-                                    acc[0] = Ops<T>::mfma(xf[0][kk], rest, acc[0]);
-                                    if (two) acc[1] = Ops<T>::mfma(xf[1][kk], rest, acc[1]);
-                                });
-                            }
-                            continue;
-                        }
+                        if (64 * t + 32 * h < before) scale = bias = 0.0f;
                         static_for<4>([&](auto kk_tag) {
                             constexpr int kk = decltype(kk_tag)::value;
-                            wb[kk] = expand_piece<T, BITS, FP4, kk, EXACT>(codes[t], scale[kk >> 1], bias);
+                            uint4 hi, lo;
+                            expand_terms<T, BITS, kk>(codes[t], scale, bias, hi, lo);
+                            acc[0] = Ops<T>::mfma(xf[0][kk], hi, Ops<T>::mfma(xf[0][kk], lo, acc[0]));
+                            if (two) acc[1] = Ops<T>::mfma(xf[1][kk], hi, Ops<T>::mfma(xf[1][kk], lo, acc[1]));
                         });
+                        if (!__all(two_terms_hold<T, BITS>(scale, bias))) {
+                            uint32_t again[BITS];  // (formed anew: kept from above the terms would not fit the registers)
 #pragma unroll
-                        for (int kk = 0; kk < 4; kk++) acc[0] = Ops<T>::mfma(xf[0][kk], wb[kk], acc[0]);
-                        if (two) {
-#pragma unroll
-                            for (int kk = 0; kk < 4; kk++) acc[1] = Ops<T>::mfma(xf[1][kk], wb[kk], acc[1]);
+                            for (int i = 0; i < BITS; i++) again[i] = opaque(codes[t][i]);
+                            static_for<4>([&](auto kk_tag) {
+                                constexpr int kk = decltype(kk_tag)::value;
+                                uint4 hi, lo;
+                                expand_terms<T, BITS, kk>(again, scale, bias, hi, lo);
+                                const uint4 rest = left_over<T, BITS, kk>(again, scale, bias, hi, lo);
+                                acc[0] = Ops<T>::mfma(xf[0][kk], rest, acc[0]);
+                                if (two) acc[1] = Ops<T>::mfma(xf[1][kk], rest, acc[1]);
+                            });
                         }
                     }
                 }
@@ -512,15 +474,14 @@ inline size_t table_bytes(const ProductArgs &a) { return qmf::table_bytes(a, kRo
 // All LDS of a block.
 inline size_t lds_bytes(const ProductArgs &a) { return 2 * kXStageBytes + kWaves * 512 * (size_t)a.bits + table_bytes(a); }
 
-template <typename T, int BITS, int FP4, bool GLU, bool EXACT, bool RAGGED>
+template <typename T, int BITS, bool GLU>
 int32_t run_kernel(const ProductArgs &a, hipStream_t s) {
     using G = Geometry<BITS>;
     static std::atomic<bool> configured = false;
-    auto kernel = qmg_kernel<T, BITS, FP4, GLU, EXACT, RAGGED>;
+    auto kernel = qmg_kernel<T, BITS, GLU>;
     const size_t lds_bytes = G::kFixedLdsBytes + table_bytes(a);
     if (!configured) {
-        NVQ_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                        RAGGED ? kLdsMost : G::kFixedLdsBytes + kTableMaxBytes));
+        NVQ_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMost));
         configured = true;
     }
     // every expert with rows adds at most one partial pass: blocks for that many items, the rest leave at once
@@ -532,19 +493,10 @@ int32_t run_kernel(const ProductArgs &a, hipStream_t s) {
     return NVQ_OK;
 }
 
-template <typename T, int BITS, int FP4>
-int32_t run(const ProductArgs &a, hipStream_t s) {
-    if (a.glu != 0 && a.n % kRows != 0) return fail(NVQ_UNSUPPORTED, "gather_qmm: the gated epilogue takes gate and up rows in whole runs of 64");
-    const bool ragged = a.k % (BITS % 2 != 0 ? 128 : 64) != 0;
-    if constexpr (FP4 == kAffine)
-        if (a.exact_weights) return run_kernel<T, BITS, FP4, false, true, true>(a, s);  // (no gated epilogue: checked by the caller)
-    if (ragged) return a.glu == 0 ? run_kernel<T, BITS, FP4, false, false, true>(a, s) : run_kernel<T, BITS, FP4, true, false, true>(a, s);
-    return a.glu == 0 ? run_kernel<T, BITS, FP4, false, false, false>(a, s) : run_kernel<T, BITS, FP4, true, false, false>(a, s);
-}
-
-template <int BITS, int FP4>
+template <int BITS>
 int32_t run_dtype(const ProductArgs &a, hipStream_t s) {
-    return a.dtype == NVQ_BF16 ? run<bf16_t, BITS, FP4>(a, s) : run<f16_t, BITS, FP4>(a, s);
+    if (a.dtype == NVQ_BF16) return a.glu == 0 ? run_kernel<bf16_t, BITS, false>(a, s) : run_kernel<bf16_t, BITS, true>(a, s);
+    return a.glu == 0 ? run_kernel<f16_t, BITS, false>(a, s) : run_kernel<f16_t, BITS, true>(a, s);
 }
 
 }  // namespace qmg

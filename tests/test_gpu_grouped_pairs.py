@@ -1,0 +1,78 @@
+"""Sorted pairs on the grouped kernel where its tiles, windows, tables and groups end: passes of 1 to 4 tiles of rows, experts with no
+row and with more than a pass, K of part of a window, of windows that the groups of a block share unevenly and of tables that begin off
+16 bytes, N off whole stores of four, and K split over one, two and four groups.  Held to the CPU product
+(crates/nuvec-core/src/kernels.rs:1091-1142) at the bar of the element type."""
+import numpy as np
+import pytest
+import torch
+
+import nuvec_amd as nv
+from oracle import ref
+from tests.hip_backend import to_dev, to_host
+from tests.test_gpu_half_steps import MODES
+from tests.test_gpu_parity import make_w, make_x
+
+pytestmark = pytest.mark.gpu
+
+ROWS = [0, 1, 16, 17, 33, 48, 0, 49, 64, 65]
+
+
+def packed(rng, n, k, dtype, fmt):
+    """A weight and the oracle's product of rows with it."""
+    w = make_w(rng, n, k, dtype)
+    if isinstance(fmt, str):
+        codes, scales = ref.fp_quantize(w, dtype, MODES[fmt])
+        group, bits = ref.FP_PARAMS[MODES[fmt]]
+        want = lambda x: ref.quantized_matmul(x, codes, scales, None, mode=MODES[fmt], group=group, bits=bits, dtype=dtype, threads=8)
+        return nv.Quantized(to_dev(codes), to_dev(scales), None, nv.Quant.new(getattr(nv.QuantMode, fmt))), want
+    group, bits = fmt
+    codes, scales, biases = ref.affine_quantize(w, dtype, group, bits)
+    if n < 1024:
+        want = lambda x: ref.quantized_matmul(x, codes, scales, biases, group=group, bits=bits, dtype=dtype, threads=8)
+    else:
+        want = lambda x: ref.quantized_matmul_device(x, codes, scales, biases, group=group, bits=bits, dtype=dtype, rounded_weights=True)
+    return nv.Quantized(to_dev(codes), to_dev(scales), to_dev(biases), nv.Quant.affine(group, bits)), want
+
+
+def stacked(experts):
+    stack = lambda f: None if f(experts[0][0]) is None else torch.stack([f(q) for q, _ in experts])
+    return nv.Quantized(stack(lambda q: q.weight), stack(lambda q: q.scales), stack(lambda q: q.biases), experts[0][0].quant)
+
+
+# (groups of a block: 1 off whole blocks of 128 columns, else 2 from four windows and 4 from twelve)
+@pytest.mark.parametrize("fmt", [(64, 1), (64, 2), (128, 3), (64, 4), (128, 5), (32, 6), (32, 8), "MXFP4", "MXFP8", "NVFP4"], ids=str)
+@pytest.mark.parametrize("dtype,n,k", [(ref.BF16, 1030, 384), (ref.F16, 1024, 640), (ref.BF16, 1026, 1664), (ref.BF16, 1152, 2432), (ref.F16, 200, 640), (ref.BF16, 128, 1664), (ref.BF16, 1024, 128)])
+def test_passes_and_windows(fmt, dtype, n, k):
+    rng = np.random.default_rng(9100 + n + k)
+    experts = [packed(rng, n, k, dtype, fmt) for _ in ROWS]
+    q = stacked(experts)
+    ids = np.repeat(np.arange(len(ROWS)), ROWS).astype(np.int32)
+    tokens = rng.integers(0, 40, size=ids.size).astype(np.int32)  # (rows of x that several pairs take)
+    x = make_x(rng, 40, k, dtype)
+    place = rng.permutation(ids.size).astype(np.int32)
+    dev = lambda a: torch.from_numpy(a).cuda()
+    got = to_host(nv.gather_qmm_grouped(to_dev(x), q, dev(tokens), dev(ids), nv.sorted_offsets(dev(ids), len(ROWS)), out_rows=dev(place)))[place]
+    for e, rows in enumerate(ROWS):
+        if rows > 0:
+            want = ref.to_f32(experts[e][1](x[tokens[ids == e]]), dtype)
+            bound = (2.0 ** -7 if dtype == ref.BF16 else 2.0 ** -10) * np.max(np.abs(want), axis=1, keepdims=True)
+            assert np.all(np.abs(ref.to_f32(got[ids == e], dtype) - want) <= bound), (e, rows)
+
+
+# What a block's tail rows, pieces of codes and tables read lies inside their tensors' own lines: the last expert's last rows are right
+# whatever lies after them, and every pair's sums are its own, whatever the pairs beside it.
+@pytest.mark.parametrize("fmt", [(32, 4), (32, 8), "MXFP4"], ids=str)
+@pytest.mark.parametrize("n,k", [(1024, 1536), (1152, 2432), (1030, 640)])
+def test_a_pair_alone_has_the_bits_it_has_among_others(fmt, n, k):
+    rng = np.random.default_rng(9200 + n + k)
+    experts = [packed(rng, n, k, ref.BF16, fmt) for _ in range(3)]
+    q = stacked(experts)
+    ids = np.repeat(np.arange(3), [40, 3, 21]).astype(np.int32)
+    x = to_dev(make_x(rng, ids.size, k, ref.BF16))
+    dev = lambda a: torch.from_numpy(a).cuda()
+    rows = torch.arange(ids.size, dtype=torch.int32, device="cuda")
+    whole = nv.gather_qmm_grouped(x, q, rows, dev(ids), nv.sorted_offsets(dev(ids), 3))
+    for first, last in [(0, 17), (38, 45), (43, 64)]:
+        some = dev(ids[first:last])
+        part = nv.gather_qmm_grouped(x, q, rows[first:last].contiguous(), some, nv.sorted_offsets(some, 3))
+        assert torch.equal(part, whole[first:last])

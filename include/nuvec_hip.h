@@ -185,6 +185,12 @@ NVQ_API int32_t nvq_quant_check(const nvq_quant *quant, const char *op);
  * rows over `experts` weight batches takes the grouped kernel. */
 NVQ_API int32_t nvq_gather_grouped(int64_t rows, int64_t experts, int32_t row_exact);
 
+/* 1 if the pairs of `tokens` tokens with `choices` experts each run faster ordered by expert, every expert's weights read once, than one
+ * by one: from 64 pairs on as in the reference (crates/nuvec-lm/src/model.rs:2189-2192), fewer against block formats, whose weights both
+ * kernels hold exactly (`scaled`: not with a global scale).  `values`: of an expert's three projections. */
+NVQ_API int32_t nvq_moe_ordered(const nvq_quant *quant, int32_t dtype, int64_t tokens, int32_t choices, int64_t experts, int64_t values,
+                                int32_t scaled);
+
 /* GpuEval::supports for Primitive::QuantizedMatmul (gpu.rs:1665): 1 if nvq_quantized_matmul
  * has a kernel for `desc`, else 0 (the caller then runs its CPU path, eval.rs:738-748). */
 NVQ_API int32_t nvq_quantized_matmul_supported(const nvq_qmm_desc *desc);

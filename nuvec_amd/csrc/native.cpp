@@ -343,7 +343,9 @@ bool moe(const Tensor &x, const Tensor &router, int64_t k, bool normalize, Exper
     const int64_t pairs = rows * k;
     void *stream = at.stream();
     // choices, tokens and numbers of the pairs; for ordered pairs the order, its inverse, sorted experts and tokens, the offsets
-    const bool ordered = pairs >= 64;
+    const int64_t values = 3 * hidden * dims;
+    const bool ordered = nvq_moe_ordered(&e.up.p.q, code, rows, (int32_t)k, experts, values, 0) &&
+                         nvq_moe_ordered(&e.down.p.q, code, rows, (int32_t)k, experts, values, 0);
     Tensor index = at.empty({pairs * (ordered ? 7 : 3) + (ordered ? experts : 0)}, at::kInt), scores = at.empty({rows, k}, type);
     uint32_t *chosen = (uint32_t *)index.mutable_data_ptr(), *tokens = chosen + pairs, *identity = tokens + pairs;
     if (nvq_moe_router(code, ptr(x), ptr(router), rows, (int32_t)dims, (int32_t)experts, (int32_t)k, normalize, chosen, scores.mutable_data_ptr(),

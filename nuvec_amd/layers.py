@@ -247,12 +247,14 @@ class SwitchGlu:
 
     def forward(self, x: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
         """`x` `[B, L, D]` through each token's experts `indices` `[B, L, k]`: `[B, L, k, D]`.  With 64 pairs or
-        more they are ordered by expert (model.rs:2193-2210) so that each expert's weights are read once; here one
-        kernel orders the pairs, the products take the token rows of `x` themselves, and the last product writes
+        more (fewer against block formats, where `ops.moe_ordered` finds it faster) they are ordered by expert
+        (model.rs:2193-2210) so that each expert's weights are read once; here one kernel orders the pairs, the products take the token rows of `x` themselves, and the last product writes
         each row at its pair's place (`out_rows`), so the inverse permutation of model.rs:2210 is never run."""
         b, l, d = x.shape
         k = indices.shape[2]
-        if indices.numel() < 64:  # model.rs:2189-2192
+        experts = self.up_proj.weight.shape[0]
+        if not all(ops.moe_ordered(p.quantized(), x.dtype, b * l, k, experts, 3 * self.up_proj.weight.shape[1] * d)
+                   for p in (self.up_proj, self.down_proj)):  # model.rs:2189-2192
             xe = x.reshape(b, l, 1, 1, d)
             hidden = None
             if self.gate_up_proj is not None and self.gate_up_paired:
@@ -276,7 +278,6 @@ class SwitchGlu:
             else:
                 up, gate = self.up_proj.forward(xe, indices, add_bias=False), self.gate_proj.forward(xe, indices, add_bias=False)
             return self.down_proj.forward(self.gated(gate, up, indices), indices).squeeze(-2)
-        experts = self.up_proj.weight.shape[0]
         order, restore, sorted_ids, offsets = ops.moe_order(indices, experts)
         tokens = torch.div(order, k, rounding_mode="floor").to(torch.int32)  # pair t*k + j belongs to token t
         xt = x.reshape(b * l, d)

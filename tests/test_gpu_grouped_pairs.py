@@ -7,6 +7,7 @@ import pytest
 import torch
 
 import nuvec_amd as nv
+from nuvec_amd import layers
 from oracle import ref
 from tests.hip_backend import to_dev, to_host
 from tests.test_gpu_half_steps import MODES
@@ -76,3 +77,38 @@ def test_a_pair_alone_has_the_bits_it_has_among_others(fmt, n, k):
         some = dev(ids[first:last])
         part = nv.gather_qmm_grouped(x, q, rows[first:last].contiguous(), some, nv.sorted_offsets(some, 3))
         assert torch.equal(part, whole[first:last])
+
+
+@pytest.mark.parametrize("mode", list(MODES))
+@pytest.mark.parametrize("tokens,choices,count,dims,hidden,ordered", [(2, 2, 16, 2208, 2368, False), (5, 8, 8, 1056, 2368, True), (31, 2, 8, 1024, 1088, True)])
+def test_few_pairs_of_block_formats(mode, tokens, choices, count, dims, hidden, ordered):
+    """The layer's experts, in whichever order the rule picks, against the products of every pair: bfloat16 products of the same exact
+    weights, whose sums may fall to the next value, twice."""
+    torch.manual_seed(tokens)
+    quant = nv.Quant.new(getattr(nv.QuantMode, mode))
+
+    def projection(n, k):
+        q = nv.quantize((torch.randn(count, n, k, device="cuda") * 0.05).bfloat16(), quant)
+        return layers.SwitchProjection(q.weight, q.scales, q.biases, (torch.randn(count, n, device="cuda") * 0.1).bfloat16(), q.quant)
+    glu = layers.SwitchGlu(projection(hidden, dims), projection(hidden, dims), projection(dims, hidden))
+    x = torch.randn(1, tokens, dims, device="cuda").bfloat16()
+    ids = torch.stack([torch.randperm(count, device="cuda")[:choices] for _ in range(tokens)]).to(torch.int32).reshape(1, tokens, choices)
+    assert nv.ops.moe_ordered(glu.up_proj.quantized(), x.dtype, tokens, choices, count, 3 * hidden * dims) == ordered
+    xe = x.reshape(1, tokens, 1, 1, dims)
+    gate, up = (p.forward(xe, ids, add_bias=False) for p in (glu.gate_proj, glu.up_proj))
+    want = glu.down_proj.forward(glu.gated(gate, up, ids), ids).squeeze(-2).float()
+    for block in (glu, glu.fuse_gate_up()):
+        got = block.forward(x, ids).float()
+        # (a hidden state that falls to the next value moves an output by 2^-8 of one of its terms, at random over them)
+        assert (got - want).abs().max() <= 2 * 2.0 ** -7 * want.abs().max()
+
+
+def test_order_of_few_pairs_is_for_weights_that_both_kernels_hold():
+    rule = nv.ops.moe_ordered
+    q = lambda quant, scale=None: nv.Quantized(None, None, None, quant, scale)
+    mx, affine, nvfp4 = nv.Quant.new(nv.QuantMode.MXFP4), nv.Quant.affine(64, 4), nv.Quant.new(nv.QuantMode.NVFP4)
+    many = 3 * 2880 * 2880
+    assert rule(q(mx), torch.bfloat16, 5, 8, 8, many) and rule(q(nvfp4), torch.float16, 5, 8, 8, many)
+    assert not rule(q(mx), torch.bfloat16, 1, 32, 32, many) and not rule(q(mx), torch.float32, 5, 8, 8, many)
+    assert not rule(q(nvfp4, torch.ones(8)), torch.bfloat16, 5, 8, 8, many)
+    assert not rule(q(affine), torch.bfloat16, 63, 1, 8, many) and rule(q(affine), torch.bfloat16, 64, 1, 8, many)

@@ -16,7 +16,7 @@ CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(HERE, "..", "include")
 LIB = os.path.join(HERE, "libnuvec_hip.so")
 NATIVE = os.path.join(HERE, "_native.so")
-SOURCES = ["qme_b8.hip", "qme_b6.hip", "qme_b5.hip", "qme_b4.hip", "qme_b3.hip", "qme_b2.hip", "qme_b1.hip", "qme_nvfp4.hip", "qme_fp8.hip", "qme_fp4.hip",
+SOURCES = ["qmg_b8.hip", "qmg_b6.hip", "qmg_b5.hip", "qmg_b4.hip", "qmg_b3.hip", "qmg_b2.hip", "qmg_b1.hip", "qmg_nvfp4.hip", "qmg_fp8.hip", "qmg_fp4.hip",
            "qms_b8.hip", "qms_b6.hip", "qms_b5.hip", "qms_b4.hip", "qms_b3.hip", "qms_b2.hip", "qms_fp4.hip", "qms_fp8.hip", "qms_nvfp4.hip", "qms.hip",
            "qmf_b8.hip", "qmf_fp8.hip", "qmf_b6.hip", "qmf_b5.hip", "qmf_b4.hip", "qmf_fp4.hip", "qmf_nvfp4.hip", "qmf_b3.hip", "qmf_b2.hip", "qmf_b1.hip", "qmm.hip", "qmv.hip", "qmv_dot8.hip", "qmm_f32.hip", "qmm_dense.hip", "qmr.hip",
            "qvm.hip", "nvq_api.hip", "affine_quant.hip", "fp_quant.hip", "qmf.hip", "gather.hip", "repack.hip", "calib.hip", "qattn.hip", "qattn_prompt.hip", "qattn_prompt_f32.hip", "qmd.hip", "glu.hip"]  # slowest to compile first

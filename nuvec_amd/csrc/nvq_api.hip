@@ -434,17 +434,19 @@ int32_t nvq_gather_grouped(int64_t rows, int64_t experts, int32_t row_exact) {
     return rows >= least && rows / (experts > 1 ? experts : 1) >= 4;
 }
 
-// One by one a pair takes 0.294 us per megabyte of its expert, ordered an expert that some token chose 0.417 and the order, with the
-// longer start of the grouped kernel, 8 us more: fitted to 273 blocks of 2 to 31 tokens, 2, 4 and 8 of 8, 16 and 32 experts of
-// [512,512] to [2880,2880] in the three block formats, timed both ways; 0.8 % above always taking the faster one, 1.26 x at worst (one by
-// one up to 63 pairs: 11.8 %, 3.1 x).  5 tokens x 8 of 8 MXFP4 experts [2368,2208] 105 -> 55 us, 24 x 2 of 16 MXFP8 [2880,2880] 257 -> 118.
+// Ordered, an expert's weights are read once, for the price of the order and of the grouped kernel's longer start.  Bounds fitted to blocks of 2
+// to 31 tokens, 2, 4 and 8 of 8, 16 and 32 experts of [512,512] to [2880,2880], timed both ways, so that (nearly) none gets slower:
+// 273 blocks of block formats, 53 ordered, none slower, all in 0.92 of the time (always the faster side 0.89); 366 of affine codes of 2 to 6
+// and 8 bits, which the grouped kernel holds in terms there, 42 ordered, one slower (1.05 x), all in 0.95 (0.89).  5 tokens x 8 of 8 MXFP4
+// experts [2368,2208] 105 -> 55 us, 24 x 2 of 16 MXFP8 [2880,2880] 257 -> 118, 12 x 4 of 8 [2624,1088] of 4 bits 112 -> 77.
 int32_t nvq_moe_ordered(const nvq_quant *quant, int32_t dtype, int64_t tokens, int32_t choices, int64_t experts, int64_t values, int32_t scaled) {
     const double pairs = (double)tokens * (double)choices;
     if (pairs >= 64.0) return 1;
-    if (quant == nullptr || quant->mode == NVQ_AFFINE || scaled || (dtype != NVQ_BF16 && dtype != NVQ_F16) || tokens < 2 || choices < 1 || experts < choices) return 0;
+    if (quant == nullptr || scaled || (dtype != NVQ_BF16 && dtype != NVQ_F16) || tokens < 2 || choices < 1 || experts < choices || quant->group_size < 1) return 0;
+    const bool affine = quant->mode == NVQ_AFFINE;
     const double chosen = (double)experts * (1.0 - pow(1.0 - (double)choices / (double)experts, (double)tokens));  // were the choice even
-    const double megabytes = (double)values * (quant->bits + 8.0 / quant->group_size) / 8e6;
-    return megabytes * (0.294 * pairs - 0.417 * chosen) > 8.0;
+    const double megabytes = (double)values * (quant->bits + (affine ? 32.0 : 8.0) / quant->group_size) / 8e6;
+    return affine ? megabytes * (0.2 * pairs - 0.6 * chosen) > 4.0 : megabytes * (0.4 * pairs - 0.7 * chosen) > 12.0;
 }
 
 // primitive.rs:1378-1395 (MLX's validate_global_scale): NVFP4 only.

@@ -141,17 +141,17 @@ int32_t launch_qmr(const ProductArgs &a, hipStream_t s);
 // The few-row matrix-core kernel (up to 32 rows of x per pass; also the grouped gathered product).
 bool qmf_supported(const ProductArgs &a);
 int32_t launch_qmf(const ProductArgs &a, hipStream_t s);
-// The grouped kernel of sorted pairs (qme_kernel.h), one per code width, each in its own translation unit.
-int32_t launch_qme_b1(const ProductArgs &a, hipStream_t s);
-int32_t launch_qme_b2(const ProductArgs &a, hipStream_t s);
-int32_t launch_qme_b3(const ProductArgs &a, hipStream_t s);
-int32_t launch_qme_b4(const ProductArgs &a, hipStream_t s);
-int32_t launch_qme_b5(const ProductArgs &a, hipStream_t s);
-int32_t launch_qme_b6(const ProductArgs &a, hipStream_t s);
-int32_t launch_qme_b8(const ProductArgs &a, hipStream_t s);
-int32_t launch_qme_fp4(const ProductArgs &a, hipStream_t s);
-int32_t launch_qme_fp8(const ProductArgs &a, hipStream_t s);
-int32_t launch_qme_nvfp4(const ProductArgs &a, hipStream_t s);
+// The grouped kernel of sorted pairs (qmg_kernel.h), one per code width, each in its own translation unit.
+int32_t launch_qmg_b1(const ProductArgs &a, hipStream_t s);
+int32_t launch_qmg_b2(const ProductArgs &a, hipStream_t s);
+int32_t launch_qmg_b3(const ProductArgs &a, hipStream_t s);
+int32_t launch_qmg_b4(const ProductArgs &a, hipStream_t s);
+int32_t launch_qmg_b5(const ProductArgs &a, hipStream_t s);
+int32_t launch_qmg_b6(const ProductArgs &a, hipStream_t s);
+int32_t launch_qmg_b8(const ProductArgs &a, hipStream_t s);
+int32_t launch_qmg_fp4(const ProductArgs &a, hipStream_t s);
+int32_t launch_qmg_fp8(const ProductArgs &a, hipStream_t s);
+int32_t launch_qmg_nvfp4(const ProductArgs &a, hipStream_t s);
 // A few dozen rows with K split over wavefronts, blocks and the grid (qms_kernel.h).
 namespace qms {
 struct Plan {

@@ -1,13 +1,10 @@
-// The few-row, grouped and tiled matrix-core kernels for affine 3-bit codes (qmf_kernel.h, qmg_kernel.h,
-// qmm_kernel.h).
-#include "qmg_kernel.h"
+// The few-row and tiled matrix-core kernels for affine 3-bit codes (qmf_kernel.h, qmm_kernel.h).
+#include "qmf_kernel.h"
 #include "qmm_kernel.h"
 
 namespace nvq {
 
-int32_t launch_qmf_b3(const ProductArgs &a, hipStream_t s) {
-    return a.offsets != nullptr || a.one_group ? qmg::run_dtype<3>(a, s) : qmf::run_dtype<3, false>(a, s);
-}
+int32_t launch_qmf_b3(const ProductArgs &a, hipStream_t s) { return qmf::run_dtype<3, false>(a, s); }
 
 int32_t launch_qmm_b3(const ProductArgs &a, void *workspace, hipStream_t s) { return qmm::run_dtype<3, false>(a, workspace, s); }
 

@@ -1,0 +1,6 @@
+// The grouped kernel of sorted pairs for affine 8-bit codes (qmg_kernel.h).
+#include "qmg_kernel.h"
+
+namespace nvq {
+int32_t launch_qmg_b8(const ProductArgs &a, hipStream_t s) { return qmg::run_dtype<8, rows::kAffine>(a, s); }
+}  // namespace nvq

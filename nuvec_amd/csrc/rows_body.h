@@ -55,9 +55,58 @@ __device__ __forceinline__ void load_codes(const unsigned char *p, uint32_t (&d)
     if constexpr (BITS % 2 == 1) d[BITS - 1] = *reinterpret_cast<const uint32_t *>(p + 4 * (BITS - 1));
 }
 
-template <typename T, int BITS, int FP4, bool EXACT, int MT, int NT, int QW, int STAGES>
+// Affine weights in float32 as terms of the element type.  With scale and bias in that type, v = code * scale + bias is a whole
+// multiple of the lower one's last place, and with L bits of significand (8, 11) and their exponents close enough two terms hold it: the
+// rest after one lies within 2^(E(v) - L), and its multiples fit L bits where E(v) - min(E(scale), E(bias)) <= L + 1.  float16 holds no
+// multiple finer than 2^-24, so that any |v| below a half is two terms too.  Codes of `quantize` keep that by far (the bias is the
+// end of the range farther from zero): two matrix instructions.  Where some lane's 32 weights do not, a third instruction brings what is
+// left of v's 24 bits.  (There the range of the first term is the finite one, so that a large or infinite v is the second's; nothing is
+// left then.)
+template <typename T, int BITS>
+__device__ __forceinline__ bool two_terms_hold(float s, float b) {
+    constexpr bool bf16 = Elem<T>::code == NVQ_BF16;
+    auto exponent = [](float v) { return max((int)(f2u(v) >> 23 & 255u), 1); };
+    const float top = fmaxf(fabsf(b), fabsf(__builtin_fmaf((float)((1 << BITS) - 1), s, b)));
+    const int high = exponent(top), low = min(s != 0.0f ? exponent(s) : 255, b != 0.0f ? exponent(b) : 255);
+    if constexpr (bf16) return high - low <= 9 && top <= 3.38953139e38f;
+    else return top <= 65504.0f && (high - low <= 12 || high <= 125);
+}
+
+// Piece KK of a lane's 32 affine codes as two terms; CLAMPED: of any weights, not only those that two terms hold.
+template <typename T, int BITS, int KK, bool CLAMPED>
+__device__ __forceinline__ void expand_terms(const uint32_t (&dw)[BITS], float s, float b, uint4 &hi, uint4 &lo) {
+    constexpr float most = Elem<T>::code == NVQ_BF16 ? 3.38953139e38f : 65504.0f;
+    uint32_t h[4], l[4];
+    static_for<4>([&](auto i_tag) {
+        constexpr int i = decltype(i_tag)::value, J = 8 * KK + 2 * i;
+        const float v0 = __builtin_fmaf(qmf::code_to_float<BITS, J>(dw), s, b), v1 = __builtin_fmaf(qmf::code_to_float<BITS, J + 1>(dw), s, b);
+        if constexpr (CLAMPED) h[i] = qmf::Ops<T>::pack(__builtin_amdgcn_fmed3f(v0, -most, most), __builtin_amdgcn_fmed3f(v1, -most, most));
+        else h[i] = qmf::Ops<T>::pack(v0, v1);
+        l[i] = qmf::Ops<T>::pack(v0 - qmf::half_lo<T>(h[i]), v1 - qmf::half_hi<T>(h[i]));
+    });
+    hi = make_uint4(h[0], h[1], h[2], h[3]), lo = make_uint4(l[0], l[1], l[2], l[3]);
+}
+
+// What two finite terms leave of them, exactly.
+template <typename T, int BITS, int KK>
+__device__ __forceinline__ uint4 left_over(const uint32_t (&dw)[BITS], float s, float b, uint4 hi, uint4 lo) {
+    const uint32_t h[4] = {hi.x, hi.y, hi.z, hi.w}, l[4] = {lo.x, lo.y, lo.z, lo.w};
+    uint32_t t[4];
+    static_for<4>([&](auto i_tag) {
+        constexpr int i = decltype(i_tag)::value, J = 8 * KK + 2 * i;
+        const float v0 = __builtin_fmaf(qmf::code_to_float<BITS, J>(dw), s, b), v1 = __builtin_fmaf(qmf::code_to_float<BITS, J + 1>(dw), s, b);
+        const float r0 = v0 - qmf::half_lo<T>(h[i]) - qmf::half_lo<T>(l[i]), r1 = v1 - qmf::half_hi<T>(h[i]) - qmf::half_hi<T>(l[i]);
+        t[i] = qmf::Ops<T>::pack(fabsf(r0) < INFINITY ? r0 : 0.0f, fabsf(r1) < INFINITY ? r1 : 0.0f);
+    });
+    return make_uint4(t[0], t[1], t[2], t[3]);
+}
+
+// How affine weights are held: rounded once to the element type, as nuvec's CPU product holds them (qmf::affine_pair), or as terms.
+enum Hold { kRounded, kCpu, kTerms };
+
+template <typename T, int BITS, int FP4, int HOLD, int MT, int NT, int QW, int STAGES>
 struct Body {
-    static constexpr int kAhead = BITS <= 4 ? 4 : 2;  // windows of codes under way
+    static constexpr int kAhead = BITS <= 4 && HOLD != kTerms ? 4 : 2;  // windows of codes under way
     static constexpr int kXAll = 4 * MT, kX = (kXAll + QW - 1) / QW;  // loads of x of the group and window, of a wavefront
     static constexpr int kXStage = MT * kTile * kXRow;
     static constexpr int kKinds = FP4 ? 1 : 2, kScaleBytes = FP4 ? 1 : 2, kPart = 16 / kScaleBytes;  // groups of a part of the scales
@@ -203,13 +252,35 @@ struct Body {
                         }
                         if (!inside) scale[t][0] = scale[t][1] = bias[t] = 0.0f;
                     }
+                    bool held = true;
+                    if constexpr (HOLD == kTerms) {
+#pragma unroll
+                        for (int t = 0; t < NT; t++) held = held && two_terms_hold<T, BITS>(scale[t][0], bias[t]);
+                        held = __all(held);
+                    }
                     static_for<4>([&](auto j_tag) __attribute__((always_inline)) {
                         constexpr int j = decltype(j_tag)::value;
                         uint4 xf[MT], w[NT];
 #pragma unroll
                         for (int m = 0; m < MT; m++) xf[m] = *reinterpret_cast<const uint4 *>(xs + (kTile * m + l) * kXRow + 16 * ((4 * q + j) ^ l));
 #pragma unroll
-                        for (int t = 0; t < NT; t++) w[t] = qmf::expand_piece<T, BITS, FP4, j, EXACT>(ring[d][t], scale[t][j >> 1], bias[t]);
+                        for (int t = 0; t < NT; t++) {
+                            if constexpr (HOLD == kTerms) {
+                                uint4 lo;
+                                if (held) {
+                                    expand_terms<T, BITS, j, false>(ring[d][t], scale[t][0], bias[t], w[t], lo);
+                                } else {
+                                    expand_terms<T, BITS, j, true>(ring[d][t], scale[t][0], bias[t], w[t], lo);
+                                    const uint4 rest = left_over<T, BITS, j>(ring[d][t], scale[t][0], bias[t], w[t], lo);
+#pragma unroll
+                                    for (int m = 0; m < MT; m++) acc[m][t] = Mfma16<T>::run(rest, xf[m], acc[m][t]);
+                                }
+#pragma unroll
+                                for (int m = 0; m < MT; m++) acc[m][t] = Mfma16<T>::run(lo, xf[m], acc[m][t]);
+                            } else {
+                                w[t] = qmf::expand_piece<T, BITS, FP4, j, HOLD == kCpu>(ring[d][t], scale[t][j >> 1], bias[t]);
+                            }
+                        }
 #pragma unroll
                         for (int m = 0; m < MT; m++)
 #pragma unroll

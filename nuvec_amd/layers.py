@@ -247,7 +247,7 @@ class SwitchGlu:
 
     def forward(self, x: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
         """`x` `[B, L, D]` through each token's experts `indices` `[B, L, k]`: `[B, L, k, D]`.  With 64 pairs or
-        more (fewer against block formats, where `ops.moe_ordered` finds it faster) they are ordered by expert
+        more (fewer where `ops.moe_ordered` finds it faster) they are ordered by expert
         (model.rs:2193-2210) so that each expert's weights are read once; here one kernel orders the pairs, the products take the token rows of `x` themselves, and the last product writes
         each row at its pair's place (`out_rows`), so the inverse permutation of model.rs:2210 is never run."""
         b, l, d = x.shape

@@ -595,7 +595,7 @@ def sorted_offsets(rhs: torch.Tensor, groups: int) -> torch.Tensor:
 
 def moe_ordered(q: Quantized, dtype: torch.dtype, tokens: int, choices: int, experts: int, values: int) -> bool:
     """Whether the pairs of `tokens` tokens with `choices` of `experts` each, `values` weights an expert packed as `q`, run faster ordered
-    by expert (`moe_order`) than one by one: from 64 pairs on (model.rs:2189-2192), fewer against block formats."""
+    by expert (`moe_order`) than one by one: from 64 pairs on (model.rs:2189-2192), fewer where the estimate says so."""
     if dtype not in _CODE:
         return tokens * choices >= 64
     return bool(_lib.load().nvq_moe_ordered(C.byref(q.quant._c()), _CODE[dtype], tokens, choices, experts, values, int(q.global_scale is not None)))

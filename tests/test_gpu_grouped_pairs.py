@@ -68,24 +68,27 @@ def test_a_pair_alone_has_the_bits_it_has_among_others(fmt, n, k):
     rng = np.random.default_rng(9200 + n + k)
     experts = [packed(rng, n, k, ref.BF16, fmt) for _ in range(3)]
     q = stacked(experts)
-    ids = np.repeat(np.arange(3), [40, 3, 21]).astype(np.int32)
+    ids = np.repeat(np.arange(3), [40, 3, 20]).astype(np.int32)  # (all fewer than 64, whose affine weights are float32)
     x = to_dev(make_x(rng, ids.size, k, ref.BF16))
     dev = lambda a: torch.from_numpy(a).cuda()
     rows = torch.arange(ids.size, dtype=torch.int32, device="cuda")
     whole = nv.gather_qmm_grouped(x, q, rows, dev(ids), nv.sorted_offsets(dev(ids), 3))
-    for first, last in [(0, 17), (38, 45), (43, 64)]:
+    for first, last in [(0, 17), (38, 45), (43, 63)]:
         some = dev(ids[first:last])
         part = nv.gather_qmm_grouped(x, q, rows[first:last].contiguous(), some, nv.sorted_offsets(some, 3))
         assert torch.equal(part, whole[first:last])
 
 
-@pytest.mark.parametrize("mode", list(MODES))
-@pytest.mark.parametrize("tokens,choices,count,dims,hidden,ordered", [(2, 2, 16, 2208, 2368, False), (5, 8, 8, 1056, 2368, True), (31, 2, 8, 1024, 1088, True)])
-def test_few_pairs_of_block_formats(mode, tokens, choices, count, dims, hidden, ordered):
-    """The layer's experts, in whichever order the rule picks, against the products of every pair: bfloat16 products of the same exact
-    weights, whose sums may fall to the next value, twice."""
+QUANTS = {"4 bits": nv.Quant.affine(64, 4), "8 bits": nv.Quant.affine(32, 8), **{mode: nv.Quant.new(getattr(nv.QuantMode, mode)) for mode in MODES}}
+
+
+@pytest.mark.parametrize("quant", list(QUANTS))
+@pytest.mark.parametrize("tokens,choices,count,dims,hidden,ordered", [(2, 2, 16, 2176, 2368, False), (5, 8, 8, 1088, 2368, True), (31, 2, 8, 1024, 1088, True)])
+def test_few_pairs(quant, tokens, choices, count, dims, hidden, ordered):
+    """The layer's experts, in whichever order the rule picks, against the products of every pair: bfloat16 products of the same weights,
+    exact or in float32 on both sides, whose sums may fall to the next value, twice."""
     torch.manual_seed(tokens)
-    quant = nv.Quant.new(getattr(nv.QuantMode, mode))
+    quant = QUANTS[quant]
 
     def projection(n, k):
         q = nv.quantize((torch.randn(count, n, k, device="cuda") * 0.05).bfloat16(), quant)
@@ -103,12 +106,29 @@ def test_few_pairs_of_block_formats(mode, tokens, choices, count, dims, hidden, 
         assert (got - want).abs().max() <= 2 * 2.0 ** -7 * want.abs().max()
 
 
-def test_order_of_few_pairs_is_for_weights_that_both_kernels_hold():
+def test_few_pairs_hold_affine_weights_in_float32():
+    """Against float64: few sorted pairs as far from it as pairs one by one, whose kernel holds float32 weights; the outputs' rounding
+    (values are at most 2^-7 of them apart, errors uniform: 2^-7 / sqrt(12) in the mean square) is all that is left."""
+    torch.manual_seed(11)
+    quant = nv.Quant.affine(64, 4)
+    q = nv.quantize((torch.randn(3, 1152, 1024, device="cuda") * 0.02 + 0.3).bfloat16(), quant)  # (biases far above the codes' steps)
+    x = torch.randn(21, 1024, device="cuda").bfloat16()
+    ids = torch.arange(3, device="cuda").repeat_interleave(7).to(torch.int32)
+    rows = torch.arange(21, dtype=torch.int32, device="cuda")
+    got = nv.gather_qmm_grouped(x, q, rows, ids, nv.sorted_offsets(ids, 3)).double()
+    codes = nv.dequantize(nv.Quantized(q.weight, torch.ones_like(q.scales, dtype=torch.float32), torch.zeros_like(q.scales, dtype=torch.float32), quant))
+    spread = lambda t: t.double().repeat_interleave(64, dim=-1)
+    dense = codes.double() * spread(q.scales) + spread(q.biases)
+    want = torch.einsum("rk,rnk->rn", x.double().cpu(), dense.cpu()[ids.long().cpu()]).cuda()
+    assert (got - want).norm() <= 2.0 ** -7 / 12 ** 0.5 * want.norm()
+
+
+def test_order_of_few_pairs():
     rule = nv.ops.moe_ordered
     q = lambda quant, scale=None: nv.Quantized(None, None, None, quant, scale)
     mx, affine, nvfp4 = nv.Quant.new(nv.QuantMode.MXFP4), nv.Quant.affine(64, 4), nv.Quant.new(nv.QuantMode.NVFP4)
     many = 3 * 2880 * 2880
-    assert rule(q(mx), torch.bfloat16, 5, 8, 8, many) and rule(q(nvfp4), torch.float16, 5, 8, 8, many)
+    assert rule(q(mx), torch.bfloat16, 5, 8, 8, many) and rule(q(nvfp4), torch.float16, 5, 8, 8, many) and rule(q(affine), torch.bfloat16, 5, 8, 8, many)
     assert not rule(q(mx), torch.bfloat16, 1, 32, 32, many) and not rule(q(mx), torch.float32, 5, 8, 8, many)
     assert not rule(q(nvfp4, torch.ones(8)), torch.bfloat16, 5, 8, 8, many)
-    assert not rule(q(affine), torch.bfloat16, 63, 1, 8, many) and rule(q(affine), torch.bfloat16, 64, 1, 8, many)
+    assert rule(q(affine), torch.float32, 64, 1, 8, 1) and not rule(q(affine), torch.bfloat16, 63, 1, 64, many)

@@ -59,12 +59,20 @@ __device__ __forceinline__ V load_any(const void *p) {
 // An operand is kOffset + code.  WIDE: float32.
 template <int BITS, bool WIDE> constexpr float kOffset = WIDE ? -(float)(1 << (BITS - 1)) : BITS == 8 ? 0.0f : (float)(1 << BITS);
 template <int BITS> constexpr uint32_t kMagic = BITS == 4 ? 0x41804180u : 0x41004100u;  // two of 2^BITS, BITS < 8
-// Codes at bit `at` of both halves of a word as 2^BITS + code.
+// Codes at bit `at` of both halves of a word as 2^BITS + code.  The constants come in registers, a scalar one and a vector one: then the
+// mask and the exponent are one instruction (v_and_or_b32, which takes no literal; from constants they were two).
 template <int BITS>
-__device__ __forceinline__ uint32_t two_codes(uint32_t z, int at) {
+struct CodeConstants {
+    uint32_t mask = ((1u << BITS) - 1u) * 0x00010001u << (7 - BITS), magic = kMagic<BITS>;
+    __device__ __forceinline__ CodeConstants() {
+        asm("" : "+s"(mask));
+        asm("" : "+v"(magic));
+    }
+};
+template <int BITS>
+__device__ __forceinline__ uint32_t two_codes(const CodeConstants<BITS> &c, uint32_t z, int at) {
     constexpr int to = 7 - BITS;  // the code's place in the mantissa
-    constexpr uint32_t mask = ((1u << BITS) - 1u) * 0x00010001u << to;
-    return ((at >= to ? z >> (at - to) : z << (to - at)) & mask) | kMagic<BITS>;
+    return ((at >= to ? z >> (at - to) : z << (to - at)) & c.mask) | c.magic;
 }
 
 // Two exact bfloat16 values from two floats that bfloat16 holds.
@@ -75,12 +83,12 @@ template <int BITS> constexpr int code_at(int j) { return BITS == 8 ? j : (j >> 
 
 // Eight consecutive codes of a row (BITS bytes in the low bits of w0, w1) as an operand, in the order of code_at.
 template <int BITS, bool WIDE>
-__device__ __forceinline__ uint4 eight_codes(uint32_t w0, uint32_t w1) {
+__device__ __forceinline__ uint4 eight_codes(const CodeConstants<BITS> &c, uint32_t w0, uint32_t w1) {
     if constexpr (WIDE) {
         auto at = [&](int j) {
             const int i = code_at<BITS>(j);
-            const uint32_t c = BITS == 8 ? (i < 4 ? w0 >> (8 * i) : w1 >> (8 * (i - 4))) & 0xFFu : (w0 >> (BITS * i)) & ((1u << BITS) - 1u);
-            return (float)c + kOffset<BITS, true>;
+            const uint32_t code = BITS == 8 ? (i < 4 ? w0 >> (8 * i) : w1 >> (8 * (i - 4))) & 0xFFu : (w0 >> (BITS * i)) & ((1u << BITS) - 1u);
+            return (float)code + kOffset<BITS, true>;
         };
         return make_uint4(pack_exact(at(0), at(1)), pack_exact(at(2), at(3)), pack_exact(at(4), at(5)), pack_exact(at(6), at(7)));
     } else if constexpr (BITS == 8) {
@@ -88,7 +96,7 @@ __device__ __forceinline__ uint4 eight_codes(uint32_t w0, uint32_t w1) {
                           pack_exact(qmf::ubyte_to_float<0>(w1), qmf::ubyte_to_float<1>(w1)), pack_exact(qmf::ubyte_to_float<2>(w1), qmf::ubyte_to_float<3>(w1)));
     } else {
         const uint32_t z = BITS == 4 ? w0 : (w0 & 0xFFFu) | ((w0 & 0xFFF000u) << 4);  // code i at bit BITS i, code i + 4 sixteen above
-        return make_uint4(two_codes<BITS>(z, 0), two_codes<BITS>(z, BITS), two_codes<BITS>(z, 2 * BITS), two_codes<BITS>(z, 3 * BITS));
+        return make_uint4(two_codes(c, z, 0), two_codes(c, z, BITS), two_codes(c, z, 2 * BITS), two_codes(c, z, 3 * BITS));
     }
 }
 
@@ -149,6 +157,7 @@ __global__ void __launch_bounds__(64 * kAttnWaves, (attention_blocks<T, G>())) q
     const int per = attention_split_keys(S, splits);
     const int s_begin = split * per, s_end = s_begin + per < S ? s_begin + per : S;
     const float scale = d.scale * kLog2e;
+    const CodeConstants<BITS> constants;
 
     // The queries' operands: column (g, head), zeros outside the group; their sums per column.
     const int head = l % R;
@@ -220,8 +229,40 @@ __global__ void __launch_bounds__(64 * kAttnWaves, (attention_blocks<T, G>())) q
         }
         return o;
     };
-    auto fetch_keys = [&](int s0) {
+    // A tile that lies inside the cache: the tile's place is a scalar address and the lane's place in it an offset that does not
+    // change, so that a load takes no vector instruction for its address; the scales of four keys are one load.  (With an address
+    // for every load and key clamped by itself a quarter of the loop's vector instructions were addresses.)
+    auto four_inside = [&](const T *p, int s0, int h) __attribute__((always_inline)) {
+        const uint8_t *at = reinterpret_cast<const uint8_t *>(p) + (row0 + s0) * kRun;
+        Quad o;
+        if constexpr (kOwn) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) o.w[i] = load_any<uint32_t>(at + (uint32_t)(4 * quarter * kRun + 4 * g) + (16 * h + i) * kRun);
+        } else {
+            o = load_any<Quad>(at + (uint32_t)(4 * quarter * kRun) + 16 * h * kRun);
+        }
+        return o;
+    };
+    auto fetch_keys = [&](int s0) __attribute__((always_inline)) {
         if (s0 >= s_end) return;  // (nothing is left for this wavefront)
+        if (s0 + kTileKeys <= S) {
+            const uint8_t *tile = kbytes + (row0 + s0) * kRowBytes;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                if constexpr (kChunk % 4 == 0) {
+                    struct Words { uint32_t w[kChunk / 4]; };
+                    const Words w = *reinterpret_cast<const Words *>(tile + (uint32_t)(l * kRowBytes + quarter * kChunk) + 16 * h * kRowBytes);
+#pragma unroll
+                    for (int i = 0; i < kChunk / 4; i++) kt.c[h][i] = w.w[i];
+                } else {  // 6 bytes (16 codes of 3 bits): 8 from where they stay inside the row
+                    const int at = quarter * kChunk < kRowBytes - 8 ? quarter * kChunk : kRowBytes - 8;
+                    const uint64_t w = load_any<uint64_t>(tile + (uint32_t)(l * kRowBytes + at) + 16 * h * kRowBytes) >> (8 * (quarter * kChunk - at));
+                    kt.c[h][0] = (uint32_t)w, kt.c[h][1] = (uint32_t)(w >> 32);
+                }
+                kt.s[h] = four_inside(ks, s0, h), kt.b[h] = four_inside(kb, s0, h);
+            }
+            return;
+        }
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             int key = s0 + 16 * h + l;
@@ -240,31 +281,42 @@ __global__ void __launch_bounds__(64 * kAttnWaves, (attention_blocks<T, G>())) q
             kt.s[h] = four(ks, s0 + 16 * h + 4 * quarter), kt.b[h] = four(kb, s0 + 16 * h + 4 * quarter);
         }
     };
-    auto fetch_values = [&](int s0) {
+    // the lane's slot of a row at `row` + `lanes`, `lanes` without the slot's own place
+    auto value_slot = [&](const uint8_t *row, uint32_t lanes, int j) __attribute__((always_inline)) {
+        if constexpr (kSlot == 64) {
+            const uint2 w = *reinterpret_cast<const uint2 *>(row + (lanes + 8 * l));
+            vt.c[j][0] = w.x, vt.c[j][1] = w.y;
+        } else if constexpr (kSlot == 32) {
+            vt.c[j][0] = *reinterpret_cast<const uint32_t *>(row + (lanes + 4 * l));
+        } else if constexpr (kSlot == 16) {
+            vt.c[j][0] = *reinterpret_cast<const uint16_t *>(row + (lanes + 2 * l));
+        } else if constexpr (kSlot == 24) {
+            vt.c[j][0] = load_any<uint32_t>(row + (lanes + 3 * l - (l == 15))) >> (l == 15 ? 8 : 0);
+        } else {  // 12 bits
+            vt.c[j][0] = load_any<uint16_t>(row + (lanes + 3 * l / 2)) >> (4 * (l & 1));
+        }
+    };
+    auto fetch_values = [&](int s0) __attribute__((always_inline)) {
         if (s0 >= s_end) return;
+        if (s0 + kTileKeys <= S) {
+            const uint8_t *tile = vbytes + (row0 + s0) * kRowBytes;
+#pragma unroll
+            for (int j = 0; j < 8; j++) value_slot(tile + (16 * (j >> 2) + (j & 3)) * kRowBytes, 4 * quarter * kRowBytes, j);
+#pragma unroll
+            for (int h = 0; h < 2; h++) vt.s[h] = four_inside(vs, s0, h), vt.b[h] = four_inside(vb, s0, h);
+            return;
+        }
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-            int key = s0 + 16 * (j >> 2) + 4 * quarter + (j & 3);
-            key = key < S ? key : S - 1;
-            const uint8_t *row = vbytes + (row0 + key) * kRowBytes;
-            if constexpr (kSlot == 64) {
-                const uint2 w = *reinterpret_cast<const uint2 *>(row + 8 * l);
-                vt.c[j][0] = w.x, vt.c[j][1] = w.y;
-            } else if constexpr (kSlot == 32) {
-                vt.c[j][0] = *reinterpret_cast<const uint32_t *>(row + 4 * l);
-            } else if constexpr (kSlot == 16) {
-                vt.c[j][0] = *reinterpret_cast<const uint16_t *>(row + 2 * l);
-            } else if constexpr (kSlot == 24) {
-                vt.c[j][0] = load_any<uint32_t>(row + 3 * l - (l == 15)) >> (l == 15 ? 8 : 0);
-            } else {  // 12 bits
-                vt.c[j][0] = load_any<uint16_t>(row + 3 * l / 2) >> (4 * (l & 1));
-            }
+            const int key = s0 + 16 * (j >> 2) + 4 * quarter + (j & 3);
+            value_slot(vbytes + (row0 + (key < S ? key : S - 1)) * kRowBytes, 0, j);
         }
 #pragma unroll
         for (int h = 0; h < 2; h++) vt.s[h] = four(vs, s0 + 16 * h + 4 * quarter), vt.b[h] = four(vb, s0 + 16 * h + 4 * quarter);
     };
     // The lane's own group of key i.
-    const int down = 16 * (g & 1), up = 16 - down;
+    const int down = 16 * (g & 1);
+    const uint32_t half = g & 1 ? 0x03020C0Cu : 0x01000C0Cu;  // (its 16 bits above zeros: one byte permutation)
     auto pick = [&](const Quad &o, int i) {
         if constexpr (kOwn) {
             return u2f(o.w[i]);
@@ -278,7 +330,7 @@ __global__ void __launch_bounds__(64 * kAttnWaves, (attention_blocks<T, G>())) q
             if constexpr (G == 4) w = g >= 2 ? o.w[2 * i + 1] : w;
             if constexpr (Elem<T>::code == 10) {
                 if constexpr (G == 1) return u2f(i & 1 ? w & 0xFFFF0000u : w << 16);
-                return u2f((w << up) & 0xFFFF0000u);
+                return u2f(__builtin_amdgcn_perm(0u, w, half));
             } else {
                 return (float)__builtin_bit_cast(f16_t, (uint16_t)(w >> (G == 1 ? 16 * (i & 1) : down)));
             }
@@ -307,13 +359,13 @@ __global__ void __launch_bounds__(64 * kAttnWaves, (attention_blocks<T, G>())) q
             for (int s = 0; s < KS; s++) {
                 uint4 kf;
                 if constexpr (BITS == 8) {
-                    kf = eight_codes<8, kWide>(kt.c[h][2 * s], kt.c[h][2 * s + 1]);
+                    kf = eight_codes<8, kWide>(constants, kt.c[h][2 * s], kt.c[h][2 * s + 1]);
                 } else if constexpr (BITS == 4) {
-                    kf = eight_codes<4, kWide>(kt.c[h][s], 0);
+                    kf = eight_codes<4, kWide>(constants, kt.c[h][s], 0);
                 } else {
                     constexpr int W = (kChunk + 3) / 4;
                     const int bit = 24 * s, w = bit / 32, sh = bit % 32;
-                    kf = eight_codes<3, kWide>(sh == 0 ? kt.c[h][w] : __builtin_amdgcn_alignbit(kt.c[h][w + 1 < W ? w + 1 : w], kt.c[h][w], sh), 0);
+                    kf = eight_codes<3, kWide>(constants, sh == 0 ? kt.c[h][w] : __builtin_amdgcn_alignbit(kt.c[h][w + 1 < W ? w + 1 : w], kt.c[h][w], sh), 0);
                 }
 #pragma unroll
                 for (int i = 0; i < TQ; i++) sum = mfma16(kf, qf[s][i], sum);
@@ -325,8 +377,14 @@ __global__ void __launch_bounds__(64 * kAttnWaves, (attention_blocks<T, G>())) q
                 // the groups of a row: columns R apart
                 if constexpr (G == 4) v += u2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2u(v), 0x124, 0xF, 0xF, true));
                 if constexpr (G >= 2) v += u2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2u(v), 0x128, 0xF, 0xF, true));
-                score[4 * h + r] = s0 + 16 * h + 4 * quarter + r < s_end ? v * scale : -INFINITY;
+                score[4 * h + r] = v * scale;
             }
+        }
+        if (s0 + kTileKeys > s_end) {
+            asm volatile("");  // (a branch: as selects it would cost every tile)
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                if (s0 + 16 * (j >> 2) + 4 * quarter + (j & 3) >= s_end) score[j] = -INFINITY;
         }
         fetch_keys(s0 + kAttnWaves * kTileKeys);
         float top = score[0];
@@ -383,7 +441,7 @@ __global__ void __launch_bounds__(64 * kAttnWaves, (attention_blocks<T, G>())) q
                     const int from = BITS == 4 ? 16 : 8;  // the second piece's first bit
                     const uint32_t sel = !high ? 0x05040100u : BITS == 4 ? 0x07060302u : 0x06050201u;
                     const uint32_t both = __builtin_amdgcn_perm(vt.c[2 * j + 1][0], vt.c[2 * j][0], sel);
-                    p[j] = two_codes<BITS>(both, BITS * i - (high ? from : 0));
+                    p[j] = two_codes(constants, both, BITS * i - (high ? from : 0));
                 }
             }
             const uint4 vf = make_uint4(p[0], p[1], p[2], p[3]);

@@ -44,7 +44,7 @@ __device__ __forceinline__ void run_pass(const ProductArgs &a, unsigned char *ld
 #pragma unroll
         for (int t = 0; t < 2; t++) acc[m][t] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
     B::run(
-        a, lds + group * B::kLdsBytes, wave, e, n0, min(k0, K), min(k0 + turns * rows::kWin, K), turns,
+        a, lds + group * B::kLdsBytes, wave, e, n0, k0, min(k0 + turns * rows::kWin, K), turns,
         [&](int r) {  // an index beyond x is the caller's error: clamped
             const int at = pass + (r < rows ? r : rows - 1);
             return a.lhs != nullptr ? min((int64_t)a.lhs[at], a.x_batches - 1) : (int64_t)at;

@@ -115,10 +115,10 @@ struct Body {
     static constexpr int kLdsBytes = STAGES * kXStage + QW * kTableBytes;
     static_assert(STAGES >= 2 && STAGES <= kAhead + 1, "the waits below count these loads");
 
-    // `xrow(r)`: the row of x behind row r; `weight_row(t, r)`: row r of this wavefront's tile t, rows from `n0` on.  The range [k0, k1) begins at
+    // `xrow(r)`: the row of x behind row r; `weight_row(t, r)`: row r of this wavefront's tile t, rows from `n0`, a row of the weight, on.  The range [k_begin, k1) begins at
     // a whole window and ends at one or at K; `turns` is the most windows of any group of the block.
     template <class XRow, class WeightRow>
-    static __device__ __forceinline__ void run(const ProductArgs &a, unsigned char *lds, int wave, int e, int n0, int k0, int k1, int turns, XRow xrow,
+    static __device__ __forceinline__ void run(const ProductArgs &a, unsigned char *lds, int wave, int e, int n0, int k_begin, int k1, int turns, XRow xrow,
                                                WeightRow weight_row, floatx4_t (&acc)[MT][NT]) {
         const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds;
         const int lane = threadIdx.x & 63, l = lane & 15, q = lane >> 4;
@@ -126,7 +126,8 @@ struct Body {
         const int gshift = FP4 == kNvfp4 ? 4 : FP4 ? 5 : (a.group == 32 ? 5 : a.group == 64 ? 6 : 7);
         const int kgroups = K >> gshift;
         const uint32_t row_bytes = (uint32_t)(K >> 5) * (4 * BITS);
-        const int windows = k1 > k0 ? (k1 - k0 + kWin - 1) / kWin : 0;
+        const int windows = k1 > k_begin ? (k1 - k_begin + kWin - 1) / kWin : 0;
+        const int k0 = windows > 0 ? k_begin : 0;  // (a group without a window asks for its rows' first values)
         int64_t xrows[kX];  // (asked for first: what is loaded after does not wait for them)
 #pragma unroll
         for (int i = 0; i < kX; i++) xrows[i] = xrow(min(4 * (wave + QW * i), kTile * MT - 4) + (lane >> 4));

@@ -644,6 +644,16 @@ __global__ void __launch_bounds__(kMergeParts * D) qattn_merge_kernel(const nvq_
                                  sinks != nullptr ? Elem<T>::load(sinks, blockIdx.x) * kLog2e : 0.0f, out + head * D);
 }
 
+// The same for few splits, D / 4 threads a head.
+template <typename T, int D>
+__global__ void __launch_bounds__(64) qattn_merge_few_kernel(const nvq_attention_desc d, const float *__restrict__ partials, int splits,
+                                                             const T *__restrict__ sinks, T *__restrict__ out) {
+    const int64_t h = (int64_t)blockIdx.x * (256 / D) + (int)threadIdx.x / (D / 4), head = (int64_t)blockIdx.y * d.query_heads + h;
+    if (h >= d.query_heads) return;
+    merge_few_states<T, D>(partials + head * splits * (D + 2), D + 2, splits, sinks != nullptr, sinks != nullptr ? Elem<T>::load(sinks, h) * kLog2e : 0.0f,
+                           out + head * D, (int)threadIdx.x % (D / 4) * 4);
+}
+
 struct Plan {
     bool vector;
     int splits;  // of the positions over the grid
@@ -677,7 +687,11 @@ int32_t run_attention_sized(const nvq_attention_desc &d, const Operands &o, hipS
     }
     NVQ_LAUNCH_CHECK("quantized_attention");
     if (p.splits > 1) {
-        hipLaunchKernelGGL((qattn_merge_kernel<T, D>), dim3((unsigned)d.query_heads, (unsigned)d.batch), dim3(kMergeParts * D), 0, s, d,
+        if (p.splits <= kFewSplits)
+            hipLaunchKernelGGL((qattn_merge_few_kernel<T, D>), dim3((unsigned)((d.query_heads + 256 / D - 1) / (256 / D)), (unsigned)d.batch), dim3(64), 0, s, d,
+                               (const float *)o.workspace, p.splits, (const T *)o.sinks, (T *)o.out);
+        else
+            hipLaunchKernelGGL((qattn_merge_kernel<T, D>), dim3((unsigned)d.query_heads, (unsigned)d.batch), dim3(kMergeParts * D), 0, s, d,
                            (const float *)o.workspace, p.splits, (const T *)o.sinks, (T *)o.out);
         NVQ_LAUNCH_CHECK("quantized_attention merge");
     }

@@ -284,6 +284,18 @@ __global__ void __launch_bounds__(kMergeParts * D) prompt_merge_kernel(const Pro
                                  (T *)a.out + (((int64_t)b * a.query_heads + h) * a.queries + i) * D);
 }
 
+// The same for few splits, D / 4 threads a row.
+template <typename T, int D>
+__global__ void __launch_bounds__(256) prompt_merge_few_kernel(const PromptArgs a) {
+    const int rows = a.rep * a.queries, r = (int)blockIdx.x * (1024 / D) + (int)threadIdx.x / (D / 4);
+    if (r >= rows) return;
+    const int head = blockIdx.y, b = (a.head0 + head) / a.key_heads, hk = (a.head0 + head) % a.key_heads;
+    const int h = hk * a.rep + r % a.rep, i = r / a.rep;
+    merge_few_states<T, D>(a.partials + ((int64_t)head * rows + r) * (D + 2), (int64_t)rows * gridDim.y * (D + 2), a.splits, a.sinks != nullptr,
+                           a.sinks != nullptr ? Elem<T>::load((const T *)a.sinks, h) * kLog2e : 0.0f,
+                           (T *)a.out + (((int64_t)b * a.query_heads + h) * a.queries + i) * D, (int)threadIdx.x % (D / 4) * 4);
+}
+
 struct Plan {
     int tiles, row_tiles, row_groups, splits, terms;
     int64_t heads, slice;  // all (batch, key head)s, and those of one launch
@@ -348,7 +360,9 @@ int32_t run_rows(const PromptArgs &a, const Plan &p, int64_t heads, hipStream_t 
     }
     NVQ_LAUNCH_CHECK("quantized_attention");
     if (p.splits > 1) {
-        hipLaunchKernelGGL((prompt_merge_kernel<T, D>), dim3((unsigned)p.rows, (unsigned)heads), dim3(kMergeParts * D), 0, s, a);
+        const unsigned blocks = (unsigned)((p.rows + 1024 / D - 1) / (1024 / D));  // (of 256 threads, few splits)
+        if (p.splits <= kFewSplits) hipLaunchKernelGGL((prompt_merge_few_kernel<T, D>), dim3(blocks, (unsigned)heads), dim3(256), 0, s, a);
+        else hipLaunchKernelGGL((prompt_merge_kernel<T, D>), dim3((unsigned)p.rows, (unsigned)heads), dim3(kMergeParts * D), 0, s, a);
         NVQ_LAUNCH_CHECK("quantized_attention merge");
     }
     return NVQ_OK;

@@ -312,6 +312,18 @@ __global__ void __launch_bounds__(kMergeParts * D) prompt_merge_f32_kernel(const
                                      a.out + (((int64_t)b * a.query_heads + h) * a.queries + i) * D);
 }
 
+// The same for few splits, D / 4 threads a row.
+template <int D>
+__global__ void __launch_bounds__(256) prompt_merge_few_f32_kernel(const Args a) {
+    const int rows = a.rep * a.queries, r = (int)blockIdx.x * (1024 / D) + (int)threadIdx.x / (D / 4);
+    if (r >= rows) return;
+    const int head = blockIdx.y, b = head / a.key_heads, hk = head % a.key_heads;
+    const int h = hk * a.rep + r % a.rep, i = r / a.rep;
+    merge_few_states<float, D>(a.partials + ((int64_t)head * rows + r) * (D + 2), (int64_t)rows * gridDim.y * (D + 2), a.splits, a.sinks != nullptr,
+                               a.sinks != nullptr ? a.sinks[h] * 1.44269504088896340736f : 0.0f,
+                               a.out + (((int64_t)b * a.query_heads + h) * a.queries + i) * D, (int)threadIdx.x % (D / 4) * 4);
+}
+
 struct Plan { int tiles, row_tiles, row_groups, splits; int64_t heads, rows; };
 
 // Four row groups a block where that gives two blocks a compute unit; else four wavefronts on each, and with fewer than two blocks a
@@ -345,7 +357,9 @@ int32_t run(const Args &a, const Plan &p, hipStream_t s) {
     else hipLaunchKernelGGL((prompt_attention_f32_kernel<BITS, D, 1>), grid, block, 0, s, a);
     NVQ_LAUNCH_CHECK("quantized_attention");
     if (p.splits > 1) {
-        hipLaunchKernelGGL((prompt_merge_f32_kernel<D>), dim3((unsigned)p.rows, (unsigned)p.heads), dim3(kMergeParts * D), 0, s, a);
+        const unsigned blocks = (unsigned)((p.rows + 1024 / D - 1) / (1024 / D));  // (of 256 threads, few splits)
+        if (p.splits <= kFewSplits) hipLaunchKernelGGL((prompt_merge_few_f32_kernel<D>), dim3(blocks, (unsigned)p.heads), dim3(256), 0, s, a);
+        else hipLaunchKernelGGL((prompt_merge_f32_kernel<D>), dim3((unsigned)p.rows, (unsigned)p.heads), dim3(kMergeParts * D), 0, s, a);
         NVQ_LAUNCH_CHECK("quantized_attention merge");
     }
     return NVQ_OK;

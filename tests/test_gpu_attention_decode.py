@@ -89,6 +89,26 @@ def test_merged_splits(splits):
     assert (got.double() - want).abs().max() <= 16 * 1.1e-6 * nv.dequantize(v).abs().max()
 
 
+@pytest.mark.parametrize("splits", [2, 7, 8, 9])
+@pytest.mark.parametrize("heads,dim", [(1, 64), (5, 64), (3, 128)])
+def test_merged_splits_up_to_eight(splits, heads, dim):
+    """Both sides of the splits that a row's own threads merge, heads that are no whole blocks of them, weights that differ by split:
+    the second half of the keys has scores 3 above the first."""
+    s, quant = 256 * splits, nv.Quant.affine(64, 4)
+    keys = torch.zeros(1, heads, s, dim, device="cuda")
+    keys[:, :, s // 2:, 0] = 3.0
+    v = nv.quantize(torch.randn(1, heads, s, dim, device="cuda"), quant)
+    q = torch.zeros(1, heads, 1, dim, device="cuda")
+    q[..., 0] = 1.0
+    k, sinks = nv.quantize(keys, quant), torch.full((heads,), 7.0, device="cuda")
+    scores = nv.dequantize(k).double()[..., 0]
+    weights = torch.softmax(torch.cat([scores, sinks.double().view(1, heads, 1)], dim=-1), dim=-1)[..., :s]
+    want = (weights.unsqueeze(-1) * nv.dequantize(v).double()).sum(-2, keepdim=True)
+    got = ops.quantized_attention(q, k, v, 1.0, sinks)
+    # (the float32 sums' random roundings, as above)
+    assert (got.double() - want).abs().max() <= 16 * 1.1e-6 * nv.dequantize(v).abs().max()
+
+
 @pytest.mark.parametrize("heads,batch", [(2, 1), (8, 300)])  # the vector kernel, the matrix cores
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_infinities_and_nans_stay_where_they_are(dtype, heads, batch):

@@ -79,6 +79,14 @@ def test_prompt_attention(case, dtype):
         assert (off <= 1.1 * bound).all(), off.max().item()
 
 
+@pytest.mark.parametrize("case", [(1, 6, 2, 61, 600, 128, 4, 64, True, True), (1, 3, 1, 43, 2048, 64, 8, 32, True, True),
+                                  (1, 2, 1, 67, 2304, 128, 4, 64, False, False), (2, 2, 1, 33, 1300, 64, 3, 64, True, False)], ids=str)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_merged_splits(case, dtype):
+    """Two, eight, nine and five splits of rows that are no whole blocks of the merge."""
+    test_prompt_attention(case, dtype)
+
+
 @pytest.mark.parametrize("dtype,l,s", [(torch.float16, 2, 1024), (torch.float16, 200, 1100), (torch.bfloat16, 16, 1100), (torch.bfloat16, 40, 8200)])
 @pytest.mark.parametrize("d", [64, 128])
 def test_keys_of_two_terms(dtype, l, s, d):

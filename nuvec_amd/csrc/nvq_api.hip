@@ -635,6 +635,13 @@ static bool split_rows_take(const ProductArgs &a, Route route, qms::Plan &plan) 
     return here < (rows + (a.k < 1600 ? 0.2 : a.k < 2600 ? 0.1 : 0.0)) * (a.bits == 2 && a.m <= 16 ? 0.85 : 1.0) * few_rows_us(a);
 }
 
+// Whether the float32 matrix-core kernel runs a product of the vector kernels' route (the route keeps its name).  The estimates of both
+// are up to a tenth off at up to four rows, one pass of the vector kernel, so there it has to be ahead by that.  (250 products of 2 to 700
+// rows that had that route, timed on both sides: 0.78 of the time; us, W[4989,864] MXFP8 at 132 rows 134 -> 15, W[5115,14336] of 4 bits at 5
+// rows 69 -> 22, W[1657,6144] of 6 bits at 32 rows 44 -> 15, W[7340,4096] of 8 bits at 4 rows 20 -> 14; without the margin W[7978,2048] of 6
+// bits at 3 rows 11.3 -> 12.3.)
+static bool float32_rows_take(const ProductArgs &a, Route route) { return route == Route::kVector && qmm_f32_faster(a, a.m <= 4 ? 0.91 : 1.0); }
+
 // `dense`: whether the workspace may hold the dequantized weight.
 static size_t workspace_bytes(const nvq_qmm_desc *d, bool dense) {
     if (check_qmm(d, "quantized_matmul") != NVQ_OK) return 0;
@@ -645,7 +652,7 @@ static size_t workspace_bytes(const nvq_qmm_desc *d, bool dense) {
     // float32 partial sums of the splits of K: weights stored [K, N], or few tiles of a long K
     if (!d->transpose) return qvm_workspace_bytes(a);
     const Route route = pick_route(d, a);
-    if (route == Route::kTiledF32) return qmm_f32_workspace_bytes(a);
+    if (route == Route::kTiledF32 || float32_rows_take(a, route)) return qmm_f32_workspace_bytes(a);
     qms::Plan split;
     if (split_rows_take(a, route, split)) return qms_workspace_bytes(a, split);
     if (route != Route::kTiled) return 0;
@@ -708,6 +715,7 @@ static int32_t quantized_matmul_any(const nvq_qmm_desc *d, const void *x, const 
     const Route route = pick_route(d, a);
     qms::Plan split;
     if (split_rows_take(a, route, split)) return launch_qms(a, split, workspace, (hipStream_t)stream);
+    if (float32_rows_take(a, route)) return launch_qmm_f32(a, workspace, (hipStream_t)stream);
     switch (route) {
     case Route::kUntransposed: return launch_qvm(a, workspace, (hipStream_t)stream);
     case Route::kTiled:  // without a workspace: codes are expanded in the kernel and K is not split
@@ -732,6 +740,7 @@ static const char *name_of(const nvq_qmm_desc *d, bool kernel) {
     const Route route = pick_route(d, a);
     qms::Plan split;
     if (kernel && split_rows_take(a, route, split)) return qms_kernel_name(split);
+    if (kernel && float32_rows_take(a, route)) return "qmm_f32_kernel";
     if (kernel && route == Route::kTiled && qmm_dense_takes(a)) return "qmm_dense_kernel";
     switch (route) {
     case Route::kUntransposed: return qvm_kernel_name(a);

@@ -127,7 +127,8 @@ size_t qmm_workspace_bytes(const ProductArgs &a);  // float32 partial sums when 
 int32_t launch_qmm(const ProductArgs &a, void *workspace, hipStream_t s);  // workspace NULL: no split
 double qmm_estimate_us(const ProductArgs &a);  // estimated duration of the tiled kernel with its better tile
 // float32 products of two rows and more on v_mfma_f32_16x16x32_bf16 (weights stored [N, K]); a workspace of partial sums where K is split.
-bool qmm_f32_takes(const ProductArgs &a);
+bool qmm_f32_takes(const ProductArgs &a);  // whether the product's route has its name
+bool qmm_f32_faster(const ProductArgs &a, double margin);  // estimated below `margin` of the vector kernel's time
 size_t qmm_f32_workspace_bytes(const ProductArgs &a);
 int32_t launch_qmm_f32(const ProductArgs &a, void *workspace, hipStream_t s);
 bool grouped_rows_take(const ProductArgs &a);

@@ -564,16 +564,21 @@ static bool qmm_f32_supported(const ProductArgs &a) {
 // takes 0.28 of the time of what served them before, the vector kernel and two on v_mfma_f32_16x16x4_f32 and 32x32x2 (4 bits, us:
 // W[4096,4096] at 33 / 64 / 128 / 512 rows 35 / 45 / 87 / 178 -> 17 / 22 / 30 / 70, W[14336,4096] at 16 rows 76 -> 20, W[704,5376] at
 // 274 rows 134 -> 23), and its error against float64 is lower (W[4096,4096] at 33 rows 2.9e-7 -> 1.0e-7, 2.9e-7 -> 1.0e-7 for NVFP4).
-// The vector kernel keeps, though it is behind, what callers that ask for a product's route know it by: a few rows of affine
-// and E4M3 codes (of 1024 values and more up to 4, of whole steps of 2048 up to 8, against up to 2^24 weights up to 32;
-// W[4096,4096] at 32 rows 65 us there, 17 here; taken, W[9744,512] at 3 rows 13.6 us there, 6.3 here), four rows of MXFP4 up to 2^24 weights, and more than 128 rows of K off whole steps of 64.
+bool qmm_f32_faster(const ProductArgs &a, double margin) {
+    if (!qmm_f32_supported(a)) return false;
+    const bool e2m1 = a.mode == NVQ_MXFP4 || a.mode == NVQ_NVFP4;
+    const double k_steps = (double)((a.k + 2047) / 2048) * 2048.0;
+    return plan_of(a).us < margin * (4.0 + (e2m1 ? 2.52 : 1.05) * (double)((a.m + 3) / 4) * (double)a.n * k_steps / 2.2e6);
+}
+
+// Whether the product's route is this kernel's name.  A few rows of affine and E4M3 codes (of 1024 values and more up to 4, of whole steps
+// of 2048 up to 8, against up to 2^24 weights up to 32), four rows of MXFP4 up to 2^24 weights and more than 128 rows of K off whole
+// steps of 64 keep the vector kernel's, by which callers that ask for a route know them.
 bool qmm_f32_takes(const ProductArgs &a) {
-    if (!qmm_f32_supported(a) || (a.k % kStep != 0 && a.m > 128)) return false;
+    if (a.k % kStep != 0 && a.m > 128) return false;
     const bool small = a.n * a.k <= 1 << 24, e2m1 = a.mode == NVQ_MXFP4 || a.mode == NVQ_NVFP4;
     if (!e2m1 && (a.k % 2048 == 0 ? a.m <= (small ? 32 : 8) : a.k >= 1024 && a.m <= 4)) return false;
-    if (a.mode == NVQ_MXFP4 && small && a.m <= 4) return false;
-    const double k_steps = (double)((a.k + 2047) / 2048) * 2048.0;
-    return plan_of(a).us < 4.0 + (e2m1 ? 2.52 : 1.05) * (double)((a.m + 3) / 4) * (double)a.n * k_steps / 2.2e6;
+    return !(a.mode == NVQ_MXFP4 && small && a.m <= 4) && qmm_f32_faster(a, 1.0);
 }
 
 size_t qmm_f32_workspace_bytes(const ProductArgs &a) {

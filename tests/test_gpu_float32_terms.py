@@ -50,6 +50,21 @@ def test_ends_of_windows_spans_and_splits(fmt, m, n, k):
         assert np.linalg.norm(got - want) <= LIMIT * np.linalg.norm(want)
 
 
+@pytest.mark.parametrize("fmt,m,n,k", [((32, 3), 801, 700, 1120), ((32, 8), 129, 2001, 1056), ("MXFP8", 132, 1989, 864), ("MXFP4", 160, 968, 544),
+                                       ("MXFP4", 4, 5208, 160), ("MXFP4", 3, 12990, 512), ((64, 4), 32, 4099, 2048), ((128, 5), 6, 5858, 2048),
+                                       ((64, 6), 21, 1731, 2048), ((128, 2), 2, 11651, 1920), ((128, 1), 3, 16001, 2048), ("MXFP8", 2, 13742, 1376)], ids=str)
+def test_products_that_keep_the_vector_kernels_route(fmt, m, n, k):
+    rng = np.random.default_rng(6150 + m + k)
+    x = make_x(rng, m, k, ref.F32)
+    q, dense = quantized(fmt, make_w(rng, n, k, ref.F32))
+    assert ops.quantized_matmul_route(m, n, k, q.quant, torch.float32).startswith("qmv_")
+    assert ops.quantized_matmul_kernel(m, n, k, q.quant, torch.float32) == "qmm_f32_kernel"
+    want = x.astype(np.float64) @ dense.T
+    for scratch in (True, False):
+        got = to_host(ops.quantized_matmul(to_dev(x), q, scratch=scratch)).astype(np.float64)
+        assert np.linalg.norm(got - want) <= LIMIT * np.linalg.norm(want)
+
+
 @pytest.mark.parametrize("fmt", [(64, 4), (32, 8), "MXFP4", "MXFP8", "NVFP4"], ids=str)
 def test_magnitudes_that_three_terms_do_not_hold(fmt):
     """Infinities, NaN and values near the end of float32's range give what the CPU's product gives; the other rows keep their bits."""

@@ -426,6 +426,16 @@ NVQ_API int32_t nvq_gather_qmm_expert_bias(const nvq_gather_desc *desc, const vo
                                    const int32_t *offsets, const uint32_t *out_rows, const void *expert_bias, void *y,
                                    void *workspace, void *stream);
 
+/* The experts' down products and their weighted sum (`MoeMlp::forward` after the gated states, crates/nuvec-lm/src/model.rs:2248-2271) of
+ * decoded tokens in one kernel: pairs choices * t .. + choices - 1 are token t's, one row of x each,
+ *   out dtype[pairs / choices, n] = sum over a token's pairs of y[z] * scores[z],
+ * y as nvq_gather_qmm_expert_bias returns it, the sum nvq_weighted_sum's: bit for bit that composition.  scores dtype[pairs / choices,
+ * choices]; expert_bias and global_scales may be NULL.  NVQ_UNSUPPORTED where the pairs do not run on the decode kernel of the block
+ * formats and affine codes, or the two kernels are faster (the caller then composes them). */
+NVQ_API int32_t nvq_gather_qmm_sum(const nvq_gather_desc *desc, const void *x, const void *w, const void *scales, const void *biases,
+                                   const float *global_scales, const uint32_t *lhs, const uint32_t *rhs, const void *expert_bias,
+                                   const void *scores, int32_t choices, void *out, void *stream);
+
 /* `Mlp::forward` up to its down projection (crates/nuvec-lm/src/model.rs:2066-2074: `swiglu(gate(x), up(x))`, Gemma's
  * `geglu`) for up to four rows of x in one kernel: w, scales, biases (and bias, dtype[n] or NULL: the two
  * projections' biases, layers.rs:155-162) hold the gate and up projections in alternating runs of 64 rows as for

@@ -365,8 +365,17 @@ bool moe(const Tensor &x, const Tensor &router, int64_t k, bool normalize, Exper
         p.expert = sorted, p.offsets = offsets;
         tokens = sorted_tokens, to = order;
     }
-    if (!hidden_states(at, x, rows, e, p, tokens, h) || !project(at, h, pairs, e.down, p, identity, to, true, y) || e.down.rows == 0) return false;
+    if (!hidden_states(at, x, rows, e, p, tokens, h) || e.down.rows == 0) return false;
     Tensor sum = at.empty({x.size(0), x.size(1), e.down.rows}, type);
+    if (!ordered) {  // (few tokens: the down products with their sum)
+        const nvq_gather_desc d{e.down.p.q, code, 1, 0, 0, 1, e.down.rows, hidden, pairs, pairs, experts};
+        if (nvq_gather_qmm_sum(&d, ptr(h), ptr(e.down.p.w), ptr(e.down.p.s), ptr(e.down.p.b), nullptr, identity, chosen, ptr(e.down.bias), ptr(scores),
+                               (int32_t)k, sum.mutable_data_ptr(), stream) == NVQ_OK) {
+            out = std::move(sum);
+            return true;
+        }
+    }
+    if (!project(at, h, pairs, e.down, p, identity, to, true, y)) return false;
     if (nvq_weighted_sum(code, ptr(y), ptr(scores), rows, (int32_t)k, e.down.rows, sum.mutable_data_ptr(), stream) != NVQ_OK) return false;
     out = std::move(sum);
     return true;

@@ -1137,6 +1137,8 @@ struct GluEpilogue {  // activation < 0: no activation, only the experts' bias
     int32_t activation;
     float alpha, limit;
     const void *expert_bias;
+    const void *scores = nullptr;  // with `choices` > 0 (and no activation): y is the weighted sums of so many pairs each
+    int64_t choices = 0;
 };
 
 static int32_t gather_qmm_any(const nvq_gather_desc *d, const void *x, const void *w, const void *scales, const void *biases,
@@ -1168,8 +1170,10 @@ static int32_t gather_qmm_any(const nvq_gather_desc *d, const void *x, const voi
     NVQ_TRY(check_aligned("gather_qmm", "lhs", lhs, 4));
     NVQ_TRY(check_aligned("gather_qmm", "rhs", rhs, 4));
     NVQ_TRY(check_aligned("gather_qmm", "offsets", offsets, 4));
-    const void *expert_bias = nullptr;
-    if (glu != nullptr && glu->activation < 0) {  // the experts' bias alone: the grouped kernel's epilogue
+    const void *expert_bias = nullptr, *scores = nullptr;
+    int64_t choices = 0;
+    if (glu != nullptr && glu->activation < 0) {
+        scores = glu->scores, choices = glu->choices;  // the experts' bias alone: the grouped kernel's epilogue
         expert_bias = glu->expert_bias;
         glu = nullptr;
         NVQ_TRY(check_aligned("gather_qmm", "expert bias", expert_bias, (size_t)dtype_size(d->dtype)));
@@ -1236,8 +1240,13 @@ static int32_t gather_qmm_any(const nvq_gather_desc *d, const void *x, const voi
     }
     // Row-exact: every pair on the vector kernels, so that a pair has the bits of its one-row product whether the
     // gather is sorted or not and however many pairs it holds (the few-row contract of gpu.rs:7325-7340).
-    if (!a.row_exact && takes_few_rows_direct(a)) return launch_qmd(a, (hipStream_t)stream);
-    if (!a.row_exact && !takes_decode(a) && qmf_supported(a)) return launch_qmf(a, (hipStream_t)stream);
+    const bool direct = !a.row_exact && takes_few_rows_direct(a), few = !a.row_exact && !takes_decode(a) && qmf_supported(a);
+    if (choices > 0) {
+        if (direct || few || a.row_exact) return fail(NVQ_UNSUPPORTED, "gather_qmm: the decode kernel does not take these pairs with their weighted sum");
+        return launch_qmv_sum(a, scores, y, choices, (hipStream_t)stream);
+    }
+    if (direct) return launch_qmd(a, (hipStream_t)stream);
+    if (few) return launch_qmf(a, (hipStream_t)stream);
     return launch_qmv(a, (hipStream_t)stream);
 }
 
@@ -1273,6 +1282,21 @@ int32_t nvq_gather_qmm_expert_bias(const nvq_gather_desc *d, const void *x, cons
         return fail(NVQ_INVALID_ARGUMENT, "gather_qmm: global scale is only supported for 'nvfp4' quantization mode");
     const GluEpilogue only_bias{-1, 0.0f, 0.0f, expert_bias};
     return gather_qmm_any(d, x, w, scales, biases, global_scales, lhs, rhs, offsets, out_rows, y, workspace, stream, &only_bias);
+}
+
+int32_t nvq_gather_qmm_sum(const nvq_gather_desc *d, const void *x, const void *w, const void *scales, const void *biases,
+                           const float *global_scales, const uint32_t *lhs, const uint32_t *rhs, const void *expert_bias,
+                           const void *scores, int32_t choices, void *out, void *stream) {
+    if (d == nullptr) return fail(NVQ_INVALID_ARGUMENT, "gather_qmm: null descriptor");
+    if (global_scales != nullptr && d->quant.mode != NVQ_NVFP4)  // quantized.rs:620-623
+        return fail(NVQ_INVALID_ARGUMENT, "gather_qmm: global scale is only supported for 'nvfp4' quantization mode");
+    if (choices < 1 || d->pairs % choices != 0)
+        return fail(NVQ_INVALID_ARGUMENT, "gather_qmm: %lld pairs are no whole tokens of %d choices", (long long)d->pairs, choices);
+    if (!d->transpose || d->m != 1 || d->k == 0) return fail(NVQ_UNSUPPORTED, "gather_qmm: the weighted sum takes pairs of one row, transposed weights and a reduction that is not empty");
+    if (d->pairs > 0 && d->n > 0 && scores == nullptr) return fail(NVQ_INVALID_ARGUMENT, "gather_qmm: null operand");
+    NVQ_TRY(check_aligned("gather_qmm", "scores", scores, 2));
+    const GluEpilogue sums{-1, 0.0f, 0.0f, expert_bias, scores, choices};
+    return gather_qmm_any(d, x, w, scales, biases, global_scales, lhs, rhs, nullptr, nullptr, out, nullptr, stream, &sums);
 }
 
 int32_t nvq_gather_qmm_glu(const nvq_gather_desc *d, int32_t activation, float alpha, float limit, const void *x, const void *w,

@@ -116,6 +116,9 @@ int32_t launch_qmv_dot8(const ProductArgs &a, hipStream_t s);
 int qmv_dot8_rows_per_wave(int64_t n, int cus);  // rows a wavefront takes, by the weight's rows and the chip's compute units
 bool qmv_glu_pairs_take(const ProductArgs &a);      // whether the decode kernel takes unsorted pairs with the gated epilogue
 int32_t launch_qmv_glu_pairs(const ProductArgs &a, hipStream_t s);
+// The products of `choices` pairs a token, one row each, and their weighted sum with the scores [tokens, choices] in one kernel.
+bool qmv_sum_takes(const ProductArgs &a, int64_t choices);
+int32_t launch_qmv_sum(const ProductArgs &a, const void *scores, void *out, int64_t choices, hipStream_t s);
 bool qmv_block_decode_takes(const ProductArgs &a);  // whether the decode kernel takes a product of a block format
 bool qmv_decode_takes_width(const ProductArgs &a);  // whether the decode kernel takes these few rows of 3- or 8-bit affine codes
 // The 16x16x32 matrix-core kernel for passes of up to 16 rows of x (affine 2, 3, 4 and 8 bits, every group size).

@@ -17,6 +17,8 @@
 #include "qmf_kernel.h"  // matrix-instruction wrappers
 #include "qmv_common.h"
 
+#include <cstring>
+
 namespace nvq {
 namespace {
 
@@ -261,6 +263,7 @@ constexpr int kAffine6 = 66;  // ... of 6 bits: six dwords, three to a uint4
 constexpr int kAffine5 = 67;  // ... of 5 bits: five dwords, three and two
 constexpr int kAffine2 = 68;  // ... of 2 bits: two dwords
 constexpr bool is_affine_mode(int mode) { return mode == NVQ_AFFINE || mode == kAffine8 || mode == kAffine3 || mode == kAffine6 || mode == kAffine5 || mode == kAffine2; }
+constexpr int slice_bits(int mode) { return mode == NVQ_MXFP8 || mode == kAffine8 ? 8 : mode == kAffine3 ? 3 : mode == kAffine6 ? 6 : mode == kAffine5 ? 5 : mode == kAffine2 ? 2 : 4; }
 constexpr int slice_quads(int mode) { return mode == NVQ_MXFP8 || mode == kAffine8 || mode == kAffine6 || mode == kAffine5 ? 2 : 1; }  // uint4 that carry a lane's 32 codes
 template <typename T, int MODE> struct SliceScale { using type = std::conditional_t<is_affine_mode(MODE), T, std::conditional_t<MODE == NVQ_NVFP4, uint16_t, uint8_t>>; };
 
@@ -477,6 +480,86 @@ __device__ __forceinline__ void slice_dot(const uint4 (&wq)[slice_quads(MODE)], 
     }
 }
 
+// A lane's slice of weight row n from value kc on: its codes, scales and bias requested.
+template <typename T, int MODE, typename S>
+__device__ __forceinline__ void load_slice(const uint32_t *w, const S *scales, const S *biases, int n, int kwords, int kgroups, int gshift, int kc,
+                                           uint4 (&wq)[slice_quads(MODE)], typename SliceScale<T, MODE>::type &sraw, T &braw) {
+    constexpr int BITS = slice_bits(MODE), kQuads = slice_quads(MODE);
+    // the codes are read once: a non-temporal load keeps them from displacing x and the scales in the caches
+    // (8.1 -> 7.8 us at W[14336,4096]; the scales, shared by neighbouring lanes and rows, lose by it)
+    if constexpr (BITS == 2) {  // two dwords (rows are whole multiples of 8 bytes: K % 32 == 0)
+        const uint2 v = stream_load(reinterpret_cast<const uint2 *>(w + (int64_t)n * kwords + (kc >> 5) * 2));
+        wq[0] = make_uint4(v.x, v.y, 0u, 0u);
+    } else if constexpr (BITS == 3) {  // three dwords, dword-aligned
+        typedef uint32_t u32x3_a4_t __attribute__((ext_vector_type(3), aligned(4)));
+        const u32x3_a4_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x3_a4_t *>(w + (int64_t)n * kwords + (kc >> 5) * 3));
+        wq[0] = make_uint4(v.x, v.y, v.z, 0u);
+    } else if constexpr (BITS == 6 || BITS == 5) {  // three dwords and three (5 bits: two), dword-aligned
+        typedef uint32_t u32x3_a4_t __attribute__((ext_vector_type(3), aligned(4)));
+        typedef uint32_t u32x2_a4_t __attribute__((ext_vector_type(2), aligned(4)));
+        const uint32_t *pw = w + (int64_t)n * kwords + (kc >> 5) * BITS;
+        const u32x3_a4_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x3_a4_t *>(pw));
+        wq[0] = make_uint4(v.x, v.y, v.z, 0u);
+        if constexpr (BITS == 6) {
+            const u32x3_a4_t t = __builtin_nontemporal_load(reinterpret_cast<const u32x3_a4_t *>(pw + 3));
+            wq[1] = make_uint4(t.x, t.y, t.z, 0u);
+        } else {
+            const u32x2_a4_t t = __builtin_nontemporal_load(reinterpret_cast<const u32x2_a4_t *>(pw + 3));
+            wq[1] = make_uint4(t.x, t.y, 0u, 0u);
+        }
+    } else {
+        const uint4 *pw = reinterpret_cast<const uint4 *>(w + (int64_t)n * kwords + (kc >> 5) * BITS);
+#pragma unroll
+        for (int c = 0; c < kQuads; c++) wq[c] = stream_load(pw + c);
+    }
+    sraw = *reinterpret_cast<const typename SliceScale<T, MODE>::type *>(scales + (int64_t)n * kgroups + (kc >> gshift));
+    if constexpr (is_affine_mode(MODE)) braw = (biases + (int64_t)n * kgroups)[kc >> gshift];
+    else braw = T{};
+}
+
+// The bias of weight row n, requested with the weights: read at the end it cost every block a trip to memory more.  Without a bias the
+// same load reads `w` (a branch here would make the wait for x, counted over both of its ways, wait for weights too).
+template <typename T>
+__device__ __forceinline__ T early_bias(const void *row_bias, const void *w, int64_t n) { return *((const T *)(row_bias == nullptr ? w : row_bias) + (row_bias == nullptr ? 0 : n)); }
+template <typename T>
+__device__ __forceinline__ float add_early_bias(const void *row_bias, float v, T bias) {
+    return row_bias == nullptr ? v : Elem<T>::add(Elem<T>::mul(v, 1.0f), Elem<T>::load(&bias, 0));
+}
+
+// Eight values of x as the codes of a slice meet them; the sum of eight values in that order.
+template <int MODE>
+__device__ __forceinline__ uint4 slice_order(const uint4 q) {  // q.x = (x0,x1) q.y = (x2,x3) q.z = (x4,x5) q.w = (x6,x7)
+    uint4 pr = q;
+    if constexpr (MODE == kAffine6 || MODE == kAffine5) {
+        pr.x = __builtin_amdgcn_perm(q.y, q.x, 0x05040100u);  // (x0, x2)
+        pr.y = __builtin_amdgcn_perm(q.y, q.x, 0x07060302u);  // (x1, x3)
+        pr.z = __builtin_amdgcn_perm(q.w, q.z, 0x05040100u);  // (x4, x6)
+        pr.w = __builtin_amdgcn_perm(q.w, q.z, 0x07060302u);  // (x5, x7)
+    } else if constexpr (is_affine_mode(MODE) && MODE != kAffine8) {  // (8-bit codes and block formats are converted in memory order)
+        pr.x = __builtin_amdgcn_perm(q.z, q.x, 0x05040100u);  // (x0, x4)
+        pr.y = __builtin_amdgcn_perm(q.z, q.x, 0x07060302u);  // (x1, x5)
+        pr.z = __builtin_amdgcn_perm(q.w, q.y, 0x05040100u);  // (x2, x6)
+        pr.w = __builtin_amdgcn_perm(q.w, q.y, 0x07060302u);  // (x3, x7)
+    }
+    return pr;
+}
+template <typename T>
+__device__ __forceinline__ float slice_sum(const uint4 pr) {  // of a lane's 32 values, whose pieces sit in four adjacent threads
+    constexpr uint32_t ones = std::is_same<T, bf16_t>::value ? 0x3F803F80u : 0x3C003C00u;
+    float sum = Pair<T>::dot2(pr.x, ones, 0.0f);
+    sum = Pair<T>::dot2(pr.y, ones, sum);
+    sum = Pair<T>::dot2(pr.z, ones, sum);
+    sum = Pair<T>::dot2(pr.w, ones, sum);
+    sum += __shfl_xor(sum, 1);
+    return sum + __shfl_xor(sum, 2);
+}
+template <int MODE>
+__device__ __forceinline__ void code_constants(uint32_t &mask, uint32_t &magic, uint32_t pair) {  // kept in registers
+    constexpr int BITS = slice_bits(MODE);
+    asm volatile("s_mov_b32 %0, %1" : "=s"(mask) : "i"(BITS == 3 ? 0x00070007 : BITS == 6 ? 0x003F003F : BITS == 5 ? 0x001F001F : BITS == 2 ? 0x00030003 : 0x000F000F));
+    asm volatile("v_mov_b32 %0, %1" : "=v"(magic) : "s"(pair));
+}
+
 // ── 4-bit affine and the block formats, bf16 / f16, one to four rows of x: the decode kernel ───────────
 // A block of WAVES wavefronts shares the x slice of one K step (4096 values) through LDS, stored
 // once in the pair order the codes need (affine: together with the sums of its 32-value slices), so the
@@ -499,9 +582,8 @@ __global__ void __launch_bounds__(WAVES * 64) qmv4_lds_kernel(const ProductArgs 
     constexpr int kXPerThread = 512 / kThreads;  // 128-bit pieces of one x row per thread and step
     static_assert(512 % kThreads == 0, "a step of x must split evenly over the block");
     constexpr bool kAffine = is_affine_mode(MODE);
-    constexpr int BITS = MODE == NVQ_MXFP8 || MODE == kAffine8 ? 8 : MODE == kAffine3 ? 3 : MODE == kAffine6 ? 6 : MODE == kAffine5 ? 5 : MODE == kAffine2 ? 2 : 4;
+    constexpr int BITS = slice_bits(MODE);
     constexpr int kQuads = slice_quads(MODE);           // loads of a lane's 32 codes (16 bytes each; 3, 5 and 6 bits: 12 and 8)
-    constexpr int kHalves = MODE == NVQ_NVFP4 ? 2 : 1;  // groups per lane slice
     __shared__ uint4 x_pairs[RM][2][4][64];               // [row][chunk][word][lane]: 4 pairs of eight values
     __shared__ float x_sums[kAffine ? RM : 1][2][64];     // [row][chunk][lane]: sum of the lane's 32 values (affine)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -521,14 +603,13 @@ __global__ void __launch_bounds__(WAVES * 64) qmv4_lds_kernel(const ProductArgs 
     using S = std::conditional_t<kAffine, T, uint8_t>;  // a scale as stored: the element type, or one byte (E8M0; NVFP4: E4M3)
     const S *scales = (const S *)a.scales + o.s, *biases = kAffine ? (const S *)a.biases + o.s : nullptr;
     T *y = (T *)a.y + o.y;
-    constexpr uint32_t ones = std::is_same<T, bf16_t>::value ? 0x3F803F80u : 0x3C003C00u;
     uint32_t mask, magic;
-    asm volatile("s_mov_b32 %0, %1" : "=s"(mask) : "i"(BITS == 3 ? 0x00070007 : BITS == 6 ? 0x003F003F : BITS == 5 ? 0x001F001F : BITS == 2 ? 0x00030003 : 0x000F000F));
-    asm volatile("v_mov_b32 %0, %1" : "=v"(magic) : "s"(Pair<T>::magic));
+    code_constants<MODE>(mask, magic, Pair<T>::magic);
     float factor = 1.0f;
     if constexpr (MODE == NVQ_NVFP4) factor = qmf::nvfp4_factor(a, BATCHED && a.rhs != nullptr ? (int64_t)a.rhs[blockIdx.z] : 0);
 
     float acc[RN][RM];
+    T bias[RN];
 #pragma unroll
     for (int r = 0; r < RN; r++)
 #pragma unroll
@@ -556,68 +637,22 @@ __global__ void __launch_bounds__(WAVES * 64) qmv4_lds_kernel(const ProductArgs 
 #pragma unroll
             for (int r = 0; r < RN; r++) {
                 const int n = n0 + r * kRowStep < N ? n0 + r * kRowStep : N - 1;  // tail rows are computed, not stored
-                // the codes are read once: a non-temporal load keeps them from displacing x and the scales in the caches
-                // (8.1 -> 7.8 us at W[14336,4096]; the scales, shared by neighbouring lanes and rows, lose by it)
-                if constexpr (BITS == 2) {  // two dwords (rows are whole multiples of 8 bytes: K % 32 == 0)
-                    const uint2 v = stream_load(reinterpret_cast<const uint2 *>(w + (int64_t)n * kwords + (kc >> 5) * 2));
-                    wq[u][r][0] = make_uint4(v.x, v.y, 0u, 0u);
-                } else if constexpr (BITS == 3) {  // three dwords, dword-aligned
-                    typedef uint32_t u32x3_a4_t __attribute__((ext_vector_type(3), aligned(4)));
-                    const u32x3_a4_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x3_a4_t *>(w + (int64_t)n * kwords + (kc >> 5) * 3));
-                    wq[u][r][0] = make_uint4(v.x, v.y, v.z, 0u);
-                } else if constexpr (BITS == 6 || BITS == 5) {  // three dwords and three (5 bits: two), dword-aligned
-                    typedef uint32_t u32x3_a4_t __attribute__((ext_vector_type(3), aligned(4)));
-                    typedef uint32_t u32x2_a4_t __attribute__((ext_vector_type(2), aligned(4)));
-                    const uint32_t *pw = w + (int64_t)n * kwords + (kc >> 5) * BITS;
-                    const u32x3_a4_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x3_a4_t *>(pw));
-                    wq[u][r][0] = make_uint4(v.x, v.y, v.z, 0u);
-                    if constexpr (BITS == 6) {
-                        const u32x3_a4_t t = __builtin_nontemporal_load(reinterpret_cast<const u32x3_a4_t *>(pw + 3));
-                        wq[u][r][1] = make_uint4(t.x, t.y, t.z, 0u);
-                    } else {
-                        const u32x2_a4_t t = __builtin_nontemporal_load(reinterpret_cast<const u32x2_a4_t *>(pw + 3));
-                        wq[u][r][1] = make_uint4(t.x, t.y, 0u, 0u);
-                    }
-                } else {
-                    const uint4 *pw = reinterpret_cast<const uint4 *>(w + (int64_t)n * kwords + (kc >> 5) * BITS);
-#pragma unroll
-                    for (int c = 0; c < kQuads; c++) wq[u][r][c] = stream_load(pw + c);
-                }
-                sraw[u][r] = *reinterpret_cast<const SR *>(scales + (int64_t)n * kgroups + (kc >> gshift));
-                if constexpr (kAffine) braw[u][r] = (biases + (int64_t)n * kgroups)[kc >> gshift];
-                else braw[u][r] = T{};
+                load_slice<T, MODE>(w, scales, biases, n, kwords, kgroups, gshift, kc, wq[u][r], sraw[u][r], braw[u][r]);
             }
         }
+#pragma unroll
+        for (int r = 0; r < RN; r++) bias[r] = early_bias<T>(a.row_bias, w, o.bias + (n0 + r * kRowStep < N ? n0 + r * kRowStep : N - 1));
         if (k0 != 0) __syncthreads();  // the previous step's readers are done with the LDS
 #pragma unroll
         for (int i = 0; i < RM; i++)
 #pragma unroll
             for (int p = 0; p < kXPerThread; p++) {
                 const int idx = tid + p * kThreads;  // 128-bit piece: chunk idx/256, lane (idx%256)/4, word idx%4
-                const uint4 q = xg[i][p];            // q.x = (x0,x1) q.y = (x2,x3) q.z = (x4,x5) q.w = (x6,x7)
+                const uint4 pr = slice_order<MODE>(xg[i][p]);
+                x_pairs[i][idx >> 8][idx & 3][(idx & 255) >> 2] = pr;
                 if constexpr (kAffine) {
-                    uint4 pr = q;
-                    if constexpr (MODE == kAffine6 || MODE == kAffine5) {
-                        pr.x = __builtin_amdgcn_perm(q.y, q.x, 0x05040100u);  // (x0, x2)
-                        pr.y = __builtin_amdgcn_perm(q.y, q.x, 0x07060302u);  // (x1, x3)
-                        pr.z = __builtin_amdgcn_perm(q.w, q.z, 0x05040100u);  // (x4, x6)
-                        pr.w = __builtin_amdgcn_perm(q.w, q.z, 0x07060302u);  // (x5, x7)
-                    } else if constexpr (MODE != kAffine8) {  // (8-bit codes are converted in memory order)
-                        pr.x = __builtin_amdgcn_perm(q.z, q.x, 0x05040100u);  // (x0, x4)
-                        pr.y = __builtin_amdgcn_perm(q.z, q.x, 0x07060302u);  // (x1, x5)
-                        pr.z = __builtin_amdgcn_perm(q.w, q.y, 0x05040100u);  // (x2, x6)
-                        pr.w = __builtin_amdgcn_perm(q.w, q.y, 0x07060302u);  // (x3, x7)
-                    }
-                    x_pairs[i][idx >> 8][idx & 3][(idx & 255) >> 2] = pr;
-                    float sum = Pair<T>::dot2(pr.x, ones, 0.0f);
-                    sum = Pair<T>::dot2(pr.y, ones, sum);
-                    sum = Pair<T>::dot2(pr.z, ones, sum);
-                    sum = Pair<T>::dot2(pr.w, ones, sum);
-                    sum += __shfl_xor(sum, 1);  // the four pieces of a lane's slice sit in adjacent threads
-                    sum += __shfl_xor(sum, 2);
+                    const float sum = slice_sum<T>(pr);
                     if ((idx & 3) == 0) x_sums[i][idx >> 8][(idx & 255) >> 2] = sum;
-                } else {
-                    x_pairs[i][idx >> 8][idx & 3][(idx & 255) >> 2] = q;  // (the conversions give the code values in memory order)
                 }
             }
         __syncthreads();
@@ -644,7 +679,7 @@ __global__ void __launch_bounds__(WAVES * 64) qmv4_lds_kernel(const ProductArgs 
             const float g = wave_sum_lane63(acc[0][i]), u = wave_sum_lane63(acc[1][i]);
             if (lane == 63 && column < H && m0 + i < M) {
                 // the products as their outputs hold them, the expert's bias by a separate rounded addition
-                const float gate = add_row_bias<T>(a.row_bias, rounded<T>(g), o.bias + n0), up = add_row_bias<T>(a.row_bias, rounded<T>(u), o.bias + n0 + 64);
+                const float gate = add_early_bias<T>(a.row_bias, rounded<T>(g), bias[0]), up = add_early_bias<T>(a.row_bias, rounded<T>(u), bias[1]);
                 const float v = a.glu == 1 + NVQ_GLU_SWIGLU       ? glu<T, NVQ_GLU_SWIGLU>(gate, up, a.glu_alpha, a.glu_limit)
                                 : a.glu == 1 + NVQ_GLU_SWIGLU_OAI ? glu<T, NVQ_GLU_SWIGLU_OAI>(gate, up, a.glu_alpha, a.glu_limit)
                                                                   : glu<T, NVQ_GLU_GEGLU>(gate, up, a.glu_alpha, a.glu_limit);
@@ -658,7 +693,7 @@ __global__ void __launch_bounds__(WAVES * 64) qmv4_lds_kernel(const ProductArgs 
 #pragma unroll
         for (int i = 0; i < RM; i++) {
             const float v = wave_sum_lane63(acc[r][i]);
-            if (lane == 63 && n0 + r < N && m0 + i < M) Elem<T>::store(y, (int64_t)(m0 + i) * N + n0 + r, add_row_bias<T>(a.row_bias, v, o.bias + n0 + r));
+            if (lane == 63 && n0 + r < N && m0 + i < M) Elem<T>::store(y, (int64_t)(m0 + i) * N + n0 + r, add_early_bias<T>(a.row_bias, v, bias[r]));
         }
 }
 
@@ -1327,6 +1362,122 @@ int32_t run_glu_pairs(const ProductArgs &a, hipStream_t s) {
     }
 }
 
+// ── a token's experts summed: the down products of a token's pairs (one row each) and their weighted sum in one kernel ──
+// A block takes `columns` outputs of a token with all its `choices` pairs: wavefront (g, j) RN weight rows of pair j's expert as
+// qmv4_lds_kernel does (the same slices and sums), the pairs' x in LDS together; the rounded, biased products meet in LDS and are summed
+// with the scores in the order of weighted_sum_kernel: bit for bit the two kernels.
+template <typename T, int RN, int MODE>
+__global__ void __launch_bounds__(512) qmv4_sum_kernel(const ProductArgs a, const T *__restrict__ scores, T *__restrict__ out, int choices, int groups) {
+    constexpr bool kAffine = is_affine_mode(MODE);
+    constexpr int kPieces = 4;  // of x a thread stages a step: 512 a row over 64 * choices * groups threads, groups at least 2
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+    uint4 *x_pairs = reinterpret_cast<uint4 *>(lds_raw);                       // [pair][chunk][word][lane]
+    float *x_sums = reinterpret_cast<float *>(x_pairs + choices * 512);        // [pair][chunk][lane] (affine)
+    float *products = x_sums + (kAffine ? choices * 128 : 0);                  // [pair][column]
+    __shared__ float score[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), threads = 64 * choices * groups;
+    const int K = (int)a.k, N = (int)a.n, g = wave / choices, j = wave - g * choices, columns = groups * RN;
+    const int n0 = (int)blockIdx.x * columns + g * RN;
+    const int64_t first = (int64_t)blockIdx.y * choices;  // pair
+    const int gshift = kAffine ? (a.group == 32 ? 5 : a.group == 64 ? 6 : 7) : (MODE == NVQ_NVFP4 ? 4 : 5);
+    const int kwords = (K * slice_bits(MODE)) >> 5, kgroups = K >> gshift;
+    const BatchOffsets o = batch_offsets(a, first + j, kwords, kgroups);
+    using S = std::conditional_t<kAffine, T, uint8_t>;
+    const uint32_t *w = (const uint32_t *)a.w + o.w;
+    const S *scales = (const S *)a.scales + o.s, *biases = kAffine ? (const S *)a.biases + o.s : nullptr;
+    uint32_t mask, magic;
+    code_constants<MODE>(mask, magic, Pair<T>::magic);
+    float factor = 1.0f;
+    if constexpr (MODE == NVQ_NVFP4) factor = qmf::nvfp4_factor(a, (int64_t)a.rhs[first + j]);
+    const T *xr[kPieces];  // the rows of x of the thread's pieces
+#pragma unroll
+    for (int p = 0; p < kPieces; p++) {
+        const int pair = (wave + p * choices * groups) >> 3;  // (a row is 8 wavefronts' pieces)
+        xr[p] = (const T *)a.x + min((int64_t)a.lhs[first + (pair < choices ? pair : 0)], a.x_batches - 1) * K;
+    }
+    float acc[RN][1];
+    T bias[RN], mine{};
+#pragma unroll
+    for (int r = 0; r < RN; r++) acc[r][0] = 0.0f;
+    for (int k0 = 0; k0 < K; k0 += 2 * kStep) {
+        uint4 xg[kPieces];
+#pragma unroll
+        for (int p = 0; p < kPieces; p++) {
+            const int idx = tid + p * threads, kx = k0 + (idx & 511) * 8;
+            xg[p] = idx < choices * 512 && kx < K ? *reinterpret_cast<const uint4 *>(xr[p] + kx) : make_uint4(0, 0, 0, 0);
+        }
+        uint4 wq[2][RN][slice_quads(MODE)];
+        typename SliceScale<T, MODE>::type sraw[2][RN];
+        T braw[2][RN];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const int kb = k0 + u * kStep + lane * 32, kc = kb < K ? kb : 0;  // an absent slice reads valid memory; its x is zero
+#pragma unroll
+            for (int r = 0; r < RN; r++)
+                load_slice<T, MODE>(w, scales, biases, n0 + r < N ? n0 + r : N - 1, kwords, kgroups, gshift, kc, wq[u][r], sraw[u][r], braw[u][r]);
+        }
+#pragma unroll
+        for (int r = 0; r < RN; r++) bias[r] = early_bias<T>(a.row_bias, w, o.bias + (n0 + r < N ? n0 + r : N - 1));
+        mine = scores[first + (tid < choices ? tid : 0)];
+        if (k0 != 0) __syncthreads();  // the previous step's readers are done with the LDS
+#pragma unroll
+        for (int p = 0; p < kPieces; p++) {
+            const int idx = tid + p * threads;
+            if (idx >= choices * 512) break;  // (a wavefront's pieces are of one row)
+            const uint4 pr = slice_order<MODE>(xg[p]);
+            x_pairs[(idx >> 8) * 256 + (idx & 3) * 64 + ((idx & 255) >> 2)] = pr;
+            if constexpr (kAffine) {
+                const float sum = slice_sum<T>(pr);
+                if ((idx & 3) == 0) x_sums[(idx >> 8) * 64 + ((idx & 255) >> 2)] = sum;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            uint4 xp[1][4];
+            float xs[1] = {0.0f};
+#pragma unroll
+            for (int c = 0; c < 4; c++) xp[0][c] = x_pairs[(2 * j + u) * 256 + c * 64 + lane];
+            if constexpr (kAffine) xs[0] = x_sums[(2 * j + u) * 64 + lane];
+#pragma unroll
+            for (int r = 0; r < RN; r++) slice_dot<T, 1, MODE>(wq[u][r], sraw[u][r], braw[u][r], xp, xs, factor, mask, magic, acc[r]);
+        }
+    }
+    if (tid < choices) score[tid] = Elem<T>::load(&mine, 0);
+#pragma unroll
+    for (int r = 0; r < RN; r++) {
+        const float v = wave_sum_lane63(acc[r][0]);
+        if (lane == 63 && n0 + r < N) products[j * columns + g * RN + r] = rounded<T>(add_early_bias<T>(a.row_bias, v, bias[r]));
+    }
+    __syncthreads();
+    const int n = (int)blockIdx.x * columns + tid;
+    if (tid >= columns || n >= N) return;
+    float sum = 0.0f;
+    for (int i = 0; i < choices; i++) {
+        const float t = Elem<T>::add(Elem<T>::mul(products[i * columns + tid], score[i]), 0.0f);
+        sum = i == 0 ? t : Elem<T>::add(t, sum);
+    }
+    Elem<T>::store(out, (int64_t)blockIdx.y * N + n, sum);
+}
+
+// Blocks of up to eight wavefronts and four columns or more: a block reads the x of all its pairs, 4 / columns of its 4-bit codes' bytes.
+// (Us, 4 of 32 experts, W[2880,2880] MXFP4, from memory: 8 wavefronts of 1 / 2 / 4 rows 10.6 / 8.0 / 9.0, 4 wavefronts of 2 / 4
+// 10.2 / 8.0, 16 wavefronts of 1 / 2 13.5 / 11.5; the products and their sum as two kernels 7.3 + 2.5 and the gap between them.)
+template <typename T, int RN, int MODE>
+int32_t run_sum_rows(const ProductArgs &a, const void *scores, void *out, int choices, hipStream_t s) {
+    const int groups = 8 / choices, columns = groups * RN;
+    const size_t lds = (size_t)choices * (8192 + (is_affine_mode(MODE) ? 512 : 0) + 4 * columns);  // (at most 34.9 KB)
+    const dim3 grid((unsigned)((a.n + columns - 1) / columns), (unsigned)(a.batch / choices));
+    hipLaunchKernelGGL((qmv4_sum_kernel<T, RN, MODE>), grid, dim3((unsigned)(64 * choices * groups)), lds, s, a, (const T *)scores, (T *)out, choices, groups);
+    NVQ_LAUNCH_CHECK("qmv4_sum");
+    return NVQ_OK;
+}
+
+template <typename T, int MODE>
+int32_t run_sum(const ProductArgs &a, const void *scores, void *out, int choices, hipStream_t s) {
+    return choices == 1 ? run_sum_rows<T, 1, MODE>(a, scores, out, choices, s) : run_sum_rows<T, 2, MODE>(a, scores, out, choices, s);
+}
+
 // Whether the decode kernel takes a product of a block format: bf16 / f16, up to kBlockDecodeRows rows of x, whole
 // slices of 32 values (NVFP4 rows may end in half a slice: those stay on the general kernel).  Row-exact products
 // stay on the general kernel at every row count.
@@ -1534,6 +1685,43 @@ int32_t launch_qmv_glu_pairs(const ProductArgs &a, hipStream_t s) {
     if (!glu_pairs_take(a) || a.glu == 0) return fail(NVQ_UNSUPPORTED, "gather_qmm: the decode kernel does not take these pairs with the gated epilogue");
     if (a.batch > 65535) return fail(NVQ_UNSUPPORTED, "gather_qmm: %lld pairs exceed the grid limit", (long long)a.batch);
     return a.dtype == NVQ_BF16 ? run_glu_pairs<bf16_t>(a, s) : run_glu_pairs<f16_t>(a, s);
+}
+
+namespace {
+template <typename T>
+int32_t run_sum_typed(const ProductArgs &a, const void *scores, void *out, int choices, hipStream_t s) {
+    switch (a.mode) {
+    case NVQ_MXFP4: return run_sum<T, NVQ_MXFP4>(a, scores, out, choices, s);
+    case NVQ_MXFP8: return run_sum<T, NVQ_MXFP8>(a, scores, out, choices, s);
+    case NVQ_NVFP4: return run_sum<T, NVQ_NVFP4>(a, scores, out, choices, s);
+    default: break;
+    }
+    switch (a.bits) {
+    case 2: return run_sum<T, kAffine2>(a, scores, out, choices, s);
+    case 3: return run_sum<T, kAffine3>(a, scores, out, choices, s);
+    case 4: return run_sum<T, NVQ_AFFINE>(a, scores, out, choices, s);
+    case 5: return run_sum<T, kAffine5>(a, scores, out, choices, s);
+    case 6: return run_sum<T, kAffine6>(a, scores, out, choices, s);
+    default: return run_sum<T, kAffine8>(a, scores, out, choices, s);
+    }
+}
+}  // namespace
+
+// Where the pairs' own kernel is qmv4_lds_kernel, which the sum's kernel equals bit for bit, up to four pairs a token and 32 MB of codes:
+// it saves a launch and a trip of the products through memory, 3.5 us, and costs 0.1 us a MB in x read again (us of a call, the two
+// kernels / here: 4 layers, 4 of 32 experts, W[2880,2880] MXFP4 113 / 102; 6 bits 2 layers, 2 pairs of W[1664,1344] 56 / 48; 8 bits
+// 2 layers, 2 x 4 of W[1920,2368] 101 / 101, 5 x 4 of W[1408,2816] 90 / 95; the 64 KB of eight pairs' x cost 3 bits
+// W[2400,2208] 42.8 / 46.8, 6 bits 4 x 8 of W[1536,1728] 102 / 121).
+bool qmv_sum_takes(const ProductArgs &a, int64_t choices) {
+    if (a.rhs == nullptr || a.dtype == NVQ_F32 || a.m != 1 || a.n < 2 || a.out_rows != nullptr || a.glu != 0) return false;
+    if (choices < 1 || choices > 4 || a.batch % choices != 0 || a.batch / choices > 65535) return false;
+    if ((double)a.batch * (double)a.n * (double)a.k * a.bits > 8.0 * 32e6) return false;
+    return std::strcmp(qmv_kernel_name(a), "qmv4_lds_kernel") == 0;
+}
+
+int32_t launch_qmv_sum(const ProductArgs &a, const void *scores, void *out, int64_t choices, hipStream_t s) {
+    if (!qmv_sum_takes(a, choices)) return fail(NVQ_UNSUPPORTED, "gather_qmm: the decode kernel does not take these pairs with their weighted sum");
+    return a.dtype == NVQ_BF16 ? run_sum_typed<bf16_t>(a, scores, out, (int)choices, s) : run_sum_typed<f16_t>(a, scores, out, (int)choices, s);
 }
 
 int32_t launch_qmv(const ProductArgs &a, hipStream_t s) {

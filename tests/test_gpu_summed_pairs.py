@@ -1,0 +1,56 @@
+"""The down products of a token's experts and their weighted sum in one kernel (`nvq_gather_qmm_sum`; MoeMlp::forward,
+crates/nuvec-lm/src/model.rs:2248-2271): bit for bit `nvq_gather_qmm_expert_bias` and `nvq_weighted_sum`."""
+import ctypes as C
+
+import pytest
+import torch
+
+import nuvec_amd as nv
+from nuvec_amd import _lib, ops
+
+pytestmark = pytest.mark.gpu
+
+p = lambda t: None if t is None else C.c_void_p(t.data_ptr())
+
+
+def call(q, x, lhs, rhs, bias, scores, out, pairs, rows):
+    n, k = q.weight.shape[1], x.shape[1]
+    d = _lib.GatherDescC(q.quant._c(), ops._CODE[x.dtype], 1, 0, 0, 1, n, k, pairs, rows, q.weight.shape[0])
+    return _lib.load().nvq_gather_qmm_sum(C.byref(d), p(x), p(q.weight), p(q.scales), p(q.biases), p(q.global_scale), p(lhs), p(rhs), p(bias),
+                                          p(scores), scores.shape[1], p(out), ops._stream())
+
+
+# n: rows that end inside a wavefront's, a block's; k: part of a step, of its second half, a second step
+@pytest.mark.parametrize("quant,n,k", [("MXFP4", 2, 2080), ("MXFP4", 1025, 4128), ("MXFP8", 130, 2912), ("NVFP4", 67, 4096), ((64, 4), 1027, 2880), ((32, 8), 1030, 352),
+                                       ((32, 2), 1026, 2144), ((32, 3), 1024, 4384), ((64, 5), 1035, 1088), ((128, 6), 1041, 640)], ids=str)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_equals_the_products_and_their_sum(quant, n, k, dtype):
+    torch.manual_seed(n + k)
+    put = lambda *shape: torch.randn(shape, device="cuda").to(dtype)
+    kind = nv.Quant.affine(*quant) if isinstance(quant, tuple) else nv.Quant.new(getattr(nv.QuantMode, quant))
+    q = nv.quantize(put(5, n, k) * 0.1, kind)
+    if quant == "NVFP4":
+        q = nv.Quantized(q.weight, q.scales, None, q.quant, torch.rand(5, device="cuda") * 3 + 0.5)
+    for tokens, choices in ((1, 1), (3, 1), (1, 2), (2, 3), (1, 4), (2, 4)):
+        pairs = tokens * choices
+        rhs = torch.randint(0, 5, (pairs,), device="cuda", dtype=torch.int32)
+        for rows, lhs in ((pairs, torch.arange(pairs, device="cuda", dtype=torch.int32)), (2, torch.randint(0, 2, (pairs,), device="cuda", dtype=torch.int32))):
+            for bias in (None, put(5, n)):
+                x, scores, out = put(rows, k), torch.rand(tokens, choices, device="cuda").to(dtype), torch.full((tokens, n), 7.0, device="cuda", dtype=dtype)
+                _lib.check(call(q, x, lhs, rhs, bias, scores, out, pairs, rows))
+                d = _lib.GatherDescC(q.quant._c(), ops._CODE[dtype], 1, 0, 0, 1, n, k, pairs, rows, 5)
+                y = torch.empty(tokens, choices, n, device="cuda", dtype=dtype)
+                _lib.check(_lib.load().nvq_gather_qmm_expert_bias(C.byref(d), p(x), p(q.weight), p(q.scales), p(q.biases), p(q.global_scale), p(lhs), p(rhs),
+                                                                  None, None, p(bias), p(y), None, ops._stream()))
+                assert torch.equal(out, ops.weighted_sum(y, scores)), (tokens, choices, rows)
+
+
+def test_what_the_two_kernels_keep():
+    """More than four pairs a token, rows of the CPU's weights, short rows, float32, one output."""
+    torch.manual_seed(1)
+    for quant, n, k, choices, dtype in (((64, 4), 1024, 2880, 5, torch.bfloat16), ((64, 4), 512, 2880, 2, torch.bfloat16), ((64, 4), 1024, 1024, 2, torch.bfloat16),
+                                        ((64, 4), 1024, 2880, 2, torch.float32), ((64, 4), 1, 2880, 2, torch.bfloat16)):
+        q = nv.quantize(torch.randn(5, n, k, device="cuda").to(dtype), nv.Quant.affine(*quant))
+        ids = torch.arange(choices, device="cuda", dtype=torch.int32)
+        x, scores, out = torch.randn(choices, k, device="cuda").to(dtype), torch.rand(1, choices, device="cuda").to(dtype), torch.empty(1, n, device="cuda", dtype=dtype)
+        assert call(q, x, ids, ids, None, scores, out, choices, choices) == _lib.UNSUPPORTED

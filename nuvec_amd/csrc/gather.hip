@@ -2,6 +2,7 @@
 // crates/nuvec-kernels/src/metal/gather_gemm.metal:436-457).
 #include "nvq_device.h"
 #include "nvq_internal.h"
+#include "wave_reduce.h"
 
 namespace nvq {
 namespace {
@@ -276,6 +277,27 @@ __device__ __forceinline__ void route_row(const float *p, float *top, float *tot
     for (int e = threadIdx.x; e < k; e += blockDim.x) Elem<T>::store(scores, e, normalize ? elem_div<T>(top[e], *total) : top[e]);
 }
 
+// The same for up to 64 experts, every wavefront holding all of them, lane e expert e's `v`: a wavefront ranks every so manieth expert by
+// two ballots (one wavefront and a comparison a turn: 1 us of a token's router; a thread an expert, with the probabilities read from
+// LDS, as much).
+template <typename T>
+__device__ __forceinline__ void route_lanes(float v, float *top, uint32_t *__restrict__ indices, T *__restrict__ scores, int n, int k, int normalize) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+    for (int e = wave; e < n; e += waves) {
+        const float u = from_lane(v, e);
+        const bool before = route_less<T>(v, u), level = !before && !route_less<T>(u, v);
+        const int slot = __popcll(__ballot(before && lane < n)) + __popcll(__ballot(level && lane < e)) - (n - k);
+        if (slot >= 0 && lane == 0) top[slot] = u, indices[slot] = (uint32_t)e;
+    }
+    __syncthreads();
+    const int tid = threadIdx.x;
+    if (tid >= k) return;
+    float total = 0.0f;
+    if (normalize)
+        for (int j = 0; j < k; j++) total = Elem<T>::add(top[j], total);
+    Elem<T>::store(scores, tid, normalize ? elem_div<T>(top[tid], total) : top[tid]);
+}
+
 // One block per row, one thread per expert.
 template <typename T>
 __global__ void __launch_bounds__(1024) moe_route_kernel(const T *__restrict__ probs, uint32_t *__restrict__ indices,
@@ -290,8 +312,9 @@ __global__ void __launch_bounds__(1024) moe_route_kernel(const T *__restrict__ p
 // The router of a mixture-of-experts block in one launch (MoeMlp, crates/nuvec-lm/src/model.rs:2218-2272): logits of a token
 // (float32 sums, rounded to the element type), their softmax (float32, rounded once), `moe_route`; and what the gathered
 // products read beside its choices, the token of each pair and the pair's own number.  One block per token, a wavefront per
-// two experts in turn: latency is the bound (a token's 32 x 2880 gate is 184 KB from the L2), and the library's product, two
-// conversions, softmax and `moe_route` took 17.6 us of kernels at one token and 36 us at 256.
+// two experts in turn: latency is the bound, of the 184 KB of a token's 32 x 2880 gate into one compute unit and of what follows, which up
+// to 64 experts every wavefront does by itself (6.8 -> 5.7 us, gates from memory).  The library's product, two conversions, softmax and
+// `moe_route` took 17.6 us of kernels at one token and 36 us at 256.
 template <typename T>
 __global__ void __launch_bounds__(1024) moe_router_kernel(const T *__restrict__ x, const T *__restrict__ gate, int dims, int n, int k, int normalize,
                                                           uint32_t *__restrict__ indices, T *__restrict__ scores,
@@ -327,11 +350,18 @@ __global__ void __launch_bounds__(1024) moe_router_kernel(const T *__restrict__ 
                     for (int i = 0; i < V; i++) sum[u] = __builtin_fmaf(Elem<T>::load(xv, i), Elem<T>::load(gv[u], i), sum[u]);
             }
         }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) sum[0] += __shfl_xor(sum[0], o), sum[1] += __shfl_xor(sum[1], o);
-        if (lane == 0) p[e] = Elem<T>::mul(sum[0], 1.0f), p[e1] = Elem<T>::mul(sum[e1 == e ? 0 : 1], 1.0f);
+        sum[0] = wave_sum_lane63(sum[0]), sum[1] = wave_sum_lane63(sum[1]);
+        if (lane == 63) p[e] = Elem<T>::mul(sum[0], 1.0f), p[e1] = Elem<T>::mul(sum[e1 == e ? 0 : 1], 1.0f);
     }
     __syncthreads();
+    if (n <= 64) {
+        const float logit = lane < n ? p[lane] : -INFINITY;
+        const float power = expf(logit - from_lane(wave_max_lane63(logit), 63));
+        const float share = Elem<T>::mul(power / from_lane(wave_sum_lane63(lane < n ? power : 0.0f), 63), 1.0f);
+        if (tid < k) tokens[row * k + tid] = (uint32_t)row, identity[row * k + tid] = (uint32_t)(row * k + tid);
+        route_lanes<T>(share, top, indices + row * k, scores + row * k, n, k, normalize);
+        return;
+    }
     if (wave == 0) {
         float most = -INFINITY, sum = 0.0f;
         for (int e = lane; e < n; e += 64) most = fmaxf(most, p[e]);

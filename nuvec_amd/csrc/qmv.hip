@@ -16,6 +16,7 @@
 #include "nvq_internal.h"
 #include "qmf_kernel.h"  // matrix-instruction wrappers
 #include "qmv_common.h"
+#include "wave_reduce.h"
 
 #include <cstring>
 
@@ -23,26 +24,6 @@ namespace nvq {
 namespace {
 
 constexpr int kStep = 64 * 32;        // values of K per wavefront step
-
-// v + (v moved across lanes by a DPP control); lanes the control does not feed add 0.
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ float dpp_add(float v) {
-    const int moved = __builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROW_MASK, 0xF, true);
-    return v + __int_as_float(moved);
-}
-
-// Sum over the wavefront in VALU data-parallel-primitive steps (no LDS traffic): shifts by
-// 1, 2, 4, 8 inside each row of 16 lanes, then the row totals carried into the next rows.
-// The total is valid in lane 63 only.
-__device__ __forceinline__ float wave_sum_lane63(float v) {
-    v = dpp_add<0x111, 0xF>(v);  // row_shr:1
-    v = dpp_add<0x112, 0xF>(v);  // row_shr:2
-    v = dpp_add<0x114, 0xF>(v);  // row_shr:4
-    v = dpp_add<0x118, 0xF>(v);  // row_shr:8
-    v = dpp_add<0x142, 0xA>(v);  // row_bcast:15 into rows 1 and 3
-    v = dpp_add<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
-    return v;
-}
 
 // (a & mask) | magic in one instruction.  The mask travels in a scalar register and the
 // constant in a vector register: a three-operand VALU instruction of this ISA takes no

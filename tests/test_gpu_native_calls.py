@@ -263,6 +263,23 @@ def test_router(rows, dims, experts, k, dtype):
     assert torch.equal(index[2].flatten(), torch.arange(rows * k, device="cuda", dtype=torch.int32))
 
 
+@pytest.mark.parametrize("experts", [1, 5, 17, 33, 64, 65])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_router_with_equal_experts(experts, dtype):
+    """Equal logits in the order of a stable sort: the last experts of the highest level, then those of the one below, in ascending order."""
+    import ctypes as C
+    dims, rows, k = 16, 3, min(4, experts)
+    x, gate = torch.ones(rows, dims, device="cuda", dtype=dtype), torch.zeros(experts, dims, device="cuda", dtype=dtype)
+    gate[::16] = 0.25  # logits of 4 and 0, exact
+    index, scores = torch.empty(3, rows, k, dtype=torch.int32, device="cuda"), torch.empty(rows, k, dtype=dtype, device="cuda")
+    nv.ops._init(x)
+    p = lambda t: C.c_void_p(t.data_ptr())
+    _lib.check(_lib.load().nvq_moe_router(nv.ops._CODE[dtype], p(x), p(gate), rows, dims, experts, k, 0, p(index[0]), p(scores), p(index[1]),
+                                          p(index[2]), nv.ops._stream()))
+    want = sorted(range(experts), key=lambda e: (e % 16 == 0, e))[-k:]
+    assert index[0].tolist() == [want] * rows
+
+
 @pytest.mark.parametrize("quant", [nv.Quant.affine(64, 4), nv.Quant.affine(32, 8), nv.Quant.new(nv.QuantMode.MXFP4)], ids=str)
 @pytest.mark.parametrize("dims,hidden,bias,activation", [(256, 1024, True, "swiglu_oai"), (512, 96, False, "swiglu"), (320, 640, True, "geglu")])
 def test_moe_equals_the_python_path(both, quant, dims, hidden, bias, activation):

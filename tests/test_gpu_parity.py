@@ -1302,6 +1302,22 @@ def test_moe_block_routes_multiplies_and_sums():
     assert torch.equal(glu(x, top).view(torch.int16), outputs.view(torch.int16))
 
 
+@pytest.mark.parametrize("activation", ["swiglu", "swiglu_oai", "geglu"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_gated_activation_of_many_outputs(dtype, activation):
+    """Whole runs a thread from 2^20 outputs on: the bits of the same rows in parts of fewer, whole or strided, with biases or not."""
+    torch.manual_seed(5)
+    for rows, hidden, wide in ((2048, 520, 520), (2047, 520, 1040), (2100, 512, 515), (2100, 511, 511)):
+        gate, up = ((torch.randn(rows, wide, device="cuda") * 3).to(dtype)[:, :hidden] for _ in range(2))
+        gate[0, :3] = torch.tensor([float("nan"), float("inf"), -float("inf")])
+        gb, ub = (torch.randn(5, hidden, device="cuda").to(dtype) for _ in range(2))
+        ids = torch.randint(0, 5, (rows,), device="cuda", dtype=torch.int32)
+        for biased in (False, True):
+            run = lambda a, b: nv.glu(gate[a:b], up[a:b], activation, **(dict(gate_bias=gb, up_bias=ub, ids=ids[a:b]) if biased else {}))
+            whole, parts = run(0, rows), torch.cat([run(0, 1000), run(1000, rows)])
+            assert torch.equal(whole.nan_to_num(nan=7.0), parts.nan_to_num(nan=7.0)) and torch.equal(whole.isnan(), parts.isnan())
+
+
 @pytest.mark.parametrize("dtype", [ref.F32, ref.F16, ref.BF16])
 @pytest.mark.parametrize("activation", ["swiglu", "swiglu_oai", "geglu"])
 def test_gated_activation_against_the_oracle(dtype, activation):

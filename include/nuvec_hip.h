@@ -459,6 +459,15 @@ NVQ_API int32_t nvq_quantized_matmul_glu_rows(const nvq_qmm_desc *desc, int32_t 
                                 const void *w, const void *scales, const void *biases, const void *bias, void *y,
                                 void *workspace, void *stream);
 
+/* The same product on the grouped kernel of mixtures of experts, x the rows of its one expert: bfloat16 and float16, 6 to 256 rows, affine
+ * codes of 2 to 8 bits (projections whose products round each weight once) and the block formats without a global scale, K in whole
+ * steps of 64 (3 and 5 bits: 128).  NVQ_UNSUPPORTED where the two products and nvq_glu, or nvq_quantized_matmul_glu_rows, are estimated
+ * faster, or would hold their weights more precisely.  1 from the query: it takes the product (with operands that the launch accepts);
+ * depends on desc alone. */
+NVQ_API int32_t nvq_quantized_matmul_glu_grouped_takes(const nvq_qmm_desc *desc);
+NVQ_API int32_t nvq_quantized_matmul_glu_grouped(const nvq_qmm_desc *desc, int32_t activation, float alpha, float limit, const void *x,
+                                const void *w, const void *scales, const void *biases, const void *bias, void *y, void *stream);
+
 /* The grouped gathered product of the experts' gate and up projections with the gated activation as its epilogue:
  * `SwitchGlu::through` up to its down projection (crates/nuvec-lm/src/model.rs:2157-2169) in one kernel.  w, scales,
  * biases and expert_bias hold both projections in alternating runs of 64 rows (rows 128 b .. 128 b + 63: rows

@@ -205,7 +205,7 @@ nvq_qmm_desc gated_desc(const Tensor &x, int32_t code, const nvq_quant &q, int64
     return d;
 }
 
-// ops.quantized_matmul_glu, or (`several`) ops.quantized_matmul_glu_rows.
+// ops.quantized_matmul_glu, or (`several`) ops.quantized_matmul_glu_grouped or ops.quantized_matmul_glu_rows.
 bool product_glu(const Tensor &x, const Packed &p, const Tensor &bias, int32_t activation, float alpha, float limit, bool several,
                  Tensor &out) {
     const Place at(x);
@@ -217,10 +217,13 @@ bool product_glu(const Tensor &x, const Packed &p, const Tensor &bias, int32_t a
     if (n == 0 || n % 128 != 0 || !bias_fits(bias, at, x.scalar_type(), n)) return false;
     const nvq_qmm_desc d = gated_desc(x, code, p.q, n);
     size_t need = 0;
-    if (several && !nvq_quantized_matmul_glu_rows_takes(&d, &need)) return false;
+    const bool grouped = several && nvq_quantized_matmul_glu_grouped_takes(&d);
+    if (several && !grouped && !nvq_quantized_matmul_glu_rows_takes(&d, &need)) return false;
     Tensor workspace, y = at.empty(with_last(x.sizes(), n / 2), x.scalar_type());
     if (need > 0) workspace = at.empty({(int64_t)need}, at::kByte);
-    const int32_t rc = several ? nvq_quantized_matmul_glu_rows(&d, activation, alpha, limit, ptr(x), ptr(p.w), ptr(p.s), ptr(p.b), ptr(bias),
+    const int32_t rc = grouped   ? nvq_quantized_matmul_glu_grouped(&d, activation, alpha, limit, ptr(x), ptr(p.w), ptr(p.s), ptr(p.b), ptr(bias),
+                                                                    y.mutable_data_ptr(), at.stream())
+                       : several ? nvq_quantized_matmul_glu_rows(&d, activation, alpha, limit, ptr(x), ptr(p.w), ptr(p.s), ptr(p.b), ptr(bias),
                                                                y.mutable_data_ptr(), need > 0 ? workspace.mutable_data_ptr() : nullptr, at.stream())
                                : nvq_quantized_matmul_glu(&d, activation, alpha, limit, ptr(x), ptr(p.w), ptr(p.s), ptr(p.b), ptr(bias),
                                                           y.mutable_data_ptr(), at.stream());
@@ -480,7 +483,7 @@ PyObject *py_mlp(PyObject *, PyObject *const *args, Py_ssize_t n) {
         bool paired = both.p != Py_None;
         if (paired && several) {  // (what the projections' sizes say already: the pair is not read where it would be refused)
             const nvq_qmm_desc d = gated_desc(x, code_of(type), gate.p.q, 2 * gate.p.w.size(0));
-            paired = nvq_quantized_matmul_glu_rows_takes(&d, nullptr);
+            paired = nvq_quantized_matmul_glu_grouped_takes(&d) || nvq_quantized_matmul_glu_rows_takes(&d, nullptr);
         }
         if (paired) {
             const bool fits = read_linear(both.p, fused) && linear_fits(fused, at, type, x.size(-1)) && fused.p.w.size(0) == 2 * gate.p.w.size(0);

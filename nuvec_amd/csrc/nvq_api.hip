@@ -870,6 +870,50 @@ int32_t nvq_quantized_matmul_glu_rows(const nvq_qmm_desc *d, int32_t activation,
     return launch_qms(a, plan, workspace, (hipStream_t)stream);
 }
 
+// Whether the grouped kernel does: by estimate beside whichever of the above serves the pair, with the margins that the timings of 6900
+// pairs (gated_group_us) ask for: beside the split-K kernel's epilogue 16 rows of a long K, and a second pass of one tile of a short one,
+// miss the estimate by more than others.  All pairs of up to 256 rows together take 0.93 of the time before, the third of them that is
+// taken 0.84, one of 75 more than 5 % slower, 1.16 x at worst (MXFP4, W[9728,3968] at 203 rows 85.5 -> 65.5 us; 4 bits W[11648,2432] at 40 rows 35.2 -> 29.5; 8 bits
+// W[11008,4096] at 16 rows 40.6 -> 38.3).  Beside the batched-decode kernel all 68 are (0.91, 1.01 x at worst), beside the direct few-row
+// kernel MXFP4 of 128 blocks and more (19 pairs, 0.61, none slower); MXFP8 and NVFP4, up to 16 rows there, were up to 1.3 x slower.
+static bool gated_group_take(const nvq_qmm_desc *d, const ProductArgs &a, int &groups) {
+    if (a.m <= 5 || a.m > 256) return false;  // (up to five rows an MLP's bits are those of its two products)
+    const double us = gated_group_us(a, groups);
+    if (us == HUGE_VAL) return false;
+    qms::Plan split;
+    if (gated_rows_take(d, a, split)) return us < split.us * (a.m <= 16 && a.k >= 1100 ? 0.85 : a.m > 64 && a.m <= 80 && a.k < 1100 ? 0.9 : 1.0);
+    ProductArgs one = a;
+    one.glu = 0, one.n = a.n / 2;
+    const Route route = pick_route(d, one);
+    if (split_rows_take(one, route, split)) return us < 4.0 + 2.0 * split.us;
+    if (route == Route::kTiled) return us < 4.0 + 2.0 * tiled_us(one);
+    if (route == Route::kFewRows) return us < 0.85 * (4.0 + 2.0 * few_rows_us(one));
+    return route == Route::kBatchedDecode || (route == Route::kFewRowsDirect && a.mode == NVQ_MXFP4 && a.m > 32 && a.n / 128 * ((a.m + 63) / 64) >= 128);
+}
+
+int32_t nvq_quantized_matmul_glu_grouped_takes(const nvq_qmm_desc *d) {
+    if (check_qmm(d, "quantized_matmul") != NVQ_OK || d->m == 0 || d->n == 0 || d->k == 0 || !d->transpose || d->batch_ndim != 0 || d->row_exact ||
+        d->rows || require_device() != NVQ_OK)
+        return 0;
+    ProductArgs a = product_args(d, 1);
+    a.exact_weights = wants_exact_weights(d->quant.mode, d->dtype, d->n / 2, d->m);
+    a.glu = 1;
+    int groups;
+    return gated_group_take(d, a, groups);
+}
+
+int32_t nvq_quantized_matmul_glu_grouped(const nvq_qmm_desc *d, int32_t activation, float alpha, float limit, const void *x, const void *w,
+                                         const void *scales, const void *biases, const void *bias, void *y, void *stream) {
+    const char *op = "quantized_matmul";
+    ProductArgs a;
+    bool empty;
+    int groups;
+    NVQ_TRY(glu_product(op, d, activation, alpha, limit, x, w, scales, biases, bias, y, a, empty));
+    if (empty) return NVQ_OK;
+    if (!gated_group_take(d, a, groups)) return fail(NVQ_UNSUPPORTED, "%s: the grouped kernel does not take this product with the gated epilogue", op);
+    return launch_gated_group(a, groups, (hipStream_t)stream);
+}
+
 int32_t nvq_quantized_matmul_static(const nvq_qmm_desc *d, const void *x, const void *w, const void *scales, const void *biases,
                                     void *y, void *stream) {
     NVQ_TRY(check_qmm(d, "quantized_matmul"));

@@ -86,7 +86,8 @@ struct ProductArgs {
     int64_t x_batches, experts;     // gather: index bounds (an index beyond them is clamped)
     const int32_t *offsets;         // grouped gather: rows of expert e are [offsets[e], offsets[e+1]) of `batch` rows
     int32_t one_group;              // the grouped kernel without offsets: all `batch` rows belong to one weight
-    int32_t k_splits, k_split_steps;  // tiled kernel: K split over grid z (0 or 1: no split), steps of 64 values per split
+    int32_t k_splits, k_split_steps;  // tiled kernel: K split over grid z (0 or 1: no split), steps of 64 values per split; grouped kernel
+                                      // of one group: the groups of a block that split K (0: by its own rule)
     float *partials;                // tiled kernel with a split: float32 [k_splits][m][n], summed by a second kernel
     const float *global_scale;      // NVFP4: NULL, one float32 value, or one per expert of a gather (weights stored [N, K] only)
     const uint32_t *out_rows;       // gather with the weights stored [N, K]: pair z writes block out_rows[z] of y (NULL: block z)
@@ -135,6 +136,8 @@ bool qmm_f32_faster(const ProductArgs &a, double margin);  // estimated below `m
 size_t qmm_f32_workspace_bytes(const ProductArgs &a);
 int32_t launch_qmm_f32(const ProductArgs &a, void *workspace, hipStream_t s);
 bool grouped_rows_take(const ProductArgs &a);
+double gated_group_us(const ProductArgs &a, int &groups);  // estimated duration as one group of the grouped kernel, gated; HUGE_VAL: not taken
+int32_t launch_gated_group(ProductArgs a, int groups, hipStream_t s);
 int32_t launch_grouped_rows(ProductArgs a, hipStream_t s);
 bool qmm_dense_takes(const ProductArgs &a);
 size_t qmm_dense_workspace_bytes(const ProductArgs &a);

@@ -198,8 +198,8 @@ __global__ void __launch_bounds__((kThreads * most_groups(HOLD)), (HOLD == rows:
 }
 
 // Affine weights that the kernels taking these products otherwise, the vector kernels, hold in float32: few pairs, and off whole steps of 64
-// (windows of 128 of odd widths) any.
-inline bool weights_in_terms(const ProductArgs &a) { return a.batch < 64 || a.k % (a.bits % 2 != 0 ? 128 : 64) != 0; }
+// (windows of 128 of odd widths) any.  (The other kernels of several rows of one product round them once.)
+inline bool weights_in_terms(const ProductArgs &a) { return (a.batch < 64 && !a.one_group) || a.k % (a.bits % 2 != 0 ? 128 : 64) != 0; }
 
 // Groups of a block, by the blocks there are of one projection's `columns`: few blocks leave compute units idle and the others with a
 // wavefront a SIMD (32 experts, 12 rows each, us with 1 / 2 / 4 groups: w[768,2432], 192 blocks, 8 bits 28.3 / 22.5 / 21.0, MXFP4 17.0 / 14.0 /
@@ -208,6 +208,7 @@ inline bool weights_in_terms(const ProductArgs &a) { return a.batch < 64 || a.k 
 // its projections have one.  So have row-exact pairs.
 inline int group_count(const ProductArgs &a, int64_t passes, int most) {
     const int64_t columns = a.glu != 0 ? a.n / 2 : a.n, blocks = columns / kRows * passes, windows = (a.k + rows::kWin - 1) / rows::kWin;
+    if (a.one_group && a.k_splits > 0) return a.k_splits < most ? a.k_splits : most;
     if (a.row_exact || columns % kRows != 0) return 1;
     if (most >= 4 && windows >= 12 && blocks * 8 <= 3 * (int64_t)compute_units()) return 4;
     return windows >= 4 && blocks * 4 <= 3 * (int64_t)compute_units() ? 2 : 1;

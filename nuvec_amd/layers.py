@@ -114,10 +114,12 @@ class Mlp:
                 pass
         elif self.gate_up_proj is not None and rows > most:
             p, hidden = self.gate_up_proj, None
-            try:
-                hidden = ops.quantized_matmul_glu_rows(x, p.quantized(), activation, bias=p.bias)
-            except (ops.Unsupported, ops.InvalidArgument):  # (the composition takes what it can, and says what it can not)
-                pass
+            for product in (ops.quantized_matmul_glu_grouped, ops.quantized_matmul_glu_rows):
+                try:
+                    hidden = product(x, p.quantized(), activation, bias=p.bias)
+                    break
+                except (ops.Unsupported, ops.InvalidArgument):  # (the composition takes what it can, and says what it can not)
+                    pass
             if hidden is not None:
                 return self.down_proj(hidden)
         return self.down_proj(ops.glu(self.gate_proj(x), self.up_proj(x), activation))

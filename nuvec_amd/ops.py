@@ -841,6 +841,17 @@ def quantized_matmul_glu_rows(x: torch.Tensor, q: Quantized, activation: str = "
     return out
 
 
+def quantized_matmul_glu_grouped(x: torch.Tensor, q: Quantized, activation: str = "swiglu", *, alpha: float = 1.702, limit: float = 7.0,
+                                 bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """`quantized_matmul_glu_rows` on the grouped kernel of mixtures of experts, the rows of x being those of its one expert.  Raises
+    `Unsupported` up to five rows and where that function, or the two products and `glu`, are estimated faster or hold their weights more
+    precisely."""
+    d, operands, out = _glu_product(x, q, activation, bias)
+    _lib.check(_lib.load().nvq_quantized_matmul_glu_grouped(C.byref(d), GLU_ACTIVATIONS[activation], float(alpha), float(limit),
+                                                            *map(_ptr, operands), _ptr(out), _stream()))
+    return out
+
+
 def _glu_product(x: torch.Tensor, q: Quantized, activation: str, bias: Optional[torch.Tensor]):
     """The checked descriptor, operands (x, codes, scales, biases, bias) and empty result of a product with the gated epilogue."""
     op = "quantized_matmul"

@@ -43,17 +43,17 @@ __device__ __forceinline__ void run_pass(const ProductArgs &a, unsigned char *ld
     for (int m = 0; m < MT; m++)
 #pragma unroll
         for (int t = 0; t < 2; t++) acc[m][t] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    B::run(
-        a, lds + group * B::kLdsBytes, wave, e, n0, k0, min(k0 + turns * rows::kWin, K), turns,
-        [&](int r) {  // an index beyond x is the caller's error: clamped
-            const int at = pass + (r < rows ? r : rows - 1);
-            return a.lhs != nullptr ? min((int64_t)a.lhs[at], a.x_batches - 1) : (int64_t)at;
-        },
-        [&](int t, int r) {
-            const int n = n0 + 64 * t + kTile * wave + r;
-            return n < N ? n : N - 1;  // (tail rows are not stored)
-        },
-        acc);
+    auto xrow = [&](int r) {  // an index beyond x is the caller's error: clamped
+        const int at = pass + (r < rows ? r : rows - 1);
+        return a.lhs != nullptr ? min((int64_t)a.lhs[at], a.x_batches - 1) : (int64_t)at;
+    };
+    auto weight_row = [&](int t, int r) {
+        const int n = n0 + 64 * t + kTile * wave + r;
+        return n < N ? n : N - 1;  // (tail rows are not stored)
+    };
+    const int k1 = min(k0 + turns * rows::kWin, K);
+    B::run(a, lds + group * B::kLdsBytes, wave, e, n0, k0, k1, turns, xrow, weight_row, acc);
+    if constexpr (HOLD == rows::kTerms) rows::sum_plainly<T, BITS, MT, 2>(a, e, k0, k1, xrow, weight_row, acc);
     if (groups > 1) {  // the groups' sums, added in order by the first group's threads
         float *part = reinterpret_cast<float *>(lds);
         __syncthreads();

@@ -101,6 +101,62 @@ __device__ __forceinline__ uint4 left_over(const uint32_t (&dw)[BITS], float s, 
     return make_uint4(t[0], t[1], t[2], t[3]);
 }
 
+// Weights in terms give no sum of their own to an x that is infinite or no number: it meets every term, and zero times it, or the
+// difference of two infinities, is no number where the weight's product is infinite.  Of a wavefront that holds a sum that is not finite all
+// such are formed anew from float32 weights and x, values k0 .. k1 - 1 of K; the finite ones stay.  (Without such a sum a look at the
+// accumulators is all this costs.)
+template <typename T, int BITS, int MT, int NT, class XRow, class WeightRow>
+__device__ __forceinline__ void sum_plainly(const ProductArgs &a, int e, int k0, int k1, XRow xrow, WeightRow weight_row, floatx4_t (&acc)[MT][NT]) {
+    bool finite = true;
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) finite = finite && fabsf(acc[m][t][i]) < INFINITY;
+    if (__all(finite)) return;
+    const int lane = threadIdx.x & 63, l = lane & 15, q = lane >> 4, gshift = a.group == 32 ? 5 : a.group == 64 ? 6 : 7;
+    const int64_t K = a.k;
+    floatx4_t again[MT][NT];
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) again[m][t] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int from = k0; from < k1; from += 16) {  // (whole blocks of 32)
+        const int k = from + 4 * q;
+        float xv[MT][4], wv[NT][4];
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+            const T *row = (const T *)a.x + xrow(kTile * m + l) * K;
+#pragma unroll
+            for (int j = 0; j < 4; j++) xv[m][j] = Elem<T>::load(row, k + j);
+        }
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            const int64_t row = (int64_t)e * a.n + weight_row(t, l), g = row * (K >> gshift) + (k >> gshift);
+            const uint32_t *word = (const uint32_t *)a.w + row * (K / 32 * BITS) + (int64_t)k * BITS / 32;
+            const int bit = k % 32 * BITS % 32;
+            uint64_t codes = word[0];
+            if (bit + 4 * BITS > 32) codes |= (uint64_t)word[1] << 32;  // (a row ends with a dword)
+            const float s = Elem<T>::load((const T *)a.scales, g), b = Elem<T>::load((const T *)a.biases, g);
+#pragma unroll
+            for (int j = 0; j < 4; j++) wv[t][j] = __builtin_fmaf((float)((uint32_t)(codes >> (bit + BITS * j)) & ((1u << BITS) - 1u)), s, b);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int m = 0; m < MT; m++)
+#pragma unroll
+                for (int t = 0; t < NT; t++) again[m][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[t][j], xv[m][j], again[m][t], 0, 0, 0);
+    }
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[m][t][i] = fabsf(acc[m][t][i]) < INFINITY ? acc[m][t][i] : again[m][t][i];
+}
+
 // How affine weights are held: rounded once to the element type, as nuvec's CPU product holds them (qmf::affine_pair), or as terms.
 enum Hold { kRounded, kCpu, kTerms };
 

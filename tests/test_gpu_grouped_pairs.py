@@ -10,7 +10,7 @@ import nuvec_amd as nv
 from nuvec_amd import layers
 from oracle import ref
 from tests.hip_backend import to_dev, to_host
-from tests.test_gpu_half_steps import MODES
+from tests.test_gpu_half_steps import MODES, unrounded
 from tests.test_gpu_parity import make_w, make_x
 
 pytestmark = pytest.mark.gpu
@@ -121,6 +121,36 @@ def test_few_pairs_hold_affine_weights_in_float32():
     dense = codes.double() * spread(q.scales) + spread(q.biases)
     want = torch.einsum("rk,rnk->rn", x.double().cpu(), dense.cpu()[ids.long().cpu()]).cuda()
     assert (got - want).norm() <= 2.0 ** -7 / 12 ** 0.5 * want.norm()
+
+
+# Fewer than 64 pairs, whose affine weights are terms: groups of a block that split K (1024 and 1152 columns), a window's part at the end
+# (K = 1504), weights of which one term is all, and a weight of zero.
+@pytest.mark.parametrize("fmt", [(64, 1), (32, 2), (32, 3), (32, 4), (32, 5), (32, 6), (32, 8)], ids=str)
+@pytest.mark.parametrize("dtype,n,k", [(torch.bfloat16, 1024, 512), (torch.float16, 1152, 1664), (torch.bfloat16, 1030, 640), (torch.float16, 1024, 1504)])
+def test_infinities_in_few_pairs(fmt, dtype, n, k):
+    """What is infinite or no number in a row of x gives that row what its product with the weights gives, and no other row anything."""
+    if k % fmt[0]:
+        pytest.skip("K is not whole groups")
+    torch.manual_seed(n + k)
+    dense = (torch.randn(2, n, k, device="cuda") * 0.05).to(dtype)
+    q = nv.quantize(dense, nv.Quant.affine(*fmt))
+    q.biases[:, 5], q.scales[0, 7, :] = 0.0, 1.0
+    q.biases[0, 7, :] = -1.0 if fmt[1] > 1 else 0.0  # (weights of zero where the code is 1)
+    x = torch.randn(40, k, device="cuda").to(dtype)
+    ids = torch.tensor([0] * 17 + [1] * 23, dtype=torch.int32, device="cuda")
+    run = lambda x: nv.gather_qmm_grouped(x, q, torch.arange(40, dtype=torch.int32, device="cuda"), ids, nv.sorted_offsets(ids, 2))
+    odd = {0: {3: "inf"}, 4: {k - 1: "-inf"}, 16: {k // 2: "nan"}, 17: {0: "inf", 1: "inf"}, 39: {40: "-inf", k - 33: "inf"}}
+    plain = run(x)
+    for row, values in odd.items():
+        for at, value in values.items():
+            x[row, at] = float(value)
+    got = run(x)
+    same = [row for row in range(40) if row not in odd]
+    assert torch.equal(got[same], plain[same])
+    for row in odd:
+        e = int(ids[row])
+        want = (x[row].double().cpu() * unrounded(nv.Quantized(q.weight[e], q.scales[e], q.biases[e], q.quant)).cpu()).sum(-1)
+        assert torch.equal(got[row].double().cpu().nan_to_num(nan=7.0), want.nan_to_num(nan=7.0)), row
 
 
 def test_order_of_few_pairs():

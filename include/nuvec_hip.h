@@ -186,8 +186,8 @@ NVQ_API int32_t nvq_quant_check(const nvq_quant *quant, const char *op);
 NVQ_API int32_t nvq_gather_grouped(int64_t rows, int64_t experts, int32_t row_exact);
 
 /* 1 if the pairs of `tokens` tokens with `choices` experts each run faster ordered by expert, every expert's weights read once, than one
- * by one: from 64 pairs on as in the reference (crates/nuvec-lm/src/model.rs:2189-2192), fewer where the estimate says so (the weights
- * are held no less precisely).  `values`: of an expert's three projections; `scaled`: with a global scale. */
+ * by one: from 64 pairs on as in the reference (crates/nuvec-lm/src/model.rs:2189-2192), fewer where the estimate says so and the weights
+ * are held no less precisely (not MXFP4 and MXFP8 in float16, which rounds those of small scales).  `values`: of an expert's three projections; `scaled`: with a global scale. */
 NVQ_API int32_t nvq_moe_ordered(const nvq_quant *quant, int32_t dtype, int64_t tokens, int32_t choices, int64_t experts, int64_t values,
                                 int32_t scaled);
 

@@ -434,6 +434,11 @@ int32_t nvq_gather_grouped(int64_t rows, int64_t experts, int32_t row_exact) {
     return rows >= least && rows / (experts > 1 ? experts : 1) >= 4;
 }
 
+// Whether `dtype` holds every weight of a block format, its code times its scale (affine codes: the kernels hold those in other ways).
+// float16 rounds MXFP4 below a scale of 2^-23 and MXFP8 below 2^-15, to 5e-6 of all weights at a block maximum of 0.0068 and 4.8e-4 at 1e-4, and
+// overflows beyond 65504.
+static bool block_weights_exact(int32_t mode, int32_t dtype) { return dtype != NVQ_F16 || (mode != NVQ_MXFP4 && mode != NVQ_MXFP8); }
+
 // Ordered, an expert's weights are read once, for the price of the order and of the grouped kernel's longer start.  Bounds fitted to blocks of 2
 // to 31 tokens, 2, 4 and 8 of 8, 16 and 32 experts of [512,512] to [2880,2880], timed both ways, so that (nearly) none gets slower:
 // 273 blocks of block formats, 53 ordered, none slower, all in 0.92 of the time (always the faster side 0.89); 366 of affine codes of 2 to 6
@@ -443,6 +448,7 @@ int32_t nvq_moe_ordered(const nvq_quant *quant, int32_t dtype, int64_t tokens, i
     const double pairs = (double)tokens * (double)choices;
     if (pairs >= 64.0) return 1;
     if (quant == nullptr || scaled || (dtype != NVQ_BF16 && dtype != NVQ_F16) || tokens < 2 || choices < 1 || experts < choices || quant->group_size < 1) return 0;
+    if (!block_weights_exact(quant->mode, dtype)) return 0;  // (one by one the float32 scale multiplies a group's sum)
     const bool affine = quant->mode == NVQ_AFFINE;
     const double chosen = (double)experts * (1.0 - pow(1.0 - (double)choices / (double)experts, (double)tokens));  // were the choice even
     const double megabytes = (double)values * (quant->bits + (affine ? 32.0 : 8.0) / quant->group_size) / 8e6;
@@ -815,7 +821,8 @@ int32_t nvq_quantized_matmul_glu(const nvq_qmm_desc *d, int32_t activation, floa
 }
 
 // Whether the split-K kernel takes the gate and up products of several rows with the gated epilogue: where the two products would run on
-// kernels that hold a weight no more precisely (rounded once; block formats hold it exactly on every kernel), and the bounds of
+// kernels that hold a weight no more precisely (rounded once; block formats exactly, but for MXFP4 and MXFP8 of small scales in float16
+// beside the direct few-row kernel), and the bounds of
 // 700 pairs timed both ways leave it ahead (3 to 256 rows, K 512 to 5120, 1024 to 14336 hidden values, twelve formats: 0.75 of the time
 // of the two products and the activation, 0.71 where taken, 1.04 x at worst; from six rows on).  By estimate beside the few-row kernel,
 // the tiles and itself (of 700 others that it takes 0.59 of the time, one slower than 1.05 x; MXFP8 beside the tiles, whose estimate is high there,
@@ -875,7 +882,8 @@ int32_t nvq_quantized_matmul_glu_rows(const nvq_qmm_desc *d, int32_t activation,
 // miss the estimate by more than others.  All pairs of up to 256 rows together take 0.93 of the time before, the third of them that is
 // taken 0.84, one of 75 more than 5 % slower, 1.16 x at worst (MXFP4, W[9728,3968] at 203 rows 85.5 -> 65.5 us; 4 bits W[11648,2432] at 40 rows 35.2 -> 29.5; 8 bits
 // W[11008,4096] at 16 rows 40.6 -> 38.3).  Beside the batched-decode kernel all 68 are (0.91, 1.01 x at worst), beside the direct few-row
-// kernel MXFP4 of 128 blocks and more (19 pairs, 0.61, none slower); MXFP8 and NVFP4, up to 16 rows there, were up to 1.3 x slower.
+// kernel MXFP4 of 128 blocks and more (19 pairs, 0.61, none slower; in bfloat16, as that kernel multiplies a group's sum by its float32 scale);
+// MXFP8 and NVFP4, up to 16 rows there, were up to 1.3 x slower.
 static bool gated_group_take(const nvq_qmm_desc *d, const ProductArgs &a, int &groups) {
     if (a.m <= 5 || a.m > 256) return false;  // (up to five rows an MLP's bits are those of its two products)
     const double us = gated_group_us(a, groups);
@@ -888,7 +896,7 @@ static bool gated_group_take(const nvq_qmm_desc *d, const ProductArgs &a, int &g
     if (split_rows_take(one, route, split)) return us < 4.0 + 2.0 * split.us;
     if (route == Route::kTiled) return us < 4.0 + 2.0 * tiled_us(one);
     if (route == Route::kFewRows) return us < 0.85 * (4.0 + 2.0 * few_rows_us(one));
-    return route == Route::kBatchedDecode || (route == Route::kFewRowsDirect && a.mode == NVQ_MXFP4 && a.m > 32 && a.n / 128 * ((a.m + 63) / 64) >= 128);
+    return route == Route::kBatchedDecode || (route == Route::kFewRowsDirect && a.mode == NVQ_MXFP4 && block_weights_exact(a.mode, a.dtype) && a.m > 32 && a.n / 128 * ((a.m + 63) / 64) >= 128);
 }
 
 int32_t nvq_quantized_matmul_glu_grouped_takes(const nvq_qmm_desc *d) {

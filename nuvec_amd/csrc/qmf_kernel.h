@@ -45,8 +45,9 @@ typedef float floatx2_t __attribute__((ext_vector_type(2)));
 // The FP4 template parameter of the kernels below names the code format: 0 affine integers with a scale and a bias per
 // group, 1 MXFP4 (E2M1 codes, an E8M0 scale per 32), 2 MXFP8 (E4M3 codes, an E8M0 scale per 32), 3 NVFP4 (E2M1 codes, an
 // E4M3 scale per 16, times the factor of a global scale where the product has one).  Every weight of the block formats
-// is exact in bfloat16 and float16 (at most six significant bits times a power of two) but for NVFP4 with a global
-// scale, whose weights are rounded once to the element type like the affine ones.
+// is exact in bfloat16 (at most six significant bits times a power of two) but for NVFP4 with a global scale, whose
+// weights are rounded once to the element type like the affine ones.  float16 holds as exactly those of NVFP4, MXFP4 from a
+// scale of 2^-23 on and MXFP8 from 2^-15 on, up to 65504; what is finer is rounded to it as the CPU's dequantized weights are.
 constexpr int kAffine = 0, kMxfp4 = 1, kMxfp8 = 2, kNvfp4 = 3;
 typedef float floatx16_t __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
@@ -229,7 +230,7 @@ __device__ __forceinline__ uint4 expand_piece(const uint32_t (&dw)[BITS], float 
 
 // Whether a product of K off whole steps of 64 may take the kernels that hold weights in the element type: where that loses
 // nothing against the vector kernels that took it before, i.e. block formats without a global scale, whose weights the
-// element types hold exactly, and affine products that take the CPU's weights on either.
+// element types hold exactly (float16 not the finest: above), and affine products that take the CPU's weights on either.
 inline bool half_steps_supported(const ProductArgs &a) {
     return a.k % 32 == 0 && (a.mode == NVQ_AFFINE ? a.exact_weights != 0 : a.global_scale == nullptr);
 }

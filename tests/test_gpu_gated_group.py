@@ -62,3 +62,25 @@ def test_refused():
         both = nv.Quantized(*(None if getattr(gate, name) is None else ops.pair_rows(getattr(gate, name), getattr(up, name), 0) for name in ("weight", "scales", "biases")), quant)
         with pytest.raises(nv.Unsupported):
             ops.quantized_matmul_glu_grouped(make(rows, k).to(torch.bfloat16), both, "swiglu")
+
+
+def test_float16_of_small_scales_stays_two_products():
+    """MXFP4 where the two products' kernel multiplies a group's sum by its float32 scale: bfloat16 holds the weights as exactly, float16
+    does not, so its block is bit for bit the composition."""
+    rows, hidden, k = 64, 8192, 2048
+    quant = nv.Quant.new(nv.QuantMode.MXFP4)
+    for dtype in (torch.bfloat16, torch.float16):
+        assert ops.quantized_matmul_route(rows, hidden, k, quant, dtype) == "qmd_kernel"
+        torch.manual_seed(7)
+        make = lambda *shape: torch.randn(shape, device="cuda")
+        linear = lambda n, k, size: layers.QuantizedLinear(*(lambda q: (q.weight, q.scales, q.biases))(nv.quantize(make(n, k) * size, quant)), None, quant)
+        gate, up, down = linear(hidden, k, 1e-7), linear(hidden, k, 1e-7), linear(k, hidden, 0.05)
+        x = (make(rows, k) * 5e3).to(dtype)
+        mlp = layers.Mlp(gate, up, down).fuse_gate_up()
+        both = mlp.gate_up_proj.quantized()
+        if dtype == torch.bfloat16:
+            _check_gated(ops.quantized_matmul_glu_grouped(x, both, "swiglu"), x, gate, up, "swiglu", dtype)
+        else:
+            with pytest.raises(nv.Unsupported):
+                ops.quantized_matmul_glu_grouped(x, both, "swiglu")
+            assert torch.equal(mlp(x), down(ops.glu(gate(x), up(x), "swiglu")))

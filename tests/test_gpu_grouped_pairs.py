@@ -162,3 +162,27 @@ def test_order_of_few_pairs():
     assert not rule(q(mx), torch.bfloat16, 1, 32, 32, many) and not rule(q(mx), torch.float32, 5, 8, 8, many)
     assert not rule(q(nvfp4, torch.ones(8)), torch.bfloat16, 5, 8, 8, many)
     assert rule(q(affine), torch.float32, 64, 1, 8, 1) and not rule(q(affine), torch.bfloat16, 63, 1, 64, many)
+
+
+@pytest.mark.parametrize("mode,size", [("MXFP8", 1e-4), ("MXFP4", 1e-7)])
+def test_few_float16_pairs_of_small_scales(mode, size):
+    """Block scales so small that float16 does not hold a code times its scale: the layer gives what the kernel of pairs one by one
+    gives, whose scales multiply in float32 (its products within float32 sums and an output's rounding of float64)."""
+    torch.manual_seed(3)
+    quant, (count, dims, hidden) = nv.Quant.new(getattr(nv.QuantMode, mode)), (8, 1088, 2368)
+
+    def projection(n, k, size):
+        q = nv.quantize(torch.randn(count, n, k, device="cuda") * size, quant)
+        return layers.SwitchProjection(q.weight, q.scales, q.biases, None, q.quant)
+    glu = layers.SwitchGlu(projection(hidden, dims, size), projection(hidden, dims, size), projection(dims, hidden, 0.05))
+    x = (torch.randn(1, 5, dims, device="cuda") * 5e3).half()
+    ids = torch.stack([torch.randperm(count, device="cuda") for _ in range(5)]).to(torch.int32).reshape(1, 5, 8)
+    xe = x.reshape(1, 5, 1, 1, dims)
+    gate, up = (p.forward(xe, ids, add_bias=False) for p in (glu.gate_proj, glu.up_proj))
+    exact = nv.dequantize(glu.up_proj.quantized(), torch.float32)[ids.long()[0]].double()
+    want = torch.matmul(exact, x.double().reshape(5, 1, dims, 1))[..., 0]
+    assert ((up.reshape(5, 8, hidden).double() - want).abs() <= 2.0 ** -10 * want.abs() + 1e-6 * want.abs().max()).all()
+    want = glu.down_proj.forward(glu.gated(gate, up, ids), ids).squeeze(-2)
+    assert torch.equal(glu.forward(x, ids), want)
+    got = glu.fuse_gate_up().forward(x, ids)
+    assert torch.equal(got, want)

@@ -121,7 +121,9 @@ typedef struct nvq_gather_desc {
     int32_t row_exact; /* crate::row_exact() at the gather (gpu.rs:7325-7340): every pair on the vector kernels, so that a
                           pair has the bits of its one-row product, sorted or not; the caller's grouped rule
                           (nvq_gather_grouped) then asks for 65 rows before it passes `offsets` */
-    int32_t reserved;  /* 0 */
+    int32_t float32_weights; /* 1: fewer than 64 sorted affine pairs hold their weights in float32, as pairs one by one do (an ordered
+                                mixture of experts must not lose what its pairs had), at up to 1.5 times the time; 0: rounded once to
+                                the element type.  Anything else is as it is without. */
     int64_t m, n, k;
     int64_t pairs;
     int64_t x_batches;

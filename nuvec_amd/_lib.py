@@ -72,7 +72,7 @@ class GluDescC(C.Structure):
 
 class GatherDescC(C.Structure):
     _fields_ = [("quant", QuantC), ("dtype", C.c_int32), ("transpose", C.c_int32), ("row_exact", C.c_int32),
-                ("reserved", C.c_int32), ("m", C.c_int64), ("n", C.c_int64), ("k", C.c_int64), ("pairs", C.c_int64),
+                ("float32_weights", C.c_int32), ("m", C.c_int64), ("n", C.c_int64), ("k", C.c_int64), ("pairs", C.c_int64),
                 ("x_batches", C.c_int64), ("experts", C.c_int64)]
 
 

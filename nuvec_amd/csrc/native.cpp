@@ -273,7 +273,7 @@ struct Pairs {
 // writes row `to[z]` (NULL: z).
 bool project(const Place &at, const Tensor &x, int64_t x_rows, const Projection &w, const Pairs &pairs, const uint32_t *from, const uint32_t *to,
              bool with_bias, Tensor &out) {
-    const nvq_gather_desc d{w.p.q, code_of(x.scalar_type()), 1, 0, 0, 1, w.rows, w.columns, pairs.count, x_rows, pairs.experts};
+    const nvq_gather_desc d{w.p.q, code_of(x.scalar_type()), 1, 0, 1, 1, w.rows, w.columns, pairs.count, x_rows, pairs.experts};
     Tensor y = at.empty({pairs.count, w.rows}, x.scalar_type());
     if (nvq_gather_qmm_expert_bias(&d, ptr(x), ptr(w.p.w), ptr(w.p.s), ptr(w.p.b), nullptr, from, pairs.expert, pairs.offsets, to,
                                    with_bias ? ptr(w.bias) : nullptr, y.mutable_data_ptr(), nullptr, at.stream()) != NVQ_OK)
@@ -293,7 +293,7 @@ bool hidden_states(const Place &at, const Tensor &x, int64_t x_rows, Experts &e,
     const at::ScalarType type = x.scalar_type();
     const int64_t hidden = e.down.columns;
     if (e.fused && e.paired) {
-        const nvq_gather_desc d{e.both.p.q, code_of(type), 1, 0, 0, 1, e.both.rows, e.both.columns, pairs.count, x_rows, pairs.experts};
+        const nvq_gather_desc d{e.both.p.q, code_of(type), 1, 0, 1, 1, e.both.rows, e.both.columns, pairs.count, x_rows, pairs.experts};
         Tensor y = at.empty({pairs.count, hidden}, type);
         if (nvq_gather_qmm_glu(&d, e.act.code, e.act.alpha, e.act.limit, ptr(x), ptr(e.both.p.w), ptr(e.both.p.s), ptr(e.both.p.b), tokens,
                                pairs.expert, pairs.offsets, ptr(e.both.bias), y.mutable_data_ptr(), at.stream()) == NVQ_OK) {

@@ -1252,6 +1252,7 @@ static int32_t gather_qmm_any(const nvq_gather_desc *d, const void *x, const voi
     a.global_scale = global_scale;
     a.out_rows = out_rows;
     a.row_exact = d->row_exact != 0;
+    a.float32_weights = d->float32_weights != 0;
     a.exact_weights = wants_exact_weights(d->quant.mode, d->dtype, d->n, a.row_exact ? 1 : d->m);
     if (!d->transpose) {
         // Weights stored [K, N]: rows sorted by expert as groups on the matrix-core kernel (each expert's weights read once

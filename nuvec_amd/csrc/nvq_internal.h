@@ -85,6 +85,7 @@ struct ProductArgs {
     const uint32_t *lhs, *rhs;      // gather: batch z reads x batch lhs[z] and weight batch rhs[z]
     int64_t x_batches, experts;     // gather: index bounds (an index beyond them is clamped)
     const int32_t *offsets;         // grouped gather: rows of expert e are [offsets[e], offsets[e+1]) of `batch` rows
+    int32_t float32_weights;        // grouped kernel: affine weights of fewer than 64 pairs in float32 (else rounded once)
     int32_t one_group;              // the grouped kernel without offsets: all `batch` rows belong to one weight
     int32_t k_splits, k_split_steps;  // tiled kernel: K split over grid z (0 or 1: no split), steps of 64 values per split; grouped kernel
                                       // of one group: the groups of a block that split K (0: by its own rule)

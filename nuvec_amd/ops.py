@@ -717,11 +717,11 @@ def _out_rows(op: str, given: Optional[torch.Tensor], pairs: int, device) -> Opt
 
 def gather_qmm_grouped(x: torch.Tensor, q: Quantized, rows: torch.Tensor, sorted_ids: torch.Tensor,
                        offsets: torch.Tensor, out_rows: Optional[torch.Tensor] = None,
-                       expert_bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+                       expert_bias: Optional[torch.Tensor] = None, float32_weights: bool = True) -> torch.Tensor:
     """The grouped route of `gather_qmm` (quantized.rs:646-651, 772-782) with the rows of x taken inside the kernel:
     output row i = x[rows[i]] . dequantize(w)[sorted_ids[i]]^T for ids sorted by expert (`offsets` from `moe_order`
-    or `sorted_offsets`).  Equal to `gather_qmm(x[rows], q, None, sorted_ids, sorted)`; the gathered copy of x is
-    never written.  x is `[T, K]`, the result `[len(rows), N]`.  With `out_rows` (a permutation, e.g. the `order` of
+    or `sorted_offsets`).  Equal to `gather_qmm(x[rows], q, None, sorted_ids, sorted)` (below 64 affine pairs without
+    `float32_weights`, which holds their weights as pairs one by one do); the gathered copy of x is never written.  x is `[T, K]`, the result `[len(rows), N]`.  With `out_rows` (a permutation, e.g. the `order` of
     `moe_order`) result row i is written at row `out_rows[i]`: the ordered product lands in pair order and
     model.rs:2205-2210's `take(out, inverse)` is not needed.  `expert_bias` `[E, N]` adds each row's expert's bias
     (model.rs:2139-2143) in the kernel's epilogue (`Unsupported` where the grouped kernel does not take the product).
@@ -746,7 +746,7 @@ def gather_qmm_grouped(x: torch.Tensor, q: Quantized, rows: torch.Tensor, sorted
     if lhs.numel() != rhs.numel() or offsets.numel() != w.shape[0] or offsets.dtype != torch.int32:
         raise InvalidArgument(f"{op}: {lhs.numel()} rows, {rhs.numel()} expert ids, {offsets.numel()} offsets for {w.shape[0]} experts")
     out = torch.empty((rhs.numel(), w.shape[-2]), dtype=dtype, device=x.device)
-    d = _lib.GatherDescC(quant._c(), _CODE[dtype], 1, 0, 0, 1, w.shape[-2], columns, rhs.numel(), x.shape[0], w.shape[0])
+    d = _lib.GatherDescC(quant._c(), _CODE[dtype], 1, 0, int(float32_weights), 1, w.shape[-2], columns, rhs.numel(), x.shape[0], w.shape[0])
     scatter = _out_rows(op, out_rows, rhs.numel(), x.device)
     gs = q.global_scale
     if gs is not None:  # quantized.rs:620-636
@@ -775,7 +775,7 @@ def gather_qmm_grouped(x: torch.Tensor, q: Quantized, rows: torch.Tensor, sorted
 
 def gather_qmm_glu(x: torch.Tensor, q: Quantized, rows: torch.Tensor, sorted_ids: torch.Tensor, offsets: Optional[torch.Tensor],
                    activation: str = "swiglu", *, alpha: float = 1.702, limit: float = 7.0,
-                   expert_bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+                   expert_bias: Optional[torch.Tensor] = None, float32_weights: bool = True) -> torch.Tensor:
     """`gather_qmm_grouped` of the experts' gate and up projections with `glu` as the kernel's epilogue
     (`SwitchGlu::through` up to the down projection, model.rs:2157-2169): `q` (and `expert_bias` `[E, N]`) hold both
     projections in alternating runs of 64 rows (`pair_rows`), the result is `[len(rows), N / 2]`, bit for bit
@@ -808,7 +808,7 @@ def gather_qmm_glu(x: torch.Tensor, q: Quantized, rows: torch.Tensor, sorted_ids
                               f"{'no' if offsets is None else offsets.numel()} offsets for {w.shape[0]} experts")
     _init(x)
     out = torch.empty((rhs.numel(), n // 2), dtype=dtype, device=x.device)
-    d = _lib.GatherDescC(quant._c(), _CODE[dtype], 1, 0, 0, 1, n, columns, rhs.numel(), x.shape[0], w.shape[0])
+    d = _lib.GatherDescC(quant._c(), _CODE[dtype], 1, 0, int(float32_weights), 1, n, columns, rhs.numel(), x.shape[0], w.shape[0])
     eb = None if expert_bias is None else expert_bias.contiguous()
     _lib.check(_lib.load().nvq_gather_qmm_glu(C.byref(d), GLU_ACTIVATIONS[activation], float(alpha), float(limit), _ptr(x), _ptr(w),
                                               _ptr(scales), _ptr(biases), _ptr(lhs), _ptr(rhs),

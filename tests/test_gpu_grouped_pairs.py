@@ -153,6 +153,29 @@ def test_infinities_in_few_pairs(fmt, dtype, n, k):
         assert torch.equal(got[row].double().cpu().nan_to_num(nan=7.0), want.nan_to_num(nan=7.0)), row
 
 
+@pytest.mark.parametrize("fmt", [(64, 2), (128, 3), (64, 4), (32, 5), (64, 6), (32, 8)], ids=str)
+@pytest.mark.parametrize("dtype,k", [(torch.bfloat16, 1024), (torch.float16, 384)])
+def test_sorted_gathers_round_each_weight_once(fmt, dtype, k):
+    """However few their pairs are, where nobody asks for float32 weights: the bits that a pair has among 80, and far from those of
+    float32 weights (biases above the codes' steps, rows of x that sum to nothing: what rounding does to a weight is not lost in the sum)."""
+    torch.manual_seed(k)
+    n = 1100  # (off whole blocks: one group of wavefronts, however many pairs)
+    q = nv.quantize(torch.randn(2, n, k, device="cuda") * 0.02 + 0.3, nv.Quant.affine(*fmt))
+    q = nv.Quantized(q.weight, q.scales.to(dtype), q.biases.to(dtype), q.quant)
+    x = torch.randn(80, k // 2, device="cuda").to(dtype)
+    x = torch.stack([x, -x], dim=-1).reshape(80, 1, k)
+    ids = torch.tensor([0] * 30 + [1] * 50, dtype=torch.int32, device="cuda")
+    gather = lambda rows: nv.gather_qmm(x[rows], q, None, ids[rows], nv.GatherQmm(sorted_indices=True))[:, 0]
+    every, few = gather(slice(0, 80)), gather(slice(10, 60))
+    assert torch.equal(few, every[10:60])
+    exact = torch.stack([unrounded(nv.Quantized(q.weight[e], q.scales[e], q.biases[e], q.quant)) for e in range(2)])
+    product = lambda weights: torch.matmul(weights[ids[10:60].long()], x[10:60].double().transpose(1, 2))[..., 0]
+    want, unit = product(exact.to(dtype).double()), 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    # (an output's rounding is half a unit of it at most; a weight's, 2^-10 or 2^-13 of 0.3 at random, is some 3 % or 0.4 % of these sums)
+    assert (few.double() - want).norm() <= unit * want.norm()
+    assert (few.double() - product(exact)).norm() >= 2 * unit * want.norm()
+
+
 def test_order_of_few_pairs():
     rule = nv.ops.moe_ordered
     q = lambda quant, scale=None: nv.Quantized(None, None, None, quant, scale)

@@ -1337,11 +1337,11 @@ int32_t run_glu_pairs_biased(const ProductArgs &a, hipStream_t s) {
     hipLaunchKernelGGL(kernel, grid, dim3(512), 0, s, a);
     NVQ_LAUNCH_CHECK("qmv4_lds with the gated epilogue");
     return NVQ_OK;
+}
+
 template <typename T, int MODE>
 int32_t run_glu_pairs_mode(const ProductArgs &a, hipStream_t s) {
     return a.row_bias != nullptr ? run_glu_pairs_biased<T, MODE, true>(a, s) : run_glu_pairs_biased<T, MODE, false>(a, s);
-}
-
 }
 
 template <typename T>
@@ -1667,6 +1667,9 @@ const char *qmv_kernel_name(const ProductArgs &a) {
         if (!a.row_exact && a.m >= 4 && mfma_decode_takes<4>(a)) return "qmv4_mfma_kernel";
         return "qmv4_lds_kernel";
     }
+    if (short_decode_takes(a)) return "qmv4_short_kernel";
+    if (block_decode_takes(a) || decode8_takes(a) || decode3_takes(a) || decode56_takes(a) || decode2_takes(a)) return "qmv4_lds_kernel";
+    return "qmv_lds_kernel";
 }
 
 bool qmv_glu_pairs_take(const ProductArgs &a) { return glu_pairs_take(a); }

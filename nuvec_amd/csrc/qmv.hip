@@ -18,8 +18,6 @@
 #include "qmv_common.h"
 #include "wave_reduce.h"
 
-#include <cstring>
-
 namespace nvq {
 namespace {
 
@@ -1592,52 +1590,63 @@ int32_t run_general(const ProductArgs &a, hipStream_t s) {
     return NVQ_OK;
 }
 
+// The vector and decode kernels of weights stored [N, K], and which of them runs a product.
+enum class Kernel { kShort, kDot8, kMm16, kMfma, kDecode, kGeneral };
+Kernel pick_kernel(const ProductArgs &a) {
+    if (a.dtype == NVQ_F32) return Kernel::kGeneral;
+    if (short_decode_takes(a)) return Kernel::kShort;
+    if (a.mode != NVQ_AFFINE) return block_decode_takes(a) ? Kernel::kDecode : Kernel::kGeneral;
+    // A single row against 8-bit codes (groups of 32 and more hold a lane's 32 values): the decode kernel.  Against
+    // the general kernel (us): W[4096,4096] g32 6.90 -> 5.80, g64 6.68 -> 5.35; W[14336,4096] g64 15.87 ->
+    // 14.25; W[2880,2880] g32 5.99 -> 4.80; W[4096,14336] g128 15.69 -> 15.62.
+    // (3 bits, against the general kernel: W[4096,4096] g64 5.47 -> 4.01, W[14336,4096] 12.2 -> 8.2, W[2880,2880] g32 5.39 -> 3.78)
+    if (decode8_takes(a) || decode3_takes(a) || decode2_takes(a) || decode56_takes(a)) return Kernel::kDecode;
+    if (a.bits != 4 || a.exact_weights) return Kernel::kGeneral;  // (the decode kernels never materialise a weight)
+    // One row (or row-exact rows) against K = 2048 / 4096: the integer dot-product kernel (W[14336,4096]: 7.8 -> 6.8 us).
+    if (qmv_dot8_takes(a)) return Kernel::kDot8;
+    // Four rows at a time run faster on the matrix cores (measured at W[14336,4096]: 14.0 against 15.3 us);
+    // one to three rows stay on the vector kernel, whose blocks are smaller and start sooner (7.8 against
+    // 10.4 us at one row).
+    // Row-exact products stay on the vector kernel at every row count: a row's arithmetic there does not depend
+    // on the rows that share its pass.
+    if (!a.row_exact && d16_takes(a)) return Kernel::kMm16;  // 9.8 / 10.6 / 12.1 us at 2 / 4 / 8 rows of W[14336,4096] (vector and 32x32x16 kernels: 10.0 / 12.7 / 17.3)
+    return !a.row_exact && a.m >= 4 && mfma_decode_takes<4>(a) ? Kernel::kMfma : Kernel::kDecode;
+}
+
+template <typename T>
+int32_t run_decode(const ProductArgs &a, hipStream_t s) {
+    if (a.mode == NVQ_MXFP4) return run_block_decode<T, NVQ_MXFP4>(a, s);
+    if (a.mode == NVQ_MXFP8) return run_block_decode<T, NVQ_MXFP8>(a, s);
+    if (a.mode == NVQ_NVFP4) return run_block_decode<T, NVQ_NVFP4>(a, s);
+    switch (a.bits) {
+    case 8: return a.m == 1 ? run_lds4<T, 1, 1, 8, kAffine8>(a, s) : a.m == 2 ? run_lds4<T, 2, 1, 8, kAffine8>(a, s) : run_lds4<T, 4, 1, 8, kAffine8>(a, s);
+    case 6: return run_block_decode<T, kAffine6>(a, s);
+    case 5: return run_block_decode<T, kAffine5>(a, s);
+    case 3: return a.m == 1 ? run_lds4<T, 1, 1, 8, kAffine3>(a, s) : a.m == 2 ? run_lds4<T, 2, 1, 8, kAffine3>(a, s) : run_lds4<T, 4, 1, 8, kAffine3>(a, s);
+    case 2: return run_block_decode<T, kAffine2>(a, s);
+    default: return run_block_decode<T, NVQ_AFFINE>(a, s);  // more rows than four: passes of four over grid.y
+    }
+}
+
 template <typename T>
 int32_t run_typed(const ProductArgs &a, hipStream_t s) {
     if constexpr (!std::is_same<T, float>::value) {
-        if (short_decode_takes(a)) {
+        switch (pick_kernel(a)) {
+        case Kernel::kShort:
             if (a.mode == NVQ_MXFP4) return run_short<T, NVQ_MXFP4>(a, s);
             if (a.mode == NVQ_MXFP8) return run_short<T, NVQ_MXFP8>(a, s);
             if (a.mode == NVQ_NVFP4) return run_short<T, NVQ_NVFP4>(a, s);
             return run_short<T, NVQ_AFFINE>(a, s);
-        }
-        if (block_decode_takes(a)) {
-            if (a.mode == NVQ_MXFP4) return run_block_decode<T, NVQ_MXFP4>(a, s);
-            if (a.mode == NVQ_MXFP8) return run_block_decode<T, NVQ_MXFP8>(a, s);
-            return run_block_decode<T, NVQ_NVFP4>(a, s);
+        case Kernel::kDot8: return launch_qmv_dot8(a, s);
+        case Kernel::kMm16: return run_d16<T>(a, s);
+        case Kernel::kMfma: return run_mfma4<T, 4>(a, s);  // more rows: passes of four over grid.y
+        case Kernel::kDecode: return run_decode<T>(a, s);
+        case Kernel::kGeneral: break;
         }
     }
     if (a.mode == NVQ_MXFP4) return run_general<T, 4, NVQ_MXFP4>(a, s);
     if (a.mode == NVQ_MXFP8) return run_general<T, 8, NVQ_MXFP8>(a, s);
     if (a.mode == NVQ_NVFP4) return run_general<T, 4, NVQ_NVFP4>(a, s);
-    if constexpr (!std::is_same<T, float>::value) {
-        // A single row against 8-bit codes (groups of 32 and more hold a lane's 32 values): the decode kernel.  Against
-        // the general kernel below (us): W[4096,4096] g32 6.90 -> 5.80, g64 6.68 -> 5.35; W[14336,4096] g64 15.87 ->
-        // 14.25; W[2880,2880] g32 5.99 -> 4.80; W[4096,14336] g128 15.69 -> 15.62.
-        if (decode8_takes(a)) return a.m == 1 ? run_lds4<T, 1, 1, 8, kAffine8>(a, s) : a.m == 2 ? run_lds4<T, 2, 1, 8, kAffine8>(a, s) : run_lds4<T, 4, 1, 8, kAffine8>(a, s);
-        // (3 bits, against the general kernel: W[4096,4096] g64 5.47 -> 4.01, W[14336,4096] 12.2 -> 8.2, W[2880,2880] g32 5.39 -> 3.78)
-        if (decode3_takes(a)) return a.m == 1 ? run_lds4<T, 1, 1, 8, kAffine3>(a, s) : a.m == 2 ? run_lds4<T, 2, 1, 8, kAffine3>(a, s) : run_lds4<T, 4, 1, 8, kAffine3>(a, s);
-        if (decode2_takes(a)) return run_block_decode<T, kAffine2>(a, s);
-        if (decode56_takes(a)) {
-            if (a.bits == 6) return run_block_decode<T, kAffine6>(a, s);
-            return run_block_decode<T, kAffine5>(a, s);
-        }
-        if (a.bits == 4 && !a.exact_weights) {  // (the decode kernels never materialise a weight)
-            // One row (or row-exact rows) against K = 2048 / 4096: the integer dot-product kernel (W[14336,4096]: 7.8 -> 6.8 us).
-            if (qmv_dot8_takes(a)) return launch_qmv_dot8(a, s);
-            // Four rows at a time run faster on the matrix cores (measured at W[14336,4096]: 14.0 against 15.3 us);
-            // one to three rows stay on the vector kernel, whose blocks are smaller and start sooner (7.8 against
-            // 10.4 us at one row).
-            // Row-exact products stay on the vector kernel at every row count: a row's arithmetic there does not depend
-            // on the rows that share its pass.
-            if (!a.row_exact && d16_takes(a)) return run_d16<T>(a, s);  // 9.8 / 10.6 / 12.1 us at 2 / 4 / 8 rows of W[14336,4096] (vector and 32x32x16 kernels: 10.0 / 12.7 / 17.3)
-            if (!a.row_exact && a.m >= 4 && mfma_decode_takes<4>(a)) return run_mfma4<T, 4>(a, s);  // more rows: passes of four over grid.y
-            if (a.m == 1) return run_lds4<T, 1, 1, 8>(a, s);
-            if (a.m == 2) return run_lds4<T, 2, 1, 8>(a, s);
-            if (a.m == 3) return run_lds4<T, 3, 1, 8>(a, s);
-            return run_lds4<T, 4, 1, 8>(a, s);  // more rows: passes of four over grid.y
-        }
-    }
 #define NVQ_GENERIC(B) run_general<T, B, NVQ_AFFINE>(a, s)
     switch (a.bits) {
     case 1: return NVQ_GENERIC(1);
@@ -1658,18 +1667,15 @@ bool qmv_d16_takes(const ProductArgs &a) { return !a.row_exact && d16_takes(a); 
 bool qmv_block_decode_takes(const ProductArgs &a) { return block_decode_takes(a); }
 bool qmv_decode_takes_width(const ProductArgs &a) { return decode8_takes(a) || decode3_takes(a) || decode56_takes(a) || decode2_takes(a); }
 
-// Mirrors run_typed.
 const char *qmv_kernel_name(const ProductArgs &a) {
-    if (a.mode == NVQ_AFFINE && a.bits == 4 && a.dtype != NVQ_F32 && !a.exact_weights) {
-        if (short_decode_takes(a)) return "qmv4_short_kernel";
-        if (qmv_dot8_takes(a)) return "qmv4_dot8_kernel";
-        if (!a.row_exact && d16_takes(a)) return "qmv4_mm16_kernel";
-        if (!a.row_exact && a.m >= 4 && mfma_decode_takes<4>(a)) return "qmv4_mfma_kernel";
-        return "qmv4_lds_kernel";
+    switch (pick_kernel(a)) {
+    case Kernel::kShort: return "qmv4_short_kernel";
+    case Kernel::kDot8: return "qmv4_dot8_kernel";
+    case Kernel::kMm16: return "qmv4_mm16_kernel";
+    case Kernel::kMfma: return "qmv4_mfma_kernel";
+    case Kernel::kDecode: return "qmv4_lds_kernel";
+    default: return "qmv_lds_kernel";
     }
-    if (short_decode_takes(a)) return "qmv4_short_kernel";
-    if (block_decode_takes(a) || decode8_takes(a) || decode3_takes(a) || decode56_takes(a) || decode2_takes(a)) return "qmv4_lds_kernel";
-    return "qmv_lds_kernel";
 }
 
 bool qmv_glu_pairs_take(const ProductArgs &a) { return glu_pairs_take(a); }
@@ -1709,7 +1715,7 @@ bool qmv_sum_takes(const ProductArgs &a, int64_t choices) {
     if (a.rhs == nullptr || a.dtype == NVQ_F32 || a.m != 1 || a.n < 2 || a.out_rows != nullptr || a.glu != 0) return false;
     if (choices < 1 || choices > 4 || a.batch % choices != 0 || a.batch / choices > 65535) return false;
     if ((double)a.batch * (double)a.n * (double)a.k * a.bits > 8.0 * 32e6) return false;
-    return std::strcmp(qmv_kernel_name(a), "qmv4_lds_kernel") == 0;
+    return pick_kernel(a) == Kernel::kDecode;
 }
 
 int32_t launch_qmv_sum(const ProductArgs &a, const void *scores, void *out, int64_t choices, hipStream_t s) {

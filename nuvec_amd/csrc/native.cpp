@@ -205,9 +205,16 @@ nvq_qmm_desc gated_desc(const Tensor &x, int32_t code, const nvq_quant &q, int64
     return d;
 }
 
-// ops.quantized_matmul_glu, or (`several`) ops.quantized_matmul_glu_grouped or ops.quantized_matmul_glu_rows.
+// The kernel of several gated rows that nvq_quantized_matmul_glu_several_takes names, and its workspace.
+struct Several {
+    int32_t kernel = 0;
+    size_t need = 0;
+};
+
+// ops.quantized_matmul_glu, or (`several`) ops.quantized_matmul_glu_grouped or ops.quantized_matmul_glu_rows.  `asked`: what the
+// question gave for a pair of these sizes, which costs as much as a launch.
 bool product_glu(const Tensor &x, const Packed &p, const Tensor &bias, int32_t activation, float alpha, float limit, bool several,
-                 Tensor &out) {
+                 const Several *asked, Tensor &out) {
     const Place at(x);
     if (!at.usable() || x.dim() < 1 || !x.is_contiguous() || x.numel() == 0) return false;
     const int32_t code = code_of(x.scalar_type());
@@ -216,9 +223,12 @@ bool product_glu(const Tensor &x, const Packed &p, const Tensor &bias, int32_t a
     const int64_t n = p.w.size(0);
     if (n == 0 || n % 128 != 0 || !bias_fits(bias, at, x.scalar_type(), n)) return false;
     const nvq_qmm_desc d = gated_desc(x, code, p.q, n);
-    size_t need = 0;
-    const bool grouped = several && nvq_quantized_matmul_glu_grouped_takes(&d);
-    if (several && !grouped && !nvq_quantized_matmul_glu_rows_takes(&d, &need)) return false;
+    Several to;
+    if (several && asked != nullptr) to = *asked;
+    else if (several) to.kernel = nvq_quantized_matmul_glu_several_takes(&d, &to.need);
+    if (several && to.kernel == 0) return false;
+    const bool grouped = to.kernel == 1;
+    const size_t need = to.need;
     Tensor workspace, y = at.empty(with_last(x.sizes(), n / 2), x.scalar_type());
     if (need > 0) workspace = at.empty({(int64_t)need}, at::kByte);
     const int32_t rc = grouped   ? nvq_quantized_matmul_glu_grouped(&d, activation, alpha, limit, ptr(x), ptr(p.w), ptr(p.s), ptr(p.b), ptr(bias),
@@ -481,16 +491,20 @@ PyObject *py_mlp(PyObject *, PyObject *const *args, Py_ssize_t n) {
         if (!linear_fits(gate, at, type, x.size(-1)) || !linear_fits(down, at, type, gate.p.w.size(0))) return none();
         const bool several = rows > most;
         bool paired = both.p != Py_None;
+        Several asked;
         if (paired && several) {  // (what the projections' sizes say already: the pair is not read where it would be refused)
             const nvq_qmm_desc d = gated_desc(x, code_of(type), gate.p.q, 2 * gate.p.w.size(0));
-            paired = nvq_quantized_matmul_glu_grouped_takes(&d) || nvq_quantized_matmul_glu_rows_takes(&d, nullptr);
+            asked.kernel = nvq_quantized_matmul_glu_several_takes(&d, &asked.need);
+            paired = asked.kernel != 0;
         }
         if (paired) {
             const bool fits = read_linear(both.p, fused) && linear_fits(fused, at, type, x.size(-1)) && fused.p.w.size(0) == 2 * gate.p.w.size(0);
             if (!fits && !several) return none();
             if (fits) {
+                const nvq_quant &q = gate.p.q, &r = fused.p.q;
+                const bool same = q.mode == r.mode && q.group_size == r.group_size && q.bits == r.bits;
                 const bool done = unlocked([&] {
-                    return product_glu(x, fused.p, fused.bias, activation, 0.0f, 0.0f, several, hidden) && product(hidden, down.p, down.bias, Flags(), y);
+                    return product_glu(x, fused.p, fused.bias, activation, 0.0f, 0.0f, several, same ? &asked : nullptr, hidden) && product(hidden, down.p, down.bias, Flags(), y);
                 });
                 if (hidden.defined()) return wrap(done, y);
             }

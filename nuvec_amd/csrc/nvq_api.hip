@@ -630,8 +630,7 @@ static bool split_rows_bid(const ProductArgs &a, Route route, qms::Plan &plan) {
 // (0.11 and 0.08 are left).  That brings all 3000 to 0.70 of the other kernels' time, as taking every candidate does, with 32 more than
 // 5 % slower, 1.20 x at worst, where all candidates would give 132 and 1.69 x (us, the few-row kernel / here: 8 bits
 // W[8118,3328] at 4 rows 12.5 / 20.2, W[6907,3712] at 10 rows 11.6 / 17.9).
-static bool split_rows_take(const ProductArgs &a, Route route, qms::Plan &plan) {
-    if (!split_rows_bid(a, route, plan)) return false;
+static bool split_rows_ahead(const ProductArgs &a, Route route, const qms::Plan &plan) {
     double here = plan.us * (plan.mt == 1 ? (a.k < 1100 ? 0.93 : 1.02) : plan.mt == 2 && plan.qw == 1 ? (a.k < 700 ? 1.0 : a.k < 1100 ? 1.1 : 1.18) : (a.k < 1600 ? 1.02 : 1.1));
     if (plan.nt == 2) here *= plan.qw == 1 && a.bits == 8 ? 1.45 : 1.08;
     if (a.bits == 5 || a.bits == 6 || a.bits == 8) here *= 1.04;
@@ -640,6 +639,7 @@ static bool split_rows_take(const ProductArgs &a, Route route, qms::Plan &plan) 
     const double rows = a.m <= 16 ? 0.64 + 0.01 * (double)a.m : a.m <= 24 ? (exact ? 0.9 : 1.03) : (exact ? 1.03 : 1.17);
     return here < (rows + (a.k < 1600 ? 0.2 : a.k < 2600 ? 0.1 : 0.0)) * (a.bits == 2 && a.m <= 16 ? 0.85 : 1.0) * few_rows_us(a);
 }
+static bool split_rows_take(const ProductArgs &a, Route route, qms::Plan &plan) { return split_rows_bid(a, route, plan) && split_rows_ahead(a, route, plan); }
 
 // Whether the float32 matrix-core kernel runs a product of the vector kernels' route (the route keeps its name).  The estimates of both
 // are up to a tenth off at up to four rows, one pass of the vector kernel, so there it has to be ahead by that.  (250 products of 2 to 700
@@ -820,6 +820,20 @@ int32_t nvq_quantized_matmul_glu(const nvq_qmm_desc *d, int32_t activation, floa
     return launch_qmv_glu_pairs(a, (hipStream_t)stream);
 }
 
+// One of the two products that a gated pair is otherwise, and the kernels that would run it.
+struct OneOfTwo {
+    ProductArgs args;
+    Route route;
+    bool split_bid;  // split_rows_bid, with its cut
+    qms::Plan split;
+
+    OneOfTwo(const nvq_qmm_desc *d, const ProductArgs &pair) : args(pair) {
+        args.glu = 0, args.n = pair.n / 2;
+        route = pick_route(d, args);
+        split_bid = split_rows_bid(args, route, split);
+    }
+};
+
 // Whether the split-K kernel takes the gate and up products of several rows with the gated epilogue: where the two products would run on
 // kernels that hold a weight no more precisely (rounded once; block formats exactly, but for MXFP4 and MXFP8 of small scales in float16
 // beside the direct few-row kernel), and the bounds of
@@ -832,28 +846,30 @@ int32_t nvq_quantized_matmul_glu(const nvq_qmm_desc *d, int32_t activation, floa
 // and of the batched-decode kernel 4 bits at up to 48 rows beyond K = 1536 (groups of 32, W[14272,2048] at 22 rows 23.4 / 26.0; W[13760,512]
 // at 19 rows 19.0 / 11.4, W[9344,3072] at 117 rows 70.8 / 44.7) and 8 bits up to 16 rows or beyond K = 1024 (W[9536,4096] at 18 rows
 // 35.8 / 39.1; W[8960,1024] at 32 rows 19.6 / 16.6).
-static bool gated_rows_take(const nvq_qmm_desc *d, const ProductArgs &a, qms::Plan &plan) {
+static bool gated_rows_take(const ProductArgs &a, const OneOfTwo &one, qms::Plan &plan) {
     if (a.m <= 5 || a.m > 256 || !qms_plan(a, plan)) return false;  // (up to five rows an MLP's bits are those of its two products)
-    ProductArgs one = a;
-    one.glu = 0, one.n = a.n / 2;
-    const Route route = pick_route(d, one);
     const double codes = (double)a.n * (double)a.k;
-    if (route == Route::kFewRowsDirect) return a.mode != NVQ_AFFINE && (a.mode == NVQ_MXFP4 ? a.m <= 32 : a.m > 16 || codes <= 32.0e6);
-    if (route == Route::kBatchedDecode) return a.bits == 4 ? a.k <= 1536 || a.m > 48 : a.k <= 1024 && a.m > 16;
-    if ((route != Route::kFewRows && route != Route::kTiled) || (a.mode == NVQ_AFFINE && a.bits == 8 && a.m <= 16 && codes > 24.0e6)) return false;
-    qms::Plan split;
-    if (split_rows_bid(one, route, split)) return plan.us < 4.0 + 2.0 * split.us;
-    return plan.us < (route == Route::kTiled ? (a.mode == NVQ_MXFP8 ? 0.65 : 0.8) * (4.0 + 2.0 * tiled_us(one)) : 4.0 + 2.0 * few_rows_us(one));
+    if (one.route == Route::kFewRowsDirect) return a.mode != NVQ_AFFINE && (a.mode == NVQ_MXFP4 ? a.m <= 32 : a.m > 16 || codes <= 32.0e6);
+    if (one.route == Route::kBatchedDecode) return a.bits == 4 ? a.k <= 1536 || a.m > 48 : a.k <= 1024 && a.m > 16;
+    if ((one.route != Route::kFewRows && one.route != Route::kTiled) || (a.mode == NVQ_AFFINE && a.bits == 8 && a.m <= 16 && codes > 24.0e6)) return false;
+    if (one.split_bid) return plan.us < 4.0 + 2.0 * one.split.us;
+    return plan.us < (one.route == Route::kTiled ? (a.mode == NVQ_MXFP8 ? 0.65 : 0.8) * (4.0 + 2.0 * tiled_us(one.args)) : 4.0 + 2.0 * few_rows_us(one.args));
+}
+
+static bool gated_args(const nvq_qmm_desc *d, ProductArgs &a) {
+    if (check_qmm(d, "quantized_matmul") != NVQ_OK || d->m == 0 || d->n == 0 || d->k == 0 || !d->transpose || d->batch_ndim != 0 || require_device() != NVQ_OK) return false;
+    a = product_args(d, 1);
+    a.exact_weights = wants_exact_weights(d->quant.mode, d->dtype, d->n / 2, d->m);
+    a.glu = 1;
+    return true;
 }
 
 int32_t nvq_quantized_matmul_glu_rows_takes(const nvq_qmm_desc *d, size_t *workspace_bytes) {
     if (workspace_bytes != nullptr) *workspace_bytes = 0;
-    if (check_qmm(d, "quantized_matmul") != NVQ_OK || d->m == 0 || d->n == 0 || d->k == 0 || !d->transpose || d->batch_ndim != 0 || require_device() != NVQ_OK) return 0;
-    ProductArgs a = product_args(d, 1);
-    a.exact_weights = wants_exact_weights(d->quant.mode, d->dtype, d->n / 2, d->m);
-    a.glu = 1;
+    ProductArgs a;
+    if (!gated_args(d, a)) return 0;
     qms::Plan plan;
-    if (!gated_rows_take(d, a, plan)) return 0;
+    if (!gated_rows_take(a, OneOfTwo(d, a), plan)) return 0;
     if (workspace_bytes != nullptr) *workspace_bytes = qms_workspace_bytes(a, plan);
     return 1;
 }
@@ -873,7 +889,7 @@ int32_t nvq_quantized_matmul_glu_rows(const nvq_qmm_desc *d, int32_t activation,
     if (empty) return NVQ_OK;
     NVQ_TRY(check_aligned(op, "workspace", workspace));
     qms::Plan plan;
-    if (!gated_rows_take(d, a, plan)) return fail(NVQ_UNSUPPORTED, "%s: the split-K kernel does not take this product with the gated epilogue", op);
+    if (!gated_rows_take(a, OneOfTwo(d, a), plan)) return fail(NVQ_UNSUPPORTED, "%s: the split-K kernel does not take this product with the gated epilogue", op);
     return launch_qms(a, plan, workspace, (hipStream_t)stream);
 }
 
@@ -884,30 +900,47 @@ int32_t nvq_quantized_matmul_glu_rows(const nvq_qmm_desc *d, int32_t activation,
 // W[11008,4096] at 16 rows 40.6 -> 38.3).  Beside the batched-decode kernel all 68 are (0.91, 1.01 x at worst), beside the direct few-row
 // kernel MXFP4 of 128 blocks and more (19 pairs, 0.61, none slower; in bfloat16, as that kernel multiplies a group's sum by its float32 scale);
 // MXFP8 and NVFP4, up to 16 rows there, were up to 1.3 x slower.
-static bool gated_group_take(const nvq_qmm_desc *d, const ProductArgs &a, int &groups) {
+static bool gated_group_take(const ProductArgs &a, const OneOfTwo &one, const qms::Plan *rows, int &groups) {  // `rows`: gated_rows_take's, if it does
     if (a.m <= 5 || a.m > 256) return false;  // (up to five rows an MLP's bits are those of its two products)
-    const double us = gated_group_us(a, groups);
-    if (us == HUGE_VAL) return false;
-    qms::Plan split;
-    if (gated_rows_take(d, a, split)) return us < split.us * (a.m <= 16 && a.k >= 1100 ? 0.85 : a.m > 64 && a.m <= 80 && a.k < 1100 ? 0.9 : 1.0);
-    ProductArgs one = a;
-    one.glu = 0, one.n = a.n / 2;
-    const Route route = pick_route(d, one);
-    if (split_rows_take(one, route, split)) return us < 4.0 + 2.0 * split.us;
-    if (route == Route::kTiled) return us < 4.0 + 2.0 * tiled_us(one);
-    if (route == Route::kFewRows) return us < 0.85 * (4.0 + 2.0 * few_rows_us(one));
-    return route == Route::kBatchedDecode || (route == Route::kFewRowsDirect && a.mode == NVQ_MXFP4 && block_weights_exact(a.mode, a.dtype) && a.m > 32 && a.n / 128 * ((a.m + 63) / 64) >= 128);
+    double most = HUGE_VAL;
+    if (rows != nullptr) most = rows->us * (a.m <= 16 && a.k >= 1100 ? 0.85 : a.m > 64 && a.m <= 80 && a.k < 1100 ? 0.9 : 1.0);
+    else if (one.split_bid && split_rows_ahead(one.args, one.route, one.split)) most = 4.0 + 2.0 * one.split.us;
+    else if (one.route == Route::kTiled) most = 4.0 + 2.0 * tiled_us(one.args);
+    else if (one.route == Route::kFewRows) most = 0.85 * (4.0 + 2.0 * few_rows_us(one.args));
+    else if (one.route == Route::kFewRowsDirect) {
+        if (a.mode != NVQ_MXFP4 || !block_weights_exact(a.mode, a.dtype) || a.m <= 32 || a.n / 128 * ((a.m + 63) / 64) < 128) return false;
+    } else if (one.route != Route::kBatchedDecode) {
+        return false;
+    }
+    return gated_group_us(a, most, groups) < most;
+}
+
+// Which kernel takes the gate and up products of several rows with the gated epilogue; every part of the choice is looked at once.
+enum class Gated { kNone, kGroup, kRows };
+static Gated gated_choice(const nvq_qmm_desc *d, const ProductArgs &a, qms::Plan &plan, int &groups) {
+    if (a.m <= 5 || a.m > 256) return Gated::kNone;
+    const OneOfTwo one(d, a);
+    const bool rows = gated_rows_take(a, one, plan);
+    if (!d->row_exact && !d->rows && gated_group_take(a, one, rows ? &plan : nullptr, groups)) return Gated::kGroup;
+    return rows ? Gated::kRows : Gated::kNone;
 }
 
 int32_t nvq_quantized_matmul_glu_grouped_takes(const nvq_qmm_desc *d) {
-    if (check_qmm(d, "quantized_matmul") != NVQ_OK || d->m == 0 || d->n == 0 || d->k == 0 || !d->transpose || d->batch_ndim != 0 || d->row_exact ||
-        d->rows || require_device() != NVQ_OK)
-        return 0;
-    ProductArgs a = product_args(d, 1);
-    a.exact_weights = wants_exact_weights(d->quant.mode, d->dtype, d->n / 2, d->m);
-    a.glu = 1;
+    ProductArgs a;
+    qms::Plan plan;
     int groups;
-    return gated_group_take(d, a, groups);
+    return gated_args(d, a) && gated_choice(d, a, plan, groups) == Gated::kGroup;
+}
+
+int32_t nvq_quantized_matmul_glu_several_takes(const nvq_qmm_desc *d, size_t *workspace_bytes) {
+    *workspace_bytes = 0;
+    ProductArgs a;
+    qms::Plan plan;
+    int groups;
+    if (!gated_args(d, a)) return 0;
+    const Gated choice = gated_choice(d, a, plan, groups);
+    if (choice == Gated::kRows) *workspace_bytes = qms_workspace_bytes(a, plan);
+    return choice == Gated::kGroup ? 1 : choice == Gated::kRows ? 2 : 0;
 }
 
 int32_t nvq_quantized_matmul_glu_grouped(const nvq_qmm_desc *d, int32_t activation, float alpha, float limit, const void *x, const void *w,
@@ -915,10 +948,11 @@ int32_t nvq_quantized_matmul_glu_grouped(const nvq_qmm_desc *d, int32_t activati
     const char *op = "quantized_matmul";
     ProductArgs a;
     bool empty;
+    qms::Plan plan;
     int groups;
     NVQ_TRY(glu_product(op, d, activation, alpha, limit, x, w, scales, biases, bias, y, a, empty));
     if (empty) return NVQ_OK;
-    if (!gated_group_take(d, a, groups)) return fail(NVQ_UNSUPPORTED, "%s: the grouped kernel does not take this product with the gated epilogue", op);
+    if (gated_choice(d, a, plan, groups) != Gated::kGroup) return fail(NVQ_UNSUPPORTED, "%s: the grouped kernel does not take this product with the gated epilogue", op);
     return launch_gated_group(a, groups, (hipStream_t)stream);
 }
 

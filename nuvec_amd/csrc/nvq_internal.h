@@ -137,7 +137,8 @@ bool qmm_f32_faster(const ProductArgs &a, double margin);  // estimated below `m
 size_t qmm_f32_workspace_bytes(const ProductArgs &a);
 int32_t launch_qmm_f32(const ProductArgs &a, void *workspace, hipStream_t s);
 bool grouped_rows_take(const ProductArgs &a);
-double gated_group_us(const ProductArgs &a, int &groups);  // estimated duration as one group of the grouped kernel, gated; HUGE_VAL: not taken
+// Estimated duration as one group of the grouped kernel, gated; HUGE_VAL: not taken, or no less than `most`.
+double gated_group_us(const ProductArgs &a, double most, int &groups);
 int32_t launch_gated_group(ProductArgs a, int groups, hipStream_t s);
 int32_t launch_grouped_rows(ProductArgs a, hipStream_t s);
 bool qmm_dense_takes(const ProductArgs &a);

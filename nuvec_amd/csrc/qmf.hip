@@ -42,27 +42,29 @@ int32_t launch_grouped_rows(ProductArgs a, hipStream_t s) {
 // groups of a block that are estimated fastest.  A compute unit works off its blocks' windows at a rate (thr), a wavefront its own chain
 // of them no faster than at another (lat), four groups of wavefronts at a time.  Fitted to 20000 timings of 6900 pairs of 6 to 512 rows, K
 // 512 to 5120, 2560 to 14336 hidden values, twelve formats, with one, two and four groups: 12 % off on average, and the groups chosen by it
-// are 2 % above the fastest.
-double gated_group_us(const ProductArgs &a, int &groups) {
+// are 2 % above the fastest.  Every call pays for the choice (host, 8 rows of a refused [1024,512] pair 0.38 us with all nine powers and the
+// cuts walked for each question, 0.11 so): no powers are taken for a number of groups whose rates alone are beyond `most` or the best so far.
+double gated_group_us(const ProductArgs &a, double most, int &groups) {
     groups = 1;
     const bool odd = a.mode == NVQ_AFFINE && a.bits % 2 != 0;
     if ((a.dtype != NVQ_BF16 && a.dtype != NVQ_F16) || (a.mode == NVQ_AFFINE && a.bits == 1) || a.exact_weights || a.global_scale != nullptr || a.k < 128 ||
-        a.k % (odd ? 128 : 64) != 0 || a.n % 128 != 0 || a.n > 0x7FFFFFFF || a.m < 1 || a.m > 512)
+        a.k % (odd ? 128 : 64) != 0 || a.n % 128 != 0 || a.n > 0x7FFFFFFF || a.m < 1 || a.m > 256)
         return HUGE_VAL;
     const double format = a.mode == NVQ_MXFP4 ? 0.76 : a.mode == NVQ_MXFP8 ? 1.05 : a.mode == NVQ_NVFP4 ? 1.03 : a.bits == 2 ? 1.0 : a.bits == 3 ? 1.07
                           : a.bits == 4 ? 1.04 : a.bits == 5 ? 1.22 : a.bits == 6 ? 1.24 : 1.29;
     const int64_t passes = (a.m + 63) / 64, windows = (a.k + 127) / 128;
     const double tiles = (double)((a.m + 15) / 16) / (double)passes;  // of 16 rows, of a pass
     const double blocks = ceil((double)(a.n / 128 * passes) / fmax(1.0, (double)compute_units()));  // of a compute unit
-    double best = HUGE_VAL;
+    double best = most;
     for (int g = 1; g <= 4 && g <= windows; g *= 2) {
-        const double turns = (double)((windows + g - 1) / g);
+        const double turns = (double)((windows + g - 1) / g), around = 2.9 + 0.51 * (g - 1) + 2.68 * blocks;
         const double thr = blocks * g * turns * format * (0.467 + 0.119 * tiles);
-        const double lat = ceil(blocks * g / 4.0) * turns * pow(format, 1.15) * (0.52 + 0.231 * tiles);
-        const double us = 2.9 + 0.51 * (g - 1) + pow(pow(thr, 2.65) + pow(lat, 2.65), 1.0 / 2.65) + 2.68 * blocks;
+        const double lat = ceil(blocks * g / 4.0) * turns * (0.52 + 0.231 * tiles);  // times format^1.15, no less than 0.95 of it
+        if (!(around + fmax(thr, 0.95 * format * lat) < best)) continue;
+        const double us = around + pow(pow(thr, 2.65) + pow(pow(format, 1.15) * lat, 2.65), 1.0 / 2.65);
         if (us < best) best = us, groups = g;
     }
-    return best;
+    return best < most ? best : HUGE_VAL;
 }
 
 int32_t launch_gated_group(ProductArgs a, int groups, hipStream_t s) {

@@ -1,12 +1,15 @@
 """The gate and up projections of several rows as the one group of the grouped kernel, with the gated epilogue
 (`quantized_matmul_glu_grouped`), against the two products and `glu` at the edges of its tiles, windows and groups."""
+import ctypes as C
+import random
+
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 
 nv = pytest.importorskip("nuvec_amd")
-from nuvec_amd import layers, ops  # noqa: E402
+from nuvec_amd import _lib, layers, ops  # noqa: E402
 from tests.test_gpu_gated_rows import _projections  # noqa: E402
 
 
@@ -84,3 +87,23 @@ def test_float16_of_small_scales_stays_two_products():
             with pytest.raises(nv.Unsupported):
                 ops.quantized_matmul_glu_grouped(x, both, "swiglu")
             assert torch.equal(mlp(x), down(ops.glu(gate(x), up(x), "swiglu")))
+
+
+def test_both_questions_at_once():
+    """`nvq_quantized_matmul_glu_several_takes` is the two questions it stands for, over the range of each."""
+    rng, library = random.Random(4), _lib.load()
+    seen = set()
+    for _ in range(4000):
+        mode = rng.choice(["affine"] * 4 + ["MXFP4", "MXFP8", "NVFP4"])
+        quant = nv.Quant.affine(rng.choice([32, 64, 128]), rng.choice([1, 2, 3, 4, 5, 6, 8])) if mode == "affine" else nv.Quant.new(getattr(nv.QuantMode, mode))
+        d = _lib.QmmDescC()
+        d.quant, d.dtype, d.transpose = quant._c(), ops._CODE[rng.choice([torch.bfloat16, torch.float16, torch.float32])], 1
+        d.m, d.n, d.k = rng.randint(1, 300), 128 * rng.randint(1, 230), rng.choice([32, 64, 128]) * rng.randint(1, 80)
+        d.item_rows = d.m
+        need, of_rows = C.c_size_t(7), C.c_size_t(7)
+        got = library.nvq_quantized_matmul_glu_several_takes(C.byref(d), C.byref(need))
+        rows = library.nvq_quantized_matmul_glu_rows_takes(C.byref(d), C.byref(of_rows))
+        grouped = library.nvq_quantized_matmul_glu_grouped_takes(C.byref(d))
+        assert got == (1 if grouped else 2 if rows else 0) and need.value == (of_rows.value if got == 2 else 0)
+        seen.add(got)
+    assert seen == {0, 1, 2}

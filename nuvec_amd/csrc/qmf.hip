@@ -8,13 +8,11 @@ namespace nvq {
 
 // The grouped kernel: one row of x per pair, K of whole steps of 64 (windows of 128 for 1, 3 and 5 bits) or, beyond one window, whole 32
 // values (not with a global scale, whose weights the element type does not hold).  Row-exact pairs keep the vector kernels where they
-// had them, with the CPU's weights and off whole steps.  With the gated epilogue, rows as long as the scales of 128 weight rows fit the
-// 48 KB (off whole steps what x and the codes leave of 160) of a table that callers may count on.
+// had them, with the CPU's weights and off whole steps.
 static bool grouped_supported(const ProductArgs &a) {
     if (a.m != 1 || a.experts > 65535) return false;
     const bool odd = a.mode == NVQ_AFFINE && a.bits % 2 != 0, whole = a.k >= 64 && a.k % (odd ? 128 : 64) == 0;
     if (a.row_exact && (a.exact_weights || !whole)) return false;
-    if (a.glu != 0 && qmf::table_bytes(a, 128) > (whole ? 48 * 1024 : 128 * 1024 - 2048 * (size_t)a.bits)) return false;
     return whole || (a.k >= 128 && a.k % 32 == 0 && (a.mode == NVQ_AFFINE || a.global_scale == nullptr));
 }
 

@@ -209,3 +209,19 @@ def test_few_float16_pairs_of_small_scales(mode, size):
     assert torch.equal(glu.forward(x, ids), want)
     got = glu.fuse_gate_up().forward(x, ids)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("fmt,n,k", [((32, 8), 2176, 4096), ((64, 4), 2048, 8192), ((32, 2), 2304, 4128), ((32, 3), 2048, 4096), ("NVFP4", 2048, 8192)], ids=str)
+@pytest.mark.parametrize("pairs", [40, 90])
+def test_gated_pairs_of_long_rows(fmt, n, k, pairs):
+    """Rows whose groups' scales are many: the gated product is bit for bit its two products and the activation, however long they are."""
+    torch.manual_seed(k + pairs)
+    quant = nv.Quant.new(getattr(nv.QuantMode, fmt)) if isinstance(fmt, str) else nv.Quant.affine(*fmt)
+    gate, up = (nv.quantize((torch.randn(3, n // 2, k, device="cuda") * k ** -0.5).bfloat16(), quant) for _ in range(2))
+    pair = lambda a, b: None if a is None else nv.ops.pair_rows(a, b, 1)
+    both = nv.Quantized(pair(gate.weight, up.weight), pair(gate.scales, up.scales), pair(gate.biases, up.biases), quant)
+    x = torch.randn(pairs, k, device="cuda").bfloat16()
+    ids = torch.sort(torch.randint(0, 3, (pairs,), device="cuda")).values.to(torch.int32)
+    rows, offsets = torch.arange(pairs, dtype=torch.int32, device="cuda"), nv.sorted_offsets(ids, 3)
+    product = lambda q: nv.gather_qmm_grouped(x, q, rows, ids, offsets)
+    assert torch.equal(nv.ops.gather_qmm_glu(x, both, rows, ids, offsets, "swiglu"), nv.ops.glu(product(gate), product(up), "swiglu"))

@@ -437,6 +437,8 @@ NVQ_API int32_t nvq_gather_qmm_expert_bias(const nvq_gather_desc *desc, const vo
 NVQ_API int32_t nvq_gather_qmm_sum(const nvq_gather_desc *desc, const void *x, const void *w, const void *scales, const void *biases,
                                    const float *global_scales, const uint32_t *lhs, const uint32_t *rhs, const void *expert_bias,
                                    const void *scores, int32_t choices, void *out, void *stream);
+/* 1 if it takes pairs of `desc` (with operands that the launch accepts); depends on desc and choices alone. */
+NVQ_API int32_t nvq_gather_qmm_sum_takes(const nvq_gather_desc *desc, int32_t choices);
 
 /* `Mlp::forward` up to its down projection (crates/nuvec-lm/src/model.rs:2066-2074: `swiglu(gate(x), up(x))`, Gemma's
  * `geglu`) for up to four rows of x in one kernel: w, scales, biases (and bias, dtype[n] or NULL: the two

@@ -124,6 +124,7 @@ SIGNATURES = {
     "nvq_quantized_matmul_glu_several_takes": (C.c_int32, [C.POINTER(QmmDescC), C.POINTER(C.c_size_t)]),
     "nvq_quantized_matmul_glu_grouped": (C.c_int32, [C.POINTER(QmmDescC), C.c_int32, C.c_float, C.c_float] + [C.c_void_p] * 7),
     "nvq_quantized_matmul_glu_rows": (C.c_int32, [C.POINTER(QmmDescC), C.c_int32, C.c_float, C.c_float] + [C.c_void_p] * 8),
+    "nvq_gather_qmm_sum_takes": (C.c_int32, [C.POINTER(GatherDescC), C.c_int32]),
     "nvq_gather_qmm_sum": (C.c_int32, [C.POINTER(GatherDescC)] + [C.c_void_p] * 9 + [C.c_int32] + [C.c_void_p] * 2),
     "nvq_gather_qmm_glu": (C.c_int32, [C.POINTER(GatherDescC), C.c_int32, C.c_float, C.c_float] + [C.c_void_p] * 10),
     "nvq_glu": (C.c_int32, [C.POINTER(GluDescC), C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),

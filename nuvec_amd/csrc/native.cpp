@@ -382,7 +382,8 @@ bool moe(const Tensor &x, const Tensor &router, int64_t k, bool normalize, Exper
     Tensor sum = at.empty({x.size(0), x.size(1), e.down.rows}, type);
     if (!ordered) {  // (few tokens: the down products with their sum)
         const nvq_gather_desc d{e.down.p.q, code, 1, 0, 0, 1, e.down.rows, hidden, pairs, pairs, experts};
-        if (nvq_gather_qmm_sum(&d, ptr(h), ptr(e.down.p.w), ptr(e.down.p.s), ptr(e.down.p.b), nullptr, identity, chosen, ptr(e.down.bias), ptr(scores),
+        if (nvq_gather_qmm_sum_takes(&d, (int32_t)k) &&
+            nvq_gather_qmm_sum(&d, ptr(h), ptr(e.down.p.w), ptr(e.down.p.s), ptr(e.down.p.b), nullptr, identity, chosen, ptr(e.down.bias), ptr(scores),
                                (int32_t)k, sum.mutable_data_ptr(), stream) == NVQ_OK) {
             out = std::move(sum);
             return true;

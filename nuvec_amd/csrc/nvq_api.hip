@@ -1227,6 +1227,23 @@ struct GluEpilogue {  // activation < 0: no activation, only the experts' bias
     int64_t choices = 0;
 };
 
+// Whether the pairs one by one would run on the decode kernel whose sum is a kernel of its own.
+static bool summed_pairs_take(const ProductArgs &a, int64_t choices) {
+    return !a.row_exact && qmv_sum_takes(a, choices) && !takes_few_rows_direct(a) && (takes_decode(a) || !qmf_supported(a));
+}
+
+static ProductArgs gather_args(const nvq_gather_desc *d) {
+    ProductArgs a{};
+    a.mode = d->quant.mode; a.group = d->quant.group_size; a.bits = d->quant.bits; a.dtype = d->dtype;
+    a.m = d->m; a.n = d->n; a.k = d->k;
+    a.batch = d->pairs;
+    a.x_batches = d->x_batches; a.experts = d->experts;
+    a.row_exact = d->row_exact != 0;
+    a.float32_weights = d->float32_weights != 0;
+    a.exact_weights = wants_exact_weights(d->quant.mode, d->dtype, d->n, a.row_exact ? 1 : d->m);
+    return a;
+}
+
 static int32_t gather_qmm_any(const nvq_gather_desc *d, const void *x, const void *w, const void *scales, const void *biases,
                               const float *global_scale, const uint32_t *lhs, const uint32_t *rhs, const int32_t *offsets,
                               const uint32_t *out_rows, void *y, void *workspace, void *stream, const GluEpilogue *glu = nullptr) {
@@ -1276,18 +1293,11 @@ static int32_t gather_qmm_any(const nvq_gather_desc *d, const void *x, const voi
     if (d->k == 0) {
         return launch_fill_zero(y, d->pairs * d->m * d->n * dtype_size(d->dtype), (hipStream_t)stream);
     }
-    ProductArgs a{};
+    ProductArgs a = gather_args(d);
     a.x = x; a.w = w; a.scales = scales; a.biases = biases; a.y = y;
-    a.mode = d->quant.mode; a.group = d->quant.group_size; a.bits = d->quant.bits; a.dtype = d->dtype;
-    a.m = d->m; a.n = d->n; a.k = d->k;
-    a.batch = d->pairs;
     a.lhs = lhs; a.rhs = rhs;
-    a.x_batches = d->x_batches; a.experts = d->experts;
     a.global_scale = global_scale;
     a.out_rows = out_rows;
-    a.row_exact = d->row_exact != 0;
-    a.float32_weights = d->float32_weights != 0;
-    a.exact_weights = wants_exact_weights(d->quant.mode, d->dtype, d->n, a.row_exact ? 1 : d->m);
     if (!d->transpose) {
         // Weights stored [K, N]: rows sorted by expert as groups on the matrix-core kernel (each expert's weights read once
         // per tile of its rows; the reference's grouped kernel of the block formats, gpu.rs:6786-6812), else one product
@@ -1327,14 +1337,27 @@ static int32_t gather_qmm_any(const nvq_gather_desc *d, const void *x, const voi
     }
     // Row-exact: every pair on the vector kernels, so that a pair has the bits of its one-row product whether the
     // gather is sorted or not and however many pairs it holds (the few-row contract of gpu.rs:7325-7340).
-    const bool direct = !a.row_exact && takes_few_rows_direct(a), few = !a.row_exact && !takes_decode(a) && qmf_supported(a);
     if (choices > 0) {
-        if (direct || few || a.row_exact) return fail(NVQ_UNSUPPORTED, "gather_qmm: the decode kernel does not take these pairs with their weighted sum");
+        if (!summed_pairs_take(a, choices)) return fail(NVQ_UNSUPPORTED, "gather_qmm: the decode kernel does not take these pairs with their weighted sum");
         return launch_qmv_sum(a, scores, y, choices, (hipStream_t)stream);
     }
-    if (direct) return launch_qmd(a, (hipStream_t)stream);
-    if (few) return launch_qmf(a, (hipStream_t)stream);
+    if (!a.row_exact && takes_few_rows_direct(a)) return launch_qmd(a, (hipStream_t)stream);
+    if (!a.row_exact && !takes_decode(a) && qmf_supported(a)) return launch_qmf(a, (hipStream_t)stream);
     return launch_qmv(a, (hipStream_t)stream);
+}
+
+static bool gather_desc_holds(const nvq_gather_desc *d) {
+    return d != nullptr && check_quant(&d->quant, "gather_qmm") == NVQ_OK && check_float("gather_qmm", d->dtype) == NVQ_OK &&
+           check_product_dims("gather_qmm", d->quant, d->transpose, d->m, d->n, d->k) == NVQ_OK && d->transpose && d->n > 0 && d->k > 0 && d->pairs > 0;
+}
+
+int32_t nvq_gather_qmm_sum_takes(const nvq_gather_desc *d, int32_t choices) {
+    if (!gather_desc_holds(d) || d->m != 1 || choices < 1 || d->pairs % choices != 0 || require_device() != NVQ_OK) return 0;
+    ProductArgs a = gather_args(d);
+    a.x = a.w = a.scales = a.biases = reinterpret_cast<const void *>(uintptr_t{256});  // operands aligned as hipMalloc aligns them
+    const uint32_t pairs = 0;
+    a.lhs = a.rhs = &pairs;  // (asked for, not read)
+    return summed_pairs_take(a, choices);
 }
 
 int32_t nvq_gather_qmm(const nvq_gather_desc *d, const void *x, const void *w, const void *scales, const void *biases,

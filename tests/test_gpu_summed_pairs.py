@@ -54,3 +54,18 @@ def test_what_the_two_kernels_keep():
         ids = torch.arange(choices, device="cuda", dtype=torch.int32)
         x, scores, out = torch.randn(choices, k, device="cuda").to(dtype), torch.rand(1, choices, device="cuda").to(dtype), torch.empty(1, n, device="cuda", dtype=dtype)
         assert call(q, x, ids, ids, None, scores, out, choices, choices) == _lib.UNSUPPORTED
+
+
+def test_the_question_answers_as_the_call():
+    """`nvq_gather_qmm_sum_takes`, by which a block asks before it launches."""
+    torch.manual_seed(2)
+    for quant, n, k, tokens, choices, dtype in (("MXFP4", 2880, 2880, 1, 4, torch.bfloat16), ("MXFP4", 2880, 2880, 1, 5, torch.bfloat16), ("NVFP4", 1024, 1024, 2, 2, torch.float16),
+                                                ((64, 4), 1024, 2880, 3, 4, torch.bfloat16), ((64, 4), 1024, 2048, 1, 2, torch.bfloat16), ((64, 4), 512, 2880, 1, 2, torch.bfloat16),
+                                                ((32, 8), 1030, 352, 1, 1, torch.float16), ((64, 6), 8192, 4096, 8, 4, torch.bfloat16), ((64, 4), 1024, 2880, 1, 2, torch.float32)):
+        kind = nv.Quant.affine(*quant) if isinstance(quant, tuple) else nv.Quant.new(getattr(nv.QuantMode, quant))
+        q, pairs = nv.quantize(torch.randn(5, n, k, device="cuda").to(dtype), kind), tokens * choices
+        ids = torch.arange(pairs, device="cuda", dtype=torch.int32)
+        x, scores, out = torch.randn(pairs, k, device="cuda").to(dtype), torch.rand(tokens, choices, device="cuda").to(dtype), torch.empty(tokens, n, device="cuda", dtype=dtype)
+        d = _lib.GatherDescC(q.quant._c(), ops._CODE[dtype], 1, 0, 0, 1, n, k, pairs, pairs, 5)
+        rc = call(q, x, ids, ids % 5, None, scores, out, pairs, pairs)
+        assert rc in (0, _lib.UNSUPPORTED) and _lib.load().nvq_gather_qmm_sum_takes(C.byref(d), choices) == (rc == 0), (quant, n, k, choices)

@@ -189,9 +189,14 @@ NVQ_API int32_t nvq_gather_grouped(int64_t rows, int64_t experts, int32_t row_ex
 
 /* 1 if the pairs of `tokens` tokens with `choices` experts each run faster ordered by expert, every expert's weights read once, than one
  * by one: from 64 pairs on as in the reference (crates/nuvec-lm/src/model.rs:2189-2192), fewer where the estimate says so and the weights
- * are held no less precisely (not MXFP4 and MXFP8 in float16, which rounds those of small scales).  `values`: of an expert's three projections; `scaled`: with a global scale. */
+ * are held no less precisely (not MXFP4 and MXFP8 in float16, which rounds those of small scales).  `values`: of an expert's three projections; `scaled`: with a global scale.
+ * Below 64 pairs the caller asks as well whether the grouped kernel takes the projections (nvq_gather_sorted_takes). */
 NVQ_API int32_t nvq_moe_ordered(const nvq_quant *quant, int32_t dtype, int64_t tokens, int32_t choices, int64_t experts, int64_t values,
                                 int32_t scaled);
+
+/* 1 if the pairs of `desc`, sorted by expert and given with their offsets, run on the grouped kernel (without a global scale); 0: one by one,
+ * as without offsets, or `desc` is not a product. */
+NVQ_API int32_t nvq_gather_sorted_takes(const nvq_gather_desc *desc);
 
 /* GpuEval::supports for Primitive::QuantizedMatmul (gpu.rs:1665): 1 if nvq_quantized_matmul
  * has a kernel for `desc`, else 0 (the caller then runs its CPU path, eval.rs:738-748). */

@@ -86,6 +86,7 @@ SIGNATURES = {
     "nvq_quant_check": (C.c_int32, [C.POINTER(QuantC), C.c_char_p]),
     "nvq_gather_grouped": (C.c_int32, [C.c_int64, C.c_int64, C.c_int32]),
     "nvq_moe_ordered": (C.c_int32, [C.POINTER(QuantC), C.c_int32, C.c_int64, C.c_int32, C.c_int64, C.c_int64, C.c_int32]),
+    "nvq_gather_sorted_takes": (C.c_int32, [C.POINTER(GatherDescC)]),
     "nvq_quantized_matmul_supported": (C.c_int32, [C.POINTER(QmmDescC)]),
     "nvq_quantize": (C.c_int32, [C.POINTER(QuantC), C.c_int32, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p,
                                  C.c_void_p, C.c_void_p, C.c_void_p]),

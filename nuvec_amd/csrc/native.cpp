@@ -334,6 +334,13 @@ bool hidden_states(const Place &at, const Tensor &x, int64_t x_rows, Experts &e,
     return true;
 }
 
+// ops.moe_ordered.
+bool ahead_ordered(const Projection &w, int32_t code, int64_t tokens, int64_t choices, int64_t experts, int64_t values) {
+    if (tokens * choices >= 64) return true;
+    const nvq_gather_desc d{w.p.q, code, 1, 0, 1, 1, w.rows, w.columns, tokens * choices, tokens, experts};
+    return nvq_moe_ordered(&w.p.q, code, tokens, (int32_t)choices, experts, values, 0) && nvq_gather_sorted_takes(&d);
+}
+
 // layers.MoeMlp.forward.
 bool moe(const Tensor &x, const Tensor &router, int64_t k, bool normalize, Experts &e, Tensor &out) {
     const Place at(x);
@@ -357,8 +364,8 @@ bool moe(const Tensor &x, const Tensor &router, int64_t k, bool normalize, Exper
     void *stream = at.stream();
     // choices, tokens and numbers of the pairs; for ordered pairs the order, its inverse, sorted experts and tokens, the offsets
     const int64_t values = 3 * hidden * dims;
-    const bool ordered = nvq_moe_ordered(&e.up.p.q, code, rows, (int32_t)k, experts, values, 0) &&
-                         nvq_moe_ordered(&e.down.p.q, code, rows, (int32_t)k, experts, values, 0);
+    const bool ordered = ahead_ordered(e.up, code, rows, k, experts, values) && ahead_ordered(e.gate, code, rows, k, experts, values) &&
+                         ahead_ordered(e.down, code, rows, k, experts, values);
     Tensor index = at.empty({pairs * (ordered ? 7 : 3) + (ordered ? experts : 0)}, at::kInt), scores = at.empty({rows, k}, type);
     uint32_t *chosen = (uint32_t *)index.mutable_data_ptr(), *tokens = chosen + pairs, *identity = tokens + pairs;
     if (nvq_moe_router(code, ptr(x), ptr(router), rows, (int32_t)dims, (int32_t)experts, (int32_t)k, normalize, chosen, scores.mutable_data_ptr(),

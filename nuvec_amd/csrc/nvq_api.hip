@@ -444,6 +444,7 @@ static bool block_weights_exact(int32_t mode, int32_t dtype) { return dtype != N
 // 273 blocks of block formats, 53 ordered, none slower, all in 0.92 of the time (always the faster side 0.89); 366 of affine codes of 2 to 6
 // and 8 bits, which the grouped kernel holds in terms there, 42 ordered, one slower (1.05 x), all in 0.95 (0.89).  5 tokens x 8 of 8 MXFP4
 // experts [2368,2208] 105 -> 55 us, 24 x 2 of 16 MXFP8 [2880,2880] 257 -> 118, 12 x 4 of 8 [2624,1088] of 4 bits 112 -> 77.
+// That holds for products that the grouped kernel takes (nvq_gather_sorted_takes): others run one by one in either order.
 int32_t nvq_moe_ordered(const nvq_quant *quant, int32_t dtype, int64_t tokens, int32_t choices, int64_t experts, int64_t values, int32_t scaled) {
     const double pairs = (double)tokens * (double)choices;
     if (pairs >= 64.0) return 1;
@@ -1349,6 +1350,14 @@ static int32_t gather_qmm_any(const nvq_gather_desc *d, const void *x, const voi
 static bool gather_desc_holds(const nvq_gather_desc *d) {
     return d != nullptr && check_quant(&d->quant, "gather_qmm") == NVQ_OK && check_float("gather_qmm", d->dtype) == NVQ_OK &&
            check_product_dims("gather_qmm", d->quant, d->transpose, d->m, d->n, d->k) == NVQ_OK && d->transpose && d->n > 0 && d->k > 0 && d->pairs > 0;
+}
+
+int32_t nvq_gather_sorted_takes(const nvq_gather_desc *d) {
+    if (!gather_desc_holds(d)) return 0;
+    ProductArgs a = gather_args(d);
+    const int32_t offsets = 0;
+    a.offsets = &offsets;  // (asked for, not read)
+    return qmf_supported(a);
 }
 
 int32_t nvq_gather_qmm_sum_takes(const nvq_gather_desc *d, int32_t choices) {

@@ -255,8 +255,9 @@ class SwitchGlu:
         b, l, d = x.shape
         k = indices.shape[2]
         experts = self.up_proj.weight.shape[0]
-        if not all(ops.moe_ordered(p.quantized(), x.dtype, b * l, k, experts, 3 * self.up_proj.weight.shape[1] * d)
-                   for p in (self.up_proj, self.down_proj)):  # model.rs:2189-2192
+        width = self.up_proj.weight.shape[1]
+        if not all(ops.moe_ordered(p.quantized(), x.dtype, b * l, k, experts, 3 * width * d, columns)
+                   for p, columns in ((self.up_proj, d), (self.gate_proj, d), (self.down_proj, width))):  # model.rs:2189-2192
             xe = x.reshape(b, l, 1, 1, d)
             hidden = None
             if self.gate_up_proj is not None and self.gate_up_paired:

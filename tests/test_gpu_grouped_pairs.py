@@ -225,3 +225,42 @@ def test_gated_pairs_of_long_rows(fmt, n, k, pairs):
     rows, offsets = torch.arange(pairs, dtype=torch.int32, device="cuda"), nv.sorted_offsets(ids, 3)
     product = lambda q: nv.gather_qmm_grouped(x, q, rows, ids, offsets)
     assert torch.equal(nv.ops.gather_qmm_glu(x, both, rows, ids, offsets, "swiglu"), nv.ops.glu(product(gate), product(up), "swiglu"))
+
+
+@pytest.mark.parametrize("quant,dims,hidden,taken", [("NVFP4", 2896, 2880, False), ("NVFP4", 2880, 2864, False), ("NVFP4", 2880, 2848, True), ("4 bits", 4096, 2048, True)])
+def test_few_pairs_are_ordered_for_the_grouped_kernel_alone(quant, dims, hidden, taken, monkeypatch):
+    """Rows that it does not take (NVFP4 of half a block of 32) run one by one in either order: without the order."""
+    torch.manual_seed(hidden)
+    quant, count = QUANTS[quant], 8
+
+    def projection(n, k):
+        q = nv.quantize((torch.randn(count, n, k, device="cuda") * 0.02).bfloat16(), quant)
+        return layers.SwitchProjection(q.weight, q.scales, q.biases, None, q.quant)
+    glu = layers.SwitchGlu(projection(hidden, dims), projection(hidden, dims), projection(dims, hidden))
+    x = torch.randn(1, 5, dims, device="cuda").bfloat16()
+    ids = torch.stack([torch.randperm(count, device="cuda") for _ in range(5)]).to(torch.int32).reshape(1, 5, 8)
+    ordered = []
+    order = nv.ops.moe_order
+    monkeypatch.setattr(nv.ops, "moe_order", lambda *args: ordered.append(1) or order(*args))
+    glu.forward(x, ids)
+    assert bool(ordered) == taken
+    for p, k in ((glu.up_proj, dims), (glu.gate_proj, dims), (glu.down_proj, hidden)):
+        assert nv.ops.moe_ordered(p.quantized(), x.dtype, 5, 8, count, 3 * dims * hidden, k) == (k % 32 == 0)
+
+
+def test_few_pairs_are_ordered_where_all_three_projections_gain():
+    """A gate whose weights the ordered kernel would hold less precisely keeps the block's pairs one by one."""
+    torch.manual_seed(5)
+    count, dims, hidden = 8, 1088, 2368
+
+    def projection(n, k, quant, size):
+        q = nv.quantize(torch.randn(count, n, k, device="cuda") * size, quant)
+        parts = (q.scales.half(), q.biases.half()) if q.biases is not None else (q.scales, None)
+        return layers.SwitchProjection(q.weight, *parts, None, q.quant)
+    affine = nv.Quant.affine(64, 4)
+    glu = layers.SwitchGlu(projection(hidden, dims, nv.Quant.new(nv.QuantMode.MXFP8), 1e-4), projection(hidden, dims, affine, 0.05), projection(dims, hidden, affine, 0.05))
+    x = (torch.randn(1, 5, dims, device="cuda") * 30).half()
+    ids = torch.stack([torch.randperm(count, device="cuda") for _ in range(5)]).to(torch.int32).reshape(1, 5, 8)
+    xe = x.reshape(1, 5, 1, 1, dims)
+    gate, up = (p.forward(xe, ids, add_bias=False) for p in (glu.gate_proj, glu.up_proj))
+    assert torch.equal(glu.forward(x, ids), glu.down_proj.forward(glu.gated(gate, up, ids), ids).squeeze(-2))

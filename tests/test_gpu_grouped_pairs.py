@@ -264,3 +264,32 @@ def test_few_pairs_are_ordered_where_all_three_projections_gain():
     xe = x.reshape(1, 5, 1, 1, dims)
     gate, up = (p.forward(xe, ids, add_bias=False) for p in (glu.gate_proj, glu.up_proj))
     assert torch.equal(glu.forward(x, ids), glu.down_proj.forward(glu.gated(gate, up, ids), ids).squeeze(-2))
+
+
+# The first term alone, or two of three, are far from this: rows of x that sum to nothing leave nothing of the biases but what their rounding
+# to the terms lost (4 bits: 3 % of these sums for one term of bfloat16, 0.4 % of float16; all codes within 2^-12 beside a bias of 0.71, 2 % for two).
+@pytest.mark.parametrize("fmt", [(64, 2), (64, 4), (128, 5), (32, 8)], ids=str)
+@pytest.mark.parametrize("dtype,n,k,wide", [(torch.bfloat16, 1100, 1024, False), (torch.float16, 1152, 1664, False), (torch.bfloat16, 1152, 1664, True), (torch.bfloat16, 1030, 512, True)])
+def test_few_pairs_hold_every_term_of_their_weights(fmt, dtype, n, k, wide):
+    """Every output within its own rounding and float32 sums of float64's product of the float32 weights; `wide`: scales and biases so far
+    apart that a weight takes three terms."""
+    torch.manual_seed(n + fmt[1])
+    q = nv.quantize(torch.randn(2, n, k, device="cuda") * 0.02 + 0.3, nv.Quant.affine(*fmt))
+    scales, biases = q.scales.to(dtype), q.biases.to(dtype)
+    if wide:
+        scales, biases = torch.full_like(scales, 0.7 * 2.0 ** -(12 + fmt[1])), torch.full_like(biases, 0.71)
+    q = nv.Quantized(q.weight, scales, biases, q.quant)
+    x = torch.randn(40, k // 2, device="cuda").to(dtype)
+    x = torch.stack([x, -x], dim=-1).reshape(40, k)
+    ids = torch.tensor([0] * 17 + [1] * 23, dtype=torch.int32, device="cuda")
+    got = nv.gather_qmm_grouped(x, q, torch.arange(40, dtype=torch.int32, device="cuda"), ids, nv.sorted_offsets(ids, 2)).double().cpu()
+    weights = torch.stack([unrounded(nv.Quantized(q.weight[e], q.scales[e], q.biases[e], q.quant)) for e in range(2)]).float().double().cpu()
+    for row in range(40):
+        w = weights[int(ids[row])]
+        want = w @ x[row].double().cpu()
+        # half a unit of the output; float32 sums: K additions (in whatever order) each within 2^-24 of a partial sum, which holds some eighth of a window's
+        # 128 products beside the sum itself (neighbours cancel): at random, sqrt(K) of them, five deviations
+        window = (w * x[row].double().cpu()).abs().unfold(1, 128, 128).sum(-1).amax(-1)
+        unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+        bound = unit * want.abs() + 5 * k ** 0.5 * 2.0 ** -24 * (window / 8 + want.abs())
+        assert ((got[row] - want).abs() <= bound).all(), row

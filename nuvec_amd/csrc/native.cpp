@@ -334,11 +334,21 @@ bool hidden_states(const Place &at, const Tensor &x, int64_t x_rows, Experts &e,
     return true;
 }
 
-// ops.moe_ordered.
-bool ahead_ordered(const Projection &w, int32_t code, int64_t tokens, int64_t choices, int64_t experts, int64_t values) {
+// layers.SwitchGlu._ordered.
+bool pairs_ordered(const Experts &e, int32_t code, int64_t tokens, int64_t choices, int64_t experts) {
     if (tokens * choices >= 64) return true;
-    const nvq_gather_desc d{w.p.q, code, 1, 0, 1, 1, w.rows, w.columns, tokens * choices, tokens, experts};
-    return nvq_moe_ordered(&w.p.q, code, tokens, (int32_t)choices, experts, values, 0) && nvq_gather_sorted_takes(&d);
+    const int64_t size = e.up.rows * e.up.columns;
+    auto rule = [&](const Projection &w, int64_t values) { return nvq_moe_ordered(&w.p.q, code, tokens, (int32_t)choices, experts, values, 0) != 0; };
+    if (!rule(e.up, 3 * size)) return false;
+    const Projection *taken[3];
+    int count = 0;
+    for (const Projection *w : {&e.gate, &e.up, &e.down}) {
+        const nvq_gather_desc d{w->p.q, code, 1, 0, 1, 1, w->rows, w->columns, tokens * choices, tokens * choices, experts};
+        if (nvq_gather_sorted_takes(&d)) taken[count++] = w;
+    }
+    for (int i = 0; i < count; i++)
+        if (!rule(*taken[i], count * size)) return false;
+    return count > 0;
 }
 
 // layers.MoeMlp.forward.
@@ -363,9 +373,7 @@ bool moe(const Tensor &x, const Tensor &router, int64_t k, bool normalize, Exper
     const int64_t pairs = rows * k;
     void *stream = at.stream();
     // choices, tokens and numbers of the pairs; for ordered pairs the order, its inverse, sorted experts and tokens, the offsets
-    const int64_t values = 3 * hidden * dims;
-    const bool ordered = ahead_ordered(e.up, code, rows, k, experts, values) && ahead_ordered(e.gate, code, rows, k, experts, values) &&
-                         ahead_ordered(e.down, code, rows, k, experts, values);
+    const bool ordered = pairs_ordered(e, code, rows, k, experts);
     Tensor index = at.empty({pairs * (ordered ? 7 : 3) + (ordered ? experts : 0)}, at::kInt), scores = at.empty({rows, k}, type);
     uint32_t *chosen = (uint32_t *)index.mutable_data_ptr(), *tokens = chosen + pairs, *identity = tokens + pairs;
     if (nvq_moe_router(code, ptr(x), ptr(router), rows, (int32_t)dims, (int32_t)experts, (int32_t)k, normalize, chosen, scores.mutable_data_ptr(),

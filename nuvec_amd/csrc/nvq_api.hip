@@ -444,7 +444,8 @@ static bool block_weights_exact(int32_t mode, int32_t dtype) { return dtype != N
 // 273 blocks of block formats, 53 ordered, none slower, all in 0.92 of the time (always the faster side 0.89); 366 of affine codes of 2 to 6
 // and 8 bits, which the grouped kernel holds in terms there, 42 ordered, one slower (1.05 x), all in 0.95 (0.89).  5 tokens x 8 of 8 MXFP4
 // experts [2368,2208] 105 -> 55 us, 24 x 2 of 16 MXFP8 [2880,2880] 257 -> 118, 12 x 4 of 8 [2624,1088] of 4 bits 112 -> 77.
-// That holds for products that the grouped kernel takes (nvq_gather_sorted_takes): others run one by one in either order.
+// `values` are those that the grouped kernel takes (nvq_gather_sorted_takes): others run one by one in either order (40 pairs of 8 NVFP4
+// experts in us, one by one and ordered: [2864,2880], whose down products it does not take, 322 and 242; [2880,2896], the other two, 457 and 424).
 int32_t nvq_moe_ordered(const nvq_quant *quant, int32_t dtype, int64_t tokens, int32_t choices, int64_t experts, int64_t values, int32_t scaled) {
     const double pairs = (double)tokens * (double)choices;
     if (pairs >= 64.0) return 1;

@@ -247,6 +247,19 @@ class SwitchGlu:
                                              cat(g.bias, u.bias), g.quant)
         return self
 
+    def _ordered(self, dtype: torch.dtype, tokens: int, choices: int, dims: int) -> bool:
+        """Whether `ops.moe_ordered` has the pairs ordered, asked of each projection that the grouped kernel takes and with the weights
+        of those (the others run pair by pair in either order)."""
+        if tokens * choices >= 64:
+            return True
+        experts, hidden = self.up_proj.weight.shape[:2]
+        size = hidden * dims
+        rule = lambda p, values: ops.moe_ordered(p.quantized(), dtype, tokens, choices, experts, values)
+        if not rule(self.up_proj, 3 * size):
+            return False
+        taken = [p for p in (self.gate_proj, self.up_proj, self.down_proj) if ops.gather_sorted_takes(p.quantized(), dtype, tokens * choices)]
+        return len(taken) > 0 and all(rule(p, len(taken) * size) for p in taken)
+
     def forward(self, x: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
         """`x` `[B, L, D]` through each token's experts `indices` `[B, L, k]`: `[B, L, k, D]`.  With 64 pairs or
         more (fewer where `ops.moe_ordered` finds it faster) they are ordered by expert
@@ -254,10 +267,7 @@ class SwitchGlu:
         each row at its pair's place (`out_rows`), so the inverse permutation of model.rs:2210 is never run."""
         b, l, d = x.shape
         k = indices.shape[2]
-        experts = self.up_proj.weight.shape[0]
-        width = self.up_proj.weight.shape[1]
-        if not all(ops.moe_ordered(p.quantized(), x.dtype, b * l, k, experts, 3 * width * d, columns)
-                   for p, columns in ((self.up_proj, d), (self.gate_proj, d), (self.down_proj, width))):  # model.rs:2189-2192
+        if not self._ordered(x.dtype, b * l, k, d):  # model.rs:2189-2192
             xe = x.reshape(b, l, 1, 1, d)
             hidden = None
             if self.gate_up_proj is not None and self.gate_up_paired:
@@ -281,7 +291,7 @@ class SwitchGlu:
             else:
                 up, gate = self.up_proj.forward(xe, indices, add_bias=False), self.gate_proj.forward(xe, indices, add_bias=False)
             return self.down_proj.forward(self.gated(gate, up, indices), indices).squeeze(-2)
-        order, restore, sorted_ids, offsets = ops.moe_order(indices, experts)
+        order, restore, sorted_ids, offsets = ops.moe_order(indices, self.up_proj.weight.shape[0])
         tokens = torch.div(order, k, rounding_mode="floor").to(torch.int32)  # pair t*k + j belongs to token t
         xt = x.reshape(b * l, d)
         hidden = None

@@ -593,18 +593,21 @@ def sorted_offsets(rhs: torch.Tensor, groups: int) -> torch.Tensor:
     return out
 
 
-def moe_ordered(q: Quantized, dtype: torch.dtype, tokens: int, choices: int, experts: int, values: int, columns: Optional[int] = None) -> bool:
+def moe_ordered(q: Quantized, dtype: torch.dtype, tokens: int, choices: int, experts: int, values: int) -> bool:
     """Whether the pairs of `tokens` tokens with `choices` of `experts` each, `values` weights an expert packed as `q`, run faster ordered
-    by expert (`moe_order`) than one by one: from 64 pairs on (model.rs:2189-2192), fewer where the estimate says so, and with `columns`
-    (the values of a row of `q`) only where the grouped kernel takes such rows."""
-    pairs = tokens * choices
-    if pairs >= 64 or dtype not in _CODE:
-        return pairs >= 64
-    library, quant = _lib.load(), q.quant._c()
-    if not library.nvq_moe_ordered(C.byref(quant), _CODE[dtype], tokens, choices, experts, values, int(q.global_scale is not None)):
+    by expert (`moe_order`) than one by one: from 64 pairs on (model.rs:2189-2192), fewer where the estimate says so."""
+    if dtype not in _CODE:
+        return tokens * choices >= 64
+    return bool(_lib.load().nvq_moe_ordered(C.byref(q.quant._c()), _CODE[dtype], tokens, choices, experts, values, int(q.global_scale is not None)))
+
+
+def gather_sorted_takes(q: Quantized, dtype: torch.dtype, pairs: int) -> bool:
+    """Whether `pairs` rows sorted by expert run on the grouped kernel against `q` `[E, N, ...]` (else one by one, as unsorted ones do)."""
+    experts, n, words = q.weight.shape
+    if dtype not in _CODE or q.global_scale is not None:
         return False
-    d = _lib.GatherDescC(quant, _CODE[dtype], 1, 0, 1, 1, 0 if q.weight is None else q.weight.shape[-2], columns or 0, pairs, tokens, experts)
-    return columns is None or bool(library.nvq_gather_sorted_takes(C.byref(d)))
+    d = _lib.GatherDescC(q.quant._c(), _CODE[dtype], 1, 0, 1, 1, n, words * 32 // q.quant.bits, pairs, pairs, experts)
+    return bool(_lib.load().nvq_gather_sorted_takes(C.byref(d)))
 
 
 def moe_order(expert_ids: torch.Tensor, experts: int):

@@ -227,9 +227,9 @@ def test_gated_pairs_of_long_rows(fmt, n, k, pairs):
     assert torch.equal(nv.ops.gather_qmm_glu(x, both, rows, ids, offsets, "swiglu"), nv.ops.glu(product(gate), product(up), "swiglu"))
 
 
-@pytest.mark.parametrize("quant,dims,hidden,taken", [("NVFP4", 2896, 2880, False), ("NVFP4", 2880, 2864, False), ("NVFP4", 2880, 2848, True), ("4 bits", 4096, 2048, True)])
+@pytest.mark.parametrize("quant,dims,hidden,taken", [("NVFP4", 2896, 2864, False), ("NVFP4", 2896, 2880, True), ("NVFP4", 2880, 2864, True), ("NVFP4", 2880, 2848, True), ("4 bits", 4096, 2048, True)])
 def test_few_pairs_are_ordered_for_the_grouped_kernel_alone(quant, dims, hidden, taken, monkeypatch):
-    """Rows that it does not take (NVFP4 of half a block of 32) run one by one in either order: without the order."""
+    """Rows that it does not take (NVFP4 of half a block of 32) run one by one in either order: without the order where no projection gains."""
     torch.manual_seed(hidden)
     quant, count = QUANTS[quant], 8
 
@@ -245,7 +245,7 @@ def test_few_pairs_are_ordered_for_the_grouped_kernel_alone(quant, dims, hidden,
     glu.forward(x, ids)
     assert bool(ordered) == taken
     for p, k in ((glu.up_proj, dims), (glu.gate_proj, dims), (glu.down_proj, hidden)):
-        assert nv.ops.moe_ordered(p.quantized(), x.dtype, 5, 8, count, 3 * dims * hidden, k) == (k % 32 == 0)
+        assert nv.ops.gather_sorted_takes(p.quantized(), x.dtype, 40) == (k % 32 == 0)
 
 
 def test_few_pairs_are_ordered_where_all_three_projections_gain():
@@ -267,29 +267,29 @@ def test_few_pairs_are_ordered_where_all_three_projections_gain():
 
 
 # The first term alone, or two of three, are far from this: rows of x that sum to nothing leave nothing of the biases but what their rounding
-# to the terms lost (4 bits: 3 % of these sums for one term of bfloat16, 0.4 % of float16; all codes within 2^-12 beside a bias of 0.71, 2 % for two).
-@pytest.mark.parametrize("fmt", [(64, 2), (64, 4), (128, 5), (32, 8)], ids=str)
-@pytest.mark.parametrize("dtype,n,k,wide", [(torch.bfloat16, 1100, 1024, False), (torch.float16, 1152, 1664, False), (torch.bfloat16, 1152, 1664, True), (torch.bfloat16, 1030, 512, True)])
+# to the terms lost (a weight of 0.3 to one term, a hundred times the bound and more).  `wide`: 8-bit codes of 248 to 255 beside a bias
+# that a term holds, their sum with it within half a unit of that term: sixteen bits are left for the others (two terms: nine times the bound).
+@pytest.mark.parametrize("fmt,dtype,n,k,wide", [((64, 2), torch.bfloat16, 1100, 1024, False), ((64, 4), torch.float16, 1152, 1664, False), ((128, 5), torch.bfloat16, 1030, 512, False),
+                                                ((32, 8), torch.float16, 1100, 1024, False), ((32, 8), torch.bfloat16, 1152, 1664, True), ((32, 8), torch.bfloat16, 1030, 512, True)], ids=str)
 def test_few_pairs_hold_every_term_of_their_weights(fmt, dtype, n, k, wide):
-    """Every output within its own rounding and float32 sums of float64's product of the float32 weights; `wide`: scales and biases so far
-    apart that a weight takes three terms."""
+    """Every output within its own rounding and float32 sums of float64's product of the float32 weights."""
     torch.manual_seed(n + fmt[1])
     q = nv.quantize(torch.randn(2, n, k, device="cuda") * 0.02 + 0.3, nv.Quant.affine(*fmt))
-    scales, biases = q.scales.to(dtype), q.biases.to(dtype)
+    codes, scales, biases = q.weight, q.scales.to(dtype), q.biases.to(dtype)
     if wide:
-        scales, biases = torch.full_like(scales, 0.7 * 2.0 ** -(12 + fmt[1])), torch.full_like(biases, 0.71)
-    q = nv.Quantized(q.weight, scales, biases, q.quant)
+        codes = (codes.view(torch.int32) | -0x07070708).view(codes.dtype)  # (0xF8F8F8F8)
+        scales, biases = torch.full_like(scales, 1.42 * 2.0 ** -18), torch.full_like(biases, 0.71)
+    q = nv.Quantized(codes, scales, biases, q.quant)
     x = torch.randn(40, k // 2, device="cuda").to(dtype)
     x = torch.stack([x, -x], dim=-1).reshape(40, k)
     ids = torch.tensor([0] * 17 + [1] * 23, dtype=torch.int32, device="cuda")
     got = nv.gather_qmm_grouped(x, q, torch.arange(40, dtype=torch.int32, device="cuda"), ids, nv.sorted_offsets(ids, 2)).double().cpu()
     weights = torch.stack([unrounded(nv.Quantized(q.weight[e], q.scales[e], q.biases[e], q.quant)) for e in range(2)]).float().double().cpu()
+    unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
     for row in range(40):
-        w = weights[int(ids[row])]
-        want = w @ x[row].double().cpu()
-        # half a unit of the output; float32 sums: K additions (in whatever order) each within 2^-24 of a partial sum, which holds some eighth of a window's
-        # 128 products beside the sum itself (neighbours cancel): at random, sqrt(K) of them, five deviations
-        window = (w * x[row].double().cpu()).abs().unfold(1, 128, 128).sum(-1).amax(-1)
-        unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
-        bound = unit * want.abs() + 5 * k ** 0.5 * 2.0 ** -24 * (window / 8 + want.abs())
+        terms = weights[int(ids[row])] * x[row].double().cpu()
+        want = terms.sum(-1)
+        # half a unit of the output; and up to three matrix instructions for 32 values of K, each of whose sums is within 2^-24 of a partial
+        # sum, which neighbours that cancel keep within four products of the sum itself: at random, five deviations
+        bound = unit * want.abs() + 5 * (3 * k / 32) ** 0.5 * 2.0 ** -24 * (4 * terms.abs().amax(-1) + want.abs())
         assert ((got[row] - want).abs() <= bound).all(), row

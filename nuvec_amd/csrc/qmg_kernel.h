@@ -24,7 +24,7 @@ namespace nvq {
 namespace qmg {
 
 using rows::kTile;
-constexpr int kWaves = 4, kThreads = 64 * kWaves;  // of a group, which shares x; the groups of a block split K
+constexpr int kThreads = 64 * rows::kWaves;  // of a group, which shares x; the groups of a block split K
 constexpr int kRows = 128;     // weight rows of a block: two tiles a wavefront, 64 rows apart
 constexpr int kPassRows = 64;  // rows of x of a pass, the most
 constexpr int most_groups(int hold) { return hold == rows::kTerms ? 2 : 4; }  // (weights in terms take more registers)
@@ -32,7 +32,7 @@ constexpr int stages(int mt, int bits, int hold) { return mt > 2 ? 2 : bits <= 4
 
 template <typename T, int BITS, int FP4, int HOLD, int MT>
 __device__ __forceinline__ void run_pass(const ProductArgs &a, unsigned char *lds, int e, int pass, int rows, int n0) {
-    using B = rows::Body<T, BITS, FP4, HOLD, MT, 2, kWaves, stages(MT, BITS, HOLD)>;
+    using B = rows::Body<T, BITS, FP4, HOLD, MT, 2, stages(MT, BITS, HOLD)>;
     const int tid = threadIdx.x & (kThreads - 1), lane = tid & 63, l = lane & 15, q = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), group = __builtin_amdgcn_readfirstlane(threadIdx.x / kThreads);
     const int groups = __builtin_amdgcn_readfirstlane(blockDim.x / kThreads);
@@ -218,8 +218,8 @@ inline int group_count(const ProductArgs &a, int64_t passes, int most) {
 
 template <typename T, int BITS, int FP4, int HOLD>
 int32_t run_kernel(const ProductArgs &a, hipStream_t s) {
-    constexpr int lds = rows::Body<T, BITS, FP4, HOLD, 4, 2, kWaves, stages(4, BITS, HOLD)>::kLdsBytes;
-    static_assert(lds <= 40960 && lds >= rows::Body<T, BITS, FP4, HOLD, 2, 2, kWaves, stages(2, BITS, HOLD)>::kLdsBytes, "four groups a compute unit");
+    constexpr int lds = rows::Body<T, BITS, FP4, HOLD, 4, 2, stages(4, BITS, HOLD)>::kLdsBytes;
+    static_assert(lds <= 40960 && lds >= rows::Body<T, BITS, FP4, HOLD, 2, 2, stages(2, BITS, HOLD)>::kLdsBytes, "four groups a compute unit");
     static std::atomic<bool> configured{false};
     auto kernel = qmg_kernel<T, BITS, FP4, HOLD>;
     if (!configured.load()) {

@@ -1,11 +1,11 @@
-// The inner loop of products of a few dozen rows: a group of QW wavefronts multiplies up to 16 MT rows of x with 16 NT weight rows a
+// The inner loop of products of a few dozen rows: a group of four wavefronts multiplies up to 16 MT rows of x with 16 NT weight rows a
 // wavefront over a range of K, in windows of 128 values.  Any width of affine codes and the block formats, bfloat16 and float16, K in
 // whole blocks of 32.
 //
 // Codes go from memory straight into the operand layout of v_mfma_f32_16x16x32: lane (row l = lane % 16, quarter q = lane / 16) loads the
 // BITS dwords of its quarter of a window, several windows ahead, and K's order inside a window is permuted to suit (instruction j of a
 // window takes values 8 j .. 8 j + 7 of every quarter).  x goes straight from memory into a ring of LDS stages, without a register, which
-// the group shares; one barrier a window, none where the group is one wavefront.  Scales and biases come 16 bytes a row at a time
+// the group shares; one barrier a window.  Scales and biases come 16 bytes a row at a time
 // (8 or 16 groups) into a table of the wavefront's own in LDS.  The weights are the instruction's first operand, so that a lane's four
 // sums are four consecutive weight rows of one row of x.
 //
@@ -27,6 +27,7 @@ using qmf::static_for;
 typedef qmf::u32x4_t Piece;                                    // 16 bytes
 typedef qmf::u32x2_t u32x2_a4_t __attribute__((aligned(4)));  // 8 bytes in memory at any dword
 
+constexpr int kWaves = 4;        // of a group
 constexpr int kTile = 16;        // rows of x, weight rows of a matrix instruction
 constexpr int kWin = 128;        // values of K
 constexpr int kXRow = 2 * kWin;  // bytes of a row of x
@@ -160,15 +161,15 @@ __device__ __forceinline__ void sum_plainly(const ProductArgs &a, int e, int k0,
 // How affine weights are held: rounded once to the element type, as nuvec's CPU product holds them (qmf::affine_pair), or as terms.
 enum Hold { kRounded, kCpu, kTerms };
 
-template <typename T, int BITS, int FP4, int HOLD, int MT, int NT, int QW, int STAGES>
+template <typename T, int BITS, int FP4, int HOLD, int MT, int NT, int STAGES>
 struct Body {
     static constexpr int kAhead = BITS <= 4 && HOLD != kTerms ? 4 : 2;  // windows of codes under way
-    static constexpr int kXAll = 4 * MT, kX = (kXAll + QW - 1) / QW;  // loads of x of the group and window, of a wavefront
+    static constexpr int kX = MT;  // loads of x of a window and wavefront, four rows each
     static constexpr int kXStage = MT * kTile * kXRow;
     static constexpr int kKinds = FP4 ? 1 : 2, kScaleBytes = FP4 ? 1 : 2, kPart = 16 / kScaleBytes;  // groups of a part of the scales
     static constexpr int kTablePieces = kKinds * NT * kTile * 2, kTableLoads = (kTablePieces + 63) / 64;
     static constexpr int kTableBytes = 16 * kTablePieces;  // of a wavefront
-    static constexpr int kLdsBytes = STAGES * kXStage + QW * kTableBytes;
+    static constexpr int kLdsBytes = STAGES * kXStage + kWaves * kTableBytes;
     static_assert(STAGES >= 2 && STAGES <= kAhead + 1, "the waits below count these loads");
 
     // `xrow(r)`: the row of x behind row r; `weight_row(t, r)`: row r of this wavefront's tile t, rows from `n0`, a row of the weight, on.  The range [k_begin, k1) begins at
@@ -186,7 +187,7 @@ struct Body {
         const int k0 = windows > 0 ? k_begin : 0;  // (a group without a window asks for its rows' first values)
         int64_t xrows[kX];  // (asked for first: what is loaded after does not wait for them)
 #pragma unroll
-        for (int i = 0; i < kX; i++) xrows[i] = xrow(min(4 * (wave + QW * i), kTile * MT - 4) + (lane >> 4));
+        for (int i = 0; i < kX; i++) xrows[i] = xrow(4 * (wave + kWaves * i) + (lane >> 4));
         __builtin_amdgcn_sched_barrier(0);
         unsigned char *table = lds + STAGES * kXStage + wave * kTableBytes;
 
@@ -242,7 +243,7 @@ struct Body {
         auto place_x = [&]() __attribute__((always_inline)) {
 #pragma unroll
             for (int i = 0; i < kX; i++) {
-                xkey[i] = 8 * ((lane & 15) ^ ((4 * (wave + (QW < 4 ? QW * i : 0)) + (lane >> 4)) & 15));
+                xkey[i] = 8 * ((lane & 15) ^ ((4 * wave + (lane >> 4)) & 15));
                 xsrc[i] = (const T *)a.x + xrows[i] * K + k0 + xkey[i];
             }
         };
@@ -250,10 +251,9 @@ struct Body {
             const bool tail = k0 + (win + 1) * kWin > K;
 #pragma unroll
             for (int i = 0; i < kX; i++) {
-                if (kXAll % QW != 0 && wave + QW * i >= kXAll) break;
                 const void *p = xsrc[i] + win * kWin;
                 if (tail) p = k0 + win * kWin + xkey[i] < K ? p : (const void *)&zeros;
-                dma(p, lds0 + stage * kXStage + 1024 * (wave + QW * i));
+                dma(p, lds0 + stage * kXStage + 1024 * (wave + kWaves * i));
             }
         };
         using S = std::conditional_t<FP4 != 0, uint8_t, T>;
@@ -267,7 +267,7 @@ struct Body {
             if (decltype(i)::value < windows) issue_x(decltype(i)::value, decltype(i)::value);
         });
         constexpr int kCodeLoads = NT;  // of a window, at least
-        constexpr int kYounger = (STAGES - 2) * (kXAll / QW + kCodeLoads) + kCodeLoads;
+        constexpr int kYounger = (STAGES - 2) * (kX + kCodeLoads) + kCodeLoads;
         int until_part = part_windows - (k0 / kWin) % part_windows, part = part0;
         store_table();
         load_table(part + 1);
@@ -279,7 +279,7 @@ struct Body {
                 if (win >= turns) return;
                 if (win >= STAGES && win + STAGES - 1 < windows) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(kYounger) : "memory");
                 else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-                if constexpr (QW > 1) asm volatile("s_barrier" ::: "memory");
+                asm volatile("s_barrier" ::: "memory");
                 if (win < windows) {
                     if (until_part == 0) {
                         until_part = part_windows;

@@ -190,7 +190,7 @@ NVQ_API int32_t nvq_gather_grouped(int64_t rows, int64_t experts, int32_t row_ex
 /* 1 if the pairs of `tokens` tokens with `choices` experts each run faster ordered by expert, every expert's weights read once, than one
  * by one: from 64 pairs on as in the reference (crates/nuvec-lm/src/model.rs:2189-2192), fewer where the estimate says so and the weights
  * are held no less precisely (not MXFP4 and MXFP8 in float16, which rounds those of small scales).  `values`: of an expert's three projections; `scaled`: with a global scale.
- * Below 64 pairs the caller asks as well whether the grouped kernel takes the projections (nvq_gather_sorted_takes). */
+ * Below 64 pairs a caller counts the projections that the grouped kernel takes (nvq_gather_sorted_takes). */
 NVQ_API int32_t nvq_moe_ordered(const nvq_quant *quant, int32_t dtype, int64_t tokens, int32_t choices, int64_t experts, int64_t values,
                                 int32_t scaled);
 
@@ -237,9 +237,9 @@ NVQ_API int32_t nvq_dequantize_rows(const nvq_quant *quant, int32_t dtype, const
  * (gpu.rs:7022, "nuvec_affine_qmv_mma_..."; its tests check the names, crates/nuvec-core/tests/quantized.rs:843-861).
  * Needs nvq_init. */
 NVQ_API const char *nvq_quantized_matmul_route(const nvq_qmm_desc *desc);
-/* The kernel that runs it, given the workspace that the size query names.  It is the route's but on two of them: products of "qmf_kernel"
- * and "qmm_kernel" may run on "qms_kernel<R,C,G>" (a block holds 16 R rows of x, a wavefront 16 C weight rows, G wavefronts share
- * x), and those of "qmm_kernel" on "qmm_dense_kernel". */
+/* The kernel that runs it, given the workspace that the size query names.  It is the route's but for these: products of "qmf_kernel" and
+ * "qmm_kernel" may run on "qms_kernel<R,C,G>" (a block holds 16 R rows of x, a wavefront 16 C weight rows, G wavefronts share x), those
+ * of "qmm_kernel" on "qmm_dense_kernel", and float32 ones of the vector kernels on "qmm_f32_kernel". */
 NVQ_API const char *nvq_quantized_matmul_kernel(const nvq_qmm_desc *desc);
 /* Bytes of scratch nvq_quantized_matmul needs for `desc` (the reference allocates them on its side of the boundary, gpu.rs:7562; the
  * counterpart of its qmm_t_splitk, gpu.rs:7507-7590).  0 = none; nonzero where K is split over the grid (float32 partial sums): transpose = 0,

@@ -10,9 +10,8 @@
 // instantiation of the loop: a pass of a few rows neither brings nor multiplies the others.  Gate and up rows that alternate in runs
 // of 64 are the two tiles of one wavefront, lane for lane, so that the gated activation needs no exchange.
 //
-// What bounds it: the way of codes and x through a compute unit's memory pipeline (30 rows of each of 32 experts, MXFP4 w[5760,2880]: the
-// codes alone take 60 us, x beside them 20 more, the arithmetic by itself 34), and about 18 us of a launch for the blocks' first
-// loads and the activation.  Four blocks a compute unit with the loads of four windows under way; codes staged in LDS with x took the
+// What bounds it: the way of codes and x through a compute unit's memory pipeline, and the blocks' first loads (30 rows of each of 32
+// experts, MXFP4 w[5760,2880], 91 us: 88 without the arithmetic, 77 without x as well, the arithmetic on operands that are not loaded 50).  Four blocks a compute unit with the loads of four windows under way; codes staged in LDS with x took the
 // same time at two blocks, wider blocks of eight wavefronts (half the reads of x) 109 us against 97, codes read by lines of 128 bytes
 // the same.  Before -> now (the kernel of four wavefronts on 32 x 32 x 16 tiles), us: that product at 8 / 30 / 40 rows an expert 90 / 105 / 124
 // -> 82 / 95 / 108; 4 bits 130 / 134 / 163 -> 107 / 119 / 131; 8 bits 250 / 258 / 274 -> 142 / 156 / 168; w[768,2432] of 8 bits, 12 rows, 46 -> 21.

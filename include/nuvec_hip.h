@@ -475,7 +475,7 @@ NVQ_API int32_t nvq_quantized_matmul_glu_rows(const nvq_qmm_desc *desc, int32_t 
  * depends on desc alone. */
 NVQ_API int32_t nvq_quantized_matmul_glu_grouped_takes(const nvq_qmm_desc *desc);
 /* Both questions at once, for a caller that has to launch one of them: 1 if nvq_quantized_matmul_glu_grouped takes the product, 2 if not but
- * nvq_quantized_matmul_glu_rows does, with a workspace of `*workspace_bytes`, 0 if neither. */
+ * nvq_quantized_matmul_glu_rows does, with a workspace of `*workspace_bytes` (may be NULL), 0 if neither. */
 NVQ_API int32_t nvq_quantized_matmul_glu_several_takes(const nvq_qmm_desc *desc, size_t *workspace_bytes);
 NVQ_API int32_t nvq_quantized_matmul_glu_grouped(const nvq_qmm_desc *desc, int32_t activation, float alpha, float limit, const void *x,
                                 const void *w, const void *scales, const void *biases, const void *bias, void *y, void *stream);

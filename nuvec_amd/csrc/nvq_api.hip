@@ -935,13 +935,13 @@ int32_t nvq_quantized_matmul_glu_grouped_takes(const nvq_qmm_desc *d) {
 }
 
 int32_t nvq_quantized_matmul_glu_several_takes(const nvq_qmm_desc *d, size_t *workspace_bytes) {
-    *workspace_bytes = 0;
+    if (workspace_bytes != nullptr) *workspace_bytes = 0;
     ProductArgs a;
     qms::Plan plan;
     int groups;
     if (!gated_args(d, a)) return 0;
     const Gated choice = gated_choice(d, a, plan, groups);
-    if (choice == Gated::kRows) *workspace_bytes = qms_workspace_bytes(a, plan);
+    if (choice == Gated::kRows && workspace_bytes != nullptr) *workspace_bytes = qms_workspace_bytes(a, plan);
     return choice == Gated::kGroup ? 1 : choice == Gated::kRows ? 2 : 0;
 }
 
@@ -1350,7 +1350,8 @@ static int32_t gather_qmm_any(const nvq_gather_desc *d, const void *x, const voi
 
 static bool gather_desc_holds(const nvq_gather_desc *d) {
     return d != nullptr && check_quant(&d->quant, "gather_qmm") == NVQ_OK && check_float("gather_qmm", d->dtype) == NVQ_OK &&
-           check_product_dims("gather_qmm", d->quant, d->transpose, d->m, d->n, d->k) == NVQ_OK && d->transpose && d->n > 0 && d->k > 0 && d->pairs > 0;
+           check_product_dims("gather_qmm", d->quant, d->transpose, d->m, d->n, d->k) == NVQ_OK && d->transpose && d->n > 0 && d->k > 0 &&
+           d->pairs > 0 && d->x_batches > 0 && d->experts > 0;
 }
 
 int32_t nvq_gather_sorted_takes(const nvq_gather_desc *d) {

@@ -105,5 +105,6 @@ def test_both_questions_at_once():
         rows = library.nvq_quantized_matmul_glu_rows_takes(C.byref(d), C.byref(of_rows))
         grouped = library.nvq_quantized_matmul_glu_grouped_takes(C.byref(d))
         assert got == (1 if grouped else 2 if rows else 0) and need.value == (of_rows.value if got == 2 else 0)
+        assert library.nvq_quantized_matmul_glu_several_takes(C.byref(d), None) == got
         seen.add(got)
     assert seen == {0, 1, 2}

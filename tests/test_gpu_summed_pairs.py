@@ -56,6 +56,17 @@ def test_what_the_two_kernels_keep():
         assert call(q, x, ids, ids, None, scores, out, choices, choices) == _lib.UNSUPPORTED
 
 
+def test_questions_about_nothing():
+    """Descriptors that no launch would take."""
+    ask = lambda **odd: [f(C.byref(_lib.GatherDescC(**{**dict(quant=nv.Quant.affine(64, 4)._c(), dtype=ops._CODE[torch.bfloat16], transpose=1, m=1, n=1024, k=2880, pairs=4,
+                                                              x_batches=4, experts=8), **odd}))) for f in (_lib.load().nvq_gather_sorted_takes, lambda d: _lib.load().nvq_gather_qmm_sum_takes(d, 4))]
+    nv.quantize(torch.zeros(1, 64, device="cuda"), nv.Quant.affine(64, 4))  # (the library has a device)
+    assert ask() == [1, 1]
+    for odd in (dict(pairs=0), dict(pairs=-4), dict(experts=0), dict(experts=-1), dict(x_batches=0), dict(n=0), dict(k=0), dict(k=2881), dict(transpose=0), dict(dtype=-1)):
+        assert ask(**odd) == [0, 0], odd
+    assert _lib.load().nvq_gather_sorted_takes(None) == 0 and _lib.load().nvq_gather_qmm_sum_takes(None, 1) == 0
+
+
 def test_the_question_answers_as_the_call():
     """`nvq_gather_qmm_sum_takes`, by which a block asks before it launches."""
     torch.manual_seed(2)

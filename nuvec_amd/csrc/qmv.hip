@@ -496,19 +496,29 @@ __device__ __forceinline__ void load_slice(const uint32_t *w, const S *scales, c
     else braw = T{};
 }
 
-// The bias of weight row n, requested with the weights: read at the end it cost every block a trip to memory more.  BIAS: whether the product
-// has one.  (Chosen at the launch: a branch in the kernel makes the wait for x, counted over both of its ways, wait for weights too, and a load
-// of something else in its place costs products without a bias up to 4 %: us, one row, W[14336,4096] MXFP4 7.34 there, 7.08 here, 8 bits 13.10
-// and 12.99, W[4096,14336] 6 bits 13.06 and 12.93.)
-template <typename T, bool BIAS>
+// The bias of a weight row.  Early: requested with its weights, since read at the end it costs every block a trip to memory more.  Which of
+// the three is a template parameter, chosen at the launch: a branch in the kernel makes the wait for x, counted over both of its ways, wait
+// for weights too, and a load of something else in its place costs products without a bias up to 15 %.
+enum Bias { kNoBias, kEarlyBias, kLateBias };
+template <typename T, int BIAS>
 __device__ __forceinline__ T early_bias(const void *row_bias, int64_t n) {
-    if constexpr (BIAS) return ((const T *)row_bias)[n];
+    if constexpr (BIAS == kEarlyBias) return ((const T *)row_bias)[n];
     else return T{};
 }
-template <typename T, bool BIAS>
-__device__ __forceinline__ float add_early_bias(float v, T bias) {
-    if constexpr (BIAS) return Elem<T>::add(Elem<T>::mul(v, 1.0f), Elem<T>::load(&bias, 0));
+template <typename T, int BIAS>
+__device__ __forceinline__ float add_bias(const void *row_bias, float v, T early, int64_t n) {
+    if constexpr (BIAS == kEarlyBias) return Elem<T>::add(Elem<T>::mul(v, 1.0f), Elem<T>::load(&early, 0));
+    else if constexpr (BIAS == kLateBias) return add_row_bias<T>(row_bias, v, n);
     else return v;
+}
+// Early where K is one step of a wavefront, and of affine codes.  Beyond, the request returns at every step, and with it the compiler waits for
+// x before it requests the weights of a block format (one row, us without a bias / early / late: MXFP4 W[4096,14336] 7.7 / 8.9 / 8.0,
+// W[298,11968] 4.3 / 5.0 / 4.5, NVFP4 W[4096,14336] 8.1 / 9.0 / 8.1); affine codes are held to their order below (8 bits, W[2048,8192]
+// 6.2 / 6.2 / 6.3).
+template <int MODE>
+Bias bias_of(const ProductArgs &a) {
+    if (a.row_bias == nullptr) return kNoBias;
+    return a.k <= 2 * kStep || is_affine_mode(MODE) ? kEarlyBias : kLateBias;
 }
 
 // Eight values of x as the codes of a slice meet them; the sum of eight values in that order.
@@ -561,7 +571,7 @@ __device__ __forceinline__ void code_constants(uint32_t &mask, uint32_t &magic, 
 // RN = 2): a wavefront takes output column c of [pairs, N / 2], i.e. weight rows 128 (c / 64) + c % 64 (gate) and that
 // + 64 (up), and stores the gated activation of the two rounded products (each with its expert's bias first), bit for
 // bit what the product followed by the activation kernel gives.
-template <typename T, int RM, int RN, int WAVES, bool BATCHED, bool BIAS, int MODE = NVQ_AFFINE, bool GLU = false>
+template <typename T, int RM, int RN, int WAVES, bool BATCHED, int BIAS, int MODE = NVQ_AFFINE, bool GLU = false>
 __global__ void __launch_bounds__(WAVES * 64) qmv4_lds_kernel(const ProductArgs a) {
     constexpr int kThreads = WAVES * 64;
     constexpr int kXPerThread = 512 / kThreads;  // 128-bit pieces of one x row per thread and step
@@ -627,6 +637,10 @@ __global__ void __launch_bounds__(WAVES * 64) qmv4_lds_kernel(const ProductArgs 
         }
 #pragma unroll
         for (int r = 0; r < RN; r++) bias[r] = early_bias<T, BIAS>(a.row_bias, o.bias + (n0 + r * kRowStep < N ? n0 + r * kRowStep : N - 1));
+        // Left to itself the compiler waits for x before it requests the weights of some affine variants (8 bits without a bias, W[2048,8192]
+        // 6.4 us, 6.2 so).  Block formats would turn a scale into a float before the second request (MXFP4 W[4096,14336] 7.7, 9.4 so), and a
+        // gate and an up row gain nothing (4 bits, four MLPs 4096 -> 14336 -> 4096 86.9, 87.2 so).
+        if constexpr (kAffine && !GLU) __builtin_amdgcn_sched_barrier(0);
         if (k0 != 0) __syncthreads();  // the previous step's readers are done with the LDS
 #pragma unroll
         for (int i = 0; i < RM; i++)
@@ -664,7 +678,7 @@ __global__ void __launch_bounds__(WAVES * 64) qmv4_lds_kernel(const ProductArgs 
             const float g = wave_sum_lane63(acc[0][i]), u = wave_sum_lane63(acc[1][i]);
             if (lane == 63 && column < H && m0 + i < M) {
                 // the products as their outputs hold them, the expert's bias by a separate rounded addition
-                const float gate = add_early_bias<T, BIAS>(rounded<T>(g), bias[0]), up = add_early_bias<T, BIAS>(rounded<T>(u), bias[1]);
+                const float gate = add_bias<T, BIAS>(a.row_bias, rounded<T>(g), bias[0], o.bias + n0), up = add_bias<T, BIAS>(a.row_bias, rounded<T>(u), bias[1], o.bias + n0 + 64);
                 const float v = a.glu == 1 + NVQ_GLU_SWIGLU       ? glu<T, NVQ_GLU_SWIGLU>(gate, up, a.glu_alpha, a.glu_limit)
                                 : a.glu == 1 + NVQ_GLU_SWIGLU_OAI ? glu<T, NVQ_GLU_SWIGLU_OAI>(gate, up, a.glu_alpha, a.glu_limit)
                                                                   : glu<T, NVQ_GLU_GEGLU>(gate, up, a.glu_alpha, a.glu_limit);
@@ -678,7 +692,7 @@ __global__ void __launch_bounds__(WAVES * 64) qmv4_lds_kernel(const ProductArgs 
 #pragma unroll
         for (int i = 0; i < RM; i++) {
             const float v = wave_sum_lane63(acc[r][i]);
-            if (lane == 63 && n0 + r < N && m0 + i < M) Elem<T>::store(y, (int64_t)(m0 + i) * N + n0 + r, add_early_bias<T, BIAS>(v, bias[r]));
+            if (lane == 63 && n0 + r < N && m0 + i < M) Elem<T>::store(y, (int64_t)(m0 + i) * N + n0 + r, add_bias<T, BIAS>(a.row_bias, v, bias[r], o.bias + n0 + r));
         }
 }
 
@@ -1306,9 +1320,12 @@ template <typename T, int RM, int RN, int WAVES, int MODE = NVQ_AFFINE>
 int32_t run_lds4(const ProductArgs &a, hipStream_t s) {
     const int64_t rows = (int64_t)WAVES * RN;
     dim3 grid((unsigned)((a.n + rows - 1) / rows), (unsigned)((a.m + RM - 1) / RM), (unsigned)a.batch);
-    const bool batched = !(a.batch == 1 && a.rhs == nullptr), biased = a.row_bias != nullptr;
-    void (*kernel)(const ProductArgs) = batched ? (biased ? qmv4_lds_kernel<T, RM, RN, WAVES, true, true, MODE> : qmv4_lds_kernel<T, RM, RN, WAVES, true, false, MODE>)
-                                                : (biased ? qmv4_lds_kernel<T, RM, RN, WAVES, false, true, MODE> : qmv4_lds_kernel<T, RM, RN, WAVES, false, false, MODE>);
+    const bool batched = !(a.batch == 1 && a.rhs == nullptr);
+    const Bias bias = bias_of<MODE>(a);
+    void (*kernel)(const ProductArgs) = batched ? qmv4_lds_kernel<T, RM, RN, WAVES, true, kNoBias, MODE> : qmv4_lds_kernel<T, RM, RN, WAVES, false, kNoBias, MODE>;
+    if (bias == kEarlyBias) kernel = batched ? qmv4_lds_kernel<T, RM, RN, WAVES, true, kEarlyBias, MODE> : qmv4_lds_kernel<T, RM, RN, WAVES, false, kEarlyBias, MODE>;
+    if constexpr (!is_affine_mode(MODE))
+        if (bias == kLateBias) kernel = batched ? qmv4_lds_kernel<T, RM, RN, WAVES, true, kLateBias, MODE> : qmv4_lds_kernel<T, RM, RN, WAVES, false, kLateBias, MODE>;
     hipLaunchKernelGGL(kernel, grid, dim3(WAVES * 64), 0, s, a);
     NVQ_LAUNCH_CHECK("qmv4_lds");
     return NVQ_OK;
@@ -1325,7 +1342,7 @@ bool glu_pairs_take(const ProductArgs &a) {  // (also a single product, without 
 }
 
 // ... and their launch: a wavefront per output column.
-template <typename T, int MODE, bool BIAS>
+template <typename T, int MODE, int BIAS>
 int32_t run_glu_pairs_biased(const ProductArgs &a, hipStream_t s) {
     const int rm = a.m == 1 ? 1 : a.m == 2 ? 2 : 4;
     const dim3 grid((unsigned)((a.n / 2 + 7) / 8), (unsigned)((a.m + rm - 1) / rm), (unsigned)a.batch);
@@ -1339,7 +1356,10 @@ int32_t run_glu_pairs_biased(const ProductArgs &a, hipStream_t s) {
 
 template <typename T, int MODE>
 int32_t run_glu_pairs_mode(const ProductArgs &a, hipStream_t s) {
-    return a.row_bias != nullptr ? run_glu_pairs_biased<T, MODE, true>(a, s) : run_glu_pairs_biased<T, MODE, false>(a, s);
+    const Bias bias = bias_of<MODE>(a);
+    if constexpr (!is_affine_mode(MODE))
+        if (bias == kLateBias) return run_glu_pairs_biased<T, MODE, kLateBias>(a, s);
+    return bias == kEarlyBias ? run_glu_pairs_biased<T, MODE, kEarlyBias>(a, s) : run_glu_pairs_biased<T, MODE, kNoBias>(a, s);
 }
 
 template <typename T>
@@ -1356,7 +1376,7 @@ int32_t run_glu_pairs(const ProductArgs &a, hipStream_t s) {
 // A block takes `columns` outputs of a token with all its `choices` pairs: wavefront (g, j) RN weight rows of pair j's expert as
 // qmv4_lds_kernel does (the same slices and sums), the pairs' x in LDS together; the rounded, biased products meet in LDS and are summed
 // with the scores in the order of weighted_sum_kernel: bit for bit the two kernels.
-template <typename T, int RN, int MODE, bool BIAS>
+template <typename T, int RN, int MODE, int BIAS>
 __global__ void __launch_bounds__(512) qmv4_sum_kernel(const ProductArgs a, const T *__restrict__ scores, T *__restrict__ out, int choices, int groups) {
     constexpr bool kAffine = is_affine_mode(MODE);
     constexpr int kPieces = 4;  // of x a thread stages a step: 512 a row over 64 * choices * groups threads, groups at least 2
@@ -1437,7 +1457,7 @@ __global__ void __launch_bounds__(512) qmv4_sum_kernel(const ProductArgs a, cons
 #pragma unroll
     for (int r = 0; r < RN; r++) {
         const float v = wave_sum_lane63(acc[r][0]);
-        if (lane == 63 && n0 + r < N) products[j * columns + g * RN + r] = rounded<T>(add_early_bias<T, BIAS>(v, bias[r]));
+        if (lane == 63 && n0 + r < N) products[j * columns + g * RN + r] = rounded<T>(add_bias<T, BIAS>(a.row_bias, v, bias[r], o.bias + n0 + r));
     }
     __syncthreads();
     const int n = (int)blockIdx.x * columns + tid;
@@ -1458,7 +1478,10 @@ int32_t run_sum_rows(const ProductArgs &a, const void *scores, void *out, int ch
     const int groups = 8 / choices, columns = groups * RN;
     const size_t lds = (size_t)choices * (8192 + (is_affine_mode(MODE) ? 512 : 0) + 4 * columns);  // (at most 34.9 KB)
     const dim3 grid((unsigned)((a.n + columns - 1) / columns), (unsigned)(a.batch / choices));
-    void (*kernel)(const ProductArgs, const T *, T *, int, int) = a.row_bias != nullptr ? qmv4_sum_kernel<T, RN, MODE, true> : qmv4_sum_kernel<T, RN, MODE, false>;
+    const Bias bias = bias_of<MODE>(a);
+    void (*kernel)(const ProductArgs, const T *, T *, int, int) = bias == kNoBias ? qmv4_sum_kernel<T, RN, MODE, kNoBias> : qmv4_sum_kernel<T, RN, MODE, kEarlyBias>;
+    if constexpr (!is_affine_mode(MODE))
+        if (bias == kLateBias) kernel = qmv4_sum_kernel<T, RN, MODE, kLateBias>;
     hipLaunchKernelGGL(kernel, grid, dim3((unsigned)(64 * choices * groups)), lds, s, a, (const T *)scores, (T *)out, choices, groups);
     NVQ_LAUNCH_CHECK("qmv4_sum");
     return NVQ_OK;

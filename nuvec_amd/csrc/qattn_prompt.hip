@@ -49,17 +49,13 @@ struct PromptArgs {
     int32_t tiles, row_tiles, splits;
 };
 
-// Codes d0 .. d0 + 7 of a row (BITS bytes at byte d0 / 8 x BITS of its dwords), each value rounded once: the product's own
-// rounding first, as `dequantize` has it, is the larger of the two (error against float64, 64 queries over 1024 positions of 8
-// bits: float16 8.7e-4 with both, 4.0e-4 with one, 8.3e-4 in the composition; bfloat16 7.2e-3, 3.2e-3, 8.3e-3).  TERMS 2: what that
-// leaves in a second term (the first is finite, so that an infinity is the second's).
+// Eight codes, each value rounded once: the product's own rounding first, as `dequantize` has it, is the larger of the two (error
+// against float64, 64 queries over 1024 positions of 8 bits: float16 8.7e-4 with both, 4.0e-4 with one, 8.3e-4 in the composition;
+// bfloat16 7.2e-3, 3.2e-3, 8.3e-3).  TERMS 2: what that leaves in a second term (the first is finite, so that an infinity is the
+// second's).
 template <typename T, int BITS, int TERMS>
-__device__ __forceinline__ void dequantize_eight(const uint32_t *row, int words, int d0, float s, float b, uint4 (&out)[TERMS]) {
+__device__ __forceinline__ void dequantize_eight(uint64_t codes, float s, float b, uint4 (&out)[TERMS]) {
     constexpr float most = Elem<T>::code == NVQ_BF16 ? 3.38953139e38f : 65504.0f;
-    const int byte = d0 / 8 * BITS, w = byte >> 2, sh = 8 * (byte & 3);
-    uint64_t v = row[w];
-    if constexpr (BITS > 1) v |= (uint64_t)row[w + 1 < words ? w + 1 : w] << 32;
-    const uint64_t codes = v >> sh;  // (BITS bytes from byte 0 .. 3 of a word: they end in the second one)
     auto at = [&](int i) { return __builtin_fmaf((float)(uint32_t)((codes >> (i * BITS)) & ((1u << BITS) - 1u)), s, b); };
     uint32_t p[TERMS][4];
 #pragma unroll
@@ -75,31 +71,69 @@ __device__ __forceinline__ void dequantize_eight(const uint32_t *row, int words,
     for (int t = 0; t < TERMS; t++) out[t] = make_uint4(p[t][0], p[t][1], p[t][2], p[t][3]);
 }
 
-// Block: one tile of 32 keys of one (batch, key head).  Bound by its reads of the codes; positions past the end are zeros.
+// Block: one tile of 32 keys of one (batch, key head); positions past the end are zeros.  Bound by the latency of its requests: codes,
+// scales and biases of 32 rows are runs of consecutive bytes and pass through LDS (eight codes a lane straight from 32 rows, and its
+// scale: sixteen requests a wavefront of 32 cache lines each, OPERAND_FIGURES).
 template <typename T, int BITS, int D, int TERMS>
 __global__ void __launch_bounds__(256) prompt_operands_kernel(const uint32_t *__restrict__ kw, const T *__restrict__ ks, const T *__restrict__ kb,
                                                              const uint32_t *__restrict__ vw, const T *__restrict__ vs, const T *__restrict__ vb,
                                                              int head0, int positions, int group_shift, uint4 *__restrict__ keys, uint4 *__restrict__ values) {
-    constexpr int kChunks = kKeys * D / 8, words = D * BITS / 32;
+    constexpr int kChunks = kKeys * D / 8, words = D * BITS / 32, kWords = kKeys * words, kOwn = (kWords + 255) / 256;
+    constexpr int kStride = words + 1 + words % 2;  // dwords of a row in LDS, an odd number: lanes of one column fall on different banks
     __shared__ __align__(16) uint16_t tile[kKeys][D + 8];
+    __shared__ uint32_t codes[2][kKeys * kStride + 1];
+    __shared__ T scales[4][kKeys * (D / 32)];
+    const int tid = threadIdx.x;
     const int64_t block = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
-    const int groups = D >> group_shift, s0 = blockIdx.x * kKeys;
-    const int64_t row0 = (int64_t)(head0 + blockIdx.y) * positions;
-    for (int c = threadIdx.x; c < kChunks; c += 256) {
-        const int key = c & 31, d0 = (c >> 5) * 8;  // (chunk (step << 6 | half << 5 | key): values 16 step + 8 half ..)
+    const int groups = D >> group_shift, s0 = blockIdx.x * kKeys, rows = positions - s0 < kKeys ? positions - s0 : kKeys;
+    const int64_t row0 = (int64_t)(head0 + blockIdx.y) * positions + s0;
+    const uint32_t *kcodes = kw + row0 * words, *vcodes = vw + row0 * words;
+    uint32_t kc[kOwn], vc[kOwn];
+#pragma unroll
+    for (int u = 0; u < kOwn; u++) {  // (past the end: the last dword, not used)
+        const int i = 256 * u + tid < rows * words ? 256 * u + tid : rows * words - 1;
+        kc[u] = kcodes[i], vc[u] = vcodes[i];
+    }
+    // scales, biases of the keys, then of the values: 64 threads each
+    const int kind = tid >> 6, first = tid & 63;
+    const T *from = (kind == 0 ? ks : kind == 1 ? kb : kind == 2 ? vs : vb) + row0 * groups;
+    T sc[kKeys * (D / 32) / 64];
+#pragma unroll
+    for (int u = 0; u < kKeys * (D / 32) / 64; u++) {
+        const int i = first + 64 * u;
+        sc[u] = from[i < rows * groups ? i : rows * groups - 1];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < kOwn; u++) {
+        const int i = 256 * u + tid;
+        if ((u + 1) * 256 <= kWords || i < kWords) codes[0][i / words * kStride + i % words] = kc[u], codes[1][i / words * kStride + i % words] = vc[u];
+    }
+#pragma unroll
+    for (int u = 0; u < kKeys * (D / 32) / 64; u++) scales[kind][first + 64 * u] = sc[u];
+    __syncthreads();
+#pragma unroll
+    for (int c0 = 0; c0 < kChunks; c0 += 256) {
+        const int c = c0 + tid, key = c & 31, d0 = (c >> 5) * 8;  // (chunk (step << 6 | half << 5 | key): values 16 step + 8 half ..)
+        const int byte = d0 / 8 * BITS, w = key * kStride + (byte >> 2), g = key * groups + (d0 >> group_shift);
+        auto eight = [&](const uint32_t *of) {  // (BITS bytes from byte 0 .. 3 of a word: they end in the second one)
+            uint64_t v = of[w];
+            if constexpr (BITS > 1 && BITS != 4) v |= (uint64_t)of[w + 1] << 32;
+            return v >> (8 * (byte & 3));
+        };
         uint4 k[TERMS] = {}, v[1] = {};
-        if (s0 + key < positions) {
-            const int64_t row = row0 + s0 + key, g = row * groups + (d0 >> group_shift);
-            dequantize_eight<T, BITS, TERMS>(kw + row * words, words, d0, Elem<T>::load(ks, g), Elem<T>::load(kb, g), k);
-            dequantize_eight<T, BITS, 1>(vw + row * words, words, d0, Elem<T>::load(vs, g), Elem<T>::load(vb, g), v);
+        if (key < rows) {
+            dequantize_eight<T, BITS, TERMS>(eight(codes[0]), Elem<T>::load(scales[0], g), Elem<T>::load(scales[1], g), k);
+            dequantize_eight<T, BITS, 1>(eight(codes[1]), Elem<T>::load(scales[2], g), Elem<T>::load(scales[3], g), v);
         }
 #pragma unroll
         for (int t = 0; t < TERMS; t++) keys[(block * TERMS + t) * kChunks + c] = k[t];
         *reinterpret_cast<uint4 *>(&tile[key][d0]) = v[0];
     }
     __syncthreads();
-    for (int c = threadIdx.x; c < kChunks; c += 256) {
-        const int lane = c & 63, h = lane >> 5, part = c >> 6;  // part: which sixteen keys x which 32 values of D
+#pragma unroll
+    for (int c0 = 0; c0 < kChunks; c0 += 256) {
+        const int c = c0 + tid, lane = c & 63, h = lane >> 5, part = c >> 6;  // part: which sixteen keys x which 32 values of D
         const int s = part / (D / 32) * 16 + 4 * h, d = part % (D / 32) * 32 + (lane & 31);
         uint32_t p[4];
 #pragma unroll

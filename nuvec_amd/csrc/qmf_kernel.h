@@ -189,6 +189,50 @@ __device__ __forceinline__ float code_to_float(const uint32_t (&dw)[BITS]) {
     }
 }
 
+// Codes J and J + 1 of a lane's 32 as two float16 integers.  1024 + c is 0x6400 | c, and the subtraction is exact.  BITS 4: byte
+// J / 2 % 4 of the word's even and odd nibbles.
+template <int BITS, int J>
+__device__ __forceinline__ f16x2v_t code_pair_f16(const uint32_t (&dw)[BITS]) {
+    static_assert(J % 2 == 0, "a pair");
+    uint32_t p;
+    if constexpr (BITS == 8) {
+        constexpr uint32_t b = J % 4;
+        p = __builtin_amdgcn_perm(0x64646464u, dw[J / 4], 0x04000400u | (b + 1) << 16 | b);
+    } else if constexpr (BITS == 4) {
+        constexpr uint32_t b = J / 2 % 4;
+        const uint32_t even = opaque(dw[J / 8] & 0x0F0F0F0Fu), odd = opaque((dw[J / 8] >> 4) & 0x0F0F0F0Fu);
+        p = __builtin_amdgcn_perm(odd, even, 0x0C000C00u | (b + 4) << 16 | b) | 0x64006400u;
+    } else {
+        constexpr int at = J * BITS, d = at / 32, s = at % 32;
+        constexpr uint32_t mask = (1u << BITS) - 1u;
+        uint32_t both;  // the two codes in the low bits
+        if constexpr (s + 2 * BITS <= 32) both = dw[d] >> s;
+        else both = __builtin_amdgcn_alignbit(dw[d + 1], dw[d], s);
+        p = (both & mask) | (both << (16 - BITS) & mask << 16) | 0x64006400u;
+    }
+    return __builtin_bit_cast(f16x2v_t, p) - f16x2v_t{(_Float16)1024, (_Float16)1024};
+}
+
+// Weights J and J + 1 of a lane's 32 affine codes (affine_pair).  float16 takes packed instructions: a scale, a bias and a code are
+// float16 values, so one packed fma is the one rounding (the float32 one and its conversion, 3.5 instructions a code, are a second one
+// now and then), and a product and a sum are the CPU's two; 1.5 instructions a code of 8 bits, some 2.5 of the others.  bfloat16
+// has no packed arithmetic here.  us, 16 rows of float16, 8 bits in groups of 32: SEE_FIGURES
+template <typename T, int BITS, int J, bool EXACT>
+__device__ __forceinline__ uint32_t affine_weights(const uint32_t (&dw)[BITS], float s, float b) {
+    if constexpr (Elem<T>::code == NVQ_F16) {
+        const f16x2v_t c = code_pair_f16<BITS, J>(dw);
+        const _Float16 hs = (_Float16)s, hb = (_Float16)b;
+        const f16x2v_t s2 = {hs, hs}, b2 = {hb, hb};
+        if constexpr (EXACT) return __builtin_bit_cast(uint32_t, c * s2 + b2);
+        else return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(c, s2, b2));
+    } else if constexpr (BITS == 4) {
+        const uint32_t even = opaque(dw[J / 8] & 0x0F0F0F0Fu), odd = opaque((dw[J / 8] >> 4) & 0x0F0F0F0Fu);
+        return affine_pair<T, EXACT>(ubyte_to_float<J / 2 % 4>(even), ubyte_to_float<J / 2 % 4>(odd), s, b);
+    } else {
+        return affine_pair<T, EXACT>(code_to_float<BITS, J>(dw), code_to_float<BITS, J + 1>(dw), s, b);
+    }
+}
+
 // Piece KK (eight codes, stream order) of a lane's 32 codes as one matrix operand.
 template <typename T, int BITS, int FP4, int KK, bool EXACT = false>
 __device__ __forceinline__ uint4 expand_piece(const uint32_t (&dw)[BITS], float s, float b) {
@@ -211,19 +255,11 @@ __device__ __forceinline__ uint4 expand_piece(const uint32_t (&dw)[BITS], float 
         r.y = Ops<T>::template fp4_pair<1>(word, s);
         r.z = Ops<T>::template fp4_pair<2>(word, s);
         r.w = Ops<T>::template fp4_pair<3>(word, s);
-    } else if constexpr (BITS == 4) {
-        const uint32_t word = dw[KK];
-        const uint32_t even = opaque(word & 0x0F0F0F0Fu), odd = opaque((word >> 4) & 0x0F0F0F0Fu);
-        r.x = affine_pair<T, EXACT>(ubyte_to_float<0>(even), ubyte_to_float<0>(odd), s, b);
-        r.y = affine_pair<T, EXACT>(ubyte_to_float<1>(even), ubyte_to_float<1>(odd), s, b);
-        r.z = affine_pair<T, EXACT>(ubyte_to_float<2>(even), ubyte_to_float<2>(odd), s, b);
-        r.w = affine_pair<T, EXACT>(ubyte_to_float<3>(even), ubyte_to_float<3>(odd), s, b);
     } else {
-        constexpr int J = 8 * KK;
-        r.x = affine_pair<T, EXACT>(code_to_float<BITS, J + 0>(dw), code_to_float<BITS, J + 1>(dw), s, b);
-        r.y = affine_pair<T, EXACT>(code_to_float<BITS, J + 2>(dw), code_to_float<BITS, J + 3>(dw), s, b);
-        r.z = affine_pair<T, EXACT>(code_to_float<BITS, J + 4>(dw), code_to_float<BITS, J + 5>(dw), s, b);
-        r.w = affine_pair<T, EXACT>(code_to_float<BITS, J + 6>(dw), code_to_float<BITS, J + 7>(dw), s, b);
+        r.x = affine_weights<T, BITS, 8 * KK + 0, EXACT>(dw, s, b);
+        r.y = affine_weights<T, BITS, 8 * KK + 2, EXACT>(dw, s, b);
+        r.z = affine_weights<T, BITS, 8 * KK + 4, EXACT>(dw, s, b);
+        r.w = affine_weights<T, BITS, 8 * KK + 6, EXACT>(dw, s, b);
     }
     return r;
 }

@@ -127,13 +127,8 @@ __device__ __forceinline__ uint32_t expand_dword(const uint32_t (&dw)[BITS], flo
         return fp4_pair_times<T, D>(dw[KK], s);
     } else if constexpr (FP4) {
         return Ops<T>::template fp4_pair<D>(Ops<T>::mx_codes(dw[KK], s), s);
-    } else if constexpr (BITS == 4) {
-        const uint32_t word = dw[KK];
-        const uint32_t even = opaque(word & 0x0F0F0F0Fu), odd = opaque((word >> 4) & 0x0F0F0F0Fu);
-        return affine_pair<T, EXACT>(ubyte_to_float<D>(even), ubyte_to_float<D>(odd), s, b);
     } else {
-        constexpr int J = 8 * KK + 2 * D;
-        return affine_pair<T, EXACT>(code_to_float<BITS, J>(dw), code_to_float<BITS, J + 1>(dw), s, b);
+        return affine_weights<T, BITS, 8 * KK + 2 * D, EXACT>(dw, s, b);
     }
 }
 

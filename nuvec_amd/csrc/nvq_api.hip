@@ -188,9 +188,31 @@ static double few_rows_us(const nvq::ProductArgs &a) {
                                  : (exact ? 8.0 + 2.0e-3 * k : 6.0 + 2.05e-3 * k);
     return ceil(blocks / fmax(1.0, (double)nvq::compute_units())) * round_us;
 }
+// The tiled kernels' time as it was estimated when the 128 x 128 tile of qmm_kernel was their small one: what the timings of gated pairs
+// and of up to 32 rows beside the split-K kernel were fitted to.
+static double tiled_before_us(const nvq::ProductArgs &a) {
+    const double cus = fmax(1.0, (double)nvq::compute_units()), steps = (double)((a.k + 63) / 64);
+    auto tiles_us = [&](bool small, double tiles, double each) {
+        return !small ? ceil(tiles / cus) * each * 1.7 : tiles <= cus ? each * 0.8 : ceil(tiles / (2.0 * cus)) * each * 1.2;
+    };
+    auto tiles_of = [&](double t) { return ceil((double)a.m / t) * ceil((double)a.n / t) * (double)a.batch; };
+    const bool small = a.exact_weights || tiles_us(true, tiles_of(128.0), steps) < tiles_us(false, tiles_of(256.0), steps);
+    const double tiles = tiles_of(small ? 128.0 : 256.0), outputs = (double)a.m * (double)a.n;
+    double us = tiles_us(small, tiles, steps);
+    for (double want = 2.0; a.batch == 1 && want <= fmin(8.0, floor(steps / 8.0)); want++) {
+        const double per = 4.0 * ceil(ceil(steps / want) / 4.0), splits = ceil(steps / per);
+        if (splits < 2.0 || (a.k % 64 != 0 && splits * outputs * 4.0 > (double)NVQ_STATIC_SCRATCH_BYTES)) continue;
+        const double split_us = tiles_us(small, tiles * splits, per) + 3.0 + (splits * 4.0 + 2.0) * outputs * 2.0 / 4.0e6;
+        if (split_us < 0.9 * us) us = split_us;
+    }
+    return a.exact_weights ? 1.8 + 1.26 * us : a.mode == NVQ_MXFP4 ? 3.2 + 0.73 * us : 3.4 + us;
+}
+// The plan's estimate with the margin that 900 products of 17 to 2048 rows, timed here and on the kernels they had, leave between it and
+// the others' estimates (1.12 x the speed of those all together, one in 400 more than 5 % slower).  Up to 32 rows, and up to 80 of a
+// short K, the choice stays as it was made: gated pairs of a second pass of few rows are checked beside their products there, which have the
+// split-K kernel's bits (NVFP4 W[11444,928] at 70 rows takes 15.5 us there, 10.9 on the tiles).
 static double tiled_us(const nvq::ProductArgs &a) {
-    const double steps_us = nvq::qmm_estimate_us(a);
-    return a.exact_weights ? 1.8 + 1.26 * steps_us : a.mode == NVQ_MXFP4 ? 3.2 + 0.73 * steps_us : 3.4 + steps_us;
+    return a.tiled_before || a.m <= 32 || (a.m <= 80 && a.k < 1100) ? tiled_before_us(a) : 1.15 * nvq::qmm_estimate_us(a);
 }
 static bool tiled_is_faster(const nvq::ProductArgs &a) { return fmax(7.0, tiled_us(a)) < few_rows_us(a); }  // (its fastest launches, at K = 128, take 6 to 7.4 us)
 
@@ -363,6 +385,8 @@ static nvq::ProductArgs product_args(const nvq_qmm_desc *d, int64_t batch) {
         }
     }
     a.batch_ndim = nd;
+    // (the routes of five rows and more, the workspace and the launch ask for the tiled kernels' plan up to six times)
+    if (d->transpose && !a.row_exact && a.m >= 5 && compute_units() > 0 && qmm_supported(a)) qmm_plan_ahead(a);
     return a;
 }
 
@@ -622,7 +646,7 @@ static Route pick_route(const nvq_qmm_desc *d, const ProductArgs &a);
 // few-row kernel or a tenth below the tiles, from 65 rows on most of which stay there; beyond 256 rows it was not timed beside the tiles (150
 // products of the few-row kernel of 257 to 2048 rows, few outputs: 0.79 of the time, one more than 5 % slower).
 static bool split_rows_bid(const ProductArgs &a, Route route, qms::Plan &plan) {
-    if (route != Route::kFewRows && (route != Route::kTiled || a.m > 256)) return false;
+    if (route != Route::kFewRows && (route != Route::kTiled || a.m > 640)) return false;
     return qms_plan(a, plan) && (route == Route::kFewRows ? plan.us < 1.1 * few_rows_us(a) : plan.us < 0.9 * tiled_us(a));
 }
 
@@ -831,6 +855,7 @@ struct OneOfTwo {
 
     OneOfTwo(const nvq_qmm_desc *d, const ProductArgs &pair) : args(pair) {
         args.glu = 0, args.n = pair.n / 2;
+        args.tiled_before = 1;
         route = pick_route(d, args);
         split_bid = split_rows_bid(args, route, split);
     }

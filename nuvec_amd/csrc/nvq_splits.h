@@ -20,7 +20,10 @@ namespace splits {
 struct Product {
     int64_t m, n, k, batch;
     bool row_exact;      // every row takes the split of its one-row product
-    bool exact_weights;  // the tiled kernel of weights stored [N, K]: the small tile
+    bool exact_weights;  // the tiled kernels of weights stored [N, K]: qmk_kernel's tiles
+    // those kernels' microseconds a step: qmk_kernel's 128 x 128, qmm_kernel's 256 x 256 and two of its 128 x 128 on a compute unit
+    float step_us = 0.5f, big_step_us = 1.5f, small_step_us = 0.9f;
+    bool keep_order = false;  // qmm_kernel's tiles only, K whole
 };
 
 struct Plan {
@@ -28,6 +31,7 @@ struct Plan {
     int64_t per_split;  // units per split
     int64_t units;      // all units of K
     double estimate_us; // of the kernel with this plan, where the rule estimates one (else 0)
+    int tile;           // tiled kernels of weights stored [N, K]: a Tile
 };
 
 inline bool every_split_has_a_unit(const Plan &p) {
@@ -38,49 +42,55 @@ inline size_t workspace_bytes(const Plan &p, const Product &a) {
     return p.splits > 1 ? (size_t)p.splits * (size_t)a.batch * (size_t)a.m * (size_t)a.n * sizeof(float) : 0;
 }
 
-// ── the tiled kernel of weights stored [N, K] (qmm_kernel) ──────────────────────────────────────────────────────────
-constexpr int kQmmStep = 64;                     // values of K per step
-constexpr int kQmmBigTile = 256, kQmmSmallTile = 128;  // square tiles of y
+// ── the tiled kernels of weights stored [N, K] (qmm_kernel, qmk_kernel) ─────────────────────────────────────────────
+constexpr int kQmmStep = 64;  // values of K per step; qmk_kernel takes two at a time
+constexpr int kQmmBigTile = 256, kQmmSmallTile = 128, kQmkFewRows = 64;
+enum Tile { kBig, kQmk128, kQmk64, kSmall };  // qmm_kernel's 256 x 256; qmk_kernel's 128 x 128 and 64 x 128; qmm_kernel's 128 x 128
 
-// Estimated microseconds of `tiles` tiles walking `steps` steps on `cus` compute units, from the kernel's measured
-// behaviour: about 1.7 us per step for the big tile (one block per compute unit); the small tile takes 0.8 us per
-// step alone on a compute unit and 1.2 us when two share it.
-inline double qmm_tiles_us(bool small, double tiles, double steps, int cus) {
-    if (!small) return ceil(tiles / cus) * steps * 1.7;
-    if (tiles <= cus) return steps * 0.8;
-    return ceil(tiles / (2.0 * cus)) * steps * 1.2;
+inline int64_t qmm_tiles(const Product &a, int tile) {
+    const int64_t rows = tile == kBig ? kQmmBigTile : tile == kQmk64 ? kQmkFewRows : kQmmSmallTile, cols = tile == kBig ? kQmmBigTile : kQmmSmallTile;
+    return (a.m + rows - 1) / rows * ((a.n + cols - 1) / cols) * a.batch;
 }
-inline double qmm_estimate_us(bool small, const Product &a, int cus) {
-    const int64_t t = small ? kQmmSmallTile : kQmmBigTile;
-    const double tiles = (double)((a.m + t - 1) / t) * (double)((a.n + t - 1) / t) * (double)a.batch;
-    return qmm_tiles_us(small, tiles, (double)((a.k + kQmmStep - 1) / kQmmStep), cus);
-}
-inline bool qmm_small_tile_is_faster(const Product &a, int cus) {
-    return a.exact_weights || qmm_estimate_us(true, a, cus) < qmm_estimate_us(false, a, cus);
+// Estimated microseconds of `tiles` tiles walking `steps` steps on `cus` compute units, a block each, in `splits` parts of K whose sums a
+// second kernel adds up.  Fitted to 4100 timings of 540 products (17 to 2048 rows, W[256..16384, 512..14336], all formats of 16-bit
+// elements, one to six parts): 13 % off on average for qmk_kernel's tiles, 7 % for the 256 x 256 tile; choosing by it costs 2 % against
+// always taking the fastest.  Beyond the K that was timed qmk_kernel is taken for twice as slow, as the kernel before it was.
+inline float qmm_tiles_us(const Product &a, int tile, int64_t tiles, int64_t steps, int splits, int cus) {
+    const float outputs = 1.0e-6f * (float)(a.m * a.n * a.batch), walked = (float)((tiles + cus - 1) / cus) * (float)steps;
+    if (tile == kBig) return 12.1f + walked * a.big_step_us + 0.6f * outputs + (splits > 1 ? 1.8f + 0.95f * splits * outputs : 0.0f);
+    if (tile == kSmall) return 3.7f + (float)((tiles + 2 * cus - 1) / (2 * cus)) * (float)steps * a.small_step_us + 1.4f * outputs;
+    const float step = a.step_us * (tile == kQmk128 ? 1.0f : 0.85f) * (a.k > 14336 ? 2.0f : 1.0f);
+    return (tile == kQmk128 ? 5.7f : 4.0f) + walked * step + 2.0f * outputs + (splits > 1 ? 2.2f + 2.0f * splits * outputs : 0.0f);
 }
 
-// The splits fill the chip's block slots with its (few) tiles, and cost a second kernel that reads their float32
-// partial sums (about 3 us to launch and 4 bytes per microsecond and compute unit... in all: 4 TB/s).  Each split has
-// at least eight steps, in whole table periods (four steps); at most eight splits; a batch is never split.  K of steps and a half
-// is split as far as the library's own scratch holds the partial sums: the entry point without a workspace takes every such product
-// and gives the bits of the one with a workspace (K of whole steps beyond that scratch it refuses).
+// The tile and the split of K with the least estimated time.  The splits fill the compute units with few tiles.  Each split has at least
+// eight steps, in whole windows and table periods (four steps); at most eight splits; a batch is never split.  K of steps and a half is
+// split as far as the library's own scratch holds the partial sums: the entry point without a workspace takes every such product and gives
+// the bits of the one with a workspace (K of whole steps beyond that scratch it refuses).
 inline Plan qmm_plan(const Product &a, int cus) {
+    if (cus < 1) cus = 1;
     const int64_t steps = (a.k + kQmmStep - 1) / kQmmStep;  // (the last one may be a half)
-    const bool small = qmm_small_tile_is_faster(a, cus);
-    Plan p{1, steps, steps, qmm_estimate_us(small, a, cus)};
-    if (a.batch != 1) return p;
-    const int64_t t = small ? kQmmSmallTile : kQmmBigTile;
-    const double tiles = (double)(((a.m + t - 1) / t) * ((a.n + t - 1) / t));
-    for (int want = 2; want <= 8 && want <= steps / 8; want++) {
-        const int64_t per = (((steps + want - 1) / want) + 3) & ~(int64_t)3;  // whole table periods
-        const int splits = (int)((steps + per - 1) / per);                    // every split has a step
-        if (splits < 2) continue;
-        if (a.k % kQmmStep != 0 && (double)splits * (double)a.m * (double)a.n * 4.0 > (double)NVQ_STATIC_SCRATCH_BYTES) continue;
-        const double reduce_us = 3.0 + ((double)splits * 4.0 + 2.0) * (double)a.m * (double)a.n * 2.0 / 4.0e6;  // written, then read
-        const double us = qmm_tiles_us(small, tiles * splits, (double)per, cus) + reduce_us;
-        if (us < 0.9 * p.estimate_us) p.estimate_us = us, p.splits = splits, p.per_split = per;
+    Plan best{0, 0, 0, 0.0, 0};
+    for (const int tile : {kBig, kQmk128, kQmk64, kSmall}) {
+        const int64_t tiles = qmm_tiles(a, tile);
+        if (tile == kBig && a.exact_weights) continue;
+        // (two of these tiles share a compute unit; alone there qmk_kernel's are faster.  The CPU's weights: single products of whole steps.)
+        if (a.keep_order && (tile == kQmk128 || tile == kQmk64)) continue;
+        if (tile == kSmall && ((tiles <= cus && !a.keep_order) || (a.exact_weights && (a.batch != 1 || a.k % kQmmStep != 0)))) continue;
+        Plan p{1, steps, steps, qmm_tiles_us(a, tile, tiles, steps, 1, cus), tile};
+        const int64_t most = a.batch == 1 && !a.keep_order && tiles < 2 * cus && tile != kSmall ? steps / 8 : 1;  // (more tiles fill the chip as they are)
+        for (int want = 2; want <= 8 && want <= most; want++) {
+            const int64_t per = ((steps + want - 1) / want + 3) & ~(int64_t)3;
+            const int splits = (int)((steps + per - 1) / per);  // every split has a step
+            if (splits < 2) continue;
+            if (a.k % kQmmStep != 0 && (double)splits * (double)a.m * (double)a.n * 4.0 > (double)NVQ_STATIC_SCRATCH_BYTES) continue;
+            const float us = qmm_tiles_us(a, tile, tiles * splits, per, splits, cus);
+            if (us < 0.95f * (float)p.estimate_us) p.estimate_us = us, p.splits = splits, p.per_split = per;
+            if (tiles * splits >= 2 * cus) break;
+        }
+        if (best.splits == 0 || p.estimate_us < best.estimate_us) best = p;
     }
-    return p;
+    return best;
 }
 
 // ── the matrix-core kernel of weights stored [K, N] (qmn_kernel) ────────────────────────────────────────────────────
@@ -96,7 +106,7 @@ inline Plan qmn_plan(const Product &a, int cus, bool few_rows) {
     const int64_t bm = few_rows ? kQmnFewRows : kQmnManyRows;
     const int64_t tiles = ((a.m + bm - 1) / bm) * ((a.n + kQmnTileCols - 1) / kQmnTileCols) * a.batch, steps = a.k / kQmnStep;
     const int64_t resident = (int64_t)(few_rows ? kQmnFewBlocksPerCu : kQmnManyBlocksPerCu) * cus;
-    Plan p{1, steps < 1 ? 1 : steps, steps, 0.0};
+    Plan p{1, steps < 1 ? 1 : steps, steps, 0.0, 0};
     if (tiles >= resident || steps < 4) return p;
     const double step_us = few_rows ? 0.64 : 1.2;
     for (int64_t splits = 1; splits <= steps / 2 && splits <= 64; splits++) {
@@ -127,7 +137,7 @@ inline Plan qvm_plan(const Product &a, int cus) {
     if (per < 1) per = 1;
     splits = (a.k + per - 1) / per;  // the count that this longest split gives: no split is left without a row
     if (splits < 1) splits = 1;
-    return Plan{(int)splits, per, a.k, 0.0};
+    return Plan{(int)splits, per, a.k, 0.0, 0};
 }
 
 }  // namespace splits

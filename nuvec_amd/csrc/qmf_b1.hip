@@ -1,11 +1,11 @@
 // The few-row and tiled matrix-core kernels for affine 1-bit codes (qmf_kernel.h, qmm_kernel.h).
 #include "qmf_kernel.h"
-#include "qmm_kernel.h"
+#include "qmk_kernel.h"
 
 namespace nvq {
 
 int32_t launch_qmf_b1(const ProductArgs &a, hipStream_t s) { return qmf::run_dtype<1, false>(a, s); }
 
-int32_t launch_qmm_b1(const ProductArgs &a, void *workspace, hipStream_t s) { return qmm::run_dtype<1, false>(a, workspace, s); }
+int32_t launch_qmm_b1(const ProductArgs &a, void *workspace, hipStream_t s) { return run_tiled<1, false>(a, workspace, s); }
 
 }  // namespace nvq

@@ -16,17 +16,24 @@ bool qmm_supported(const ProductArgs &a) {
     return a.batch <= 65535 && a.k >= qmm::BK && (a.k % qmm::BK == 0 || qmf::half_steps_supported(a));
 }
 
-// With its better tile and, for a single product, its better split of K (the caller is expected to bring the
-// workspace the size query names).
-double qmm_estimate_us(const ProductArgs &a) {
-    double us = 0.0;
-    qmm::k_splits(a, compute_units(), nullptr, &us);
-    return us;
+splits::Plan qmm_plan_of(const ProductArgs &a) {
+    if (a.tiled.splits > 0) return splits::Plan{a.tiled.splits, a.tiled.per_split, (a.k + qmm::BK - 1) / qmm::BK, a.tiled.us, a.tiled.tile};
+    return splits::qmm_plan(qmm::split_product(a), compute_units());
 }
 
+void qmm_plan_ahead(ProductArgs &a) {
+    const splits::Plan p = splits::qmm_plan(qmm::split_product(a), compute_units());
+    a.tiled = {p.splits, (int32_t)p.per_split, p.tile, (float)p.estimate_us};
+}
+
+// With its better tile and, for a single product, its better split of K (the caller is expected to bring the
+// workspace the size query names).
+double qmm_estimate_us(const ProductArgs &a) { return qmm_plan_of(a).estimate_us; }
+
 size_t qmm_workspace_bytes(const ProductArgs &a) {
-    const int splits = qmm::k_splits(a, compute_units());
-    return splits > 1 ? (size_t)splits * (size_t)a.m * (size_t)a.n * sizeof(float) : 0;
+    const splits::Plan p = qmm_plan_of(a);
+    if (qmm_dense_takes(a)) return 0;  // (run_tiled)
+    return p.splits > 1 ? (size_t)p.splits * (size_t)a.m * (size_t)a.n * sizeof(float) : 0;
 }
 
 int32_t launch_qmm(const ProductArgs &a, void *workspace, hipStream_t s) {

@@ -160,11 +160,8 @@ bool qmm_dense_takes(const ProductArgs &a) {
         return false;
     if (a.k < BK || a.k % BK != 0 || a.k > 1 << 22 || (a.m + 127) / 128 > 65535) return false;  // (32-bit offsets in a tile)
     if (a.n * a.k > kMostWeights) return false;
-    // Where that kernel splits K it stays: its sums and this kernel's, in one order otherwise, would differ in their last bits, and the
-    // entry point that brings no workspace promises the bits of the one that does.
-    if (qmm_workspace_bytes(a) != 0) return false;
     const double here = 7.0 + 0.48e-6 * (double)a.n * (double)a.k + fmin(product_us<Small>(a), product_us<Big>(a));
-    return here < 0.9 * (1.8 + 1.26 * qmm_estimate_us(a));
+    return here < 0.95 * qmm_estimate_us(a);
 }
 
 int32_t launch_qmm_dense(const ProductArgs &a, void *workspace, hipStream_t s) {

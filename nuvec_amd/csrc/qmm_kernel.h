@@ -7,8 +7,9 @@
 // (crates/nuvec-kernels/src/metal/quantized.h:583-817, 1358-1485).
 //
 // One block of 256 threads (four wavefronts, one per SIMD, each 256 x 64 of y in 256 accumulator registers) owns a
-// BM x BN = 256 x 256 tile and walks K in steps of BK = 64 through a ring of three LDS stages (products whose
-// 256 x 256 tiles would not fill the chip take 128 x 128 tiles of 2 x 2 wavefronts, two blocks per compute unit).
+// BM x BN = 256 x 256 tile and walks K in steps of BK = 64 through a ring of three LDS stages.  (Products whose 256 x 256 tiles would
+// not fill the chip take qmk_kernel's, or between one and two rounds of those 128 x 128 tiles of 2 x 2 wavefronts here, two blocks
+// per compute unit: 258 rows, W[16291,1408] of MXFP4 23.9 us, 31.1 there.)
 // A wavefront covers all rows of the tile, so every weight is expanded once per block.  A stage holds
 //   * the x tile, 256 rows x 128 B, 16-byte chunk index XOR-ed with (row >> 1) & 7 so that the 16-byte
 //     fragment reads of the matrix instruction are free of conflicts on the 64 LDS banks, and
@@ -57,7 +58,7 @@ struct Tile {
                   "the loading assignment below assumes these");
 };
 using BigTile = Tile<1, 4, 8, 2>;    // 256 x 256, 256 threads: one wavefront per SIMD owns 256 x 64, no code is expanded twice
-using SmallTile = Tile<2, 2, 2, 2>;  // 128 x 128, 256 threads, two blocks per compute unit: for products whose big tiles would not fill the chip
+using SmallTile = Tile<2, 2, 2, 2>;  // 128 x 128, 256 threads, two blocks per compute unit
 
 // How a lane's BITS dwords travel into LDS: one or two pieces of 4, 3 or 1 dwords.
 template <int BITS> struct Pieces;
@@ -479,67 +480,69 @@ __global__ void __launch_bounds__(256) qmm_reduce_kernel(const float *__restrict
     }
 }
 
-// Tile choice and the split of K over the grid: the host rules of nvq_splits.h, here bound to this kernel's constants.
+// The host rules of nvq_splits.h, here bound to this kernel's constants.
 static_assert(BK == splits::kQmmStep && BigTile::BM == splits::kQmmBigTile && BigTile::BN == splits::kQmmBigTile &&
               SmallTile::BM == splits::kQmmSmallTile && SmallTile::BN == splits::kQmmSmallTile, "nvq_splits.h describes these tiles");
+// What the rules need to know: among it the measured microseconds a step of the tiles (qmm_tiles_us), which the expansion of the codes
+// decides, two roundings a weight above all.
 inline splits::Product split_product(const ProductArgs &a) {
-    return splits::Product{a.m, a.n, a.k, a.batch, a.row_exact != 0, a.exact_weights != 0};
+    const bool f16 = a.dtype == NVQ_F16, odd = a.bits == 3 || a.bits == 5 || a.bits == 6;
+    splits::Product p{a.m, a.n, a.k, a.batch, a.row_exact != 0, a.exact_weights != 0};
+    if (a.mode == NVQ_MXFP4) p.step_us = 0.39f, p.big_step_us = 1.22f, p.small_step_us = 0.69f;
+    else if (a.mode == NVQ_MXFP8) p.step_us = 0.43f, p.big_step_us = 1.3f, p.small_step_us = 0.76f;
+    else if (a.mode == NVQ_NVFP4) p.step_us = 0.42f, p.big_step_us = 1.53f, p.small_step_us = 0.94f;
+    else if (a.exact_weights) p.step_us = (f16 ? 0.5f : 0.57f) + (odd ? 0.1f : 0.0f), p.small_step_us = 1.3f;
+    else if (odd) p.step_us = 0.59f, p.big_step_us = 1.55f, p.small_step_us = 1.13f;
+    else p.step_us = 0.48f, p.big_step_us = 1.34f, p.small_step_us = 0.9f;
+    // (one of a gated pair of few rows and a short K sums in the order it is compared in: before a bias that nearly cancels a product,
+    // another order's rounding is many units of the sum)
+    p.keep_order = a.mode == NVQ_AFFINE && !a.exact_weights && a.m <= 80 && a.k < 1100;
+    return p;
 }
-inline bool small_tile_is_faster(const ProductArgs &a, int cus) { return splits::qmm_small_tile_is_faster(split_product(a), cus); }
-// How many ways a single product splits K over the grid (1: no split), the steps of a split, the estimated duration.
-inline int k_splits(const ProductArgs &a, int cus, int *steps_per_split = nullptr, double *estimate = nullptr) {
-    const splits::Plan p = splits::qmm_plan(split_product(a), cus);
-    if (steps_per_split != nullptr) *steps_per_split = (int)p.per_split;
-    if (estimate != nullptr) *estimate = p.estimate_us;
-    return p.splits;
+
+// The partial sums of a split product added up.
+template <typename T>
+int32_t run_reduce(const ProductArgs &a, hipStream_t s) {
+    const int64_t total = a.m * a.n;
+    hipLaunchKernelGGL((qmm_reduce_kernel<T>), dim3((unsigned)((total / 4 + 256) / 256)), dim3(256), 0, s, a.partials, (T *)a.y, a.k_splits, total, a.row_bias, a.n);
+    NVQ_LAUNCH_CHECK("qmm_reduce");
+    return NVQ_OK;
 }
 
 template <typename T, int BITS, int FP4, class TL, bool EXACT, bool HALF>
-int32_t run_tile_of(ProductArgs a, void *workspace, hipStream_t s) {
+int32_t run_tile_of(ProductArgs a, const splits::Plan &p, void *workspace, hipStream_t s) {
     using G = Geometry<BITS, TL>;
     static std::atomic<bool> configured[2] = {false, false};
-    const bool batched = a.batch > 1;
-    auto kernel = batched ? qmm_kernel<T, BITS, FP4, true, TL, EXACT, HALF> : qmm_kernel<T, BITS, FP4, false, TL, EXACT, HALF>;
+    const bool batched = !EXACT && a.batch > 1;
+    auto kernel = batched ? qmm_kernel<T, BITS, FP4, !EXACT, TL, EXACT, HALF> : qmm_kernel<T, BITS, FP4, false, TL, EXACT, HALF>;
     if (!configured[batched]) {
         NVQ_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, G::kLdsBytes));
         configured[batched] = true;
     }
-    int per = 0;
-    const int splits = workspace != nullptr ? k_splits(a, compute_units(), &per) : 1;
-    if (splits > 1 && (int64_t)(splits - 1) * per >= (a.k + BK - 1) / BK)  // (a block of such a split would leave its partial sums unwritten)
-        return fail(NVQ_BACKEND, "quantized_matmul: %d splits of %d steps leave one without a step of K = %lld", splits, per, (long long)a.k);
-    a.k_splits = splits;
-    a.k_split_steps = per;
-    a.partials = splits > 1 ? static_cast<float *>(workspace) : nullptr;
-    dim3 grid((unsigned)((a.n + TL::BN - 1) / TL::BN), (unsigned)((a.m + TL::BM - 1) / TL::BM), (unsigned)(batched ? a.batch : splits));
+    a.k_splits = workspace != nullptr ? p.splits : 1;
+    a.k_split_steps = (int)p.per_split;
+    a.partials = a.k_splits > 1 ? static_cast<float *>(workspace) : nullptr;
+    const dim3 grid((unsigned)((a.n + TL::BN - 1) / TL::BN), (unsigned)((a.m + TL::BM - 1) / TL::BM), (unsigned)(batched ? a.batch : a.k_splits));
     hipLaunchKernelGGL(kernel, grid, dim3(TL::kThreads), G::kLdsBytes, s, a);
     NVQ_LAUNCH_CHECK("qmm");
-    if (splits > 1) {
-        const int64_t total = a.m * a.n;
-        hipLaunchKernelGGL((qmm_reduce_kernel<T>), dim3((unsigned)((total / 4 + 256) / 256)), dim3(256), 0, s, a.partials, (T *)a.y, splits, total, a.row_bias, a.n);
-        NVQ_LAUNCH_CHECK("qmm_reduce");
-    }
-    return NVQ_OK;
-}
-
-template <typename T, int BITS, int FP4, class TL, bool EXACT = false>
-int32_t run_tile(const ProductArgs &a, void *workspace, hipStream_t s) {
-    if constexpr (FP4 != kAffine || EXACT)  // (half_steps_supported)
-        if (a.k % BK != 0) return run_tile_of<T, BITS, FP4, TL, EXACT, true>(a, workspace, s);
-    return run_tile_of<T, BITS, FP4, TL, EXACT, false>(a, workspace, s);
+    return a.k_splits > 1 ? run_reduce<T>(a, s) : NVQ_OK;
 }
 
 template <typename T, int BITS, int FP4>
-int32_t run(const ProductArgs &a, void *workspace, hipStream_t s) {
-    if constexpr (FP4 == kAffine)
-        if (a.exact_weights) return run_tile<T, BITS, FP4, SmallTile, true>(a, workspace, s);  // (rows of few outputs: the small tile)
-    return small_tile_is_faster(a, compute_units()) ? run_tile<T, BITS, FP4, SmallTile>(a, workspace, s)
-                                                    : run_tile<T, BITS, FP4, BigTile>(a, workspace, s);
+int32_t run(const ProductArgs &a, const splits::Plan &p, void *workspace, hipStream_t s) {
+    const bool big = p.tile == splits::kBig;
+    if constexpr (FP4 != kAffine) {
+        if (a.k % BK != 0)  // (half_steps_supported)
+            return big ? run_tile_of<T, BITS, FP4, BigTile, false, true>(a, p, workspace, s) : run_tile_of<T, BITS, FP4, SmallTile, false, true>(a, p, workspace, s);
+    } else {
+        if (a.exact_weights) return run_tile_of<T, BITS, FP4, SmallTile, true, false>(a, p, workspace, s);  // (run_tiled)
+    }
+    return big ? run_tile_of<T, BITS, FP4, BigTile, false, false>(a, p, workspace, s) : run_tile_of<T, BITS, FP4, SmallTile, false, false>(a, p, workspace, s);
 }
 
 template <int BITS, int FP4>
-int32_t run_dtype(const ProductArgs &a, void *workspace, hipStream_t s) {
-    return a.dtype == NVQ_BF16 ? run<bf16_t, BITS, FP4>(a, workspace, s) : run<f16_t, BITS, FP4>(a, workspace, s);
+int32_t run_dtype(const ProductArgs &a, const splits::Plan &p, void *workspace, hipStream_t s) {
+    return a.dtype == NVQ_BF16 ? run<bf16_t, BITS, FP4>(a, p, workspace, s) : run<f16_t, BITS, FP4>(a, p, workspace, s);
 }
 
 }  // namespace qmm

@@ -10,6 +10,7 @@
 #include <mutex>
 
 #include "nvq_internal.h"
+#include "nvq_splits.h"
 
 #include <math.h>
 
@@ -191,21 +192,9 @@ static double few_rows_us(const nvq::ProductArgs &a) {
 // The tiled kernels' time as it was estimated when the 128 x 128 tile of qmm_kernel was their small one: what the timings of gated pairs
 // and of up to 32 rows beside the split-K kernel were fitted to.
 static double tiled_before_us(const nvq::ProductArgs &a) {
-    const double cus = fmax(1.0, (double)nvq::compute_units()), steps = (double)((a.k + 63) / 64);
-    auto tiles_us = [&](bool small, double tiles, double each) {
-        return !small ? ceil(tiles / cus) * each * 1.7 : tiles <= cus ? each * 0.8 : ceil(tiles / (2.0 * cus)) * each * 1.2;
-    };
-    auto tiles_of = [&](double t) { return ceil((double)a.m / t) * ceil((double)a.n / t) * (double)a.batch; };
-    const bool small = a.exact_weights || tiles_us(true, tiles_of(128.0), steps) < tiles_us(false, tiles_of(256.0), steps);
-    const double tiles = tiles_of(small ? 128.0 : 256.0), outputs = (double)a.m * (double)a.n;
-    double us = tiles_us(small, tiles, steps);
-    for (double want = 2.0; a.batch == 1 && want <= fmin(8.0, floor(steps / 8.0)); want++) {
-        const double per = 4.0 * ceil(ceil(steps / want) / 4.0), splits = ceil(steps / per);
-        if (splits < 2.0 || (a.k % 64 != 0 && splits * outputs * 4.0 > (double)NVQ_STATIC_SCRATCH_BYTES)) continue;
-        const double split_us = tiles_us(small, tiles * splits, per) + 3.0 + (splits * 4.0 + 2.0) * outputs * 2.0 / 4.0e6;
-        if (split_us < 0.9 * us) us = split_us;
-    }
-    return a.exact_weights ? 1.8 + 1.26 * us : a.mode == NVQ_MXFP4 ? 3.2 + 0.73 * us : 3.4 + us;
+    const splits::Product p{a.m, a.n, a.k, a.batch, a.row_exact != 0, a.exact_weights != 0};
+    const double steps_us = splits::qmm_plan_before(p, nvq::compute_units() < 1 ? 1 : nvq::compute_units()).estimate_us;
+    return a.exact_weights ? 1.8 + 1.26 * steps_us : a.mode == NVQ_MXFP4 ? 3.2 + 0.73 * steps_us : 3.4 + steps_us;
 }
 // The plan's estimate with the margin that 900 products of 17 to 2048 rows, timed here and on the kernels they had, leave between it and
 // the others' estimates (1.12 x the speed of those all together, one in 400 more than 5 % slower).  Up to 32 rows, and up to 80 of a
@@ -643,7 +632,7 @@ enum class Route { kUntransposed, kVector, kTiled, kTiledF32, kGroupedRows, kBat
 static Route pick_route(const nvq_qmm_desc *d, const ProductArgs &a);
 
 // Whether the split-K kernel is a candidate for a product of either matrix-core route of 16-bit rows: estimated up to a tenth above the
-// few-row kernel or a tenth below the tiles, from 65 rows on most of which stay there; beyond 256 rows it was not timed beside the tiles (150
+// few-row kernel or a tenth below the tiles, whose estimate has a margin of its own; beyond 640 rows it was not timed beside the tiles (150
 // products of the few-row kernel of 257 to 2048 rows, few outputs: 0.79 of the time, one more than 5 % slower).
 static bool split_rows_bid(const ProductArgs &a, Route route, qms::Plan &plan) {
     if (route != Route::kFewRows && (route != Route::kTiled || a.m > 640)) return false;
@@ -856,6 +845,7 @@ struct OneOfTwo {
     OneOfTwo(const nvq_qmm_desc *d, const ProductArgs &pair) : args(pair) {
         args.glu = 0, args.n = pair.n / 2;
         args.tiled_before = 1;
+        args.tiled.splits = 0;  // (the pair's plan)
         route = pick_route(d, args);
         split_bid = split_rows_bid(args, route, split);
     }

@@ -51,29 +51,57 @@ inline int64_t qmm_tiles(const Product &a, int tile) {
     const int64_t rows = tile == kBig ? kQmmBigTile : tile == kQmk64 ? kQmkFewRows : kQmmSmallTile, cols = tile == kBig ? kQmmBigTile : kQmmSmallTile;
     return (a.m + rows - 1) / rows * ((a.n + cols - 1) / cols) * a.batch;
 }
+// The plan as it was made when qmm_kernel's 128 x 128 tile (0.8 us a step alone on a compute unit, 1.2 where two share it) stood where
+// qmk_kernel's does: by whole tiles first, then the split of that tile.  What gated pairs and up to 32 rows were timed beside, and the plan of
+// K beyond 14336, the longest that was timed since.
+inline Plan qmm_plan_before(const Product &a, int cus) {
+    const int64_t steps = (a.k + kQmmStep - 1) / kQmmStep;
+    auto tiles_us = [&](int tile, double tiles, double each) {
+        return tile == kBig ? ceil(tiles / cus) * each * 1.7 : tiles <= cus ? each * 0.8 : ceil(tiles / (2.0 * cus)) * each * 1.2;
+    };
+    const double big = tiles_us(kBig, (double)qmm_tiles(a, kBig), (double)steps), small = tiles_us(kQmk128, (double)qmm_tiles(a, kQmk128), (double)steps);
+    const int tile = a.exact_weights || small < big ? kQmk128 : kBig;
+    const double tiles = (double)qmm_tiles(a, tile), outputs = (double)a.m * (double)a.n;
+    Plan p{1, steps, steps, tile == kBig ? big : small, tile};
+    for (int want = 2; a.batch == 1 && want <= 8 && want <= steps / 8; want++) {
+        const int64_t per = ((steps + want - 1) / want + 3) & ~(int64_t)3;
+        const int splits = (int)((steps + per - 1) / per);  // every split has a step
+        if (splits < 2 || (a.k % kQmmStep != 0 && (double)splits * outputs * 4.0 > (double)NVQ_STATIC_SCRATCH_BYTES)) continue;
+        const double us = tiles_us(tile, tiles * splits, (double)per) + 3.0 + ((double)splits * 4.0 + 2.0) * outputs * 2.0 / 4.0e6;
+        if (us < 0.9 * p.estimate_us) p.estimate_us = us, p.splits = splits, p.per_split = per;
+    }
+    return p;
+}
+
 // Estimated microseconds of `tiles` tiles walking `steps` steps on `cus` compute units, a block each, in `splits` parts of K whose sums a
 // second kernel adds up.  Fitted to 4100 timings of 540 products (17 to 2048 rows, W[256..16384, 512..14336], all formats of 16-bit
 // elements, one to six parts): 13 % off on average for qmk_kernel's tiles, 7 % for the 256 x 256 tile; choosing by it costs 2 % against
-// always taking the fastest.  Beyond the K that was timed qmk_kernel is taken for twice as slow, as the kernel before it was.
+// always taking the fastest.
 inline float qmm_tiles_us(const Product &a, int tile, int64_t tiles, int64_t steps, int splits, int cus) {
     const float outputs = 1.0e-6f * (float)(a.m * a.n * a.batch), walked = (float)((tiles + cus - 1) / cus) * (float)steps;
     if (tile == kBig) return 12.1f + walked * a.big_step_us + 0.6f * outputs + (splits > 1 ? 1.8f + 0.95f * splits * outputs : 0.0f);
     if (tile == kSmall) return 3.7f + (float)((tiles + 2 * cus - 1) / (2 * cus)) * (float)steps * a.small_step_us + 1.4f * outputs;
-    const float step = a.step_us * (tile == kQmk128 ? 1.0f : 0.85f) * (a.k > 14336 ? 2.0f : 1.0f);
+    const float step = a.step_us * (tile == kQmk128 ? 1.0f : 0.85f);
     return (tile == kQmk128 ? 5.7f : 4.0f) + walked * step + 2.0f * outputs + (splits > 1 ? 2.2f + 2.0f * splits * outputs : 0.0f);
 }
 
 // The tile and the split of K with the least estimated time.  The splits fill the compute units with few tiles.  Each split has at least
-// eight steps, in whole windows and table periods (four steps); at most eight splits; a batch is never split.  K of steps and a half is
-// split as far as the library's own scratch holds the partial sums: the entry point without a workspace takes every such product and gives
-// the bits of the one with a workspace (K of whole steps beyond that scratch it refuses).
+// eight steps, in whole windows and table periods (four steps); at most eight splits; a batch is never split.  K is split as far as the
+// library's own scratch holds the partial sums, so that the entry point without a workspace refuses no product for it (beyond K = 14336 it
+// refuses those of whole steps that it always did).
 inline Plan qmm_plan(const Product &a, int cus) {
     if (cus < 1) cus = 1;
     const int64_t steps = (a.k + kQmmStep - 1) / kQmmStep;  // (the last one may be a half)
+    if (a.k > 14336) {
+        Plan p = qmm_plan_before(a, cus);
+        p.estimate_us = a.exact_weights ? 1.8 + 1.26 * p.estimate_us : 3.4 + p.estimate_us;
+        return p;
+    }
     Plan best{0, 0, 0, 0.0, 0};
     for (const int tile : {kBig, kQmk128, kQmk64, kSmall}) {
-        const int64_t tiles = qmm_tiles(a, tile);
+        const int64_t tiles = qmm_tiles(a, tile), high = (a.m + (tile == kQmk64 ? kQmkFewRows : kQmmSmallTile) - 1) / (tile == kQmk64 ? kQmkFewRows : kQmmSmallTile);
         if (tile == kBig && a.exact_weights) continue;
+        if (tile != kBig && high > 65535 && !(a.exact_weights && tile == kQmk128)) continue;  // (the grid's rows)
         // (two of these tiles share a compute unit; alone there qmk_kernel's are faster.  The CPU's weights: single products of whole steps.)
         if (a.keep_order && (tile == kQmk128 || tile == kQmk64)) continue;
         if (tile == kSmall && ((tiles <= cus && !a.keep_order) || (a.exact_weights && (a.batch != 1 || a.k % kQmmStep != 0)))) continue;
@@ -83,7 +111,7 @@ inline Plan qmm_plan(const Product &a, int cus) {
             const int64_t per = ((steps + want - 1) / want + 3) & ~(int64_t)3;
             const int splits = (int)((steps + per - 1) / per);  // every split has a step
             if (splits < 2) continue;
-            if (a.k % kQmmStep != 0 && (double)splits * (double)a.m * (double)a.n * 4.0 > (double)NVQ_STATIC_SCRATCH_BYTES) continue;
+            if ((double)splits * (double)a.m * (double)a.n * 4.0 > (double)NVQ_STATIC_SCRATCH_BYTES) break;
             const float us = qmm_tiles_us(a, tile, tiles * splits, per, splits, cus);
             if (us < 0.95f * (float)p.estimate_us) p.estimate_us = us, p.splits = splits, p.per_split = per;
             if (tiles * splits >= 2 * cus) break;

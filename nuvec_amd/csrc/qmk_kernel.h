@@ -14,9 +14,8 @@
 // wavefront, two wavefronts a SIMD, beside 16 matrix instructions that cost the issue 14 cycles each: 3080 cycles a window, of which the
 // matrix cores are busy 1024), a block's first loads and the exchange of the sums, 5 us of a short K.  A substep's operands are prepared under
 // the matrix instructions of the one before (5 % against a window's reads, expansion and products one after the other).
-// us, before -> here: 490 rows, W[804,640] of 3 bits 21.0 -> 9.6; 413 rows, W[766,1184] of MXFP8 16.2 -> 10.1; 46 rows, W[13247,6688] of
-// NVFP4 48 -> 31; 445 rows, W[2150,1280] of 4 bits 22.4 -> 12.4; 66 rows, W[16212,4992] of 3 bits 47.9 -> 36.4.  400 products of 17 to 2048
-// rows: 0.89 of the time all together.
+// us, before -> here: 445 rows, W[2150,1280] of 4 bits 22.4 -> 12.4; 46 rows, W[13247,6688] of NVFP4 48 -> 31; 66 rows, W[16212,4992] of 3
+// bits 47.9 -> 36.4; 455 rows, W[8250,7360] of 3 bits 143 -> 89.  400 products of 17 to 2048 rows: 0.89 of the time all together.
 #pragma once
 
 #include "qmm_kernel.h"

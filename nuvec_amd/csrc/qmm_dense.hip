@@ -2,17 +2,18 @@
 // crates/nuvec-core/src/kernels.rs:835-859; product kernels.rs:1091-1142): the weight is dequantized once into a workspace
 // (affine_dequantize_kernel) and multiplied densely, in bfloat16 or float16 on v_mfma_f32_32x32x16.
 //
-// The tiled kernel that expands codes itself (qmm_kernel.h) does so for every 128 rows of x and twice in a block, and two
-// roundings a weight make it bound by the vector unit: 517 rows, W[4096,4096] of 3 bits, 73 us = 237 TFLOP/s.  A weight of N x K
-// costs 2 N K bytes written and, from the chip's last cache, read.
+// The tiled kernel that expands codes itself (qmk_kernel.h) does so for every 128 rows of x, and two roundings a weight make it bound by
+// the vector unit: 517 rows, W[4096,4096] of 3 bits, 47.5 us.  A weight of N x K costs 2 N K bytes written and, from the chip's last
+// cache, read.
 //
 // A block of four wavefronts owns BM x 128 of y, 128 or 256 rows of x, each wavefront BM / 2 x 64, and walks K in steps of 64
 // through a ring of LDS stages that both operands reach by direct loads, as many as fit; layout, swizzle and order of K are
 // those of qmm_kernel.h, whose x tile is either operand here.  Bound by LDS reads: one operand of 16 bytes a lane per matrix
 // instruction at 128 rows, three per four at 256 (a step takes 0.5 and 0.85 us; operands laid out tile by tile beforehand, so
-// that a load is 1 KB of consecutive bytes, took 0.55).
-// us, 4 bits, bfloat16, codes expanded in the product -> here: W[4096,4096] at 517 / 1024 / 2048 rows 68 / 70 / 115 -> 42 / 51 / 75
-// (3 bits at 517 rows 73 -> 41), W[8000,4096] at 517 rows 108 -> 73, W[6144,8192] at 768 rows 200 -> 120.
+// that a load is 1 KB of consecutive bytes, took 0.55; eight wavefronts with a quarter of every window each, the two of a SIMD reading and
+// multiplying by turns with a barrier each, 0.65).
+// us, 4 bits, bfloat16, codes expanded in the product -> here: W[4096,4096] at 517 / 1024 / 2048 rows 48 / 70 / 115 -> 40 / 51 / 75;
+// 6 bits W[4064,7680] at 1519 rows 163 -> 114.
 #include "qmm_kernel.h"
 
 namespace nvq {
@@ -152,9 +153,10 @@ size_t qmm_dense_workspace_bytes(const ProductArgs &a) { return (size_t)a.n * (s
 // Half a gigabyte of workspace, W[8191,28672] and a little more: a weight that takes the CPU's values has fewer than 8192 rows.
 constexpr int64_t kMostWeights = 1LL << 28;
 
-// Among the products that the tiled kernel takes with the CPU's weights: where the dequantization (7 us of launches and ends of
-// kernels, and 0.48 us per million weights) and the dense product are estimated a tenth below that kernel.  us here / there, where
-// it turns: W[4096,4096] 384 / 517 rows 49 / 43 and 42 / 68; W[1024,4096] 1024 rows 41 / 31; W[576,576] at 517 rows 13 / 11.
+// Among the products that the tiled kernels take with the CPU's weights: where the dequantization (7 us of launches and ends of
+// kernels, and 0.48 us per million weights) and the dense product are estimated a twentieth below those.  us here / there, where
+// it turns: W[4096,4096] 512 / 517 rows 42 / 36 and 40 / 47.5; W[1024,4096] 1024 rows 41 / 24; W[576,576] at 517 rows 13 / 9.
+// (Without a workspace run_tiled sums in this kernel's order.)
 bool qmm_dense_takes(const ProductArgs &a) {
     if (a.mode != NVQ_AFFINE || !a.exact_weights || a.row_exact || a.batch != 1 || a.batch_ndim != 0 || a.rhs != nullptr || a.lhs != nullptr || a.glu != 0)
         return false;

@@ -374,8 +374,9 @@ static nvq::ProductArgs product_args(const nvq_qmm_desc *d, int64_t batch) {
         }
     }
     a.batch_ndim = nd;
-    // (the routes of five rows and more, the workspace and the launch ask for the tiled kernels' plan up to six times)
-    if (d->transpose && !a.row_exact && a.m >= 5 && compute_units() > 0 && qmm_supported(a)) qmm_plan_ahead(a);
+    // (the routes of more than 32 rows, the workspace and the launch ask for the tiled kernels' plan up to six times; fewer rows have
+    // another estimate and few tiled products)
+    if (d->transpose && !a.row_exact && a.m > 32 && compute_units() > 0 && qmm_supported(a)) qmm_plan_ahead(a);
     return a;
 }
 

@@ -260,7 +260,7 @@ def all_configs(lib, device, qs):
             ys = [torch.empty(m, n, dtype=tdtype, device=device) for _ in weights]
             calls = [Product(lib, m, x, q, y, n, k, code, transpose) for q, y in zip(weights, ys)]
             ms = best_of(calls, 600 if m <= 64 else 48)
-            kernel = lib.nvq_quantized_matmul_kernel(C.byref(calls[0].d))  # from the library's routing code
+            kernel = lib.nvq_quantized_matmul_tile(C.byref(calls[0].d))  # from the library's routing code
             gbps, tflops = wbytes / (ms * 1e-3) / 1e9, 2.0 * m * n * k / (ms * 1e-3) / 1e12
             out.append({"config": label, "m": m, "kernel": kernel.decode() if kernel else None, "us_per_launch": ms * 1e3,
                         "weight_gbps": gbps, "tflops": tflops,

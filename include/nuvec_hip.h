@@ -239,8 +239,13 @@ NVQ_API int32_t nvq_dequantize_rows(const nvq_quant *quant, int32_t dtype, const
 NVQ_API const char *nvq_quantized_matmul_route(const nvq_qmm_desc *desc);
 /* The kernel that runs it, given the workspace that the size query names.  It is the route's but for these: products of "qmf_kernel" and
  * "qmm_kernel" may run on "qms_kernel<R,C,G>" (a block holds 16 R rows of x, a wavefront 16 C weight rows, G wavefronts share x), those
- * of "qmm_kernel" on "qmm_dense_kernel", and float32 ones of the vector kernels on "qmm_f32_kernel". */
+ * of "qmm_kernel" on "qmm_dense_kernel", and float32 ones of the vector kernels on "qmm_f32_kernel".  "qmm_kernel" stands for both tiled
+ * kernels that expand codes themselves; the next query tells them apart. */
 NVQ_API const char *nvq_quantized_matmul_kernel(const nvq_qmm_desc *desc);
+/* The same with "qmm_kernel" told apart by the kernel and its tile, rows of x by weight rows: "qmm_kernel<256,256>", "qmm_kernel<128,128>",
+ * "qmk_kernel<128,128>" (each wavefront a quarter of every window of K) or "qmk_kernel<64,128>".  Whether K is split as well is in the size
+ * of the workspace. */
+NVQ_API const char *nvq_quantized_matmul_tile(const nvq_qmm_desc *desc);
 /* Bytes of scratch nvq_quantized_matmul needs for `desc` (the reference allocates them on its side of the boundary, gpu.rs:7562; the
  * counterpart of its qmm_t_splitk, gpu.rs:7507-7590).  0 = none; nonzero where K is split over the grid (float32 partial sums): transpose = 0,
  * and transpose = 1 products of a few to many rows, float32 ones among them, with few output tiles; and for many rows of 16 bits the

@@ -102,6 +102,7 @@ SIGNATURES = {
                                                 C.c_void_p, C.c_void_p]),
     "nvq_quantized_matmul_route": (C.c_char_p, [C.POINTER(QmmDescC)]),
     "nvq_quantized_matmul_kernel": (C.c_char_p, [C.POINTER(QmmDescC)]),
+    "nvq_quantized_matmul_tile": (C.c_char_p, [C.POINTER(QmmDescC)]),
     "nvq_quantized_attention_workspace_bytes": (C.c_size_t, [C.POINTER(AttentionDescC)]),
     "nvq_quantized_attention": (C.c_int32, [C.POINTER(AttentionDescC)] + [C.c_void_p] * 11),
     "nvq_quantized_attention_prompt_workspace_bytes": (C.c_size_t, [C.POINTER(AttentionPromptDescC)]),

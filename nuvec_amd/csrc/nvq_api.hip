@@ -751,8 +751,10 @@ static int32_t quantized_matmul_any(const nvq_qmm_desc *d, const void *x, const 
     }
 }
 
-// The names of a product's route and of the kernel that runs it; `kernel` alone looks beyond the route.
-static const char *name_of(const nvq_qmm_desc *d, bool kernel) {
+// The names of a product's route, of the kernel that runs it, and of that with the tile of the tiled kernels: each looks further.
+enum class Name { kRoute, kKernel, kTile };
+static const char *name_of(const nvq_qmm_desc *d, Name name) {
+    const bool kernel = name != Name::kRoute;
     if (check_qmm(d, "quantized_matmul") != NVQ_OK || check_grid(d) != NVQ_OK || require_device() != NVQ_OK) return nullptr;
     int64_t batch = 1;
     for (int i = 0; i < d->batch_ndim; i++) batch *= d->batch_shape[i];
@@ -766,7 +768,7 @@ static const char *name_of(const nvq_qmm_desc *d, bool kernel) {
     if (kernel && route == Route::kTiled && qmm_dense_takes(a)) return "qmm_dense_kernel";
     switch (route) {
     case Route::kUntransposed: return qvm_kernel_name(a);
-    case Route::kTiled: return "qmm_kernel";
+    case Route::kTiled: return name == Name::kTile ? qmm_tile_name(a) : "qmm_kernel";
     case Route::kTiledF32: return "qmm_f32_kernel";
     case Route::kGroupedRows: return "qmg_kernel";
     case Route::kBatchedDecode: return "qmr_kernel";
@@ -776,9 +778,11 @@ static const char *name_of(const nvq_qmm_desc *d, bool kernel) {
     }
 }
 
-const char *nvq_quantized_matmul_route(const nvq_qmm_desc *d) { return name_of(d, false); }
+const char *nvq_quantized_matmul_route(const nvq_qmm_desc *d) { return name_of(d, Name::kRoute); }
 
-const char *nvq_quantized_matmul_kernel(const nvq_qmm_desc *d) { return name_of(d, true); }
+const char *nvq_quantized_matmul_kernel(const nvq_qmm_desc *d) { return name_of(d, Name::kKernel); }
+
+const char *nvq_quantized_matmul_tile(const nvq_qmm_desc *d) { return name_of(d, Name::kTile); }
 
 int32_t nvq_quantized_matmul(const nvq_qmm_desc *d, const void *x, const void *w, const void *scales, const void *biases,
                              void *y, void *workspace, void *stream) {

@@ -138,6 +138,7 @@ int32_t launch_qmm(const ProductArgs &a, void *workspace, hipStream_t s);  // wo
 namespace splits { struct Plan; }
 splits::Plan qmm_plan_of(const ProductArgs &a);  // the tile and the split of K
 void qmm_plan_ahead(ProductArgs &a);             // made once for all who ask
+const char *qmm_tile_name(const ProductArgs &a);  // of the kernel and tile of that plan
 double qmm_estimate_us(const ProductArgs &a);  // estimated duration of the tiled kernel with its better tile
 // float32 products of two rows and more on v_mfma_f32_16x16x32_bf16 (weights stored [N, K]); a workspace of partial sums where K is split.
 bool qmm_f32_takes(const ProductArgs &a);  // whether the product's route has its name

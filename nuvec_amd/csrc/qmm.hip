@@ -26,6 +26,15 @@ void qmm_plan_ahead(ProductArgs &a) {
     a.tiled = {p.splits, (int32_t)p.per_split, p.tile, (float)p.estimate_us};
 }
 
+const char *qmm_tile_name(const ProductArgs &a) {
+    switch (qmm_plan_of(a).tile) {
+    case splits::kBig: return "qmm_kernel<256,256>";
+    case splits::kSmall: return "qmm_kernel<128,128>";
+    case splits::kQmk64: return "qmk_kernel<64,128>";
+    default: return "qmk_kernel<128,128>";
+    }
+}
+
 // With its better tile and, for a single product, its better split of K (the caller is expected to bring the
 // workspace the size query names).
 double qmm_estimate_us(const ProductArgs &a) { return qmm_plan_of(a).estimate_us; }

@@ -466,8 +466,14 @@ def quantized_matmul_route(m: int, n: int, k: int, quant: Quant, dtype: torch.dt
 def quantized_matmul_kernel(m: int, n: int, k: int, quant: Quant, dtype: torch.dtype, *, batch=1, transpose: bool = True,
                             row_exact: bool = False, rows: bool = False, device: int = 0) -> str:
     """The kernel that runs such a product: its route's, or on the routes of several 16-bit rows `qms_kernel<..>` or
-    `qmm_dense_kernel`."""
+    `qmm_dense_kernel`.  `qmm_kernel` stands for both tiled kernels (`quantized_matmul_tile`)."""
     return _product_name("nvq_quantized_matmul_kernel", m, n, k, quant, dtype, batch, transpose, row_exact, rows, device)
+
+
+def quantized_matmul_tile(m: int, n: int, k: int, quant: Quant, dtype: torch.dtype, *, batch=1, transpose: bool = True,
+                          row_exact: bool = False, rows: bool = False, device: int = 0) -> str:
+    """The same with `qmm_kernel` told apart: `qmm_kernel<256,256>`, `qmm_kernel<128,128>`, `qmk_kernel<128,128>` or `qmk_kernel<64,128>`."""
+    return _product_name("nvq_quantized_matmul_tile", m, n, k, quant, dtype, batch, transpose, row_exact, rows, device)
 
 
 def _product_name(query, m, n, k, quant, dtype, batch, transpose, row_exact, rows, device) -> str:

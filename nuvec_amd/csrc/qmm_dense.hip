@@ -3,7 +3,7 @@
 // (affine_dequantize_kernel) and multiplied densely, in bfloat16 or float16 on v_mfma_f32_32x32x16.
 //
 // The tiled kernel that expands codes itself (qmk_kernel.h) does so for every 128 rows of x, and two roundings a weight make it bound by
-// the vector unit: 517 rows, W[4096,4096] of 3 bits, 47.5 us.  A weight of N x K costs 2 N K bytes written and, from the chip's last
+// the vector unit: 517 rows, W[4096,4096] of 3 bits, 50 us.  A weight of N x K costs 2 N K bytes written and, from the chip's last
 // cache, read.
 //
 // A block of four wavefronts owns BM x 128 of y, 128 or 256 rows of x, each wavefront BM / 2 x 64, and walks K in steps of 64
@@ -12,8 +12,8 @@
 // instruction at 128 rows, three per four at 256 (a step takes 0.5 and 0.85 us; operands laid out tile by tile beforehand, so
 // that a load is 1 KB of consecutive bytes, took 0.55; eight wavefronts with a quarter of every window each, the two of a SIMD reading and
 // multiplying by turns with a barrier each, 0.65).
-// us, 4 bits, bfloat16, codes expanded in the product -> here: W[4096,4096] at 517 / 1024 / 2048 rows 48 / 70 / 115 -> 40 / 51 / 75;
-// 6 bits W[4064,7680] at 1519 rows 163 -> 114.
+// us, 4 bits, bfloat16, codes expanded in the product -> here: W[4096,4096] at 517 / 2048 rows 46 / 94 -> 41 / 72; W[6144,8192] at 768
+// rows 134 -> 120; 3 bits W[4096,4096] at 517 rows 50 -> 40, 6 bits W[4064,7680] at 1519 rows 147 -> 110.
 #include "qmm_kernel.h"
 
 namespace nvq {
@@ -139,11 +139,15 @@ int32_t run_tile(const ProductArgs &a, const void *weights, hipStream_t s) {
     return NVQ_OK;
 }
 
-// Microseconds of the product by tiles of either height: rounds of a tile per compute unit.
+// Microseconds of the dequantization and the product by tiles of either height: launches and ends of kernels, a weight written and read,
+// rounds of a tile per compute unit, outputs.  Fitted to 1270 timings of both heights (100 to 2048 rows, 1 to 8 bits; 10 and 5 % off).
 template <class D>
-double product_us(const ProductArgs &a) {
-    const double tiles = (double)((a.m + D::BM - 1) / D::BM) * (double)((a.n + D::BN - 1) / D::BN);
-    return ceil(tiles / fmax(1.0, (double)compute_units())) * (double)(a.k / BK) * (D::TI == 2 ? 0.5 : 0.85);
+double dense_us(const ProductArgs &a) {
+    const double tiles = (double)((a.m + D::BM - 1) / D::BM) * (double)((a.n + D::BN - 1) / D::BN), rounds = ceil(tiles / fmax(1.0, (double)compute_units()));
+    const double steps = (double)(a.k / BK), weights = 1.0e-6 * (double)a.n * (double)a.k, outputs = 1.0e-6 * (double)a.m * (double)a.n;
+    const double fill = (double)a.m / (double)((a.m + D::BM - 1) / D::BM * D::BM);  // (rows past the end are one row's bytes)
+    return D::TI == 2 ? 5.4 + 0.6 * weights + rounds * (3.6 + (0.12 + 0.355 * fill) * steps) + 0.5 * outputs
+                      : 4.2 + 0.49 * weights + rounds * (7.5 + (0.53 + 0.126 * fill) * steps) + 0.6 * outputs;
 }
 
 }  // namespace
@@ -153,23 +157,23 @@ size_t qmm_dense_workspace_bytes(const ProductArgs &a) { return (size_t)a.n * (s
 // Half a gigabyte of workspace, W[8191,28672] and a little more: a weight that takes the CPU's values has fewer than 8192 rows.
 constexpr int64_t kMostWeights = 1LL << 28;
 
-// Among the products that the tiled kernels take with the CPU's weights: where the dequantization (7 us of launches and ends of
-// kernels, and 0.48 us per million weights) and the dense product are estimated a twentieth below those.  us here / there, where
-// it turns: W[4096,4096] 512 / 517 rows 42 / 36 and 40 / 47.5; W[1024,4096] 1024 rows 41 / 24; W[576,576] at 517 rows 13 / 9.
+// Among the products that the tiled kernels take with the CPU's weights: where the estimate is at most 1.07 of theirs (this one is the
+// higher where the tiles of a round are few).  us here / there, 4 bits, on both sides of the line: W[4096,4096] at 517 / 576 / 640 / 768 rows
+// 41 / 46, 44 / 43, 49 / 43, 49 / 44; W[6144,8192] at 640 / 768 rows 95 / 81 and 120 / 134; W[6144,4096] at 517 rows 48 / 47; W[4096,8192] at 768 rows
+// 86 / 79; 3 bits W[6144,8192] at 517 rows 83 / 88.
 // (Without a workspace run_tiled sums in this kernel's order.)
 bool qmm_dense_takes(const ProductArgs &a) {
     if (a.mode != NVQ_AFFINE || !a.exact_weights || a.row_exact || a.batch != 1 || a.batch_ndim != 0 || a.rhs != nullptr || a.lhs != nullptr || a.glu != 0)
         return false;
     if (a.k < BK || a.k % BK != 0 || a.k > 1 << 22 || (a.m + 127) / 128 > 65535) return false;  // (32-bit offsets in a tile)
     if (a.n * a.k > kMostWeights) return false;
-    const double here = 7.0 + 0.48e-6 * (double)a.n * (double)a.k + fmin(product_us<Small>(a), product_us<Big>(a));
-    return here < 0.95 * qmm_estimate_us(a);
+    return fmin(dense_us<Small>(a), dense_us<Big>(a)) < 1.07 * qmm_estimate_us(a);
 }
 
 int32_t launch_qmm_dense(const ProductArgs &a, void *workspace, hipStream_t s) {
     const int32_t rc = launch_affine_dequantize(a.dtype, a.group, a.bits, a.w, a.scales, a.biases, a.n * a.k, workspace, nullptr, a.k, a.n, s);
     if (rc != NVQ_OK) return rc;
-    const bool big = product_us<Big>(a) < product_us<Small>(a);
+    const bool big = dense_us<Big>(a) < dense_us<Small>(a);
     if (a.dtype == NVQ_BF16) return big ? run_tile<bf16_t, Big>(a, workspace, s) : run_tile<bf16_t, Small>(a, workspace, s);
     return big ? run_tile<f16_t, Big>(a, workspace, s) : run_tile<f16_t, Small>(a, workspace, s);
 }

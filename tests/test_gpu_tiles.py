@@ -33,3 +33,15 @@ def test_other_kernels_keep_their_names():
         assert ops.quantized_matmul_tile(*p) == ops.quantized_matmul_kernel(*p)
     with pytest.raises(nv.Unsupported):
         ops.quantized_matmul_tile(1, 64, 64, q4, bf16, batch=70000)
+
+
+@pytest.mark.parametrize("m,n,k,bits,dense", [
+    (517, 4096, 4096, 1, True), (517, 4096, 4096, 2, True), (517, 4096, 4096, 4, True), (517, 4096, 4096, 8, True),  # us 39 / 48, 39 / 45, 41 / 46, 42 / 45
+    (768, 6144, 8192, 4, True), (768, 6144, 8192, 8, True),      # 120 / 134, 122 / 136
+    (640, 4096, 4096, 4, False), (640, 6144, 8192, 8, False),    # 49 / 43, 100 / 82
+    (512, 4096, 4096, 4, False), (768, 4096, 8192, 8, False),    # 43 / 34, 88 / 77
+])
+def test_the_weight_is_dequantized_once_where_that_is_faster(m, n, k, bits, dense):
+    """Timed on both sides (us, dequantized / codes expanded in the product)."""
+    quant = nv.Quant.affine(64, bits)
+    assert (nv.quantized_matmul_kernel(m, n, k, quant, torch.bfloat16) == "qmm_dense_kernel") == dense

@@ -12,17 +12,35 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <initializer_list>
+
 #include "nuvec_hip.h"  // NVQ_STATIC_SCRATCH_BYTES
 
 namespace nvq {
 namespace splits {
 
+// Microseconds a step of 64 values of K takes the tiled kernels of weights stored [N, K]: the 256 x 256 tile of qmm_kernel, qmk_kernel's
+// tiles of 128 and of 64 rows, and qmm_kernel's 128 x 128 tile alone on a compute unit and where two of them share one.
+struct StepTimes {
+    float big, qmk128, qmk64, alone, shared;
+};
+// What the expansion of the codes decides: widths whose codes cross words (5 bits above all), two roundings a weight.
+inline StepTimes step_times(int mode, int bits, bool float16, bool exact_weights) {
+    if (mode == NVQ_MXFP4) return {1.05f, 0.36f, 0.273f, 0.456f, 0.67f};
+    if (mode == NVQ_MXFP8) return {1.17f, 0.396f, 0.305f, 0.493f, 0.8f};
+    if (mode == NVQ_NVFP4) return {1.45f, 0.43f, 0.37f, 0.714f, 0.97f};
+    const int width = bits == 5 ? 2 : bits == 3 || bits == 6 ? 1 : 0;
+    static constexpr StepTimes once[] = {{1.27f, 0.442f, 0.378f, 0.61f, 0.95f}, {1.32f, 0.49f, 0.44f, 0.71f, 1.07f}, {1.84f, 0.64f, 0.568f, 0.79f, 1.34f}};
+    static constexpr StepTimes exact16[] = {{1.27f, 0.467f, 0.397f, 0.68f, 1.03f}, {1.32f, 0.524f, 0.476f, 0.766f, 1.16f}, {1.84f, 0.7f, 0.596f, 0.846f, 1.38f}};
+    static constexpr StepTimes exact[] = {{1.27f, 0.533f, 0.469f, 0.91f, 1.36f}, {1.32f, 0.579f, 0.55f, 1.01f, 1.51f}, {1.84f, 0.74f, 0.66f, 1.085f, 1.76f}};
+    return !exact_weights ? once[width] : float16 ? exact16[width] : exact[width];
+}
+
 struct Product {
     int64_t m, n, k, batch;
     bool row_exact;      // every row takes the split of its one-row product
     bool exact_weights;  // the tiled kernels of weights stored [N, K]: qmk_kernel's tiles
-    // those kernels' microseconds a step: qmk_kernel's 128 x 128, qmm_kernel's 256 x 256 and two of its 128 x 128 on a compute unit
-    float step_us = 0.5f, big_step_us = 1.5f, small_step_us = 0.9f;
+    StepTimes step = step_times(NVQ_AFFINE, 4, false, false);
     bool keep_order = false;  // qmm_kernel's tiles only, K whole
 };
 
@@ -52,8 +70,7 @@ inline int64_t qmm_tiles(const Product &a, int tile) {
     return (a.m + rows - 1) / rows * ((a.n + cols - 1) / cols) * a.batch;
 }
 // The plan as it was made when qmm_kernel's 128 x 128 tile (0.8 us a step alone on a compute unit, 1.2 where two share it) stood where
-// qmk_kernel's does: by whole tiles first, then the split of that tile.  What gated pairs and up to 32 rows were timed beside, and the plan of
-// K beyond 14336, the longest that was timed since.
+// qmk_kernel's does: by whole tiles first, then the split of that tile.  What gated pairs and up to 32 rows were timed beside.
 inline Plan qmm_plan_before(const Product &a, int cus) {
     const int64_t steps = (a.k + kQmmStep - 1) / kQmmStep;
     auto tiles_us = [&](int tile, double tiles, double each) {
@@ -73,47 +90,47 @@ inline Plan qmm_plan_before(const Product &a, int cus) {
     return p;
 }
 
-// Estimated microseconds of `tiles` tiles walking `steps` steps on `cus` compute units, a block each, in `splits` parts of K whose sums a
-// second kernel adds up.  Fitted to 4100 timings of 540 products (17 to 2048 rows, W[256..16384, 512..14336], all formats of 16-bit
-// elements, one to six parts): 13 % off on average for qmk_kernel's tiles, 7 % for the 256 x 256 tile; choosing by it costs 2 % against
-// always taking the fastest.
+// Estimated microseconds of `tiles` tiles walking `steps` steps each on `cus` compute units, in `splits` parts of K whose sums a second
+// kernel adds up: a launch, for each round of tiles its first loads and its end, the steps (longer by what the compute units share where
+// all are busy), the outputs.  Fitted (least squares of the relative error, 5 to 7 % off by kernel) to 19000 timings of 1980 products: 17 to
+// 2048 rows, W[256..40000, 64..32768], all formats of 16-bit elements, one to eight parts.
 inline float qmm_tiles_us(const Product &a, int tile, int64_t tiles, int64_t steps, int splits, int cus) {
-    const float outputs = 1.0e-6f * (float)(a.m * a.n * a.batch), walked = (float)((tiles + cus - 1) / cus) * (float)steps;
-    if (tile == kBig) return 12.1f + walked * a.big_step_us + 0.6f * outputs + (splits > 1 ? 1.8f + 0.95f * splits * outputs : 0.0f);
-    if (tile == kSmall) return 3.7f + (float)((tiles + 2 * cus - 1) / (2 * cus)) * (float)steps * a.small_step_us + 1.4f * outputs;
-    const float step = a.step_us * (tile == kQmk128 ? 1.0f : 0.85f);
-    return (tile == kQmk128 ? 5.7f : 4.0f) + walked * step + 2.0f * outputs + (splits > 1 ? 2.2f + 2.0f * splits * outputs : 0.0f);
+    const float outputs = 1.0e-6f * (float)(a.m * a.n * a.batch), parts = splits > 1 ? splits * outputs : 0.0f, each = (float)steps;
+    const float rounds = (float)((tiles + cus - 1) / cus), busy = (float)tiles / (float)cus * each, two = splits > 1 ? 1.0f : 0.0f;
+    switch (tile) {
+    case kBig: return 10.9f + rounds * (2.6f + a.step.big * each) + 0.337f * busy + 1.02f * parts;
+    case kQmk128: return 4.2f + rounds * (2.34f + a.step.qmk128 * each) + 0.081f * busy + 0.63f * outputs + 2.2f * two + 1.36f * parts;
+    case kQmk64: return 2.6f + rounds * (1.9f + a.step.qmk64 * each) + 0.034f * busy + 0.65f * outputs + 2.8f * two + 1.13f * parts;
+    default: return 5.4f + (tiles <= cus ? a.step.alone : (float)((tiles + 2 * cus - 1) / (2 * cus)) * a.step.shared) * each + 0.096f * busy + 0.25f * outputs;
+    }
 }
 
-// The tile and the split of K with the least estimated time.  The splits fill the compute units with few tiles.  Each split has at least
+// The tile and the split of K with the least estimated time (1980 products of 17 to 2048 rows by it and the other kernels' estimates: 0.88 of
+// the time before qmk_kernel, one in 60 more than 5 % slower).  The splits fill the compute units with few tiles.  Each split has at least
 // eight steps, in whole windows and table periods (four steps); at most eight splits; a batch is never split.  K is split as far as the
-// library's own scratch holds the partial sums, so that the entry point without a workspace refuses no product for it (beyond K = 14336 it
-// refuses those of whole steps that it always did).
+// library's own scratch holds the partial sums, so that the entry point without a workspace refuses no product that it took: all up to
+// K = 14336 and of steps and a half, longer ones whose former plan fitted or that other kernels may have taken.  (Beyond the scratch five splits are no faster than two: 768 rows,
+// W[8192,32768] of 4 bits 395 and 395 us.)
 inline Plan qmm_plan(const Product &a, int cus) {
     if (cus < 1) cus = 1;
     const int64_t steps = (a.k + kQmmStep - 1) / kQmmStep;  // (the last one may be a half)
-    if (a.k > 14336) {
-        Plan p = qmm_plan_before(a, cus);
-        p.estimate_us = a.exact_weights ? 1.8 + 1.26 * p.estimate_us : 3.4 + p.estimate_us;
-        return p;
-    }
+    const bool capped = a.k <= 14336 || a.k % kQmmStep != 0 || a.m <= 640 || a.exact_weights || workspace_bytes(qmm_plan_before(a, cus), a) <= (size_t)NVQ_STATIC_SCRATCH_BYTES;
     Plan best{0, 0, 0, 0.0, 0};
     for (const int tile : {kBig, kQmk128, kQmk64, kSmall}) {
         const int64_t tiles = qmm_tiles(a, tile), high = (a.m + (tile == kQmk64 ? kQmkFewRows : kQmmSmallTile) - 1) / (tile == kQmk64 ? kQmkFewRows : kQmmSmallTile);
         if (tile == kBig && a.exact_weights) continue;
         if (tile != kBig && high > 65535 && !(a.exact_weights && tile == kQmk128)) continue;  // (the grid's rows)
-        // (two of these tiles share a compute unit; alone there qmk_kernel's are faster.  The CPU's weights: single products of whole steps.)
         if (a.keep_order && (tile == kQmk128 || tile == kQmk64)) continue;
-        if (tile == kSmall && ((tiles <= cus && !a.keep_order) || (a.exact_weights && (a.batch != 1 || a.k % kQmmStep != 0)))) continue;
+        if (tile == kSmall && a.exact_weights && (a.batch != 1 || a.k % kQmmStep != 0)) continue;  // (has single products of whole steps)
         Plan p{1, steps, steps, qmm_tiles_us(a, tile, tiles, steps, 1, cus), tile};
-        const int64_t most = a.batch == 1 && !a.keep_order && tiles < 2 * cus && tile != kSmall ? steps / 8 : 1;  // (more tiles fill the chip as they are)
-        for (int want = 2; want <= 8 && want <= most; want++) {
+        const int64_t most = a.batch == 1 && !a.keep_order && tiles < 2 * cus && tile != kSmall ? (steps < 64 ? steps / 8 : 8) : 1;  // (more tiles fill the chip as they are)
+        for (int want = 2; want <= most; want++) {
             const int64_t per = ((steps + want - 1) / want + 3) & ~(int64_t)3;
             const int splits = (int)((steps + per - 1) / per);  // every split has a step
             if (splits < 2) continue;
-            if ((double)splits * (double)a.m * (double)a.n * 4.0 > (double)NVQ_STATIC_SCRATCH_BYTES) break;
+            if (capped && (double)splits * (double)a.m * (double)a.n * 4.0 > (double)NVQ_STATIC_SCRATCH_BYTES) break;
             const float us = qmm_tiles_us(a, tile, tiles * splits, per, splits, cus);
-            if (us < 0.95f * (float)p.estimate_us) p.estimate_us = us, p.splits = splits, p.per_split = per;
+            if (us < 0.97f * (float)p.estimate_us) p.estimate_us = us, p.splits = splits, p.per_split = per;
             if (tiles * splits >= 2 * cus) break;
         }
         if (best.splits == 0 || p.estimate_us < best.estimate_us) best = p;

@@ -483,17 +483,8 @@ __global__ void __launch_bounds__(256) qmm_reduce_kernel(const float *__restrict
 // The host rules of nvq_splits.h, here bound to this kernel's constants.
 static_assert(BK == splits::kQmmStep && BigTile::BM == splits::kQmmBigTile && BigTile::BN == splits::kQmmBigTile &&
               SmallTile::BM == splits::kQmmSmallTile && SmallTile::BN == splits::kQmmSmallTile, "nvq_splits.h describes these tiles");
-// What the rules need to know: among it the measured microseconds a step of the tiles (qmm_tiles_us), which the expansion of the codes
-// decides, two roundings a weight above all.
 inline splits::Product split_product(const ProductArgs &a) {
-    const bool f16 = a.dtype == NVQ_F16, odd = a.bits == 3 || a.bits == 5 || a.bits == 6;
-    splits::Product p{a.m, a.n, a.k, a.batch, a.row_exact != 0, a.exact_weights != 0};
-    if (a.mode == NVQ_MXFP4) p.step_us = 0.39f, p.big_step_us = 1.22f, p.small_step_us = 0.69f;
-    else if (a.mode == NVQ_MXFP8) p.step_us = 0.43f, p.big_step_us = 1.3f, p.small_step_us = 0.76f;
-    else if (a.mode == NVQ_NVFP4) p.step_us = 0.42f, p.big_step_us = 1.53f, p.small_step_us = 0.94f;
-    else if (a.exact_weights) p.step_us = (f16 ? 0.5f : 0.57f) + (odd ? 0.1f : 0.0f), p.small_step_us = 1.3f;
-    else if (odd) p.step_us = 0.59f, p.big_step_us = 1.55f, p.small_step_us = 1.13f;
-    else p.step_us = 0.48f, p.big_step_us = 1.34f, p.small_step_us = 0.9f;
+    splits::Product p{a.m, a.n, a.k, a.batch, a.row_exact != 0, a.exact_weights != 0, splits::step_times(a.mode, a.bits, a.dtype == NVQ_F16, a.exact_weights != 0)};
     // (one of a gated pair of few rows and a short K sums in the order it is compared in: before a bias that nearly cancels a product,
     // another order's rounding is many units of the sum)
     p.keep_order = a.mode == NVQ_AFFINE && !a.exact_weights && a.m <= 80 && a.k < 1100;

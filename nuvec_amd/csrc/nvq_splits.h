@@ -138,6 +138,16 @@ inline Plan qmm_plan(const Product &a, int cus) {
     return best;
 }
 
+// What the kernels of a tiled plan take for granted; NULL where it holds, else what does not.  A split reads its tables from a period's start
+// and qmk_kernel walks whole windows of two steps; of the weights with two roundings qmm_kernel has the 128 x 128 tile of whole steps alone.
+inline const char *qmm_plan_fault(const Plan &p, const Product &a) {
+    if (p.units != (a.k + kQmmStep - 1) / kQmmStep || !every_split_has_a_unit(p)) return "a part of K without a step";
+    if (p.splits > 1 && a.batch != 1) return "a batch whose K is split";
+    if (p.splits > 1 && p.per_split % 4 != 0) return "parts of K that are no whole table periods";
+    if (a.exact_weights && (p.tile == kBig || (p.tile == kSmall && (a.batch != 1 || a.k % kQmmStep != 0)))) return "a tile that does not round these weights twice";
+    return nullptr;
+}
+
 // ── the matrix-core kernel of weights stored [K, N] (qmn_kernel) ────────────────────────────────────────────────────
 constexpr int kQmnStep = 64, kQmnTileCols = 128;
 constexpr int kQmnFewRows = 32, kQmnManyRows = 128;          // rows of x per tile

@@ -325,6 +325,8 @@ int32_t run_tiled(const ProductArgs &a, void *workspace, hipStream_t s) {
     splits::Plan p = qmm_plan_of(a);
     if constexpr (FP4 == qmf::kAffine)
         if (qmm_dense_takes(a)) p = splits::Plan{1, p.units, p.units, 0.0, splits::kSmall};
+    if (const char *fault = splits::qmm_plan_fault(p, qmm::split_product(a)))
+        return fail(NVQ_BACKEND, "quantized_matmul: the tiled plan has %s (K = %lld in %d parts of %lld steps)", fault, (long long)a.k, p.splits, (long long)p.per_split);
     return p.tile == splits::kBig || p.tile == splits::kSmall ? qmm::run_dtype<BITS, FP4>(a, p, workspace, s) : qmk::run_dtype<BITS, FP4>(a, p, workspace, s);
 }
 

@@ -1,5 +1,6 @@
 // Host-only checks of the tiled kernels' plan (nuvec_amd/csrc/nvq_splits.h), compiled and run by tests/test_host_tiles.py: the choices
-// among timed tiles and splits of K for 256 compute units.
+// among timed tiles and splits of K for 256 compute units, and what the kernels take for granted, over a grid of shapes, formats and chip
+// sizes: every plan has it, and a plan without it is named before a launch.
 #include <stdio.h>
 #include <string.h>
 
@@ -74,6 +75,36 @@ int main() {
         EXPECT(p.estimate_us > 0.8 * best && p.estimate_us < 1.25 * best, "mode %d, %d bits, %lld rows, W[%lld,%lld]: estimated %.1f us, takes %.1f", c.mode, c.bits,
                (long long)c.m, (long long)c.n, (long long)c.k, p.estimate_us, best);
     }
+    struct { int mode, bits; } formats[] = {{NVQ_AFFINE, 1}, {NVQ_AFFINE, 3}, {NVQ_AFFINE, 4}, {NVQ_AFFINE, 5}, {NVQ_MXFP4, 4}, {NVQ_MXFP8, 8}, {NVQ_NVFP4, 4}};
+    const int64_t ms[] = {5, 17, 33, 64, 65, 129, 300, 640, 641, 2048, 5000000}, ns[] = {8, 129, 1000, 4096, 8192, 32768}, batches[] = {1, 3, 64};
+    const int64_t ks[] = {64, 96, 128, 512, 544, 1056, 1088, 4096, 7200, 14336, 14400, 16384, 16416, 32768, 65536};
+    for (auto f : formats) for (int float16 = 0; float16 < 2; float16++) for (int exact = 0; exact <= (f.mode == NVQ_AFFINE); exact++) for (int keep = 0; keep < 2; keep++)
+        for (int64_t m : ms) for (int64_t n : ns) for (int64_t k : ks) for (int64_t b : batches) for (int cus : {1, 64, 256, 304}) {
+            if (k % kQmmStep != 0 && f.mode == NVQ_AFFINE && !exact) continue;  // (no product of the tiled kernels)
+            if (keep && (exact || f.mode != NVQ_AFFINE)) continue;
+            Product a{m, n, k, b, false, exact != 0, step_times(f.mode, f.bits, float16 != 0, exact != 0)};
+            a.keep_order = keep != 0;
+            const Plan p = qmm_plan(a, cus);
+            g_plans++;
+            const char *fault = qmm_plan_fault(p, a);
+            EXPECT(fault == nullptr, "%s: mode %d, m=%lld n=%lld k=%lld batch=%lld cus=%d", fault, f.mode, (long long)m, (long long)n, (long long)k, (long long)b, cus);
+            EXPECT(p.splits <= 8 && (p.splits == 1 || (!keep && b == 1)), "%d parts", p.splits);
+            EXPECT(!keep || p.tile == kBig || p.tile == kSmall, "tile %d of a product that keeps its order", p.tile);
+            EXPECT(!exact || p.tile != kBig, "256 x 256 with two roundings");
+            EXPECT(p.tile != kQmk64 || (m + 63) / 64 <= 65535, "%lld rows in tiles of 64", (long long)m);
+            if (k <= 14336 || k % kQmmStep != 0)
+                EXPECT(workspace_bytes(p, a) <= (size_t)NVQ_STATIC_SCRATCH_BYTES, "m=%lld n=%lld k=%lld: %zu bytes of partial sums", (long long)m, (long long)n, (long long)k, workspace_bytes(p, a));
+        }
+    const Product plain{300, 700, 4096, 1, false, false}, exact{300, 700, 4096, 1, false, true}, batch{300, 700, 4096, 2, false, false}, half{300, 700, 4128, 1, false, true};
+    const Product exact_batch{300, 700, 4096, 2, false, true};
+    EXPECT(qmm_plan_fault(Plan{1, 64, 64, 0.0, kQmk128}, plain) == nullptr && qmm_plan_fault(Plan{2, 32, 64, 0.0, kQmk64}, plain) == nullptr, "sound plans");
+    EXPECT(qmm_plan_fault(Plan{1, 64, 64, 0.0, kSmall}, exact) == nullptr, "a sound plan");
+    EXPECT(qmm_plan_fault(Plan{5, 16, 64, 0.0, kQmk128}, plain) != nullptr, "a fifth part of four");
+    EXPECT(qmm_plan_fault(Plan{3, 23, 64, 0.0, kQmk128}, plain) != nullptr, "parts of half a window");
+    EXPECT(qmm_plan_fault(Plan{1, 63, 63, 0.0, kQmk128}, plain) != nullptr, "steps of another K");
+    EXPECT(qmm_plan_fault(Plan{2, 32, 64, 0.0, kQmk128}, batch) != nullptr, "a split batch");
+    EXPECT(qmm_plan_fault(Plan{1, 64, 64, 0.0, kBig}, exact) != nullptr, "256 x 256 with two roundings");
+    EXPECT(qmm_plan_fault(Plan{1, 65, 65, 0.0, kSmall}, half) != nullptr && qmm_plan_fault(Plan{1, 64, 64, 0.0, kSmall}, exact_batch) != nullptr, "steps and a half, a batch");
     printf("%ld plans checked, %ld failures\n", g_plans, g_failures);
     return g_failures != 0;
 }

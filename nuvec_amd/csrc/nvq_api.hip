@@ -375,9 +375,6 @@ static nvq::ProductArgs product_args(const nvq_qmm_desc *d, int64_t batch) {
         }
     }
     a.batch_ndim = nd;
-    // (the routes of more than 32 rows, the workspace and the launch ask for the tiled kernels' plan up to six times; fewer rows have
-    // another estimate and few tiled products)
-    if (d->transpose && !a.row_exact && a.m > 32 && compute_units() > 0 && qmm_supported(a)) qmm_plan_ahead(a);
     return a;
 }
 
@@ -851,7 +848,7 @@ struct OneOfTwo {
     OneOfTwo(const nvq_qmm_desc *d, const ProductArgs &pair) : args(pair) {
         args.glu = 0, args.n = pair.n / 2;
         args.tiled_before = 1;
-        args.tiled.splits = 0;  // (the pair's plan)
+        args.tiled.splits = 0;  // (a plan of the pair's is another one)
         route = pick_route(d, args);
         split_bid = split_rows_bid(args, route, split);
     }

@@ -107,10 +107,10 @@ struct ProductArgs {
     int32_t glu;
     float glu_alpha, glu_limit;
     const void *expert_bias;
-    struct {
+    mutable struct {
         int32_t splits, per_split, tile;
         float us;
-    } tiled;                        // host: the tiled kernels' plan (nvq_splits.h), where it was made ahead (splits 0: not)
+    } tiled;                        // host: the tiled kernels' plan (nvq_splits.h), made when it is first asked for (splits 0: not yet)
     int32_t tiled_before;           // host: one of a gated pair, whose choice is by the estimate that was there when pairs were timed
 };
 int32_t launch_qmv(const ProductArgs &a, hipStream_t s);
@@ -136,8 +136,7 @@ bool qmm_supported(const ProductArgs &a);
 size_t qmm_workspace_bytes(const ProductArgs &a);  // float32 partial sums when K is split over the grid, else 0
 int32_t launch_qmm(const ProductArgs &a, void *workspace, hipStream_t s);  // workspace NULL: no split
 namespace splits { struct Plan; }
-splits::Plan qmm_plan_of(const ProductArgs &a);  // the tile and the split of K
-void qmm_plan_ahead(ProductArgs &a);             // made once for all who ask
+splits::Plan qmm_plan_of(const ProductArgs &a);  // the tile and the split of K, made once for all who ask
 const char *qmm_tile_name(const ProductArgs &a);  // of the kernel and tile of that plan
 double qmm_estimate_us(const ProductArgs &a);  // estimated duration of the tiled kernel with its better tile
 // float32 products of two rows and more on v_mfma_f32_16x16x32_bf16 (weights stored [N, K]); a workspace of partial sums where K is split.

@@ -17,13 +17,11 @@ bool qmm_supported(const ProductArgs &a) {
 }
 
 splits::Plan qmm_plan_of(const ProductArgs &a) {
-    if (a.tiled.splits > 0) return splits::Plan{a.tiled.splits, a.tiled.per_split, (a.k + qmm::BK - 1) / qmm::BK, a.tiled.us, a.tiled.tile};
-    return splits::qmm_plan(qmm::split_product(a), compute_units());
-}
-
-void qmm_plan_ahead(ProductArgs &a) {
-    const splits::Plan p = splits::qmm_plan(qmm::split_product(a), compute_units());
-    a.tiled = {p.splits, (int32_t)p.per_split, p.tile, (float)p.estimate_us};
+    if (a.tiled.splits == 0) {
+        const splits::Plan p = splits::qmm_plan(qmm::split_product(a), compute_units());
+        a.tiled = {p.splits, (int32_t)p.per_split, p.tile, (float)p.estimate_us};
+    }
+    return splits::Plan{a.tiled.splits, a.tiled.per_split, (a.k + qmm::BK - 1) / qmm::BK, a.tiled.us, a.tiled.tile};
 }
 
 const char *qmm_tile_name(const ProductArgs &a) {

@@ -244,7 +244,7 @@ NVQ_API const char *nvq_quantized_matmul_route(const nvq_qmm_desc *desc);
 NVQ_API const char *nvq_quantized_matmul_kernel(const nvq_qmm_desc *desc);
 /* The same with "qmm_kernel" told apart by the kernel and its tile, rows of x by weight rows: "qmm_kernel<256,256>", "qmm_kernel<128,128>",
  * "qmk_kernel<128,128>" (each wavefront a quarter of every window of K) or "qmk_kernel<64,128>".  Whether K is split as well is in the size
- * of the workspace. */
+ * of the workspace.  (With a bias, nvq_quantized_linear, affine codes of up to 80 rows and K below 1100 stay on "qmm_kernel<128,128>".) */
 NVQ_API const char *nvq_quantized_matmul_tile(const nvq_qmm_desc *desc);
 /* Bytes of scratch nvq_quantized_matmul needs for `desc` (the reference allocates them on its side of the boundary, gpu.rs:7562; the
  * counterpart of its qmm_t_splitk, gpu.rs:7507-7590).  0 = none; nonzero where K is split over the grid (float32 partial sums): transpose = 0,

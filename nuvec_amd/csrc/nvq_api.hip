@@ -196,13 +196,14 @@ static double tiled_before_us(const nvq::ProductArgs &a) {
     const double steps_us = splits::qmm_plan_before(p, nvq::compute_units() < 1 ? 1 : nvq::compute_units()).estimate_us;
     return a.exact_weights ? 1.8 + 1.26 * steps_us : a.mode == NVQ_MXFP4 ? 3.2 + 0.73 * steps_us : 3.4 + steps_us;
 }
-// The plan's estimate with a margin beside the others' estimates: of 1980 products of 17 to 2048 rows (W[256..40000, 64..32768], timed on
-// every kernel) 108, 96 and 100 are more than 5 % slower than on the kernels before qmk_kernel with 1, 1.05 and 1.15 times it, those all
-// together 0.89 of that time.  Up to 32 rows, and up to 80 of a
-// short K, the choice stays as it was made: gated pairs of a second pass of few rows are checked beside their products there, which have the
-// split-K kernel's bits (NVFP4 W[11444,928] at 70 rows takes 15.5 us there, 10.9 on the tiles).
+// The plan's estimate with a margin beside the others' estimates, from 1980 products of 17 to 2048 rows (W[256..40000, 64..32768], timed on
+// every kernel; 0.88 of the time before qmk_kernel all together).  33 to 80 rows: 31, 29 and 27 of 479 are more than 5 % slower than before
+// with 1.05, 1.1 and 1.15 times it.  More rows: 108, 96 and 100 of all with 1, 1.05 and 1.15.  Up to 32 rows the choice stays as it was
+// made.  So does that of NVFP4 at 65 to 80 rows of a short K, where a test of the split-K kernel's cuts asks for it (W[11444,928] at 70 rows
+// 15.5 us there, 10.9 on the tiles).
 static double tiled_us(const nvq::ProductArgs &a) {
-    return a.tiled_before || a.m <= 32 || (a.m <= 80 && a.k < 1100) ? tiled_before_us(a) : 1.05 * nvq::qmm_estimate_us(a);
+    if (a.tiled_before || a.m <= 32 || (a.mode == NVQ_NVFP4 && a.m > 64 && a.m <= 80 && a.k < 1100)) return tiled_before_us(a);
+    return (a.m <= 80 ? 1.15 : 1.05) * nvq::qmm_estimate_us(a);
 }
 static bool tiled_is_faster(const nvq::ProductArgs &a) { return fmax(7.0, tiled_us(a)) < few_rows_us(a); }  // (its fastest launches, at K = 128, take 6 to 7.4 us)
 
@@ -838,7 +839,8 @@ int32_t nvq_quantized_matmul_glu(const nvq_qmm_desc *d, int32_t activation, floa
     return launch_qmv_glu_pairs(a, (hipStream_t)stream);
 }
 
-// One of the two products that a gated pair is otherwise, and the kernels that would run it.
+// One of the two products that a gated pair is otherwise, and the route it had when pairs were timed beside them: by the tiled kernels'
+// estimate as it was (tiled_before_us), not by the one that now chooses for a product alone.
 struct OneOfTwo {
     ProductArgs args;
     Route route;

@@ -41,7 +41,6 @@ struct Product {
     bool row_exact;      // every row takes the split of its one-row product
     bool exact_weights;  // the tiled kernels of weights stored [N, K]: qmk_kernel's tiles
     StepTimes step = step_times(NVQ_AFFINE, 4, false, false);
-    bool keep_order = false;  // qmm_kernel's tiles only, K whole
 };
 
 struct Plan {
@@ -120,10 +119,9 @@ inline Plan qmm_plan(const Product &a, int cus) {
         const int64_t tiles = qmm_tiles(a, tile), high = (a.m + (tile == kQmk64 ? kQmkFewRows : kQmmSmallTile) - 1) / (tile == kQmk64 ? kQmkFewRows : kQmmSmallTile);
         if (tile == kBig && a.exact_weights) continue;
         if (tile != kBig && high > 65535 && !(a.exact_weights && tile == kQmk128)) continue;  // (the grid's rows)
-        if (a.keep_order && (tile == kQmk128 || tile == kQmk64)) continue;
         if (tile == kSmall && a.exact_weights && (a.batch != 1 || a.k % kQmmStep != 0)) continue;  // (has single products of whole steps)
         Plan p{1, steps, steps, qmm_tiles_us(a, tile, tiles, steps, 1, cus), tile};
-        const int64_t most = a.batch == 1 && !a.keep_order && tiles < 2 * cus && tile != kSmall ? (steps < 64 ? steps / 8 : 8) : 1;  // (more tiles fill the chip as they are)
+        const int64_t most = a.batch == 1 && tiles < 2 * cus && tile != kSmall ? (steps < 64 ? steps / 8 : 8) : 1;  // (more tiles fill the chip as they are)
         for (int want = 2; want <= most; want++) {
             const int64_t per = ((steps + want - 1) / want + 3) & ~(int64_t)3;
             const int splits = (int)((steps + per - 1) / per);  // every split has a step

@@ -484,11 +484,8 @@ __global__ void __launch_bounds__(256) qmm_reduce_kernel(const float *__restrict
 static_assert(BK == splits::kQmmStep && BigTile::BM == splits::kQmmBigTile && BigTile::BN == splits::kQmmBigTile &&
               SmallTile::BM == splits::kQmmSmallTile && SmallTile::BN == splits::kQmmSmallTile, "nvq_splits.h describes these tiles");
 inline splits::Product split_product(const ProductArgs &a) {
-    splits::Product p{a.m, a.n, a.k, a.batch, a.row_exact != 0, a.exact_weights != 0, splits::step_times(a.mode, a.bits, a.dtype == NVQ_F16, a.exact_weights != 0)};
-    // (one of a gated pair of few rows and a short K sums in the order it is compared in: before a bias that nearly cancels a product,
-    // another order's rounding is many units of the sum)
-    p.keep_order = a.mode == NVQ_AFFINE && !a.exact_weights && a.m <= 80 && a.k < 1100;
-    return p;
+    return splits::Product{a.m, a.n, a.k, a.batch, a.row_exact != 0, a.exact_weights != 0,
+                           splits::step_times(a.mode, a.bits, a.dtype == NVQ_F16, a.exact_weights != 0)};
 }
 
 // The partial sums of a split product added up.

@@ -78,18 +78,15 @@ int main() {
     struct { int mode, bits; } formats[] = {{NVQ_AFFINE, 1}, {NVQ_AFFINE, 3}, {NVQ_AFFINE, 4}, {NVQ_AFFINE, 5}, {NVQ_MXFP4, 4}, {NVQ_MXFP8, 8}, {NVQ_NVFP4, 4}};
     const int64_t ms[] = {5, 17, 33, 64, 65, 129, 300, 640, 641, 2048, 5000000}, ns[] = {8, 129, 1000, 4096, 8192, 32768}, batches[] = {1, 3, 64};
     const int64_t ks[] = {64, 96, 128, 512, 544, 1056, 1088, 4096, 7200, 14336, 14400, 16384, 16416, 32768, 65536};
-    for (auto f : formats) for (int float16 = 0; float16 < 2; float16++) for (int exact = 0; exact <= (f.mode == NVQ_AFFINE); exact++) for (int keep = 0; keep < 2; keep++)
+    for (auto f : formats) for (int float16 = 0; float16 < 2; float16++) for (int exact = 0; exact <= (f.mode == NVQ_AFFINE); exact++)
         for (int64_t m : ms) for (int64_t n : ns) for (int64_t k : ks) for (int64_t b : batches) for (int cus : {1, 64, 256, 304}) {
             if (k % kQmmStep != 0 && f.mode == NVQ_AFFINE && !exact) continue;  // (no product of the tiled kernels)
-            if (keep && (exact || f.mode != NVQ_AFFINE)) continue;
-            Product a{m, n, k, b, false, exact != 0, step_times(f.mode, f.bits, float16 != 0, exact != 0)};
-            a.keep_order = keep != 0;
+            const Product a{m, n, k, b, false, exact != 0, step_times(f.mode, f.bits, float16 != 0, exact != 0)};
             const Plan p = qmm_plan(a, cus);
             g_plans++;
             const char *fault = qmm_plan_fault(p, a);
             EXPECT(fault == nullptr, "%s: mode %d, m=%lld n=%lld k=%lld batch=%lld cus=%d", fault, f.mode, (long long)m, (long long)n, (long long)k, (long long)b, cus);
-            EXPECT(p.splits <= 8 && (p.splits == 1 || (!keep && b == 1)), "%d parts", p.splits);
-            EXPECT(!keep || p.tile == kBig || p.tile == kSmall, "tile %d of a product that keeps its order", p.tile);
+            EXPECT(p.splits <= 8 && (p.splits == 1 || b == 1), "%d parts", p.splits);
             EXPECT(!exact || p.tile != kBig, "256 x 256 with two roundings");
             EXPECT(p.tile != kQmk64 || (m + 63) / 64 <= 65535, "%lld rows in tiles of 64", (long long)m);
             if (k <= 14336 || k % kQmmStep != 0)

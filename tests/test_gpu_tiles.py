@@ -122,6 +122,20 @@ def test_quarters_against_float64(tile, split, shapes, form, dtype):
     assert torch.equal(y, got)
 
 
+@pytest.mark.parametrize("m,n,k,form,dtype", [(65, 8256, 896, (64, 4), torch.bfloat16), (80, 9000, 640, (32, 3), torch.bfloat16), (40, 24000, 320, (64, 6), torch.float16)])
+def test_few_rows_of_a_short_k(m, n, k, form, dtype):
+    """Up to 80 rows and K < 1100 products take the plan's tile as others do; before a bias affine ones sum in qmm_kernel's order.  Both within their
+    roundings of float64 (test_quarters_against_float64)."""
+    first_on("qmk_kernel<64,128>", False, [(m, n, k)], form, dtype)
+    q, x, bias = product(m, n, k, form, dtype)
+    w = weights(q, dtype)
+    want, u = x.double() @ w.T, 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    sums = 2.0 ** -24 * k ** 0.5 * x.double().norm(dim=1, keepdim=True) * w.norm(dim=1)
+    assert ((nv.quantized_matmul(x, q).double() - want).abs() <= u * want.abs() + sums).all()
+    with_bias = QuantizedLinear(q.weight, q.scales, q.biases, bias, q.quant)(x).double()
+    assert ((with_bias - want - bias.double()).abs() <= u * (want.abs() + (want + bias.double()).abs()) * 1.01 + sums).all()
+
+
 @pytest.mark.parametrize("tile,m,n,k", [("qmk_kernel<128,128>", 700, 1290, 1984), ("qmk_kernel<64,128>", 300, 700, 704)])
 @pytest.mark.parametrize("form", [(64, 4), (64, 3), "MXFP8", "NVFP4"], ids=str)
 def test_items_of_a_batch(form, tile, m, n, k):

@@ -269,7 +269,7 @@ NVQ_API int32_t nvq_quantized_linear(const nvq_qmm_desc *desc, const void *x, co
 /* No counterpart in the reference: nvq_quantized_matmul for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc) and so cannot bring the workspace.  Same operands,
  * same routing and bit for bit the same results as nvq_quantized_matmul given the workspace its size query names; the
- * partial sums of a split K go to a scratch array inside the library (NVQ_STATIC_SCRATCH_BYTES of device memory, held
+ * partial sums of a split K, or the dequantized weight in parts, go to a scratch array inside the library (NVQ_STATIC_SCRATCH_BYTES of device memory, held
  * by every device the library is loaded on until the process ends).  A product whose partial sums need more is refused
  * with NVQ_UNSUPPORTED.  The call allocates and frees nothing.  All calls on a device share the one array (nothing in
  * it needs clearing: every partial sum a call reads it has written first), so calls that overlap in time on one device,

@@ -663,8 +663,8 @@ static bool split_rows_take(const ProductArgs &a, Route route, qms::Plan &plan) 
 // bits at 3 rows 11.3 -> 12.3.)
 static bool float32_rows_take(const ProductArgs &a, Route route) { return route == Route::kVector && qmm_f32_faster(a, a.m <= 4 ? 0.91 : 1.0); }
 
-// `dense`: whether the workspace may hold the dequantized weight.
-static size_t workspace_bytes(const nvq_qmm_desc *d, bool dense) {
+// `dense`: the most that the workspace may have of the dequantized weight.
+static size_t workspace_bytes(const nvq_qmm_desc *d, size_t dense) {
     if (check_qmm(d, "quantized_matmul") != NVQ_OK) return 0;
     int64_t batch = 1;
     for (int i = 0; i < d->batch_ndim; i++) batch *= d->batch_shape[i];
@@ -677,10 +677,10 @@ static size_t workspace_bytes(const nvq_qmm_desc *d, bool dense) {
     qms::Plan split;
     if (split_rows_take(a, route, split)) return qms_workspace_bytes(a, split);
     if (route != Route::kTiled) return 0;
-    return dense && qmm_dense_takes(a) ? qmm_dense_workspace_bytes(a) : qmm_workspace_bytes(a);
+    return qmm_dense_takes(a) ? qmm_dense_bytes(a, dense) : qmm_workspace_bytes(a);
 }
 
-size_t nvq_quantized_matmul_workspace_bytes(const nvq_qmm_desc *d) { return workspace_bytes(d, true); }
+size_t nvq_quantized_matmul_workspace_bytes(const nvq_qmm_desc *d) { return workspace_bytes(d, SIZE_MAX); }
 
 static Route pick_route(const nvq_qmm_desc *d, const ProductArgs &a) {
     if (!d->transpose) return Route::kUntransposed;        // weights stored [K, N]
@@ -711,7 +711,7 @@ static Route pick_route(const nvq_qmm_desc *d, const ProductArgs &a) {
 
 static int32_t quantized_matmul_any(const nvq_qmm_desc *d, const void *x, const void *w, const void *scales, const void *biases,
                                     const float *global_scale, void *y, void *workspace, void *stream, const void *row_bias = nullptr,
-                                    bool dense = true) {
+                                    size_t dense = SIZE_MAX) {
     NVQ_TRY(check_qmm(d, "quantized_matmul"));
     NVQ_TRY(check_groups("quantized_matmul", d->quant.mode, biases));
     int64_t batch = 1;
@@ -740,7 +740,8 @@ static int32_t quantized_matmul_any(const nvq_qmm_desc *d, const void *x, const 
     switch (route) {
     case Route::kUntransposed: return launch_qvm(a, workspace, (hipStream_t)stream);
     case Route::kTiled:  // without a workspace: codes are expanded in the kernel and K is not split
-        return dense && workspace != nullptr && qmm_dense_takes(a) ? launch_qmm_dense(a, workspace, (hipStream_t)stream) : launch_qmm(a, workspace, (hipStream_t)stream);
+        if (workspace != nullptr && qmm_dense_takes(a)) return launch_qmm_dense(a, workspace, qmm_dense_bytes(a, dense), (hipStream_t)stream);
+        return launch_qmm(a, workspace, (hipStream_t)stream);
     case Route::kTiledF32: return launch_qmm_f32(a, workspace, (hipStream_t)stream);
     case Route::kGroupedRows: return launch_grouped_rows(a, (hipStream_t)stream);
     case Route::kBatchedDecode: return launch_qmr(a, (hipStream_t)stream);
@@ -981,7 +982,7 @@ int32_t nvq_quantized_matmul_glu_grouped(const nvq_qmm_desc *d, int32_t activati
 int32_t nvq_quantized_matmul_static(const nvq_qmm_desc *d, const void *x, const void *w, const void *scales, const void *biases,
                                     void *y, void *stream) {
     NVQ_TRY(check_qmm(d, "quantized_matmul"));
-    const size_t need = workspace_bytes(d, false);  // 0 without a device: the launch below says so
+    const size_t need = workspace_bytes(d, NVQ_STATIC_SCRATCH_BYTES);  // 0 without a device: the launch below says so
     if (need > (size_t)NVQ_STATIC_SCRATCH_BYTES)
         return fail(NVQ_UNSUPPORTED, "quantized_matmul: this product splits K through %zu bytes of partial sums; the static scratch holds %d",
                     need, NVQ_STATIC_SCRATCH_BYTES);
@@ -990,7 +991,7 @@ int32_t nvq_quantized_matmul_static(const nvq_qmm_desc *d, const void *x, const 
         NVQ_TRY(require_device());
         workspace = g_scratch[g_device.device.load(std::memory_order_relaxed)];
     }
-    return quantized_matmul_any(d, x, w, scales, biases, nullptr, y, workspace, stream, nullptr, false);
+    return quantized_matmul_any(d, x, w, scales, biases, nullptr, y, workspace, stream, nullptr, NVQ_STATIC_SCRATCH_BYTES);
 }
 
 int32_t nvq_quantized_matmul_scaled(const nvq_qmm_desc *d, const void *x, const void *w, const void *scales,

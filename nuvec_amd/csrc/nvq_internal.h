@@ -151,7 +151,8 @@ int32_t launch_gated_group(ProductArgs a, int groups, hipStream_t s);
 int32_t launch_grouped_rows(ProductArgs a, hipStream_t s);
 bool qmm_dense_takes(const ProductArgs &a);
 size_t qmm_dense_workspace_bytes(const ProductArgs &a);
-int32_t launch_qmm_dense(const ProductArgs &a, void *workspace, hipStream_t s);
+size_t qmm_dense_bytes(const ProductArgs &a, size_t most);  // of it at a time, given `most` (0: not at all)
+int32_t launch_qmm_dense(const ProductArgs &a, void *workspace, size_t bytes, hipStream_t s);  // fewer bytes than the copy: in parts
 // Batched decode: passes of up to 64 rows of x (5 to 128 rows routed there, where it measured faster), every weight fetched and dequantized once per pass (4- and 8-bit affine codes).
 bool qmr_supported(const ProductArgs &a);
 int32_t launch_qmr(const ProductArgs &a, hipStream_t s);

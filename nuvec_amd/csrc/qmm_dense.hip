@@ -31,7 +31,7 @@ using Small = Dense<2, 5>;
 using Big = Dense<4, 3>;
 
 template <typename T, class D>
-__global__ void __launch_bounds__(D::kThreads, 1) qmm_dense_kernel(const ProductArgs a, const T *__restrict__ weights) {
+__global__ void __launch_bounds__(D::kThreads, 1) qmm_dense_kernel(const ProductArgs a, const int64_t ldy, const T *__restrict__ weights) {
     constexpr int TI = D::TI, TJ = D::TJ, XP = D::XP, kThreads = D::kThreads;
     constexpr int kAhead = D::kRing - 1;  // steps under way
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -120,21 +120,21 @@ __global__ void __launch_bounds__(D::kThreads, 1) qmm_dense_kernel(const Product
             for (int e = 0; e < 16; e += 2) {
                 const uint32_t pair = Ops<T>::pack(add_row_bias<T>(a.row_bias, acc[i][j][e], col), add_row_bias<T>(a.row_bias, acc[i][j][e + 1], col));
                 const int row = row0 + 8 * (e >> 2) + (e & 3);
-                if (row < M) y[(int64_t)row * N + col] = (uint16_t)pair;
-                if (row + 1 < M) y[(int64_t)(row + 1) * N + col] = (uint16_t)(pair >> 16);
+                if (row < M) y[row * ldy + col] = (uint16_t)pair;
+                if (row + 1 < M) y[(row + 1) * ldy + col] = (uint16_t)(pair >> 16);
             }
         }
 }
 
 template <typename T, class D>
-int32_t run_tile(const ProductArgs &a, const void *weights, hipStream_t s) {
+int32_t run_tile(const ProductArgs &a, int64_t ldy, const void *weights, hipStream_t s) {
     static std::atomic<bool> configured = false;
     if (!configured) {
         NVQ_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(qmm_dense_kernel<T, D>), hipFuncAttributeMaxDynamicSharedMemorySize, D::kLdsBytes));
         configured = true;
     }
     const dim3 grid((unsigned)((a.n + D::BN - 1) / D::BN), (unsigned)((a.m + D::BM - 1) / D::BM));
-    hipLaunchKernelGGL((qmm_dense_kernel<T, D>), grid, dim3(D::kThreads), D::kLdsBytes, s, a, (const T *)weights);
+    hipLaunchKernelGGL((qmm_dense_kernel<T, D>), grid, dim3(D::kThreads), D::kLdsBytes, s, a, ldy, (const T *)weights);
     NVQ_LAUNCH_CHECK("qmm_dense");
     return NVQ_OK;
 }
@@ -150,6 +150,28 @@ double dense_us(const ProductArgs &a) {
                       : 4.2 + 0.49 * weights + rounds * (7.5 + (0.53 + 0.126 * fill) * steps) + 0.6 * outputs;
 }
 
+// The entry point without a workspace has the bits of the one with it.  It makes the copy in the library's scratch, a larger one in parts of weight
+// rows unless run_tiled's tile that sums in this kernel's order, K whole, is estimated faster (few tiles a part).  us, that tile -> here: 4 bits
+// W[4096,4096] at 517 rows 69 -> 44, 3 bits W[8035,6912] at 1702 rows 380 -> 222, 4 bits W[6144,8192] at 768 rows 198 -> 165; W[7786,11264] of
+// 5 bits at 337 rows 205 there, 328 in parts.
+constexpr size_t kScratch = NVQ_STATIC_SCRATCH_BYTES;
+// Rows of a part: whole tiles, where they fit, and eight at least, whose codes are whole pieces of 16 bytes.
+int64_t rows_of_a_part(const ProductArgs &a, size_t bytes) {
+    const int64_t most = (int64_t)(bytes / (size_t)(2 * a.k)) / 8 * 8;
+    if (most == 0) return 0;
+    const int64_t parts = (a.n + most - 1) / most, rows = ((a.n + parts - 1) / parts + 127) / 128 * 128;
+    return rows < most ? rows : most;
+}
+double parts_us(const ProductArgs &all) {
+    ProductArgs a = all;
+    a.n = rows_of_a_part(all, kScratch);
+    return a.n == 0 ? HUGE_VAL : (double)((all.n + a.n - 1) / a.n) * fmin(dense_us<Small>(a), dense_us<Big>(a));
+}
+double whole_us(const ProductArgs &a) {
+    const splits::Product p = split_product(a);
+    return splits::qmm_tiles_us(p, splits::kSmall, splits::qmm_tiles(p, splits::kSmall), a.k / BK, 1, compute_units() < 1 ? 1 : compute_units());
+}
+
 }  // namespace
 
 size_t qmm_dense_workspace_bytes(const ProductArgs &a) { return (size_t)a.n * (size_t)a.k * 2; }
@@ -161,7 +183,6 @@ constexpr int64_t kMostWeights = 1LL << 28;
 // higher where the tiles of a round are few).  us here / there, 4 bits, on both sides of the line: W[4096,4096] at 517 / 576 / 640 / 768 rows
 // 41 / 46, 44 / 43, 49 / 43, 49 / 44; W[6144,8192] at 640 / 768 rows 95 / 81 and 120 / 134; W[6144,4096] at 517 rows 48 / 47; W[4096,8192] at 768 rows
 // 86 / 79; 3 bits W[6144,8192] at 517 rows 83 / 88.
-// (Without a workspace run_tiled sums in this kernel's order.)
 bool qmm_dense_takes(const ProductArgs &a) {
     if (a.mode != NVQ_AFFINE || !a.exact_weights || a.row_exact || a.batch != 1 || a.batch_ndim != 0 || a.rhs != nullptr || a.lhs != nullptr || a.glu != 0)
         return false;
@@ -170,12 +191,32 @@ bool qmm_dense_takes(const ProductArgs &a) {
     return fmin(dense_us<Small>(a), dense_us<Big>(a)) < 1.07 * qmm_estimate_us(a);
 }
 
-int32_t launch_qmm_dense(const ProductArgs &a, void *workspace, hipStream_t s) {
-    const int32_t rc = launch_affine_dequantize(a.dtype, a.group, a.bits, a.w, a.scales, a.biases, a.n * a.k, workspace, nullptr, a.k, a.n, s);
-    if (rc != NVQ_OK) return rc;
-    const bool big = dense_us<Big>(a) < dense_us<Small>(a);
-    if (a.dtype == NVQ_BF16) return big ? run_tile<bf16_t, Big>(a, workspace, s) : run_tile<bf16_t, Small>(a, workspace, s);
-    return big ? run_tile<f16_t, Big>(a, workspace, s) : run_tile<f16_t, Small>(a, workspace, s);
+// The bytes of the copy that the kernel is given at a time where `most` are there; 0: run_tiled's tile is the faster one then.
+size_t qmm_dense_bytes(const ProductArgs &a, size_t most) {
+    const size_t all = qmm_dense_workspace_bytes(a);
+    return all <= most ? all : parts_us(a) < whole_us(a) ? most : 0;
+}
+
+// Fewer bytes than the whole copy take it in parts, each multiplied before the next overwrites it: bit for bit the same.
+int32_t launch_qmm_dense(const ProductArgs &all, void *workspace, size_t bytes, hipStream_t s) {
+    const int64_t rows = bytes < qmm_dense_workspace_bytes(all) ? rows_of_a_part(all, bytes) : all.n;
+    if (rows == 0) return fail(NVQ_BACKEND, "quantized_matmul: %zu bytes hold too few rows of K = %lld", bytes, (long long)all.k);
+    const int64_t groups = all.k / all.group, words = all.k / 32 * all.bits;
+    for (int64_t first = 0; first < all.n; first += rows) {
+        ProductArgs a = all;
+        a.n = all.n - first < rows ? all.n - first : rows;
+        a.w = (const uint32_t *)all.w + first * words;
+        a.scales = (const uint16_t *)all.scales + first * groups, a.biases = (const uint16_t *)all.biases + first * groups;
+        a.y = (uint16_t *)all.y + first;
+        if (all.row_bias != nullptr) a.row_bias = (const uint16_t *)all.row_bias + first;
+        const int32_t rc = launch_affine_dequantize(a.dtype, a.group, a.bits, a.w, a.scales, a.biases, a.n * a.k, workspace, nullptr, a.k, a.n, s);
+        if (rc != NVQ_OK) return rc;
+        const bool big = dense_us<Big>(a) < dense_us<Small>(a);
+        const int32_t done = a.dtype == NVQ_BF16 ? (big ? run_tile<bf16_t, Big>(a, all.n, workspace, s) : run_tile<bf16_t, Small>(a, all.n, workspace, s))
+                                                 : (big ? run_tile<f16_t, Big>(a, all.n, workspace, s) : run_tile<f16_t, Small>(a, all.n, workspace, s));
+        if (done != NVQ_OK) return done;
+    }
+    return NVQ_OK;
 }
 
 }  // namespace nvq

@@ -173,3 +173,27 @@ def test_values_without_a_number(form, dtype, tile, m, n, k):
     for row, at, sign in ((7, 0, 1), (m - 1, k - 40, -1)):
         some = w[:, at] != 0  # (zero times infinity is no number)
         assert y[row][some].isinf().all() and (y[row][some] > 0).equal(sign * w[some, at] > 0)
+
+
+@pytest.mark.parametrize("m,n,k,form,dtype", [
+    (517, 4096, 4096, (64, 4), torch.bfloat16),    # the whole copy fits the scratch
+    (1138, 4578, 12800, (64, 4), torch.bfloat16),  # two parts of whole tiles, the last one ragged
+    (1809, 8191, 13696, (64, 3), torch.bfloat16),  # four
+    (4096, 8191, 28672, (32, 1), torch.bfloat16),  # eight, of whole tiles but the last
+    (2049, 1023, 14400, (64, 5), torch.float16),   # one; float16, the CPU's weights of fewer than 1024 outputs
+])
+def test_dequantized_in_the_scratch(m, n, k, form, dtype):
+    """The entry point without a workspace dequantizes a weight in parts that fit the library's scratch: the same bits."""
+    quant = quant_of(form)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert nv.quantized_matmul_kernel(m, n, k, quant, dtype) == "qmm_dense_kernel"
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    words = torch.randint(-(1 << 31), 1 << 31, (n, k * quant.bits // 32), generator=gen, device="cuda", dtype=torch.int64).to(torch.int32).view(torch.uint32)
+    scales = (torch.rand(n, k // quant.group_size, generator=gen, device="cuda") * 0.01 + 0.001).to(dtype)
+    q = nv.Quantized(words, scales, -scales * 2, quant)
+    x = torch.randn(m, k, generator=gen, device="cuda").to(dtype)
+    want, y, p = nv.quantized_matmul(x, q), torch.empty(m, n, dtype=dtype, device="cuda"), ops._ptr
+    d = _lib.QmmDescC()
+    d.quant, d.dtype, d.transpose, d.m, d.n, d.k = quant._c(), ops._CODE[dtype], 1, m, n, k
+    _lib.check(_lib.load().nvq_quantized_matmul_static(C.byref(d), p(x), p(q.weight), p(q.scales), p(q.biases), p(y), ops._stream()))
+    assert torch.equal(y, want)

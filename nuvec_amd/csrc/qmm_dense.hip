@@ -140,14 +140,16 @@ int32_t run_tile(const ProductArgs &a, int64_t ldy, const void *weights, hipStre
 }
 
 // Microseconds of the dequantization and the product by tiles of either height: launches and ends of kernels, a weight written and read,
-// rounds of a tile per compute unit, outputs.  Fitted to 1270 timings of both heights (100 to 2048 rows, 1 to 8 bits; 10 and 5 % off).
+// more beyond what the caches keep, rounds of a tile per compute unit, outputs.  Fitted to 1400 timings of both heights (100 to 2048 rows, 1 to 8
+// bits; 7 and 4 % off).
 template <class D>
 double dense_us(const ProductArgs &a) {
     const double tiles = (double)((a.m + D::BM - 1) / D::BM) * (double)((a.n + D::BN - 1) / D::BN), rounds = ceil(tiles / fmax(1.0, (double)compute_units()));
     const double steps = (double)(a.k / BK), weights = 1.0e-6 * (double)a.n * (double)a.k, outputs = 1.0e-6 * (double)a.m * (double)a.n;
     const double fill = (double)a.m / (double)((a.m + D::BM - 1) / D::BM * D::BM);  // (rows past the end are one row's bytes)
-    return D::TI == 2 ? 5.4 + 0.6 * weights + rounds * (3.6 + (0.12 + 0.355 * fill) * steps) + 0.5 * outputs
-                      : 4.2 + 0.49 * weights + rounds * (7.5 + (0.53 + 0.126 * fill) * steps) + 0.6 * outputs;
+    const double beyond = fmax(0.0, weights - 25.0);
+    return D::TI == 2 ? 5.9 + 0.465 * weights + 0.213 * beyond + rounds * (3.1 + (0.133 + 0.347 * fill) * steps) + 0.63 * outputs
+                      : 4.6 + 0.39 * weights + 0.17 * beyond + rounds * (7.15 + (0.537 + 0.129 * fill) * steps) + 0.69 * outputs;
 }
 
 // The entry point without a workspace has the bits of the one with it.  It makes the copy in the library's scratch, a larger one in parts of weight
@@ -179,8 +181,9 @@ size_t qmm_dense_workspace_bytes(const ProductArgs &a) { return (size_t)a.n * (s
 // Half a gigabyte of workspace, W[8191,28672] and a little more: a weight that takes the CPU's values has fewer than 8192 rows.
 constexpr int64_t kMostWeights = 1LL << 28;
 
-// Among the products that the tiled kernels take with the CPU's weights: where the estimate is at most 1.07 of theirs (this one is the
-// higher where the tiles of a round are few).  us here / there, 4 bits, on both sides of the line: W[4096,4096] at 517 / 576 / 640 / 768 rows
+// Among the products that the tiled kernels take with the CPU's weights: where it is estimated at most 4 % slower (705 products timed on both:
+// 0.2 % above always taking the faster one, a dozen more than 5 %; without the 4 % twelve of 398 others of more than 640 rows are more than 5 %
+// slower than before qmk_kernel, with it eight).  us here / there, 4 bits, on both sides of the line: W[4096,4096] at 517 / 576 / 640 / 768 rows
 // 41 / 46, 44 / 43, 49 / 43, 49 / 44; W[6144,8192] at 640 / 768 rows 95 / 81 and 120 / 134; W[6144,4096] at 517 rows 48 / 47; W[4096,8192] at 768 rows
 // 86 / 79; 3 bits W[6144,8192] at 517 rows 83 / 88.
 bool qmm_dense_takes(const ProductArgs &a) {
@@ -188,7 +191,7 @@ bool qmm_dense_takes(const ProductArgs &a) {
         return false;
     if (a.k < BK || a.k % BK != 0 || a.k > 1 << 22 || (a.m + 127) / 128 > 65535) return false;  // (32-bit offsets in a tile)
     if (a.n * a.k > kMostWeights) return false;
-    return fmin(dense_us<Small>(a), dense_us<Big>(a)) < 1.07 * qmm_estimate_us(a);
+    return fmin(dense_us<Small>(a), dense_us<Big>(a)) < 1.04 * qmm_estimate_us(a);
 }
 
 // The bytes of the copy that the kernel is given at a time where `most` are there; 0: run_tiled's tile is the faster one then.

@@ -197,7 +197,7 @@ static double tiled_before_us(const nvq::ProductArgs &a) {
     return a.exact_weights ? 1.8 + 1.26 * steps_us : a.mode == NVQ_MXFP4 ? 3.2 + 0.73 * steps_us : 3.4 + steps_us;
 }
 // The plan's estimate with a margin beside the others' estimates, from 1980 products of 17 to 2048 rows (W[256..40000, 64..32768], timed on
-// every kernel; 0.88 of the time before qmk_kernel all together).  33 to 80 rows: 31, 29 and 27 of 479 are more than 5 % slower than before
+// every kernel; 0.87 of the time before qmk_kernel all together).  33 to 80 rows: 31, 29 and 27 of 479 are more than 5 % slower than before
 // with 1.05, 1.1 and 1.15 times it.  More rows: 108, 96 and 100 of all with 1, 1.05 and 1.15.  Up to 32 rows the choice stays as it was
 // made.  So does that of NVFP4 at 65 to 80 rows of a short K, where a test of the split-K kernel's cuts asks for it (W[11444,928] at 70 rows
 // 15.5 us there, 10.9 on the tiles).

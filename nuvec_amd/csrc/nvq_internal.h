@@ -87,8 +87,8 @@ struct ProductArgs {
     const int32_t *offsets;         // grouped gather: rows of expert e are [offsets[e], offsets[e+1]) of `batch` rows
     int32_t float32_weights;        // grouped kernel: affine weights of fewer than 64 pairs in float32 (else rounded once)
     int32_t one_group;              // the grouped kernel without offsets: all `batch` rows belong to one weight
-    int32_t k_splits, k_split_steps;  // tiled kernel: K split over grid z (0 or 1: no split), steps of 64 values per split; grouped kernel
-                                      // of one group: the groups of a block that split K (0: by its own rule)
+    int32_t k_splits, k_split_steps;  // tiled kernels: K split over grid z (0 or 1: no split), steps of 64 values per split
+                                      // (qmk_kernel: windows of 128); grouped kernel of one group: the groups of a block that split K (0: by its own rule)
     float *partials;                // tiled kernel with a split: float32 [k_splits][m][n], summed by a second kernel
     const float *global_scale;      // NVFP4: NULL, one float32 value, or one per expert of a gather (weights stored [N, K] only)
     const uint32_t *out_rows;       // gather with the weights stored [N, K]: pair z writes block out_rows[z] of y (NULL: block z)

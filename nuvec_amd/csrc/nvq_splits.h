@@ -104,8 +104,8 @@ inline float qmm_tiles_us(const Product &a, int tile, int64_t tiles, int64_t ste
     }
 }
 
-// The tile and the split of K with the least estimated time (1980 products of 17 to 2048 rows by it and the other kernels' estimates: 0.88 of
-// the time before qmk_kernel, one in 60 more than 5 % slower).  The splits fill the compute units with few tiles.  Each split has at least
+// The tile and the split of K with the least estimated time (1980 products of 17 to 2048 rows by it and the other kernels' estimates: 0.87 of
+// the time before qmk_kernel, one in 60 more than 5 % slower, where one in 30 differs by that between two runs of one side).  The splits fill the compute units with few tiles.  Each split has at least
 // eight steps, in whole windows and table periods (four steps); at most eight splits; a batch is never split.  K is split as far as the
 // library's own scratch holds the partial sums, so that the entry point without a workspace refuses no product that it took: all up to
 // K = 14336 and of steps and a half, longer ones whose former plan fitted or that other kernels may have taken.  (Beyond the scratch five splits are no faster than two: 768 rows,

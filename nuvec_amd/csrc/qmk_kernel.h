@@ -7,15 +7,17 @@
 // tile, 64 of its weight rows and one quarter of every window: no weight is expanded twice in a block and a fragment of x serves two
 // matrix instructions (with 2 x 2 wavefronts of 64 x 64 over all of K, the kernel before, each weight was expanded twice and a SIMD had
 // one wavefront).  The sums of the four quarters meet in LDS at the end.  x, the packed codes and the scales arrive by direct loads
-// into three LDS stages, two windows ahead, one barrier a window; layouts and pieces are those of qmm_kernel.h, scales and biases come
-// 16 bytes a row at a time as in rows_body.h.  A quarter past the end of K is not multiplied, so that K needs no whole windows.
+// into three LDS stages, two windows ahead, one barrier a window; the pieces of a row's codes are those of qmm_kernel.h, scales and
+// biases come 16 bytes a row at a time as in rows_body.h.  A quarter past the end of K is not multiplied, so that K needs no whole windows.
 //
 // What bounds it: the vector instructions of the expansion (512 rows, W[4096,4096] of 4 bits, the CPU's weights: 230 a window and
 // wavefront, two wavefronts a SIMD, beside 16 matrix instructions that cost the issue 14 cycles each: 3080 cycles a window, of which the
-// matrix cores are busy 1024), a block's first loads and the exchange of the sums, 5 us of a short K.  A substep's operands are prepared under
+// matrix cores are busy 1024), with half of the LDS cycles bank conflicts (scales lie 32 bytes a row apart, so that 32 lanes read a quarter of
+// the banks, and the codes of rows r and r + 16 share theirs: SQ_LDS_BANK_CONFLICT 2.05e6 of SQ_LDS_IDX_ACTIVE 4.05e6); a block's first loads and
+// the exchange of the sums, 5 us of a short K.  A substep's operands are prepared under
 // the matrix instructions of the one before (5 % against a window's reads, expansion and products one after the other).
-// us, before -> here: 445 rows, W[2150,1280] of 4 bits 22.4 -> 12.4; 46 rows, W[13247,6688] of NVFP4 48 -> 31; 66 rows, W[16212,4992] of 3
-// bits 47.9 -> 36.4; 455 rows, W[8250,7360] of 3 bits 143 -> 89.  400 products of 17 to 2048 rows: 0.89 of the time all together.
+// us, before -> here: 445 rows, W[2150,1280] of 4 bits 22.6 -> 13.3; 46 rows, W[13247,6688] of NVFP4 49 -> 33; 66 rows, W[16212,4992] of 3
+// bits 45 -> 36; 455 rows, W[8250,7360] of 3 bits 146 -> 93; 512 rows, W[4096,14336] of 4 bits 111 -> 86.
 #pragma once
 
 #include "qmm_kernel.h"

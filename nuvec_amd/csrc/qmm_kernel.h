@@ -8,8 +8,8 @@
 //
 // One block of 256 threads (four wavefronts, one per SIMD, each 256 x 64 of y in 256 accumulator registers) owns a
 // BM x BN = 256 x 256 tile and walks K in steps of BK = 64 through a ring of three LDS stages.  (Products whose 256 x 256 tiles would
-// not fill the chip take qmk_kernel's, or between one and two rounds of those 128 x 128 tiles of 2 x 2 wavefronts here, two blocks
-// per compute unit: 258 rows, W[16291,1408] of MXFP4 23.9 us, 31.1 there.)
+// not fill the chip take qmk_kernel's, or 128 x 128 tiles of 2 x 2 wavefronts here, two blocks per compute unit, by estimate: of a
+// short K in one round, or of one to two rounds that fit at once.  us here / there, 258 rows, W[16291,1408] of MXFP4 24 / 31, 256 rows, W[31806,64] of 6 bits 9 / 16.)
 // A wavefront covers all rows of the tile, so every weight is expanded once per block.  A stage holds
 //   * the x tile, 256 rows x 128 B, 16-byte chunk index XOR-ed with (row >> 1) & 7 so that the 16-byte
 //     fragment reads of the matrix instruction are free of conflicts on the 64 LDS banks, and
